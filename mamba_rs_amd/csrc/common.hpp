@@ -178,6 +178,41 @@ bool tiny_m3_step_ok(int dtype, int input_dim, int dm, int di, int nh, int hd, i
 int launch_tiny_m3_step(hipStream_t st, const TinyM3StepArgs &a);
 bool tiny_step_ok(int dtype, int input_dim, int dm, int di, int ds, int dc, int dr, int xd);
 int launch_tiny_step(hipStream_t st, const TinyStepArgs &a);
+// A whole Mamba-1 backbone step in one resident launch (resident_step.hip), 16-bit storage.  G workgroups per batch row, each owning nc
+// channels and oc out_proj columns (resident_plan fills these in).  weights: n_layers blocks of resident_layer_bytes(), each
+// packed by launch_resident_pack from a layer's weights as the engine holds them.  norm_w: layer 0's norm weight.  xch: batch *
+// xch_stride 64-bit words and epoch: 32 words per row, all zero before the first launch; broken: one word of pinned host memory.
+struct ResidentLayer {   // in_t [2 d_inner][d_model], out_t [d_model][d_inner], dt_t [d_inner][dt_rank] transposed, x_proj [d_inner][xd]; next_nw: the norm weight after, or null
+    const void *in_t, *out_t, *x_proj, *dt_t; const float *a_neg, *conv_w, *conv_b, *D, *dt_b, *next_nw;
+};
+struct ResidentArgs {
+    const void *weights;
+    const float *input, *norm_w, *norm_f;
+    float *conv_state, *ssm_state, *temporal;
+    void *temporal_t;
+    unsigned long long *xch;
+    unsigned *epoch, *broken;
+    size_t xch_stride;
+    float eps;
+    int n_layers, batch, dm, di, ds, dc, dr, xd, G, nc, oc;
+};
+bool resident_plan(ResidentArgs &a, int dtype);   // false: the shape is outside the route
+size_t resident_layer_bytes(const ResidentArgs &a);
+int launch_resident_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
+int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);   // dev: a copy of `a` on the device
+// resident_gate.hip: whether this process's engines may take the resident route on a GPU (a claim counts the engine's
+// workgroups until it is released), and an engine's turn -- held while a step is launched.
+bool resident_claim(int device, int workgroups);
+void resident_release(int device, int workgroups, hipStream_t st);
+class ResidentTurn {
+public:
+    ResidentTurn(int device, hipStream_t st);
+    ~ResidentTurn();
+    ResidentTurn(const ResidentTurn &) = delete;
+    ResidentTurn &operator=(const ResidentTurn &) = delete;
+private:
+    int device_;
+};
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,
                             int64_t rows, int di, int dr);
@@ -218,6 +253,8 @@ struct LmHooks {
     size_t (*state_bytes)(void *self);               // recurrent state, for save / restore around a warm-up run
     int (*state_copy)(void *self, void *buf, int restore);
     int (*prefill)(void *self, const int *dev_tokens, const void *embed, int vocab, int T);   // tokens [batch, T] on device
+    int resident_device;      // the GPU whose ResidentTurn a step's launch needs, or -1
+    int (*check)(void *self); // after a synchronisation: an error if a step could not be completed
 };
 // gathers rows of the embedding table (storage type) as f32: out[r, :] = embed[clamp(tokens[r]), :] (engine prefill staging)
 int launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab);

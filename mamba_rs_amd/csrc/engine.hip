@@ -8,6 +8,7 @@
 // stream, states, a_neg, D, biases and norm weights stay f32 (inference.rs:150-165).
 //
 // Decode, per layer (the reference launches 10 kernels + 4 GEMMs, inference.rs:993-1252):
+//   16-bit storage, a few rows of a model up to d_model 1024: the whole step is one resident launch (resident_step.hip);
 //   16-bit storage, batch <= 64: four kernels on the library's own skinny GEMM (gemm_skinny.hip) -- in_proj with the
 //     RMSNorm folded around it and the conv step + SiLU as epilogue, x_proj, one kernel for dt_proj + dt-bias + softplus
 //     + state update + B/C gather + SiLU gate, out_proj with the residual add as epilogue;
@@ -23,6 +24,7 @@
 #include <new>
 #include <vector>
 #include <algorithm>
+#include <optional>
 
 namespace mrs {
 
@@ -283,6 +285,9 @@ struct mrs_backbone {
     hipStream_t stream;
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
+    int resident;                 // a few rows: the step as one resident launch (resident_step.hip)
+    ResidentArgs res_args, *res_args_dev;
+    unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
     TinyStepLayer *tiny_layers;   // small f32 models: the layer table of the single-launch step (null: kernel chains)
     std::vector<LayerDev> layers;
     float *input_proj_w, *input_proj_b, *norm_f;
@@ -579,6 +584,66 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
     return MRS_OK;
 }
 
+// Resident step (resident_step.hip) for the rows whose workgroups fit on the chip together: chosen before the weights are laid out (the
+// kernel chains' tiled copies are then not needed), set up behind them.
+static void choose_resident(mrs_backbone *bb) {
+    const mrs_m1_config &c = bb->cfg;
+    const char *e = getenv("MRS_DECODE_NO_RESIDENT");
+    if ((e && atoi(e) != 0) || !bb->skinny) return;
+    ResidentArgs &a = bb->res_args;
+    a.eps = c.rms_norm_eps; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
+    a.ds = c.d_state; a.dc = c.d_conv; a.dr = bb->dr; a.xd = bb->xd;
+    if (bb->batch > 256 || !resident_plan(a, bb->dtype) || !resident_claim(bb->device, a.G * a.batch)) return;
+    bb->resident = 1;
+    bb->tiled = bb->wide = 0;
+}
+
+static int arm_resident(mrs_backbone *bb) {
+    const ResidentArgs &a = bb->res_args;
+    MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.epoch, 0, (size_t)a.batch * 128, bb->stream));
+    *bb->res_broken = 0;
+    return MRS_OK;
+}
+
+static int setup_resident(mrs_backbone *bb) {
+    if (!bb->resident) return MRS_OK;
+    const int L = bb->cfg.n_layers;
+    ResidentArgs &a = bb->res_args;
+    a.input = bb->identity_proj ? bb->d_input : bb->step_s.residual;
+    a.norm_f = bb->norm_f; a.conv_state = bb->conv_state; a.ssm_state = bb->ssm_state; a.temporal = bb->temporal; a.temporal_t = bb->temporal_t;
+    MRS_TRY(dev_alloc(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
+    MRS_TRY(dev_alloc(bb, (void **)&a.epoch, (size_t)a.batch * 128));
+    MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
+    a.broken = bb->res_broken;
+    MRS_TRY(arm_resident(bb));
+    const size_t per_layer = resident_layer_bytes(a);
+    char *w = nullptr;
+    MRS_TRY(dev_alloc(bb, (void **)&w, per_layer * (size_t)L));
+    a.weights = w; a.norm_w = bb->layers[0].norm_w;
+    for (int l = 0; l < L; l++, w += per_layer) {
+        LayerDev &d = bb->layers[l];
+        if (!d.dt_w_t) {
+            MRS_TRY(dev_alloc(bb, &d.dt_w_t, (size_t)bb->dr * bb->di * esize(bb->dtype)));
+            MRS_TRY(launch_transpose(bb->stream, bb->dtype, d.dt_w_t, d.dt_w, bb->dr, bb->di));
+        }
+        const ResidentLayer rl = {d.in_proj_t, d.out_proj_t, d.x_proj, d.dt_w_t, d.a_neg, d.conv_w, d.conv_b, d.D, d.dt_b,
+                                  l + 1 < L ? bb->layers[l + 1].norm_w : nullptr};
+        MRS_TRY(launch_resident_pack(bb->stream, a, w, rl));
+    }
+    MRS_TRY(dev_alloc(bb, (void **)&bb->res_args_dev, sizeof(ResidentArgs)));
+    MRS_HIP(hipMemcpyAsync(bb->res_args_dev, &a, sizeof(ResidentArgs), hipMemcpyHostToDevice, bb->stream));
+    return MRS_OK;
+}
+
+// After a synchronisation: whether every resident step found all its workgroups on the chip.
+static int check_resident(mrs_backbone *bb) {
+    if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
+        return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
+                               "or set MRS_DECODE_NO_RESIDENT=1");
+    return MRS_OK;
+}
+
 extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mrs_m1_weights *w,
                                    const mrs_m1_config *cfg, int input_dim, int batch, int dtype) {
     if (!out || !w || !cfg || !w->layers || !w->norm_f_weight) return fail(MRS_E_NULL, "mrs_backbone_create: null pointer");
@@ -653,6 +718,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
             getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
             bb->skinny = 1;
     }
+    choose_resident(bb);
     int *flag = nullptr;
     MRS_CREATE_TRY(dev_alloc(bb, (void **)&flag, sizeof(int)));
     for (int l = 0; l < L; l++) {
@@ -694,7 +760,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
             MRS_CREATE_TRY(launch_tile_weight(bb->stream, bb->dtype, d.in_proj_p, d.in_proj_t, 2 * di, dm));
             MRS_CREATE_TRY(launch_tile_weight(bb->stream, bb->dtype, d.out_proj_p, d.out_proj_t, dm, di));
         }
-        if (bb->skinny || bb->split_xproj) {
+        if ((bb->skinny && !bb->resident) || bb->split_xproj) {
             MRS_CREATE_TRY(dev_alloc(bb, &d.x_proj_t, (size_t)di * xd * esize(bb->dtype)));
             MRS_CREATE_TRY(launch_transpose(bb->stream, bb->dtype, d.x_proj_t, d.x_proj, di, xd));
             if (bb->tiled || bb->split_xproj) {
@@ -737,6 +803,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
     MRS_CREATE_TRY(dev_alloc(bb, (void **)&bb->temporal, (size_t)batch * dm * 4));
     MRS_CREATE_TRY(dev_alloc(bb, &bb->temporal_t, (size_t)batch * dm * esize(dtype)));
     MRS_CREATE_TRY(alloc_scratch(bb, &bb->step_s, batch, 1));
+    MRS_CREATE_TRY(setup_resident(bb));
     MRS_CREATE_TRY(mrs_backbone_reset(bb));
     { hipError_t e = hipStreamSynchronize(bb->stream);
       if (e != hipSuccess) { mrs_backbone_destroy(bb); return fail(MRS_E_HIP, "create sync: %s", hipGetErrorString(e)); } }
@@ -749,8 +816,10 @@ extern "C" void mrs_backbone_destroy(mrs_backbone *bb) {
     if (!bb) return;
     hipSetDevice(bb->device);
     if (bb->stream) hipStreamSynchronize(bb->stream);
+    if (bb->resident) resident_release(bb->device, bb->res_args.G * bb->res_args.batch, bb->stream);
     if (bb->graph_exec) hipGraphExecDestroy(bb->graph_exec);
     if (bb->graph) hipGraphDestroy(bb->graph);
+    if (bb->res_broken) hipHostFree(bb->res_broken);
     for (void *p : bb->allocs) hipFree(p);
     for (void *p : bb->prefill_allocs) hipFree(p);
     gemm_tuner_destroy(bb->tuner);
@@ -764,10 +833,18 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
     const size_t L = bb->cfg.n_layers, B = bb->batch;
     MRS_HIP(hipMemsetAsync(bb->conv_state, 0, L * B * bb->di * bb->cfg.d_conv * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->ssm_state, 0, L * B * bb->di * bb->cfg.d_state * 4, bb->stream));
+    if (bb->res_broken && *(volatile unsigned *)bb->res_broken) {   // a resident step gave up: its exchange words start over with the state
+        MRS_HIP(hipStreamSynchronize(bb->stream));
+        return arm_resident(bb);
+    }
     return MRS_OK;
 }
 
 static int step_body(mrs_backbone *bb) {
+    if (bb->resident) {
+        if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
+        return launch_resident_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+    }
     if (bb->tiny_layers) {
         TinyStepArgs a = {};
         a.layers = bb->tiny_layers; a.input = bb->d_input;
@@ -784,8 +861,15 @@ static int step_body(mrs_backbone *bb) {
     return run_layers(bb, &bb->step_s, 1);
 }
 
+// An engine's turn while a step is launched, where the step is a resident launch (device < 0: it is not).
+struct StepTurn {
+    std::optional<ResidentTurn> turn;
+    StepTurn(int device, hipStream_t st) { if (device >= 0) turn.emplace(device, st); }
+};
+
 extern "C" int mrs_backbone_step_gpu_only(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_step_gpu_only: null engine");
+    const StepTurn turn(bb->resident ? bb->device : -1, bb->stream);
     if (bb->graph_ready) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
     return step_body(bb);
 }
@@ -796,7 +880,7 @@ extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *ou
     MRS_TRY(mrs_backbone_step_gpu_only(bb));
     MRS_HIP(hipMemcpyAsync(output, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident(bb);
 }
 
 // One eager warm step (library handles pick their kernels), reset, then capture the step body
@@ -811,7 +895,8 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     MRS_HIP(hipMalloc(&save, cb + sb));
     hipMemcpyAsync(save, bb->conv_state, cb, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync((char *)save + cb, bb->ssm_state, sb, hipMemcpyDeviceToDevice, bb->stream);
-    int rc = step_body(bb);
+    int rc;
+    { const StepTurn turn(bb->resident ? bb->device : -1, bb->stream); rc = step_body(bb); }
     hipMemcpyAsync(bb->conv_state, save, cb, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->ssm_state, (char *)save + cb, sb, hipMemcpyDeviceToDevice, bb->stream);
     hipStreamSynchronize(bb->stream);
@@ -879,13 +964,13 @@ extern "C" float *mrs_backbone_temporal_ptr(mrs_backbone *bb) { return bb ? bb->
 extern "C" int mrs_backbone_temporal_dtype(mrs_backbone *bb) { return bb ? MRS_F32 : -1; }
 extern "C" int mrs_backbone_decode_route(mrs_backbone *bb) {
     if (!bb) return -1;
-    return bb->tiny_layers ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
+    return bb->tiny_layers || bb->resident ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
 }
 extern "C" int mrs_backbone_download_temporal(mrs_backbone *bb, float *out) {
     if (!bb || !out) return fail(MRS_E_NULL, "mrs_backbone_download_temporal: null pointer");
     MRS_HIP(hipMemcpyAsync(out, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident(bb);
 }
 extern "C" int mrs_backbone_set_gemm_tuning(mrs_backbone *bb, int on) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_set_gemm_tuning: null engine");
@@ -897,7 +982,7 @@ extern "C" float *mrs_backbone_prefill_input_ptr(mrs_backbone *bb) { return bb ?
 extern "C" int mrs_backbone_sync(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_sync: null engine");
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident(bb);
 }
 
 extern "C" int mrs_backbone_state_ptrs(mrs_backbone *bb, int layer, float **conv_state, float **ssm_state) {
@@ -914,7 +999,7 @@ extern "C" int mrs_backbone_download_state(mrs_backbone *bb, int layer, float *c
     if (conv_state) MRS_HIP(hipMemcpyAsync(conv_state, c, (size_t)bb->batch * bb->di * bb->cfg.d_conv * 4, hipMemcpyDeviceToHost, bb->stream));
     if (ssm_state) MRS_HIP(hipMemcpyAsync(ssm_state, s, (size_t)bb->batch * bb->di * bb->cfg.d_state * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident(bb);
 }
 
 // ---- LM: embedding + tied head + greedy loop, all on device -------------------------------
@@ -1019,12 +1104,14 @@ static int m1_hook_prefill(void *self, const int *dev_tokens, const void *embed,
     MRS_TRY(launch_embed_gather(bb->stream, bb->dtype, bb->prefill_in, embed, dev_tokens, (int64_t)bb->batch * T, bb->cfg.d_model, vocab));
     return mrs_backbone_prefill_device(bb, bb->prefill_in, T);
 }
+static int m1_hook_check(void *self) { return check_resident((mrs_backbone *)self); }
 static LmHooks m1_hooks(mrs_backbone *bb) {
     LmHooks h = {};
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
     h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy; h.prefill = m1_hook_prefill;
+    h.resident_device = bb->resident ? bb->device : -1; h.check = m1_hook_check;
     return h;
 }
 
@@ -1141,6 +1228,7 @@ extern "C" int mrs_lm_set_tokens(mrs_lm *lm, const int *tokens) {
 // token, backbone step, tied head, argmax -> next token (left in the device token buffer).
 extern "C" int mrs_lm_decode_step(mrs_lm *lm) {
     if (!lm) return fail(MRS_E_NULL, "mrs_lm_decode_step: null engine");
+    const StepTurn turn(lm->eng.resident_device, lm->eng.stream);
     if (lm->graph_ready) { MRS_HIP(hipGraphLaunch(lm->graph_exec, lm->eng.stream)); return MRS_OK; }
     return lm_decode_body(lm);
 }
@@ -1155,7 +1243,7 @@ extern "C" int mrs_lm_capture_graph(mrs_lm *lm) {
     MRS_HIP(hipMalloc(&save, sbytes + tb));
     int rc = bb->state_copy(bb->self, save, 0);
     hipMemcpyAsync((char *)save + sbytes, lm->tokens, tb, hipMemcpyDeviceToDevice, bb->stream);
-    if (!rc) rc = lm_decode_body(lm);
+    if (!rc) { const StepTurn turn(bb->resident_device, bb->stream); rc = lm_decode_body(lm); }
     if (!rc) rc = bb->state_copy(bb->self, save, 1);
     hipMemcpyAsync(lm->tokens, (char *)save + sbytes, tb, hipMemcpyDeviceToDevice, bb->stream);
     hipStreamSynchronize(bb->stream);
@@ -1177,7 +1265,7 @@ extern "C" int mrs_lm_get_tokens(mrs_lm *lm, int *tokens) {
     if (!lm || !tokens) return fail(MRS_E_NULL, "mrs_lm_get_tokens: null pointer");
     MRS_HIP(hipMemcpyAsync(tokens, lm->tokens, (size_t)lm->batch * sizeof(int), hipMemcpyDeviceToHost, lm->eng.stream));
     MRS_HIP(hipStreamSynchronize(lm->eng.stream));
-    return MRS_OK;
+    return lm->eng.check ? lm->eng.check(lm->eng.self) : MRS_OK;
 }
 
 extern "C" int mrs_lm_last_logits(mrs_lm *lm, float *logits) {
@@ -1185,7 +1273,7 @@ extern "C" int mrs_lm_last_logits(mrs_lm *lm, float *logits) {
     MRS_HIP(hipMemcpy2DAsync(logits, (size_t)lm->vocab * 4, lm->logits, (size_t)lm->vocab_padded * 4, (size_t)lm->vocab * 4, lm->batch,
                              hipMemcpyDeviceToHost, lm->eng.stream));
     MRS_HIP(hipStreamSynchronize(lm->eng.stream));
-    return MRS_OK;
+    return lm->eng.check ? lm->eng.check(lm->eng.self) : MRS_OK;
 }
 
 // Prefill helper for the LM: token ids [batch, T] (host) -> embeddings on device -> backbone prefill,
@@ -1343,6 +1431,7 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
     bool stopped = false;
     for (int s = 0; s < steps && running > 0; s++) {
         if (lm->gen_graph_ready) {
+            const StepTurn turn(bb->resident_device, st);
             MRS_HIP(hipGraphLaunch(lm->gen_graph_exec, st));
         } else if (s == 1) {
             // the first step ran eagerly (the GEMM library settles its choices); capture the step now and replay it from here on
@@ -1356,8 +1445,10 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
             e = hipGraphInstantiate(&lm->gen_graph_exec, gph, nullptr, nullptr, 0);
             if (e != hipSuccess) { hipGraphDestroy(gph); return fail(MRS_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e)); }
             lm->gen_graph = gph; lm->gen_graph_ready = 1;
+            const StepTurn turn(bb->resident_device, st);
             MRS_HIP(hipGraphLaunch(lm->gen_graph_exec, st));
         } else {
+            const StepTurn turn(bb->resident_device, st);
             MRS_TRY(gen_forward(lm));
             MRS_TRY(gen_pick(lm));
         }
@@ -1383,6 +1474,7 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
     MRS_HIP(hipMemcpy2DAsync(out_tokens, (size_t)out_stride * sizeof(int), lm->gen_dyn_host.out, (size_t)lm->gen_dyn_host.out_stride * sizeof(int),
                              (size_t)std::min(out_stride, lm->gen_dyn_host.out_stride) * sizeof(int), B, hipMemcpyDeviceToHost, st));
     MRS_HIP(hipStreamSynchronize(st));
+    if (bb->check) MRS_TRY(bb->check(bb->self));
     if (cb) {
         // stopped by the callback: what was handed over; else whatever the loop has not handed over yet (after a
         // prefilled prompt the first token exists before the first step, so the hand-over runs one step behind)

@@ -1224,6 +1224,6 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = nullptr;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
-    h.prefill = m3_hook_prefill;
+    h.prefill = m3_hook_prefill; h.resident_device = -1;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");
 }

@@ -1,0 +1,156 @@
+// Building blocks of the resident decode steps (resident_step.hip): one launch walks the whole network, G workgroups
+// share every layer's columns, and what a layer's phases need from each other travels through memory while the workgroups stay
+// on the chip.
+//
+// Exchange: a value and the number of the layer it belongs to (its tag) are one 64-bit word, stored and polled with relaxed
+// agent-scope atomics.  The word is its own flag, so a phase costs one store and one load to the coherence point of the
+// chip -- no counter, no fence, no cache write-back.  Measured for all-to-all exchanges of 768 values, two workgroup
+// barriers included: 1.3 us among 32 workgroups, 1.5 among 64, 1.8 among 128, 2.4 among 256 (a counter barrier over 256
+// workgroups: 2.3 to 3.7 us and the data still to be fetched; a kernel boundary in a graph: about 4 us).
+// A layer's exchanges form a cycle (residual -> x_proj shares -> y -> residual), each of them all-to-all, so a buffer is
+// rewritten only after every reader of its last contents has published something that depends on them: one buffer per
+// exchange is enough.
+//
+// Every wait is bounded (kSpinLimit polls, about two seconds): a workgroup that gives up leaves, the others follow, the
+// output rows become NaN and `broken` (host memory) is raised, which the engine turns into an error.  It does not happen as
+// long as all workgroups of a launch fit on the chip together, which the engine's slot budget sees to.
+#pragma once
+#include "common.hpp"
+#include "mfma_tiles.hpp"
+
+namespace mrs {
+
+typedef unsigned long long u64;
+constexpr unsigned kSpinLimit = 1u << 21;
+
+__device__ __forceinline__ void xch_put(u64 *p, float v, unsigned tag) {
+    __hip_atomic_store(p, ((u64)tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 xch_get(const u64 *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+__device__ __forceinline__ int here_s(int v) { asm volatile("" : "+s"(v)); return v; }   // the same for a value all lanes share
+
+// A table that no kernel writes, read through the scalar cache.
+template <typename V> using scalar_table = const __attribute__((address_space(4))) V *;
+template <typename V> __device__ __forceinline__ scalar_table<V> as_table(const V *p) { return (scalar_table<V>)(uintptr_t)p; }
+
+// Sum over the 16 lanes of a DPP row, in every lane of it.
+__device__ __forceinline__ float row16_sum(float v) {
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xf, 0xf, false));   // row_ror:8
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124, 0xf, 0xf, false));
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x122, 0xf, 0xf, false));
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x121, 0xf, 0xf, false));
+    return v;
+}
+
+// Keeps what is computed from v inside the scope it is used in: a layer loop's many lane-dependent addresses would otherwise all
+// be hoisted out of it, and spilled.
+__device__ __forceinline__ int here(int v) { asm volatile("" : "+v"(v)); return v; }
+
+// base (the same for the whole wave) + a 32-bit lane offset in bytes: one scalar base and one vector register per access
+template <typename V> __device__ __forceinline__ V ld_off(const void *base, unsigned bytes) {
+    return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + bytes);
+}
+
+// One wave copies the 1 KB pieces first, first + step, ... below `pieces` of contiguous memory to LDS byte address `to` (both 16-byte
+// aligned) without passing through registers.  The compiler's wait counting does not see it: dma_wait() by the same wave and a
+// workgroup barrier come before the data is read.  Requests are spaced (s_sleep 1: 64 clocks): a compute unit's requests are
+// served in order, and a burst of them would stand in front of the exchange's stores and polls.
+__device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int first, int pieces, int step) {
+    const u64 at = (u64)(uintptr_t)from;   // the same for the whole wave
+    const u64 src = (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)at) | (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32;
+    const unsigned lane16 = (unsigned)(threadIdx.x & 63) * 16u, dst0 = __builtin_amdgcn_readfirstlane(to);
+#pragma unroll 1
+    for (int i = first; i < pieces; i += step) {
+        const unsigned voff = (unsigned)i * 1024u + lane16, dst = dst0 + (unsigned)i * 1024u;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_sleep 1" ::"s"(dst), "v"(voff), "s"(src) : "m0", "memory");
+    }
+}
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Sum over a wave, in lane 63.
+__device__ __forceinline__ float wave_sum_last(float v) {
+    v = row16_sum(v);
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x142, 0xa, 0xf, false));   // row_bcast:15 into rows 1 and 3
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x143, 0xc, 0xf, false));   // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+constexpr int kComputeWaves = 8;
+
+// Two f32 in one exchange word: the lowest mantissa bit of each carries the parity of the layer's tag (a buffer's entries are
+// rewritten every layer, so what is not of this layer is of the one before).
+__device__ __forceinline__ u64 pair_word(float a, float b, unsigned tag) {
+    const unsigned x = (__float_as_uint(a) & ~1u) | (tag & 1u), y = (__float_as_uint(b) & ~1u) | (tag & 1u);
+    return (u64)y << 32 | x;
+}
+// Two 16-bit values and the tag.
+template <typename T> __device__ __forceinline__ u64 half_pair_word(T a, T b, unsigned tag) {
+    return (u64)tag << 32 | (unsigned)__builtin_bit_cast(uint16_t, b) << 16 | __builtin_bit_cast(uint16_t, a);
+}
+__device__ __forceinline__ void xch_put_word(u64 *p, u64 w) { __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Polls the KU words base[idx(0)] .. base[idx(KU - 1)] until ready(word) holds for all of them.  False when the wait was given up.
+template <int KU, class IDX, class READY>
+__device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, u64 (&r)[KU]) {
+    for (unsigned spins = 0; spins <= kSpinLimit; spins++) {
+        bool have = true;
+#pragma unroll
+        for (int u = 0; u < KU; u++) r[u] = xch_get(base + idx(u));
+#pragma unroll
+        for (int u = 0; u < KU; u++) have = have && ready(r[u]);
+        if (have) return true;
+    }
+    return false;
+}
+
+// One row's product on the matrix cores, K split over the computing waves in steps of 32 (step wave, wave + 8, ...; at most KS per wave):
+// the weight in LDS as [K / 8][cols][8], 16 CT columns of it (columns past `cols` repeat the last one), x in LDS.  take() brings this
+// wave's pieces of the weight into registers, which can be done while x is still on its way; run() leaves this wave's share of
+// column c in out[wave * 16 CT + c].  Only one of the sixteen rows of a matrix instruction is used: what the product costs is
+// bringing the weights from LDS.
+template <typename T, int KS, int CT> struct RowProduct {
+    uint4 w[KS][CT];
+    __device__ __forceinline__ void take(const T *wl, int cols, int ksteps, int ct) {
+        const int t = here(threadIdx.x), l = t & 63, n = l & 15, kg = l >> 4, w0 = __builtin_amdgcn_readfirstlane(t >> 6);
+        const uint4 *wp = reinterpret_cast<const uint4 *>(wl);
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+            if (c < ct) {
+                const int col = min(c * 16 + n, cols - 1);
+#pragma unroll
+                for (int s = 0; s < KS; s++)
+                    if (w0 + kComputeWaves * s < ksteps) w[s][c] = wp[(unsigned)(((w0 + kComputeWaves * s) * 4 + kg) * cols + col)];
+            }
+    }
+    __device__ __forceinline__ void run(const T *x, int ksteps, int ct, float *out) const {
+        const int t = here(threadIdx.x), l = t & 63, kg = l >> 4, w0 = __builtin_amdgcn_readfirstlane(t >> 6);
+        v4f acc[CT];
+#pragma unroll
+        for (int c = 0; c < CT; c++) acc[c] = (v4f){0.f, 0.f, 0.f, 0.f};
+        uint4 a[KS];
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+            if (w0 + kComputeWaves * s < ksteps) a[s] = reinterpret_cast<const uint4 *>(x)[(w0 + kComputeWaves * s) * 4 + kg];   // the same for all rows
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+            if (w0 + kComputeWaves * s < ksteps) {
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[c] = Mma32<T>::mma(a[s], w[s][c], acc[c]);
+            }
+        if (l < 16) {   // row 0, column l % 16 is register 0 of lanes 0 to 15
+#pragma unroll
+            for (int c = 0; c < CT; c++)
+                if (c < ct) out[w0 * 16 * ct + c * 16 + l] = acc[c][0];
+        }
+    }
+};
+// the waves' shares of column c, added in wave order
+__device__ __forceinline__ float row_sum(const float *out, int cols16, int c) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kComputeWaves; w++) v += out[w * cols16 + c];
+    return v;
+}
+
+}  // namespace mrs
