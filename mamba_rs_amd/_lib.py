@@ -71,6 +71,12 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def host_rows_call(name: str):
+    """An entry point fn(engine, input, output) on host rows as a callable taking plain addresses: building the typed pointer
+    objects of the general binding costs more than the call itself (a few microseconds of a step of fifty)."""
+    return ctypes.CFUNCTYPE(c_int, _P, _P, _P)((name, load()))
+
+
 def exported_names() -> list[str]:
     return sorted(_SIGNATURES)
 

@@ -155,12 +155,15 @@ int launch_transpose(hipStream_t st, int dtype, void *Wt, const void *W, int K, 
 struct TinyStepLayer {
     const float *norm_w, *in_proj, *conv_w, *conv_b, *x_proj, *dt_w, *dt_b, *a_neg, *D, *out_proj;
 };
+struct HostRows { float *out; unsigned *done; unsigned seq; };   // host_io.hpp: where a step leaves its rows for the host (out null: nowhere)
 struct TinyStepArgs {
     const TinyStepLayer *layers;
     const float *input, *in_w, *in_b, *norm_f;
     float *conv_state, *ssm_state, *temporal;
     float eps;
     int n_layers, batch, input_dim, dm, di, ds, dc, dr, xd;
+    float *input_copy;   // input is pinned host memory: the device's input rows, kept up to date (or null)
+    HostRows host;
 };
 // The same for the Mamba-3 SISO backbone (csrc/tiny_m3_step.hip): in_proj [dm][ip], out_proj [di][dm] row-major f32;
 // states as the engine holds them ([layer][batch]...).
@@ -173,6 +176,8 @@ struct TinyM3StepArgs {
     float *ssm, *kst, *vst, *angle, *temporal;
     float eps, a_floor;
     int n_layers, batch, input_dim, dm, di, nh, hd, ds, ng, nr, ip, outproj_norm;
+    float *input_copy;
+    HostRows host;
 };
 bool tiny_m3_step_ok(int dtype, int input_dim, int dm, int di, int nh, int hd, int ds, int ng, int nr, int ip);
 int launch_tiny_m3_step(hipStream_t st, const TinyM3StepArgs &a);

@@ -19,6 +19,7 @@
 #include "common.hpp"
 #include "glue.hpp"
 #include "gemm_tune.hpp"
+#include "host_io.hpp"
 #include <rocblas/rocblas.h>
 #include <stdlib.h>
 #include <new>
@@ -288,6 +289,7 @@ struct mrs_backbone {
     int resident;                 // a few rows: the step as one resident launch (resident_step.hip)
     ResidentArgs res_args, *res_args_dev;
     unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
+    HostIo io;                    // step()'s rows in pinned host memory
     TinyStepLayer *tiny_layers;   // small f32 models: the layer table of the single-launch step (null: kernel chains)
     std::vector<LayerDev> layers;
     float *input_proj_w, *input_proj_b, *norm_f;
@@ -803,6 +805,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
     MRS_CREATE_TRY(dev_alloc(bb, (void **)&bb->temporal, (size_t)batch * dm * 4));
     MRS_CREATE_TRY(dev_alloc(bb, &bb->temporal_t, (size_t)batch * dm * esize(dtype)));
     MRS_CREATE_TRY(alloc_scratch(bb, &bb->step_s, batch, 1));
+    MRS_CREATE_TRY(host_io_create(&bb->io, batch, input_dim, dm));
     MRS_CREATE_TRY(setup_resident(bb));
     MRS_CREATE_TRY(mrs_backbone_reset(bb));
     { hipError_t e = hipStreamSynchronize(bb->stream);
@@ -820,6 +823,7 @@ extern "C" void mrs_backbone_destroy(mrs_backbone *bb) {
     if (bb->graph_exec) hipGraphExecDestroy(bb->graph_exec);
     if (bb->graph) hipGraphDestroy(bb->graph);
     if (bb->res_broken) hipHostFree(bb->res_broken);
+    host_io_destroy(&bb->io);
     for (void *p : bb->allocs) hipFree(p);
     for (void *p : bb->prefill_allocs) hipFree(p);
     gemm_tuner_destroy(bb->tuner);
@@ -840,7 +844,8 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
     return MRS_OK;
 }
 
-static int step_body(mrs_backbone *bb) {
+// host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
+static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
     if (bb->resident) {
         if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
         return launch_resident_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
@@ -852,6 +857,7 @@ static int step_body(mrs_backbone *bb) {
         a.norm_f = bb->norm_f; a.conv_state = bb->conv_state; a.ssm_state = bb->ssm_state; a.temporal = bb->temporal;
         a.eps = bb->cfg.rms_norm_eps; a.n_layers = bb->cfg.n_layers; a.batch = bb->batch; a.input_dim = bb->input_dim;
         a.dm = bb->cfg.d_model; a.di = bb->di; a.ds = bb->cfg.d_state; a.dc = bb->cfg.d_conv; a.dr = bb->dr; a.xd = bb->xd;
+        if (host) { a.input = bb->io.in; a.input_copy = bb->d_input; a.host = *host; }
         return launch_tiny_step(bb->stream, a);
     }
     // identity projection on the own-GEMM chain: the first layer's prenorm kernel reads the input and writes the
@@ -870,16 +876,27 @@ struct StepTurn {
 extern "C" int mrs_backbone_step_gpu_only(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_step_gpu_only: null engine");
     const StepTurn turn(bb->resident ? bb->device : -1, bb->stream);
-    if (bb->graph_ready) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
+    if (bb->graph_ready && !one_launch) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
     return step_body(bb);
 }
 
 extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *output) {
     if (!bb || !input || !output) return fail(MRS_E_NULL, "mrs_backbone_step: null pointer");
-    MRS_HIP(hipMemcpyAsync(bb->d_input, input, (size_t)bb->batch * bb->input_dim * 4, hipMemcpyHostToDevice, bb->stream));
-    MRS_TRY(mrs_backbone_step_gpu_only(bb));
-    MRS_HIP(hipMemcpyAsync(output, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
-    MRS_HIP(hipStreamSynchronize(bb->stream));
+    const int B = bb->batch, dm = bb->cfg.d_model, n = B * bb->input_dim;
+    HostIo &io = bb->io;
+    memcpy(io.in, input, (size_t)n * 4);
+    const HostRows host = {io.out, io.done, ++io.seq};
+    if (bb->tiny_layers) {
+        MRS_TRY(step_body(bb, &host));
+    } else {
+        hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
+        MRS_TRY(mrs_backbone_step_gpu_only(bb));
+        hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
+        MRS_TRY(check_launch("host row kernels"));
+    }
+    MRS_TRY(host_io_wait(&io, bb->stream));
+    memcpy(output, io.out, (size_t)B * dm * 4);
     return check_resident(bb);
 }
 

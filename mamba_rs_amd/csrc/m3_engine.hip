@@ -15,6 +15,7 @@
 // Shapes the skinny GEMM does not take (f32 storage above four rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
 #include "common.hpp"
 #include "gemm_tune.hpp"
+#include "host_io.hpp"
 #include <stdlib.h>
 #include "glue.hpp"
 #include "m3_math.hpp"
@@ -561,6 +562,7 @@ struct mrs_m3_backbone {
     hipStream_t stream;
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
+    HostIo io;              // step()'s rows in pinned host memory
     TinyM3StepLayer *tiny_layers;   // small f32 models: the layer table of the single-launch step (null: kernel chains)
     std::vector<Layer3> layers;
     std::vector<void *> allocs;
@@ -631,7 +633,8 @@ int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
     return check_launch("m3_layer_step_kernel");
 }
 
-int step_body3(mrs_m3_backbone *bb) {
+// host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
+int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
     const mrs_m3_config &c = bb->cfg;
     if (bb->tiny_layers) {
         TinyM3StepArgs a = {};
@@ -641,6 +644,7 @@ int step_body3(mrs_m3_backbone *bb) {
         a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.input_dim = bb->input_dim;
         a.dm = c.d_model; a.di = bb->di; a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr; a.ip = bb->ip;
         a.outproj_norm = c.is_outproj_norm;
+        if (host) { a.input = bb->io.in; a.input_copy = bb->d_input; a.host = *host; }
         return launch_tiny_m3_step(bb->stream, a);
     }
     const int dm = c.d_model, di = bb->di, B = bb->batch, dt = bb->dtype, L = c.n_layers, ip = bb->ip;
@@ -711,6 +715,7 @@ extern "C" void mrs_m3_backbone_destroy(mrs_m3_backbone *bb) {
     if (bb->graph) hipGraphDestroy(bb->graph);
     for (void *p : bb->allocs) hipFree(p);
     for (void *p : bb->pf_allocs) hipFree(p);
+    host_io_destroy(&bb->io);
     gemm_tuner_destroy(bb->tuner);
     if (bb->blas) rocblas_destroy_handle(bb->blas);
     if (bb->stream) hipStreamDestroy(bb->stream);
@@ -844,6 +849,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     MRS_CREATE_TRY(dev_alloc3(bb, &bb->normed, B16 * dm * es));
     MRS_CREATE_TRY(dev_alloc3(bb, &bb->gated, B16 * di * es));
     MRS_CREATE_TRY(dev_alloc3(bb, &bb->out, B * dm * es));
+    MRS_CREATE_TRY(host_io_create(&bb->io, batch, input_dim, dm));
     MRS_CREATE_TRY(mrs_m3_backbone_reset(bb));
     { hipError_t e = hipStreamSynchronize(bb->stream);
       if (e != hipSuccess) { mrs_m3_backbone_destroy(bb); return fail(MRS_E_HIP, "create sync: %s", hipGetErrorString(e)); } }
@@ -854,16 +860,27 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
 
 extern "C" int mrs_m3_backbone_step_gpu_only(mrs_m3_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_step_gpu_only: null engine");
-    if (bb->graph_ready) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    // (a step of one launch is launched quicker than a graph of one node)
+    if (bb->graph_ready && !bb->tiny_layers) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
     return step_body3(bb);
 }
 
 extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, float *output) {
     if (!bb || !input || !output) return fail(MRS_E_NULL, "mrs_m3_backbone_step: null pointer");
-    MRS_HIP(hipMemcpyAsync(bb->d_input, input, (size_t)bb->batch * bb->input_dim * 4, hipMemcpyHostToDevice, bb->stream));
-    MRS_TRY(mrs_m3_backbone_step_gpu_only(bb));
-    MRS_HIP(hipMemcpyAsync(output, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
-    MRS_HIP(hipStreamSynchronize(bb->stream));
+    const int B = bb->batch, dm = bb->cfg.d_model, n = B * bb->input_dim;
+    HostIo &io = bb->io;
+    memcpy(io.in, input, (size_t)n * 4);
+    const HostRows host = {io.out, io.done, ++io.seq};
+    if (bb->tiny_layers) {
+        MRS_TRY(step_body3(bb, &host));
+    } else {
+        hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
+        MRS_TRY(mrs_m3_backbone_step_gpu_only(bb));
+        hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
+        MRS_TRY(check_launch("host row kernels"));
+    }
+    MRS_TRY(host_io_wait(&io, bb->stream));
+    memcpy(output, io.out, (size_t)B * dm * 4);
     return MRS_OK;
 }
 

@@ -7,6 +7,7 @@
 // the trapezoidal state update, D skip, SiLU gate or RMSNormGated), states updated in place.  Only the order of the
 // dot-product sums differs from the kernel chain, and it is fixed.
 #include "tiny_rows.hpp"
+#include "host_io.hpp"
 #include "m3_math.hpp"
 
 namespace mrs {
@@ -30,7 +31,11 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_m3_backbone_step_kernel(Tin
     const int lg = ds >> 2, per_head = hd * lg, tasks = nh * per_head;   // one lane-task per float4 of SSM state
     const int na = nr > 0 ? nr : 1;
 
-    for (int i = tid; i < a.input_dim; i += kTinyThreads) xin[i] = a.input[(int64_t)b * a.input_dim + i];
+    for (int i = tid; i < a.input_dim; i += kTinyThreads) {
+        const float v = a.input[(int64_t)b * a.input_dim + i];
+        xin[i] = v;
+        if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + i] = v;   // (the input came straight from host memory)
+    }
     __syncthreads();
     if (a.in_w) {
         gemv_rows(a.in_w, a.input_dim, dm, xin, res, part, a.in_b);
@@ -144,7 +149,12 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_m3_backbone_step_kernel(Tin
     float ss = 0.0f;
     for (int i = tid; i < dm; i += kTinyThreads) ss = fmaf(res[i], res[i], ss);
     const float inv = rms_inv(block_sum(ss, red), dm, a.eps);
-    for (int i = tid; i < dm; i += kTinyThreads) a.temporal[(int64_t)b * dm + i] = res[i] * inv * a.norm_f[i];
+    for (int i = tid; i < dm; i += kTinyThreads) {
+        const float v = res[i] * inv * a.norm_f[i];
+        a.temporal[(int64_t)b * dm + i] = v;
+        if (a.host.out) a.host.out[(int64_t)b * dm + i] = v;
+    }
+    if (a.host.out) host_row_done(a.host, b);
 }
 
 size_t tiny_m3_lds_bytes(int input_dim, int dm, int di, int nh, int ds, int ng, int ip) {

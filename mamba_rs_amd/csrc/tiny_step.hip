@@ -8,6 +8,7 @@
 // written in place.  Arithmetic per element is that of the separate kernels (same softplus, SiLU, exp2 forms, f32
 // accumulation); only the order of the dot-product sums differs, and it is fixed (same result on every run).
 #include "tiny_rows.hpp"
+#include "host_io.hpp"
 #include <algorithm>
 
 namespace mrs {
@@ -32,7 +33,11 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
 
     TinyStepLayer lnext = a.layers[0];
     // input row -> residual stream (identity or projection + bias)
-    for (int i = tid; i < a.input_dim; i += kTinyThreads) xin[i] = a.input[(int64_t)b * a.input_dim + i];
+    for (int i = tid; i < a.input_dim; i += kTinyThreads) {
+        const float v = a.input[(int64_t)b * a.input_dim + i];
+        xin[i] = v;
+        if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + i] = v;   // (the input came straight from host memory)
+    }
     __syncthreads();
     if (a.in_w) {
         gemv_rows(a.in_w, a.input_dim, dm, xin, res, part, a.in_b);
@@ -151,7 +156,12 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     float ss = 0.0f;
     for (int i = tid; i < dm; i += kTinyThreads) ss = fmaf(res[i], res[i], ss);
     const float inv = rms_inv(block_sum(ss, red), dm, a.eps);
-    for (int i = tid; i < dm; i += kTinyThreads) a.temporal[(int64_t)b * dm + i] = res[i] * inv * a.norm_f[i];
+    for (int i = tid; i < dm; i += kTinyThreads) {
+        const float v = res[i] * inv * a.norm_f[i];
+        a.temporal[(int64_t)b * dm + i] = v;
+        if (a.host.out) a.host.out[(int64_t)b * dm + i] = v;
+    }
+    if (a.host.out) host_row_done(a.host, b);
 }
 
 size_t tiny_lds_bytes(const TinyStepArgs &a) {

@@ -257,6 +257,7 @@ class GpuMamba3Backbone:
         h = c_void_p()
         _call("mrs_m3_backbone_create", byref(h), gpu_ordinal, byref(cw), byref(cc), input_dim, batch, int(self.dtype))
         self._h = h
+        self._step = _lib.host_rows_call("mrs_m3_backbone_step")
 
     @classmethod
     def new(cls, gpu_ordinal, weights, cfg, input_dim, batch):
@@ -278,7 +279,9 @@ class GpuMamba3Backbone:
         if inp.size != self.batch * self.input_dim:
             raise ValueError(f"input must hold batch*input_dim = {self.batch * self.input_dim} values")
         out = np.empty((self.batch, self.cfg.d_model), np.float32)
-        _call("mrs_m3_backbone_step", self._h, _fp(inp), _fp(out))
+        rc = self._step(self._h, inp.ctypes.data, out.ctypes.data)
+        if rc != 0:
+            raise _lib.MambaHipError("mrs_m3_backbone_step", rc, _bind().mrs_last_error().decode())
         return out
 
     def step_gpu_only(self):
