@@ -1,5 +1,6 @@
 // Shared device/host helpers for libmamba_hip (gfx950 only).
 #pragma once
+#include <optional>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -205,6 +206,24 @@ bool resident_plan(ResidentArgs &a, int dtype);   // false: the shape is outside
 size_t resident_layer_bytes(const ResidentArgs &a);
 int launch_resident_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
 int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);   // dev: a copy of `a` on the device
+// The same for the Mamba-3 SISO backbone (resident_m3_step.hip); ex: columns of in_proj behind z and x that a workgroup owns.
+struct ResidentM3Layer {   // in_t [ip][d_model] and out_t [d_model][d_inner] transposed; next_nw: the norm weight after, or null
+    const void *in_t, *out_t; const float *bnw, *cnw, *b_bias, *c_bias, *D, *dt_bias, *next_nw;
+};
+struct ResidentM3Args {
+    const void *weights;
+    const float *input, *norm_w, *norm_f;
+    float *ssm, *kst, *vst, *angle, *temporal;
+    unsigned long long *xch;
+    unsigned *epoch, *broken;
+    size_t xch_stride;
+    float eps, a_floor;
+    int n_layers, batch, dm, di, nh, hd, ds, ng, nr, G, nc, oc, ex;
+};
+bool resident_m3_plan(ResidentM3Args &a, int dtype);
+size_t resident_m3_layer_bytes(const ResidentM3Args &a);
+int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, const ResidentM3Layer &w);
+int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev);
 // resident_gate.hip: whether this process's engines may take the resident route on a GPU (a claim counts the engine's
 // workgroups until it is released), and an engine's turn -- held while a step is launched.
 bool resident_claim(int device, int workgroups);
@@ -217,6 +236,11 @@ public:
     ResidentTurn &operator=(const ResidentTurn &) = delete;
 private:
     int device_;
+};
+// An engine's turn while a step is launched, where the step is a resident launch (device < 0: it is not).
+struct StepTurn {
+    std::optional<ResidentTurn> turn;
+    StepTurn(int device, hipStream_t st) { if (device >= 0) turn.emplace(device, st); }
 };
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,

@@ -25,7 +25,6 @@
 #include <new>
 #include <vector>
 #include <algorithm>
-#include <optional>
 
 namespace mrs {
 
@@ -866,12 +865,6 @@ static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
     if (!bb->step_src) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
     return run_layers(bb, &bb->step_s, 1);
 }
-
-// An engine's turn while a step is launched, where the step is a resident launch (device < 0: it is not).
-struct StepTurn {
-    std::optional<ResidentTurn> turn;
-    StepTurn(int device, hipStream_t st) { if (device >= 0) turn.emplace(device, st); }
-};
 
 extern "C" int mrs_backbone_step_gpu_only(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_step_gpu_only: null engine");

@@ -12,6 +12,7 @@
 //      registers, y = H q + D x, and the SiLU gate (optionally RMSNormGated over the head) -- the formulas of
 //      mamba3_layer_step (src/mamba3_siso/cpu/inference.rs:68-258) and kernels/mamba3_ops.cu;
 //   3. out_proj with the residual add, the next layer's pre-scaled operand and row sums of squares as epilogue.
+// At a few rows of a 16-bit model the whole step is one resident launch (resident_m3_step.hip).
 // Shapes the skinny GEMM does not take (f32 storage above four rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
 #include "common.hpp"
 #include "gemm_tune.hpp"
@@ -563,6 +564,9 @@ struct mrs_m3_backbone {
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
     HostIo io;              // step()'s rows in pinned host memory
+    int resident;                 // a few rows: the step as one resident launch (resident_m3_step.hip)
+    ResidentM3Args res_args, *res_args_dev;
+    unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
     TinyM3StepLayer *tiny_layers;   // small f32 models: the layer table of the single-launch step (null: kernel chains)
     std::vector<Layer3> layers;
     std::vector<void *> allocs;
@@ -633,9 +637,83 @@ int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
     return check_launch("m3_layer_step_kernel");
 }
 
+// The input rows in the residual stream: input . W + b.
+int project_input3(mrs_m3_backbone *bb) {
+    const int B = bb->batch, dm = bb->cfg.d_model;
+    const int64_t n = (int64_t)B * dm;
+    hipLaunchKernelGGL(bias_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->residual, bb->input_proj_b, n, dm);
+    const float one = 1.0f;
+    MRS_BLAS(rocblas_gemm_ex(bb->blas, rocblas_operation_none, rocblas_operation_none, dm, B, bb->input_dim, &one, bb->input_proj_w,
+                             rocblas_datatype_f32_r, dm, bb->d_input, rocblas_datatype_f32_r, bb->input_dim, &one, bb->residual,
+                             rocblas_datatype_f32_r, dm, bb->residual, rocblas_datatype_f32_r, dm, rocblas_datatype_f32_r,
+                             rocblas_gemm_algo_standard, 0, 0));
+    return MRS_OK;
+}
+
+// Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together: chosen before the weights are laid out
+// (the kernel chain's tiled copies are then not needed), set up behind them.
+void choose_resident3(mrs_m3_backbone *bb) {
+    const mrs_m3_config &c = bb->cfg;
+    const char *e = getenv("MRS_DECODE_NO_RESIDENT");
+    // (RMSNormGated sums over a head, whose channels lie in several workgroups: the kernel chain)
+    if ((e && atoi(e) != 0) || !bb->skinny || c.is_outproj_norm) return;
+    ResidentM3Args &a = bb->res_args;
+    a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
+    a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr;
+    if (bb->batch > 256 || !resident_m3_plan(a, bb->dtype) || !resident_claim(bb->device, a.G * a.batch)) return;
+    bb->resident = 1;
+    bb->tiled = 0;
+}
+
+int arm_resident3(mrs_m3_backbone *bb) {
+    const ResidentM3Args &a = bb->res_args;
+    MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.epoch, 0, (size_t)a.batch * 128, bb->stream));
+    *bb->res_broken = 0;
+    return MRS_OK;
+}
+
+int setup_resident3(mrs_m3_backbone *bb) {
+    if (!bb->resident) return MRS_OK;
+    const int L = bb->cfg.n_layers;
+    ResidentM3Args &a = bb->res_args;
+    a.input = bb->identity_proj ? bb->d_input : bb->residual;
+    a.norm_f = bb->norm_f; a.ssm = bb->ssm; a.kst = bb->kst; a.vst = bb->vst; a.angle = bb->angle; a.temporal = bb->temporal;
+    MRS_TRY(dev_alloc3(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
+    MRS_TRY(dev_alloc3(bb, (void **)&a.epoch, (size_t)a.batch * 128));
+    MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
+    a.broken = bb->res_broken;
+    MRS_TRY(arm_resident3(bb));
+    const size_t per_layer = resident_m3_layer_bytes(a);
+    char *w = nullptr;
+    MRS_TRY(dev_alloc3(bb, (void **)&w, per_layer * (size_t)L));
+    a.weights = w; a.norm_w = bb->layers[0].norm_w;
+    for (int l = 0; l < L; l++, w += per_layer) {
+        const Layer3 &d = bb->layers[l];
+        const ResidentM3Layer rl = {d.in_proj_t, d.out_proj_t, d.bnw, d.cnw, d.b_bias, d.c_bias, d.D, d.dt_bias,
+                                    l + 1 < L ? bb->layers[l + 1].norm_w : nullptr};
+        MRS_TRY(launch_resident_m3_pack(bb->stream, a, w, rl));
+    }
+    MRS_TRY(dev_alloc3(bb, (void **)&bb->res_args_dev, sizeof(ResidentM3Args)));
+    MRS_HIP(hipMemcpyAsync(bb->res_args_dev, &a, sizeof(ResidentM3Args), hipMemcpyHostToDevice, bb->stream));
+    return MRS_OK;
+}
+
+// After a synchronisation: whether every resident step found all its workgroups on the chip.
+int check_resident3(mrs_m3_backbone *bb) {
+    if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
+        return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
+                               "or set MRS_DECODE_NO_RESIDENT=1");
+    return MRS_OK;
+}
+
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
 int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
     const mrs_m3_config &c = bb->cfg;
+    if (bb->resident) {
+        if (!bb->identity_proj) MRS_TRY(project_input3(bb));
+        return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+    }
     if (bb->tiny_layers) {
         TinyM3StepArgs a = {};
         a.layers = bb->tiny_layers; a.input = bb->d_input;
@@ -656,13 +734,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
         if (bb->skinny) src = bb->d_input;   // the first prenorm kernel reads the input and writes the residual stream
         else MRS_HIP(hipMemcpyAsync(bb->residual, bb->d_input, (size_t)B * dm * 4, hipMemcpyDeviceToDevice, bb->stream));
     } else {
-        const int64_t n = (int64_t)B * dm;
-        hipLaunchKernelGGL(bias_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->residual, bb->input_proj_b, n, dm);
-        const float one = 1.0f;
-        MRS_BLAS(rocblas_gemm_ex(bb->blas, rocblas_operation_none, rocblas_operation_none, dm, B, bb->input_dim, &one, bb->input_proj_w,
-                                 rocblas_datatype_f32_r, dm, bb->d_input, rocblas_datatype_f32_r, bb->input_dim, &one, bb->residual,
-                                 rocblas_datatype_f32_r, dm, bb->residual, rocblas_datatype_f32_r, dm, rocblas_datatype_f32_r,
-                                 rocblas_gemm_algo_standard, 0, 0));
+        MRS_TRY(project_input3(bb));
     }
     for (int l = 0; l < L; l++) {
         const Layer3 &lw = bb->layers[l];
@@ -704,6 +776,10 @@ extern "C" int mrs_m3_backbone_reset(mrs_m3_backbone *bb) {
     MRS_HIP(hipMemsetAsync(bb->kst, 0, L * B * nh * ds * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->vst, 0, L * B * nh * hd * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->angle, 0, L * B * nh * na * 4, bb->stream));
+    if (check_resident3(bb)) {   // a resident step gave up: its exchange words start over with the state
+        MRS_HIP(hipStreamSynchronize(bb->stream));
+        return arm_resident3(bb);
+    }
     return MRS_OK;
 }
 
@@ -711,8 +787,10 @@ extern "C" void mrs_m3_backbone_destroy(mrs_m3_backbone *bb) {
     if (!bb) return;
     hipSetDevice(bb->device);
     if (bb->stream) hipStreamSynchronize(bb->stream);
+    if (bb->resident) resident_release(bb->device, bb->res_args.G * bb->res_args.batch, bb->stream);
     if (bb->graph_exec) hipGraphExecDestroy(bb->graph_exec);
     if (bb->graph) hipGraphDestroy(bb->graph);
+    if (bb->res_broken) hipHostFree(bb->res_broken);
     for (void *p : bb->allocs) hipFree(p);
     for (void *p : bb->pf_allocs) hipFree(p);
     host_io_destroy(&bb->io);
@@ -773,6 +851,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     // f32 storage: the row-wise route of the same GEMM, one to four rows
     if (dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 && getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
         bb->skinny = 1;
+    choose_resident3(bb);
     float *stage = nullptr;
     {
         size_t big = (size_t)dm * ip;
@@ -850,6 +929,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     MRS_CREATE_TRY(dev_alloc3(bb, &bb->gated, B16 * di * es));
     MRS_CREATE_TRY(dev_alloc3(bb, &bb->out, B * dm * es));
     MRS_CREATE_TRY(host_io_create(&bb->io, batch, input_dim, dm));
+    MRS_CREATE_TRY(setup_resident3(bb));
     MRS_CREATE_TRY(mrs_m3_backbone_reset(bb));
     { hipError_t e = hipStreamSynchronize(bb->stream);
       if (e != hipSuccess) { mrs_m3_backbone_destroy(bb); return fail(MRS_E_HIP, "create sync: %s", hipGetErrorString(e)); } }
@@ -860,8 +940,9 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
 
 extern "C" int mrs_m3_backbone_step_gpu_only(mrs_m3_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_step_gpu_only: null engine");
-    // (a step of one launch is launched quicker than a graph of one node)
-    if (bb->graph_ready && !bb->tiny_layers) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    const StepTurn turn(bb->resident ? bb->device : -1, bb->stream);
+    const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
+    if (bb->graph_ready && !one_launch) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
     return step_body3(bb);
 }
 
@@ -881,7 +962,7 @@ extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, flo
     }
     MRS_TRY(host_io_wait(&io, bb->stream));
     memcpy(output, io.out, (size_t)B * dm * 4);
-    return MRS_OK;
+    return check_resident3(bb);
 }
 
 // One eager warm step on a saved copy of the state (library handles pick their kernels), then capture the step body
@@ -897,7 +978,8 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     hipMemcpyAsync(save + n0, bb->kst, n1, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(save + n0 + n1, bb->vst, n2, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(save + n0 + n1 + n2, bb->angle, n3, hipMemcpyDeviceToDevice, bb->stream);
-    int rc = step_body3(bb);
+    int rc;
+    { const StepTurn turn(bb->resident ? bb->device : -1, bb->stream); rc = step_body3(bb); }
     hipMemcpyAsync(bb->ssm, save, n0, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->kst, save + n0, n1, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->vst, save + n0 + n1, n2, hipMemcpyDeviceToDevice, bb->stream);
@@ -1175,14 +1257,14 @@ extern "C" float *mrs_m3_backbone_temporal_ptr(mrs_m3_backbone *bb) { return bb 
 extern "C" int mrs_m3_backbone_temporal_dtype(mrs_m3_backbone *bb) { return bb ? MRS_F32 : -1; }
 extern "C" int mrs_m3_backbone_decode_route(mrs_m3_backbone *bb) {
     if (!bb) return -1;
-    return bb->tiny_layers ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
+    return bb->tiny_layers || bb->resident ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
 }
 extern "C" float *mrs_m3_backbone_input_ptr(mrs_m3_backbone *bb) { return bb ? bb->d_input : nullptr; }
 extern "C" void *mrs_m3_backbone_stream(mrs_m3_backbone *bb) { return bb ? (void *)bb->stream : nullptr; }
 extern "C" int mrs_m3_backbone_sync(mrs_m3_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_sync: null engine");
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident3(bb);
 }
 
 // Copies layer `layer`'s state to host buffers (any may be null): ssm [batch,nh,hd,ds], k [batch,nh,ds], v [batch,nh,hd],
@@ -1196,7 +1278,7 @@ extern "C" int mrs_m3_backbone_download_state(mrs_m3_backbone *bb, int layer, fl
     if (v) MRS_HIP(hipMemcpyAsync(v, bb->vst + l * B * nh * hd, B * nh * hd * 4, hipMemcpyDeviceToHost, bb->stream));
     if (angle) MRS_HIP(hipMemcpyAsync(angle, bb->angle + l * B * nh * na, B * nh * na * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident3(bb);
 }
 
 // ---- the Mamba-3 engine behind the LM loop (GpuMamba3LM, src/module/gpu_lm3.rs:54-400) ---------------------------
@@ -1205,6 +1287,7 @@ void m3_state_sizes(mrs_m3_backbone *bb, size_t (&n)[4]) {
     const size_t L = bb->cfg.n_layers, B = bb->batch, nh = bb->nh, hd = bb->cfg.headdim, ds = bb->cfg.d_state, na = bb->nr > 0 ? bb->nr : 1;
     n[0] = L * B * nh * hd * ds * 4; n[1] = L * B * nh * ds * 4; n[2] = L * B * nh * hd * 4; n[3] = L * B * nh * na * 4;
 }
+int m3_hook_check(void *self) { return check_resident3((mrs_m3_backbone *)self); }
 int m3_hook_step(void *self) { return step_body3((mrs_m3_backbone *)self); }
 int m3_hook_reset(void *self) { return mrs_m3_backbone_reset((mrs_m3_backbone *)self); }
 size_t m3_hook_state_bytes(void *self) {
@@ -1241,6 +1324,6 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = nullptr;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
-    h.prefill = m3_hook_prefill; h.resident_device = -1;
+    h.prefill = m3_hook_prefill; h.resident_device = bb->resident ? bb->device : -1; h.check = m3_hook_check;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");
 }

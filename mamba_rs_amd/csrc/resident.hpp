@@ -1,4 +1,4 @@
-// Building blocks of the resident decode steps (resident_step.hip): one launch walks the whole network, G workgroups
+// Building blocks of the resident decode steps (resident_step.hip, resident_m3_step.hip): one launch walks the whole network, G workgroups
 // share every layer's columns, and what a layer's phases need from each other travels through memory while the workgroups stay
 // on the chip.
 //
@@ -76,7 +76,10 @@ __device__ __forceinline__ float wave_sum_last(float v) {
     return v;
 }
 
-constexpr int kComputeWaves = 8;
+constexpr int kComputeWaves = 8, kCompute = 64 * kComputeWaves;
+constexpr int kResThreads = kCompute + 4 * 64;   // eight waves compute, four bring weights
+__host__ __device__ constexpr int up1k(int n) { return (n + 1023) & ~1023; }
+constexpr size_t kResLdsMax = 160 * 1024 - 256;
 
 // Two f32 in one exchange word: the lowest mantissa bit of each carries the parity of the layer's tag (a buffer's entries are
 // rewritten every layer, so what is not of this layer is of the one before).
@@ -151,6 +154,122 @@ __device__ __forceinline__ float row_sum(const float *out, int cols16, int c) {
 #pragma unroll
     for (int w = 0; w < kComputeWaves; w++) v += out[w * cols16 + c];
     return v;
+}
+
+// The waves that bring weights: wave 10 out_proj's, the others in_proj's, 11 the small block as well.  Each buffer is refilled as
+// soon as the phase that reads it is over and is there before the barrier in front of its next use; requests go out
+// where the computing waves wait for their neighbours (a wave that is still issuing them holds up a barrier).  A layer has five
+// barriers, behind: 1 in_proj, 2 the second exchange, 3 y, 4 out_proj, 5 the next operand.
+struct WeightFeed {
+    const char *blk;              // this workgroup's block of layer 0: in_proj part, out_proj part, small block, each of whole kilobytes
+    size_t next;                  // ... to that of the next layer
+    unsigned win, wout, small;    // LDS byte addresses; the small blocks of two layers lie one after the other
+    int out, small_at, small_bytes;   // offsets in the block
+};
+__device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, const int &bad) {
+    const char *blk = f.blk;
+    const bool out_wave = wave == 10, small_wave = wave == 11;
+    const int iw = wave == 11 ? 2 : wave - 8, in_pieces = f.out >> 10, in_mid = in_pieces / 2, out_pieces = (f.small_at - f.out) >> 10;
+    auto bring_in = [&](const char *p, int from, int to) { dma_to_lds(f.win, p, from + iw, to, 3); };
+    auto bring_out = [&](const char *p) { dma_to_lds(f.wout, p + f.out, 0, out_pieces, 1); };
+    auto bring_small = [&](const char *p, int l) { dma_to_lds(f.small + (l & 1) * f.small_bytes, p + f.small_at, 0, f.small_bytes >> 10, 1); };
+    if (out_wave) bring_out(blk);
+    else bring_in(blk, 0, in_pieces);
+    if (small_wave) bring_small(blk, 0);
+    if (!out_wave) dma_wait();
+    lds_barrier();   // layer 0's row is there
+#pragma unroll 1
+    for (int l = 0; l < nl; l++) {
+        const bool more = l + 1 < nl;
+        blk += f.next;   // the next layer's
+        lds_barrier();   // 1
+        if (small_wave && more) bring_small(blk, l + 1);
+        if (!out_wave && more) bring_in(blk, 0, in_mid);
+        if (out_wave) dma_wait();
+        lds_barrier();   // 2
+        if (bad) return;
+        if (!out_wave && more) bring_in(blk, in_mid, in_pieces);
+        lds_barrier();   // 3
+        if (bad) return;
+        if (!out_wave) dma_wait();
+        lds_barrier();   // 4
+        if (out_wave && more) bring_out(blk);
+        lds_barrier();   // 5
+        if (bad) return;
+    }
+}
+
+// The parts of a layer that both networks share.
+__device__ __forceinline__ float inv_rms(float s, int dm, float eps) {
+    float rms = sqrtf(s / (float)dm + eps);
+    if (!isfinite(rms) || rms < 1e-20f) rms = 1.0f;   // the reference's finite guard (kernels/norms.cu:58-61)
+    return 1.0f / rms;
+}
+
+// y of all channels (exchange 3) to LDS.
+template <typename T> __device__ __forceinline__ bool take_y(const u64 *e3, int di, unsigned tag, T *ys) {
+    bool ok = true;
+#pragma unroll 1
+    for (int i0 = 0; i0 < di >> 1; i0 += 2 * kCompute) {
+        const int t = i0 + here(threadIdx.x), n3 = di >> 1;
+        if (t < n3) {
+            u64 r[2];
+            ok = ok && xch_poll<2>(e3, [&](int u) { return (unsigned)(u == 1 && t + kCompute < n3 ? t + kCompute : t); },
+                                   [&](u64 w) { return (unsigned)(w >> 32) == tag; }, r);
+            *reinterpret_cast<unsigned *>(ys + 2 * t) = (unsigned)r[0];
+            if (t + kCompute < n3) *reinterpret_cast<unsigned *>(ys + 2 * (t + kCompute)) = (unsigned)r[1];
+        }
+    }
+    return ok;
+}
+
+// out_proj's columns join the residual stream (thread p holds columns o0 + 2 p and + 1); the next layer's operand (next_nw: its norm
+// weight for these columns, null behind the last layer) and the workgroup's sum of squares go out.
+template <typename T>
+__device__ __forceinline__ void put_operand(const float *pre2, int oc, int o0, int src, const float *next_nw, u64 *e1, u64 *e1s, unsigned tag, float &res0, float &res1) {
+    if (here(threadIdx.x) >= 16) return;
+    const int p = here(threadIdx.x);
+    float sq = 0.0f;
+    if (p < oc >> 1) {
+        const T a0 = (T)row_sum(pre2, 16, 2 * p), a1 = (T)row_sum(pre2, 16, 2 * p + 1);
+        res0 += Store<T>::ld(&a0); res1 += Store<T>::ld(&a1);
+        sq = fmaf(res0, res0, res1 * res1);
+        if (next_nw) {
+            const float2 nw = *reinterpret_cast<const float2 *>(next_nw + 2 * p);
+            xch_put_word(e1 + (unsigned)((o0 >> 1) + p), half_pair_word<T>((T)(res0 * nw.x), (T)(res1 * nw.y), tag));
+        }
+    }
+    sq = row16_sum(sq);
+    if (p == 0) xch_put(e1s + src, sq, tag);
+}
+
+// Exchange 1: the next operand row to xs (if there is one), the row's scale to *inv.
+template <typename T>
+__device__ __forceinline__ bool take_operand(const u64 *e1, const u64 *e1s, int G, int dm, float eps, unsigned tag, bool more, T *xs, float *inv) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const auto tagged = [&](u64 w) { return (unsigned)(w >> 32) == tag; };
+    bool ok = true;
+    if (wave == kComputeWaves - 1) {
+        // the workgroups' sums of squares: this wave, in workgroup order within a lane
+        float s = 0.0f;
+#pragma unroll 1
+        for (int g = here(lane); g < G; g += 64) {
+            u64 r[1];
+            ok = ok && xch_poll<1>(e1s, [&](int) { return (unsigned)g; }, tagged, r);
+            s += __uint_as_float((unsigned)r[0]);
+        }
+        s = wave_sum_last(s);
+        if (lane == 63) *inv = inv_rms(s, dm, eps);
+    }
+    if (more) {
+#pragma unroll 1
+        for (int t = here(threadIdx.x); t < dm >> 1; t += kCompute) {
+            u64 r[1];
+            ok = ok && xch_poll<1>(e1, [&](int) { return (unsigned)t; }, tagged, r);
+            *reinterpret_cast<unsigned *>(xs + 2 * t) = (unsigned)r[0];
+        }
+    }
+    return ok;
 }
 
 }  // namespace mrs

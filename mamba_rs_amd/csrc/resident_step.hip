@@ -22,12 +22,9 @@ namespace mrs {
 namespace {
 
 constexpr int kDs = 16, kDc = 4;           // states and conv taps of a channel
-constexpr int kResThreads = 12 * 64;       // eight waves compute, four bring weights
-constexpr int kCompute = 64 * kComputeWaves;
 constexpr int kMaxNc = 24, kMaxOc = 16, kMaxXd = 128, kMaxDr = 64;   // bounds of the fixed LDS areas
 constexpr int kInSteps = 4, kInTiles = 2 * kMaxNc / 16, kOutSteps = 8;      // k-steps of 32 per computing wave and 16-column tiles held in registers
 
-__host__ __device__ constexpr int up1k(int n) { return (n + 1023) & ~1023; }
 // What a workgroup needs of a layer besides the two big weights, as one block (byte offsets): x_proj rows [nc / 8][xd][8], dt weights
 // [nc][dr], A [nc][16], conv taps [nc][4], conv bias, D, dt bias [nc], the next layer's norm weight for its columns [oc].
 struct SmallBlock { int xw, dtw, aneg, cw, cb, D, dtb, nw, bytes; };
@@ -82,42 +79,10 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
     if (tid == 0) bad = 0;
 
     if (wave >= kComputeWaves) {
-        // ---- the waves that bring weights: wave 10 out_proj's, the others in_proj's, 11 the small block as well.  Each buffer is refilled as
-        // soon as the phase that reads it is over and is there before the barrier in front of its next use; requests go out
-        // where the computing waves wait for their neighbours (a wave that is still issuing them holds up a barrier).
-        const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         const LayerBlock lb = layer_block(dm, di, nc, oc, xd, dr);
-        const char *blk = (const char *)a->weights + (size_t)src * lb.bytes;   // this workgroup's block of layer 0
-        const size_t next = (size_t)G * lb.bytes;
-        const bool out_wave = wave == 10, small_wave = wave == 11;
-        const int iw = wave == 11 ? 2 : wave - 8, in_pieces = lb.out >> 10, in_mid = in_pieces / 2, out_pieces = (lb.small - lb.out) >> 10;
-        auto bring_in = [&](const char *p, int from, int to) { dma_to_lds(lds0 + L.win, p, from + iw, to, 3); };
-        auto bring_out = [&](const char *p) { dma_to_lds(lds0 + L.wout, p + lb.out, 0, out_pieces, 1); };
-        auto bring_small = [&](const char *p, int l) { dma_to_lds(lds0 + L.small + (l & 1) * sb.bytes, p + lb.small, 0, sb.bytes >> 10, 1); };
-        if (out_wave) bring_out(blk);
-        else bring_in(blk, 0, in_pieces);
-        if (small_wave) bring_small(blk, 0);
-        if (!out_wave) dma_wait();
-        lds_barrier();   // layer 0's row is there
-#pragma unroll 1
-        for (int l = 0; l < nl; l++) {
-            const bool more = l + 1 < nl;
-            blk += next;     // the next layer's
-            lds_barrier();   // 1: in_proj done
-            if (small_wave && more) bring_small(blk, l + 1);
-            if (!out_wave && more) bring_in(blk, 0, in_mid);
-            if (out_wave) dma_wait();
-            lds_barrier();   // 2: x_proj row there
-            if (bad) return;
-            if (!out_wave && more) bring_in(blk, in_mid, in_pieces);
-            lds_barrier();   // 3: y there, the scan step done
-            if (bad) return;
-            if (!out_wave) dma_wait();
-            lds_barrier();   // 4: out_proj done
-            if (out_wave && more) bring_out(blk);
-            lds_barrier();   // 5: operand row there
-            if (bad) return;
-        }
+        const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
+        bring_weights({(const char *)a->weights + (size_t)src * lb.bytes, (size_t)G * lb.bytes, lds0 + L.win, lds0 + L.wout, lds0 + L.small, lb.out, lb.small,
+                       sb.bytes}, wave, nl, bad);
         return;
     }
 
@@ -153,16 +118,11 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
     }
     ss = wave_sum_last(ss);
     if (lane == 63) pre2[wave] = ss;
-    auto inv_rms = [&](float s) {
-        float rms = sqrtf(s / (float)dm + a->eps);
-        if (!isfinite(rms) || rms < 1e-20f) rms = 1.0f;   // the reference's finite guard (kernels/norms.cu:58-61)
-        return 1.0f / rms;
-    };
     lds_barrier();
     float inv0 = 0.0f;   // layer 0's row scale; later ones come through LDS
 #pragma unroll
     for (int w = 0; w < kComputeWaves; w++) inv0 += pre2[w];
-    inv0 = inv_rms(inv0);
+    inv0 = inv_rms(inv0, dm, a->eps);
 
     RowProduct<T, kInSteps, kInTiles> pin;
     RowProduct<T, kOutSteps, 1> pout;
@@ -265,17 +225,7 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         }
         // ---- y of all channels
         pout.take(wout, oc, di >> 5, 1);   // while y is on its way
-        const auto tagged = [&](u64 w) { return (unsigned)(w >> 32) == tag; };
-#pragma unroll 1
-        for (int i0 = 0; i0 < di >> 1; i0 += 2 * kCompute) {
-            const int t = i0 + here(tid), n3 = di >> 1;
-            if (t < n3) {
-                u64 r[2];
-                ok = ok && xch_poll<2>(e3, [&](int u) { return (unsigned)(u == 1 && t + kCompute < n3 ? t + kCompute : t); }, tagged, r);
-                *reinterpret_cast<unsigned *>(ys + 2 * t) = (unsigned)r[0];
-                if (t + kCompute < n3) *reinterpret_cast<unsigned *>(ys + 2 * (t + kCompute)) = (unsigned)r[1];
-            }
-        }
+        ok = take_y(e3, di, tag, ys) && ok;
         if (!ok) bad = 1;
         if (more && conv_wave) cwin = ld_off<float4>(cst + (l + 1) * cst_l, (unsigned)min(here(lane), nc - 1) * 16u);
         lds_barrier();   // 3
@@ -283,42 +233,9 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         // ---- out_proj, residual, the next operand
         pout.run(ys, di >> 5, 1, pre2);
         lds_barrier();   // 4
-        if (here(tid) < 16) {
-            const int p = here(tid);
-            float sq = 0.0f;
-            if (p < oc >> 1) {
-                const T a0 = (T)row_sum(pre2, 16, 2 * p), a1 = (T)row_sum(pre2, 16, 2 * p + 1);
-                res0 += Store<T>::ld(&a0); res1 += Store<T>::ld(&a1);
-                sq = fmaf(res0, res0, res1 * res1);
-                if (more) {
-                    const float2 nw = *reinterpret_cast<const float2 *>(small + sb.nw + p * 8);
-                    xch_put_word(e1 + (unsigned)((o0 >> 1) + p), half_pair_word<T>((T)(res0 * nw.x), (T)(res1 * nw.y), tag));
-                }
-            }
-            sq = row16_sum(sq);
-            if (p == 0) xch_put(e1s + src, sq, tag);
-        }
+        put_operand<T>(pre2, oc, o0, src, more ? reinterpret_cast<const float *>(small + sb.nw) : nullptr, e1, e1s, tag, res0, res1);
         if (more) pin.take(win, 2 * nc, dm >> 5, ct_in);   // while the operand row is on its way
-        if (wave == kComputeWaves - 1) {
-            // the workgroups' sums of squares: this wave, in workgroup order within a lane
-            float s = 0.0f;
-#pragma unroll 1
-            for (int g = here(lane); g < G; g += 64) {
-                u64 r[1];
-                ok = ok && xch_poll<1>(e1s, [&](int) { return (unsigned)g; }, tagged, r);
-                s += __uint_as_float((unsigned)r[0]);
-            }
-            s = wave_sum_last(s);
-            if (lane == 63) invl[0] = inv_rms(s);
-        }
-        if (more) {
-#pragma unroll 1
-            for (int t = here(tid); t < dm >> 1; t += kCompute) {
-                u64 r[1];
-                ok = ok && xch_poll<1>(e1, [&](int) { return (unsigned)t; }, tagged, r);
-                *reinterpret_cast<unsigned *>(xs + 2 * t) = (unsigned)r[0];
-            }
-        }
+        ok = take_operand(e1, e1s, G, dm, a->eps, tag, more, xs, invl) && ok;
         if (!ok) bad = 1;
         lds_barrier();   // 5
         if (bad) break;
@@ -384,8 +301,6 @@ __global__ __launch_bounds__(256) void pack_layer_kernel(char *__restrict__ dst,
     *reinterpret_cast<uint4 *>(dst + (size_t)s * lb.bytes + at) = v;
 }
 
-constexpr size_t kLdsMax = 160 * 1024 - 256;
-
 }  // namespace
 
 static bool shape_ok(const ResidentArgs &a, int dtype) {
@@ -395,7 +310,7 @@ static bool shape_ok(const ResidentArgs &a, int dtype) {
 }
 static bool plan_ok(const ResidentArgs &a) {
     return a.nc >= 8 && a.nc % 8 == 0 && a.nc <= kMaxNc && a.nc * a.G == a.di && a.oc >= 2 && a.oc % 2 == 0 && a.oc <= kMaxOc && a.oc * a.G == a.dm &&
-           (size_t)res_lds(a.dm, a.di, a.nc, a.oc, a.xd, a.dr).total <= kLdsMax;
+           (size_t)res_lds(a.dm, a.di, a.nc, a.oc, a.xd, a.dr).total <= kResLdsMax;
 }
 
 // As few workgroups as the weights' buffers in LDS allow: an exchange among 64 takes 1.5 us, among 128 1.8 us, and the weights
@@ -425,7 +340,7 @@ int launch_resident_pack(hipStream_t st, const ResidentArgs &a, void *dst, const
 
 template <typename T>
 static int launch_resident_t(hipStream_t st, const ResidentArgs &a, const ResidentArgs *dev) {
-    static const hipError_t attr = hipFuncSetAttribute((const void *)resident_step_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)resident_step_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResLdsMax);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "resident step: LDS size: %s", hipGetErrorString(attr));
     hipLaunchKernelGGL((resident_step_kernel<T>), dim3((unsigned)(a.G * a.batch)), dim3(kResThreads), (size_t)res_lds(a.dm, a.di, a.nc, a.oc, a.xd, a.dr).total, st, dev);
     return check_launch("resident_step_kernel");
