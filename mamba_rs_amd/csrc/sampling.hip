@@ -21,6 +21,8 @@ constexpr int kListCap = 8192;   // bracket entries gathered into LDS
 constexpr int kMaxBlocks = 1024; // block totals of the index-ordered walk
 constexpr int kBinCopies = 32;   // copies of each histogram bin, one per lane modulo 32
 constexpr int kFinish = 512;     // a bracket this small is resolved by ranking its entries against each other
+constexpr int kGroups = kSampThreads / 4;   // the short route: maxima of the entries that four neighbouring threads walk
+constexpr int kShortK = 128;     // ... and the largest top-k it takes
 
 struct SampShared {
     double d_slots[kSampWaves][16];
@@ -36,6 +38,12 @@ struct SampShared {
     unsigned long long hist[16];
     unsigned long long res_ge, res_gt;
     uint32_t res_key;
+    alignas(16) uint32_t group_max[kGroups];
+    struct { float x; int i; } cand[kFinish];          // the short route's candidates, in no order
+    float kept_x[kShortK];                             // the top-k survivors in index order
+    int kept_i[kShortK];
+    uint32_t kept_key[kShortK];                        // bit patterns of their weights
+    unsigned long long kept_mass[kShortK];
 };
 
 template <typename T> __device__ __forceinline__ T wave_sum(T v) {
@@ -344,6 +352,128 @@ template <typename W> __device__ int ordered_find(const Row &row, W w, double ta
     return r;
 }
 
+// The k entries that top-k keeps (largest values, among equal ones the lowest indices), in index order in sh.kept_x / kept_i, for
+// k <= kShortK; false if the row's shape does not allow it (the caller then searches).  group_key: the largest ordered key among the
+// entries this thread walks in Row::each.
+//
+// The k-th largest of the kGroups group maxima is a value that at least k entries reach, and few more do (-kGroups ln(1 - k /
+// kGroups) if the large values lie anywhere: 56 for k = 50, 177 for k = 128), so one more pass over the row collects every
+// entry that can matter and all that follows walks a list of that length.  It does not fit for rows whose large values crowd
+// into few groups (an ascending vocabulary) or with long runs of equal values.
+// Row passes are what a draw costs (about 7 us each at 50280 entries, one workgroup per row): eight with both filters through the
+// searches, two through here.
+__device__ bool short_top_k(const Row &row, uint32_t group_key, int k, SampShared &sh) {
+    const int tid = threadIdx.x;
+    group_key = max(group_key, (uint32_t)__shfl_xor((int)group_key, 1, kWave));
+    group_key = max(group_key, (uint32_t)__shfl_xor((int)group_key, 2, kWave));
+    if ((tid & 3) == 0) sh.group_max[tid >> 2] = group_key;
+    if (tid == 0) sh.n_list = 0;
+    __syncthreads();
+    if (tid < kGroups) {
+        const uint32_t mine = sh.group_max[tid];
+        int rank = 0;
+#pragma unroll 8
+        for (int u = 0; u < kGroups; u += 4) {
+            const uint4 o = *reinterpret_cast<const uint4 *>(&sh.group_max[u]);
+            rank += (o.x > mine || (o.x == mine && u < tid)) + (o.y > mine || (o.y == mine && u + 1 < tid)) +
+                    (o.z > mine || (o.z == mine && u + 2 < tid)) + (o.w > mine || (o.w == mine && u + 3 < tid));
+        }
+        if (rank == k - 1) sh.res_key = mine;
+    }
+    __syncthreads();
+    const uint32_t floor_key = sh.res_key;
+    row.each([&](int i, float x) {
+        if (ordered_key(x) >= floor_key) {
+            const int slot = atomicAdd(&sh.n_list, 1);
+            if (slot < kFinish) { sh.cand[slot].x = x; sh.cand[slot].i = i; }
+        }
+    });
+    __syncthreads();
+    const int n = sh.n_list;
+    if (n < k || n > kFinish) return false;   // (uniform)
+    bool keep = false;
+    uint32_t key = 0;
+    int idx = 0;
+    if (tid < n) {
+        key = ordered_key(sh.cand[tid].x);
+        idx = sh.cand[tid].i;
+        int rank = 0;
+        for (int u = 0; u < n; u++) {
+            const uint32_t ku = ordered_key(sh.cand[u].x);
+            rank += ku > key || (ku == key && sh.cand[u].i < idx);
+        }
+        keep = rank < k;
+        sh.list[tid] = keep ? (uint32_t)idx : 0xffffffffu;
+    }
+    __syncthreads();
+    if (keep) {
+        int pos = 0;
+        for (int u = 0; u < n; u++) pos += sh.list[u] < (uint32_t)idx;
+        sh.kept_x[pos] = sh.cand[tid].x;
+        sh.kept_i[pos] = idx;
+    }
+    __syncthreads();
+    return true;
+}
+
+// Softmax, top-p, min-p and the draw over the m <= kShortK survivors that short_top_k left, by the rules of the general route below: the
+// same integer masses, the running sums in f64.
+__device__ int short_draw(int m, int vocab, float xmax, const mrs_sampler &sp, bool topp_on, SampShared &sh) {
+    const int tid = threadIdx.x;
+    float e = 0.0f;
+    uint32_t key = 0;
+    if (tid < m) {
+        e = __expf(sh.kept_x[tid] - xmax);
+        key = __float_as_uint(e);
+        sh.kept_key[tid] = key;
+        sh.kept_mass[tid] = fixed_weight(key);
+    }
+    __syncthreads();
+    if (tid < m && topp_on) {
+        unsigned long long total = 0, above = 0, equal = 0;
+        int ties_before = 0;
+        for (int u = 0; u < m; u++) {
+            const uint32_t ku = sh.kept_key[u];
+            const unsigned long long c = sh.kept_mass[u];
+            total += c;
+            above += ku > key ? c : 0ull;
+            equal += ku == key ? c : 0ull;
+            ties_before += ku == key && u < tid;
+        }
+        const unsigned long long thr = (unsigned long long)((double)sp.top_p * (double)total);
+        // an entry goes if what lies above it crosses the goal already, or its equals of lower index take the sum across
+        if (key == 0u || above > thr) e = 0.0f;
+        else if (above + equal > thr) {
+            const unsigned long long v = fixed_weight(key);
+            if (v != 0 && (unsigned long long)ties_before >= (thr - above) / v + 1ull) e = 0.0f;
+        }
+    }
+    if (sp.min_p > 0.0f && e < sp.min_p) e = 0.0f;
+    __syncthreads();
+    if (tid < m) sh.kept_x[tid] = e;
+    __syncthreads();
+    if (tid < kWave) {
+        const double w0 = 2 * tid < m ? (double)sh.kept_x[2 * tid] : 0.0, w1 = 2 * tid + 1 < m ? (double)sh.kept_x[2 * tid + 1] : 0.0;
+        double inc = w0 + w1;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const double t = __shfl_up(inc, d, kWave);
+            if (tid >= d) inc += t;
+        }
+        const double target = (double)sh.draw * __shfl(inc, kWave - 1, kWave);
+        const unsigned long long hit = __ballot(inc > target);
+        int tok = vocab - 1;   // (no weight at all: the general route's fall-through)
+        if (hit) {
+            const int src = (int)__ffsll((long long)hit) - 1;
+            const bool first = inc - w1 > target;
+            tok = __shfl(first ? sh.kept_i[min(2 * tid, m - 1)] : sh.kept_i[min(2 * tid + 1, m - 1)], src, kWave);
+        }
+        if (tid == 0) sh.found = tok;
+    }
+    __syncthreads();
+    return sh.found;
+}
+
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
 
 // logits [rows, ld] f32 are read only; `work` [rows, ld] receives the penalised logits of rows with a penalty.  seen [rows, vocab] counts how often a token sits in the row's seen list (the penalty is applied once per
@@ -371,6 +501,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
     Row row{lrow, vocab, vec, 1.0f};
     float best = -INFINITY;
     int bi = 0;
+    uint32_t top_key = 0;   // the largest ordered key this thread meets
     if (pen_on) {   // the penalised (and scaled) row goes to `work`; later passes read it from there
         float *wrow = work + (int64_t)rowi * ld;
         const unsigned *srow = seen + (int64_t)rowi * vocab;
@@ -379,6 +510,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
             x *= inv_t;
             wrow[i] = x;
             if (x >= best) { best = x; bi = i; }   // a thread meets its entries in ascending index order
+            top_key = max(top_key, ordered_key(x));
         });
         row.x = wrow;
         __syncthreads();   // the row is read back by other threads below (same workgroup, global memory)
@@ -386,6 +518,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
         row.scale = inv_t;   // temperature alone is applied on every read
         row.each([&](int i, float x) {
             if (x >= best) { best = x; bi = i; }
+            top_key = max(top_key, ordered_key(x));
         });
     }
 #pragma unroll
@@ -408,8 +541,29 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
     }
     const float xmax = best;
 
+    // the draw: one xoshiro256++ output per sampled token, mapped to [0, 1) by its top 24 bits
+    if (tid == 0) {
+        unsigned long long *s = rng + (int64_t)rowi * 4;
+        uint64_t s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
+        const uint64_t result = rotl64(s0 + s3, 23) + s0;
+        const uint64_t t = s1 << 17;
+        s2 ^= s0; s3 ^= s1; s1 ^= s2; s0 ^= s3; s2 ^= t; s3 = rotl64(s3, 45);
+        s[0] = s0; s[1] = s1; s[2] = s2; s[3] = s3;
+        sh.draw = (float)(result >> 40) / 16777216.0f;
+    }
+
     // top-k: key of the k-th largest value, then how many entries equal to it stay (lowest indices first)
     const bool topk_on = sp.top_k > 0 && sp.top_k < vocab;
+    const bool topp_on = isfinite(sp.top_p) && sp.top_p > 0.0f && sp.top_p < 1.0f;
+    if (topk_on && sp.top_k <= kShortK) {
+        __syncthreads();   // sh.draw
+        if (short_top_k(row, top_key, sp.top_k, sh)) {
+            const int tok = short_draw(sp.top_k, vocab, xmax, sp, topp_on, sh);
+            if (tid == 0) tokens[rowi] = tok;
+            return;
+        }
+        __syncthreads();
+    }
     uint32_t kkey = 0;       // keep_k(i) = key > kkey, or key == kkey and i <= k_tie_last
     int k_tie_last = vocab;
     if (topk_on) {
@@ -431,7 +585,6 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
 
     // top-p: the largest weight value v whose mass of entries >= v still exceeds p * Z; entries above v stay, and as
     // many entries equal to v as it takes to cross p (sample.rs:170-204 on the descending order)
-    const bool topp_on = isfinite(sp.top_p) && sp.top_p > 0.0f && sp.top_p < 1.0f;
     uint32_t pkey = 0;
     int p_tie_last = vocab;
     if (topp_on) {
@@ -462,18 +615,8 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
         return e;
     };
 
-    // the draw: one xoshiro256++ output per sampled token, mapped to [0, 1) by its top 24 bits
-    if (tid == 0) {
-        unsigned long long *s = rng + (int64_t)rowi * 4;
-        uint64_t s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
-        const uint64_t result = rotl64(s0 + s3, 23) + s0;
-        const uint64_t t = s1 << 17;
-        s2 ^= s0; s3 ^= s1; s1 ^= s2; s0 ^= s3; s2 ^= t; s3 = rotl64(s3, 45);
-        s[0] = s0; s[1] = s1; s[2] = s2; s[3] = s3;
-        sh.draw = (float)(result >> 40) / 16777216.0f;
-    }
-    __syncthreads();
     // first index whose running sum of kept weights exceeds draw x (their total)
+    __syncthreads();   // sh.draw
     const int tok = ordered_find(row, final_weight, (double)sh.draw, true, sh);
     if (tid == 0) tokens[rowi] = tok;
 }

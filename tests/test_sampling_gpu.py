@@ -108,6 +108,35 @@ def test_many_draws_stay_inside_the_filtered_support_and_follow_the_distribution
     assert np.abs(freq - probs[support]).max() < 0.05
 
 
+@pytest.mark.parametrize("shape", ["spread", "ascending", "tied", "short", "crowded"])
+def test_top_k_by_group_maxima_keeps_what_the_search_keeps(shape):
+    """top-k up to 128 collects its candidates above a floor taken from the maxima of 256 groups of the row; 129 always searches.
+    Rows it was made for (spread), whose large values sit in few groups (ascending: more candidates than the list holds, so it
+    searches after all; crowded: in one thread's entries), with thousands of equal values across the k-th place (tied) and with
+    fewer entries than groups (short), against the oracle; k = 1, the largest k it takes, and one more."""
+    rng = np.random.default_rng(7)
+    vocab = {"short": 131, "ascending": 50280, "tied": 6000, "crowded": 20000, "spread": 50280}[shape]
+    row = (rng.standard_normal(vocab) * 2).astype(np.float32)
+    if shape == "ascending":
+        row = np.sort(row)
+    if shape == "tied":
+        row = np.round(row)
+    if shape == "crowded":
+        row[4096:4100] += 20.0
+        row[8192:8196] += 20.0
+    params = [SampleParams(temperature=t, top_k=k, top_p=p, min_p=m) for t, p, m in ((1.0, 1.0, 0.0), (0.7, 0.9, 0.0), (1.5, 0.95, 0.05))
+              for k in (1, 2, 50, 127, 128, 129)]
+    seeds = [31 + r for r in range(len(params))]
+    print(f"case short top-k {shape}", flush=True)
+    tok, state = device_sample(np.tile(row, (len(params), 1)), params, seeds)
+    near = 0
+    for r, p in enumerate(params):
+        d, want_state = check_row(int(tok[r]), row, p, seeds[r])
+        near += d
+        assert [int(v) for v in state[r]] == want_state, r
+    assert near <= 1
+
+
 def test_ties_keep_the_lower_index_and_greedy_keeps_the_last_maximum():
     vocab = 4096
     rng = np.random.default_rng(2)
