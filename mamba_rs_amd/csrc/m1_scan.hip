@@ -11,6 +11,7 @@
 // segment; the state h[n] of a channel lives in that lane's registers for the
 // whole sequence and is written back once.
 #include "common.hpp"
+#include <algorithm>
 #include <stdlib.h>
 #include <mutex>
 
@@ -226,11 +227,12 @@ constexpr int kSpan = 2 * kGroup;    // steps per loop iteration and per staged 
 // keeps the vector ALU issuing -- and fill the 1024 SIMDs of the chip evenly: a SIMD with one wave more than the others
 // sets the time of the launch (4 x 4096 x 5120: 9 chunks = 2880 waves 375 us, 10 chunks = 3200 waves 404 us).
 constexpr int kSimds = 1024;   // 256 compute units x 4
+constexpr int kMaxChunks = 32;
 static SplitPlan make_split_plan(int batch, int Tlen, int di) {
     const int tiles = (di + kWave - 1) / kWave;
     const int64_t base = (int64_t)batch * tiles;
     static const int target = [] { const char *e = getenv("MRS_SCAN_TARGET_WAVES"); return e ? atoi(e) : 0; }();
-    int cmax = 32;                               // the entering-state fold is O(C) per wave
+    int cmax = kMaxChunks;                       // the entering-state fold is O(C) per wave
     if (cmax > Tlen / 32) cmax = Tlen / 32;      // chunks of at least 32 steps
     int c;
     if (target > 0) {
@@ -255,6 +257,14 @@ static SplitPlan make_split_plan(int batch, int Tlen, int di) {
     if (c < 1) c = 1;
     int len = (Tlen + c - 1) / c;
     len = (len + kSpan - 1) / kSpan * kSpan;
+    // Held back by the chunk limit the chip is less than full, and the rounding to whole spans should not empty it further (777 steps:
+    // 24 chunks become 17 of 48 steps): the shortest chunk the limits allow.  A layer of a 1 x 777 prompt at d_inner 2048 takes
+    // 99.7 us with 17 chunks, 93.3 with 25; of 1 x 300 78.7 / 72.4, of 1 x 200 at d_inner 1536 75.9 / 70.5.  (Chunks of one span do
+    // no better: the fold over the chunks before grows as the chunks shrink.)
+    if (c == cmax) {
+        const int shortest = std::max(2 * kSpan, ((Tlen + kMaxChunks - 1) / kMaxChunks + kSpan - 1) / kSpan * kSpan);
+        if (shortest < len && (Tlen + shortest - 1) / shortest * base <= 2 * kSimds) len = shortest;
+    }
     c = (Tlen + len - 1) / len;
     return {c, len};
 }
@@ -268,8 +278,6 @@ struct SplitWs {
     float *sumd;    // [B][C-1][di]
     size_t floats;  // whole workspace, in 4-byte words
 };
-
-constexpr int kMaxChunks = 32;
 
 // The flag area comes first and has one size whatever the shape of the call, so that a buffer shared by calls of
 // different shapes (the library's static one, an engine's scratch) never has one call's summaries where another call's
