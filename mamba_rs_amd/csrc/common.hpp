@@ -125,6 +125,7 @@ struct SkinnyEpi {
     // x_proj of a wide model is 12 tiles over K = 5120)
     int ksplit;
     int kslice;          // set by the launcher: 32-wide k-steps per slice
+    int any_rows;        // mode 0, 16-bit storage: no limit on M
     // tiled route (gemm_wide.hip) and matrix-core route of gemm_skinny.hip: A is stored [k-step][row tile][lane][8] -- the matrix-core operand in lane order, 16-row
     // tiles (tiled_a_index), rows past M present with any contents -- instead of row-major
     int a_tiled;

@@ -496,6 +496,13 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
     return MRS_OK;
 }
 
+// x_proj of a prefill of few rows: its result is a few dozen columns, so the vendor kernel has a workgroup or two per 96 rows (17.8 us at 777 x 96
+// x 2048); the 16 x 16-tile GEMM splits K over its waves and fills the chip (about 7 us), and a launch of it costs the host a
+// fraction of a library call.  Its operand re-reads grow with the tiles: up to two workgroups per compute unit it is ahead
+// (a layer, vendor / own: 64 rows at d_inner 1536 86 / 73 us, 500 rows 86 / 84, 1500 rows 96.5 / 95.3, 2048 rows 111 / 114; at
+// d_inner 5120 300 rows 174 / 168, 1024 rows 241 / 246).
+static bool own_xproj(const LayerDev &lw, int64_t rows, int xd) { return lw.x_proj_p && (rows + 15) / 16 * ((xd + 15) / 16) <= 2 * 256; }
+
 static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
     const int dm = bb->cfg.d_model, di = bb->di, ds = bb->cfg.d_state, dc = bb->cfg.d_conv, dr = bb->dr, xd = bb->xd;
     const int B = bb->batch, dt = bb->dtype;
@@ -542,7 +549,13 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
             }
         } else {
             MRS_TRY(mrs_conv1d_seq_silu(bb->stream, dt, s->u, conv, s->proj, 2 * di, lw.conv_w, lw.conv_b, B, T, di, dc));
-            MRS_TRY(gemm_rm(bb, dt, s->xdbl, xd, s->u, di, lw.x_proj, (int)rows, xd, di));
+            if (own_xproj(lw, rows, xd)) {
+                SkinnyEpi xp = {};
+                xp.w_tiled = 1; xp.any_rows = 1;
+                MRS_TRY(launch_skinny_gemm(bb->stream, dt, s->xdbl, 0, xd, s->u, di, lw.x_proj_p, (int)rows, xd, di, xp));
+            } else {
+                MRS_TRY(gemm_rm(bb, dt, s->xdbl, xd, s->u, di, lw.x_proj, (int)rows, xd, di));
+            }
             if (lw.dt_w_t && dt_proj_softplus_ok(dt, di, dr, xd, s->delta, s->xdbl, lw.dt_w_t)) {
                 // dt_proj + bias + softplus in one matrix-core kernel (K = dt_rank is tiny: the op is one write of delta)
                 MRS_TRY(launch_dt_proj_softplus(bb->stream, dt, s->delta, s->xdbl, xd, lw.dt_w_t, lw.dt_b, rows, di, dr));
@@ -761,10 +774,11 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
             MRS_CREATE_TRY(launch_tile_weight(bb->stream, bb->dtype, d.in_proj_p, d.in_proj_t, 2 * di, dm));
             MRS_CREATE_TRY(launch_tile_weight(bb->stream, bb->dtype, d.out_proj_p, d.out_proj_t, dm, di));
         }
-        if ((bb->skinny && !bb->resident) || bb->split_xproj) {
+        const bool tile_xproj = bb->dtype != MRS_F32 && di % 32 == 0;   // decode on tiled operands; prefill of few rows
+        if (bb->skinny || tile_xproj) {
             MRS_CREATE_TRY(dev_alloc(bb, &d.x_proj_t, (size_t)di * xd * esize(bb->dtype)));
             MRS_CREATE_TRY(launch_transpose(bb->stream, bb->dtype, d.x_proj_t, d.x_proj, di, xd));
-            if (bb->tiled || bb->split_xproj) {
+            if (tile_xproj) {
                 MRS_CREATE_TRY(dev_alloc(bb, &d.x_proj_p, tiled_weight_elems(xd, di) * esize(bb->dtype)));
                 MRS_CREATE_TRY(launch_tile_weight(bb->stream, bb->dtype, d.x_proj_p, d.x_proj_t, xd, di));
             }

@@ -603,7 +603,8 @@ bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, 
 
 int launch_skinny_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wt,
                        int M, int N, int K, const SkinnyEpi &ep) {
-    if (!skinny_gemm_ok(dtype, M, N, K, lda, A, Wt))
+    const int row_check = ep.any_rows && ep.mode == 0 && dtype != MRS_F32 ? std::min(M, 1) : M;
+    if (!skinny_gemm_ok(dtype, row_check, N, K, lda, A, Wt))
         return fail(MRS_E_SHAPE, "skinny gemm: needs 16-bit storage with 1 <= M <= 128, K %% 32 == 0, lda %% 8 == 0, or f32 storage with M <= 4, "
                                  "K %% 128 == 0, lda %% 4 == 0; 16-byte aligned A and Wt (got dtype=%d M=%d N=%d K=%d lda=%lld)", dtype, M, N, K,
                     (long long)lda);
