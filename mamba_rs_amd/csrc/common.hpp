@@ -145,6 +145,10 @@ size_t tiled_weight_elems(int N, int K);
 int launch_tile_weight(hipStream_t st, int dtype, void *Wp, const void *Wt, int N, int K);
 int launch_tiled_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wp, int M,
                       int N, int K, const SkinnyEpi &ep);
+// C[M,N] = A[M,K] . Wt[N,K]^T for a prefill of some hundred rows (gemm_mid.hip), 16-bit storage, C in the storage type or f32
+bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
+bool mid_gemm_wins(int64_t M, int N, int K);
+int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 int skinny_max_rows();   // rows the 16-bit matrix-core route takes (128; MRS_SKINNY_MAX_ROWS overrides)
 bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, const void *Wt);
 int launch_skinny_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wt,

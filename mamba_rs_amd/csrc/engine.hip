@@ -377,6 +377,13 @@ static int gemm_rm_t(mrs_backbone *bb, int dtype, void *C, int ldc, const void *
     return gemm_ex_tuned(bb->tuner, bb->blas, bb->stream, 1, N, M, K, Wt, t, K, A, t, lda, C, t, ldc);
 }
 
+// in_proj and out_proj of a prefill: the own kernel where the rows are few, else the library
+static int prefill_projection(mrs_backbone *bb, int dtype, void *C, int ldc, const void *A, int lda, const void *W, const void *Wt, int M, int N, int K) {
+    if (Wt && mid_gemm_wins(M, N, K) && mid_gemm_ok(dtype, 0, C, ldc, A, lda, Wt, M, N, K))
+        return launch_mid_gemm(bb->stream, dtype, 0, C, ldc, A, lda, Wt, M, N, K);
+    return Wt ? gemm_rm_t(bb, dtype, C, ldc, A, lda, Wt, M, N, K) : gemm_rm(bb, dtype, C, ldc, A, lda, W, M, N, K);
+}
+
 static int launch_add_rmsnorm(mrs_backbone *bb, float *residual, const void *add, void *out, bool out_f32, const float *w,
                               int64_t rows, int64_t out_stride, void *out2 = nullptr) {
     return launch_add_rmsnorm_any(bb->stream, bb->dtype, residual, add, out, out_f32, out2, w, bb->cfg.rms_norm_eps, rows, bb->cfg.d_model,
@@ -517,7 +524,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
         const char *z = (const char *)s->proj + (size_t)di * es;  // gate half of in_proj's output
         const char *xb = (const char *)s->xdbl;
         MRS_TRY(launch_add_rmsnorm(bb, s->residual, l == 0 ? nullptr : s->out, s->normed, false, lw.norm_w, rows, dm));
-        if (lw.in_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj_t, (int)rows, 2 * di, dm));
+        if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, 2 * di, dm));
+        else if (lw.in_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj_t, (int)rows, 2 * di, dm));
         else MRS_TRY(gemm_rm(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, (int)rows, 2 * di, dm));
         if (T == 1) {
             MRS_TRY(launch_conv1d_step(bb->stream, dt, s->u, conv, s->proj, 2 * di, lw.conv_w, lw.conv_b, B, di, dc, 1));
@@ -579,7 +587,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
             MRS_TRY(mrs_ssm_scan_fwd_ex(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg,
                                         lw.D, z, 2 * di, flags, s->scan_ws, s->scan_ws_bytes, B, T, di, ds));
         }
-        if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
+        if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
+        else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));
     }
     if (T == 1) {

@@ -1107,6 +1107,11 @@ int launch_add_rmsnorm3(mrs_m3_backbone *bb, float *residual, const void *add, v
                                   bb->cfg.d_model);
 }
 
+// A projection of a prefill (dense rows, weight as the transposed copy) on the own kernel instead of the library's
+bool own_projection(int dt, int out_f32, const void *C, int ldc, const void *A, const void *Wt, int64_t rows, int N, int K) {
+    return Wt && mid_gemm_wins(rows, N, K) && mid_gemm_ok(dt, out_f32, C, ldc, A, K, Wt, rows, N, K);
+}
+
 int prefill_body3(mrs_m3_backbone *bb, int T) {
     const mrs_m3_config &c = bb->cfg;
     const int dm = c.d_model, di = bb->di, B = bb->batch, dt = bb->dtype, L = c.n_layers, ip = bb->ip, nh = bb->nh, hd = c.headdim, ds = c.d_state;
@@ -1149,8 +1154,13 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             } else {
                 // the vendor kernels for the transposed operand are faster at these shapes (the copy's first nb rows, then the rest)
                 if (lw.in_proj_t) {
-                    MRS_TRY(gemm(1, nb, lw.in_proj_t, dm, bb->pf_bulk, t, nb));
-                    MRS_TRY(gemm(1, ns, (const char *)lw.in_proj_t + (size_t)nb * dm * es, dm, bb->pf_proj, f32t, ns));
+                    const char *wt = (const char *)lw.in_proj_t, *wt_rest = wt + (size_t)nb * dm * es;
+                    if (own_projection(dt, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm))
+                        MRS_TRY(launch_mid_gemm(bb->stream, dt, 0, bb->pf_bulk, nb, bb->pf_normed, dm, wt, rows, nb, dm));
+                    else MRS_TRY(gemm(1, nb, wt, dm, bb->pf_bulk, t, nb));
+                    if (own_projection(dt, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm))
+                        MRS_TRY(launch_mid_gemm(bb->stream, dt, 1, bb->pf_proj, ns, bb->pf_normed, dm, wt_rest, rows, ns, dm));
+                    else MRS_TRY(gemm(1, ns, wt_rest, dm, bb->pf_proj, f32t, ns));
                 } else {
                     MRS_TRY(gemm(0, nb, lw.in_proj, ip, bb->pf_bulk, t, nb));
                     MRS_TRY(gemm(0, ns, (const char *)lw.in_proj + (size_t)nb * es, ip, bb->pf_proj, f32t, ns));
@@ -1212,7 +1222,9 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             MRS_TRY(mrs_m3_seq_fwd(bb->stream, dt, ssm, kst, vst, bb->pf_y, bb->pf_x, bb->pf_K, bb->pf_Q, al, be, ga, lw.D, B, T, nh, hd, ds));
         }
         if (!gate_in_scan) MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_gate_t<T_>(bb, lw, rows, bulk, ldb)));
-        MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));
+        if (own_projection(dt, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
+            MRS_TRY(launch_mid_gemm(bb->stream, dt, 0, bb->pf_out, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di));
+        else MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));
     }
     // only the last position of each sequence is kept: final residual add + norm_f on those rows
     for (int b = 0; b < B; b++) {

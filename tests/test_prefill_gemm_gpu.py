@@ -1,0 +1,44 @@
+"""GPU: the prefill projections of few rows (the 64 x 64-tile kernel, and x_proj on the decode chain's 16 x 16 tiles) through one
+layer of the engine, against the CPU route on storage-rounded weights."""
+import numpy as np
+import pytest
+
+import orc
+from util import cosine, scaled_err
+from test_engine_gpu import oracle_params
+
+pytestmark = pytest.mark.gpu
+
+from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
+
+
+@pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
+@pytest.mark.parametrize("dm,B,T", [
+    (64, 1, 2),      # one k-step of in_proj, two of out_proj: fewer than the buffers; two rows of a tile
+    (64, 1, 63),     # a row tile short of its last row
+    (64, 2, 32),     # a whole row tile
+    (128, 1, 65),    # one row past it
+    (192, 3, 43),    # three, then six k-steps; 129 rows: the third row tile holds one
+    (320, 1, 200),   # five k-steps and ten: one more than the buffers; workgroups not a multiple of eight
+    (96, 1, 70),     # K not a multiple of the k-step: in_proj (96) stays with the library, out_proj (192) does not
+])
+def test_prefill_of_few_rows_follows_the_cpu_route(dm, B, T, dtype):
+    """Every sequence's last row and the states behind it.  16-bit storage: cosine >= 0.999 per row as for the decode chains, and 5e-2 of
+    the largest element -- a tile row or column gone wrong shows in the states, which hold every channel's history."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 5)
+    P = oracle_params(w, cfg, dm, round_to=orc.BF16 if dtype == WeightDtype.BF16 else orc.F16)
+    x = (np.random.default_rng(dm + T).standard_normal((B, T, dm)) * 0.5).astype(np.float32)
+    print(f"case prefill projections d_model={dm} rows={B * T} {dtype.name}", flush=True)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    last = eng.prefill_sequence(x)
+    conv, ssm = eng.download_state(0)
+    eng.close()
+    di = cfg.d_inner()
+    for b in range(B):
+        c, s = orc.m1_zero_state(P)
+        want = orc.m1_backbone_prefill(P, x[b], c, s)[-1]
+        assert cosine(last[b], want) >= 0.999 and scaled_err(last[b], want) < 5e-2, (b, cosine(last[b], want), scaled_err(last[b], want))
+        hs, cs = s[0].reshape(di, 16), c[0].reshape(di, 3)
+        assert cosine(ssm[b], hs) >= 0.999 and scaled_err(ssm[b], hs) < 5e-2, (b, cosine(ssm[b], hs), scaled_err(ssm[b], hs))
+        assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
