@@ -11,6 +11,7 @@
 // segment; the state h[n] of a channel lives in that lane's registers for the
 // whole sequence and is written back once.
 #include "common.hpp"
+#include "scan_quad.hpp"
 #include <algorithm>
 #include <stdlib.h>
 #include <mutex>
@@ -966,6 +967,16 @@ extern "C" size_t mrs_ssm_scan_workspace_bytes(int batch, int T, int d_inner, in
     return (bytes + 255) & ~(size_t)255;
 }
 
+// Four lanes per channel (m1_scan_quad.hip) instead of one: ahead while the chip is not full of waves.  Two launches of either kernel, bf16, gated,
+// one lane / four: general A 1 x 200 x 1536 19.8 / 11.2 us, 1 x 777 x 2048 27.1 / 23.6, 1 x 2048 x 1536 42.4 / 35.5, 1 x 4000 x 1536 73.4 / 57.8 (768 waves of the
+// one-lane kernel), 4 x 300 x 2048 30.4 / 26.6 (1280), 1 x 1024 x 5120 52.3 / 57.0 (2080).  The one-lane kernel takes a diagonal-real A's
+// exponentials from one, so there the line is a matter of work: 1 x 300 x 2048 17.6 / 14.4 us, 1 x 777 x 2048 22.5 / 23.3, 1 x 1024 x 1536 24.0 / 25.0.
+static bool quad_wins(bool s4d, int64_t waves, int64_t elements, int len) {
+    return len <= kQuadLen && (s4d ? elements <= 1200000 : waves <= 1536);
+}
+// As one pass up to this many steps (64 steps 9.2 us, 128 steps 16.0 where two passes take 11).
+constexpr int kQuadSingle = 64;
+
 // Shared body of the scan entry points: argument checks, route choice, launches.  `fn` names the caller in messages.
 static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void *y, const void *delta, const void *u,
                          const void *B, const void *C, int64_t bc_stride, const float *a_neg, const float *D,
@@ -998,6 +1009,11 @@ static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void
         const int64_t pairs = (int64_t)batch * ((d_inner + kWave - 1) / kWave);
         if (plan.nchunk < 2 || (T <= 256 && pairs >= 1024 && !(flags & MRS_FORCE_PARALLEL))) split = false;
     }
+    // shorter than two chunks: one pass with four lanes per channel while the chip is not full of the serial kernel's waves
+    if (d_state == 16 && rows_ok && T >= 8 && T < kQuadSingle && (int64_t)batch * ((d_inner + kWave - 1) / kWave) <= kSimds &&
+        !(flags & (MRS_FORCE_SEQUENTIAL | MRS_FORCE_PARALLEL | MRS_SCAN_TWO_LAUNCHES)))
+        return launch_scan_quad(st, dtype, gate_mode, {h, y, delta, u, B, C, gate, bc_stride, gate_stride, a_neg, D, nullptr, nullptr, nullptr, batch, T, d_inner,
+                                                       (d_inner + kWave - 1) / kWave, 1, T});
     if ((flags & MRS_FORCE_PARALLEL) && !split && d_state == 16 && T >= 64)
         return fail(MRS_E_WORKSPACE, "%s: MRS_FORCE_PARALLEL needs a workspace and 4-byte aligned B/C rows", fn);
     if (split) {
@@ -1016,6 +1032,12 @@ static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void
         const bool wins = (s4d && waves >= 2048) || (flags & MRS_FORCE_PARALLEL);
         int one_launch = (env_two || (flags & MRS_SCAN_TWO_LAUNCHES) || !wins || !flags_fit(batch, d_inner)) ? 0
                          : ((own_buffer || (flags & MRS_SCAN_FLAGS_ZERO)) ? 2 : 1);
+        if (!one_launch && !(flags & MRS_SCAN_TWO_LAUNCHES) && !env_two && quad_wins(s4d, waves, (int64_t)batch * T * d_inner, plan.len)) {
+            const SplitWs w = carve_workspace((float *)workspace, batch, T, d_inner, plan.nchunk);
+            const bool single = T <= kQuadSingle;
+            return launch_scan_quad(st, dtype, gate_mode, {h, y, delta, u, B, C, gate, bc_stride, gate_stride, a_neg, D, w.h0copy, w.S, w.sumd, batch, T, d_inner,
+                                                           (d_inner + kWave - 1) / kWave, single ? 1 : plan.nchunk, single ? T : plan.len});
+        }
         MRS_DISPATCH_DTYPE(dtype, T_, return launch_split<T_>(st, s4d, gate_mode, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride,
                                                              (float *)workspace, plan, batch, T, d_inner, one_launch));
     }

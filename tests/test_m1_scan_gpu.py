@@ -95,6 +95,36 @@ def test_scan_t_split_route_matches_oracle(shape, dtype, s4d):
         assert_close(h, h_ref, orc.F32, "h")
 
 
+@pytest.mark.parametrize("dtype", [orc.F32, orc.BF16, orc.F16])
+@pytest.mark.parametrize("shape", [
+    (2, 8, 72), (1, 63, 200), (3, 64, 128),   # one pass: the shortest, a last group of three steps, the longest; partial channel tiles
+    (2, 65, 72), (1, 127, 64),      # two passes, a last chunk of 17 steps
+    (1, 129, 64),                   # the last of five chunks holds one step
+    (1, 333, 200), (2, 1000, 96),   # more chunks than a fold requests at once, ragged
+    (1, 4090, 64),                  # 32 chunks of the longest length
+])
+@pytest.mark.parametrize("s4d", [False, True])
+def test_scan_with_four_lanes_per_channel_matches_oracle(shape, dtype, s4d):
+    """Less than a wave per SIMD: four lanes share a channel.  B and C in rows of their own and inside wider rows (dword-aligned
+    only), an entering state, every gate; the two-launch route of the other kernel on the same inputs holds the same bar."""
+    batch, T, di = shape
+    rng = np.random.default_rng(hash((shape, dtype, s4d, 2)) & 0xFFFF)
+    inp = quantised(rng, batch, T, di, 16, dtype, s4d=s4d)
+    h0 = (rng.standard_normal((batch, di, 16)) * 0.1).astype(np.float32)
+    wide = np.zeros((batch, T, 38), np.float32)
+    wide[..., 2:18], wide[..., 20:36] = inp["B"], inp["C"]
+    wd = dev(wide, dtype)
+    for gate_mode in (0, 1, 2):
+        print(f"case four lanes per channel shape={shape} dtype={dtype} s4d={s4d} gate={gate_mode}", flush=True)
+        y_ref, h_ref = orc.m1_scan_f64(h0, inp["delta"], inp["u"], inp["B"], inp["C"], inp["a_neg"], inp["D"],
+                                       gate=inp["z"] if gate_mode else None, gate_mode=gate_mode)
+        flags = ops.A_S4D_REAL if s4d else 0
+        for extra, view in ((0, None), (0, (wd[..., 2:18], wd[..., 20:36])), (ops.SCAN_TWO_LAUNCHES, None)):
+            y, h = run_scan(inp, h0, dtype, gate_mode, flags=flags | extra, bc_view=view, split="auto")
+            assert_close(y, y_ref, dtype, "y")
+            assert_close(h, h_ref, orc.F32, "h")
+
+
 def test_scan_auto_route_threshold_and_workspace_errors():
     """Up to 256 steps (the reference's serial range, src/config.rs:21-37) the single pass is kept when its (batch row,
     channel tile) pairs fill the machine -- bitwise equal to the no-workspace call -- and MRS_FORCE_SEQUENTIAL keeps it
