@@ -12,7 +12,7 @@
 //      registers, y = H q + D x, and the SiLU gate (optionally RMSNormGated over the head) -- the formulas of
 //      mamba3_layer_step (src/mamba3_siso/cpu/inference.rs:68-258) and kernels/mamba3_ops.cu;
 //   3. out_proj with the residual add, the next layer's pre-scaled operand and row sums of squares as epilogue.
-// At a few rows of a 16-bit model the whole step is one resident launch (resident_m3_step.hip).
+// At a few rows of a shallow 16-bit model the whole step is one resident launch (resident_m3_step.hip).
 // Shapes the skinny GEMM does not take (f32 storage above four rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
 #include "common.hpp"
 #include "gemm_tune.hpp"
@@ -650,13 +650,19 @@ int project_input3(mrs_m3_backbone *bb) {
     return MRS_OK;
 }
 
+// Deepest model that takes the resident step.  It adds the same products in another order than the kernel chain, and this network's
+// angles carry a 16-bit rounding that falls the other way from layer to layer: at 24 layers of d_model 768 two such orders differ by
+// 0.8 % of the output (each 1.1 % from f32; Mamba-1: 0.17 %), and 7 of 16 greedy passes of 32 tokens leave the chain's tokens somewhere
+// (the chain's own two orders, row-wise and tiled: 5 of 16).  The step would take 212 instead of 281 us there; deep models keep their tokens.
+constexpr int kResidentM3Layers = 8;
+
 // Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together: chosen before the weights are laid out
 // (the kernel chain's tiled copies are then not needed), set up behind them.
 void choose_resident3(mrs_m3_backbone *bb) {
     const mrs_m3_config &c = bb->cfg;
     const char *e = getenv("MRS_DECODE_NO_RESIDENT");
     // (RMSNormGated sums over a head, whose channels lie in several workgroups: the kernel chain)
-    if ((e && atoi(e) != 0) || !bb->skinny || c.is_outproj_norm) return;
+    if ((e && atoi(e) != 0) || !bb->skinny || c.is_outproj_norm || c.n_layers > kResidentM3Layers) return;
     ResidentM3Args &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr;
