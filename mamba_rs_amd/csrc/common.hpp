@@ -1,11 +1,11 @@
 // Shared device/host helpers for libmamba_hip (gfx950 only).
 #pragma once
-#include <optional>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
 #include "../../include/mamba_hip.h"
+#include "resident_gate.hpp"
 
 namespace mrs {
 
@@ -229,24 +229,6 @@ bool resident_m3_plan(ResidentM3Args &a, int dtype);
 size_t resident_m3_layer_bytes(const ResidentM3Args &a);
 int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, const ResidentM3Layer &w);
 int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev);
-// resident_gate.hip: whether this process's engines may take the resident route on a GPU (a claim counts the engine's
-// workgroups until it is released), and an engine's turn -- held while a step is launched.
-bool resident_claim(int device, int workgroups);
-void resident_release(int device, int workgroups, hipStream_t st);
-class ResidentTurn {
-public:
-    ResidentTurn(int device, hipStream_t st);
-    ~ResidentTurn();
-    ResidentTurn(const ResidentTurn &) = delete;
-    ResidentTurn &operator=(const ResidentTurn &) = delete;
-private:
-    int device_;
-};
-// An engine's turn while a step is launched, where the step is a resident launch (device < 0: it is not).
-struct StepTurn {
-    std::optional<ResidentTurn> turn;
-    StepTurn(int device, hipStream_t st) { if (device >= 0) turn.emplace(device, st); }
-};
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,
                             int64_t rows, int di, int dr);
@@ -287,7 +269,7 @@ struct LmHooks {
     size_t (*state_bytes)(void *self);               // recurrent state, for save / restore around a warm-up run
     int (*state_copy)(void *self, void *buf, int restore);
     int (*prefill)(void *self, const int *dev_tokens, const void *embed, int vocab, int T);   // tokens [batch, T] on device
-    int resident_device;      // the GPU whose ResidentTurn a step's launch needs, or -1
+    ResidentSeat *seat;       // the engine's seat for resident steps: a graph with a step in it is replayed in a ResidentTurn
     int (*check)(void *self); // after a synchronisation: an error if a step could not be completed
 };
 // gathers rows of the embedding table (storage type) as f32: out[r, :] = embed[clamp(tokens[r]), :] (engine prefill staging)

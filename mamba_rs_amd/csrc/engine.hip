@@ -286,6 +286,7 @@ struct mrs_backbone {
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
     int resident;                 // a few rows: the step as one resident launch (resident_step.hip)
+    ResidentSeat seat;            // ... its place at the gate (resident_gate.hip)
     ResidentArgs res_args, *res_args_dev;
     unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
     HostIo io;                    // step()'s rows in pinned host memory
@@ -607,8 +608,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
     return MRS_OK;
 }
 
-// Resident step (resident_step.hip) for the rows whose workgroups fit on the chip together: chosen before the weights are laid out (the
-// kernel chains' tiled copies are then not needed), set up behind them.
+// Resident step (resident_step.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
+// for the steps that do not get a turn.
 static void choose_resident(mrs_backbone *bb) {
     const mrs_m1_config &c = bb->cfg;
     const char *e = getenv("MRS_DECODE_NO_RESIDENT");
@@ -616,9 +617,8 @@ static void choose_resident(mrs_backbone *bb) {
     ResidentArgs &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.ds = c.d_state; a.dc = c.d_conv; a.dr = bb->dr; a.xd = bb->xd;
-    if (bb->batch > 256 || !resident_plan(a, bb->dtype) || !resident_claim(bb->device, a.G * a.batch)) return;
+    if (bb->batch > 256 || !resident_plan(a, bb->dtype) || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
     bb->resident = 1;
-    bb->tiled = bb->wide = 0;
 }
 
 static int arm_resident(mrs_backbone *bb) {
@@ -661,6 +661,7 @@ static int setup_resident(mrs_backbone *bb) {
 
 // After a synchronisation: whether every resident step found all its workgroups on the chip.
 static int check_resident(mrs_backbone *bb) {
+    resident_idle(bb->seat);
     if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
         return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
                                "or set MRS_DECODE_NO_RESIDENT=1");
@@ -841,7 +842,7 @@ extern "C" void mrs_backbone_destroy(mrs_backbone *bb) {
     if (!bb) return;
     hipSetDevice(bb->device);
     if (bb->stream) hipStreamSynchronize(bb->stream);
-    if (bb->resident) resident_release(bb->device, bb->res_args.G * bb->res_args.batch, bb->stream);
+    resident_release(bb->seat);
     if (bb->graph_exec) hipGraphExecDestroy(bb->graph_exec);
     if (bb->graph) hipGraphDestroy(bb->graph);
     if (bb->res_broken) hipHostFree(bb->res_broken);
@@ -869,8 +870,11 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
 static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
     if (bb->resident) {
-        if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
-        return launch_resident_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+        const ResidentTurn turn(&bb->seat);
+        if (turn.go()) {
+            if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
+            return launch_resident_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+        }
     }
     if (bb->tiny_layers) {
         TinyStepArgs a = {};
@@ -891,9 +895,11 @@ static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
 
 extern "C" int mrs_backbone_step_gpu_only(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_step_gpu_only: null engine");
-    const StepTurn turn(bb->resident ? bb->device : -1, bb->stream);
     const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
-    if (bb->graph_ready && !one_launch) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    if (bb->graph_ready && !one_launch) {
+        const ResidentTurn turn(&bb->seat);
+        if (turn.go()) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    }
     return step_body(bb);
 }
 
@@ -928,8 +934,7 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     MRS_HIP(hipMalloc(&save, cb + sb));
     hipMemcpyAsync(save, bb->conv_state, cb, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync((char *)save + cb, bb->ssm_state, sb, hipMemcpyDeviceToDevice, bb->stream);
-    int rc;
-    { const StepTurn turn(bb->resident ? bb->device : -1, bb->stream); rc = step_body(bb); }
+    int rc = step_body(bb);
     hipMemcpyAsync(bb->conv_state, save, cb, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->ssm_state, (char *)save + cb, sb, hipMemcpyDeviceToDevice, bb->stream);
     hipStreamSynchronize(bb->stream);
@@ -1144,7 +1149,7 @@ static LmHooks m1_hooks(mrs_backbone *bb) {
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
     h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy; h.prefill = m1_hook_prefill;
-    h.resident_device = bb->resident ? bb->device : -1; h.check = m1_hook_check;
+    h.seat = &bb->seat; h.check = m1_hook_check;
     return h;
 }
 
@@ -1261,8 +1266,10 @@ extern "C" int mrs_lm_set_tokens(mrs_lm *lm, const int *tokens) {
 // token, backbone step, tied head, argmax -> next token (left in the device token buffer).
 extern "C" int mrs_lm_decode_step(mrs_lm *lm) {
     if (!lm) return fail(MRS_E_NULL, "mrs_lm_decode_step: null engine");
-    const StepTurn turn(lm->eng.resident_device, lm->eng.stream);
-    if (lm->graph_ready) { MRS_HIP(hipGraphLaunch(lm->graph_exec, lm->eng.stream)); return MRS_OK; }
+    if (lm->graph_ready) {
+        const ResidentTurn turn(lm->eng.seat);
+        if (turn.go()) { MRS_HIP(hipGraphLaunch(lm->graph_exec, lm->eng.stream)); return MRS_OK; }
+    }
     return lm_decode_body(lm);
 }
 
@@ -1276,7 +1283,7 @@ extern "C" int mrs_lm_capture_graph(mrs_lm *lm) {
     MRS_HIP(hipMalloc(&save, sbytes + tb));
     int rc = bb->state_copy(bb->self, save, 0);
     hipMemcpyAsync((char *)save + sbytes, lm->tokens, tb, hipMemcpyDeviceToDevice, bb->stream);
-    if (!rc) { const StepTurn turn(bb->resident_device, bb->stream); rc = lm_decode_body(lm); }
+    if (!rc) rc = lm_decode_body(lm);
     if (!rc) rc = bb->state_copy(bb->self, save, 1);
     hipMemcpyAsync(lm->tokens, (char *)save + sbytes, tb, hipMemcpyDeviceToDevice, bb->stream);
     hipStreamSynchronize(bb->stream);
@@ -1463,10 +1470,7 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
     int done = 0, emitted = 0;
     bool stopped = false;
     for (int s = 0; s < steps && running > 0; s++) {
-        if (lm->gen_graph_ready) {
-            const StepTurn turn(bb->resident_device, st);
-            MRS_HIP(hipGraphLaunch(lm->gen_graph_exec, st));
-        } else if (s == 1) {
+        if (!lm->gen_graph_ready && s == 1) {
             // the first step ran eagerly (the GEMM library settles its choices); capture the step now and replay it from here on
             MRS_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             int rc = gen_forward(lm);
@@ -1478,10 +1482,13 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
             e = hipGraphInstantiate(&lm->gen_graph_exec, gph, nullptr, nullptr, 0);
             if (e != hipSuccess) { hipGraphDestroy(gph); return fail(MRS_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e)); }
             lm->gen_graph = gph; lm->gen_graph_ready = 1;
-            const StepTurn turn(bb->resident_device, st);
-            MRS_HIP(hipGraphLaunch(lm->gen_graph_exec, st));
-        } else {
-            const StepTurn turn(bb->resident_device, st);
+        }
+        bool replayed = false;
+        if (lm->gen_graph_ready) {
+            const ResidentTurn turn(bb->seat);
+            if (turn.go()) { MRS_HIP(hipGraphLaunch(lm->gen_graph_exec, st)); replayed = true; }
+        }
+        if (!replayed) {
             MRS_TRY(gen_forward(lm));
             MRS_TRY(gen_pick(lm));
         }

@@ -565,6 +565,7 @@ struct mrs_m3_backbone {
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
     HostIo io;              // step()'s rows in pinned host memory
     int resident;                 // a few rows: the step as one resident launch (resident_m3_step.hip)
+    ResidentSeat seat;            // ... its place at the gate (resident_gate.hip)
     ResidentM3Args res_args, *res_args_dev;
     unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
     TinyM3StepLayer *tiny_layers;   // small f32 models: the layer table of the single-launch step (null: kernel chains)
@@ -656,8 +657,8 @@ int project_input3(mrs_m3_backbone *bb) {
 // (the chain's own two orders, row-wise and tiled: 5 of 16).  The step would take 212 instead of 281 us there; deep models keep their tokens.
 constexpr int kResidentM3Layers = 8;
 
-// Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together: chosen before the weights are laid out
-// (the kernel chain's tiled copies are then not needed), set up behind them.
+// Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
+// for the steps that do not get a turn.
 void choose_resident3(mrs_m3_backbone *bb) {
     const mrs_m3_config &c = bb->cfg;
     const char *e = getenv("MRS_DECODE_NO_RESIDENT");
@@ -666,9 +667,8 @@ void choose_resident3(mrs_m3_backbone *bb) {
     ResidentM3Args &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr;
-    if (bb->batch > 256 || !resident_m3_plan(a, bb->dtype) || !resident_claim(bb->device, a.G * a.batch)) return;
+    if (bb->batch > 256 || !resident_m3_plan(a, bb->dtype) || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
     bb->resident = 1;
-    bb->tiled = 0;
 }
 
 int arm_resident3(mrs_m3_backbone *bb) {
@@ -707,6 +707,7 @@ int setup_resident3(mrs_m3_backbone *bb) {
 
 // After a synchronisation: whether every resident step found all its workgroups on the chip.
 int check_resident3(mrs_m3_backbone *bb) {
+    resident_idle(bb->seat);
     if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
         return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
                                "or set MRS_DECODE_NO_RESIDENT=1");
@@ -717,8 +718,11 @@ int check_resident3(mrs_m3_backbone *bb) {
 int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
     const mrs_m3_config &c = bb->cfg;
     if (bb->resident) {
-        if (!bb->identity_proj) MRS_TRY(project_input3(bb));
-        return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+        const ResidentTurn turn(&bb->seat);
+        if (turn.go()) {
+            if (!bb->identity_proj) MRS_TRY(project_input3(bb));
+            return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+        }
     }
     if (bb->tiny_layers) {
         TinyM3StepArgs a = {};
@@ -782,7 +786,7 @@ extern "C" int mrs_m3_backbone_reset(mrs_m3_backbone *bb) {
     MRS_HIP(hipMemsetAsync(bb->kst, 0, L * B * nh * ds * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->vst, 0, L * B * nh * hd * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->angle, 0, L * B * nh * na * 4, bb->stream));
-    if (check_resident3(bb)) {   // a resident step gave up: its exchange words start over with the state
+    if (bb->res_broken && *(volatile unsigned *)bb->res_broken) {   // a resident step gave up: its exchange words start over with the state
         MRS_HIP(hipStreamSynchronize(bb->stream));
         return arm_resident3(bb);
     }
@@ -793,7 +797,7 @@ extern "C" void mrs_m3_backbone_destroy(mrs_m3_backbone *bb) {
     if (!bb) return;
     hipSetDevice(bb->device);
     if (bb->stream) hipStreamSynchronize(bb->stream);
-    if (bb->resident) resident_release(bb->device, bb->res_args.G * bb->res_args.batch, bb->stream);
+    resident_release(bb->seat);
     if (bb->graph_exec) hipGraphExecDestroy(bb->graph_exec);
     if (bb->graph) hipGraphDestroy(bb->graph);
     if (bb->res_broken) hipHostFree(bb->res_broken);
@@ -946,9 +950,11 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
 
 extern "C" int mrs_m3_backbone_step_gpu_only(mrs_m3_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_step_gpu_only: null engine");
-    const StepTurn turn(bb->resident ? bb->device : -1, bb->stream);
     const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
-    if (bb->graph_ready && !one_launch) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    if (bb->graph_ready && !one_launch) {
+        const ResidentTurn turn(&bb->seat);
+        if (turn.go()) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+    }
     return step_body3(bb);
 }
 
@@ -984,8 +990,7 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     hipMemcpyAsync(save + n0, bb->kst, n1, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(save + n0 + n1, bb->vst, n2, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(save + n0 + n1 + n2, bb->angle, n3, hipMemcpyDeviceToDevice, bb->stream);
-    int rc;
-    { const StepTurn turn(bb->resident ? bb->device : -1, bb->stream); rc = step_body3(bb); }
+    int rc = step_body3(bb);
     hipMemcpyAsync(bb->ssm, save, n0, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->kst, save + n0, n1, hipMemcpyDeviceToDevice, bb->stream);
     hipMemcpyAsync(bb->vst, save + n0 + n1, n2, hipMemcpyDeviceToDevice, bb->stream);
@@ -1342,6 +1347,6 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = nullptr;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
-    h.prefill = m3_hook_prefill; h.resident_device = bb->resident ? bb->device : -1; h.check = m3_hook_check;
+    h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");
 }

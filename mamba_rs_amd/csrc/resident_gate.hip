@@ -2,20 +2,25 @@
 //
 // A resident launch's workgroups wait for each other, so they must all get a place on the GPU.  One launch alone always does (an
 // engine takes the route only while its workgroups are at most as many as the compute units, one each); two launches that hold
-// half of the places each would wait until their spin limit.  So
+// half of the places each would wait until they give up.  So
 //   * one process per GPU has the route: the first to ask binds an abstract socket named after the GPU's PCI address, which the
 //     system takes back when the process ends, whatever way it ends; another process's engines keep the kernel chains;
-//   * inside the process, engines whose launches do not all fit together take turns: a launch waits (on the GPU, with an event)
-//     for what the previous engine's stream holds.  An engine's own steps, on its one stream, follow each other anyway, and
-//     ordinary kernels on other streams end by themselves and only delay a launch.
-#include "common.hpp"
+//   * inside the process, while the live engines' launches do not all fit together, they go one after the other: every launch is
+//     followed by an event on its own stream, and the next engine's launch waits for it (on the GPU).  An engine touches no
+//     stream but its own: another one's may be in a capture, which an event recorded from here would join.
+//   * launches from before there were that many engines carry no event.  Until the host has waited for them, or their engine has
+//     launched again, the other engines' steps are kernel chains.
+// An engine's own steps, on its one stream, follow each other anyway, and ordinary kernels on other streams end by themselves.
+#include "resident_gate.hpp"
 #include <errno.h>
 #include <mutex>
-#include <string.h>
 #include <stddef.h>
+#include <stdio.h>
+#include <string.h>
 #include <sys/socket.h>
 #include <sys/un.h>
 #include <unistd.h>
+#include <vector>
 
 namespace mrs {
 namespace {
@@ -24,8 +29,9 @@ constexpr int kMaxDevices = 64;
 struct Gate {
     std::mutex m;
     bool asked = false, ours = false;
-    int places = 0, live = 0;         // compute units; workgroups of the live engines' launches
-    hipStream_t last = nullptr;       // stream of the last launch
+    int places = 0, live = 0;             // compute units; workgroups of the live engines' launches
+    std::vector<ResidentSeat *> seats;
+    const ResidentSeat *last = nullptr;   // whose launch `event` was recorded behind
     hipEvent_t event = nullptr;
 };
 Gate g_gates[kMaxDevices];
@@ -48,7 +54,7 @@ bool bind_gpu(int device) {
 
 }  // namespace
 
-bool resident_claim(int device, int workgroups) {
+bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t stream) {
     if (device < 0 || device >= kMaxDevices) return false;
     Gate &g = g_gates[device];
     std::lock_guard<std::mutex> lock(g.m);
@@ -58,27 +64,59 @@ bool resident_claim(int device, int workgroups) {
                  hipEventCreateWithFlags(&g.event, hipEventDisableTiming) == hipSuccess && bind_gpu(device);
     }
     if (!g.ours || workgroups > g.places) return false;
+    try { g.seats.push_back(&seat); } catch (...) { return false; }
+    seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = false;
     g.live += workgroups;
     return true;
 }
 
-void resident_release(int device, int workgroups, hipStream_t st) {
-    Gate &g = g_gates[device];
+void resident_release(ResidentSeat &seat) {
+    if (seat.device < 0) return;
+    Gate &g = g_gates[seat.device];
     std::lock_guard<std::mutex> lock(g.m);
-    g.live -= workgroups;
-    if (g.last == st) g.last = nullptr;   // (its work is done: the engine has waited for its stream)
+    g.live -= seat.workgroups;
+    for (size_t i = 0; i < g.seats.size(); i++)
+        if (g.seats[i] == &seat) { g.seats.erase(g.seats.begin() + i); break; }
+    if (g.last == &seat) g.last = nullptr;   // (its work is done)
+    seat.device = -1;
 }
 
-ResidentTurn::ResidentTurn(int device, hipStream_t st) : device_(device) {
-    Gate &g = g_gates[device];
-    g.m.lock();
-    if (g.last && g.last != st && g.live > g.places) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone && hipEventRecord(g.event, g.last) == hipSuccess)
-            (void)hipStreamWaitEvent(st, g.event, 0);
-    }
-    g.last = st;
+void resident_idle(ResidentSeat &seat) {
+    if (seat.device < 0) return;
+    std::lock_guard<std::mutex> lock(g_gates[seat.device].m);
+    seat.open = false;
 }
-ResidentTurn::~ResidentTurn() { g_gates[device_].m.unlock(); }
+
+ResidentTurn::ResidentTurn(ResidentSeat *seat) : seat_(seat), go_(true) {
+    if (!seat || seat->device < 0) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(seat->stream, &cap) != hipSuccess) { go_ = false; return; }
+    if (cap != hipStreamCaptureStatusNone) return;   // recorded, not run
+    Gate &g = g_gates[seat->device];
+    g.m.lock();
+    if (g.live > g.places) {
+        for (const ResidentSeat *s : g.seats)
+            if (s != seat && s->open) go_ = false;
+        if (go_ && g.last && g.last != seat && hipStreamWaitEvent(seat->stream, g.event, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            go_ = false;
+        }
+    }
+    if (go_) locked_ = true;
+    else g.m.unlock();
+}
+
+ResidentTurn::~ResidentTurn() {
+    if (!locked_) return;
+    Gate &g = g_gates[seat_->device];
+    seat_->open = true;
+    if (g.live > g.places) {
+        if (hipEventRecord(g.event, seat_->stream) == hipSuccess) {
+            seat_->open = false;
+            g.last = seat_;
+        } else (void)hipGetLastError();
+    }
+    g.m.unlock();
+}
 
 }  // namespace mrs

@@ -63,3 +63,86 @@ def test_resident_step_follows_the_cpu_route(shape, dtype):
     assert np.array_equal(a.step(x[0]), b.step(x[0]))
     a.close()
     b.close()
+
+
+def _engines(shape, n, dtype=WeightDtype.BF16):
+    dm, L, B = shape
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
+    w = MambaWeights.init(cfg, dm, 5)
+    w.input_proj_w = np.zeros((0, dm), np.float32)
+    return [GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype) for _ in range(n)]
+
+
+def test_queued_steps_of_engines_that_do_not_fit_together():
+    """Two engines of 256 workgroups (and a third of 128): their steps are queued in turns with nothing waited for in between, so
+    each launch meets the one before still running.  Every engine ends on the bits of one that was alone."""
+    a, b = _engines((768, 6, 4), 2)
+    c, = _engines((768, 4, 2), 1)
+    rng = np.random.default_rng(2)
+    x = {e: rng.standard_normal((e.batch, 768)).astype(np.float32) for e in (a, b, c)}
+
+    def run(engines, n):
+        for e in engines:
+            e.reset()
+            e.step(x[e])
+        for _ in range(n):
+            for e in engines:
+                e.step_gpu_only()
+        return [e.download_temporal() for e in engines]
+    print("case queued steps of three engines", flush=True)
+    assert [e.decode_route() for e in (a, b, c)] == [2, 2, 2]
+    alone = [run([e], 24)[0] for e in (a, b, c)]
+    for got, want in zip(run([a, b, c], 24), alone):
+        assert np.array_equal(got, want)
+    for e in (a, b, c):
+        e.close()
+
+
+def test_an_engine_captures_while_another_one_steps():
+    """Two threads, two engines that do not fit together: one builds language models and captures their step over and over, the
+    other queues steps.  Nothing of one engine ends in the other's graph: tokens and rows are those of each one alone."""
+    import threading
+    from mamba_rs_amd import GpuMambaLM
+    a, b = _engines((768, 4, 4), 2)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((4, 768)).astype(np.float32)
+    embed = rng.standard_normal((256, 768)).astype(np.float32)
+    first = np.arange(4, dtype=np.int32)
+
+    def captured():
+        lm = GpuMambaLM(a, embed)
+        a.reset()
+        lm.set_tokens(first)
+        lm.capture_graph()
+        got = []
+        for _ in range(6):
+            lm.decode_step()
+            got.append(lm.get_tokens().tolist())
+        lm.close()
+        return got
+
+    def stepped():
+        b.reset()
+        b.step(x)
+        for _ in range(40):
+            b.step_gpu_only()
+        return b.download_temporal()
+    print("case capture beside steps", flush=True)
+    want, row = captured(), stepped()
+    res = {"a": [], "b": []}
+
+    def loop(key, fn, n):
+        try:
+            for _ in range(n):
+                res[key].append(fn())
+        except Exception as e:      # into the main thread
+            res[key].append(e)
+    ts = [threading.Thread(target=loop, args=("a", captured, 12)), threading.Thread(target=loop, args=("b", stepped, 24))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert len(res["a"]) == 12 and all(r == want for r in res["a"])
+    assert len(res["b"]) == 24 and all(isinstance(r, np.ndarray) and np.array_equal(r, row) for r in res["b"])
+    a.close()
+    b.close()
