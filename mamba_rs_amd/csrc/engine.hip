@@ -940,6 +940,7 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     hipStreamSynchronize(bb->stream);
     hipFree(save);
     if (rc) return rc;
+    const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = step_body(bb);
     hipGraph_t g = nullptr;
@@ -1289,6 +1290,7 @@ extern "C" int mrs_lm_capture_graph(mrs_lm *lm) {
     hipStreamSynchronize(bb->stream);
     hipFree(save);
     if (rc) return rc;
+    const ResidentRecording rec(bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = lm_decode_body(lm);
     hipGraph_t g = nullptr;
@@ -1472,6 +1474,7 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
     for (int s = 0; s < steps && running > 0; s++) {
         if (!lm->gen_graph_ready && s == 1) {
             // the first step ran eagerly (the GEMM library settles its choices); capture the step now and replay it from here on
+            const ResidentRecording rec(bb->seat);
             MRS_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             int rc = gen_forward(lm);
             if (!rc) rc = gen_pick(lm);

@@ -999,6 +999,7 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     hipFree(save);
     if (rc) return rc;
     if (e != hipSuccess) return fail(MRS_E_HIP, "capture warm-up: %s", hipGetErrorString(e));
+    const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = step_body3(bb);
     hipGraph_t g = nullptr;

@@ -9,7 +9,8 @@
 //     followed by an event on its own stream, and the next engine's launch waits for it (on the GPU).  An engine touches no
 //     stream but its own: another one's may be in a capture, which an event recorded from here would join.
 //   * launches from before there were that many engines carry no event.  Until the host has waited for them, or their engine has
-//     launched again, the other engines' steps are kernel chains.
+//     launched again, the other engines' steps are kernel chains;
+//   * a step that a caller captures on an engine's stream is the kernel chain: the caller's replays take no turns.
 // An engine's own steps, on its one stream, follow each other anyway, and ordinary kernels on other streams end by themselves.
 #include "resident_gate.hpp"
 #include <errno.h>
@@ -91,7 +92,7 @@ ResidentTurn::ResidentTurn(ResidentSeat *seat) : seat_(seat), go_(true) {
     if (!seat || seat->device < 0) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(seat->stream, &cap) != hipSuccess) { go_ = false; return; }
-    if (cap != hipStreamCaptureStatusNone) return;   // recorded, not run
+    if (cap != hipStreamCaptureStatusNone) { go_ = seat->recording; return; }   // recorded, not run
     Gate &g = g_gates[seat->device];
     g.m.lock();
     if (g.live > g.places) {

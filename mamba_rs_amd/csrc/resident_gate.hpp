@@ -9,13 +9,15 @@ struct ResidentSeat {
     int device = -1, workgroups = 0;   // device < 0: no claim, the engine's steps are kernel chains
     hipStream_t stream = nullptr;      // the engine's stream
     bool open = false;                 // launches that no event covers and that the host has not waited for
+    bool recording = false;            // the engine captures a step for itself
 };
 bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t stream);
 void resident_release(ResidentSeat &seat);   // the engine has waited for its stream
 void resident_idle(ResidentSeat &seat);      // the same, and goes on
 
 // An engine's turn: made before a resident launch (or the replay of a graph that holds one) and dropped right behind it.  go()
-// false: no launch now -- the step is the kernel chain, which waits for nobody.  An engine without a seat always goes.
+// false: no launch now -- the step is the kernel chain, which waits for nobody.  An engine without a seat always goes.  In a
+// capture only the engine's own recording goes: its replays take turns.  A caller's graph is replayed with no turn and gets the chain.
 class ResidentTurn {
 public:
     explicit ResidentTurn(ResidentSeat *seat);
@@ -26,6 +28,15 @@ public:
 private:
     ResidentSeat *seat_;
     bool go_, locked_ = false;
+};
+
+// While an engine captures a step for itself.
+struct ResidentRecording {
+    ResidentSeat *seat;
+    explicit ResidentRecording(ResidentSeat *s) : seat(s) { if (seat) seat->recording = true; }
+    ~ResidentRecording() { if (seat) seat->recording = false; }
+    ResidentRecording(const ResidentRecording &) = delete;
+    ResidentRecording &operator=(const ResidentRecording &) = delete;
 };
 
 }  // namespace mrs

@@ -12,14 +12,15 @@ struct Engine {
     ModelStream stream;
     int workgroups = 0;
     long last = 0;        // number of its last launch on its stream, 0: none that the host has not waited for
-    bool turns = false;
+    bool turns = false, own_capture = false;
 };
 
 const char *launch(Engine &e, std::vector<std::unique_ptr<Engine>> &all, int live, long &ordered, long &refused) {
     Model &m = model();
     m.acting = &e.stream;
     const ResidentTurn turn(e.turns ? &e.seat : nullptr);
-    if (!turn.go()) { refused++; return nullptr; }
+    if (!turn.go()) { refused += !e.stream.capturing; return nullptr; }
+    if (e.turns && e.stream.capturing && !e.own_capture) return "a launch in a caller's capture";
     if (!e.turns || e.stream.capturing) return nullptr;   // a kernel chain, or nothing that runs now
     auto &own = e.stream.before;
     if ((int)own.size() <= e.stream.id) own.resize(e.stream.id + 1, 0);
@@ -72,6 +73,7 @@ int main(int argc, char **argv) {
             all.erase(all.begin() + at);
         } else if (what < 15) {
             e.stream.capturing = !e.stream.capturing;
+            e.own_capture = e.seat.recording = e.stream.capturing && rng() % 2;
         } else if (what < 30) {
             if (e.stream.capturing) continue;   // (a captured stream cannot be waited for)
             host_wait(e, all);

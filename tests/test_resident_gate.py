@@ -24,7 +24,8 @@ def model(tmp_path_factory):
 @pytest.mark.parametrize("fail_every", [0, 7])
 def test_launches_that_do_not_fit_together_are_ordered(model, seed, fail_every):
     """Random engines, steps, waits and captures: no two launches that need more places than there are run unordered, no turn
-    records or waits on a stream but its own or on one that is in a capture, and neither does a failing event let a launch through."""
+    records or waits on a stream but its own or on one that is in a capture, a caller's capture gets no launch, and neither does a
+    failing event let one through."""
     r = model(seed, fail_every)
     assert r.returncode == 0 and r.stdout.startswith("ok "), r.stdout + r.stderr
     in_turns, refused = map(int, r.stdout.split()[1:])

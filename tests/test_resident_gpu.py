@@ -146,3 +146,70 @@ def test_an_engine_captures_while_another_one_steps():
     assert len(res["b"]) == 24 and all(isinstance(r, np.ndarray) and np.array_equal(r, row) for r in res["b"])
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("family", ["m1", "m3"])
+def test_a_caller_s_capture_gets_the_kernel_chain(family, monkeypatch):
+    """step_gpu_only and a language model's decode_step captured by the caller on the engine's stream: the graph holds the kernel
+    chain (its replays take no turns), so every replay, with eager work in between, leaves the bits of an engine that has only the
+    chain; the engine's own steps are resident before and after."""
+    import torch
+    from mamba_rs_amd import GpuMambaLM, GpuMamba3Backbone, GpuMamba3LM
+    if family == "m1":
+        make, lm_of, dm = lambda: _engines((768, 3, 4), 1)[0], GpuMambaLM, 768
+    else:
+        from test_m3_engine_gpu import perturbed
+        from test_resident_m3_gpu import cfg_
+        cfg, dm = cfg_(256, 16, 16, 1, 3), 256
+        w = perturbed(cfg, dm, 11)
+        w.input_proj_w = np.zeros(0, np.float32)
+        make, lm_of = lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, 4, WeightDtype.BF16), GpuMamba3LM
+    a = make()
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = make()
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((4, dm)).astype(np.float32)
+    embed = rng.standard_normal((128, dm)).astype(np.float32)
+    print(f"case capture by the caller {family}", flush=True)
+    resident = a.step(x)
+    chain.step(x)
+    lms = []
+    for e in (a, chain):
+        lm = lm_of(e, embed)
+        lm.set_tokens(np.arange(4, dtype=np.int32))
+        lm.decode_step()          # (the head's GEMM library settles its choice outside the captures)
+        e.sync()
+        lms.append(lm)
+    lms[0].capture_graph()
+    graphs = []
+    for e, lm in zip((a, chain), lms):
+        for call in (e.step_gpu_only, lm.decode_step):
+            side = torch.cuda.ExternalStream(e.stream())
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=side, capture_error_mode="thread_local"):
+                call()
+            graphs.append((e, side, g))
+
+    def replay(i):
+        e, side, g = graphs[i]
+        with torch.cuda.stream(side):
+            g.replay()
+    for e, lm in zip((a, chain), lms):
+        e.reset()
+        lm.set_tokens(np.arange(4, dtype=np.int32))
+    for n in range(4):
+        rows, toks = [], []
+        for i, (e, lm) in enumerate(zip((a, chain), lms)):
+            replay(2 * i + n % 2)
+            replay(2 * i + 1)
+            rows.append(lm.last_logits())
+            toks.append(lm.get_tokens())
+            _ = torch.ones(1 << 16, device="cuda").sum().item()
+        assert np.array_equal(rows[0], rows[1]) and np.array_equal(toks[0], toks[1]), n
+        assert np.isfinite(rows[0]).all()
+    a.reset()
+    assert np.array_equal(a.step(x), resident) and a.decode_route() == 2
+    del graphs
+    for e in (*lms, a, chain):
+        e.close()
