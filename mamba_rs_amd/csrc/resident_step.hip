@@ -140,18 +140,18 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         const float inv = l == 0 ? inv0 : invl[0];
         pin.run(xs, dm >> 5, ct_in, pre);
         lds_barrier();   // 1
+        float xnew = 0.0f;
         if (conv_wave) {
-            // ---- conv step + SiLU, by every wave that needs the channels; the first one stores the window
+            // ---- conv step + SiLU, by every wave that needs the channels
             const int i = min(here(lane), nc - 1);
             const float4 tap = *reinterpret_cast<const float4 *>(small + sb.cw + i * 16);
             const float bias = *reinterpret_cast<const float *>(small + sb.cb + i * 4);
             const T xr = (T)(row_sum(pre, 2 * nc, i) * inv), zr = (T)(row_sum(pre, 2 * nc, nc + i) * inv);
-            const float xnew = Store<T>::ld(&xr);
+            xnew = Store<T>::ld(&xr);
             float o = fmaf(cwin.y, tap.x, bias);
             o = fmaf(cwin.z, tap.y, o); o = fmaf(cwin.w, tap.z, o); o = fmaf(xnew, tap.w, o);
             us[i] = (T)silu(o);   // (the waves write the same values)
             zs[i] = Store<T>::ld(&zr);
-            if (wave == 0 && lane < nc) *reinterpret_cast<float4 *>(cst + l * cst_l + i * kDc) = make_float4(cwin.y, cwin.z, cwin.w, xnew);
             // ---- share of the x_proj row: 16 entries per tile
             const int n = here(lane) & 15, kg = here(lane) >> 4;
 #pragma unroll 1
@@ -199,6 +199,8 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         if (!ok) bad = 1;
         lds_barrier();   // 2
         if (bad) break;
+        // the window, by the first wave: all waves have theirs in registers, they have used it in front of the barrier
+        if (wave == 0 && lane < nc) *reinterpret_cast<float4 *>(cst + l * cst_l + lane * kDc) = make_float4(cwin.y, cwin.z, cwin.w, xnew);
         // ---- dt_proj + softplus, state update, D skip, gate: sixteen lanes per channel, one state each
         if (here(tid) < nc * kDs) {
             const int t = here(tid), n = t & 15, cl = t >> 4;

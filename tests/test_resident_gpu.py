@@ -213,3 +213,23 @@ def test_a_caller_s_capture_gets_the_kernel_chain(family, monkeypatch):
     del graphs
     for e in (*lms, a, chain):
         e.close()
+
+
+@pytest.mark.parametrize("dm,B", [(32, 4), (64, 16), (256, 8)])
+def test_conv_windows_move_by_one_step(dm, B):
+    """Narrow models, where a workgroup's waves read a conv window at nearly the time its first wave stores the next one: after every
+    step each window holds the last three entries of the one before, and a second engine has the same bits."""
+    a, b = _engines((dm, 2, B), 2)
+    rng = np.random.default_rng(dm)
+    print(f"case conv windows {dm} x {B}", flush=True)
+    assert a.decode_route() == 2
+    old = [a.download_state(l)[0] for l in range(2)]
+    for t in range(60):
+        x = rng.standard_normal((B, dm)).astype(np.float32)
+        assert np.array_equal(a.step(x), b.step(x)), t
+        for l in range(2):
+            new = a.download_state(l)[0]
+            assert np.array_equal(new[..., :3], old[l][..., 1:]), (t, l)
+            old[l] = new
+    a.close()
+    b.close()
