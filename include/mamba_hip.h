@@ -332,6 +332,11 @@ MRS_API int mrs_backbone_temporal_dtype(mrs_backbone *bb);
 #define MRS_DECODE_OWN_CHAIN 1
 #define MRS_DECODE_ONE_LAUNCH 2
 MRS_API int mrs_backbone_decode_route(mrs_backbone *bb);
+/* A 16-bit step of a few rows in one launch (MRS_DECODE_ONE_LAUNCH) begins when all its workgroups have a place on the GPU. `polls`
+ * (one to two microseconds each; 2^23 unless set) is how long it waits for that before it is called off with the state unchanged:
+ * step() then runs the kernel chain instead, queued steps end in an error at the next call that synchronises, and both hold until
+ * reset(). 0: called off at once, for trying out a program's handling of it. No effect on engines with another decode route. */
+MRS_API int mrs_backbone_set_resident_wait(mrs_backbone *bb, unsigned polls);
 /* download_temporal (inference.rs:1727-1737): the last step's / prefill's final-norm rows [batch, d_model] to the host; synchronises. */
 MRS_API int mrs_backbone_download_temporal(mrs_backbone *bb, float *out);
 MRS_API float *mrs_backbone_input_ptr(mrs_backbone *bb);
@@ -459,6 +464,7 @@ MRS_API float *mrs_m3_backbone_temporal_ptr(mrs_m3_backbone *bb);
 /* temporal_dtype (src/mamba3_siso/gpu/inference.rs:1561-1563) and the decode route, as for the Mamba-1 engine */
 MRS_API int mrs_m3_backbone_temporal_dtype(mrs_m3_backbone *bb);
 MRS_API int mrs_m3_backbone_decode_route(mrs_m3_backbone *bb);
+MRS_API int mrs_m3_backbone_set_resident_wait(mrs_m3_backbone *bb, unsigned polls);
 MRS_API float *mrs_m3_backbone_input_ptr(mrs_m3_backbone *bb);
 MRS_API void *mrs_m3_backbone_stream(mrs_m3_backbone *bb);
 MRS_API int mrs_m3_backbone_sync(mrs_m3_backbone *bb);

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass, field
-from ctypes import c_uint64, POINTER, Structure, byref, c_float, c_int, c_void_p
+from ctypes import c_uint64, POINTER, Structure, byref, c_float, c_int, c_uint, c_void_p
 
 import numpy as np
 
@@ -55,6 +55,7 @@ def _bind():
         "mrs_backbone_temporal_ptr": (P, [P]),
         "mrs_backbone_temporal_dtype": (c_int, [P]),
         "mrs_backbone_decode_route": (c_int, [P]),
+        "mrs_backbone_set_resident_wait": (c_int, [P, c_uint]),
         "mrs_backbone_download_temporal": (c_int, [P, _FP]),
         "mrs_backbone_set_gemm_tuning": (c_int, [P, c_int]),
         "mrs_backbone_input_ptr": (P, [P]),
@@ -224,6 +225,11 @@ class GpuMambaBackbone:
     def decode_route(self) -> int:
         """0: chain on the vendor GEMM, 1: the library's own fused chain, 2: a whole step in one launch."""
         return _bind().mrs_backbone_decode_route(self._h)
+
+    def set_resident_wait(self, polls: int):
+        """How long a one-launch 16-bit step waits for its places on the GPU before it is called off, in polls of one to
+        two microseconds: step() then runs the kernel chain, queued steps raise at the next call that synchronises, until reset()."""
+        _call("mrs_backbone_set_resident_wait", self._h, polls)
 
     def input_ptr(self) -> int:
         return _bind().mrs_backbone_input_ptr(self._h)

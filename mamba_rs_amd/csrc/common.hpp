@@ -192,7 +192,11 @@ int launch_tiny_step(hipStream_t st, const TinyStepArgs &a);
 // A whole Mamba-1 backbone step in one resident launch (resident_step.hip), 16-bit storage.  G workgroups per batch row, each owning nc
 // channels and oc out_proj columns (resident_plan fills these in).  weights: n_layers blocks of resident_layer_bytes(), each
 // packed by launch_resident_pack from a layer's weights as the engine holds them.  norm_w: layer 0's norm weight.  xch: batch *
-// xch_stride 64-bit words and epoch: 32 words per row, all zero before the first launch; broken: one word of pinned host memory.
+// xch_stride 64-bit words, epoch: 32 words per row, and roll: kRollHead + kRollMax words, all zero before the first launch; wait: how long a launch waits
+// for places (RollCall); broken: one word of pinned host memory, 0 or a ResidentFault.
+enum ResidentFault { kStepCalledOff = 1, kStepLost = 2 };   // no places, the states are what they were; given up in the middle
+constexpr unsigned kResidentWait = 1u << 23;                // default wait: ten to fifteen seconds
+constexpr int kRollHead = 32, kRollMax = 256;               // kRollMax: the most workgroups of a launch
 struct ResidentLayer {   // in_t [2 d_inner][d_model], out_t [d_model][d_inner], dt_t [d_inner][dt_rank] transposed, x_proj [d_inner][xd]; next_nw: the norm weight after, or null
     const void *in_t, *out_t, *x_proj, *dt_t; const float *a_neg, *conv_w, *conv_b, *D, *dt_b, *next_nw;
 };
@@ -202,8 +206,9 @@ struct ResidentArgs {
     float *conv_state, *ssm_state, *temporal;
     void *temporal_t;
     unsigned long long *xch;
-    unsigned *epoch, *broken;
+    unsigned *epoch, *roll, *broken;
     size_t xch_stride;
+    unsigned wait;
     float eps;
     int n_layers, batch, dm, di, ds, dc, dr, xd, G, nc, oc;
 };
@@ -220,8 +225,9 @@ struct ResidentM3Args {
     const float *input, *norm_w, *norm_f;
     float *ssm, *kst, *vst, *angle, *temporal;
     unsigned long long *xch;
-    unsigned *epoch, *broken;
+    unsigned *epoch, *roll, *broken;
     size_t xch_stride;
+    unsigned wait;
     float eps, a_floor;
     int n_layers, batch, dm, di, nh, hd, ds, ng, nr, G, nc, oc, ex;
 };
@@ -271,6 +277,7 @@ struct LmHooks {
     int (*prefill)(void *self, const int *dev_tokens, const void *embed, int vocab, int T);   // tokens [batch, T] on device
     ResidentSeat *seat;       // the engine's seat for resident steps: a graph with a step in it is replayed in a ResidentTurn
     int (*check)(void *self); // after a synchronisation: an error if a step could not be completed
+    bool (*go_on_chain)(void *self);   // after a synchronisation: the one step since the last check was called off, the next ones are kernel chains
 };
 // gathers rows of the embedding table (storage type) as f32: out[r, :] = embed[clamp(tokens[r]), :] (engine prefill staging)
 int launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab);

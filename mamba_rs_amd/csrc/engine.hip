@@ -617,15 +617,16 @@ static void choose_resident(mrs_backbone *bb) {
     ResidentArgs &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.ds = c.d_state; a.dc = c.d_conv; a.dr = bb->dr; a.xd = bb->xd;
-    if (bb->batch > 256 || !resident_plan(a, bb->dtype) || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
+    if (bb->batch > kRollMax || !resident_plan(a, bb->dtype) || a.G * a.batch > kRollMax || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
     bb->resident = 1;
 }
 
 static int arm_resident(mrs_backbone *bb) {
     const ResidentArgs &a = bb->res_args;
     MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
-    MRS_HIP(hipMemsetAsync(a.epoch, 0, (size_t)a.batch * 128, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4, bb->stream));
     *bb->res_broken = 0;
+    bb->seat.unseen = false;
     return MRS_OK;
 }
 
@@ -636,7 +637,9 @@ static int setup_resident(mrs_backbone *bb) {
     a.input = bb->identity_proj ? bb->d_input : bb->step_s.residual;
     a.norm_f = bb->norm_f; a.conv_state = bb->conv_state; a.ssm_state = bb->ssm_state; a.temporal = bb->temporal; a.temporal_t = bb->temporal_t;
     MRS_TRY(dev_alloc(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
-    MRS_TRY(dev_alloc(bb, (void **)&a.epoch, (size_t)a.batch * 128));
+    MRS_TRY(dev_alloc(bb, (void **)&a.epoch, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4));
+    a.roll = a.epoch + (size_t)a.batch * 32;
+    a.wait = kResidentWait;
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident(bb));
@@ -659,13 +662,23 @@ static int setup_resident(mrs_backbone *bb) {
     return MRS_OK;
 }
 
-// After a synchronisation: whether every resident step found all its workgroups on the chip.
+// After a synchronisation: whether every resident step was carried out.
+static unsigned resident_fault(const mrs_backbone *bb) { return bb->res_broken ? *(volatile unsigned *)bb->res_broken : 0; }
 static int check_resident(mrs_backbone *bb) {
     resident_idle(bb->seat);
-    if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
-        return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
-                               "or set MRS_DECODE_NO_RESIDENT=1");
+    if (const unsigned f = resident_fault(bb))
+        return fail(MRS_E_HIP, "resident decode step: %s; reset() the engine, or set MRS_DECODE_NO_RESIDENT=1",
+                    f == kStepCalledOff ? "the GPU's compute units did not come free in time (other work or another process holds them), and no step since was carried out"
+                                        : "workgroups gave up waiting for each other");
+    bb->seat.unseen = false;
     return MRS_OK;
+}
+// After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until
+// a reset, the steps are kernel chains.
+static bool go_on_chain(mrs_backbone *bb) {
+    if (resident_fault(bb) != kStepCalledOff || arm_resident(bb)) return false;
+    bb->seat.off = true;
+    return true;
 }
 
 extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mrs_m1_weights *w,
@@ -860,7 +873,8 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
     const size_t L = bb->cfg.n_layers, B = bb->batch;
     MRS_HIP(hipMemsetAsync(bb->conv_state, 0, L * B * bb->di * bb->cfg.d_conv * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->ssm_state, 0, L * B * bb->di * bb->cfg.d_state * 4, bb->stream));
-    if (bb->res_broken && *(volatile unsigned *)bb->res_broken) {   // a resident step gave up: its exchange words start over with the state
+    bb->seat.off = false;
+    if (resident_fault(bb)) {   // a resident step gave up: its exchange words start over with the state
         MRS_HIP(hipStreamSynchronize(bb->stream));
         return arm_resident(bb);
     }
@@ -908,7 +922,8 @@ extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *ou
     const int B = bb->batch, dm = bb->cfg.d_model, n = B * bb->input_dim;
     HostIo &io = bb->io;
     memcpy(io.in, input, (size_t)n * 4);
-    const HostRows host = {io.out, io.done, ++io.seq};
+    HostRows host = {io.out, io.done, ++io.seq};
+    const bool all_seen = !bb->seat.unseen;
     if (bb->tiny_layers) {
         MRS_TRY(step_body(bb, &host));
     } else {
@@ -918,6 +933,13 @@ extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *ou
         MRS_TRY(check_launch("host row kernels"));
     }
     MRS_TRY(host_io_wait(&io, bb->stream));
+    if (all_seen && go_on_chain(bb)) {   // this very step found no places
+        host.seq = ++io.seq;
+        MRS_TRY(step_body(bb));
+        hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
+        MRS_TRY(check_launch("host_out_kernel"));
+        MRS_TRY(host_io_wait(&io, bb->stream));
+    }
     memcpy(output, io.out, (size_t)B * dm * 4);
     return check_resident(bb);
 }
@@ -930,6 +952,7 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     // warm step on a copy of the state: save, run, restore
     const size_t L = bb->cfg.n_layers, B = bb->batch;
     const size_t cb = L * B * bb->di * bb->cfg.d_conv * 4, sb = L * B * bb->di * bb->cfg.d_state * 4;
+    const bool all_seen = !bb->seat.unseen;
     void *save = nullptr;
     MRS_HIP(hipMalloc(&save, cb + sb));
     hipMemcpyAsync(save, bb->conv_state, cb, hipMemcpyDeviceToDevice, bb->stream);
@@ -940,6 +963,8 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     hipStreamSynchronize(bb->stream);
     hipFree(save);
     if (rc) return rc;
+    if (all_seen) go_on_chain(bb);
+    MRS_TRY(check_resident(bb));
     const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = step_body(bb);
@@ -994,7 +1019,7 @@ extern "C" int mrs_backbone_prefill_sequence(mrs_backbone *bb, const float *inpu
     MRS_TRY(mrs_backbone_prefill_device(bb, bb->prefill_in, T));
     if (output_last) MRS_HIP(hipMemcpyAsync(output_last, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident(bb);   // (steps before it)
 }
 
 extern "C" void *mrs_backbone_stream(mrs_backbone *bb) { return bb ? (void *)bb->stream : nullptr; }
@@ -1004,6 +1029,15 @@ extern "C" int mrs_backbone_temporal_dtype(mrs_backbone *bb) { return bb ? MRS_F
 extern "C" int mrs_backbone_decode_route(mrs_backbone *bb) {
     if (!bb) return -1;
     return bb->tiny_layers || bb->resident ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
+}
+// How long a resident step waits for its places on the chip before it is called off, in polls of one to two microseconds.
+extern "C" int mrs_backbone_set_resident_wait(mrs_backbone *bb, unsigned polls) {
+    if (!bb) return fail(MRS_E_NULL, "mrs_backbone_set_resident_wait: null engine");
+    if (!bb->resident) return MRS_OK;
+    bb->res_args.wait = polls;
+    MRS_HIP(hipMemcpyAsync(bb->res_args_dev, &bb->res_args, sizeof(ResidentArgs), hipMemcpyHostToDevice, bb->stream));
+    MRS_HIP(hipStreamSynchronize(bb->stream));
+    return MRS_OK;
 }
 extern "C" int mrs_backbone_download_temporal(mrs_backbone *bb, float *out) {
     if (!bb || !out) return fail(MRS_E_NULL, "mrs_backbone_download_temporal: null pointer");
@@ -1144,13 +1178,14 @@ static int m1_hook_prefill(void *self, const int *dev_tokens, const void *embed,
     return mrs_backbone_prefill_device(bb, bb->prefill_in, T);
 }
 static int m1_hook_check(void *self) { return check_resident((mrs_backbone *)self); }
+static bool m1_hook_go_on_chain(void *self) { return go_on_chain((mrs_backbone *)self); }
 static LmHooks m1_hooks(mrs_backbone *bb) {
     LmHooks h = {};
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
     h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy; h.prefill = m1_hook_prefill;
-    h.seat = &bb->seat; h.check = m1_hook_check;
+    h.seat = &bb->seat; h.check = m1_hook_check; h.go_on_chain = m1_hook_go_on_chain;
     return h;
 }
 
@@ -1280,6 +1315,7 @@ extern "C" int mrs_lm_capture_graph(mrs_lm *lm) {
     const LmHooks *bb = &lm->eng;
     // a warm, eager step (the GEMM library settles its choices), with the recurrent state and the tokens put back after it
     const size_t sbytes = bb->state_bytes(bb->self), tb = (size_t)lm->batch * sizeof(int);
+    const bool all_seen = !bb->seat || !bb->seat->unseen;
     void *save = nullptr;
     MRS_HIP(hipMalloc(&save, sbytes + tb));
     int rc = bb->state_copy(bb->self, save, 0);
@@ -1290,6 +1326,8 @@ extern "C" int mrs_lm_capture_graph(mrs_lm *lm) {
     hipStreamSynchronize(bb->stream);
     hipFree(save);
     if (rc) return rc;
+    if (all_seen && bb->go_on_chain) bb->go_on_chain(bb->self);
+    if (bb->check) MRS_TRY(bb->check(bb->self));
     const ResidentRecording rec(bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = lm_decode_body(lm);
@@ -1343,6 +1381,7 @@ extern "C" int mrs_lm_prefill(mrs_lm *lm, mrs_backbone *prefill_bb, const int *t
     }
     hipStreamSynchronize(eng->stream);
     hipFree(dtok);
+    if (!rc && eng->check) rc = eng->check(eng->self);   // (steps before it)
     return rc;
 }
 

@@ -667,15 +667,16 @@ void choose_resident3(mrs_m3_backbone *bb) {
     ResidentM3Args &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr;
-    if (bb->batch > 256 || !resident_m3_plan(a, bb->dtype) || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
+    if (bb->batch > kRollMax || !resident_m3_plan(a, bb->dtype) || a.G * a.batch > kRollMax || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
     bb->resident = 1;
 }
 
 int arm_resident3(mrs_m3_backbone *bb) {
     const ResidentM3Args &a = bb->res_args;
     MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
-    MRS_HIP(hipMemsetAsync(a.epoch, 0, (size_t)a.batch * 128, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4, bb->stream));
     *bb->res_broken = 0;
+    bb->seat.unseen = false;
     return MRS_OK;
 }
 
@@ -686,7 +687,9 @@ int setup_resident3(mrs_m3_backbone *bb) {
     a.input = bb->identity_proj ? bb->d_input : bb->residual;
     a.norm_f = bb->norm_f; a.ssm = bb->ssm; a.kst = bb->kst; a.vst = bb->vst; a.angle = bb->angle; a.temporal = bb->temporal;
     MRS_TRY(dev_alloc3(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
-    MRS_TRY(dev_alloc3(bb, (void **)&a.epoch, (size_t)a.batch * 128));
+    MRS_TRY(dev_alloc3(bb, (void **)&a.epoch, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4));
+    a.roll = a.epoch + (size_t)a.batch * 32;
+    a.wait = kResidentWait;
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident3(bb));
@@ -705,13 +708,23 @@ int setup_resident3(mrs_m3_backbone *bb) {
     return MRS_OK;
 }
 
-// After a synchronisation: whether every resident step found all its workgroups on the chip.
+// After a synchronisation: whether every resident step was carried out.
+unsigned resident_fault3(const mrs_m3_backbone *bb) { return bb->res_broken ? *(volatile unsigned *)bb->res_broken : 0; }
 int check_resident3(mrs_m3_backbone *bb) {
     resident_idle(bb->seat);
-    if (bb->res_broken && *(volatile unsigned *)bb->res_broken)
-        return fail(MRS_E_HIP, "resident decode step: workgroups gave up waiting for each other (is another process holding the GPU?); reset() the engine, "
-                               "or set MRS_DECODE_NO_RESIDENT=1");
+    if (const unsigned f = resident_fault3(bb))
+        return fail(MRS_E_HIP, "resident decode step: %s; reset() the engine, or set MRS_DECODE_NO_RESIDENT=1",
+                    f == kStepCalledOff ? "the GPU's compute units did not come free in time (other work or another process holds them), and no step since was carried out"
+                                        : "workgroups gave up waiting for each other");
+    bb->seat.unseen = false;
     return MRS_OK;
+}
+// After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until
+// a reset, the steps are kernel chains.
+bool go_on_chain3(mrs_m3_backbone *bb) {
+    if (resident_fault3(bb) != kStepCalledOff || arm_resident3(bb)) return false;
+    bb->seat.off = true;
+    return true;
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
@@ -786,7 +799,8 @@ extern "C" int mrs_m3_backbone_reset(mrs_m3_backbone *bb) {
     MRS_HIP(hipMemsetAsync(bb->kst, 0, L * B * nh * ds * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->vst, 0, L * B * nh * hd * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->angle, 0, L * B * nh * na * 4, bb->stream));
-    if (bb->res_broken && *(volatile unsigned *)bb->res_broken) {   // a resident step gave up: its exchange words start over with the state
+    bb->seat.off = false;
+    if (resident_fault3(bb)) {   // a resident step gave up: its exchange words start over with the state
         MRS_HIP(hipStreamSynchronize(bb->stream));
         return arm_resident3(bb);
     }
@@ -963,7 +977,8 @@ extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, flo
     const int B = bb->batch, dm = bb->cfg.d_model, n = B * bb->input_dim;
     HostIo &io = bb->io;
     memcpy(io.in, input, (size_t)n * 4);
-    const HostRows host = {io.out, io.done, ++io.seq};
+    HostRows host = {io.out, io.done, ++io.seq};
+    const bool all_seen = !bb->seat.unseen;
     if (bb->tiny_layers) {
         MRS_TRY(step_body3(bb, &host));
     } else {
@@ -973,6 +988,13 @@ extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, flo
         MRS_TRY(check_launch("host row kernels"));
     }
     MRS_TRY(host_io_wait(&io, bb->stream));
+    if (all_seen && go_on_chain3(bb)) {   // this very step found no places
+        host.seq = ++io.seq;
+        MRS_TRY(step_body3(bb));
+        hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
+        MRS_TRY(check_launch("host_out_kernel"));
+        MRS_TRY(host_io_wait(&io, bb->stream));
+    }
     memcpy(output, io.out, (size_t)B * dm * 4);
     return check_resident3(bb);
 }
@@ -984,6 +1006,7 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     if (bb->graph_ready) return MRS_OK;
     const size_t L = bb->cfg.n_layers, B = bb->batch, nh = bb->nh, hd = bb->cfg.headdim, ds = bb->cfg.d_state, na = bb->nr > 0 ? bb->nr : 1;
     const size_t n0 = L * B * nh * hd * ds * 4, n1 = L * B * nh * ds * 4, n2 = L * B * nh * hd * 4, n3 = L * B * nh * na * 4;
+    const bool all_seen = !bb->seat.unseen;
     char *save = nullptr;
     MRS_HIP(hipMalloc((void **)&save, n0 + n1 + n2 + n3));
     hipMemcpyAsync(save, bb->ssm, n0, hipMemcpyDeviceToDevice, bb->stream);
@@ -999,6 +1022,8 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     hipFree(save);
     if (rc) return rc;
     if (e != hipSuccess) return fail(MRS_E_HIP, "capture warm-up: %s", hipGetErrorString(e));
+    if (all_seen) go_on_chain3(bb);
+    MRS_TRY(check_resident3(bb));
     const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
     rc = step_body3(bb);
@@ -1272,7 +1297,7 @@ extern "C" int mrs_m3_backbone_prefill_sequence(mrs_m3_backbone *bb, const float
     MRS_TRY(prefill_body3(bb, T));
     if (out_last) MRS_HIP(hipMemcpyAsync(out_last, bb->temporal, (size_t)bb->batch * bb->cfg.d_model * 4, hipMemcpyDeviceToHost, bb->stream));
     MRS_HIP(hipStreamSynchronize(bb->stream));
-    return MRS_OK;
+    return check_resident3(bb);   // (steps before it)
 }
 
 extern "C" float *mrs_m3_backbone_prefill_input_ptr(mrs_m3_backbone *bb) { return bb ? bb->pf_in : nullptr; }
@@ -1282,6 +1307,14 @@ extern "C" int mrs_m3_backbone_temporal_dtype(mrs_m3_backbone *bb) { return bb ?
 extern "C" int mrs_m3_backbone_decode_route(mrs_m3_backbone *bb) {
     if (!bb) return -1;
     return bb->tiny_layers || bb->resident ? MRS_DECODE_ONE_LAUNCH : bb->skinny ? MRS_DECODE_OWN_CHAIN : MRS_DECODE_LIBRARY_CHAIN;
+}
+extern "C" int mrs_m3_backbone_set_resident_wait(mrs_m3_backbone *bb, unsigned polls) {
+    if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_set_resident_wait: null engine");
+    if (!bb->resident) return MRS_OK;
+    bb->res_args.wait = polls;
+    MRS_HIP(hipMemcpyAsync(bb->res_args_dev, &bb->res_args, sizeof(ResidentM3Args), hipMemcpyHostToDevice, bb->stream));
+    MRS_HIP(hipStreamSynchronize(bb->stream));
+    return MRS_OK;
 }
 extern "C" float *mrs_m3_backbone_input_ptr(mrs_m3_backbone *bb) { return bb ? bb->d_input : nullptr; }
 extern "C" void *mrs_m3_backbone_stream(mrs_m3_backbone *bb) { return bb ? (void *)bb->stream : nullptr; }
@@ -1312,6 +1345,7 @@ void m3_state_sizes(mrs_m3_backbone *bb, size_t (&n)[4]) {
     n[0] = L * B * nh * hd * ds * 4; n[1] = L * B * nh * ds * 4; n[2] = L * B * nh * hd * 4; n[3] = L * B * nh * na * 4;
 }
 int m3_hook_check(void *self) { return check_resident3((mrs_m3_backbone *)self); }
+bool m3_hook_go_on_chain(void *self) { return go_on_chain3((mrs_m3_backbone *)self); }
 int m3_hook_step(void *self) { return step_body3((mrs_m3_backbone *)self); }
 int m3_hook_reset(void *self) { return mrs_m3_backbone_reset((mrs_m3_backbone *)self); }
 size_t m3_hook_state_bytes(void *self) {
@@ -1348,6 +1382,6 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = nullptr;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
-    h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check;
+    h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check; h.go_on_chain = m3_hook_go_on_chain;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");
 }

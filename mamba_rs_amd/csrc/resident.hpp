@@ -11,9 +11,10 @@
 // rewritten only after every reader of its last contents has published something that depends on them: one buffer per
 // exchange is enough.
 //
-// Every wait is bounded (kSpinLimit polls, about two seconds): a workgroup that gives up leaves, the others follow, the
-// output rows become NaN and `broken` (host memory) is raised, which the engine turns into an error.  It does not happen as
-// long as all workgroups of a launch fit on the chip together, which the engine's slot budget sees to.
+// A launch begins with a roll call (RollCall): no workgroup stores anything but exchange words before all of them are on the chip.  Ordinary kernels that hold the compute units delay it.  If the units do not come free within the wait the caller set, the
+// launch is called off as a whole: the states are what they were, the output rows become NaN, `broken` (host memory) is raised, and
+// launches queued behind it leave at once.  After the roll call a wait is over when its neighbours have done their part; those waits
+// are bounded as well (kSpinLimit polls, about two seconds), and a workgroup that gives up there leaves the states unfinished.
 #pragma once
 #include "common.hpp"
 #include "mfma_tiles.hpp"
@@ -22,6 +23,76 @@ namespace mrs {
 
 typedef unsigned long long u64;
 constexpr unsigned kSpinLimit = 1u << 21;
+
+// The roll call, by one of the waves that bring weights.  roll[0]: a launch was called off or lost, its successors do not begin;
+// roll[1]: number of the launch; roll[2 + its parity]: the verdict; behind kRollHead words, one per workgroup: the number of the last
+// launch it has answered, plus one.  A workgroup goes on when it has seen all answers and, after that, no verdict against it.  One that has
+// waited `wait` polls (one to two microseconds each) in vain first puts kDoubt there and then looks at the answers again: whoever went on
+// without seeing the doubt had seen all of them before it, so they are all there now and it goes on as well; otherwise the launch
+// is called off.  So all workgroups take the same way, also those that get a place only when others have left.  A wait of 0 calls off
+// without an answer.
+// The answers are read while the first exchange is waited for: a step takes 1 to 2 us longer for it (24 layers of d_model 1024 270 ->
+// 272 us, four of 256 at eight rows 30.5 -> 32.5).  As a count on one word, added to and polled by 256 workgroups: 4 to 11 us.
+constexpr int kRollCall = -1;   // a workgroup's state: the roll call, 0 under way, or a ResidentFault
+constexpr unsigned kDoubt = 1, kGo = 2, kOff = 3;
+struct RollCall {
+    unsigned *roll, *broken;
+    unsigned all, wait, number;
+    static __device__ __forceinline__ unsigned get(const unsigned *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    static __device__ __forceinline__ void put(unsigned *p, unsigned v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    static __device__ __forceinline__ void done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }   // what was asked for before is there, what is asked for next comes after
+    __device__ __forceinline__ int answer() {
+        const u64 head = __hip_atomic_load(reinterpret_cast<u64 *>(roll), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        number = __builtin_amdgcn_readfirstlane((unsigned)(head >> 32));
+        if (__builtin_amdgcn_readfirstlane((unsigned)head)) return kStepCalledOff;
+        if (wait && (threadIdx.x & 63) == 0) put(roll + kRollHead + blockIdx.x, number + 1u);
+        return kRollCall;
+    }
+    __device__ __forceinline__ bool answered() const {
+        bool have = true;
+        unsigned r[kRollMax / 64];
+#pragma unroll
+        for (int k = 0; k < kRollMax / 64; k++) r[k] = get(roll + kRollHead + min((unsigned)(k * 64) + (threadIdx.x & 63u), all - 1u));
+#pragma unroll
+        for (int k = 0; k < kRollMax / 64; k++) have = have && r[k] == number + 1u;
+        const bool yes = __all(have);
+        done();
+        return yes;
+    }
+    __device__ __forceinline__ int outcome() const {
+        unsigned *verdict = roll + 2 + (number & 1u);
+        const bool first = (threadIdx.x & 63) == 0;
+#pragma unroll 1
+        for (unsigned spins = 0;; spins++) {
+            const bool yes = answered();
+            const unsigned v = __builtin_amdgcn_readfirstlane(get(verdict));
+            if (v == kOff) return kStepCalledOff;
+            if (yes && v != kDoubt) break;
+            if (v == 0 && spins >= wait) {
+                unsigned none = 0;
+                const bool mine = first && __hip_atomic_compare_exchange_strong(verdict, &none, kDoubt, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!__any(mine)) continue;
+                done();
+                const bool go = answered();
+                if (first) {
+                    if (!go) {
+                        put(roll, 1u);
+                        __hip_atomic_store(broken, (unsigned)kStepCalledOff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                    put(verdict, go ? kGo : kOff);
+                }
+                if (go) break;
+                return kStepCalledOff;
+            }
+            __builtin_amdgcn_s_sleep(4);
+        }
+        if (blockIdx.x == 0 && first) {   // everybody has read the number: the next launch's
+            put(roll + 2 + ((number + 1u) & 1u), 0u);
+            put(roll + 1, number + 1u);
+        }
+        return 0;
+    }
+};
 
 __device__ __forceinline__ void xch_put(u64 *p, float v, unsigned tag) {
     __hip_atomic_store(p, ((u64)tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -94,9 +165,10 @@ template <typename T> __device__ __forceinline__ u64 half_pair_word(T a, T b, un
 }
 __device__ __forceinline__ void xch_put_word(u64 *p, u64 w) { __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Polls the KU words base[idx(0)] .. base[idx(KU - 1)] until ready(word) holds for all of them.  False when the wait was given up.
+// Polls the KU words base[idx(0)] .. base[idx(KU - 1)] until ready(word) holds for all of them.  False when the wait was given up; the
+// first exchange of a step (`state`, else null) waits as long as the roll call is not over.
 template <int KU, class IDX, class READY>
-__device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, u64 (&r)[KU]) {
+__device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, u64 (&r)[KU], const volatile int *state = nullptr) {
     for (unsigned spins = 0; spins <= kSpinLimit; spins++) {
         bool have = true;
 #pragma unroll
@@ -104,6 +176,11 @@ __device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, 
 #pragma unroll
         for (int u = 0; u < KU; u++) have = have && ready(r[u]);
         if (have) return true;
+        if (state && (spins & 63u) == 63u) {
+            const int s = *state;
+            if (s > 0) return false;
+            if (s == kRollCall) spins = 0;
+        }
     }
     return false;
 }
@@ -167,15 +244,18 @@ struct WeightFeed {
     unsigned win, wout, small;    // LDS byte addresses; the small blocks of two layers lie one after the other
     int out, small_at, small_bytes;   // offsets in the block
 };
-__device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, const int &bad) {
+__device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, volatile int &state, RollCall call) {
     const char *blk = f.blk;
-    const bool out_wave = wave == 10, small_wave = wave == 11;
+    const bool first = (threadIdx.x & 63) == 0, out_wave = wave == 10, small_wave = wave == 11;
     const int iw = wave == 11 ? 2 : wave - 8, in_pieces = f.out >> 10, in_mid = in_pieces / 2, out_pieces = (f.small_at - f.out) >> 10;
     auto bring_in = [&](const char *p, int from, int to) { dma_to_lds(f.win, p, from + iw, to, 3); };
     auto bring_out = [&](const char *p) { dma_to_lds(f.wout, p + f.out, 0, out_pieces, 1); };
     auto bring_small = [&](const char *p, int l) { dma_to_lds(f.small + (l & 1) * f.small_bytes, p + f.small_at, 0, f.small_bytes >> 10, 1); };
-    if (out_wave) bring_out(blk);
-    else bring_in(blk, 0, in_pieces);
+    if (out_wave) {
+        const int s = call.answer();
+        if (first) state = s;
+        bring_out(blk);
+    } else bring_in(blk, 0, in_pieces);
     if (small_wave) bring_small(blk, 0);
     if (!out_wave) dma_wait();
     lds_barrier();   // layer 0's row is there
@@ -186,17 +266,23 @@ __device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int 
         lds_barrier();   // 1
         if (small_wave && more) bring_small(blk, l + 1);
         if (!out_wave && more) bring_in(blk, 0, in_mid);
-        if (out_wave) dma_wait();
+        if (out_wave) {
+            if (l == 0 && state == kRollCall) {
+                const int s = call.outcome();
+                if (first) state = s;
+            }
+            dma_wait();
+        }
         lds_barrier();   // 2
-        if (bad) return;
+        if (state) return;
         if (!out_wave && more) bring_in(blk, in_mid, in_pieces);
         lds_barrier();   // 3
-        if (bad) return;
+        if (state) return;
         if (!out_wave) dma_wait();
         lds_barrier();   // 4
         if (out_wave && more) bring_out(blk);
         lds_barrier();   // 5
-        if (bad) return;
+        if (state) return;
     }
 }
 

@@ -66,7 +66,7 @@ bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t 
     }
     if (!g.ours || workgroups > g.places) return false;
     try { g.seats.push_back(&seat); } catch (...) { return false; }
-    seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = false;
+    seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = seat.unseen = seat.off = false;
     g.live += workgroups;
     return true;
 }
@@ -93,6 +93,7 @@ ResidentTurn::ResidentTurn(ResidentSeat *seat) : seat_(seat), go_(true) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(seat->stream, &cap) != hipSuccess) { go_ = false; return; }
     if (cap != hipStreamCaptureStatusNone) { go_ = seat->recording; return; }   // recorded, not run
+    if (seat->off) { go_ = false; return; }
     Gate &g = g_gates[seat->device];
     g.m.lock();
     if (g.live > g.places) {
@@ -110,7 +111,7 @@ ResidentTurn::ResidentTurn(ResidentSeat *seat) : seat_(seat), go_(true) {
 ResidentTurn::~ResidentTurn() {
     if (!locked_) return;
     Gate &g = g_gates[seat_->device];
-    seat_->open = true;
+    seat_->open = seat_->unseen = true;
     if (g.live > g.places) {
         if (hipEventRecord(g.event, seat_->stream) == hipSuccess) {
             seat_->open = false;

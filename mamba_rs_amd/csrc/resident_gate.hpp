@@ -10,6 +10,8 @@ struct ResidentSeat {
     hipStream_t stream = nullptr;      // the engine's stream
     bool open = false;                 // launches that no event covers and that the host has not waited for
     bool recording = false;            // the engine captures a step for itself
+    bool unseen = false;               // launches whose fault word the host has not looked at
+    bool off = false;                  // a launch was called off: kernel chains until the engine is reset
 };
 bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t stream);
 void resident_release(ResidentSeat &seat);   // the engine has waited for its stream

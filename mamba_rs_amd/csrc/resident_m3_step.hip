@@ -66,20 +66,20 @@ __host__ __device__ inline ResLds res_lds(int dm, int di, int cols, int oc, int 
 template <typename T>
 __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const ResidentM3Args *args) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    __shared__ int bad;
+    __shared__ int state_word;
+    volatile int &state = state_word;   // kRollCall, 0, or a ResidentFault
     const auto *a = as_table(args);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = a->G, b = blockIdx.x / G, src = blockIdx.x - b * G;
     const int dm = a->dm, di = a->di, nl = a->n_layers, nc = a->nc, oc = a->oc, ex = a->ex, ds = a->ds, nh = a->nh, hd = a->hd, ng = a->ng, nr = a->nr;
     const int c0 = src * nc, o0 = src * oc, cols = 2 * nc + ex;
     const ResLds L = res_lds(dm, di, cols, oc, ds);
     const SmallBlock sb = small_block(ds, oc);
-    if (tid == 0) bad = 0;
 
     if (wave >= kComputeWaves) {
         const LayerBlock lb = layer_block(dm, di, cols, oc, ds);
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         bring_weights({(const char *)a->weights + (size_t)src * lb.bytes, (size_t)G * lb.bytes, lds0 + L.win, lds0 + L.wout, lds0 + L.small, lb.out, lb.small,
-                       sb.bytes}, wave, nl, bad);
+                       sb.bytes}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
         return;
     }
 
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
             // the accumulated angle (f64, wrapped); a lane per coordinate
             const int n = min(here(lane), ds - 1), at = (wave == 0 ? grp : ng + grp) * ds + n, sc = 2 * ng * ds;
             u64 r[3];
-            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(u == 0 ? at : u == 1 ? sc + head : nr > 0 ? sc + 3 * nh + pair : at); }, tagged, r);
+            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(u == 0 ? at : u == 1 ? sc + head : nr > 0 ? sc + 3 * nh + pair : at); }, tagged, r, &state);
             const float raw = __uint_as_float((unsigned)r[0]);
             const float *nw = reinterpret_cast<const float *>(small + (wave == 0 ? sb.bnw : sb.cnw)), *bias = reinterpret_cast<const float *>(small + (wave == 0 ? sb.bb : sb.cb));
             const float sq = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wave_sum_last(here(lane) < ds ? raw * raw : 0.0f)), 63));
@@ -175,15 +175,15 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
             // ---- alpha, beta, gamma of the head
             const int sc = 2 * ng * ds + head;
             u64 r[3];
-            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(sc + u * nh); }, tagged, r);
+            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(sc + u * nh); }, tagged, r, &state);
             const float dtv = softplus20(__uint_as_float((unsigned)r[0]) + *reinterpret_cast<const float *>(small + sb.dtb));
             const float a_val = fminf(-heavy_tail(__uint_as_float((unsigned)r[1])), -a->a_floor), trap = sigmoidf_fast(__uint_as_float((unsigned)r[2]));
             const float al = fast_exp2(a_val * dtv * kLog2e);
             if (lane == 0) *reinterpret_cast<float4 *>(coef) = make_float4(al, al * dtv * (1.0f - trap), trap * dtv, 0.0f);
         }
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         lds_barrier();   // 2
-        if (bad) break;
+        if (state) break;
         // ---- trapezoidal update of this lane's four states, y = H q + D x, SiLU gate
         float4 kc = make_float4(0.f, 0.f, 0.f, 0.f);
         if (scans) {
@@ -214,9 +214,9 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
         // ---- y of all channels
         pout.take(wout, oc, di >> 5, 1);   // while y is on its way
         ok = take_y(e3, di, tag, ys) && ok;
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         lds_barrier();   // 3
-        if (bad) break;
+        if (state) break;
         // every workgroup of the head has used the previous k and angles for the y that is now here
         if (head_owner) {
             if (scans && p == 0) *reinterpret_cast<float4 *>(kst + l * kst_l + 4 * g) = kc;
@@ -228,12 +228,12 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
         put_operand<T>(pre2, oc, o0, src, more ? reinterpret_cast<const float *>(small + sb.nw) : nullptr, e1, e1s, tag, res0, res1);
         if (more) pin.take(win, cols, dm >> 5, ct_in);   // while the operand row is on its way
         ok = take_operand(e1, e1s, G, dm, a->eps, tag, more, xs, invl) && ok;
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         lds_barrier();   // 5
-        if (bad) break;
+        if (state) break;
     }
     // final norm of this workgroup's columns
-    const bool lost = bad != 0;
+    const bool lost = state != 0;
     if (own) {
         const float inv = invl[0];
 #pragma unroll
@@ -243,7 +243,10 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
         }
     }
     if (tid == 0) {
-        if (lost) __hip_atomic_store(a->broken, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (state == kStepLost) {
+            __hip_atomic_store(a->roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a->broken, (unsigned)kStepLost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         if (src == 0) *epoch = base + nl;   // every workgroup of the row has read it: each has published the last exchange
     }
 }
@@ -340,8 +343,8 @@ static int launch_resident_m3_t(hipStream_t st, const ResidentM3Args &a, const R
 }
 
 int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev) {
-    if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.n_layers < 1 || !a.weights || !a.norm_w || !a.norm_f || !a.input || !a.xch || !a.epoch ||
-        !a.broken || !a.temporal || !a.ssm || !a.kst || !a.vst || !a.angle || !dev)
+    if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.G * a.batch > kRollMax || a.n_layers < 1 || !a.weights || !a.norm_w || !a.norm_f || !a.input || !a.xch || !a.epoch ||
+        !a.roll || !a.broken || !a.temporal || !a.ssm || !a.kst || !a.vst || !a.angle || !dev)
         return fail(MRS_E_SHAPE, "resident Mamba-3 step: shape outside the route (d_model=%d d_inner=%d d_state=%d workgroups=%d)", a.dm, a.di, a.ds, a.G);
     return dtype == MRS_BF16 ? launch_resident_m3_t<bf16_t>(st, a, dev) : launch_resident_m3_t<f16_t>(st, a, dev);
 }

@@ -69,20 +69,20 @@ __host__ __device__ inline ResLds res_lds(int dm, int di, int nc, int oc, int xd
 template <typename T>
 __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const ResidentArgs *args) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    __shared__ int bad;
+    __shared__ int state_word;
+    volatile int &state = state_word;   // kRollCall, 0, or a ResidentFault
     const auto *a = as_table(args);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = a->G, b = blockIdx.x / G, src = blockIdx.x - b * G;
     const int dm = a->dm, di = a->di, nl = a->n_layers, nc = a->nc, oc = a->oc, xd = a->xd, dr = a->dr;
     const int c0 = src * nc, o0 = src * oc;
     const ResLds L = res_lds(dm, di, nc, oc, xd, dr);
     const SmallBlock sb = small_block(nc, oc, xd, dr);
-    if (tid == 0) bad = 0;
 
     if (wave >= kComputeWaves) {
         const LayerBlock lb = layer_block(dm, di, nc, oc, xd, dr);
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         bring_weights({(const char *)a->weights + (size_t)src * lb.bytes, (size_t)G * lb.bytes, lds0 + L.win, lds0 + L.wout, lds0 + L.small, lb.out, lb.small,
-                       sb.bytes}, wave, nl, bad);
+                       sb.bytes}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
         return;
     }
 
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
                 for (int k0 = g; k0 < G; k0 += 8 * KU) {
                     u64 r[KU];
                     ok = ok && xch_poll<KU>(e2, [&](int u) { return (unsigned)(min(k0 + 8 * u, G - 1) * hx + q); },
-                                            [&](u64 w) { return (((unsigned)w ^ tag) & 1u) == 0 && (((unsigned)(w >> 32) ^ tag) & 1u) == 0; }, r);
+                                            [&](u64 w) { return (((unsigned)w ^ tag) & 1u) == 0 && (((unsigned)(w >> 32) ^ tag) & 1u) == 0; }, r, &state);
 #pragma unroll
                     for (int u = 0; u < KU; u++) {
                         const bool in = k0 + 8 * u < G;
@@ -196,9 +196,9 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
                 if (g == 0) *reinterpret_cast<float2 *>(xdl + 2 * q) = make_float2(Store<T>::ld(&r0), Store<T>::ld(&r1));
             }
         }
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         lds_barrier();   // 2
-        if (bad) break;
+        if (state) break;
         // the window, by the first wave: all waves have theirs in registers, they have used it in front of the barrier
         if (wave == 0 && lane < nc) *reinterpret_cast<float4 *>(cst + l * cst_l + lane * kDc) = make_float4(cwin.y, cwin.z, cwin.w, xnew);
         // ---- dt_proj + softplus, state update, D skip, gate: sixteen lanes per channel, one state each
@@ -228,22 +228,22 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         // ---- y of all channels
         pout.take(wout, oc, di >> 5, 1);   // while y is on its way
         ok = take_y(e3, di, tag, ys) && ok;
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         if (more && conv_wave) cwin = ld_off<float4>(cst + (l + 1) * cst_l, (unsigned)min(here(lane), nc - 1) * 16u);
         lds_barrier();   // 3
-        if (bad) break;
+        if (state) break;
         // ---- out_proj, residual, the next operand
         pout.run(ys, di >> 5, 1, pre2);
         lds_barrier();   // 4
         put_operand<T>(pre2, oc, o0, src, more ? reinterpret_cast<const float *>(small + sb.nw) : nullptr, e1, e1s, tag, res0, res1);
         if (more) pin.take(win, 2 * nc, dm >> 5, ct_in);   // while the operand row is on its way
         ok = take_operand(e1, e1s, G, dm, a->eps, tag, more, xs, invl) && ok;
-        if (!ok) bad = 1;
+        if (!ok && state == 0) state = kStepLost;
         lds_barrier();   // 5
-        if (bad) break;
+        if (state) break;
     }
     // final norm of this workgroup's columns: f32, and once more in the storage type for a head
-    const bool lost = bad != 0;
+    const bool lost = state != 0;
     if (own) {
         const float inv = invl[0];
 #pragma unroll
@@ -255,7 +255,10 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
         }
     }
     if (tid == 0) {
-        if (lost) __hip_atomic_store(a->broken, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (state == kStepLost) {
+            __hip_atomic_store(a->roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a->broken, (unsigned)kStepLost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         if (src == 0) *epoch = base + nl;   // every workgroup of the row has read it: each has published the last exchange
     }
 }
@@ -349,7 +352,7 @@ static int launch_resident_t(hipStream_t st, const ResidentArgs &a, const Reside
 }
 
 int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev) {
-    if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.n_layers < 1 || !a.weights || !a.norm_w || !a.input || !a.xch || !a.epoch || !a.broken ||
+    if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.G * a.batch > kRollMax || a.n_layers < 1 || !a.weights || !a.norm_w || !a.input || !a.xch || !a.epoch || !a.roll || !a.broken ||
         !a.temporal || !a.temporal_t || !dev)
         return fail(MRS_E_SHAPE, "resident step: shape outside the route (d_model=%d d_inner=%d d_state=%d workgroups=%d)", a.dm, a.di, a.ds, a.G);
     return dtype == MRS_BF16 ? launch_resident_t<bf16_t>(st, a, dev) : launch_resident_t<f16_t>(st, a, dev);

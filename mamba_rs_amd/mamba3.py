@@ -7,7 +7,7 @@ reference's deterministic initialiser so that synthetic models can be built with
 from __future__ import annotations
 
 import math
-from ctypes import POINTER, Structure, byref, c_float, c_int, c_void_p
+from ctypes import POINTER, Structure, byref, c_float, c_int, c_uint, c_void_p
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -198,6 +198,7 @@ def _bind():
         "mrs_m3_backbone_temporal_ptr": (P, [P]),
         "mrs_m3_backbone_temporal_dtype": (c_int, [P]),
         "mrs_m3_backbone_decode_route": (c_int, [P]),
+        "mrs_m3_backbone_set_resident_wait": (c_int, [P, c_uint]),
         "mrs_m3_backbone_input_ptr": (P, [P]),
         "mrs_m3_backbone_stream": (P, [P]),
         "mrs_m3_backbone_sync": (c_int, [P]),
@@ -328,6 +329,10 @@ class GpuMamba3Backbone:
     def decode_route(self) -> int:
         """0: chain on the vendor GEMM, 1: the library's own fused chain, 2: a whole step in one launch."""
         return _bind().mrs_m3_backbone_decode_route(self._h)
+
+    def set_resident_wait(self, polls: int):
+        """As GpuMambaBackbone.set_resident_wait."""
+        _call("mrs_m3_backbone_set_resident_wait", self._h, polls)
 
     def input_ptr(self) -> int:
         return _bind().mrs_m3_backbone_input_ptr(self._h)

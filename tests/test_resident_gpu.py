@@ -148,22 +148,26 @@ def test_an_engine_captures_while_another_one_steps():
     b.close()
 
 
+def _family(family):
+    """(a constructor of engines of four rows on the same weights, d_model, the language model class) of either network."""
+    from mamba_rs_amd import GpuMamba3Backbone, GpuMamba3LM, GpuMambaLM
+    if family == "m1":
+        return lambda: _engines((768, 3, 4), 1)[0], 768, GpuMambaLM
+    from test_m3_engine_gpu import perturbed
+    from test_resident_m3_gpu import cfg_
+    cfg = cfg_(256, 16, 16, 1, 3)
+    w = perturbed(cfg, 256, 11)
+    w.input_proj_w = np.zeros(0, np.float32)
+    return lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, 4, WeightDtype.BF16), 256, GpuMamba3LM
+
+
 @pytest.mark.parametrize("family", ["m1", "m3"])
 def test_a_caller_s_capture_gets_the_kernel_chain(family, monkeypatch):
     """step_gpu_only and a language model's decode_step captured by the caller on the engine's stream: the graph holds the kernel
     chain (its replays take no turns), so every replay, with eager work in between, leaves the bits of an engine that has only the
     chain; the engine's own steps are resident before and after."""
     import torch
-    from mamba_rs_amd import GpuMambaLM, GpuMamba3Backbone, GpuMamba3LM
-    if family == "m1":
-        make, lm_of, dm = lambda: _engines((768, 3, 4), 1)[0], GpuMambaLM, 768
-    else:
-        from test_m3_engine_gpu import perturbed
-        from test_resident_m3_gpu import cfg_
-        cfg, dm = cfg_(256, 16, 16, 1, 3), 256
-        w = perturbed(cfg, dm, 11)
-        w.input_proj_w = np.zeros(0, np.float32)
-        make, lm_of = lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, 4, WeightDtype.BF16), GpuMamba3LM
+    make, dm, lm_of = _family(family)
     a = make()
     monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
     chain = make()
@@ -233,3 +237,71 @@ def test_conv_windows_move_by_one_step(dm, B):
             old[l] = new
     a.close()
     b.close()
+
+
+def _states(e):
+    """All recurrent states, whatever the engine's check says."""
+    from mamba_rs_amd import backbone, mamba3
+    out = []
+    for l in range(e.cfg.n_layers):
+        if isinstance(e, GpuMambaBackbone):
+            parts = [np.empty((e.batch, e.cfg.d_inner(), n), np.float32) for n in (e.cfg.d_conv, e.cfg.d_state)]
+            backbone._bind().mrs_backbone_download_state(e._h, l, *map(backbone._fp, parts))
+        else:
+            nh, hd, ds = e.cfg.nheads(), e.cfg.headdim, e.cfg.d_state
+            na = max(1, e.cfg.num_rope_angles())
+            parts = [np.empty((e.batch, *n), np.float32) for n in ((nh, hd, ds), (nh, ds), (nh, hd), (nh, na))]
+            mamba3._bind().mrs_m3_backbone_download_state(e._h, l, *map(backbone._fp, parts))
+        out += parts
+    return out
+
+
+@pytest.mark.parametrize("family", ["m1", "m3"])
+def test_a_step_that_finds_no_places(family, monkeypatch):
+    """A wait of 0 calls every resident launch off.  step() then has the kernel chain's bits, from whatever state it started in; queued
+    steps leave the state alone and raise at the next call that waits for them, however many there are; after a reset the engine
+    steps as before."""
+    from mamba_rs_amd import MambaHipError
+    make, dm, lm_of = _family(family)
+    a = make()
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = make()
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((4, 4, dm)).astype(np.float32)
+    print(f"case called off {family}", flush=True)
+    lm = lm_of(a, rng.standard_normal((128, dm)).astype(np.float32))
+    resident = [a.step(r) for r in x]
+    before = _states(a)
+
+    a.set_resident_wait(0)
+    for _ in range(50):
+        a.step_gpu_only()
+    for _ in range(2):                      # it stays an error
+        with pytest.raises(MambaHipError, match="did not come free"):
+            a.sync()
+    with pytest.raises(MambaHipError, match="did not come free"):
+        a.step(x[0])
+    assert all(np.array_equal(p, q) for p, q in zip(before, _states(a)))
+
+    a.reset()
+    for r in x:                             # called off each time the engine was reset, else on the chain at once
+        assert np.array_equal(a.step(r), chain.step(r))
+    assert all(np.array_equal(p, q) for p, q in zip(_states(a), _states(chain)))
+    a.step_gpu_only()
+    a.sync()
+    a.reset()
+    lm.set_tokens(np.arange(4, dtype=np.int32))
+    lm.capture_graph()                      # its warm-up step is called off: the replays are kernel chains until a reset
+    lm.decode_step()
+    assert np.isfinite(lm.last_logits()).all()
+    a.reset()
+    lm.decode_step()
+    with pytest.raises(MambaHipError, match="did not come free"):
+        lm.get_tokens()
+
+    a.reset()
+    a.set_resident_wait(1 << 23)
+    for r, want in zip(x, resident):
+        assert np.array_equal(a.step(r), want)
+    for e in (lm, a, chain):
+        e.close()
