@@ -666,12 +666,30 @@ static int setup_resident(mrs_backbone *bb) {
 static unsigned resident_fault(const mrs_backbone *bb) { return bb->res_broken ? *(volatile unsigned *)bb->res_broken : 0; }
 static int check_resident(mrs_backbone *bb) {
     resident_idle(bb->seat);
-    if (const unsigned f = resident_fault(bb))
+    if (const unsigned f = resident_fault(bb)) {
+        bb->seat.told = true;
         return fail(MRS_E_HIP, "resident decode step: %s; reset() the engine, or set MRS_DECODE_NO_RESIDENT=1",
                     f == kStepCalledOff ? "the GPU's compute units did not come free in time (other work or another process holds them), and no step since was carried out"
                                         : "workgroups gave up waiting for each other");
+    }
     bb->seat.unseen = false;
     return MRS_OK;
+}
+// A reset waits for the steps in front of it (one of them may still give up): their exchange words start over with the state.  An error if
+// the caller has not heard of their loss yet.
+static int restart_resident(mrs_backbone *bb) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (!bb->resident) return MRS_OK;
+    MRS_HIP(hipStreamIsCapturing(bb->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return MRS_OK;   // a caller's graph: its steps are kernel chains
+    MRS_HIP(hipStreamSynchronize(bb->stream));
+    resident_idle(bb->seat);
+    bb->seat.off = bb->seat.unseen = false;
+    if (!resident_fault(bb)) return MRS_OK;
+    MRS_TRY(arm_resident(bb));
+    const bool told = bb->seat.told;
+    bb->seat.told = false;
+    return told ? MRS_OK : fail(MRS_E_HIP, "reset: steps queued before it were not carried out (resident decode step); the engine has been reset");
 }
 // After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until
 // a reset, the steps are kernel chains.
@@ -870,15 +888,11 @@ extern "C" void mrs_backbone_destroy(mrs_backbone *bb) {
 
 extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_reset: null engine");
+    const int lost = restart_resident(bb);
     const size_t L = bb->cfg.n_layers, B = bb->batch;
     MRS_HIP(hipMemsetAsync(bb->conv_state, 0, L * B * bb->di * bb->cfg.d_conv * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->ssm_state, 0, L * B * bb->di * bb->cfg.d_state * 4, bb->stream));
-    bb->seat.off = false;
-    if (resident_fault(bb)) {   // a resident step gave up: its exchange words start over with the state
-        MRS_HIP(hipStreamSynchronize(bb->stream));
-        return arm_resident(bb);
-    }
-    return MRS_OK;
+    return lost;
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null

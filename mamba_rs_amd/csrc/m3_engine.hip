@@ -712,12 +712,30 @@ int setup_resident3(mrs_m3_backbone *bb) {
 unsigned resident_fault3(const mrs_m3_backbone *bb) { return bb->res_broken ? *(volatile unsigned *)bb->res_broken : 0; }
 int check_resident3(mrs_m3_backbone *bb) {
     resident_idle(bb->seat);
-    if (const unsigned f = resident_fault3(bb))
+    if (const unsigned f = resident_fault3(bb)) {
+        bb->seat.told = true;
         return fail(MRS_E_HIP, "resident decode step: %s; reset() the engine, or set MRS_DECODE_NO_RESIDENT=1",
                     f == kStepCalledOff ? "the GPU's compute units did not come free in time (other work or another process holds them), and no step since was carried out"
                                         : "workgroups gave up waiting for each other");
+    }
     bb->seat.unseen = false;
     return MRS_OK;
+}
+// A reset waits for the steps in front of it (one of them may still give up): their exchange words start over with the state.  An error if
+// the caller has not heard of their loss yet.
+int restart_resident3(mrs_m3_backbone *bb) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (!bb->resident) return MRS_OK;
+    MRS_HIP(hipStreamIsCapturing(bb->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return MRS_OK;   // a caller's graph: its steps are kernel chains
+    MRS_HIP(hipStreamSynchronize(bb->stream));
+    resident_idle(bb->seat);
+    bb->seat.off = bb->seat.unseen = false;
+    if (!resident_fault3(bb)) return MRS_OK;
+    MRS_TRY(arm_resident3(bb));
+    const bool told = bb->seat.told;
+    bb->seat.told = false;
+    return told ? MRS_OK : fail(MRS_E_HIP, "reset: steps queued before it were not carried out (resident decode step); the engine has been reset");
 }
 // After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until
 // a reset, the steps are kernel chains.
@@ -794,17 +812,13 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
 
 extern "C" int mrs_m3_backbone_reset(mrs_m3_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_reset: null engine");
+    const int lost = restart_resident3(bb);
     const size_t L = bb->cfg.n_layers, B = bb->batch, nh = bb->nh, hd = bb->cfg.headdim, ds = bb->cfg.d_state, na = bb->nr > 0 ? bb->nr : 1;
     MRS_HIP(hipMemsetAsync(bb->ssm, 0, L * B * nh * hd * ds * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->kst, 0, L * B * nh * ds * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->vst, 0, L * B * nh * hd * 4, bb->stream));
     MRS_HIP(hipMemsetAsync(bb->angle, 0, L * B * nh * na * 4, bb->stream));
-    bb->seat.off = false;
-    if (resident_fault3(bb)) {   // a resident step gave up: its exchange words start over with the state
-        MRS_HIP(hipStreamSynchronize(bb->stream));
-        return arm_resident3(bb);
-    }
-    return MRS_OK;
+    return lost;
 }
 
 extern "C" void mrs_m3_backbone_destroy(mrs_m3_backbone *bb) {

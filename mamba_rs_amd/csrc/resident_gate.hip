@@ -66,7 +66,7 @@ bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t 
     }
     if (!g.ours || workgroups > g.places) return false;
     try { g.seats.push_back(&seat); } catch (...) { return false; }
-    seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = seat.unseen = seat.off = false;
+    seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = seat.unseen = seat.off = seat.told = false;
     g.live += workgroups;
     return true;
 }

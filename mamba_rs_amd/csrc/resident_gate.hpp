@@ -12,6 +12,7 @@ struct ResidentSeat {
     bool recording = false;            // the engine captures a step for itself
     bool unseen = false;               // launches whose fault word the host has not looked at
     bool off = false;                  // a launch was called off: kernel chains until the engine is reset
+    bool told = false;                 // the caller has had the error for a fault
 };
 bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t stream);
 void resident_release(ResidentSeat &seat);   // the engine has waited for its stream

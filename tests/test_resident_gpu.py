@@ -305,3 +305,28 @@ def test_a_step_that_finds_no_places(family, monkeypatch):
         assert np.array_equal(a.step(r), want)
     for e in (lm, a, chain):
         e.close()
+
+
+@pytest.mark.parametrize("family", ["m1", "m3"])
+def test_a_reset_waits_for_the_steps_before_it(family):
+    """Steps that are called off while a reset is already asked for: the reset waits for them, says once that they were lost, and the
+    engine steps as a fresh one; a second reset has nothing to say."""
+    from mamba_rs_amd import MambaHipError
+    make, dm, _ = _family(family)
+    a = make()
+    x = np.random.default_rng(7).standard_normal((4, dm)).astype(np.float32)
+    print(f"case reset behind lost steps {family}", flush=True)
+    want = a.step(x)
+    a.reset()
+    for _ in range(3):
+        a.set_resident_wait(0)
+        for _ in range(20):
+            a.step_gpu_only()
+        with pytest.raises(MambaHipError, match="not carried out"):
+            a.reset()
+        a.set_resident_wait(1 << 23)
+        assert np.array_equal(a.step(x), want)
+        a.reset()
+        assert np.array_equal(a.step(x), want)
+        a.reset()
+    a.close()
