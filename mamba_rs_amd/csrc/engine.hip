@@ -626,7 +626,7 @@ static int arm_resident(mrs_backbone *bb) {
     MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
     MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4, bb->stream));
     *bb->res_broken = 0;
-    bb->seat.unseen = false;
+    bb->seat.unseen = bb->seat.told = false;
     return MRS_OK;
 }
 
@@ -686,9 +686,8 @@ static int restart_resident(mrs_backbone *bb) {
     resident_idle(bb->seat);
     bb->seat.off = bb->seat.unseen = false;
     if (!resident_fault(bb)) return MRS_OK;
-    MRS_TRY(arm_resident(bb));
     const bool told = bb->seat.told;
-    bb->seat.told = false;
+    MRS_TRY(arm_resident(bb));
     return told ? MRS_OK : fail(MRS_E_HIP, "reset: steps queued before it were not carried out (resident decode step); the engine has been reset");
 }
 // After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until
@@ -1442,9 +1441,10 @@ static int gen_forward(mrs_lm *lm) {
 }
 
 // The generation loop behind mrs_lm_generate_batch and mrs_lm_generate_streaming.  With a callback (batch 1) the host
-// looks at the slot after every step instead of every 16th and hands each new token over as it appears.
-static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const mrs_sample_params *params, int seen_includes_prompt,
-                   int *out_tokens, int out_stride, int *out_lens, mrs_token_callback cb, void *user) {
+// looks at the slot after every step instead of every 16th and hands each new token over as it appears (*handed: how many).  on_chain:
+// every step is the kernel chain.
+static int gen_loop(mrs_lm *lm, const int *prompts, const int *prompt_lens, const mrs_sample_params *params, int seen_includes_prompt,
+                    int *out_tokens, int out_stride, int *out_lens, mrs_token_callback cb, void *user, bool on_chain, int *handed) {
     if (!lm || !prompt_lens || !params || !out_tokens || !out_lens) return fail(MRS_E_NULL, "mrs_lm_generate_batch: null pointer");
     const LmHooks *bb = &lm->eng;
     hipStream_t st = bb->stream;
@@ -1516,6 +1516,7 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
         hipLaunchKernelGGL(gen_seen_prompt_kernel, dim3((unsigned)std::min(64, (max_prompt + 255) / 256), (unsigned)B), dim3(256), 0, st, lm->gen,
                            lm->gen_dyn, B, lm->vocab);
     MRS_TRY(bb->reset(bb->self));
+    if (on_chain && bb->seat) bb->seat->off = true;
     int steps = max_prompt + max_tokens;   // gpu_lm.rs:432
     if (prefill_route && running) {
         MRS_TRY(mrs_lm_prefill(lm, nullptr, prompts, prompt_lens[0]));   // state after the prompt, logits of its last position
@@ -1556,14 +1557,16 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
             if (emitted < lm->gen_dyn_host.out_stride)
                 MRS_HIP(hipMemcpyAsync(&tok, lm->gen_dyn_host.out + emitted, sizeof(int), hipMemcpyDeviceToHost, st));
             MRS_HIP(hipStreamSynchronize(st));
+            if (bb->check) MRS_TRY(bb->check(bb->self));   // no token of a step that was not carried out leaves
             ++done;
             if (olen_now > emitted) {
-                emitted++;
+                *handed = ++emitted;
                 if (cb(tok, user) != 0) { stopped = true; break; }   // the caller has seen enough
             }
         } else if (++done % 16 == 0 || s + 1 == steps) {   // the only host round trip of the loop: is anyone still running?
             MRS_HIP(hipMemcpyAsync(&running, lm->gen.n_running, sizeof(int), hipMemcpyDeviceToHost, st));
             MRS_HIP(hipStreamSynchronize(st));
+            if (bb->check) MRS_TRY(bb->check(bb->self));
         }
     }
     MRS_HIP(hipMemcpyAsync(out_lens, lm->gen.out_len, (size_t)B * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1579,6 +1582,15 @@ static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const
             if (cb(out_tokens[emitted], user) != 0) { out_lens[0] = emitted + 1; break; }
     }
     return MRS_OK;
+}
+
+// Where resident steps were called off before a token left, the kernel chain does the whole generation.
+static int gen_run(mrs_lm *lm, const int *prompts, const int *prompt_lens, const mrs_sample_params *params, int seen_includes_prompt,
+                   int *out_tokens, int out_stride, int *out_lens, mrs_token_callback cb, void *user) {
+    int handed = 0;
+    const int rc = gen_loop(lm, prompts, prompt_lens, params, seen_includes_prompt, out_tokens, out_stride, out_lens, cb, user, false, &handed);
+    if (rc != MRS_E_HIP || handed || hipStreamSynchronize(lm->eng.stream) != hipSuccess || !lm->eng.go_on_chain(lm->eng.self)) return rc;
+    return gen_loop(lm, prompts, prompt_lens, params, seen_includes_prompt, out_tokens, out_stride, out_lens, cb, user, true, &handed);
 }
 
 extern "C" int mrs_lm_generate_batch(mrs_lm *lm, const int *prompts, const int *prompt_lens, const mrs_sample_params *params,

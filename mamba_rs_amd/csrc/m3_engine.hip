@@ -676,7 +676,7 @@ int arm_resident3(mrs_m3_backbone *bb) {
     MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
     MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4, bb->stream));
     *bb->res_broken = 0;
-    bb->seat.unseen = false;
+    bb->seat.unseen = bb->seat.told = false;
     return MRS_OK;
 }
 
@@ -732,9 +732,8 @@ int restart_resident3(mrs_m3_backbone *bb) {
     resident_idle(bb->seat);
     bb->seat.off = bb->seat.unseen = false;
     if (!resident_fault3(bb)) return MRS_OK;
-    MRS_TRY(arm_resident3(bb));
     const bool told = bb->seat.told;
-    bb->seat.told = false;
+    MRS_TRY(arm_resident3(bb));
     return told ? MRS_OK : fail(MRS_E_HIP, "reset: steps queued before it were not carried out (resident decode step); the engine has been reset");
 }
 // After a synchronisation, where only one launch can have gone wrong: was it called off?  It has changed nothing; from here on, until

@@ -148,17 +148,17 @@ def test_an_engine_captures_while_another_one_steps():
     b.close()
 
 
-def _family(family):
-    """(a constructor of engines of four rows on the same weights, d_model, the language model class) of either network."""
+def _family(family, rows=4):
+    """(a constructor of engines of so many rows on the same weights, d_model, the language model class) of either network."""
     from mamba_rs_amd import GpuMamba3Backbone, GpuMamba3LM, GpuMambaLM
     if family == "m1":
-        return lambda: _engines((768, 3, 4), 1)[0], 768, GpuMambaLM
+        return lambda: _engines((768, 3, rows), 1)[0], 768, GpuMambaLM
     from test_m3_engine_gpu import perturbed
     from test_resident_m3_gpu import cfg_
     cfg = cfg_(256, 16, 16, 1, 3)
     w = perturbed(cfg, 256, 11)
     w.input_proj_w = np.zeros(0, np.float32)
-    return lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, 4, WeightDtype.BF16), 256, GpuMamba3LM
+    return lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, rows, WeightDtype.BF16), 256, GpuMamba3LM
 
 
 @pytest.mark.parametrize("family", ["m1", "m3"])
@@ -330,3 +330,41 @@ def test_a_reset_waits_for_the_steps_before_it(family):
         assert np.array_equal(a.step(x), want)
         a.reset()
     a.close()
+
+
+@pytest.mark.parametrize("family", ["m1", "m3"])
+def test_generation_hands_out_no_token_of_a_lost_step(family, monkeypatch):
+    """Streaming and batched generation whose steps are called off: from the start, the kernel chain generates instead (its own
+    engine's tokens); behind the third token, the caller has exactly the three it was given, and an error."""
+    from mamba_rs_amd import MambaHipError, SampleParams
+    make, dm, lm_of = _family(family, 1)
+    a = make()
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = make()
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    embed = np.random.default_rng(8).standard_normal((128, dm)).astype(np.float32)
+    prompt, params = [5, 9, 2], SampleParams(temperature=0.9, top_k=20, max_tokens=8, seed=3)
+    print(f"case generation behind lost steps {family}", flush=True)
+    lm, lm_chain = lm_of(a, embed), lm_of(chain, embed)
+
+    def stream(m, at=lambda n: None):
+        got = []
+
+        def take(tok):
+            got.append(tok)
+            at(len(got))
+        try:
+            m.generate_streaming(prompt, params, take)
+        except MambaHipError as e:
+            return got, e
+        return got, None
+    whole, err = stream(lm)
+    assert err is None and len(whole) == 8
+    got, err = stream(lm, lambda n: a.set_resident_wait(0) if n == 3 else None)
+    assert got == whole[:3] and "did not come free" in str(err)
+    assert stream(lm) == stream(lm_chain)                  # (the wait is still 0)
+    assert lm.generate_batch([prompt], [params]) == lm_chain.generate_batch([prompt], [params])
+    a.set_resident_wait(1 << 23)
+    assert stream(lm) == (whole, None)
+    for e in (lm, lm_chain, a, chain):
+        e.close()
