@@ -4,7 +4,9 @@
 // engine takes the route only while its workgroups are at most as many as the compute units, one each); two launches that hold
 // half of the places each would wait until they give up.  So
 //   * one process per GPU has the route: the first to ask binds an abstract socket named after the GPU's PCI address, which the
-//     system takes back when the process ends, whatever way it ends; another process's engines keep the kernel chains;
+//     system takes back when the process ends, whatever way it ends; another process's engines keep the kernel chains (of those that
+//     share a network namespace: two containers on one GPU do not see each other, and launches that meet there are called off);
+//   * an engine whose kernels may not use all compute units -- a mask on its stream or in the environment -- keeps the chains;
 //   * inside the process, while the live engines' launches do not all fit together, they go one after the other: every launch is
 //     followed by an event on its own stream, and the next engine's launch waits for it (on the GPU).  An engine touches no
 //     stream but its own: another one's may be in a capture, which an event recorded from here would join.
@@ -16,7 +18,9 @@
 #include <errno.h>
 #include <mutex>
 #include <stddef.h>
+#include <stdint.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 #include <sys/socket.h>
 #include <sys/un.h>
@@ -53,6 +57,20 @@ bool bind_gpu(int device) {
     return true;   // held until the process ends
 }
 
+// Whether kernels on a stream may use all `units` compute units.
+bool whole_gpu(hipStream_t stream, int units) {
+    const char *e = getenv("HSA_CU_MASK");   // (applied below HIP, which does not report it)
+    if (e && *e) return false;
+    uint32_t mask[32] = {0};   // (1024 units)
+    if (hipExtStreamGetCUMask(stream, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int may = 0;
+    for (uint32_t m : mask) may += __builtin_popcount(m);
+    return may >= units;
+}
+
 }  // namespace
 
 bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t stream) {
@@ -64,7 +82,7 @@ bool resident_claim(ResidentSeat &seat, int device, int workgroups, hipStream_t 
         g.ours = hipDeviceGetAttribute(&g.places, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
                  hipEventCreateWithFlags(&g.event, hipEventDisableTiming) == hipSuccess && bind_gpu(device);
     }
-    if (!g.ours || workgroups > g.places) return false;
+    if (!g.ours || workgroups > g.places || !whole_gpu(stream, g.places)) return false;
     try { g.seats.push_back(&seat); } catch (...) { return false; }
     seat.device = device; seat.workgroups = workgroups; seat.stream = stream; seat.open = seat.unseen = seat.off = seat.told = false;
     g.live += workgroups;

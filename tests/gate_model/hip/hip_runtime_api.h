@@ -1,6 +1,7 @@
 // What csrc/resident_gate.hip needs of the runtime, as a model that runs on the host (model.cpp): streams and events are vector
 // clocks, and an operation that joins somebody's capture or touches another engine's stream is counted.
 #pragma once
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 #include <vector>
@@ -34,6 +35,11 @@ inline void model_merge(std::vector<long> &a, const std::vector<long> &b) {
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipDeviceGetPCIBusId(char *s, int n, int) { strncpy(s, getenv("MODEL_BUS") ? getenv("MODEL_BUS") : "model", n); return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = model().places; return hipSuccess; }
+inline hipError_t hipExtStreamGetCUMask(hipStream_t, uint32_t n, uint32_t *mask) {
+    const char *e = getenv("MODEL_CU_MASK");   // the first word
+    for (uint32_t i = 0; i < n; i++) mask[i] = i * 32 >= (uint32_t)model().places ? 0 : i == 0 && e ? (uint32_t)strtoul(e, nullptr, 16) : ~0u;
+    return hipSuccess;
+}
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = new ModelEvent; return hipSuccess; }
 inline hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
     *c = s->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;

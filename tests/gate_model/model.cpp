@@ -1,5 +1,6 @@
 // Engines come, go, step, are waited for and are captured in a random order; whenever one launches, the launches of the others that
 // the runtime does not order before it must fit on the chip beside it.  Prints "ok <launches in turns> <refused turns>" or the fault.
+// With the argument "claim": whether one engine gets the route, which it then holds until its input ends.
 #include "resident_gate.hip"
 #include <memory>
 #include <random>
@@ -42,6 +43,14 @@ void host_wait(Engine &e, std::vector<std::unique_ptr<Engine>> &all) {
 }  // namespace
 
 int main(int argc, char **argv) {
+    if (!strcmp(argv[1], "claim")) {
+        ResidentSeat seat;
+        ModelStream stream{0};
+        printf("%d\n", resident_claim(seat, 0, 64, &stream));
+        fflush(stdout);
+        while (getchar() != EOF) {}
+        return 0;
+    }
     std::mt19937 rng((unsigned)atoi(argv[1]));
     Model &m = model();
     m.fail_every = argc > 2 ? atoi(argv[2]) : 0;

@@ -15,9 +15,28 @@ def model(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(HERE, "gate_model"), "-I", CSRC, "-o", exe,
                     os.path.join(HERE, "gate_model", "model.cpp"), "-lpthread"], check=True)
 
-    def run(*args, bus="0"):
-        return subprocess.run([exe, *map(str, args)], env={**os.environ, "MODEL_BUS": f"model{os.getpid()}.{bus}"}, capture_output=True, text=True)
+    def run(*args, bus="0", wait=True, **env):
+        cmd, env = [exe, *map(str, args)], {**os.environ, "MODEL_BUS": f"model{os.getpid()}.{bus}", **env}
+        if wait:
+            return subprocess.run(cmd, env=env, stdin=subprocess.DEVNULL, capture_output=True, text=True)
+        return subprocess.Popen(cmd, env=env, stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
     return run
+
+
+def test_one_process_per_gpu_on_the_whole_gpu(model):
+    """The route belongs to the first process that asks for a GPU until it ends; an engine that may not use every compute unit
+    does not get it."""
+    assert model("claim").stdout == "1\n"                        # (and gave it back by ending)
+    holder = model("claim", wait=False)
+    assert holder.stdout.readline() == "1\n"
+    assert model("claim").stdout == "0\n"
+    assert model("claim", bus="1").stdout == "1\n"               # another GPU
+    holder.kill()                                                # whatever way it ends
+    holder.wait()
+    assert model("claim").stdout == "1\n"
+    assert model("claim", MODEL_CU_MASK="fffffffe").stdout == "0\n"
+    assert model("claim", HSA_CU_MASK="0:0-127").stdout == "0\n"
+    assert model("claim", MODEL_CU_MASK="ffffffff", HSA_CU_MASK="").stdout == "1\n"
 
 
 @pytest.mark.parametrize("seed", range(6))

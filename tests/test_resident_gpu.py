@@ -368,3 +368,27 @@ def test_generation_hands_out_no_token_of_a_lost_step(family, monkeypatch):
     assert stream(lm) == (whole, None)
     for e in (lm, lm_chain, a, chain):
         e.close()
+
+
+def test_a_second_process_keeps_the_kernel_chain(monkeypatch, tmp_path):
+    """While this process has resident engines on the GPU, another process's engine has the kernel chain, with the chain's bits."""
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    a, = _engines((256, 2, 2), 1)
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain, = _engines((256, 2, 2), 1)
+    monkeypatch.delenv("MRS_DECODE_NO_RESIDENT")
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    x = np.random.default_rng(9).standard_normal((2, 256)).astype(np.float32)
+    np.save(tmp_path / "x.npy", x)
+    program = ("import sys; sys.path[:0] = sys.argv[1:3]; import numpy as np; from test_resident_gpu import _engines\n"
+               "e, = _engines((256, 2, 2), 1); np.save(sys.argv[3] + '/y.npy', e.step(np.load(sys.argv[3] + '/x.npy'))); print(e.decode_route())")
+    print("case a second process", flush=True)
+    r = subprocess.run([sys.executable, "-c", program, os.path.dirname(here), here, str(tmp_path)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split()[-1] == "1", r.stdout + r.stderr
+    assert np.array_equal(np.load(tmp_path / "y.npy"), chain.step(x))
+    a.step(x)
+    for e in (a, chain):
+        e.close()
