@@ -31,8 +31,9 @@ constexpr unsigned kSpinLimit = 1u << 21;
 // without seeing the doubt had seen all of them before it, so they are all there now and it goes on as well; otherwise the launch
 // is called off.  So all workgroups take the same way, also those that get a place only when others have left.  A wait of 0 calls off
 // without an answer.
-// The answers are read while the first exchange is waited for: a step takes 1 to 2 us longer for it (24 layers of d_model 1024 270 ->
-// 272 us, four of 256 at eight rows 30.5 -> 32.5).  As a count on one word, added to and polled by 256 workgroups: 4 to 11 us.
+// The answers are read while the first exchange is waited for: a step takes about a microsecond longer for it (four layers of d_model 256 at eight rows 30.8 -> 31.5 us, of d_model 64 at 32 25.8 -> 27.0;
+// 24 layers of d_model 768 within what builds differ by).
+// As a count on one word, added to and polled by 256 workgroups: 4 to 11 us.
 constexpr int kRollCall = -1;   // a workgroup's state: the roll call, 0 under way, or a ResidentFault
 constexpr unsigned kDoubt = 1, kGo = 2, kOff = 3;
 struct RollCall {
@@ -165,19 +166,20 @@ template <typename T> __device__ __forceinline__ u64 half_pair_word(T a, T b, un
 }
 __device__ __forceinline__ void xch_put_word(u64 *p, u64 w) { __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Polls the KU words base[idx(0)] .. base[idx(KU - 1)] until ready(word) holds for all of them.  False when the wait was given up; the
-// first exchange of a step (`state`, else null) waits as long as the roll call is not over.
-template <int KU, class IDX, class READY>
-__device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, u64 (&r)[KU], const volatile int *state = nullptr) {
+// Polls the KU words base[idx(0)] .. base[idx(KU - 1)] until ready(word) holds for all of them.  False when the wait was given up; a
+// step's first exchange (state() its workgroup's) waits as long as the roll call is not over.
+struct NoRollCall { __device__ __forceinline__ int operator()() const { return 0; } };
+template <int KU, class IDX, class READY, class STATE = NoRollCall>
+__device__ __forceinline__ bool xch_poll(const u64 *base, IDX idx, READY ready, u64 (&r)[KU], STATE state = STATE()) {
     for (unsigned spins = 0; spins <= kSpinLimit; spins++) {
         bool have = true;
 #pragma unroll
         for (int u = 0; u < KU; u++) r[u] = xch_get(base + idx(u));
 #pragma unroll
-        for (int u = 0; u < KU; u++) have = have && ready(r[u]);
+        for (int u = 0; u < KU; u++) have &= ready(r[u]);   // (no branch per word)
         if (have) return true;
-        if (state && (spins & 63u) == 63u) {
-            const int s = *state;
+        if ((spins & 63u) == 63u) {
+            const int s = state();
             if (s > 0) return false;
             if (s == kRollCall) spins = 0;
         }
@@ -244,7 +246,7 @@ struct WeightFeed {
     unsigned win, wout, small;    // LDS byte addresses; the small blocks of two layers lie one after the other
     int out, small_at, small_bytes;   // offsets in the block
 };
-__device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, volatile int &state, RollCall call) {
+__device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, int &state, RollCall call) {
     const char *blk = f.blk;
     const bool first = (threadIdx.x & 63) == 0, out_wave = wave == 10, small_wave = wave == 11;
     const int iw = wave == 11 ? 2 : wave - 8, in_pieces = f.out >> 10, in_mid = in_pieces / 2, out_pieces = (f.small_at - f.out) >> 10;

@@ -66,8 +66,8 @@ __host__ __device__ inline ResLds res_lds(int dm, int di, int cols, int oc, int 
 template <typename T>
 __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const ResidentM3Args *args) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    __shared__ int state_word;
-    volatile int &state = state_word;   // kRollCall, 0, or a ResidentFault
+    __shared__ int state;   // kRollCall, 0, or a ResidentFault
+    const auto state_now = [] { return __hip_atomic_load(&state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
     const auto *a = as_table(args);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = a->G, b = blockIdx.x / G, src = blockIdx.x - b * G;
     const int dm = a->dm, di = a->di, nl = a->n_layers, nc = a->nc, oc = a->oc, ex = a->ex, ds = a->ds, nh = a->nh, hd = a->hd, ng = a->ng, nr = a->nr;
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
             // the accumulated angle (f64, wrapped); a lane per coordinate
             const int n = min(here(lane), ds - 1), at = (wave == 0 ? grp : ng + grp) * ds + n, sc = 2 * ng * ds;
             u64 r[3];
-            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(u == 0 ? at : u == 1 ? sc + head : nr > 0 ? sc + 3 * nh + pair : at); }, tagged, r, &state);
+            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(u == 0 ? at : u == 1 ? sc + head : nr > 0 ? sc + 3 * nh + pair : at); }, tagged, r, state_now);
             const float raw = __uint_as_float((unsigned)r[0]);
             const float *nw = reinterpret_cast<const float *>(small + (wave == 0 ? sb.bnw : sb.cnw)), *bias = reinterpret_cast<const float *>(small + (wave == 0 ? sb.bb : sb.cb));
             const float sq = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wave_sum_last(here(lane) < ds ? raw * raw : 0.0f)), 63));
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
             // ---- alpha, beta, gamma of the head
             const int sc = 2 * ng * ds + head;
             u64 r[3];
-            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(sc + u * nh); }, tagged, r, &state);
+            ok = xch_poll<3>(e2, [&](int u) { return (unsigned)(sc + u * nh); }, tagged, r, state_now);
             const float dtv = softplus20(__uint_as_float((unsigned)r[0]) + *reinterpret_cast<const float *>(small + sb.dtb));
             const float a_val = fminf(-heavy_tail(__uint_as_float((unsigned)r[1])), -a->a_floor), trap = sigmoidf_fast(__uint_as_float((unsigned)r[2]));
             const float al = fast_exp2(a_val * dtv * kLog2e);

@@ -69,8 +69,8 @@ __host__ __device__ inline ResLds res_lds(int dm, int di, int nc, int oc, int xd
 template <typename T>
 __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const ResidentArgs *args) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    __shared__ int state_word;
-    volatile int &state = state_word;   // kRollCall, 0, or a ResidentFault
+    __shared__ int state;   // kRollCall, 0, or a ResidentFault
+    const auto state_now = [] { return __hip_atomic_load(&state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
     const auto *a = as_table(args);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = a->G, b = blockIdx.x / G, src = blockIdx.x - b * G;
     const int dm = a->dm, di = a->di, nl = a->n_layers, nc = a->nc, oc = a->oc, xd = a->xd, dr = a->dr;
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
                 for (int k0 = g; k0 < G; k0 += 8 * KU) {
                     u64 r[KU];
                     ok = ok && xch_poll<KU>(e2, [&](int u) { return (unsigned)(min(k0 + 8 * u, G - 1) * hx + q); },
-                                            [&](u64 w) { return (((unsigned)w ^ tag) & 1u) == 0 && (((unsigned)(w >> 32) ^ tag) & 1u) == 0; }, r, &state);
+                                            [&](u64 w) { return ((((unsigned)w ^ tag) | ((unsigned)(w >> 32) ^ tag)) & 1u) == 0; }, r, state_now);
 #pragma unroll
                     for (int u = 0; u < KU; u++) {
                         const bool in = k0 + 8 * u < G;
