@@ -31,8 +31,8 @@ constexpr unsigned kSpinLimit = 1u << 21;
 // without seeing the doubt had seen all of them before it, so they are all there now and it goes on as well; otherwise the launch
 // is called off.  So all workgroups take the same way, also those that get a place only when others have left.  A wait of 0 calls off
 // without an answer.
-// The answers are read while the first exchange is waited for: a step takes about a microsecond longer for it (four layers of d_model 256 at eight rows 30.8 -> 31.5 us, of d_model 64 at 32 25.8 -> 27.0;
-// 24 layers of d_model 768 within what builds differ by).
+// The answers are read while the first exchange is waited for: a step takes about a microsecond longer for it (four layers of
+// d_model 256 at eight rows 30.8 -> 31.5 us, of d_model 64 at 32 25.8 -> 27.0; 24 layers of d_model 768 within what builds differ by).
 // As a count on one word, added to and polled by 256 workgroups: 4 to 11 us.
 constexpr int kRollCall = -1;   // a workgroup's state: the roll call, 0 under way, or a ResidentFault
 constexpr unsigned kDoubt = 1, kGo = 2, kOff = 3;
@@ -153,13 +153,16 @@ constexpr int kResThreads = kCompute + 4 * 64;   // eight waves compute, four br
 __host__ __device__ constexpr int up1k(int n) { return (n + 1023) & ~1023; }
 constexpr size_t kResLdsMax = 160 * 1024 - 256;
 
-// Two f32 in one exchange word: the lowest mantissa bit of each carries the parity of the layer's tag (a buffer's entries are
-// rewritten every layer, so what is not of this layer is of the one before).  The shares are added up in f32 and rounded to 16 bits at
-// once; 32 steps at the 130m shape differ from the f32 engine by 0.17 % of the output, as the kernel chain's do.
+// Fourteen f32 in a line of eight exchange words: seven words of two each, where the lowest mantissa bit carries the parity of the layer's
+// tag (a line is rewritten every layer, so what is not of this layer is of the one before), and one of those bits with the tag.
+// The values arrive whole, infinities and NaN as well.  (Two whole f32 per word with a "not there" value that its writer puts back, so
+// that every word is written twice a layer: 24 layers of d_model 1024 9 to 14 us slower.)
+constexpr int kLineVals = 14;
 __device__ __forceinline__ u64 pair_word(float a, float b, unsigned tag) {
     const unsigned x = (__float_as_uint(a) & ~1u) | (tag & 1u), y = (__float_as_uint(b) & ~1u) | (tag & 1u);
     return (u64)y << 32 | x;
 }
+__device__ __forceinline__ unsigned with_bit(unsigned half, unsigned bits, int at) { return (half & ~1u) | (bits >> at & 1u); }
 // Two 16-bit values and the tag.
 template <typename T> __device__ __forceinline__ u64 half_pair_word(T a, T b, unsigned tag) {
     return (u64)tag << 32 | (unsigned)__builtin_bit_cast(uint16_t, b) << 16 | __builtin_bit_cast(uint16_t, a);

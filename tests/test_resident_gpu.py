@@ -392,3 +392,28 @@ def test_a_second_process_keeps_the_kernel_chain(monkeypatch, tmp_path):
     a.step(x)
     for e in (a, chain):
         e.close()
+
+
+@pytest.mark.parametrize("layer", [0, 1])
+def test_an_infinite_share_stays_infinite(layer, monkeypatch):
+    """One entry of a layer's x_proj row overflows to -inf in one workgroup's share (a dt entry whose weights are positive, so the step
+    size becomes 0 and every output is finite): the exchange hands it on as -inf, and the rows are the kernel chain's."""
+    cfg = MambaConfig(d_model=64, d_state=16, d_conv=4, expand=2, n_layers=2)
+    w = MambaWeights.init(cfg, 64, 5)
+    w.input_proj_w = np.zeros((0, 64), np.float32)
+    lw = w.layers[layer]
+    lw.conv1d_bias[3] = 8.0
+    lw.x_proj_w.reshape(cfg.d_inner(), -1)[:, 0] = 0.0
+    lw.x_proj_w.reshape(cfg.d_inner(), -1)[3, 0] = -3e38
+    lw.dt_proj_w.reshape(-1, cfg.d_inner())[0, :] = 0.5
+    a = GpuMambaBackbone.new_with_dtype(0, w, cfg, 64, 2, WeightDtype.BF16)
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = GpuMambaBackbone.new_with_dtype(0, w, cfg, 64, 2, WeightDtype.BF16)
+    print(f"case infinite share in layer {layer}", flush=True)
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    for x in np.random.default_rng(10).standard_normal((5, 2, 64)).astype(np.float32):
+        got, want = a.step(x), chain.step(x)
+        assert np.isfinite(want).all() and np.isfinite(got).all()
+        assert min(cosine(g, c) for g, c in zip(got, want)) >= 0.999
+    a.close()
+    chain.close()
