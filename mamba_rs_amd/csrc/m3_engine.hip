@@ -651,11 +651,16 @@ int project_input3(mrs_m3_backbone *bb) {
     return MRS_OK;
 }
 
-// Deepest model that takes the resident step.  It adds the same products in another order than the kernel chain, and this network's
-// angles carry a 16-bit rounding that falls the other way from layer to layer: at 24 layers of d_model 768 two such orders differ by
-// 0.8 % of the output (each 1.1 % from f32; Mamba-1: 0.17 %), and 7 of 16 greedy passes of 32 tokens leave the chain's tokens somewhere
-// (the chain's own two orders, row-wise and tiled: 5 of 16).  The step would take 212 instead of 281 us there; deep models keep their tokens.
-constexpr int kResidentM3Layers = 8;
+// Deepest model that takes the resident step.  It is as accurate as the kernel chain at every depth, but adds the same products in another
+// order; where an operand row is rounded to 16 bits, that rounding can fall the other way, and the difference grows from layer to layer.
+// Output of 32 bf16 steps, resident against chain / chain against the f32 engine, and how many of 48 greedy passes of 32 tokens
+// leave the chain's tokens (in brackets: the chain's own two orders, row-wise and tiled, against each other):
+//   d_model 768    2 layers 0.06 / 0.31 %, 0 (0)    4 0.21 / 0.44, 1 (1)    6 0.33 / 0.54, 1 (1)    8 0.44 / 0.64, 3 (3)    24 0.92 / 1.12
+//   d_model 256    2 layers 0.03 / 0.48 %, 0 (0)    4 0.19 / 0.76, 3 (3)    6 0.31 / 0.98, 4 (4)    8 0.42 / 1.21, 10 (9)
+//   d_model 64                                      4 0.01 / 0.74, 0 (0)                            8 0.06 / 1.18, 0 (0)
+// There is no depth at which it turns.  The line lies where the difference is that of the Mamba-1 step (0.17 % at 24 layers); deeper
+// models keep the chain's tokens (24 layers of d_model 768: 212 against 281 us a step).
+constexpr int kResidentM3Layers = 4;
 
 // Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
 // for the steps that do not get a turn.

@@ -69,3 +69,23 @@ def test_resident_step_follows_the_cpu_route(cfg, idim, B, dtype, monkeypatch):
     assert np.array_equal(a.step(x[0]), b.step(x[0]))
     for e in (a, b, chain):
         e.close()
+
+
+@pytest.mark.parametrize("layers,route", [(4, 2), (5, 1)])
+def test_deep_models_keep_the_kernel_chain(layers, route, monkeypatch):
+    """Five layers and more step on the chain, with its bits; up to four the resident step stays within twice the 0.2 % of the output by
+    which two orders of the chain's own sums differ there (measured, 32 steps)."""
+    cfg = cfg_(256, 16, 16, 1, layers)
+    w = perturbed(cfg, 256, 3)
+    w.input_proj_w = np.zeros(0, np.float32)
+    a = GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, 2, WeightDtype.BF16)
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, 2, WeightDtype.BF16)
+    assert (a.decode_route(), chain.decode_route()) == (route, 1)
+    x = np.random.default_rng(layers).standard_normal((32, 2, 256)).astype(np.float32)
+    got, want = np.stack([a.step(r) for r in x]), np.stack([chain.step(r) for r in x])
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"case {layers} layers: resident against chain {rel:.2e}", flush=True)
+    assert rel == 0 if route == 1 else rel < 4e-3
+    a.close()
+    chain.close()
