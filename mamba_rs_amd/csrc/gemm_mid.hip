@@ -134,7 +134,6 @@ bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void 
 int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {
     if (!mid_gemm_ok(dtype, out_f32, C, ldc, A, lda, Wt, M, N, K))
         return fail(MRS_E_SHAPE, "mid gemm: 16-bit storage, N %% 4 == 0, K %% 64 == 0, 16-byte aligned operands (M=%lld N=%d K=%d)", (long long)M, N, K);
-    const int64_t big = (M + 127) / 128 * ((N + 127) / 128);
     if (dtype == MRS_BF16)
         return out_f32 ? launch_mid<bf16_t, float>(st, C, ldc, A, lda, Wt, (int)M, N, K) : launch_mid<bf16_t, bf16_t>(st, C, ldc, A, lda, Wt, (int)M, N, K);
     return out_f32 ? launch_mid<f16_t, float>(st, C, ldc, A, lda, Wt, (int)M, N, K) : launch_mid<f16_t, f16_t>(st, C, ldc, A, lda, Wt, (int)M, N, K);
