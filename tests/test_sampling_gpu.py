@@ -137,6 +137,34 @@ def test_top_k_by_group_maxima_keeps_what_the_search_keeps(shape):
     assert near <= 1
 
 
+@pytest.mark.parametrize("vocab", [300, 50280])
+@pytest.mark.parametrize("rest", ["-inf", "lowest", "all", "nan", "-nan", "inf"])
+def test_top_k_of_masked_rows(vocab, rest):
+    """Rows whose entries but forty are masked (by -inf or the type's lowest value), all of them masked, or with NaN or infinite
+    entries among the forty.  Beyond the forty everything has no weight, so k = 128 (candidates by group maxima; at the large vocabulary
+    too many share the floor and it searches after all) and k = 129 (always the search) must pick the same token from the same draw,
+    and the oracle's where it is defined."""
+    rng = np.random.default_rng(vocab)
+    row = np.full(vocab, np.finfo(np.float32).min if rest == "lowest" else -np.inf, np.float32)
+    some = rng.choice(vocab, 40, replace=False)
+    if rest != "all":
+        row[some] = rng.standard_normal(40) * 2
+    if rest in ("nan", "inf"):
+        row[some[7]] = np.float32(rest)
+    if rest == "-nan":
+        row[some[7]] = np.array([0xffc00000], np.uint32).view(np.float32)[0]
+    opts = [dict(temperature=t, top_p=p, min_p=m) for t, p, m in ((1.0, 1.0, 0.0), (0.7, 0.9, 0.0), (1.5, 0.95, 0.05)) for _ in range(8)]
+    seeds = [900 + r for r in range(len(opts))]
+    print(f"case masked top-k {vocab} {rest}", flush=True)
+    tok, state = {}, {}
+    for k in (128, 129):
+        tok[k], state[k] = device_sample(np.tile(row, (len(opts), 1)), [SampleParams(top_k=k, **o) for o in opts], seeds)
+    assert np.array_equal(tok[128], tok[129]) and np.array_equal(state[128], state[129])
+    assert ((0 <= tok[128]) & (tok[128] < vocab)).all()
+    if rest in ("-inf", "lowest"):
+        assert sum(check_row(int(tok[128][r]), row, SampleParams(top_k=128, **o), seeds[r])[0] for r, o in enumerate(opts)) <= 1
+
+
 def test_ties_keep_the_lower_index_and_greedy_keeps_the_last_maximum():
     vocab = 4096
     rng = np.random.default_rng(2)
