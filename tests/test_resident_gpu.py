@@ -1,5 +1,5 @@
 """GPU: the resident decode step (a whole 16-bit Mamba-1 step in one launch whose workgroups exchange through memory) against
-the CPU route, and against itself: eager and replayed, alone and taking turns with a second engine."""
+the CPU route, and against itself: eager and replayed, alone, beside other engines, threads and processes, in captures, called off."""
 import numpy as np
 import pytest
 
@@ -25,8 +25,8 @@ from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtyp
 def test_resident_step_follows_the_cpu_route(shape, dtype):
     """Six steps (three eager, three replayed): every row within the 16-bit engines' tolerance of the CPU route on
     storage-rounded weights (cosine >= 0.999 as for the kernel chains: the same rounding points, sums in another order), states
-    as well.  A second engine steps in turns with the first -- together they have more workgroups than the chip has places
-    from 129 up -- and ends on the same bits: all sums are in a fixed order."""
+    as well.  A second engine steps behind the first -- each call returns with its rows, so nothing overlaps here; the queued steps
+    below do -- and ends on the same bits: all sums are in a fixed order."""
     dm, L, idim, B = shape
     cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
     w = MambaWeights.init(cfg, idim, 11)

@@ -1,5 +1,6 @@
 """GPU: the resident Mamba-3 decode step (a whole 16-bit step in one launch whose workgroups exchange through memory) against the
-CPU route, against the kernel chain it replaces, and against itself: eager and replayed, alone and taking turns with a second engine."""
+CPU route, against the kernel chain it replaces, and against itself: eager and replayed, beside a second engine (queued steps, threads and
+captures of both networks: test_resident_gpu.py)."""
 import numpy as np
 import pytest
 
@@ -29,8 +30,8 @@ def cfg_(dm, ds, hd, ng, L, rope=0.5):
 def test_resident_step_follows_the_cpu_route(cfg, idim, B, dtype, monkeypatch):
     """Six steps (three eager, three replayed): every row within the 16-bit engines' tolerance of the CPU route on
     storage-rounded weights (cosine >= 0.999, as for the kernel chain), all four states as well; the kernel chain on the same
-    weights agrees as closely.  A second engine steps in turns with the first and ends on the same bits: all sums are in a
-    fixed order."""
+    weights agrees as closely.  A second engine steps behind the first and ends on the same bits: all sums are in a fixed
+    order."""
     w = perturbed(cfg, idim, 11)
     if idim == cfg.d_model:
         w.input_proj_w = np.zeros(0, np.float32)
