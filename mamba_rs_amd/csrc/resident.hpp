@@ -140,6 +140,20 @@ __device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int fi
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Over the eight groups of eight lanes: the sum of the lanes 8 apart, in every lane.
+__device__ __forceinline__ float groups_sum(float v) {
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xf, 0xf, false));   // row_ror:8
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);   // rows 0 0 2 2 and 1 1 3 3
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);   // the lower half twice and the upper half twice
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+// Lane 7's value of the eight lanes this one belongs to.
+__device__ __forceinline__ unsigned last_of_8(unsigned v) {
+    const unsigned q = __builtin_amdgcn_mov_dpp(v, 0xff, 0xf, 0xf, true);           // quad_perm [3,3,3,3]: in the upper four
+    return __builtin_amdgcn_update_dpp(q, q, 0x141, 0xf, 0x5, false);               // row_half_mirror into the lower four (banks 0 and 2)
+}
+
 // Sum over a wave, in lane 63.
 __device__ __forceinline__ float wave_sum_last(float v) {
     v = row16_sum(v);

@@ -23,10 +23,8 @@ namespace {
 
 constexpr int kDs = 16, kDc = 4;           // states and conv taps of a channel
 constexpr int kMaxNc = 24, kMaxOc = 16, kMaxXd = 96, kMaxDr = 64;   // bounds of the fixed LDS areas
-// Lines of exchange 2 per workgroup, a wave each, and the lines from a workgroup to the next: an odd number (24 layers of d_model 768, six
-// lines: 200 us a step six apart, 179 seven apart, 206 eight apart).
+// Lines of exchange 2 per workgroup, a wave each.
 __host__ __device__ constexpr int share_lines(int xd) { return (xd + kLineVals - 1) / kLineVals; }
-__host__ __device__ constexpr int share_pitch(int xd) { return share_lines(xd) | 1; }
 static_assert(share_lines(kMaxXd) <= kComputeWaves, "");
 constexpr int kInSteps = 4, kInTiles = 2 * kMaxNc / 16, kOutSteps = 8;      // k-steps of 32 per computing wave and 16-column tiles held in registers
 
@@ -96,8 +94,8 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
     const T *win = (const T *)(smem + L.win), *wout = (const T *)(smem + L.wout);
     float *pre = (float *)(smem + Fix::pre), *pre2 = (float *)(smem + Fix::pre2), *zs = (float *)(smem + Fix::zs), *xdl = (float *)(smem + Fix::xdl),
           *invl = (float *)(smem + Fix::inv);
-    const int lines = share_lines(xd), pitch = share_pitch(xd);
-    u64 *e2 = a->xch + (size_t)b * a->xch_stride, *e1 = e2 + (size_t)G * pitch * 8, *e1s = e1 + (dm >> 1), *e3 = e1s + G;   // this row's buffers
+    const int lines = share_lines(xd);
+    u64 *e2 = a->xch + (size_t)b * a->xch_stride, *e1 = e2 + (size_t)G * lines * 8, *e1s = e1 + (dm >> 1), *e3 = e1s + G;   // this row's buffers
     unsigned *epoch = a->epoch + 32 * b;
     const unsigned base = *epoch;
     const int lane = tid & 63, ct_in = (2 * nc) >> 4;
@@ -167,35 +165,31 @@ __global__ __launch_bounds__(kResThreads) void resident_step_kernel(const Reside
             const float nb = __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(s[0]), 0xb1, 0xf, 0xf, true));   // the neighbour lane's
             const unsigned low = (unsigned)__ballot(__float_as_uint(s[0]) & 1u) & ((1u << kLineVals) - 1u);
             if (here(lane) < 16 && (n & 1) == 0)
-                xch_put_word(e2 + (unsigned)((src * pitch + wave) * 8 + (n >> 1)), n < kLineVals ? pair_word(s[0], nb, tag) : (u64)tag << 32 | low);
+                xch_put_word(e2 + (unsigned)((src * lines + wave) * 8 + (n >> 1)), n < kLineVals ? pair_word(s[0], nb, tag) : (u64)tag << 32 | low);
         }
-        // ---- the whole x_proj row: a wave per line, eight lanes per word, the shares in workgroup order within a lane, then over the lanes
+        // ---- the whole x_proj row: a wave per line, eight neighbouring lanes for a workgroup's 64 bytes (with a word's eight workgroups in
+        // neighbouring lanes instead, each of them in another line: 24 layers of d_model 768 179 us a step against 171, of 1024 266
+        // against 252), the shares in workgroup order within a lane, then over the eight groups of lanes
         bool ok = true;
         {
             constexpr int KU = 8;
-            const int g = here(tid) & 7, q = here(tid) >> 3 & 7;   // q 7: the line's low bits
+            const int q = here(tid) & 7, g = here(tid) >> 3 & 7;   // q 7: the line's low bits
             if (conv_wave) {
                 float s0 = 0.0f, s1 = 0.0f;
                 const unsigned see_lo = q == 7 ? 0u : 1u, see_hi = q == 7 ? ~0u : 1u;   // a pair's parity, or the tag
 #pragma unroll 1
                 for (int k0 = g; k0 < G; k0 += 8 * KU) {
                     u64 r[KU];
-                    ok = ok && xch_poll<KU>(e2, [&](int u) { return (unsigned)((min(k0 + 8 * u, G - 1) * pitch + wave) * 8 + q); },
+                    ok = ok && xch_poll<KU>(e2, [&](int u) { return (unsigned)((min(k0 + 8 * u, G - 1) * lines + wave) * 8 + q); },
                                             [&](u64 w) { return ((((unsigned)w ^ tag) & see_lo) | (((unsigned)(w >> 32) ^ tag) & see_hi)) == 0; }, r, state_now);
 #pragma unroll
                     for (int u = 0; u < KU; u++) {
-                        const unsigned in = k0 + 8 * u < G ? ~0u : 0u, low = __shfl((unsigned)r[u], 56 + g, kWave);
+                        const unsigned in = k0 + 8 * u < G ? ~0u : 0u, low = last_of_8((unsigned)r[u]);
                         s0 += __uint_as_float(with_bit((unsigned)r[u], low, 2 * q) & in);
                         s1 += __uint_as_float(with_bit((unsigned)(r[u] >> 32), low, 2 * q + 1) & in);
                     }
                 }
-                auto over8 = [](float v) {
-                    v += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0xb1, 0xf, 0xf, true));    // quad_perm [1,0,3,2]
-                    v += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x4e, 0xf, 0xf, true));    // quad_perm [2,3,0,1]
-                    v += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x141, 0xf, 0xf, true));   // row_half_mirror
-                    return v;
-                };
-                const T r0 = (T)over8(s0), r1 = (T)over8(s1);
+                const T r0 = (T)groups_sum(s0), r1 = (T)groups_sum(s1);
                 const int e = wave * kLineVals + 2 * q;
                 if (g == 0 && q < 7 && e < xd) *reinterpret_cast<float2 *>(xdl + e) = make_float2(Store<T>::ld(&r0), Store<T>::ld(&r1));
             }
@@ -331,7 +325,7 @@ bool resident_plan(ResidentArgs &a, int dtype) {
         a.G = a.di / a.nc;
         a.oc = a.dm / a.G;
         if (!plan_ok(a)) continue;
-        a.xch_stride = ((size_t)a.G * share_pitch(a.xd) * 8 + a.dm / 2 + a.G + a.di / 2 + 7) / 8 * 8;   // (lines of 64 bytes)
+        a.xch_stride = ((size_t)a.G * share_lines(a.xd) * 8 + a.dm / 2 + a.G + a.di / 2 + 7) / 8 * 8;   // (lines of 64 bytes)
         return true;
     }
     return false;
