@@ -11,10 +11,11 @@
 // rewritten only after every reader of its last contents has published something that depends on them: one buffer per
 // exchange is enough.
 //
-// A launch begins with a roll call (RollCall): no workgroup stores anything but exchange words before all of them are on the chip.  Ordinary kernels that hold the compute units delay it.  If the units do not come free within the wait the caller set, the
-// launch is called off as a whole: the states are what they were, the output rows become NaN, `broken` (host memory) is raised, and
-// launches queued behind it leave at once.  After the roll call a wait is over when its neighbours have done their part; those waits
-// are bounded as well (kSpinLimit polls, about two seconds), and a workgroup that gives up there leaves the states unfinished.
+// A launch begins with a roll call (RollCall): no workgroup stores anything but exchange words before all of them are on the chip.
+// Ordinary kernels that hold the compute units delay it.  If the units do not come free within the wait the caller set, the launch is
+// called off as a whole: the states are what they were, the output rows become NaN, `broken` (host memory) is raised, and launches
+// queued behind it leave at once.  After the roll call a wait is over when its neighbours have done their part; those waits are
+// bounded as well (kSpinLimit polls, about two seconds), and a workgroup that gives up there leaves the states unfinished.
 #pragma once
 #include "common.hpp"
 #include "mfma_tiles.hpp"

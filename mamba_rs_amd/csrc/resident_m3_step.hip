@@ -12,8 +12,9 @@
 // Values are rounded to the storage type where the kernel chain rounds them: the operand rows, y and out_proj's result.
 //
 // What bounds it: three all-to-all exchanges and the chain between them, not the weights (7.4 MB a layer at d_model 768).
-// Per bf16 step, kernel chain / this (routes of one build, steps queued): 24 layers of d_model 768 281 / 212 us at one row and
-// 317 / 230 at two (kept on the chain all the same, kResidentM3Layers in m3_engine.hip says why); four layers of d_model 64 52 / 38 at one row and 55 / 40 at 32; of d_model 256 56 / 46 at one and 60 / 49 at eight.
+// Per bf16 step, kernel chain / this (routes of one build, steps queued): four layers of d_model 64 46 / 26 us at one row and 49 / 27 at
+// 32; of d_model 256 47 / 30 at one and 50 / 33 at eight; of d_model 768 53 / 38 at one and 57 / 42 at two; 24 layers of 768 281 / 212 at one
+// and 317 / 230 at two (kept on the chain all the same, kResidentM3Layers in m3_engine.hip says why).
 #include "resident.hpp"
 #include "m3_math.hpp"
 
