@@ -417,3 +417,42 @@ def test_an_infinite_share_stays_infinite(layer, monkeypatch):
         assert min(cosine(g, c) for g, c in zip(got, want)) >= 0.999
     a.close()
     chain.close()
+
+
+@pytest.mark.parametrize("family", ["m1", "m3"])
+def test_a_replayed_step_that_finds_no_places(family, monkeypatch):
+    """With an input projection the engine's graph holds the resident launch: called off, its step is the kernel chain's, eager, until
+    a reset; then the graph is replayed again."""
+    if family == "m1":
+        cfg = MambaConfig(d_model=64, d_state=16, d_conv=4, expand=2, n_layers=2)
+        w = MambaWeights.init(cfg, 20, 3)
+
+        def make():
+            return GpuMambaBackbone.new_with_dtype(0, w, cfg, 20, 4, WeightDtype.F16)
+    else:
+        from mamba_rs_amd import GpuMamba3Backbone
+        from test_m3_engine_gpu import perturbed
+        from test_resident_m3_gpu import cfg_
+        cfg = cfg_(64, 16, 16, 1, 2)
+        w = perturbed(cfg, 20, 3)
+
+        def make():
+            return GpuMamba3Backbone.new_with_dtype(0, w, cfg, 20, 4, WeightDtype.F16)
+    a = make()
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = make()
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    x = np.random.default_rng(11).standard_normal((3, 4, 20)).astype(np.float32)
+    print(f"case replay called off {family}", flush=True)
+    a.capture_graph()
+    resident = [a.step(r) for r in x]
+    a.reset()
+    a.set_resident_wait(0)
+    for r in x:
+        assert np.array_equal(a.step(r), chain.step(r))
+    a.reset()
+    a.set_resident_wait(1 << 23)
+    for r, want in zip(x, resident):
+        assert np.array_equal(a.step(r), want)
+    a.close()
+    chain.close()
