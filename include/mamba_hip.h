@@ -327,7 +327,9 @@ MRS_API float *mrs_backbone_temporal_ptr(mrs_backbone *bb);
 MRS_API int mrs_backbone_temporal_dtype(mrs_backbone *bb);
 /* Which decode route the engine chose at creation (no counterpart in the reference; for tests and benchmarks that must
  * know what they measured): a whole step in one launch (small f32 models; 16-bit models up to d_model 1024 for as many rows
- * as the chip holds at once, Mamba-3 up to eight layers), the library's own fused kernel chain, or the chain built on the vendor GEMM. */
+ * as the chip holds at once, Mamba-3 up to four layers -- 16-bit ones in one process per GPU, the first that asks, and not with
+ * MRS_DECODE_NO_RESIDENT=1), the library's own fused kernel chain, or the chain built on the vendor GEMM.  The one launch and the
+ * chain add in different orders: equally far from f32, not the same bits. */
 #define MRS_DECODE_LIBRARY_CHAIN 0
 #define MRS_DECODE_OWN_CHAIN 1
 #define MRS_DECODE_ONE_LAUNCH 2

@@ -26,8 +26,8 @@ typedef unsigned long long u64;
 constexpr unsigned kSpinLimit = 1u << 21;
 
 // The roll call, by one of the waves that bring weights.  roll[0]: a launch was called off or lost, its successors do not begin;
-// roll[1]: number of the launch; roll[2 + its parity]: the verdict; behind kRollHead words, one per workgroup: the number of the last
-// launch it has answered, plus one.  A workgroup goes on when it has seen all answers and, after that, no verdict against it.  One that has
+// roll[1]: number of the launch; roll[2 + its parity]: the ruling; behind kRollHead words, one per workgroup: the number of the last
+// launch it has answered, plus one.  A workgroup goes on when it has seen all answers and, after that, no ruling against it.  One that has
 // waited `wait` polls (one to two microseconds each) in vain first puts kDoubt there and then looks at the answers again: whoever went on
 // without seeing the doubt had seen all of them before it, so they are all there now and it goes on as well; otherwise the launch
 // is called off.  So all workgroups take the same way, also those that get a place only when others have left.  A wait of 0 calls off
@@ -62,17 +62,17 @@ struct RollCall {
         return yes;
     }
     __device__ __forceinline__ int outcome() const {
-        unsigned *verdict = roll + 2 + (number & 1u);
+        unsigned *ruling = roll + 2 + (number & 1u);
         const bool first = (threadIdx.x & 63) == 0;
 #pragma unroll 1
         for (unsigned spins = 0;; spins++) {
             const bool yes = answered();
-            const unsigned v = __builtin_amdgcn_readfirstlane(get(verdict));
+            const unsigned v = __builtin_amdgcn_readfirstlane(get(ruling));
             if (v == kOff) return kStepCalledOff;
             if (yes && v != kDoubt) break;
             if (v == 0 && spins >= wait) {
                 unsigned none = 0;
-                const bool mine = first && __hip_atomic_compare_exchange_strong(verdict, &none, kDoubt, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool mine = first && __hip_atomic_compare_exchange_strong(ruling, &none, kDoubt, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (!__any(mine)) continue;
                 done();
                 const bool go = answered();
@@ -81,7 +81,7 @@ struct RollCall {
                         put(roll, 1u);
                         __hip_atomic_store(broken, (unsigned)kStepCalledOff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     }
-                    put(verdict, go ? kGo : kOff);
+                    put(ruling, go ? kGo : kOff);
                 }
                 if (go) break;
                 return kStepCalledOff;

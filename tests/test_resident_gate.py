@@ -59,15 +59,15 @@ def test_roll_call_has_one_outcome(answers):
     seen, stack, ends = set(), [(0, (0,) * N, 0, (("begin",),) * N)], set()
     NONE, DOUBT, GO, OFF = range(4)
     while stack:
-        lost, got, verdict, at = state = stack.pop()
+        lost, got, ruling, at = state = stack.pop()
         if state in seen:
             continue
         seen.add(state)
         if all(a[0] == "end" for a in at):
             ends.add(frozenset(a[1] for a in at))
 
-        def to(i, nxt, lost=lost, got=got, verdict=verdict):
-            stack.append((lost, got, verdict, at[:i] + (nxt,) + at[i + 1:]))
+        def to(i, nxt, lost=lost, got=got, ruling=ruling):
+            stack.append((lost, got, ruling, at[:i] + (nxt,) + at[i + 1:]))
         for i, a in enumerate(at):
             if a[0] == "begin":
                 to(i, ("end", OFF) if lost else ("answer",))
@@ -75,21 +75,21 @@ def test_roll_call_has_one_outcome(answers):
                 to(i, ("read", 0, True), got=got[:i] + (answers[i],) + got[i + 1:])
             elif a[0] in ("read", "read again"):
                 k, all_there = a[1] + 1, a[2] and got[a[1]] == 1
-                after = ("verdict", all_there) if a[0] == "read" else ("resolve", all_there)
+                after = ("ruling", all_there) if a[0] == "read" else ("resolve", all_there)
                 to(i, (a[0], k, all_there) if k < N else after)
-            elif a[0] == "verdict":
-                if verdict == OFF:
+            elif a[0] == "ruling":
+                if ruling == OFF:
                     to(i, ("end", OFF))
-                elif a[1] and verdict != DOUBT:
+                elif a[1] and ruling != DOUBT:
                     to(i, ("end", GO))
                 else:
                     to(i, ("read", 0, True))
-                    if verdict == NONE:
+                    if ruling == NONE:
                         to(i, ("doubt",))
             elif a[0] == "doubt":
-                to(i, ("read again", 0, True), verdict=DOUBT) if verdict == NONE else to(i, ("read", 0, True))
+                to(i, ("read again", 0, True), ruling=DOUBT) if ruling == NONE else to(i, ("read", 0, True))
             elif a[0] == "resolve":
-                to(i, ("end", GO), verdict=GO) if a[1] else to(i, ("called off",), lost=1)
+                to(i, ("end", GO), ruling=GO) if a[1] else to(i, ("called off",), lost=1)
             elif a[0] == "called off":
-                to(i, ("end", OFF), verdict=OFF)
+                to(i, ("end", OFF), ruling=OFF)
     assert ends == ({frozenset([GO]), frozenset([OFF])} if all(answers) else {frozenset([OFF])})
