@@ -456,3 +456,28 @@ def test_a_replayed_step_that_finds_no_places(family, monkeypatch):
         assert np.array_equal(a.step(r), want)
     a.close()
     chain.close()
+
+
+def test_steps_queued_before_an_engine_was_there(monkeypatch):
+    """Steps that were queued while an engine had the chip to itself carry no event: an engine that does not fit beside it steps on the
+    kernel chain until somebody has waited for them, or the first engine has launched again."""
+    a, = _engines((768, 2, 4), 1)
+    x = np.random.default_rng(12).standard_normal((4, 768)).astype(np.float32)
+    want = a.step(x)
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain, = _engines((768, 2, 4), 1)
+    monkeypatch.delenv("MRS_DECODE_NO_RESIDENT")
+    want_chain = chain.step(x)
+    assert not np.array_equal(want, want_chain)     # (the two routes can be told apart here)
+    print("case steps from before", flush=True)
+    for settle in (a.sync, a.step_gpu_only):
+        a.step_gpu_only()
+        b, = _engines((768, 2, 4), 1)
+        assert np.array_equal(b.step(x), want_chain)
+        settle()
+        b.reset()
+        assert np.array_equal(b.step(x), want)
+        b.close()
+        a.sync()
+    a.close()
+    chain.close()
