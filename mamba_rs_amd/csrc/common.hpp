@@ -191,8 +191,8 @@ bool tiny_step_ok(int dtype, int input_dim, int dm, int di, int ds, int dc, int 
 int launch_tiny_step(hipStream_t st, const TinyStepArgs &a);
 // A whole Mamba-1 backbone step in one resident launch (resident_step.hip), 16-bit storage.  G workgroups per batch row, each owning nc
 // channels and oc out_proj columns (resident_plan fills these in).  weights: n_layers blocks of resident_layer_bytes(), each
-// packed by launch_resident_pack from a layer's weights as the engine holds them.  norm_w: layer 0's norm weight.  xch: batch *
-// xch_stride 64-bit words, epoch: 32 words per row, and roll: kRollHead + kRollMax words, all zero before the first launch; wait: how long a launch waits
+// packed by launch_resident_pack from a layer's weights as the engine holds them.  norm_w: layer 0's norm weight.  xch: groups *
+// xch_stride 64-bit words, epoch: 32 words per group, and roll: kRollHead + kRollMax words, all zero before the first launch; wait: how long a launch waits
 // for places (RollCall); broken: one word of pinned host memory, 0 or a ResidentFault.
 enum ResidentFault { kStepCalledOff = 1, kStepLost = 2 };   // no places, the states are what they were; given up in the middle
 constexpr unsigned kResidentWait = 1u << 23;                // default wait: ten to fifteen seconds
@@ -211,11 +211,20 @@ struct ResidentArgs {
     unsigned wait;
     float eps;
     int n_layers, batch, dm, di, ds, dc, dr, xd, G, nc, oc;
+    void *rows_buf;     // resident_rows_bytes() of operand rows
+    int groups, rows;   // groups of G workgroups, batch rows of the largest group (more than one: resident_rows.hip)
 };
 bool resident_plan(ResidentArgs &a, int dtype);   // false: the shape is outside the route
 size_t resident_layer_bytes(const ResidentArgs &a);
 int launch_resident_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
 int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);   // dev: a copy of `a` on the device
+// The same with up to kResidentRows batch rows per group of workgroups, with its own pack and sizes (resident_rows.hip).
+constexpr int kResidentRows = 16;
+bool resident_rows_plan(ResidentArgs &a, int dtype);
+size_t resident_rows_bytes(const ResidentArgs &a);
+size_t resident_rows_layer_bytes(const ResidentArgs &a);
+int launch_resident_rows_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
+int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);
 // The same for the Mamba-3 SISO backbone (resident_m3_step.hip); ex: columns of in_proj behind z and x that a workgroup owns.
 struct ResidentM3Layer {   // in_t [ip][d_model] and out_t [d_model][d_inner] transposed; next_nw: the norm weight after, or null
     const void *in_t, *out_t; const float *bnw, *cnw, *b_bias, *c_bias, *D, *dt_bias, *next_nw;

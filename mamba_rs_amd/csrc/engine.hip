@@ -8,7 +8,8 @@
 // stream, states, a_neg, D, biases and norm weights stay f32 (inference.rs:150-165).
 //
 // Decode, per layer (the reference launches 10 kernels + 4 GEMMs, inference.rs:993-1252):
-//   16-bit storage, a few rows of a model up to d_model 1024: the whole step is one resident launch (resident_step.hip);
+//   16-bit storage, up to 32 to 128 rows of a model up to d_model 1024: the whole step is one resident launch (resident_step.hip,
+//     resident_rows.hip);
 //   16-bit storage, batch <= 64: four kernels on the library's own skinny GEMM (gemm_skinny.hip) -- in_proj with the
 //     RMSNorm folded around it and the conv step + SiLU as epilogue, x_proj, one kernel for dt_proj + dt-bias + softplus
 //     + state update + B/C gather + SiLU gate, out_proj with the residual add as epilogue;
@@ -285,7 +286,7 @@ struct mrs_backbone {
     hipStream_t stream;
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
-    int resident;                 // a few rows: the step as one resident launch (resident_step.hip)
+    int resident;                 // the step as one resident launch: 1 a group of workgroups per row (resident_step.hip), 2 several rows per group (resident_rows.hip)
     ResidentSeat seat;            // ... its place at the gate (resident_gate.hip)
     ResidentArgs res_args, *res_args_dev;
     unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
@@ -608,7 +609,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
     return MRS_OK;
 }
 
-// Resident step (resident_step.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
+// Resident step (resident_step.hip, resident_rows.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
 // for the steps that do not get a turn.
 static void choose_resident(mrs_backbone *bb) {
     const mrs_m1_config &c = bb->cfg;
@@ -617,14 +618,18 @@ static void choose_resident(mrs_backbone *bb) {
     ResidentArgs &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.ds = c.d_state; a.dc = c.d_conv; a.dr = bb->dr; a.xd = bb->xd;
-    if (bb->batch > kRollMax || !resident_plan(a, bb->dtype) || a.G * a.batch > kRollMax || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
-    bb->resident = 1;
+    // A group of workgroups per row where all of them fit, else rows by the group.  Of groups of 128 only one is better off alone (24 layers of
+    // d_model 1024: one row 261 us against 281, two 302 against 286; of 768, groups of 64: three rows 210 against 234, four 236 against 238).
+    const bool one = bb->batch <= kRollMax && resident_plan(a, bb->dtype) && a.G * a.batch <= kRollMax && (a.G <= 64 || bb->batch == 1);
+    if (!one && !resident_rows_plan(a, bb->dtype)) return;
+    if (!resident_claim(bb->seat, bb->device, a.G * a.groups, bb->stream)) return;
+    bb->resident = one ? 1 : 2;
 }
 
 static int arm_resident(mrs_backbone *bb) {
     const ResidentArgs &a = bb->res_args;
-    MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.batch * a.xch_stride * 8, bb->stream));
-    MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.xch, 0, (size_t)a.groups * a.xch_stride * 8, bb->stream));
+    MRS_HIP(hipMemsetAsync(a.epoch, 0, ((size_t)a.groups * 32 + kRollHead + kRollMax) * 4, bb->stream));
     *bb->res_broken = 0;
     bb->seat.unseen = bb->seat.told = false;
     return MRS_OK;
@@ -636,14 +641,15 @@ static int setup_resident(mrs_backbone *bb) {
     ResidentArgs &a = bb->res_args;
     a.input = bb->identity_proj ? bb->d_input : bb->step_s.residual;
     a.norm_f = bb->norm_f; a.conv_state = bb->conv_state; a.ssm_state = bb->ssm_state; a.temporal = bb->temporal; a.temporal_t = bb->temporal_t;
-    MRS_TRY(dev_alloc(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
-    MRS_TRY(dev_alloc(bb, (void **)&a.epoch, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4));
-    a.roll = a.epoch + (size_t)a.batch * 32;
+    MRS_TRY(dev_alloc(bb, (void **)&a.xch, (size_t)a.groups * a.xch_stride * 8));
+    MRS_TRY(dev_alloc(bb, (void **)&a.epoch, ((size_t)a.groups * 32 + kRollHead + kRollMax) * 4));
+    a.roll = a.epoch + (size_t)a.groups * 32;
+    if (bb->resident == 2) MRS_TRY(dev_alloc(bb, &a.rows_buf, resident_rows_bytes(a)));
     a.wait = kResidentWait;
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident(bb));
-    const size_t per_layer = resident_layer_bytes(a);
+    const size_t per_layer = bb->resident == 1 ? resident_layer_bytes(a) : resident_rows_layer_bytes(a);
     char *w = nullptr;
     MRS_TRY(dev_alloc(bb, (void **)&w, per_layer * (size_t)L));
     a.weights = w; a.norm_w = bb->layers[0].norm_w;
@@ -655,7 +661,7 @@ static int setup_resident(mrs_backbone *bb) {
         }
         const ResidentLayer rl = {d.in_proj_t, d.out_proj_t, d.x_proj, d.dt_w_t, d.a_neg, d.conv_w, d.conv_b, d.D, d.dt_b,
                                   l + 1 < L ? bb->layers[l + 1].norm_w : nullptr};
-        MRS_TRY(launch_resident_pack(bb->stream, a, w, rl));
+        MRS_TRY(bb->resident == 1 ? launch_resident_pack(bb->stream, a, w, rl) : launch_resident_rows_pack(bb->stream, a, w, rl));
     }
     MRS_TRY(dev_alloc(bb, (void **)&bb->res_args_dev, sizeof(ResidentArgs)));
     MRS_HIP(hipMemcpyAsync(bb->res_args_dev, &a, sizeof(ResidentArgs), hipMemcpyHostToDevice, bb->stream));
@@ -900,7 +906,7 @@ static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
         const ResidentTurn turn(&bb->seat);
         if (turn.go()) {
             if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
-            return launch_resident_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+            return (bb->resident == 1 ? launch_resident_step : launch_resident_rows)(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
         }
     }
     if (bb->tiny_layers) {

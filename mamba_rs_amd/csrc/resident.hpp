@@ -127,16 +127,16 @@ template <typename V> __device__ __forceinline__ V ld_off(const void *base, unsi
 
 // One wave copies the 1 KB pieces first, first + step, ... below `pieces` of contiguous memory to LDS byte address `to` (both 16-byte
 // aligned) without passing through registers.  The compiler's wait counting does not see it: dma_wait() by the same wave and a
-// workgroup barrier come before the data is read.  Requests are spaced (s_sleep 1: 64 clocks): a compute unit's requests are
+// workgroup barrier come before the data is read.  Requests are spaced (s_sleep: 64 clocks each): a compute unit's requests are
 // served in order, and a burst of them would stand in front of the exchange's stores and polls.
-__device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int first, int pieces, int step) {
+template <int SLEEP = 1> __device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int first, int pieces, int step) {
     const u64 at = (u64)(uintptr_t)from;   // the same for the whole wave
     const u64 src = (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)at) | (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32;
     const unsigned lane16 = (unsigned)(threadIdx.x & 63) * 16u, dst0 = __builtin_amdgcn_readfirstlane(to);
 #pragma unroll 1
     for (int i = first; i < pieces; i += step) {
         const unsigned voff = (unsigned)i * 1024u + lane16, dst = dst0 + (unsigned)i * 1024u;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_sleep 1" ::"s"(dst), "v"(voff), "s"(src) : "m0", "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_sleep %3" ::"s"(dst), "v"(voff), "s"(src), "n"(SLEEP) : "m0", "memory");
     }
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }

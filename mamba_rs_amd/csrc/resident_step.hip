@@ -16,44 +16,16 @@
 // once, and code that does not stay in the instruction cache costs more than the work (the same step with the weights in
 // registers and unrolled loops, 100 KB of code: 427 us for 24 layers of d_model 768; with vector dot products whose sizes are
 // run-time values, 30 KB: 285 to 340 us).
-#include "resident.hpp"
+#include "resident_m1.hpp"
 
 namespace mrs {
 namespace {
 
-constexpr int kDs = 16, kDc = 4;           // states and conv taps of a channel
-constexpr int kMaxNc = 24, kMaxOc = 16, kMaxXd = 96, kMaxDr = 64;   // bounds of the fixed LDS areas
 // Lines of exchange 2 per workgroup, a wave each.
 __host__ __device__ constexpr int share_lines(int xd) { return (xd + kLineVals - 1) / kLineVals; }
 static_assert(share_lines(kMaxXd) <= kComputeWaves, "");
 constexpr int kInSteps = 4, kInTiles = 2 * kMaxNc / 16, kOutSteps = 8;      // k-steps of 32 per computing wave and 16-column tiles held in registers
 
-// What a workgroup needs of a layer besides the two big weights, as one block (byte offsets): x_proj rows [nc / 8][xd][8], dt weights
-// [nc][dr], A [nc][16], conv taps [nc][4], conv bias, D, dt bias [nc], the next layer's norm weight for its columns [oc].
-struct SmallBlock { int xw, dtw, aneg, cw, cb, D, dtb, nw, bytes; };
-__host__ __device__ inline SmallBlock small_block(int nc, int oc, int xd, int dr) {
-    SmallBlock o;
-    o.xw = 0;
-    o.dtw = o.xw + nc * xd * 2;
-    o.aneg = o.dtw + nc * dr * 2;
-    o.cw = o.aneg + nc * kDs * 4;
-    o.cb = o.cw + nc * kDc * 4;
-    o.D = o.cb + nc * 4;
-    o.dtb = o.D + nc * 4;
-    o.nw = o.dtb + nc * 4;
-    o.bytes = up1k(o.nw + oc * 4);
-    return o;
-}
-// A workgroup's part of a layer in memory: in_proj columns [dm / 8][2 nc][8], out_proj columns [di / 8][oc][8], the small block, each
-// padded to whole kilobytes.
-struct LayerBlock { int out, small, bytes; };
-__host__ __device__ inline LayerBlock layer_block(int dm, int di, int nc, int oc, int xd, int dr) {
-    LayerBlock o;
-    o.out = up1k(2 * nc * dm * 2);
-    o.small = o.out + up1k(oc * di * 2);
-    o.bytes = o.small + small_block(nc, oc, xd, dr).bytes;
-    return o;
-}
 struct Fix {   // LDS: what has a small bound lies at fixed offsets, the weights and rows behind it (bytes)
     static constexpr int pre = 0, pre2 = pre + kComputeWaves * 2 * kMaxNc * 4, us = pre2 + kComputeWaves * 16 * 4, zs = us + 64,
                          xdl = zs + 128, inv = xdl + kMaxXd * 4, xs = inv + 64;
@@ -325,6 +297,7 @@ bool resident_plan(ResidentArgs &a, int dtype) {
         a.G = a.di / a.nc;
         a.oc = a.dm / a.G;
         if (!plan_ok(a)) continue;
+        a.groups = a.batch; a.rows = 1; a.rows_buf = nullptr;
         a.xch_stride = ((size_t)a.G * share_lines(a.xd) * 8 + a.dm / 2 + a.G + a.di / 2 + 7) / 8 * 8;   // (lines of 64 bytes)
         return true;
     }

@@ -20,6 +20,13 @@ from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtyp
     (768, 2, 768, 1),     # 24 channels and 12 out_proj columns per workgroup
     (768, 2, 768, 4),
     (1024, 2, 1024, 2),   # the widest: 128 workgroups per row, four and eight k-steps per wave
+    # several rows per group of workgroups (resident_rows.hip)
+    (256, 2, 20, 9),      # input projection; eight groups of one row and of two
+    (256, 2, 256, 128),   # full groups; dt_rank 16: a k-step of dt_proj with zeros behind it
+    (512, 2, 512, 37),    # groups of nine rows and of ten: the second wave that writes operands has one or two
+    (768, 2, 768, 5),     # groups of two rows and of one; 24 channels: a channel tile that is half empty
+    (768, 2, 768, 64),    # full groups, three k-steps per wave
+    (1024, 2, 1024, 31),  # two groups of 128 workgroups, sixteen and fifteen rows
 ])
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
 def test_resident_step_follows_the_cpu_route(shape, dtype):
@@ -153,6 +160,8 @@ def _family(family, rows=4):
     from mamba_rs_amd import GpuMamba3Backbone, GpuMamba3LM, GpuMambaLM
     if family == "m1":
         return lambda: _engines((768, 3, rows), 1)[0], 768, GpuMambaLM
+    if family == "m1rows":      # four rows on one group of 128 workgroups (resident_rows.hip)
+        return lambda: _engines((1024, 3, rows), 1)[0], 1024, GpuMambaLM
     from test_m3_engine_gpu import perturbed
     from test_resident_m3_gpu import cfg_
     cfg = cfg_(256, 16, 16, 1, 3)
@@ -161,7 +170,7 @@ def _family(family, rows=4):
     return lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, 256, rows, WeightDtype.BF16), 256, GpuMamba3LM
 
 
-@pytest.mark.parametrize("family", ["m1", "m3"])
+@pytest.mark.parametrize("family", ["m1", "m3", "m1rows"])
 def test_a_caller_s_capture_gets_the_kernel_chain(family, monkeypatch):
     """step_gpu_only and a language model's decode_step captured by the caller on the engine's stream: the graph holds the kernel
     chain (its replays take no turns), so every replay, with eager work in between, leaves the bits of an engine that has only the
@@ -256,7 +265,7 @@ def _states(e):
     return out
 
 
-@pytest.mark.parametrize("family", ["m1", "m3"])
+@pytest.mark.parametrize("family", ["m1", "m3", "m1rows"])
 def test_a_step_that_finds_no_places(family, monkeypatch):
     """A wait of 0 calls every resident launch off.  step() then has the kernel chain's bits, from whatever state it started in; queued
     steps leave the state alone and raise at the next call that waits for them, however many there are; after a reset the engine
@@ -307,7 +316,7 @@ def test_a_step_that_finds_no_places(family, monkeypatch):
         e.close()
 
 
-@pytest.mark.parametrize("family", ["m1", "m3"])
+@pytest.mark.parametrize("family", ["m1", "m3", "m1rows"])
 def test_a_reset_waits_for_the_steps_before_it(family):
     """Steps that are called off while a reset is already asked for: the reset waits for them, says once that they were lost, and the
     engine steps as a fresh one; a second reset has nothing to say."""
