@@ -284,6 +284,11 @@ struct LmHooks {
     size_t (*state_bytes)(void *self);               // recurrent state, for save / restore around a warm-up run
     int (*state_copy)(void *self, void *buf, int restore);
     int (*prefill)(void *self, const int *dev_tokens, const void *embed, int vocab, int T);   // tokens [batch, T] on device
+    // Prompts of a generation, prefix_steps steps at a time: prefix_rows gives the f32 rows [batch * steps, d_model] to fill (null: no such route),
+    // prefix_run advances the states by so many steps of them.
+    float *(*prefix_rows)(void *self);
+    int (*prefix_run)(void *self, int steps);
+    int prefix_steps;
     ResidentSeat *seat;       // the engine's seat for resident steps: a graph with a step in it is replayed in a ResidentTurn
     int (*check)(void *self); // after a synchronisation: an error if a step could not be completed
     bool (*go_on_chain)(void *self);   // after a synchronisation: the one step since the last check was called off, the next ones are kernel chains

@@ -21,6 +21,7 @@
 #include "glue.hpp"
 #include "gemm_tune.hpp"
 #include "host_io.hpp"
+#include "scan_quad.hpp"
 #include <rocblas/rocblas.h>
 #include <stdlib.h>
 #include <new>
@@ -181,6 +182,15 @@ __global__ __launch_bounds__(256) void gen_seen_prompt_kernel(GenSlots g, const 
     }
 }
 
+// Embedding rows of prompt tokens t0 .. t0 + gridDim.x - 1 of every slot: rows[slot][t][dm] f32.
+template <typename T>
+__global__ __launch_bounds__(256) void gen_prefix_kernel(float *__restrict__ rows, const T *__restrict__ embed, GenSlots g, const GenDyn *__restrict__ dyn, int t0, int dm, int vocab) {
+    const int slot = blockIdx.y, t = blockIdx.x;
+    const int tok = min(max(dyn->prompts[g.prompt_off[slot] + t0 + t], 0), vocab - 1);   // (clamped as embed_gather_kernel does)
+    float *out = rows + ((int64_t)slot * gridDim.x + t) * dm;
+    for (int i = threadIdx.x; i < dm; i += 256) out[i] = Store<T>::ld(embed + (int64_t)tok * dm + i);
+}
+
 // After a step: slots still inside their prompt take the next prompt token; slots past it take the sampled token,
 // unless it is an EOS id or max_tokens are out already -- then the slot is finished (gpu_lm.rs:494-511).  Also
 // marks which slots sample after the next step (prompt consumed, not finished) and counts the running ones.
@@ -299,7 +309,7 @@ struct mrs_backbone {
     float *conv_state, *ssm_state;
     float *d_input, *temporal;
     void *temporal_t;  // decode: temporal once more in the storage type (16-bit engines), the LM head's operand
-    Scratch step_s, prefill_s;
+    Scratch step_s, prefill_s, prefix_s;   // prefix_s: a generation's prompt, made at the first one
     float *prefill_in;  // [batch*T, input_dim] f32 staging for host input
     hipGraph_t graph;
     hipGraphExec_t graph_exec;
@@ -512,7 +522,8 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
 // d_inner 5120 300 rows 174 / 168, 1024 rows 241 / 246).
 static bool own_xproj(const LayerDev &lw, int64_t rows, int xd) { return lw.x_proj_p && (rows + 15) / 16 * ((xd + 15) / 16) <= 2 * 256; }
 
-static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
+// prefix: a piece of a generation's prompt, of which the states alone are wanted
+static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) {
     const int dm = bb->cfg.d_model, di = bb->di, ds = bb->cfg.d_state, dc = bb->cfg.d_conv, dr = bb->dr, xd = bb->xd;
     const int B = bb->batch, dt = bb->dtype;
     const int64_t rows = (int64_t)B * T;
@@ -566,29 +577,35 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T) {
             } else {
                 MRS_TRY(gemm_rm(bb, dt, s->xdbl, xd, s->u, di, lw.x_proj, (int)rows, xd, di));
             }
-            if (lw.dt_w_t && dt_proj_softplus_ok(dt, di, dr, xd, s->delta, s->xdbl, lw.dt_w_t)) {
-                // dt_proj + bias + softplus in one matrix-core kernel (K = dt_rank is tiny: the op is one write of delta)
-                MRS_TRY(launch_dt_proj_softplus(bb->stream, dt, s->delta, s->xdbl, xd, lw.dt_w_t, lw.dt_b, rows, di, dr));
+            if (prefix) {   // delta stays in f32, as the steps of these tokens would have kept it (prefix_ok has looked at the shapes)
+                MRS_TRY(launch_scan_quad(bb->stream, dt, 2, {ssm, s->y, nullptr, s->u, xb + es * dr, xb + es * (dr + ds), z, xd, 2 * di, lw.a_neg, lw.D, nullptr, nullptr, nullptr,
+                                                             B, T, di, (di + 63) / 64, 1, T, s->xdbl, lw.dt_w_t, lw.dt_b, dr}));
             } else {
-            MRS_TRY(gemm_rm(bb, dt, s->delta, di, s->xdbl, xd, lw.dt_w, (int)rows, di, dr));
-            const int64_t n = rows * di;
-            MRS_DISPATCH_DTYPE(dt, T_, {
-                constexpr int VEC = 16 / (int)sizeof(T_);
-                if (di % VEC == 0)
-                    hipLaunchKernelGGL((bias_softplus_kernel<T_, VEC>), dim3((unsigned)((n / VEC + 255) / 256)), dim3(256), 0, bb->stream, (T_ *)s->delta, lw.dt_b, n, di);
-                else
-                    hipLaunchKernelGGL((bias_softplus_kernel<T_, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, (T_ *)s->delta, lw.dt_b, n, di);
-            });
-            MRS_TRY(check_launch("bias_softplus_kernel"));
+                if (lw.dt_w_t && dt_proj_softplus_ok(dt, di, dr, xd, s->delta, s->xdbl, lw.dt_w_t)) {
+                    // dt_proj + bias + softplus in one matrix-core kernel (K = dt_rank is tiny: the op is one write of delta)
+                    MRS_TRY(launch_dt_proj_softplus(bb->stream, dt, s->delta, s->xdbl, xd, lw.dt_w_t, lw.dt_b, rows, di, dr));
+                } else {
+                MRS_TRY(gemm_rm(bb, dt, s->delta, di, s->xdbl, xd, lw.dt_w, (int)rows, di, dr));
+                const int64_t n = rows * di;
+                MRS_DISPATCH_DTYPE(dt, T_, {
+                    constexpr int VEC = 16 / (int)sizeof(T_);
+                    if (di % VEC == 0)
+                        hipLaunchKernelGGL((bias_softplus_kernel<T_, VEC>), dim3((unsigned)((n / VEC + 255) / 256)), dim3(256), 0, bb->stream, (T_ *)s->delta, lw.dt_b, n, di);
+                    else
+                        hipLaunchKernelGGL((bias_softplus_kernel<T_, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, (T_ *)s->delta, lw.dt_b, n, di);
+                });
+                MRS_TRY(check_launch("bias_softplus_kernel"));
+                }
+                // ScanMode::use_parallel picks the route (src/mamba_ssm/gpu/prefill.rs:910-956)
+                unsigned flags = MRS_GATE_SILU | MRS_SCAN_FLAGS_ZERO | (lw.s4d ? MRS_A_S4D_REAL : 0);
+                // An explicit mode is honoured; in Auto the op picks the kernel itself (same recurrence, same tolerance).
+                if (bb->cfg.scan_mode == MRS_SCAN_SEQUENTIAL) flags |= MRS_FORCE_SEQUENTIAL;
+                else if (bb->cfg.scan_mode == MRS_SCAN_PARALLEL && ds == 16 && T >= 64) flags |= MRS_FORCE_PARALLEL;
+                MRS_TRY(mrs_ssm_scan_fwd_ex(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg,
+                                            lw.D, z, 2 * di, flags, s->scan_ws, s->scan_ws_bytes, B, T, di, ds));
             }
-            // ScanMode::use_parallel picks the route (src/mamba_ssm/gpu/prefill.rs:910-956)
-            unsigned flags = MRS_GATE_SILU | MRS_SCAN_FLAGS_ZERO | (lw.s4d ? MRS_A_S4D_REAL : 0);
-            // An explicit mode is honoured; in Auto the op picks the kernel itself (same recurrence, same tolerance).
-            if (bb->cfg.scan_mode == MRS_SCAN_SEQUENTIAL) flags |= MRS_FORCE_SEQUENTIAL;
-            else if (bb->cfg.scan_mode == MRS_SCAN_PARALLEL && ds == 16 && T >= 64) flags |= MRS_FORCE_PARALLEL;
-            MRS_TRY(mrs_ssm_scan_fwd_ex(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg,
-                                        lw.D, z, 2 * di, flags, s->scan_ws, s->scan_ws_bytes, B, T, di, ds));
         }
+        if (prefix && l + 1 == L) return MRS_OK;
         if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
         else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));
@@ -1024,6 +1041,31 @@ extern "C" int mrs_backbone_alloc_prefill_scratch(mrs_backbone *bb, int T) {
     return rc;
 }
 
+// A generation's prompt, as far as all slots have one: kPrefixSteps steps at a time through the prefill's kernels, whose products take
+// batch * steps rows in one launch where a step takes batch.  The activations' buffers are the engine's from the first such prompt on.
+constexpr int kPrefixSteps = 32;
+static bool prefix_ok(const mrs_backbone *bb) {
+    const LayerDev &lw = bb->layers[0];
+    return bb->skinny && bb->dtype != MRS_F32 && bb->cfg.d_state == 16 && bb->cfg.scan_mode != MRS_SCAN_SEQUENTIAL && lw.in_proj_t && lw.out_proj_t &&
+           (int64_t)bb->batch * kPrefixSteps * bb->di <= 0x7fffffffLL / 2 && scan_quad_dt_ok(bb->dtype, kPrefixSteps, bb->dr, bb->xd, lw.dt_w_t, lw.dt_w_t);
+}
+static float *m1_hook_prefix_rows(void *self) {
+    mrs_backbone *bb = (mrs_backbone *)self;
+    if (!prefix_ok(bb)) return nullptr;
+    if (!bb->prefix_s.rows) {
+        const size_t mark = bb->allocs.size();
+        if (alloc_scratch(bb, &bb->prefix_s, (int64_t)bb->batch * kPrefixSteps, kPrefixSteps)) {   // no room: step by step
+            (void)hipGetLastError();
+            for (size_t i = mark; i < bb->allocs.size(); i++) hipFree(bb->allocs[i]);
+            bb->allocs.resize(mark);
+            bb->prefix_s = Scratch();
+            return nullptr;
+        }
+    }
+    return bb->prefix_s.residual;
+}
+static int m1_hook_prefix_run(void *self, int T) { return run_layers((mrs_backbone *)self, &((mrs_backbone *)self)->prefix_s, T, true); }
+
 extern "C" int mrs_backbone_prefill_device(mrs_backbone *bb, const float *input_dev, int T) {
     if (!bb || !input_dev) return fail(MRS_E_NULL, "mrs_backbone_prefill_device: null pointer");
     MRS_TRY(mrs_backbone_alloc_prefill_scratch(bb, T));
@@ -1204,6 +1246,7 @@ static LmHooks m1_hooks(mrs_backbone *bb) {
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
     h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy; h.prefill = m1_hook_prefill;
+    h.prefix_rows = m1_hook_prefix_rows; h.prefix_run = m1_hook_prefix_run; h.prefix_steps = kPrefixSteps;
     h.seat = &bb->seat; h.check = m1_hook_check; h.go_on_chain = m1_hook_go_on_chain;
     return h;
 }
@@ -1446,6 +1489,21 @@ static int gen_forward(mrs_lm *lm) {
     return lm_logits(lm);
 }
 
+// The slots' first n prompt tokens, in pieces of nearly equal length through the engine's prefill kernels.
+static int gen_prefix(mrs_lm *lm, int n) {
+    const LmHooks *bb = &lm->eng;
+    float *rows = bb->prefix_rows(bb->self);
+    const int pieces = (n + bb->prefix_steps - 1) / bb->prefix_steps;
+    for (int i = 0; i < pieces; i++) {
+        const int t0 = (int)((int64_t)n * i / pieces), T = (int)((int64_t)n * (i + 1) / pieces) - t0;
+        MRS_DISPATCH_DTYPE(lm->dtype, T_, hipLaunchKernelGGL((gen_prefix_kernel<T_>), dim3((unsigned)T, (unsigned)lm->batch), dim3(256), 0, bb->stream, rows, (const T_ *)lm->embed,
+                                                             lm->gen, lm->gen_dyn, t0, lm->dm, lm->vocab));
+        MRS_TRY(check_launch("gen_prefix_kernel"));
+        MRS_TRY(bb->prefix_run(bb->self, T));
+    }
+    return MRS_OK;
+}
+
 // The generation loop behind mrs_lm_generate_batch and mrs_lm_generate_streaming.  With a callback (batch 1) the host
 // looks at the slot after every step instead of every 16th and hands each new token over as it appears (*handed: how many).  on_chain:
 // every step is the kernel chain.
@@ -1495,14 +1553,18 @@ static int gen_loop(mrs_lm *lm, const int *prompts, const int *prompt_lens, cons
     std::vector<mrs_sampler> samplers(B);
     std::vector<unsigned long long> rng((size_t)B * 4);
     const bool prefill_route = seen_includes_prompt && B == 1 && prompt_lens[0] >= 256;   // PREFILL_PARALLEL_THRESHOLD, gpu_lm.rs:48
+    // what all slots' prompts have in front of their last token goes through prefill kernels (a slot without a prompt: none)
+    int common = prefill_route ? 0 : max_prompt - 1;
+    for (int i = 0; i < B; i++) common = std::min(common, prompt_lens[i] - 1);
+    if (common < 4 || !bb->prefix_rows || !bb->prefix_rows(bb->self)) common = 0;
     int64_t o = 0;
     int running = 0;
     for (int i = 0; i < B; i++) {
         off[i] = (int)o; len[i] = prompt_lens[i]; o += prompt_lens[i];
         fin[i] = prompt_lens[i] == 0;
-        pos[i] = fin[i] ? 0 : (prefill_route ? len[i] : 1);
+        pos[i] = fin[i] ? 0 : (prefill_route ? len[i] : common + 1);
         act[i] = !fin[i] && pos[i] >= len[i];
-        first[i] = fin[i] ? 0 : prompts[off[i]];
+        first[i] = fin[i] ? 0 : prompts[off[i] + common];
         mx[i] = params[i].max_tokens; neos[i] = params[i].n_eos;
         for (int e = 0; e < params[i].n_eos; e++) eos[(size_t)i * kMaxEos + e] = params[i].eos_token_ids[e];
         samplers[i] = params[i].sampler;
@@ -1528,6 +1590,10 @@ static int gen_loop(mrs_lm *lm, const int *prompts, const int *prompt_lens, cons
         MRS_TRY(mrs_lm_prefill(lm, nullptr, prompts, prompt_lens[0]));   // state after the prompt, logits of its last position
         MRS_TRY(gen_pick(lm));
         steps = max_tokens;
+    }
+    if (common) {
+        MRS_TRY(gen_prefix(lm, common));
+        steps -= common;
     }
     int done = 0, emitted = 0;
     bool stopped = false;

@@ -8,16 +8,18 @@
 //     the staged B / C rows of the chunk, which lie in LDS as f32 from the start;
 //   * activations are loaded for four steps at a time, lane g the step t + g, and handed round the four lanes by DPP operands; in the
 //     same way lane g keeps the output of step t + g, so that D u, the gate and the store happen once per four steps and lane.
+//   * a prompt of up to 64 steps can bring dt_proj along: the wave's 16 channels x 64 steps are four tiles of the matrix cores, and delta stays in
+//     f32 in LDS.  For a generation's prompt, which otherwise goes through steps that keep delta in f32; no faster than dt_proj with a
+//     rounded delta in front (24 layers, 13 x 11 rows of d_model 1024 995 / 992 us, 48 of 768 888 / 899).
 // The two passes and their workspace (chunk summaries, step sums) are those of m1_scan.hip; a short sequence is one pass.  What bounds
 // it is the issue of about 35 instructions per step and wave, four of them exponentials: 8 us per million (row, channel) steps once
 // the chip is full.  Both kernels timed: at the dispatch in m1_scan.hip.
 #include "common.hpp"
+#include "mfma_tiles.hpp"
 #include "scan_quad.hpp"
 
 namespace mrs {
 namespace {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <int K> __device__ __forceinline__ float quad_lane(float v) {   // lane K of the four
     return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), K * 0x55, 0xf, 0xf, true));
@@ -42,9 +44,12 @@ template <typename T> __device__ __forceinline__ v4f row_quad(const T *p) {
 
 // OUT false: pass A -- chunk c < nchunk - 1 from a zero state (chunk 0: the caller's, which it also copies), leaving its end state and
 // sum of delta.  OUT true: pass B -- the entering state folded from the summaries before, then y; the last chunk leaves the state.
-template <typename T, int GATE, bool OUT>
+// DT: delta is formed here.
+template <typename T, int GATE, bool OUT, bool DT = false>
 __global__ __launch_bounds__(256) void scan_quad_kernel(ScanQuadArgs a) {
-    __shared__ alignas(16) float Bs[kQuadLen][16], Cs[OUT ? kQuadLen : 1][16];
+    constexpr int kLen = DT ? kQuadDtLen : kQuadLen;
+    __shared__ alignas(16) float Bs[kLen][16], Cs[OUT ? kLen : 1][16];
+    __shared__ float Ds[DT ? kLen : 1][80];   // [step][channel of the workgroup]
     const int tile = blockIdx.x % a.tiles, rest = blockIdx.x / a.tiles, b = rest % a.batch, c = rest / a.batch;
     const int tid = threadIdx.x, lane = tid & 63, g = lane & 3, di = a.di;
     const int d = tile * 64 + (tid >> 2);
@@ -61,7 +66,7 @@ __global__ __launch_bounds__(256) void scan_quad_kernel(ScanQuadArgs a) {
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             const int64_t t = min(4 * (q0 + i) + g, ns - 1);
-            x[i] = dp[t * di];
+            if (DT) x[i] = (T)0.0f; else x[i] = dp[t * di];
             w[i] = up[t * di];
             if (GATE) z[i] = gp[t * a.gate_stride];
         }
@@ -120,6 +125,28 @@ __global__ __launch_bounds__(256) void scan_quad_kernel(ScanQuadArgs a) {
                 }
         }
     }
+    if constexpr (DT) {
+        // this wave's 16 channels: dt_proj on the matrix cores, step 16 m + 4 (l / 16) + i in register i of tile m
+        const int n = lane & 15, kg = lane >> 4, ch = min(tile * 64 + (tid >> 6) * 16 + n, di - 1), mt = (ns + 15) >> 4;
+        const T *wp = (const T *)a.dt_w + (int64_t)ch * a.dr, *xp = (const T *)a.dt_in + row0 * a.bc_stride;
+        v4f td[kLen / 16];
+#pragma unroll
+        for (int m = 0; m < kLen / 16; m++) td[m] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int k = 8 * kg; k - 8 * kg < a.dr; k += 32) {
+            const bool in = k < a.dr;
+            const uint4 none = make_uint4(0, 0, 0, 0);
+            const uint4 w = in ? *reinterpret_cast<const uint4 *>(wp + k) : none;
+#pragma unroll
+            for (int m = 0; m < kLen / 16; m++)
+                if (m < mt) td[m] = Mma32<T>::mma(in ? *reinterpret_cast<const uint4 *>(xp + (int64_t)min(16 * m + n, ns - 1) * a.bc_stride + k) : none, w, td[m]);
+        }
+        const float bias = a.dt_b[ch];
+#pragma unroll
+        for (int m = 0; m < kLen / 16; m++)
+            if (m < mt)
+#pragma unroll
+                for (int i = 0; i < 4; i++) Ds[16 * m + 4 * kg + i][(tid >> 6) * 16 + n] = softplus20(td[m][i] + bias);
+    }
     __syncthreads();
     float sd = 0.0f;
     for (int q0 = 0; q0 < nq; q0 += NB) {
@@ -129,7 +156,7 @@ __global__ __launch_bounds__(256) void scan_quad_kernel(ScanQuadArgs a) {
             const int q = q0 + i, s = 4 * q + g;
             if (q < nq) {   // (uniform)
                 const bool in = s < ns;
-                const float dl = in ? Store<T>::ld(&rd[i]) : 0.0f, uu = Store<T>::ld(&ru[i]), du = in ? dl * uu : 0.0f;
+                const float dl = !in ? 0.0f : DT ? Ds[s][tid >> 2] : Store<T>::ld(&rd[i]), uu = Store<T>::ld(&ru[i]), du = in ? dl * uu : 0.0f;
                 float y = 0.0f;
                 auto step = [&](auto kc) {
                     constexpr int k = decltype(kc)::value;
@@ -186,6 +213,13 @@ template <typename T> int launch_quad_t(hipStream_t st, int gate_mode, const Sca
         if (rc) return rc;
     }
     const dim3 grid(per * (unsigned)a.nchunk);
+    if constexpr (sizeof(T) == 2) {
+        if (a.dt_w) {
+            if (gate_mode != 2) return fail(MRS_E_SHAPE, "scan with dt_proj: gate mode %d", gate_mode);
+            hipLaunchKernelGGL((scan_quad_kernel<T, 2, true, true>), grid, dim3(256), 0, st, a);
+            return check_launch("scan_quad_kernel (dt_proj)");
+        }
+    }
     if (gate_mode == 0) hipLaunchKernelGGL((scan_quad_kernel<T, 0, true>), grid, dim3(256), 0, st, a);
     else if (gate_mode == 1) hipLaunchKernelGGL((scan_quad_kernel<T, 1, true>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((scan_quad_kernel<T, 2, true>), grid, dim3(256), 0, st, a);
@@ -194,7 +228,14 @@ template <typename T> int launch_quad_t(hipStream_t st, int gate_mode, const Sca
 
 }  // namespace
 
+bool scan_quad_dt_ok(int dtype, int T, int dr, int64_t bc_stride, const void *dt_in, const void *dt_w) {
+    return (dtype == MRS_BF16 || dtype == MRS_F16) && T >= 1 && T <= kQuadDtLen && dr >= 8 && dr % 8 == 0 && bc_stride % 8 == 0 && bc_stride >= dr && dt_w && aligned(dt_in, 16) &&
+           aligned(dt_w, 16);
+}
+
 int launch_scan_quad(hipStream_t st, int dtype, int gate_mode, const ScanQuadArgs &a) {
+    if (a.dt_w && (!scan_quad_dt_ok(dtype, a.Tlen, a.dr, a.bc_stride, a.dt_in, a.dt_w) || a.nchunk != 1 || !a.dt_b))
+        return fail(MRS_E_SHAPE, "scan with dt_proj: %d steps in %d chunks, dt_rank %d", a.Tlen, a.nchunk, a.dr);
     if (a.len < 1 || a.len > kQuadLen || a.nchunk < 1 || (int64_t)a.nchunk * a.len < a.Tlen || (int64_t)(a.nchunk - 1) * a.len >= a.Tlen || a.tiles * 64 < a.di)
         return fail(MRS_E_SHAPE, "scan: %d chunks of %d for %d steps", a.nchunk, a.len, a.Tlen);
     MRS_DISPATCH_DTYPE(dtype, T_, return launch_quad_t<T_>(st, gate_mode, a));

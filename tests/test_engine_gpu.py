@@ -448,3 +448,39 @@ def test_small_f32_models_step_in_one_launch(shape, monkeypatch):
     for t in range(steps):
         assert scaled_err(ref.step(x[t]), outs[t]) < 1e-4, t
     ref.close()
+
+
+@pytest.mark.parametrize("dm,lens,dtype", [
+    (128, (9, 5), WeightDtype.F16),              # four tokens; dt_rank 8: a quarter of a k-step of dt_proj
+    (256, (6, 40, 18), WeightDtype.BF16),        # five
+    (256, (70, 33, 81), WeightDtype.BF16),       # 32: one whole piece
+    (768, (34, 36), WeightDtype.F16),            # 33: two pieces of 16 and 17, a last tile of one step; dt_rank 48
+    (1024, (100,), WeightDtype.BF16),            # 99: four pieces
+])
+def test_prompts_of_a_generation_in_pieces(dm, lens, dtype):
+    """What all prompts have in front of their last token goes through the prefill's kernels, up to 32 steps at a time, with dt_proj inside
+    the scan: tokens are those of an engine that takes every token as a step (scan_mode SEQUENTIAL keeps the prompt out of the
+    prefill kernels), all states and the last rows within the tolerance between two routes that round at the same 16-bit points
+    (1 % in norm: three layers, each rounding its projections, u and y once)."""
+    from mamba_rs_amd import SampleParams
+    rng = np.random.default_rng(sum(lens))
+    embed = rng.standard_normal((500, dm)).astype(np.float32)
+    prompts = [rng.integers(0, 500, n).tolist() for n in lens]
+    params = [SampleParams(temperature=0.8, top_k=20, max_tokens=4, seed=i) for i in range(len(lens))]
+    out = []
+    print(f"case prompts in pieces {dm} {lens} {dtype.name}", flush=True)
+    for mode in (ScanMode.AUTO, ScanMode.SEQUENTIAL):
+        cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=3, scan_mode=mode)
+        w = MambaWeights.init(cfg, dm, 9)
+        w.input_proj_w = np.zeros((0, dm), np.float32)
+        e = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, len(lens), dtype)
+        lm = GpuMambaLM(e, embed)
+        first = lm.generate_batch(prompts, params)
+        lm.generate_batch([p[:3] for p in prompts], params)     # too short for it
+        assert lm.generate_batch(prompts, params) == first      # again, on what the others left behind
+        out.append((first, [e.download_temporal()] + [p for l in range(3) for p in e.download_state(l)]))
+        lm.close()
+        e.close()
+    assert out[0][0] == out[1][0]
+    for p, q in zip(out[0][1], out[1][1]):
+        assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
