@@ -229,16 +229,17 @@ int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const
 struct ResidentM3Layer {   // in_t [ip][d_model] and out_t [d_model][d_inner] transposed; next_nw: the norm weight after, or null
     const void *in_t, *out_t; const float *bnw, *cnw, *b_bias, *c_bias, *D, *dt_bias, *next_nw;
 };
+// row_order: the step that adds in the kernel chain's order (one row); norm_rows: every layer's norm weight, [n_layers][d_model], for it
 struct ResidentM3Args {
     const void *weights;
-    const float *input, *norm_w, *norm_f;
+    const float *input, *norm_w, *norm_f, *norm_rows;
     float *ssm, *kst, *vst, *angle, *temporal;
     unsigned long long *xch;
     unsigned *epoch, *roll, *broken;
     size_t xch_stride;
     unsigned wait;
     float eps, a_floor;
-    int n_layers, batch, dm, di, nh, hd, ds, ng, nr, G, nc, oc, ex;
+    int n_layers, batch, dm, di, nh, hd, ds, ng, nr, G, nc, oc, ex, row_order;
 };
 bool resident_m3_plan(ResidentM3Args &a, int dtype);
 size_t resident_m3_layer_bytes(const ResidentM3Args &a);

@@ -12,7 +12,7 @@
 //      registers, y = H q + D x, and the SiLU gate (optionally RMSNormGated over the head) -- the formulas of
 //      mamba3_layer_step (src/mamba3_siso/cpu/inference.rs:68-258) and kernels/mamba3_ops.cu;
 //   3. out_proj with the residual add, the next layer's pre-scaled operand and row sums of squares as epilogue.
-// At a few rows of a shallow 16-bit model the whole step is one resident launch (resident_m3_step.hip).
+// At one row of a 16-bit model, and at a few of a shallow one, the whole step is one resident launch (resident_m3_row.hip, resident_m3_step.hip).
 // Shapes the skinny GEMM does not take (f32 storage above four rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
 #include "common.hpp"
 #include "gemm_tune.hpp"
@@ -564,7 +564,7 @@ struct mrs_m3_backbone {
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)
     HostIo io;              // step()'s rows in pinned host memory
-    int resident;                 // a few rows: the step as one resident launch (resident_m3_step.hip)
+    int resident;                 // the step as one resident launch
     ResidentSeat seat;            // ... its place at the gate (resident_gate.hip)
     ResidentM3Args res_args, *res_args_dev;
     unsigned *res_broken;         // pinned host word: a resident launch gave up waiting
@@ -651,28 +651,37 @@ int project_input3(mrs_m3_backbone *bb) {
     return MRS_OK;
 }
 
-// Deepest model that takes the resident step.  It is as accurate as the kernel chain at every depth, but adds the same products in another
-// order; where an operand row is rounded to 16 bits, that rounding can fall the other way, and the difference grows from layer to layer.
+// Deepest model that takes the matrix-core resident step (resident_m3_step.hip).  It is as accurate as the kernel chain at every depth, but
+// adds the same products in another order; where an operand row is rounded to 16 bits, that rounding can fall the other way, and the
+// difference grows from layer to layer.
 // Output of 32 bf16 steps, resident against chain / chain against the f32 engine, and how many of 48 greedy passes of 32 tokens
 // leave the chain's tokens (in brackets: the chain's own two orders, row-wise and tiled, against each other):
 //   d_model 768    2 layers 0.06 / 0.31 %, 0 (0)    4 0.21 / 0.44, 1 (1)    6 0.33 / 0.54, 1 (1)    8 0.44 / 0.64, 3 (3)    24 0.92 / 1.12
 //   d_model 256    2 layers 0.03 / 0.48 %, 0 (0)    4 0.19 / 0.76, 3 (3)    6 0.31 / 0.98, 4 (4)    8 0.42 / 1.21, 10 (9)
 //   d_model 64                                      4 0.01 / 0.74, 0 (0)                            8 0.06 / 1.18, 0 (0)
 // There is no depth at which it turns.  The line lies where the difference is that of the Mamba-1 step (0.17 % at 24 layers); deeper
-// models keep the chain's tokens (24 layers of d_model 768: 212 against 281 us a step).
+// models keep the chain's tokens: at one row through the step that has the chain's bits (resident_m3_row.hip), else on the chain
+// (24 layers of d_model 768 at two rows: 230 against 317 us a step).
 constexpr int kResidentM3Layers = 4;
 
-// Resident step (resident_m3_step.hip) for the rows whose workgroups fit on the chip together.  The kernel chain stays ready beside it,
-// for the steps that do not get a turn.
+// Resident step for the rows whose workgroups fit on the chip together.  One row takes the chain's own order (resident_m3_row.hip) wherever
+// the chain is on its row-wise route, at any depth: the same bits, and the faster of the two (its comment has both).  The kernel chain
+// stays ready beside it, for the steps that do not get a turn.
 void choose_resident3(mrs_m3_backbone *bb) {
     const mrs_m3_config &c = bb->cfg;
     const char *e = getenv("MRS_DECODE_NO_RESIDENT");
     // (RMSNormGated sums over a head, whose channels lie in several workgroups: the kernel chain)
-    if ((e && atoi(e) != 0) || !bb->skinny || c.is_outproj_norm || c.n_layers > kResidentM3Layers) return;
+    if ((e && atoi(e) != 0) || !bb->skinny || c.is_outproj_norm) return;
     ResidentM3Args &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.a_floor = c.a_floor; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.nh = bb->nh; a.hd = c.headdim; a.ds = c.d_state; a.ng = c.ngroups; a.nr = bb->nr;
-    if (bb->batch > kRollMax || !resident_m3_plan(a, bb->dtype) || a.G * a.batch > kRollMax || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
+    a.row_order = bb->batch == 1 && !bb->tiled && getenv("MRS_DECODE_NO_ROWWISE") == nullptr;
+    if (bb->batch > kRollMax) return;
+    if (!a.row_order || !resident_m3_plan(a, bb->dtype)) {
+        a.row_order = 0;
+        if (c.n_layers > kResidentM3Layers || !resident_m3_plan(a, bb->dtype)) return;
+    }
+    if (a.G * a.batch > kRollMax || !resident_claim(bb->seat, bb->device, a.G * a.batch, bb->stream)) return;
     bb->resident = 1;
 }
 
@@ -698,6 +707,13 @@ int setup_resident3(mrs_m3_backbone *bb) {
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident3(bb));
+    if (a.row_order) {
+        const size_t row = (size_t)bb->cfg.d_model * 4;
+        float *rows = nullptr;
+        MRS_TRY(dev_alloc3(bb, (void **)&rows, row * L));
+        for (int l = 0; l < L; l++) MRS_HIP(hipMemcpyAsync(rows + (size_t)l * bb->cfg.d_model, bb->layers[l].norm_w, row, hipMemcpyDeviceToDevice, bb->stream));
+        a.norm_rows = rows;
+    }
     const size_t per_layer = resident_m3_layer_bytes(a);
     char *w = nullptr;
     MRS_TRY(dev_alloc3(bb, (void **)&w, per_layer * (size_t)L));

@@ -13,42 +13,15 @@
 //
 // What bounds it: three all-to-all exchanges and the chain between them, not the weights (7.4 MB a layer at d_model 768).
 // Per bf16 step, kernel chain / this (routes of one build, steps queued): four layers of d_model 64 46 / 26 us at one row and 49 / 27 at
-// 32; of d_model 256 47 / 30 at one and 50 / 33 at eight; of d_model 768 53 / 38 at one and 57 / 42 at two; 24 layers of 768 281 / 212 at one
-// and 317 / 230 at two (kept on the chain all the same, kResidentM3Layers in m3_engine.hip says why).
-#include "resident.hpp"
-#include "m3_math.hpp"
+// 32; of d_model 256 50 / 33 at eight; of d_model 768 57 / 42 at two; 24 layers of 768 317 / 230 at two (kept on the chain all the same,
+// kResidentM3Layers in m3_engine.hip says why).  One row of a width that is a multiple of 256 takes resident_m3_row.hip.
+#include "resident_m3.hpp"
 
 namespace mrs {
 namespace {
 
-constexpr int kMaxNc = 16, kMaxOc = 16, kMaxEx = 16, kMaxDs = 64;   // bounds of the fixed LDS areas and of a thread's work
 constexpr int kInSteps = 4, kInTiles = (2 * kMaxNc + kMaxEx) / 16, kOutSteps = 8;   // k-steps of 32 per computing wave, 16-column tiles
 
-// What a workgroup needs of a layer besides the two big weights (byte offsets): B and C norm weights, its head's B and C biases [ds]
-// each, the next layer's norm weight for its columns [oc], D and dt bias of its head.
-struct SmallBlock { int bnw, cnw, bb, cb, nw, D, dtb, bytes; };
-__host__ __device__ inline SmallBlock small_block(int ds, int oc) {
-    SmallBlock o;
-    o.bnw = 0;
-    o.cnw = ds * 4;
-    o.bb = 2 * ds * 4;
-    o.cb = 3 * ds * 4;
-    o.nw = 4 * ds * 4;
-    o.D = o.nw + oc * 4;
-    o.dtb = o.D + 4;
-    o.bytes = up1k(o.dtb + 4);
-    return o;
-}
-// A workgroup's part of a layer in memory: in_proj columns [dm / 8][x: nc | z: nc | shared: ex][8], out_proj columns [di / 8][oc][8], the
-// small block, each padded to whole kilobytes.
-struct LayerBlock { int out, small, bytes; };
-__host__ __device__ inline LayerBlock layer_block(int dm, int di, int cols, int oc, int ds) {
-    LayerBlock o;
-    o.out = up1k(cols * dm * 2);
-    o.small = o.out + up1k(oc * di * 2);
-    o.bytes = o.small + small_block(ds, oc).bytes;
-    return o;
-}
 struct Fix {   // LDS: what has a small bound lies at fixed offsets, the weights and rows behind it (bytes)
     static constexpr int pre = 0, pre2 = pre + kComputeWaves * 16 * kInTiles * 4, xz = pre2 + kComputeWaves * 16 * 4, kl = xz + 2 * kMaxNc * 4,
                          ql = kl + kMaxDs * 4, coef = ql + kMaxDs * 4, inv = coef + 16, xs = inv + 16;
@@ -257,7 +230,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
 struct PackArgs {
     const uint16_t *in_t, *out_t;
     const float *bnw, *cnw, *b_bias, *c_bias, *D, *dt_bias, *next_nw;
-    int dm, di, ip, ds, hd, nc, oc, ex;
+    int dm, di, ip, ds, hd, nc, oc, ex, row_order;
 };
 __global__ __launch_bounds__(256) void pack_m3_layer_kernel(char *__restrict__ dst, PackArgs p) {
     const int cols = 2 * p.nc + p.ex;
@@ -268,13 +241,13 @@ __global__ __launch_bounds__(256) void pack_m3_layer_kernel(char *__restrict__ d
     if (at >= lb.bytes) return;
     uint4 v = make_uint4(0, 0, 0, 0);
     if (at < lb.out) {
-        const int i = at >> 4, c = i % cols, k8 = i / cols;
+        const int i = at >> 4, n8 = p.dm >> 3, c = p.row_order ? i / n8 : i % cols, k8 = p.row_order ? i % n8 : i / cols;
         // in_proj's columns are [z: di | x: di | shared]
         const int col = c < p.nc ? p.di + c0 + c : c < 2 * p.nc ? c0 + c - p.nc : 2 * p.di + s * p.ex + c - 2 * p.nc;
-        if (k8 < p.dm >> 3 && col < p.ip) v = *reinterpret_cast<const uint4 *>(p.in_t + (size_t)col * p.dm + k8 * 8);
+        if (k8 < n8 && c < cols && col < p.ip) v = *reinterpret_cast<const uint4 *>(p.in_t + (size_t)col * p.dm + k8 * 8);
     } else if (at < lb.small) {
-        const int i = (at - lb.out) >> 4, c = i % p.oc, k8 = i / p.oc;
-        if (k8 < p.di >> 3) v = *reinterpret_cast<const uint4 *>(p.out_t + (size_t)(o0 + c) * p.di + k8 * 8);
+        const int i = (at - lb.out) >> 4, n8 = p.di >> 3, c = p.row_order ? i / n8 : i % p.oc, k8 = p.row_order ? i % n8 : i / p.oc;
+        if (k8 < n8 && c < p.oc) v = *reinterpret_cast<const uint4 *>(p.out_t + (size_t)(o0 + c) * p.di + k8 * 8);
     } else {
         const int q = at - lb.small;
         unsigned w[4] = {0, 0, 0, 0};
@@ -304,21 +277,21 @@ bool shape_ok(const ResidentM3Args &a, int dtype) {
 bool plan_ok(const ResidentM3Args &a) {
     return (a.nc == 8 || a.nc == 16) && a.hd % a.nc == 0 && a.nc * a.G == a.di && a.oc >= 2 && a.oc % 2 == 0 && a.oc <= kMaxOc && a.oc * a.G == a.dm &&
            a.ex >= 1 && a.ex <= kMaxEx && a.ex * a.G >= shared_cols(a) &&
-           (size_t)res_lds(a.dm, a.di, 2 * a.nc + a.ex, a.oc, a.ds).total <= kResLdsMax;
+           (a.row_order ? resident_m3_row_lds(a) : (size_t)res_lds(a.dm, a.di, 2 * a.nc + a.ex, a.oc, a.ds).total) <= kResLdsMax;
 }
 
 }  // namespace
 
-// A workgroup's channels belong to one head; as few workgroups as the plan allows, as in resident_plan().
+// (a.row_order set: the plan of resident_m3_row.hip.)  A workgroup's channels belong to one head; as few workgroups as the plan allows, as in resident_plan().
 bool resident_m3_plan(ResidentM3Args &a, int dtype) {
-    if (!shape_ok(a, dtype)) return false;
+    if (!shape_ok(a, dtype) || (a.row_order && !resident_m3_row_ok(a, dtype))) return false;
     for (a.nc = kMaxNc; a.nc >= 8; a.nc -= 8) {
         if (a.di % a.nc) continue;
         a.G = a.di / a.nc;
         a.oc = a.dm / a.G;
         a.ex = (shared_cols(a) + a.G - 1) / a.G;
         if (!plan_ok(a)) continue;
-        a.xch_stride = (size_t)(a.dm / 2 + a.G + shared_cols(a) + a.di / 2);
+        a.xch_stride = (size_t)((a.row_order ? a.dm : a.dm / 2 + a.G) + shared_cols(a) + a.di / 2);
         return true;
     }
     return false;
@@ -328,7 +301,7 @@ size_t resident_m3_layer_bytes(const ResidentM3Args &a) { return (size_t)a.G * l
 
 int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, const ResidentM3Layer &w) {
     const PackArgs p = {(const uint16_t *)w.in_t, (const uint16_t *)w.out_t, w.bnw, w.cnw, w.b_bias, w.c_bias, w.D, w.dt_bias, w.next_nw,
-                        a.dm, a.di, 2 * a.di + shared_cols(a), a.ds, a.hd, a.nc, a.oc, a.ex};
+                        a.dm, a.di, 2 * a.di + shared_cols(a), a.ds, a.hd, a.nc, a.oc, a.ex, a.row_order};
     const int n16 = layer_block(a.dm, a.di, 2 * a.nc + a.ex, a.oc, a.ds).bytes / 16;
     hipLaunchKernelGGL(pack_m3_layer_kernel, dim3((unsigned)((n16 + 255) / 256), (unsigned)a.G), dim3(256), 0, st, (char *)dst, p);
     return check_launch("pack_m3_layer_kernel");
@@ -347,6 +320,7 @@ int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, 
     if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.G * a.batch > kRollMax || a.n_layers < 1 || !a.weights || !a.norm_w || !a.norm_f || !a.input || !a.xch || !a.epoch ||
         !a.roll || !a.broken || !a.temporal || !a.ssm || !a.kst || !a.vst || !a.angle || !dev)
         return fail(MRS_E_SHAPE, "resident Mamba-3 step: shape outside the route (d_model=%d d_inner=%d d_state=%d workgroups=%d)", a.dm, a.di, a.ds, a.G);
+    if (a.row_order) return launch_resident_m3_row(st, dtype, a, dev);
     return dtype == MRS_BF16 ? launch_resident_m3_t<bf16_t>(st, a, dev) : launch_resident_m3_t<f16_t>(st, a, dev);
 }
 

@@ -90,3 +90,44 @@ def test_deep_models_keep_the_kernel_chain(layers, route, monkeypatch):
     assert rel == 0 if route == 1 else rel < 4e-3
     a.close()
     chain.close()
+
+
+@pytest.mark.parametrize("cfg,idim,dtype", [
+    (cfg_(256, 16, 16, 1, 6), 256, WeightDtype.BF16),              # 32 lanes per row of in_proj, 4 lanes per state row
+    (cfg_(256, 64, 64, 4, 5, 1.0), 20, WeightDtype.F16),           # input projection, every coordinate rotated, 16 shared columns cut short
+    (cfg_(512, 32, 32, 2, 5, 1.0), 512, WeightDtype.BF16),         # 64 lanes per row, one piece each; 8 lanes per state row
+    (cfg_(512, 32, 8, 1, 5), 512, WeightDtype.F16),                # eight channels and four columns of out_proj per workgroup: idle waves
+    (cfg_(768, 64, 64, 1, 3), 768, WeightDtype.F16),
+    (cfg_(1024, 64, 64, 1, 2), 1024, WeightDtype.BF16),
+])
+def test_one_row_keeps_the_chain_s_bits(cfg, idim, dtype, monkeypatch):
+    """One row at any depth: one launch, and output and states are the kernel chain's bit for bit -- eager, replayed, in steps that
+    are called off and run on the chain in between, and with infinities in the input (where the chain has NaN, NaN)."""
+    w = perturbed(cfg, idim, 13)
+    if idim == cfg.d_model:
+        w.input_proj_w = np.zeros(0, np.float32)
+    print(f"case one row d_model={cfg.d_model} d_state={cfg.d_state} headdim={cfg.headdim} groups={cfg.ngroups} {dtype.name}", flush=True)
+    a = GpuMamba3Backbone.new_with_dtype(0, w, cfg, idim, 1, dtype)
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = GpuMamba3Backbone.new_with_dtype(0, w, cfg, idim, 1, dtype)
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    same = lambda p, q: np.array_equal(p, q, equal_nan=True)
+    x = np.random.default_rng(idim).standard_normal((12, 1, idim)).astype(np.float32)
+    x[11, 0, 3] = np.inf
+    for t, r in enumerate(x):
+        if t == 4:
+            a.capture_graph()
+        if t == 8:      # (the state is not touched by a launch that is called off)
+            a.set_resident_wait(0)
+        assert same(a.step(r), chain.step(r)), t
+        if t >= 10:
+            continue
+        for l in range(cfg.n_layers):
+            assert all(same(p, q) for p, q in zip(a.download_state(l), chain.download_state(l))), (t, l)
+    a.reset()
+    chain.reset()
+    a.set_resident_wait(1 << 23)
+    for r in x:
+        assert same(a.step(r), chain.step(r))
+    for e in (a, chain):
+        e.close()
