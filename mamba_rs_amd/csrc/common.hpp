@@ -153,6 +153,9 @@ int skinny_max_rows();   // rows the 16-bit matrix-core route takes (128; MRS_SK
 bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, const void *Wt);
 int launch_skinny_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wt,
                        int M, int N, int K, const SkinnyEpi &ep);
+// out_proj of a prefill's last layer: of [batch * T] rows the last of every T, in place (the others of C are left alone)
+bool last_step_gemm_ok(int dtype, const void *A, const void *Wt, int batch, int T, int N, int K);
+int launch_last_step_gemm(hipStream_t st, int dtype, void *C, const void *A, const void *Wt, int batch, int T, int N, int K);
 int launch_transpose(hipStream_t st, int dtype, void *Wt, const void *W, int K, int N);
 // delta[r, d] = softplus(round(dt_in[r, :] . wt[d, :]) + bias[d]) for 16-bit storage; wt is the transposed [d_inner][dt_rank] weight
 // A whole f32 backbone step in one launch for small models (one workgroup per batch row; csrc/tiny_step.hip).  All

@@ -606,7 +606,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
             }
         }
         if (prefix && l + 1 == L) return MRS_OK;
-        if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
+        if (l + 1 == L && last_step_gemm_ok(dt, s->y, lw.out_proj_t, B, T, dm, di)) MRS_TRY(launch_last_step_gemm(bb->stream, dt, s->out, s->y, lw.out_proj_t, B, T, dm, di));
+        else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
         else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));
     }

@@ -1293,7 +1293,9 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             MRS_TRY(mrs_m3_seq_fwd(bb->stream, dt, ssm, kst, vst, bb->pf_y, bb->pf_x, bb->pf_K, bb->pf_Q, al, be, ga, lw.D, B, T, nh, hd, ds));
         }
         if (!gate_in_scan) MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_gate_t<T_>(bb, lw, rows, bulk, ldb)));
-        if (own_projection(dt, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
+        if (l + 1 == L && last_step_gemm_ok(dt, bb->pf_gated, lw.out_proj_t, B, T, dm, di))
+            MRS_TRY(launch_last_step_gemm(bb->stream, dt, bb->pf_out, bb->pf_gated, lw.out_proj_t, B, T, dm, di));
+        else if (own_projection(dt, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
             MRS_TRY(launch_mid_gemm(bb->stream, dt, 0, bb->pf_out, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di));
         else MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));
     }

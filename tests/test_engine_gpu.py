@@ -484,3 +484,30 @@ def test_prompts_of_a_generation_in_pieces(dm, lens, dtype):
     assert out[0][0] == out[1][0]
     for p, q in zip(out[0][1], out[1][1]):
         assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
+
+
+@pytest.mark.parametrize("dm,B,T,dtype", [
+    (128, 1, 16, WeightDtype.BF16),     # the shortest prompt; one row, lanes along the weight row
+    (256, 4, 33, WeightDtype.F16),      # the most rows of that route
+    (128, 5, 17, WeightDtype.BF16),     # matrix cores, part of a row tile
+    (64, 3, 16, WeightDtype.F16),       # matrix cores at few rows: a weight row of no whole 32 lanes
+    (64, 17, 40, WeightDtype.F16),      # a second row tile, of one row
+    (128, 128, 16, WeightDtype.BF16),   # the most rows
+])
+def test_prefill_projects_the_last_steps_alone_in_its_last_layer(dm, B, T, dtype):
+    """Behind the last layer's scan only the last step of each sequence goes on.  Against the same prompt in two calls, the second of eight
+    steps, whose out_proj runs over all rows: states as two calls leave them, last rows within the tolerance between two routes that
+    round at the same 16-bit points (1 % in norm: three layers, each rounding its projections, u and y once)."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=3)
+    w = MambaWeights.init(cfg, dm, 5)
+    w.input_proj_w = np.zeros((0, dm), np.float32)
+    x = np.random.default_rng(B + T).standard_normal((B, T, dm)).astype(np.float32)
+    print(f"case last steps {dm} {B}x{T} {dtype.name}", flush=True)
+    e = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    got = [e.prefill_sequence(x).copy()] + [p for l in range(3) for p in e.download_state(l)]
+    e.reset()
+    e.prefill_sequence(x[:, :T - 8].copy())
+    want = [e.prefill_sequence(x[:, T - 8:].copy()).copy()] + [p for l in range(3) for p in e.download_state(l)]
+    e.close()
+    for p, q in zip(got, want):
+        assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)

@@ -329,3 +329,22 @@ def test_small_f32_models_step_in_one_launch(case, monkeypatch):
     for t in range(steps):
         assert scaled_err(ref.step(x[t]), outs[t]) < 2e-4, t
     ref.close()
+
+
+@pytest.mark.parametrize("B,T,dtype", [(1, 16, WeightDtype.BF16), (5, 17, WeightDtype.F16), (128, 16, WeightDtype.BF16)])
+def test_prefill_projects_the_last_steps_alone_in_its_last_layer(B, T, dtype):
+    """Behind the last layer's scan only the last step of each sequence goes on.  Against the same prompt in two calls, the second of eight
+    steps, whose out_proj runs over all rows: last rows within the tolerance between two routes that round at the same 16-bit points (1 % in
+    norm: two layers, each rounding its projections, K, Q and y once)."""
+    cfg = Mamba3Config(d_model=128, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+    w = perturbed(cfg, 128, 19)
+    w.input_proj_w = np.zeros(0, np.float32)
+    x = np.random.default_rng(B + T).standard_normal((B, T, 128)).astype(np.float32)
+    print(f"case m3 last steps {B}x{T} {dtype}", flush=True)
+    e = GpuMamba3Backbone.new_with_dtype(0, w, cfg, 128, B, dtype)
+    got = e.prefill_sequence(x).copy()
+    e.reset()
+    e.prefill_sequence(x[:, :T - 8].copy())
+    want = e.prefill_sequence(x[:, T - 8:].copy()).copy()
+    e.close()
+    assert np.linalg.norm(got - want) <= 1e-2 * np.linalg.norm(want), np.linalg.norm(got - want) / np.linalg.norm(want)
