@@ -397,9 +397,9 @@ static int prefill_projection(mrs_backbone *bb, int dtype, void *C, int ldc, con
 }
 
 static int launch_add_rmsnorm(mrs_backbone *bb, float *residual, const void *add, void *out, bool out_f32, const float *w,
-                              int64_t rows, int64_t out_stride, void *out2 = nullptr) {
+                              int64_t rows, int64_t in_stride, void *out2 = nullptr) {
     return launch_add_rmsnorm_any(bb->stream, bb->dtype, residual, add, out, out_f32, out2, w, bb->cfg.rms_norm_eps, rows, bb->cfg.d_model,
-                                  out_stride);
+                                  in_stride);
 }
 
 // residual <- input (identity) or input . input_proj_w + b (f32 GEMM)
@@ -618,11 +618,9 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
     } else {
         // Only the last step of each sequence is kept (gather_last_timestep,
         // src/mamba_ssm/gpu/prefill.rs:1030-1046), so the final residual add + norm_f runs on those rows only.
-        for (int b = 0; b < B; b++) {
-            const size_t r = (size_t)b * T + (T - 1);
-            MRS_TRY(launch_add_rmsnorm(bb, s->residual + r * dm, (const char *)s->out + r * dm * es, bb->temporal + (size_t)b * dm, true,
-                                       bb->norm_f, 1, dm, bb->dtype != MRS_F32 ? (char *)bb->temporal_t + (size_t)b * dm * es : nullptr));
-        }
+        const size_t r = (size_t)(T - 1) * dm;
+        MRS_TRY(launch_add_rmsnorm(bb, s->residual + r, (const char *)s->out + r * es, bb->temporal, true, bb->norm_f, B, (int64_t)T * dm,
+                                   bb->dtype != MRS_F32 ? bb->temporal_t : nullptr));
     }
     return MRS_OK;
 }

@@ -7,15 +7,17 @@ namespace mrs {
 // One workgroup per row: residual (f32) += add (storage dtype, may be null); out = rmsnorm(residual) * w.
 // Reference: residual_add_f32_* + rmsnorm_forward_f32in_* (kernels/elementwise.cu:366-376,
 // kernels/norms.cu:21-171), with its finite guard: rms = 1 if not finite or < 1e-20 (norms.cu:58-61).
-// out2 (may be null): the same result once more in the storage type (the LM head's operand).
+// out2 (may be null): the same result once more in the storage type (the LM head's operand).  Rows of residual and add lie in_stride apart:
+// the last steps of a prefill's sequences are one launch.  (One each was bound by the launches, 3.5 us apiece: a bf16 prefill of two layers,
+// one each / this: 8, 64, 128 x 16 steps at d_model 768 91 / 68, 332 / 125, 605 / 181 us, 128 x 64 at 2560 2658 / 1615.)
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *__restrict__ residual, const T *__restrict__ add,
                                                           TO *__restrict__ out, T *__restrict__ out2, const float *__restrict__ w,
-                                                          float eps, int64_t rows, int dm, int64_t out_stride) {
+                                                          float eps, int dm, int64_t in_stride) {
     constexpr int kMaxPer = 16;  // elements per thread kept in registers (d_model <= 4096); longer rows re-read
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
-    float *r = residual + row * dm;
+    float *r = residual + row * in_stride;
     float v[kMaxPer];   // indexed by unrolled loop counters only (a run-time index would put it in scratch memory)
     float ss = 0.0f;
 #pragma unroll
@@ -24,14 +26,14 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *__restrict__ re
         float x = 0.0f;
         if (i < dm) {
             x = r[i];
-            if (add) { x += Store<T>::ld(add + row * dm + i); r[i] = x; }
+            if (add) { x += Store<T>::ld(add + row * in_stride + i); r[i] = x; }
         }
         v[k] = x;
         ss = fmaf(x, x, ss);
     }
     for (int i = threadIdx.x + 256 * kMaxPer; i < dm; i += 256) {
         float x = r[i];
-        if (add) { x += Store<T>::ld(add + row * dm + i); r[i] = x; }
+        if (add) { x += Store<T>::ld(add + row * in_stride + i); r[i] = x; }
         ss = fmaf(x, x, ss);
     }
 #pragma unroll
@@ -47,14 +49,14 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *__restrict__ re
         const int i = threadIdx.x + 256 * k;
         if (i < dm) {
             const float o = v[k] * inv * w[i];
-            Store<TO>::st(out + row * out_stride + i, o);
-            if (out2) Store<T>::st(out2 + row * out_stride + i, o);
+            Store<TO>::st(out + row * dm + i, o);
+            if (out2) Store<T>::st(out2 + row * dm + i, o);
         }
     }
     for (int i = threadIdx.x + 256 * kMaxPer; i < dm; i += 256) {
         const float o = r[i] * inv * w[i];
-        Store<TO>::st(out + row * out_stride + i, o);
-        if (out2) Store<T>::st(out2 + row * out_stride + i, o);
+        Store<TO>::st(out + row * dm + i, o);
+        if (out2) Store<T>::st(out2 + row * dm + i, o);
     }
 }
 
@@ -189,13 +191,13 @@ static __global__ __launch_bounds__(256) void bias_rows_kernel(float *__restrict
 }
 
 // residual (f32, rows x dm) += add (storage type, may be null); out = rmsnorm(residual) * w as f32 (out_f32) or in the
-// storage type; out2 (may be null): the result once more in the storage type.  Prefill-sized row counts take the
-// wave-per-row kernel.
+// storage type; out2 (may be null): the result once more in the storage type.  in_stride: from row to row of residual and add (out and
+// out2 are dense).  Prefill-sized row counts take the wave-per-row kernel.
 template <typename T>
 inline void launch_add_rmsnorm_typed(hipStream_t st, float *residual, const void *add, void *out, bool out_f32, void *out2, const float *w,
-                                     float eps, int64_t rows, int dm, int64_t out_stride) {
+                                     float eps, int64_t rows, int dm, int64_t in_stride) {
     const dim3 grid((unsigned)rows), block(256);
-    if (rows >= 64 && rows < 256 && dm % 4 == 0 && dm <= 4096 && out_stride == dm && !out2 && !out_f32) {
+    if (rows >= 64 && rows < 256 && dm % 4 == 0 && dm <= 4096 && in_stride == dm && !out2 && !out_f32) {
 #define MRS_BLK(TR) hipLaunchKernelGGL((add_rmsnorm_block_kernel<T, T, TR>), grid, block, 0, st, residual, (const T *)add, (T *)out, w, eps, dm)
         const int trips = (dm / 4 + 255) / 256;
         if (trips <= 1) MRS_BLK(1);
@@ -204,7 +206,7 @@ inline void launch_add_rmsnorm_typed(hipStream_t st, float *residual, const void
 #undef MRS_BLK
         return;
     }
-    if (rows >= 256 && dm % 4 == 0 && dm <= 4096 && out_stride == dm && !out2 && !out_f32) {
+    if (rows >= 256 && dm % 4 == 0 && dm <= 4096 && in_stride == dm && !out2 && !out_f32) {
         const dim3 g4((unsigned)((rows + 3) / 4));
 #define MRS_ROWS(TR) hipLaunchKernelGGL((add_rmsnorm_rows_kernel<T, T, TR>), g4, block, 0, st, residual, (const T *)add, (T *)out, w, eps, rows, dm)
         const int trips = (dm / 4 + 63) / 64;
@@ -216,16 +218,14 @@ inline void launch_add_rmsnorm_typed(hipStream_t st, float *residual, const void
         return;
     }
     if (out_f32)
-        hipLaunchKernelGGL((add_rmsnorm_kernel<T, float>), grid, block, 0, st, residual, (const T *)add, (float *)out, (T *)out2, w, eps, rows, dm,
-                           out_stride);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<T, float>), grid, block, 0, st, residual, (const T *)add, (float *)out, (T *)out2, w, eps, dm, in_stride);
     else
-        hipLaunchKernelGGL((add_rmsnorm_kernel<T, T>), grid, block, 0, st, residual, (const T *)add, (T *)out, (T *)out2, w, eps, rows, dm,
-                           out_stride);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<T, T>), grid, block, 0, st, residual, (const T *)add, (T *)out, (T *)out2, w, eps, dm, in_stride);
 }
 
 inline int launch_add_rmsnorm_any(hipStream_t st, int dtype, float *residual, const void *add, void *out, bool out_f32, void *out2,
-                                  const float *w, float eps, int64_t rows, int dm, int64_t out_stride) {
-    MRS_DISPATCH_DTYPE(dtype, T_, launch_add_rmsnorm_typed<T_>(st, residual, add, out, out_f32, out2, w, eps, rows, dm, out_stride));
+                                  const float *w, float eps, int64_t rows, int dm, int64_t in_stride) {
+    MRS_DISPATCH_DTYPE(dtype, T_, launch_add_rmsnorm_typed<T_>(st, residual, add, out, out_f32, out2, w, eps, rows, dm, in_stride));
     return check_launch("add_rmsnorm_kernel");
 }
 

@@ -1300,12 +1300,9 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         else MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));
     }
     // only the last position of each sequence is kept: final residual add + norm_f on those rows
-    for (int b = 0; b < B; b++) {
-        const size_t r = (size_t)b * T + (T - 1);
-        MRS_TRY(launch_add_rmsnorm3(bb, bb->pf_residual + r * dm, (const char *)bb->pf_out + r * dm * es, bb->temporal + (size_t)b * dm, true,
-                                    bb->norm_f, 1));
-    }
-    return MRS_OK;
+    const size_t r = (size_t)(T - 1) * dm;
+    return launch_add_rmsnorm_any(bb->stream, dt, bb->pf_residual + r, (const char *)bb->pf_out + r * es, bb->temporal, true, nullptr, bb->norm_f,
+                                  c.rms_norm_eps, B, dm, (int64_t)T * dm);
 }
 
 }  // namespace
