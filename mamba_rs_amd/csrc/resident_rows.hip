@@ -90,14 +90,23 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
     dma_to_lds(f.win, blk, w, in_pieces, 4);
     dma_to_lds(f.small, blk + S::lb.small, w, small_pieces, 4);
     dma_wait();
+    // The roll call's outcome is taken while the workgroup's first wait for others goes on, that is in front of the same barrier: behind it,
+    // the wait would have no end where the others are called off (xch_poll does not count while `state` is kRollCall).
+    const auto take_outcome = [&] {
+        if (roll_wave && state == kRollCall) {
+            const int s = call.outcome();
+            if (first) state = s;
+        }
+    };
     lds_barrier();   // layer 0's weights are there
     lds_barrier();   // T
+    if (state > 0) return;
 #pragma unroll 1
     for (int l = 0; l < nl; l++) {
         const bool more = l + 1 < nl;
         const char *next = blk + f.next, *ssm = f.ssm + l * f.ssm_next, *conv = f.conv + l * f.conv_next;   // the next layer's
         lds_barrier();   // A
-        if (state > 0) return;
+        if (l == 0 && f.hurry) take_outcome();
         lds_barrier();   // B
         lds_barrier();   // X
         const auto early_part = [&](auto sleep) {
@@ -110,10 +119,7 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
         };
         if (f.hurry) early_part(std::integral_constant<int, 1>());
         else early_part(std::integral_constant<int, 2>());
-        if (l == 0 && roll_wave && state == kRollCall) {
-            const int s = call.outcome();
-            if (first) state = s;
-        }
+        if (l == 0 && !f.hurry) take_outcome();
         lds_barrier();   // C
         if (state) return;
         dma_wait();   // out_proj's weights are there
@@ -332,7 +338,7 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
     lds_barrier();   // T
 
 #pragma unroll 1
-    for (int l = 0; l < nl; l++) {
+    for (int l = state > 0 ? nl : 0; l < nl; l++) {   // (not at all if it was called off before it began)
         const unsigned tag = base + 1 + l;
         const bool more = l + 1 < nl;
         const char *small = smem + S::small + (l & 1) * sb.bytes;
@@ -351,7 +357,6 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
         }
         xweights += S::layer_bytes;
         lds_barrier();   // A
-        if (state > 0) break;
         // ---- conv step + SiLU
         float xnew = 0.0f, z = 0.0f, u = 0.0f;
         if (tile_wave) {

@@ -1,6 +1,7 @@
 """The gate of the resident decode steps (csrc/resident_gate.hip) on a model of the runtime's streams, events and captures
 (gate_model/): which launches may run together, and what a turn may touch.  No GPU."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -93,3 +94,103 @@ def test_roll_call_has_one_outcome(answers):
             elif a[0] == "called off":
                 to(i, ("end", OFF), ruling=OFF)
     assert ends == ({frozenset([GO]), frozenset([OFF])} if all(answers) else {frozenset([OFF])})
+
+
+def _first_layer(tile):
+    """What the roll-call wave and the first computing wave of a workgroup of csrc/resident_rows.hip do in layer 0 up to barrier C, as
+    the source has it: barriers (capitals), `outcome`, and the waits for u ("see u") and for the x_proj rows ("see x") with what
+    goes out before them.  tile: the workgroup forms an x_proj tile."""
+    text = open(os.path.join(CSRC, "resident_rows.hip")).read()
+    feed, kernel = (text[text.index(at):] for at in ("void bring_rows_weights", "void resident_rows_kernel"))
+
+    def walk(text, marks):
+        text = text[text.index("for (int l ="):]
+        text = text[:text.index("// C") + 4]
+        found = [(m.start(), m.group(1)) for m in re.finditer(r"lds_barrier\(\);\s*// ([A-Z])", text)]
+        for pattern, what in marks:
+            at = [m.start() for m in re.finditer(pattern, text)]
+            assert len(at) <= 1, pattern
+            found += [(a, what) for a in at]
+        return [what for _, what in sorted(found)]
+    roll = walk(feed, [(r"l == 0 && f\.hurry\) take_outcome\(\)", "outcome" if tile else None),
+                       (r"l == 0 && !f\.hurry\) take_outcome\(\)", None if tile else "outcome"),
+                       (r"call\.outcome\(\)", "outcome")])
+    compute = walk(kernel, [(r"say\(xb \+ S::e2f", "put u"), (r"return find\(S::e2f", "see u" if tile else None),
+                            (r"xch_put_word\(xb \+ S::e2", "put x" if tile else None), (r"xch_poll<XW>", "see x")])
+    return tuple(w for w in roll if w), tuple(w for w in compute if w)
+
+
+def _run_to_the_end(tiles, places, programs):
+    """Every interleaving of workgroups with the programs of _first_layer (tiles[i]: which kind), at most `places` of them on the chip
+    at once.  Returns the outcomes, and the states from which nobody comes to an end any more."""
+    N = len(tiles)
+    NONE, GO, OFF, CALL = "none", "go", "off", "call"
+    # per workgroup: place in the roll-call wave's program, in the computing wave's, its state; then lost, answers, ruling, u, x
+    begin = ((None,) * N, False, frozenset(), NONE, frozenset(), frozenset())
+    after, stack, ends = {}, [begin], set()
+
+    def moves(s):
+        wgs, lost, got, ruling, u, x = s
+        running = sum(w not in (None, GO, OFF) for w in wgs)
+        for i, w in enumerate(wgs):
+            def to(w2, lost=lost, got=got, ruling=ruling, u=u, x=x, i=i):
+                return (wgs[:i] + (w2,) + wgs[i + 1:], lost, got, ruling, u, x)
+            if w is None:
+                if running < places:    # the answer: one that is already too late leaves without a word
+                    yield to(OFF) if lost else to((0, 0, CALL), got=got | {i})
+                continue
+            if w in (GO, OFF):
+                continue
+            roll, comp = programs[tiles[i]]
+            r, c, state = w
+            if r < len(roll) and c < len(comp) and roll[r] == comp[c]:          # a barrier both have come to
+                if roll[r] == "C":
+                    yield to(state if state in (GO, OFF) else "no ruling")
+                else:
+                    yield to((r + 1, c + 1, state))
+                continue
+            if roll[r] == "outcome":
+                if ruling == OFF:
+                    yield to((r + 1, c, OFF))
+                elif len(got) == N:
+                    yield to((r + 1, c, GO))
+                else:                                                            # out of patience (or not yet: no change)
+                    yield to((r + 1, c, OFF), lost=True, ruling=OFF)
+            if comp[c] == "put u":
+                yield to((r, c + 1, state), u=u | {i})
+            elif comp[c] == "put x":
+                yield to((r, c + 1, state), x=x | {i})
+            elif comp[c] in ("see u", "see x"):
+                there = len(u) == N if comp[c] == "see u" else x >= {k for k in range(N) if tiles[k]}
+                if there or state == OFF:
+                    yield to((r, c + 1, state))
+    while stack:
+        s = stack.pop()
+        if s in after:
+            continue
+        after[s] = list(moves(s))
+        stack += after[s]
+        if all(isinstance(w, str) for w in s[0]):
+            ends.add(frozenset(s[0]))
+    can_end, grown = {s for s in after if all(isinstance(w, str) for w in s[0])}, True
+    while grown:
+        more = {s for s, t in after.items() if s not in can_end and any(n in can_end for n in t)}
+        can_end |= more
+        grown = bool(more)
+    return ends, set(after) - can_end
+
+
+@pytest.mark.parametrize("tiles", [(True, False, False), (True, True, False), (True, False, False, False)])
+@pytest.mark.parametrize("short_of", [0, 1, 2])
+def test_a_step_of_many_rows_that_lacks_places_ends(tiles, short_of):
+    """Layer 0 of csrc/resident_rows.hip, barriers and waits where the source has them: whatever places are missing and whoever
+    loses patience first, every workgroup comes to an end, and all of them the same way.  (With the outcome behind the barrier that the
+    first wait stands in front of, they do not: the model sees that.)"""
+    programs = {t: _first_layer(t) for t in (True, False)}
+    assert programs[False] == (("A", "B", "X", "outcome", "C"), ("A", "put u", "B", "X", "see x", "C"))
+    assert programs[True][1] == ("A", "put u", "see u", "B", "X", "put x", "see x", "C")
+    ends, stuck = _run_to_the_end(tiles, len(tiles) - short_of, programs)
+    assert not stuck
+    assert ends == ({frozenset(["off"])} if short_of else {frozenset(["go"]), frozenset(["off"])})
+    late = {**programs, True: (("A", "B", "X", "outcome", "C"), programs[True][1])}
+    assert _run_to_the_end(tiles, len(tiles) - short_of, late)[1]
