@@ -100,11 +100,11 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
     };
     lds_barrier();   // layer 0's weights are there
     lds_barrier();   // T
-    if (state > 0) return;
 #pragma unroll 1
     for (int l = 0; l < nl; l++) {
         const bool more = l + 1 < nl;
         const char *next = blk + f.next, *ssm = f.ssm + l * f.ssm_next, *conv = f.conv + l * f.conv_next;   // the next layer's
+        if (state > 0) return;   // (called off before it began, or lost)
         lds_barrier();   // A
         if (l == 0 && f.hurry) take_outcome();
         lds_barrier();   // B
@@ -134,7 +134,6 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
         dma_wait();
         lds_barrier();   // E
         lds_barrier();   // T
-        if (state) return;
     }
 }
 
@@ -338,7 +337,7 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
     lds_barrier();   // T
 
 #pragma unroll 1
-    for (int l = state > 0 ? nl : 0; l < nl; l++) {   // (not at all if it was called off before it began)
+    for (int l = 0; l < nl; l++) {
         const unsigned tag = base + 1 + l;
         const bool more = l + 1 < nl;
         const char *small = smem + S::small + (l & 1) * sb.bytes;
@@ -356,6 +355,7 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
             for (int s = 0; s < KO; s++) xw[s] = make_uint4(0, 0, 0, 0);
         }
         xweights += S::layer_bytes;
+        if (state > 0) break;   // (called off before it began, or lost)
         lds_barrier();   // A
         // ---- conv step + SiLU
         float xnew = 0.0f, z = 0.0f, u = 0.0f;
@@ -511,7 +511,6 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
         take_sums(tag);
         orows += S::rows_bytes;
         lds_barrier();   // T
-        if (state) break;
     }
     lds_barrier();
     // final norm of this workgroup's columns: f32, and once more in the storage type for a head
