@@ -634,10 +634,14 @@ static void choose_resident(mrs_backbone *bb) {
     ResidentArgs &a = bb->res_args;
     a.eps = c.rms_norm_eps; a.n_layers = c.n_layers; a.batch = bb->batch; a.dm = c.d_model; a.di = bb->di;
     a.ds = c.d_state; a.dc = c.d_conv; a.dr = bb->dr; a.xd = bb->xd;
-    // A group of workgroups per row where all of them fit, else rows by the group.  Of groups of 128 only one is better off alone (24 layers of
-    // d_model 1024: one row 261 us against 281, two 302 against 286; of 768, groups of 64: three rows 210 against 234, four 236 against 238).
-    const bool one = bb->batch <= kRollMax && resident_plan(a, bb->dtype) && a.G * a.batch <= kRollMax && (a.G <= 64 || bb->batch == 1);
-    if (!one && !resident_rows_plan(a, bb->dtype)) return;
+    // A group of workgroups per row where all of them fit, else rows by the group.  Where both will do, groups of 128 are better off by the row
+    // only when alone (24 layers of d_model 1024: one row 261 us against 281, two 302 against 286; of 768, groups of 64: three rows 210 against 234,
+    // four 236 against 238).
+    ResidentArgs several = a;
+    const bool many = resident_rows_plan(several, bb->dtype);
+    const bool one = bb->batch <= kRollMax && resident_plan(a, bb->dtype) && a.G * a.batch <= kRollMax && (a.G <= 64 || bb->batch == 1 || !many);
+    if (!one && !many) return;
+    if (!one) a = several;
     if (!resident_claim(bb->seat, bb->device, a.G * a.groups, bb->stream)) return;
     bb->resident = one ? 1 : 2;
 }

@@ -19,7 +19,10 @@ from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtyp
     (256, 2, 256, 8),     # eight rows of 32 workgroups: every compute unit
     (768, 2, 768, 1),     # 24 channels and 12 out_proj columns per workgroup
     (768, 2, 768, 4),
-    (1024, 2, 1024, 2),   # the widest: 128 workgroups per row, four and eight k-steps per wave
+    (1024, 2, 1024, 1),   # the widest: 128 workgroups, four and eight k-steps per wave
+    (896, 2, 896, 2),     # 112 workgroups per row, a width the groups of several rows do not take
+    (640, 2, 640, 3),     # 80 per row, the same
+    (1024, 2, 1024, 2),
     # several rows per group of workgroups (resident_rows.hip)
     (256, 2, 20, 9),      # input projection; eight groups of one row and of two
     (256, 2, 256, 128),   # full groups; dt_rank 16: a k-step of dt_proj with zeros behind it
