@@ -1067,7 +1067,15 @@ static float *m1_hook_prefix_rows(void *self) {
     }
     return bb->prefix_s.residual;
 }
-static int m1_hook_prefix_run(void *self, int T) { return run_layers((mrs_backbone *)self, &((mrs_backbone *)self)->prefix_s, T, true); }
+static int m1_hook_prefix_run(void *self, int T) {
+    mrs_backbone *bb = (mrs_backbone *)self;
+    // The library's default kernels, also where timing them is on: every new length of prompt is a new row count, and timing one takes seconds.
+    GemmTuner *const tuner = bb->tuner;
+    bb->tuner = nullptr;
+    const int rc = run_layers(bb, &bb->prefix_s, T, true);
+    bb->tuner = tuner;
+    return rc;
+}
 
 extern "C" int mrs_backbone_prefill_device(mrs_backbone *bb, const float *input_dev, int T) {
     if (!bb || !input_dev) return fail(MRS_E_NULL, "mrs_backbone_prefill_device: null pointer");

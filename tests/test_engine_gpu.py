@@ -360,6 +360,40 @@ def test_prefill_with_tuned_vendor_gemms_matches_the_default_choice_and_the_cpu_
     eng.close()
 
 
+def test_generation_times_no_vendor_kernels():
+    """With set_gemm_tuning a generation whose prompts have a new length is no slower than a quarter of a first prefill of the same
+    rows, which does time the library's kernels, and it has the bits of an engine without tuning, also behind that prefill."""
+    import time
+    from mamba_rs_amd import SampleParams
+    B, T = 64, 24      # 1536 rows: in_proj and out_proj of a prompt's piece go to the library
+    cfg = MambaConfig(d_model=768, d_state=16, d_conv=4, expand=2, n_layers=2)
+    w = MambaWeights.random_lm(cfg, seed=3, std=0.05)
+    rng = np.random.default_rng(8)
+    embed = rng.standard_normal((500, 768)).astype(np.float32)
+    prompts = rng.integers(0, 500, (B, T + 1)).tolist()
+    params = [SampleParams(temperature=0.8, top_k=20, max_tokens=2, seed=i) for i in range(B)]
+    print("case generation with tuning", flush=True)
+    out = []
+    for tuned in (False, True):
+        eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, 768, B, WeightDtype.BF16)
+        lm = GpuMambaLM(eng, embed)
+        eng.set_gemm_tuning(tuned)
+        lm.generate_batch([p[:9] for p in prompts], params)
+        t0 = time.perf_counter()
+        first = lm.generate_batch(prompts, params)
+        new_length = time.perf_counter() - t0
+        if tuned:
+            x = rng.standard_normal((B, T, 768)).astype(np.float32)
+            t0 = time.perf_counter()
+            eng.prefill_sequence(x)
+            assert new_length < 0.25 * (time.perf_counter() - t0), new_length
+        assert lm.generate_batch(prompts, params) == first
+        out.append((first, [p for l in range(2) for p in eng.download_state(l)]))
+        lm.close()
+        eng.close()
+    assert out[0][0] == out[1][0] and all(np.array_equal(p, q) for p, q in zip(out[0][1], out[1][1]))
+
+
 @pytest.mark.parametrize("tuned", [False, True])
 def test_decode_above_the_own_chain_limit_runs_the_projections_from_the_transposed_copies(tuned):
     """130 rows at d_model 768: past the own chain's limit, so in_proj and out_proj go to the GEMM library reading the
