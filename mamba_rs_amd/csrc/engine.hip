@@ -1045,7 +1045,9 @@ extern "C" int mrs_backbone_alloc_prefill_scratch(mrs_backbone *bb, int T) {
 }
 
 // A generation's prompt, as far as all slots have one: kPrefixSteps steps at a time through the prefill's kernels, whose products take
-// batch * steps rows in one launch where a step takes batch.  The activations' buffers are the engine's from the first such prompt on.
+// batch * steps rows in one launch where a step takes batch.  The activations' buffers are the engine's from the first such prompt on, and they
+// are what a longer piece costs: prompts of 48 tokens, pieces of 16, 32 and 64 steps, 24 layers of d_model 768 at 1 row 2951, 2296, 1561 us, at 64 rows
+// 5943, 4779, 4066, of 1024 at 13 rows 3990, 3263, 2366; of up to 32 tokens the last two are the same (activations at 64 rows of 768: 44 and 89 MB).
 constexpr int kPrefixSteps = 32;
 static bool prefix_ok(const mrs_backbone *bb) {
     const LayerDev &lw = bb->layers[0];
@@ -1069,6 +1071,7 @@ static float *m1_hook_prefix_rows(void *self) {
 }
 static int m1_hook_prefix_run(void *self, int T) {
     mrs_backbone *bb = (mrs_backbone *)self;
+    if (T < 2 || T > kPrefixSteps) return fail(MRS_E_SHAPE, "a piece of a prompt: %d steps", T);   // (one step would be the decode chain, whose buffers these are not)
     // The library's default kernels, also where timing them is on: every new length of prompt is a new row count, and timing one takes seconds.
     GemmTuner *const tuner = bb->tuner;
     bb->tuner = nullptr;
@@ -1564,7 +1567,9 @@ static int gen_loop(mrs_lm *lm, const int *prompts, const int *prompt_lens, cons
     std::vector<mrs_sampler> samplers(B);
     std::vector<unsigned long long> rng((size_t)B * 4);
     const bool prefill_route = seen_includes_prompt && B == 1 && prompt_lens[0] >= 256;   // PREFILL_PARALLEL_THRESHOLD, gpu_lm.rs:48
-    // what all slots' prompts have in front of their last token goes through prefill kernels (a slot without a prompt: none)
+    // What all slots' prompts have in front of their last token goes through prefill kernels: the shortest prompt decides for all.  From four tokens
+    // on (a whole generation of one new token, pieces / steps, at 2, 3, 4, 5 tokens: 24 layers of d_model 768 at one row 1353 / 1018, 1353 / 1214, 1352 /
+    // 1424, 1360 / 1639 us, at 64 rows 2541 / 2192, 2540 / 2559, 2566 / 2929, 2592 / 3285; eight of 2560 at 8 rows 1497 / 1690 at two, 1502 / 2366 at four).
     int common = prefill_route ? 0 : max_prompt - 1;
     for (int i = 0; i < B; i++) common = std::min(common, prompt_lens[i] - 1);
     if (common < 4 || !bb->prefix_rows || !bb->prefix_rows(bb->self)) common = 0;
