@@ -490,12 +490,13 @@ def test_small_f32_models_step_in_one_launch(shape, monkeypatch):
     (256, (70, 33, 81), WeightDtype.BF16),       # 32: one whole piece
     (768, (34, 36), WeightDtype.F16),            # 33: two pieces of 16 and 17, a last tile of one step; dt_rank 48
     (1024, (100,), WeightDtype.BF16),            # 99: four pieces
+    (2560, (9, 40), WeightDtype.BF16),           # dt_rank 160: five k-steps of dt_proj, rows of x_proj 192 apart
 ])
 def test_prompts_of_a_generation_in_pieces(dm, lens, dtype):
     """What all prompts have in front of their last token goes through the prefill's kernels, up to 32 steps at a time, with dt_proj inside
     the scan: tokens are those of an engine that takes every token as a step (scan_mode SEQUENTIAL keeps the prompt out of the
     prefill kernels), all states and the last rows within the tolerance between two routes that round at the same 16-bit points
-    (1 % in norm: three layers, each rounding its projections, u and y once)."""
+    (1 % in norm: three layers, each rounding its projections, u and y once), and not the same bits: two routes there were."""
     from mamba_rs_amd import SampleParams
     rng = np.random.default_rng(sum(lens))
     embed = rng.standard_normal((500, dm)).astype(np.float32)
@@ -516,6 +517,7 @@ def test_prompts_of_a_generation_in_pieces(dm, lens, dtype):
         lm.close()
         e.close()
     assert out[0][0] == out[1][0]
+    assert not all(np.array_equal(p, q) for p, q in zip(out[0][1], out[1][1]))
     for p, q in zip(out[0][1], out[1][1]):
         assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
 

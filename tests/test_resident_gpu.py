@@ -22,13 +22,15 @@ from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtyp
     (1024, 2, 1024, 1),   # the widest: 128 workgroups, four and eight k-steps per wave
     (896, 2, 896, 2),     # 112 workgroups per row, a width the groups of several rows do not take
     (640, 2, 640, 3),     # 80 per row, the same
-    (1024, 2, 1024, 2),
     # several rows per group of workgroups (resident_rows.hip)
-    (256, 2, 20, 9),      # input projection; eight groups of one row and of two
-    (256, 2, 256, 128),   # full groups; dt_rank 16: a k-step of dt_proj with zeros behind it
-    (512, 2, 512, 37),    # groups of nine rows and of ten: the second wave that writes operands has one or two
-    (768, 2, 768, 5),     # groups of two rows and of one; 24 channels: a channel tile that is half empty
+    (256, 2, 20, 9),      # input projection; groups of five and four rows
+    (256, 2, 256, 128),   # eight full groups; dt_rank 16: a k-step of dt_proj with zeros behind it
+    (512, 2, 512, 37),    # groups of ten and nine rows: the second wave that writes operands has two or one
+    (768, 2, 768, 5),     # one group; 24 channels: a channel tile that is half empty
+    (768, 2, 768, 17),    # three groups, of six, six and five rows
     (768, 2, 768, 64),    # full groups, three k-steps per wave
+    (1024, 2, 1024, 2),   # the smallest group
+    (1024, 2, 1024, 3),
     (1024, 2, 1024, 31),  # two groups of 128 workgroups, sixteen and fifteen rows
 ])
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
@@ -51,7 +53,10 @@ def test_resident_step_follows_the_cpu_route(shape, dtype):
     assert a.decode_route() == 2 and b.decode_route() == 2      # one launch
     rng = np.random.default_rng(dm + B)
     x = rng.standard_normal((6, B, idim)).astype(np.float32)
-    rows = sorted({0, B // 2, B - 1})
+    # the ends of every group: eight rows wanted, at most 256 workgroups
+    groups = min(-(-B // 8), 256 // (dm // (12 if dm == 768 else 8)))
+    first = [g * (B // groups) + min(g, B % groups) for g in range(groups + 1)]
+    rows = sorted({0, B // 2, B - 1} | {r for a, b in zip(first, first[1:]) for r in (a, b - 1)})
     st = {r: orc.m1_zero_state(P) for r in rows}
     for t in range(6):
         if t == 3:
@@ -163,7 +168,7 @@ def _family(family, rows=4):
     from mamba_rs_amd import GpuMamba3Backbone, GpuMamba3LM, GpuMambaLM
     if family == "m1":
         return lambda: _engines((768, 3, rows), 1)[0], 768, GpuMambaLM
-    if family == "m1rows":      # four rows on one group of 128 workgroups (resident_rows.hip)
+    if family == "m1rows":      # rows on one group of 128 workgroups (resident_rows.hip)
         return lambda: _engines((1024, 3, rows), 1)[0], 1024, GpuMambaLM
     from test_m3_engine_gpu import perturbed
     from test_resident_m3_gpu import cfg_
@@ -378,6 +383,47 @@ def test_generation_hands_out_no_token_of_a_lost_step(family, monkeypatch):
     assert lm.generate_batch([prompt], [params]) == lm_chain.generate_batch([prompt], [params])
     a.set_resident_wait(1 << 23)
     assert stream(lm) == (whole, None)
+    for e in (lm, lm_chain, a, chain):
+        e.close()
+
+
+@pytest.mark.parametrize("family", ["m1", "m1rows"])
+def test_prompts_in_pieces_before_lost_steps(family, monkeypatch):
+    """Prompts that go through the prefill kernels in front of steps that are called off: the generation starts over on the kernel chain,
+    prompts and all, with that engine's tokens and states; behind a streamed token the caller has what it was given, and an error; the
+    next generation, with places, is the first one again."""
+    from mamba_rs_amd import MambaHipError, SampleParams
+    rows = 1 if family == "m1" else 3
+    make, dm, lm_of = _family(family, rows)
+    a = make()
+    monkeypatch.setenv("MRS_DECODE_NO_RESIDENT", "1")
+    chain = make()
+    assert (a.decode_route(), chain.decode_route()) == (2, 1)
+    rng = np.random.default_rng(13)
+    embed = rng.standard_normal((128, dm)).astype(np.float32)
+    prompts = [rng.integers(0, 128, n).tolist() for n in (41, 37, 44)[:rows]]      # two pieces
+    params = [SampleParams(temperature=0.9, top_k=20, max_tokens=6, seed=i) for i in range(rows)]
+    print(f"case prompts in pieces before lost steps {family}", flush=True)
+    lm, lm_chain = lm_of(a, embed), lm_of(chain, embed)
+    want, want_chain = lm.generate_batch(prompts, params), lm_chain.generate_batch(prompts, params)
+    a.set_resident_wait(0)
+    for _ in range(2):
+        assert lm.generate_batch(prompts, params) == want_chain
+        assert all(np.array_equal(p, q) for p, q in zip(_states(a), _states(chain)))
+    a.set_resident_wait(1 << 23)
+    assert lm.generate_batch(prompts, params) == want
+    if rows == 1:
+        got = []
+
+        def take(tok):
+            got.append(tok)
+            if len(got) == 2:
+                a.set_resident_wait(0)
+        with pytest.raises(MambaHipError, match="did not come free"):
+            lm.generate_streaming(prompts[0], params[0], take)
+        assert got == want[0][:2]
+        a.set_resident_wait(1 << 23)
+        assert lm.generate_batch(prompts, params) == want
     for e in (lm, lm_chain, a, chain):
         e.close()
 
