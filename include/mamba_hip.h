@@ -327,14 +327,14 @@ MRS_API float *mrs_backbone_temporal_ptr(mrs_backbone *bb);
 MRS_API int mrs_backbone_temporal_dtype(mrs_backbone *bb);
 /* Which decode route the engine chose at creation (no counterpart in the reference; for tests and benchmarks that must
  * know what they measured): a whole step in one launch (small f32 models; 16-bit models up to d_model 1024 for as many rows
- * as the chip holds at once, Mamba-3 up to four layers -- 16-bit ones in one process per GPU, the first that asks, and not with
+ * as the chip holds at once, Mamba-3 at one row or up to four layers -- 16-bit ones in one process per GPU, the first that asks, and not with
  * MRS_DECODE_NO_RESIDENT=1), the library's own fused kernel chain, or the chain built on the vendor GEMM.  The one launch and the
- * chain add in different orders: equally far from f32, not the same bits. */
+ * chain add in different orders: equally far from f32, not the same bits (Mamba-3 at one row of a width that is a multiple of 256: the same). */
 #define MRS_DECODE_LIBRARY_CHAIN 0
 #define MRS_DECODE_OWN_CHAIN 1
 #define MRS_DECODE_ONE_LAUNCH 2
 MRS_API int mrs_backbone_decode_route(mrs_backbone *bb);
-/* A 16-bit step of a few rows in one launch (MRS_DECODE_ONE_LAUNCH) begins when all its workgroups have a place on the GPU. `polls`
+/* A 16-bit step in one launch (MRS_DECODE_ONE_LAUNCH) begins when all its workgroups have a place on the GPU. `polls`
  * (one to two microseconds each; 2^23 unless set) is how long it waits for that before it is called off with the state unchanged:
  * step() then runs the kernel chain instead, queued steps end in an error at the next call that synchronises, and both hold until
  * reset(). 0: called off at once, for trying out a program's handling of it. No effect on engines with another decode route. */
@@ -398,7 +398,11 @@ typedef struct {
 
 /* GpuMambaLM::generate_batch (src/module/gpu_lm.rs:389-516): one prompt per batch slot, of any length (an empty
  * prompt leaves its slot finished); prompts are consumed a token per step, slots whose prompt is done sample from
- * their own generator and stop at an EOS id or at max_tokens.  The whole loop -- gather, step, head, sampling and
+ * their own generator and stop at an EOS id or at max_tokens.  On a 16-bit Mamba-1 engine with d_state 16 (own decode chain, scan mode not
+ * sequential) what ALL slots' prompts have in front of their last token, from four tokens on, goes through prefill kernels instead, up to 32
+ * steps at a time: where a slot's roundings fall, and now and then a token, then depends on the shortest prompt of the batch (a slot without
+ * a prompt, or with one of up to four tokens, keeps every slot's tokens on steps).  MRS_SCAN_SEQUENTIAL in the config takes every
+ * token as a step, whatever the other slots hold.  The whole loop -- gather, step, head, sampling and
  * the per-slot bookkeeping -- stays on the device; the host only polls how many slots are still running.
  *   prompts: all prompts back to back; prompt_lens [batch]; params [batch];
  *   out_tokens [batch, out_stride] and out_lens [batch] receive the generated ids (prompt excluded);
@@ -411,7 +415,7 @@ MRS_API int mrs_lm_generate_batch(mrs_lm *lm, const int *prompts, const int *pro
                                   int seen_includes_prompt, int *out_tokens, int out_stride, int *out_lens);
 
 /* GpuMambaLM::generate_streaming (src/module/gpu_lm.rs:334-377), batch-1 engines: the loop of mrs_lm_generate_batch with
- * the penalty history over prompt + generated tokens and the prompt through the prefill path from 256 tokens on; every
+ * the penalty history over prompt + generated tokens and the prompt through the prefill path from 256 tokens on (below that as there); every
  * new token is handed to `cb` as soon as it exists (one host round trip per step).  A nonzero return from `cb` ends the
  * generation early (the reference's callback cannot; returning 0 always reproduces it). */
 typedef int (*mrs_token_callback)(int token, void *user);

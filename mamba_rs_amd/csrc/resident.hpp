@@ -1,5 +1,5 @@
-// Building blocks of the resident decode steps (resident_step.hip, resident_m3_step.hip): one launch walks the whole network, G workgroups
-// share every layer's columns, and what a layer's phases need from each other travels through memory while the workgroups stay
+// Building blocks of the resident decode steps (resident_step.hip, resident_rows.hip, resident_m3_step.hip, resident_m3_row.hip): one launch walks
+// the whole network, G workgroups share every layer's columns, and what a layer's phases need from each other travels through memory while the workgroups stay
 // on the chip.
 //
 // Exchange: a value and the number of the layer it belongs to (its tag) are one 64-bit word, stored and polled with relaxed
@@ -7,11 +7,12 @@
 // chip -- no counter, no fence, no cache write-back.  Measured for all-to-all exchanges of 768 values, two workgroup
 // barriers included: 1.3 us among 32 workgroups, 1.5 among 64, 1.8 among 128, 2.4 among 256 (a counter barrier over 256
 // workgroups: 2.3 to 3.7 us and the data still to be fetched; a kernel boundary in a graph: about 4 us).
-// A layer's exchanges form a cycle (residual -> x_proj shares -> y -> residual), each of them all-to-all, so a buffer is
-// rewritten only after every reader of its last contents has published something that depends on them: one buffer per
-// exchange is enough.
+// A layer's exchanges form a cycle (residual -> x_proj shares -> y -> residual), and a workgroup writes its words of the next layer only
+// behind the last of them, the residual, which everybody takes from everybody and puts out after its last read of the others: one buffer
+// per exchange is enough, also for one that only a few workgroups read (resident_rows.hip: u).
 //
-// A launch begins with a roll call (RollCall): no workgroup stores anything but exchange words before all of them are on the chip.
+// A launch begins with a roll call (RollCall): no workgroup stores anything but exchange words and operand rows before all of them are on
+// the chip; states and output rows it does not touch.
 // Ordinary kernels that hold the compute units delay it.  If the units do not come free within the wait the caller set, the launch is
 // called off as a whole: the states are what they were, the output rows become NaN, `broken` (host memory) is raised, and launches
 // queued behind it leave at once.  After the roll call a wait is over when its neighbours have done their part; those waits are

@@ -1,4 +1,4 @@
-// Who may run resident decode steps (resident_step.hip, resident_m3_step.hip), and when.
+// Who may run resident decode steps (the four kernels that include resident.hpp), and when.
 //
 // A resident launch's workgroups wait for each other, so they must all get a place on the GPU.  One launch alone always does (an
 // engine takes the route only while its workgroups are at most as many as the compute units, one each); two launches that hold

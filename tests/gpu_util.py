@@ -1,4 +1,4 @@
-"""Helpers for the GPU parity tests: numpy <-> device tensors and the north-star tolerances."""
+"""Helpers for the GPU parity tests: numpy <-> device tensors and the tolerances of the 16- and 32-bit kernels."""
 from __future__ import annotations
 
 import numpy as np
