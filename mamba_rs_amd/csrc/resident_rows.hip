@@ -70,7 +70,7 @@ struct RowsFeed {
     size_t conv_next, ssm_next;   // ... to those of the next layer
     int rows;
     unsigned spare;
-    bool hurry;                   // the workgroup forms x_proj rows: it does not wait for them
+    bool hurry;                   // the workgroup forms x_proj rows: it does not wait for them, but for u, a barrier earlier
 };
 // One request: a lane asks for a line, number `first` + lane of `lines` of 128 bytes per row.
 template <int LINES, int ROW_BYTES> __device__ __forceinline__ void touch_lines(unsigned spare, const char *at, int rows, int first) {
