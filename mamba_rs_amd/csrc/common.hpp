@@ -149,6 +149,10 @@ int launch_tiled_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t l
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 bool mid_gemm_wins(int64_t M, int N, int K);
 int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
+// The same for a prefill of thousands of rows (gemm_big.hip), C in the storage type
+bool big_gemm_ok(int dtype, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
+bool big_gemm_wins(int64_t M, int N, int K);
+int launch_big_gemm(hipStream_t st, int dtype, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 int skinny_max_rows();   // rows the 16-bit matrix-core route takes (128; MRS_SKINNY_MAX_ROWS overrides)
 bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, const void *Wt);
 int launch_skinny_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wt,

@@ -389,10 +389,13 @@ static int gemm_rm_t(mrs_backbone *bb, int dtype, void *C, int ldc, const void *
     return gemm_ex_tuned(bb->tuner, bb->blas, bb->stream, 1, N, M, K, Wt, t, K, A, t, lda, C, t, ldc);
 }
 
-// in_proj and out_proj of a prefill: the own kernel where the rows are few, else the library
+// in_proj and out_proj of a prefill: an own kernel where the rows are few or the library's tiles leave much of the chip idle (while its kernels are not
+// timed per shape: the tuned choice has other tiles), else the library
 static int prefill_projection(mrs_backbone *bb, int dtype, void *C, int ldc, const void *A, int lda, const void *W, const void *Wt, int M, int N, int K) {
     if (Wt && mid_gemm_wins(M, N, K) && mid_gemm_ok(dtype, 0, C, ldc, A, lda, Wt, M, N, K))
         return launch_mid_gemm(bb->stream, dtype, 0, C, ldc, A, lda, Wt, M, N, K);
+    if (Wt && !gemm_tuner_enabled(bb->tuner) && big_gemm_wins(M, N, K) && big_gemm_ok(dtype, C, ldc, A, lda, Wt, M, N, K))
+        return launch_big_gemm(bb->stream, dtype, C, ldc, A, lda, Wt, M, N, K);
     return Wt ? gemm_rm_t(bb, dtype, C, ldc, A, lda, Wt, M, N, K) : gemm_rm(bb, dtype, C, ldc, A, lda, W, M, N, K);
 }
 

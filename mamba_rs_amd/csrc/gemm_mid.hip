@@ -22,11 +22,6 @@ namespace {
 
 constexpr int kMidThreads = 256, kTile = 64, kStepK = 64, kStages = 4;
 
-// 1 KB: lane l's 16 bytes from `from` + voff to LDS byte address `to` + 16 l.  The compiler's wait counting does not see it.
-__device__ __forceinline__ void dma_kb(unsigned to, const void *from, unsigned voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(voff), "s"(from) : "m0", "memory");
-}
-
 template <typename T, typename TO>
 __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ C, int64_t ldc, const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt,
                                                                int M, int N, int K, int mtiles) {

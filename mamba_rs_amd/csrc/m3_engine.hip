@@ -1178,9 +1178,17 @@ int launch_add_rmsnorm3(mrs_m3_backbone *bb, float *residual, const void *add, v
                                   bb->cfg.d_model);
 }
 
-// A projection of a prefill (dense rows, weight as the transposed copy) on the own kernel instead of the library's
-bool own_projection(int dt, int out_f32, const void *C, int ldc, const void *A, const void *Wt, int64_t rows, int N, int K) {
-    return Wt && mid_gemm_wins(rows, N, K) && mid_gemm_ok(dt, out_f32, C, ldc, A, K, Wt, rows, N, K);
+// A projection of a prefill (dense rows, weight as the transposed copy) on an own kernel instead of the library's: `mid` for few rows, `big` (results in
+// the storage type) where the library's tiles leave much of the chip idle, while its kernels are not timed per shape
+enum OwnProjection { kLibrary, kMid, kBig };
+OwnProjection own_projection(const mrs_m3_backbone *bb, int out_f32, const void *C, int ldc, const void *A, const void *Wt, int64_t rows, int N, int K) {
+    if (!Wt) return kLibrary;
+    if (mid_gemm_wins(rows, N, K) && mid_gemm_ok(bb->dtype, out_f32, C, ldc, A, K, Wt, rows, N, K)) return kMid;
+    return !out_f32 && !gemm_tuner_enabled(bb->tuner) && big_gemm_wins(rows, N, K) && big_gemm_ok(bb->dtype, C, ldc, A, K, Wt, rows, N, K) ? kBig : kLibrary;
+}
+int launch_own_projection(const mrs_m3_backbone *bb, OwnProjection how, int out_f32, void *C, int ldc, const void *A, const void *Wt, int64_t rows, int N, int K) {
+    if (how == kBig) return launch_big_gemm(bb->stream, bb->dtype, C, ldc, A, K, Wt, rows, N, K);
+    return launch_mid_gemm(bb->stream, bb->dtype, out_f32, C, ldc, A, K, Wt, rows, N, K);
 }
 
 int prefill_body3(mrs_m3_backbone *bb, int T) {
@@ -1226,11 +1234,11 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
                 // the vendor kernels for the transposed operand are faster at these shapes (the copy's first nb rows, then the rest)
                 if (lw.in_proj_t) {
                     const char *wt = (const char *)lw.in_proj_t, *wt_rest = wt + (size_t)nb * dm * es;
-                    if (own_projection(dt, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm))
-                        MRS_TRY(launch_mid_gemm(bb->stream, dt, 0, bb->pf_bulk, nb, bb->pf_normed, dm, wt, rows, nb, dm));
+                    if (const OwnProjection own = own_projection(bb, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm))
+                        MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm));
                     else MRS_TRY(gemm(1, nb, wt, dm, bb->pf_bulk, t, nb));
-                    if (own_projection(dt, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm))
-                        MRS_TRY(launch_mid_gemm(bb->stream, dt, 1, bb->pf_proj, ns, bb->pf_normed, dm, wt_rest, rows, ns, dm));
+                    if (const OwnProjection own = own_projection(bb, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm))
+                        MRS_TRY(launch_own_projection(bb, own, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm));
                     else MRS_TRY(gemm(1, ns, wt_rest, dm, bb->pf_proj, f32t, ns));
                 } else {
                     MRS_TRY(gemm(0, nb, lw.in_proj, ip, bb->pf_bulk, t, nb));
@@ -1295,8 +1303,8 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         if (!gate_in_scan) MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_gate_t<T_>(bb, lw, rows, bulk, ldb)));
         if (l + 1 == L && last_step_gemm_ok(dt, bb->pf_gated, lw.out_proj_t, B, T, dm, di))
             MRS_TRY(launch_last_step_gemm(bb->stream, dt, bb->pf_out, bb->pf_gated, lw.out_proj_t, B, T, dm, di));
-        else if (own_projection(dt, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
-            MRS_TRY(launch_mid_gemm(bb->stream, dt, 0, bb->pf_out, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di));
+        else if (const OwnProjection own = own_projection(bb, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
+            MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di));
         else MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));
     }
     // only the last position of each sequence is kept: final residual add + norm_f on those rows

@@ -21,4 +21,9 @@ template <> struct Mma32<f16_t> {
     }
 };
 
+// 1 KB: lane l's 16 bytes from `from` + voff to LDS byte address `to` + 16 l.  The compiler's wait counting does not see it.
+__device__ __forceinline__ void dma_kb(unsigned to, const void *from, unsigned voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(voff), "s"(from) : "m0", "memory");
+}
+
 }  // namespace mrs

@@ -42,3 +42,32 @@ def test_prefill_of_few_rows_follows_the_cpu_route(dm, B, T, dtype):
         hs, cs = s[0].reshape(di, 16), c[0].reshape(di, 3)
         assert cosine(ssm[b], hs) >= 0.999 and scaled_err(ssm[b], hs) < 5e-2, (b, cosine(ssm[b], hs), scaled_err(ssm[b], hs))
         assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
+
+
+@pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
+@pytest.mark.parametrize("dm,B,T", [
+    (128, 33, 1000),   # tiles of 192 columns, the last a third empty; two k-steps, one pair of buffers
+    (320, 11, 1187),   # tiles of 320 columns; five k-steps; the last row tile holds one row
+    (320, 13, 1024),   # whole tiles both ways
+    (448, 10, 946),    # the last column tile holds 192 of its 320; seven k-steps; workgroups not a multiple of eight
+])
+def test_long_prefill_on_the_large_tiles_follows_the_cpu_route(dm, B, T, dtype):
+    """in_proj on the 256-row tiles (row counts at which the library's would leave a round partly empty): sequences from both ends and
+    the middle of the rows, bounds as above."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 6)
+    P = oracle_params(w, cfg, dm, round_to=orc.BF16 if dtype == WeightDtype.BF16 else orc.F16)
+    x = (np.random.default_rng(dm + T).standard_normal((B, T, dm)) * 0.5).astype(np.float32)
+    print(f"case large prefill projections d_model={dm} rows={B * T} {dtype.name}", flush=True)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    last = eng.prefill_sequence(x)
+    conv, ssm = eng.download_state(0)
+    eng.close()
+    di = cfg.d_inner()
+    for b in (0, 1, B // 2, B - 2, B - 1):
+        c, s = orc.m1_zero_state(P)
+        want = orc.m1_backbone_prefill(P, x[b], c, s)[-1]
+        assert cosine(last[b], want) >= 0.999 and scaled_err(last[b], want) < 5e-2, (b, cosine(last[b], want), scaled_err(last[b], want))
+        hs, cs = s[0].reshape(di, 16), c[0].reshape(di, 3)
+        assert cosine(ssm[b], hs) >= 0.999 and scaled_err(ssm[b], hs) < 5e-2, (b, cosine(ssm[b], hs), scaled_err(ssm[b], hs))
+        assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
