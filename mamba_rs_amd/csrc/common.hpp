@@ -196,6 +196,10 @@ bool tiny_m3_step_ok(int dtype, int input_dim, int dm, int di, int nh, int hd, i
 int launch_tiny_m3_step(hipStream_t st, const TinyM3StepArgs &a);
 bool tiny_step_ok(int dtype, int input_dim, int dm, int di, int ds, int dc, int dr, int xd);
 int launch_tiny_step(hipStream_t st, const TinyStepArgs &a);
+// The rows a step starts from, where they are rows of an embedding table (storage type, [vocab][d_model]) and not in the input buffer: those of `tokens`
+// (clamped to the vocabulary), zeros where finished (may be null) says so.  embed null: the input buffer's.  The kernel that takes them leaves them in the
+// input buffer as well.
+struct TokenRows { const void *embed; const int *tokens, *finished; int vocab; };
 // A whole Mamba-1 backbone step in one resident launch (resident_step.hip), 16-bit storage.  G workgroups per batch row, each owning nc
 // channels and oc out_proj columns (resident_plan fills these in).  weights: n_layers blocks of resident_layer_bytes(), each
 // packed by launch_resident_pack from a layer's weights as the engine holds them.  norm_w: layer 0's norm weight.  xch: groups *
@@ -209,7 +213,8 @@ struct ResidentLayer {   // in_t [2 d_inner][d_model], out_t [d_model][d_inner],
 };
 struct ResidentArgs {
     const void *weights;
-    const float *input, *norm_w, *norm_f;
+    float *input;
+    const float *norm_w, *norm_f;
     float *conv_state, *ssm_state, *temporal;
     void *temporal_t;
     unsigned long long *xch;
@@ -224,14 +229,14 @@ struct ResidentArgs {
 bool resident_plan(ResidentArgs &a, int dtype);   // false: the shape is outside the route
 size_t resident_layer_bytes(const ResidentArgs &a);
 int launch_resident_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
-int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);   // dev: a copy of `a` on the device
+int launch_resident_step(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev, const TokenRows &rows);   // dev: a copy of `a` on the device
 // The same with up to kResidentRows batch rows per group of workgroups, with its own pack and sizes (resident_rows.hip).
 constexpr int kResidentRows = 16;
 bool resident_rows_plan(ResidentArgs &a, int dtype);
 size_t resident_rows_bytes(const ResidentArgs &a);
 size_t resident_rows_layer_bytes(const ResidentArgs &a);
 int launch_resident_rows_pack(hipStream_t st, const ResidentArgs &a, void *dst, const ResidentLayer &w);
-int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev);
+int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev, const TokenRows &rows);
 // The same for the Mamba-3 SISO backbone (resident_m3_step.hip); ex: columns of in_proj behind z and x that a workgroup owns.
 struct ResidentM3Layer {   // in_t [ip][d_model] and out_t [d_model][d_inner] transposed; next_nw: the norm weight after, or null
     const void *in_t, *out_t; const float *bnw, *cnw, *b_bias, *c_bias, *D, *dt_bias, *next_nw;
@@ -239,8 +244,10 @@ struct ResidentM3Layer {   // in_t [ip][d_model] and out_t [d_model][d_inner] tr
 // row_order: the step that adds in the kernel chain's order (one row); norm_rows: every layer's norm weight, [n_layers][d_model], for it
 struct ResidentM3Args {
     const void *weights;
-    const float *input, *norm_w, *norm_f, *norm_rows;
+    float *input;
+    const float *norm_w, *norm_f, *norm_rows;
     float *ssm, *kst, *vst, *angle, *temporal;
+    void *temporal_t;
     unsigned long long *xch;
     unsigned *epoch, *roll, *broken;
     size_t xch_stride;
@@ -251,14 +258,14 @@ struct ResidentM3Args {
 bool resident_m3_plan(ResidentM3Args &a, int dtype);
 size_t resident_m3_layer_bytes(const ResidentM3Args &a);
 int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, const ResidentM3Layer &w);
-int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev);
+int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows);
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,
                             int64_t rows, int di, int dr);
 // partials[row][0] = sum_k x[row][k]^2, partials[row][1..n_partials) = 0; prenorm[row][k] = round(x[row][k] * w[k])
-// a_mt != 0: prenorm is written in the tiled order of tiled_a_index with a_mt row tiles
-int launch_prenorm_rows(hipStream_t st, int dtype, float *partials, int n_partials, void *prenorm, const float *x, float *copy_to,
-                        const float *w, int M, int K, int a_mt = 0);
+// a_mt != 0: prenorm is written in the tiled order of tiled_a_index with a_mt row tiles.  With rows (an embedding table) x is written instead of read.
+int launch_prenorm_rows(hipStream_t st, int dtype, float *partials, int n_partials, void *prenorm, float *x, float *copy_to,
+                        const float *w, int M, int K, int a_mt = 0, const TokenRows &rows = {});
 
 // mrs_m3_ssd_fwd with x read in place out of wider rows (x_stride elements apart, 0 = dense; 16-bit storage only).
 // With `gen` the kernel forms K and Q itself (K and Q are not read and may be null): K = rot(angle, bn + b_bias[head]),
@@ -286,8 +293,8 @@ struct LmHooks {
     void *blas;               // rocblas_handle of the engine
     float *d_input;           // [batch, d_model] f32: the rows a step reads
     float *temporal;          // [batch, d_model] f32: final-norm output of the last step / prefill
-    void *temporal_t;         // the same in the storage type, or null when the engine keeps no such copy
-    int (*step)(void *self);                         // one decode step (capturable: launches only)
+    void *temporal_t;         // the same in the storage type (null in f32)
+    int (*step)(void *self, const TokenRows &rows);  // one decode step on those rows (capturable: launches only)
     int (*reset)(void *self);
     size_t (*state_bytes)(void *self);               // recurrent state, for save / restore around a warm-up run
     int (*state_copy)(void *self, void *buf, int restore);
@@ -302,7 +309,8 @@ struct LmHooks {
     bool (*go_on_chain)(void *self);   // after a synchronisation: the one step since the last check was called off, the next ones are kernel chains
 };
 // gathers rows of the embedding table (storage type) as f32: out[r, :] = embed[clamp(tokens[r]), :] (engine prefill staging)
-int launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab);
+int launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab,
+                        const int *finished = nullptr);
 
 // sample_token for every active row (sampling.hip); all pointers device memory
 int launch_sample_rows(hipStream_t st, int *tokens, const float *logits, float *work, int64_t ld, int rows, int vocab,

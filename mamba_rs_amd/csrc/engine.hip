@@ -111,51 +111,48 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(float *__restrict__ o
 }
 
 // Greedy pick: index of the maximum logit, the LAST one among equals (Iterator::max_by,
-// src/module/sample.rs:250-257).  Stage 1: kArgParts blocks per row reduce a slice each; stage 2 combines.
-constexpr int kArgParts = 32;
-__device__ __forceinline__ void argmax_block_reduce(float &best, int &bi) {
-    __shared__ float sv[256];
-    __shared__ int si[256];
-    sv[threadIdx.x] = best; si[threadIdx.x] = bi;
-    __syncthreads();
-    for (int s = 128; s >= 1; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            const float ov = sv[threadIdx.x + s];
-            const int oi = si[threadIdx.x + s];
-            if (ov > sv[threadIdx.x] || (ov == sv[threadIdx.x] && oi > si[threadIdx.x])) { sv[threadIdx.x] = ov; si[threadIdx.x] = oi; }
-        }
-        __syncthreads();
+// src/module/sample.rs:250-257).  A workgroup reduces a slice of 1024 V entries of a row, all asked for at once; its maximum meets the others' as one 64-bit
+// key, the value's ordered bits above the index, and the row's last workgroup to arrive leaves the token and clears the two words for the next time.  (As a
+// launch that left 32 partial maxima per row and a second one over those, 4.9 + 4.0 us in a graph at one row, this 4.0; 5.4 + 4.1 at 64, this 6.0; 5.0 + 4.0 at 16, this 4.7.)  The
+// meeting is what many rows cost: a line per row, and longer slices (eight rows to a line, slices of 2048: 6.9 us at 16 rows, 8.1 at 64).
+struct alignas(128) ArgRow { unsigned long long key; unsigned arrived; };
+template <int V> __global__ __launch_bounds__(256) void argmax_kernel(int *__restrict__ tokens, ArgRow *__restrict__ rows, const float *__restrict__ logits, int vocab, int64_t stride, int none) {
+    __shared__ unsigned long long part[4];
+    constexpr int slice = 1024 * V;
+    const int slices = (vocab + slice - 1) / slice, row = blockIdx.x / slices, tid = threadIdx.x;
+    const float *r = logits + (int64_t)row * stride;   // (16-byte aligned, and so is the stride)
+    const int i0 = ((int)blockIdx.x - row * slices) * slice + 4 * tid;
+    float v[4 * V];
+#pragma unroll
+    for (int h = 0; h < V; h++) {
+        const float4 x = *reinterpret_cast<const float4 *>(r + min((int64_t)i0 + 1024 * h, stride - 4));
+        v[4 * h] = x.x; v[4 * h + 1] = x.y; v[4 * h + 2] = x.z; v[4 * h + 3] = x.w;
     }
-    best = sv[0]; bi = si[0];
-}
-__global__ __launch_bounds__(256) void argmax_part_kernel(float *__restrict__ pv, int *__restrict__ pi,
-                                                          const float *__restrict__ logits, int vocab, int64_t stride) {
-    const int row = blockIdx.x / kArgParts, part = blockIdx.x % kArgParts;
-    const int per = (vocab + kArgParts - 1) / kArgParts;
-    const int lo = part * per, hi = min(vocab, lo + per);
-    const float *r = logits + (int64_t)row * stride;
-    float best = -INFINITY;
-    int bi = lo < vocab ? lo : vocab - 1;
-    for (int i = lo + threadIdx.x; i < hi; i += 256) {
-        const float v = r[i];
-        if (v >= best) { best = v; bi = i; }   // ascending i per thread: >= keeps the last maximum
-    }
-    argmax_block_reduce(best, bi);
-    if (threadIdx.x == 0) { pv[blockIdx.x] = best; pi[blockIdx.x] = bi; }
-}
-__global__ __launch_bounds__(64) void argmax_final_kernel(int *__restrict__ tokens, const float *__restrict__ pv,
-                                                          const int *__restrict__ pi) {
-    const int row = blockIdx.x;
     float best = -INFINITY;
     int bi = 0;
-    if (threadIdx.x < kArgParts) { best = pv[row * kArgParts + threadIdx.x]; bi = pi[row * kArgParts + threadIdx.x]; }
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        const float ov = __shfl_xor(best, m, kWave);
-        const int oi = __shfl_xor(bi, m, kWave);
-        if (ov > best || (ov == best && oi > bi)) { best = ov; bi = oi; }
+    for (int k = 0; k < 4 * V; k++) {
+        const int i = i0 + 1024 * (k >> 2) + (k & 3);
+        if (i < vocab && v[k] >= best) { best = v[k]; bi = i; }   // ascending: >= keeps the last maximum
     }
-    if (threadIdx.x == 0) tokens[row] = bi;
+    if (best == -INFINITY) bi = max(bi, none);   // nothing above it in the row (or NaN throughout)
+    const unsigned bits = __float_as_uint(best + 0.0f);   // (the two zeros are equal)
+    unsigned long long key = (unsigned long long)((bits & 0x80000000u) ? ~bits : (bits | 0x80000000u)) << 32 | (unsigned)bi;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) key = max(key, (unsigned long long)__shfl_xor((long long)key, m, kWave));
+    if ((tid & 63) == 0) part[tid >> 6] = key;
+    __syncthreads();
+    if (tid == 0) {
+        ArgRow *a = rows + row;
+        key = max(max(part[0], part[1]), max(part[2], part[3]));
+        const unsigned long long before = __hip_atomic_fetch_max(&a->key, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::"v"((unsigned)before), "v"((unsigned)(before >> 32)) : "memory");   // it has come back: the maximum is in before the arrival is counted
+        if (__hip_atomic_fetch_add(&a->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)slices - 1) {
+            tokens[row] = (int)(unsigned)__hip_atomic_load(&a->key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a->key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 // ---- generate_batch bookkeeping on the device (src/module/gpu_lm.rs:404-513) ------------------------------
@@ -288,7 +285,8 @@ struct Scratch {  // activations for M rows
 struct mrs_backbone {
     mrs_m1_config cfg;
     int input_dim, batch, dtype, di, dr, xd, identity_proj, device;
-    const float *step_src;  // decode step: where layer 0 reads its input rows (null: the residual buffer itself)
+    float *step_src;  // decode step: where layer 0 reads its input rows (null: the residual buffer itself)
+    TokenRows step_rows;    // ... or the embedding rows it takes in their place
     int split_xproj;  // library chain at up to 128 rows of a wide 16-bit model: x_proj as a K-split launch of the own GEMM
     int tiled;   // own chain from two (narrow models) or three rows up: the projections read tiled weights and tiled activation operands
     int wide;    // ... and in_proj / out_proj run on the column-tile kernel of gemm_wide.hip (wide models, up to 64 rows)
@@ -462,8 +460,10 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         float *conv = bb->conv_state + ((size_t)l * B + r0) * di * dc;
         float *ssm = bb->ssm_state + ((size_t)l * B + r0) * di * ds;
         if (l == 0) {
-            const float *src = bb->step_src ? bb->step_src + (size_t)r0 * dm : residual;
-            MRS_TRY(launch_prenorm_rows(st, dt, partials, P, normed, src, bb->step_src ? residual : nullptr, lw.norm_w, nr, dm, a_mt));
+            float *src = bb->step_src ? bb->step_src + (size_t)r0 * dm : residual;
+            TokenRows rows = bb->step_rows;   // (of this chain's rows)
+            if (rows.embed) { rows.tokens += r0; if (rows.finished) rows.finished += r0; }
+            MRS_TRY(launch_prenorm_rows(st, dt, partials, P, normed, src, bb->step_src ? residual : nullptr, lw.norm_w, nr, dm, a_mt, rows));
         }
         SkinnyEpi inp = {};
         inp.mode = 1; inp.conv_state = conv; inp.conv_w = lw.conv_w; inp.conv_b = lw.conv_b; inp.u = u; inp.di = di; inp.dc = dc;
@@ -924,14 +924,16 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
-static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
+static int step_body(mrs_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}) {
     if (bb->resident) {
         const ResidentTurn turn(&bb->seat);
         if (turn.go()) {
             if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
-            return (bb->resident == 1 ? launch_resident_step : launch_resident_rows)(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+            return (bb->resident == 1 ? launch_resident_step : launch_resident_rows)(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev, rows);
         }
     }
+    const bool taken = bb->identity_proj && bb->skinny && !bb->tiny_layers;   // the first layer's prenorm kernel takes the rows itself
+    if (rows.embed && !taken) MRS_TRY(launch_embed_gather(bb->stream, bb->dtype, bb->d_input, rows.embed, rows.tokens, bb->batch, bb->cfg.d_model, rows.vocab, rows.finished));
     if (bb->tiny_layers) {
         TinyStepArgs a = {};
         a.layers = bb->tiny_layers; a.input = bb->d_input;
@@ -944,7 +946,8 @@ static int step_body(mrs_backbone *bb, const HostRows *host = nullptr) {
     }
     // identity projection on the own-GEMM chain: the first layer's prenorm kernel reads the input and writes the
     // residual stream itself, so no copy is needed
-    bb->step_src = (bb->identity_proj && bb->skinny) ? bb->d_input : nullptr;
+    bb->step_src = taken ? bb->d_input : nullptr;
+    bb->step_rows = taken ? rows : TokenRows();
     if (!bb->step_src) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
     return run_layers(bb, &bb->step_s, 1);
 }
@@ -1157,7 +1160,6 @@ extern "C" int mrs_backbone_download_state(mrs_backbone *bb, int layer, float *c
 struct mrs_lm {
     LmHooks eng;        // decode engine (not owned)
     mrs_backbone *bb;   // the same engine when it is a Mamba-1 backbone, else null
-    void *hid_t;        // head operand in the storage type when the engine keeps none
     int vocab, vocab_padded, dm, batch, dtype;
     void *embed;        // [vocab_padded, dm] storage dtype (tied lm_head)
     void *head;         // [vocab_padded, dm] storage dtype when the head has weights of its own, else null
@@ -1175,19 +1177,18 @@ struct mrs_lm {
     int gen_ready, gen_graph_ready;
     float *logits;      // [batch, vocab_padded] f32
     int *tokens;        // [batch] current token ids on device
-    float *arg_v;       // [batch, kArgParts] partial maxima
-    int *arg_i;
+    ArgRow *arg_rows;   // [batch], zero between two picks
     std::vector<void *> allocs;
     hipGraph_t graph;
     hipGraphExec_t graph_exec;
     int graph_ready;
 };
 
-int mrs::launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab) {
+int mrs::launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab, const int *finished) {
     const int64_t n = rows * dm;
     const dim3 grid((unsigned)((n + 255) / 256)), block(256);
     MRS_DISPATCH_DTYPE(dtype, T_, hipLaunchKernelGGL((embed_gather_kernel<T_>), grid, block, 0, st, out, (const T_ *)embed, tokens, rows, dm, vocab,
-                                                     (const int *)nullptr));
+                                                     finished));
     return check_launch("embed_gather_kernel");
 }
 
@@ -1197,7 +1198,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     if (vocab < 1) return fail(MRS_E_SHAPE, "%s: vocab=%d", fn, vocab);
     mrs_lm *lm = new (std::nothrow) mrs_lm();
     if (!lm) return fail(MRS_E_HIP, "%s: out of host memory", fn);
-    lm->eng = eng; lm->bb = nullptr; lm->hid_t = nullptr;
+    lm->eng = eng; lm->bb = nullptr;
     lm->vocab = vocab; lm->vocab_padded = (vocab + 63) & ~63;  // src/hf/load.rs:59
     lm->dm = eng.d_model; lm->batch = eng.batch; lm->dtype = eng.dtype; lm->graph_ready = 0; lm->graph = nullptr; lm->graph_exec = nullptr;
     lm->head = nullptr;
@@ -1211,9 +1212,8 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     MRS_LM_HIP(hipMalloc(&lm->embed, ne * es)); lm->allocs.push_back(lm->embed);
     MRS_LM_HIP(hipMalloc((void **)&lm->logits, (size_t)lm->batch * lm->vocab_padded * 4)); lm->allocs.push_back(lm->logits);
     MRS_LM_HIP(hipMalloc((void **)&lm->tokens, (size_t)lm->batch * sizeof(int))); lm->allocs.push_back(lm->tokens);
-    MRS_LM_HIP(hipMalloc((void **)&lm->arg_v, (size_t)lm->batch * kArgParts * sizeof(float))); lm->allocs.push_back(lm->arg_v);
-    MRS_LM_HIP(hipMalloc((void **)&lm->arg_i, (size_t)lm->batch * kArgParts * sizeof(int))); lm->allocs.push_back(lm->arg_i);
-    if (!eng.temporal_t && lm->dtype != MRS_F32) { MRS_LM_HIP(hipMalloc(&lm->hid_t, (size_t)lm->batch * lm->dm * es)); lm->allocs.push_back(lm->hid_t); }
+    MRS_LM_HIP(hipMalloc((void **)&lm->arg_rows, (size_t)lm->batch * sizeof(ArgRow))); lm->allocs.push_back(lm->arg_rows);
+    MRS_LM_HIP(hipMemsetAsync(lm->arg_rows, 0, (size_t)lm->batch * sizeof(ArgRow), eng.stream));
     MRS_LM_HIP(hipMalloc((void **)&stage, ne * 4));
     MRS_LM_HIP(hipMemsetAsync(stage, 0, ne * 4, eng.stream));  // padded rows are zero
     MRS_LM_HIP(hipMemcpyAsync(stage, embed, (size_t)vocab * lm->dm * 4, hipMemcpyHostToDevice, eng.stream));
@@ -1229,7 +1229,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
 }
 
 // ---- the Mamba-1 engine behind the LM loop ----
-static int m1_hook_step(void *self) { return step_body((mrs_backbone *)self); }
+static int m1_hook_step(void *self, const TokenRows &rows) { return step_body((mrs_backbone *)self, nullptr, rows); }
 static int m1_hook_reset(void *self) { return mrs_backbone_reset((mrs_backbone *)self); }
 static size_t m1_hook_state_bytes(void *self) {
     mrs_backbone *bb = (mrs_backbone *)self;
@@ -1326,18 +1326,7 @@ static int lm_logits(mrs_lm *lm) {
     const LmHooks *bb = &lm->eng;
     const int dm = lm->dm, V = lm->vocab_padded, B = lm->batch;
     const float one = 1.0f, zero = 0.0f;
-    // the head's operand is the final norm's result in the storage type: the engine's own copy (temporal_t), or a cast
-    const void *hid = bb->temporal;
-    if (lm->dtype != MRS_F32) {
-        hid = bb->temporal_t;
-        if (!hid) {
-            const int64_t n = (int64_t)B * dm;
-            const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-            if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, bb->stream, (bf16_t *)lm->hid_t, bb->temporal, n);
-            else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, bb->stream, (f16_t *)lm->hid_t, bb->temporal, n);
-            hid = lm->hid_t;
-        }
-    }
+    const void *hid = lm->dtype != MRS_F32 ? bb->temporal_t : bb->temporal;   // the final norm's result in the storage type
     // f32 tables at one to four rows: the table is already [vocab][d_model], the layout the row-wise route of the
     // library's own GEMM walks (the vendor kernel for this shape moves the 154 MB of a 50k x 768 table at 1.6 TB/s)
     const void *table = lm->head ? lm->head : lm->embed;
@@ -1354,19 +1343,19 @@ static int lm_logits(mrs_lm *lm) {
 
 static int lm_argmax(mrs_lm *lm) {
     hipStream_t st = lm->eng.stream;
-    hipLaunchKernelGGL(argmax_part_kernel, dim3((unsigned)(lm->batch * kArgParts)), dim3(256), 0, st, lm->arg_v, lm->arg_i, lm->logits,
-                       lm->vocab, (int64_t)lm->vocab_padded);
-    hipLaunchKernelGGL(argmax_final_kernel, dim3((unsigned)lm->batch), dim3(64), 0, st, lm->tokens, lm->arg_v, lm->arg_i);
-    return check_launch("argmax kernels");
+    const int per = (lm->vocab + 31) / 32;
+    const auto pick = [&](auto kernel, int slice) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((lm->vocab + slice - 1) / slice * lm->batch)), dim3(256), 0, st, lm->tokens, lm->arg_rows, lm->logits, lm->vocab,
+                           (int64_t)lm->vocab_padded, std::min(31 * per, lm->vocab - 1));
+    };
+    if (lm->batch < 8) pick(argmax_kernel<2>, 2048);
+    else pick(argmax_kernel<8>, 8192);
+    return check_launch("argmax_kernel");
 }
 
 static int lm_decode_body(mrs_lm *lm) {
     const LmHooks *bb = &lm->eng;
-    const int64_t n = (int64_t)lm->batch * lm->dm;
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    MRS_DISPATCH_DTYPE(lm->dtype, T_, hipLaunchKernelGGL((embed_gather_kernel<T_>), grid, block, 0, bb->stream, bb->d_input,
-                                                         (const T_ *)lm->embed, lm->tokens, (int64_t)lm->batch, lm->dm, lm->vocab));
-    MRS_TRY(bb->step(bb->self));
+    MRS_TRY(bb->step(bb->self, {lm->embed, lm->tokens, nullptr, lm->vocab}));
     MRS_TRY(lm_logits(lm));
     return lm_argmax(lm);
 }
@@ -1497,12 +1486,7 @@ static int gen_pick(mrs_lm *lm) {
 // gather the slots' current tokens (zeros for finished slots), one backbone step, head
 static int gen_forward(mrs_lm *lm) {
     const LmHooks *bb = &lm->eng;
-    const int64_t n = (int64_t)lm->batch * lm->dm;
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    MRS_DISPATCH_DTYPE(lm->dtype, T_, hipLaunchKernelGGL((embed_gather_kernel<T_>), grid, block, 0, bb->stream, bb->d_input,
-                                                         (const T_ *)lm->embed, lm->tokens, (int64_t)lm->batch, lm->dm, lm->vocab,
-                                                         (const int *)lm->gen.finished));
-    MRS_TRY(bb->step(bb->self));
+    MRS_TRY(bb->step(bb->self, {lm->embed, lm->tokens, lm->gen.finished, lm->vocab}));
     return lm_logits(lm);
 }
 

@@ -575,6 +575,7 @@ struct mrs_m3_backbone {
     float *input_proj_w, *input_proj_b, *norm_f;
     float *ssm, *kst, *vst, *angle;          // [L][batch]...
     float *d_input, *temporal, *residual, *proj, *partials;
+    void *temporal_t;             // temporal once more in the storage type (16-bit engines), the LM head's operand
     void *normed, *gated, *out;
     hipGraph_t graph;
     hipGraphExec_t graph_exec;
@@ -699,7 +700,7 @@ int setup_resident3(mrs_m3_backbone *bb) {
     const int L = bb->cfg.n_layers;
     ResidentM3Args &a = bb->res_args;
     a.input = bb->identity_proj ? bb->d_input : bb->residual;
-    a.norm_f = bb->norm_f; a.ssm = bb->ssm; a.kst = bb->kst; a.vst = bb->vst; a.angle = bb->angle; a.temporal = bb->temporal;
+    a.norm_f = bb->norm_f; a.ssm = bb->ssm; a.kst = bb->kst; a.vst = bb->vst; a.angle = bb->angle; a.temporal = bb->temporal; a.temporal_t = bb->temporal_t;
     MRS_TRY(dev_alloc3(bb, (void **)&a.xch, (size_t)a.batch * a.xch_stride * 8));
     MRS_TRY(dev_alloc3(bb, (void **)&a.epoch, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4));
     a.roll = a.epoch + (size_t)a.batch * 32;
@@ -766,15 +767,17 @@ bool go_on_chain3(mrs_m3_backbone *bb) {
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
-int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
+int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}) {
     const mrs_m3_config &c = bb->cfg;
     if (bb->resident) {
         const ResidentTurn turn(&bb->seat);
         if (turn.go()) {
             if (!bb->identity_proj) MRS_TRY(project_input3(bb));
-            return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev);
+            return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev, rows);
         }
     }
+    const bool taken = bb->identity_proj && bb->skinny && !bb->tiny_layers;   // the first layer's prenorm kernel takes the rows itself
+    if (rows.embed && !taken) MRS_TRY(launch_embed_gather(bb->stream, bb->dtype, bb->d_input, rows.embed, rows.tokens, bb->batch, c.d_model, rows.vocab, rows.finished));
     if (bb->tiny_layers) {
         TinyM3StepArgs a = {};
         a.layers = bb->tiny_layers; a.input = bb->d_input;
@@ -790,9 +793,9 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
     const int P = (dm + 15) / 16;
     const int a_mt = bb->tiled ? (B + 15) / 16 : 0;   // the projections' operands in tile order (16-row tiles)
     // residual <- input (identity) or input . W + b
-    const float *src = nullptr;
+    float *src = nullptr;
     if (bb->identity_proj) {
-        if (bb->skinny) src = bb->d_input;   // the first prenorm kernel reads the input and writes the residual stream
+        if (taken) src = bb->d_input;   // the first prenorm kernel reads the input and writes the residual stream
         else MRS_HIP(hipMemcpyAsync(bb->residual, bb->d_input, (size_t)B * dm * 4, hipMemcpyDeviceToDevice, bb->stream));
     } else {
         MRS_TRY(project_input3(bb));
@@ -802,7 +805,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
         if (bb->skinny) {
             if (l == 0)
                 MRS_TRY(launch_prenorm_rows(bb->stream, dt, bb->partials, P, bb->normed, src ? src : bb->residual, src ? bb->residual : nullptr,
-                                            lw.norm_w, B, dm, a_mt));
+                                            lw.norm_w, B, dm, a_mt, taken ? rows : TokenRows()));
             SkinnyEpi inp = {};
             inp.row_scale = 1; inp.partials = bb->partials; inp.n_partials = P; inp.eps = c.rms_norm_eps;
             inp.a_tiled = inp.w_tiled = a_mt ? 1 : 0;
@@ -824,7 +827,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr) {
         }
     }
     // final residual add (library chain) + norm_f -> temporal (f32)
-    return launch_add_rmsnorm_any(bb->stream, dt, bb->residual, bb->skinny ? nullptr : bb->out, bb->temporal, true, nullptr, bb->norm_f,
+    return launch_add_rmsnorm_any(bb->stream, dt, bb->residual, bb->skinny ? nullptr : bb->out, bb->temporal, true, bb->temporal_t, bb->norm_f,
                                   c.rms_norm_eps, B, dm, dm);
 }
 
@@ -979,6 +982,8 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->angle, (size_t)L * B * nh * na * 4));
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->d_input, B * input_dim * 4));
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->temporal, B * dm * 4));
+    bb->temporal_t = nullptr;
+    if (dtype != MRS_F32) MRS_CREATE_TRY(dev_alloc3(bb, &bb->temporal_t, B * dm * es));
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->residual, B * dm * 4));
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->proj, B * ip * 4));
     MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->partials, B * ((dm + 15) / 16) * 4));
@@ -1309,7 +1314,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
     }
     // only the last position of each sequence is kept: final residual add + norm_f on those rows
     const size_t r = (size_t)(T - 1) * dm;
-    return launch_add_rmsnorm_any(bb->stream, dt, bb->pf_residual + r, (const char *)bb->pf_out + r * es, bb->temporal, true, nullptr, bb->norm_f,
+    return launch_add_rmsnorm_any(bb->stream, dt, bb->pf_residual + r, (const char *)bb->pf_out + r * es, bb->temporal, true, bb->temporal_t, bb->norm_f,
                                   c.rms_norm_eps, B, dm, (int64_t)T * dm);
 }
 
@@ -1387,7 +1392,7 @@ void m3_state_sizes(mrs_m3_backbone *bb, size_t (&n)[4]) {
 }
 int m3_hook_check(void *self) { return check_resident3((mrs_m3_backbone *)self); }
 bool m3_hook_go_on_chain(void *self) { return go_on_chain3((mrs_m3_backbone *)self); }
-int m3_hook_step(void *self) { return step_body3((mrs_m3_backbone *)self); }
+int m3_hook_step(void *self, const TokenRows &rows) { return step_body3((mrs_m3_backbone *)self, nullptr, rows); }
 int m3_hook_reset(void *self) { return mrs_m3_backbone_reset((mrs_m3_backbone *)self); }
 size_t m3_hook_state_bytes(void *self) {
     size_t n[4];
@@ -1421,7 +1426,7 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     if (!out || !bb || !embed) return fail(MRS_E_NULL, "mrs_lm3_create: null pointer");
     LmHooks h = {};
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
-    h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = nullptr;
+    h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = bb->temporal_t;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
     h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check; h.go_on_chain = m3_hook_go_on_chain;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");

@@ -36,6 +36,6 @@ __host__ __device__ inline LayerBlock layer_block(int dm, int di, int cols, int 
 // The row-order step (resident_m3_row.hip): the kernel chain's sums, term by term, for one row.  d_model = 256 KI.
 bool resident_m3_row_ok(const ResidentM3Args &a, int dtype);
 size_t resident_m3_row_lds(const ResidentM3Args &a);
-int launch_resident_m3_row(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev);
+int launch_resident_m3_row(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows);
 
 }  // namespace mrs

@@ -40,7 +40,7 @@ template <int KI> struct RowOrder {
 };
 
 template <typename T, int KI>
-__global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const ResidentM3Args *args) {
+__global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const ResidentM3Args *args, TokenRows rows) {
     using S = RowOrder<KI>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ int state;   // kRollCall, 0, or a ResidentFault
@@ -82,21 +82,22 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const Resi
     // layer 0's operand and sum of squares: 256 threads, as prenorm_rows_kernel
     float res = 0.0f;   // the residual stream: column o0 + wave, in every lane of the wave
     const int ow = min(wave, oc - 1);
-    {
-        const float *in = a->input, *nw = a->norm_w;
+    with_input_row<T>(a->input, rows, 0, dm, [&](auto in, bool taken) {
+        const float *nw = a->norm_w;
         if (wave < 4) {
             float ss = 0.0f;
 #pragma unroll
             for (int k = 0; k < KI; k++) {
-                const float v = in[tid + 256 * k];
+                const float v = in(tid + 256 * k);
                 ss = fmaf(v, v, ss);
                 Store<T>::st(xs + tid + 256 * k, v * nw[tid + 256 * k]);
             }
             ss = butterfly64(ss);
             if (lane == 0) pre[wave] = ss;
         }
-        res = in[o0 + ow];
-    }
+        res = in(o0 + ow);
+        if (taken && lane == 0 && wave < oc) a->input[o0 + wave] = res;
+    });
     lds_barrier();
     const float inv0 = inv_rms(pre[0] + pre[1] + pre[2] + pre[3], dm, a->eps);   // later row scales: from the tiles' sums
 
@@ -274,7 +275,11 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const Resi
             q[w] = butterfly64(ss);
         }
         const float inv = inv_rms(q[0] + q[1] + q[2] + q[3], dm, a->eps);
-        if (lane == 0) a->temporal[o0 + wave] = lost ? __uint_as_float(0x7fc00000u) : res * inv * a->norm_f[o0 + wave];
+        if (lane == 0) {
+            const float o = lost ? __uint_as_float(0x7fc00000u) : res * inv * a->norm_f[o0 + wave];
+            a->temporal[o0 + wave] = o;
+            Store<T>::st((T *)a->temporal_t + o0 + wave, o);
+        }
     }
     if (tid == 0) {
         if (state == kStepLost) {
@@ -285,18 +290,18 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const Resi
     }
 }
 
-template <typename T, int KI> int launch_t(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev) {
+template <typename T, int KI> int launch_t(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows) {
     static const hipError_t attr = hipFuncSetAttribute((const void *)resident_m3_row_kernel<T, KI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResLdsMax);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "resident step: LDS size: %s", hipGetErrorString(attr));
-    hipLaunchKernelGGL((resident_m3_row_kernel<T, KI>), dim3((unsigned)a.G), dim3(kResThreads), resident_m3_row_lds(a), st, dev);
+    hipLaunchKernelGGL((resident_m3_row_kernel<T, KI>), dim3((unsigned)a.G), dim3(kResThreads), resident_m3_row_lds(a), st, dev, rows);
     return check_launch("resident_m3_row_kernel");
 }
-template <typename T> int launch(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev) {
+template <typename T> int launch(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows) {
     switch (a.dm / 256) {
-    case 1: return launch_t<T, 1>(st, a, dev);
-    case 2: return launch_t<T, 2>(st, a, dev);
-    case 3: return launch_t<T, 3>(st, a, dev);
-    default: return launch_t<T, 4>(st, a, dev);
+    case 1: return launch_t<T, 1>(st, a, dev, rows);
+    case 2: return launch_t<T, 2>(st, a, dev, rows);
+    case 3: return launch_t<T, 3>(st, a, dev, rows);
+    default: return launch_t<T, 4>(st, a, dev, rows);
     }
 }
 
@@ -316,9 +321,9 @@ size_t resident_m3_row_lds(const ResidentM3Args &a) {
     }
 }
 
-int launch_resident_m3_row(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev) {
+int launch_resident_m3_row(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows) {
     if (!resident_m3_row_ok(a, dtype) || a.oc > kComputeWaves || !a.norm_rows) return fail(MRS_E_SHAPE, "resident Mamba-3 step: shape outside the row-order route");
-    return dtype == MRS_BF16 ? launch<bf16_t>(st, a, dev) : launch<f16_t>(st, a, dev);
+    return dtype == MRS_BF16 ? launch<bf16_t>(st, a, dev, rows) : launch<f16_t>(st, a, dev, rows);
 }
 
 }  // namespace mrs

@@ -38,7 +38,7 @@ __host__ __device__ inline ResLds res_lds(int dm, int di, int cols, int oc, int 
 }
 
 template <typename T>
-__global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const ResidentM3Args *args) {
+__global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const ResidentM3Args *args, TokenRows rows) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ int state;   // kRollCall, 0, or a ResidentFault
     const auto state_now = [] { return __hip_atomic_load(&state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
@@ -80,15 +80,18 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
     float res0 = 0.0f, res1 = 0.0f;
     const bool own = tid < (oc >> 1);
     float ss = 0.0f;
-    {
-        const float *in = a->input + (size_t)b * dm, *nw = a->norm_w;
+    with_input_row<T>(a->input, rows, b, dm, [&](auto in, bool taken) {
+        const float *nw = a->norm_w;
         for (int i = tid; i < dm; i += kCompute) {
-            const float v = in[i];
+            const float v = in(i);
             ss = fmaf(v, v, ss);
             Store<T>::st(xs + i, v * nw[i]);
         }
-        if (own) { res0 = in[o0 + 2 * tid]; res1 = in[o0 + 2 * tid + 1]; }
-    }
+        if (own) {
+            res0 = in(o0 + 2 * tid); res1 = in(o0 + 2 * tid + 1);
+            if (taken) *reinterpret_cast<float2 *>(a->input + (size_t)b * dm + o0 + 2 * tid) = make_float2(res0, res1);
+        }
+    });
     ss = wave_sum_last(ss);
     if (lane == 63) pre2[wave] = ss;
     lds_barrier();
@@ -213,7 +216,9 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const int n = o0 + 2 * tid + k;
-            a->temporal[(size_t)b * dm + n] = lost ? __uint_as_float(0x7fc00000u) : (k ? res1 : res0) * inv * a->norm_f[n];
+            const float o = lost ? __uint_as_float(0x7fc00000u) : (k ? res1 : res0) * inv * a->norm_f[n];
+            a->temporal[(size_t)b * dm + n] = o;
+            Store<T>::st((T *)a->temporal_t + (size_t)b * dm + n, o);
         }
     }
     if (tid == 0) {
@@ -308,20 +313,20 @@ int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, 
 }
 
 template <typename T>
-static int launch_resident_m3_t(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev) {
+static int launch_resident_m3_t(hipStream_t st, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows) {
     static const hipError_t attr = hipFuncSetAttribute((const void *)resident_m3_step_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResLdsMax);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "resident step: LDS size: %s", hipGetErrorString(attr));
     hipLaunchKernelGGL((resident_m3_step_kernel<T>), dim3((unsigned)(a.G * a.batch)), dim3(kResThreads),
-                       (size_t)res_lds(a.dm, a.di, 2 * a.nc + a.ex, a.oc, a.ds).total, st, dev);
+                       (size_t)res_lds(a.dm, a.di, 2 * a.nc + a.ex, a.oc, a.ds).total, st, dev, rows);
     return check_launch("resident_m3_step_kernel");
 }
 
-int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev) {
+int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows) {
     if (!shape_ok(a, dtype) || !plan_ok(a) || a.batch < 1 || a.G * a.batch > kRollMax || a.n_layers < 1 || !a.weights || !a.norm_w || !a.norm_f || !a.input || !a.xch || !a.epoch ||
-        !a.roll || !a.broken || !a.temporal || !a.ssm || !a.kst || !a.vst || !a.angle || !dev)
+        !a.roll || !a.broken || !a.temporal || !a.temporal_t || !a.ssm || !a.kst || !a.vst || !a.angle || !dev)
         return fail(MRS_E_SHAPE, "resident Mamba-3 step: shape outside the route (d_model=%d d_inner=%d d_state=%d workgroups=%d)", a.dm, a.di, a.ds, a.G);
-    if (a.row_order) return launch_resident_m3_row(st, dtype, a, dev);
-    return dtype == MRS_BF16 ? launch_resident_m3_t<bf16_t>(st, a, dev) : launch_resident_m3_t<f16_t>(st, a, dev);
+    if (a.row_order) return launch_resident_m3_row(st, dtype, a, dev, rows);
+    return dtype == MRS_BF16 ? launch_resident_m3_t<bf16_t>(st, a, dev, rows) : launch_resident_m3_t<f16_t>(st, a, dev, rows);
 }
 
 }  // namespace mrs

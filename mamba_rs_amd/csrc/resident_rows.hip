@@ -233,7 +233,7 @@ __device__ __forceinline__ float quarters_sum(float v) {
 }
 
 template <typename T, int KI>
-__global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const ResidentArgs *args) {
+__global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const ResidentArgs *args, TokenRows rows) {
     using S = RowsShape<KI>;
     constexpr int dm = S::dm, di = S::di, nc = S::nc, oc = S::oc, G = S::G, dr = S::dr, KO = 2 * KI;
     constexpr SmallBlock sb = S::sb;
@@ -281,25 +281,32 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
     float4 cwin, hv[4];
     float res0 = 0.0f, res1 = 0.0f;
     {
-        const float *in = a->input + (size_t)r0 * dm, *nw = a->norm_w;
+        const float *nw = a->norm_w;
         float sq = 0.0f;
-#pragma unroll
-        for (int s = 0; s < KI; s++) {
+        const auto operand = [&](int s, auto in) {
             const int k = (wave + kComputeWaves * s) * 32 + (lane >> 4) * 8;
-            const float *p = in + (size_t)min(lane & 15, nr - 1) * dm + k;
             T v[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                sq = fmaf(p[j], p[j], sq);
-                v[j] = (T)(p[j] * nw[k + j]);
+                const float p = in(k + j);
+                sq = fmaf(p, p, sq);
+                v[j] = (T)(p * nw[k + j]);
             }
             fa[s] = __builtin_bit_cast(uint4, v);
             asm volatile("" : "+v"(fa[s].x), "+v"(fa[s].y), "+v"(fa[s].z), "+v"(fa[s].w)::"memory");   // a k-step's loads at a time
-        }
+        };
+        with_input_row<T>(a->input, rows, r0 + min(lane & 15, nr - 1), dm, [&](auto in, bool) {
+#pragma unroll
+            for (int s = 0; s < KI; s++) operand(s, in);
+        });
         sq = quarters_sum(sq);
         if (tid < 2) put[tid] = 0;
         if (lane < kRows) sqs[wave * kRows + lane] = sq;
-        if (own) { res0 = in[(size_t)orow * dm + o0 + 2 * op]; res1 = in[(size_t)orow * dm + o0 + 2 * op + 1]; }
+        if (own)
+            with_input_row<T>(a->input, rows, r0 + orow, dm, [&](auto in, bool taken) {
+                res0 = in(o0 + 2 * op); res1 = in(o0 + 2 * op + 1);
+                if (taken) *reinterpret_cast<float2 *>(a->input + (size_t)(r0 + orow) * dm + o0 + 2 * op) = make_float2(res0, res1);
+            });
         for (int i = tid; i < kRows * S::xdtp; i += kCompute) xdt[i] = (T)0.0f;   // (what lies behind dt_rank stays zero)
     }
     lds_barrier();
@@ -588,14 +595,14 @@ int launch_resident_rows_pack(hipStream_t st, const ResidentArgs &a, void *dst, 
 }
 
 template <typename T, int KI>
-static int launch_rows_k(hipStream_t st, const ResidentArgs &a, const ResidentArgs *dev) {
+static int launch_rows_k(hipStream_t st, const ResidentArgs &a, const ResidentArgs *dev, const TokenRows &rows) {
     static const hipError_t attr = hipFuncSetAttribute((const void *)resident_rows_kernel<T, KI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResLdsMax);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "resident step: LDS size: %s", hipGetErrorString(attr));
-    hipLaunchKernelGGL((resident_rows_kernel<T, KI>), dim3((unsigned)(RowsShape<KI>::G * a.groups)), dim3(kResThreads), (size_t)RowsShape<KI>::lds, st, dev);
+    hipLaunchKernelGGL((resident_rows_kernel<T, KI>), dim3((unsigned)(RowsShape<KI>::G * a.groups)), dim3(kResThreads), (size_t)RowsShape<KI>::lds, st, dev, rows);
     return check_launch("resident_rows_kernel");
 }
 
-int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev) {
+int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const ResidentArgs *dev, const TokenRows &rows) {
     ResidentArgs plan = a;
     const bool ok = resident_rows_plan(plan, dtype) && plan.G == a.G && a.groups >= 1 && a.groups <= a.batch && a.groups * a.G <= kRollMax &&
                     a.rows == (a.batch + a.groups - 1) / a.groups && a.rows <= kRows && a.xch_stride == plan.xch_stride && a.n_layers >= 1 && a.weights && a.norm_w && a.input &&
@@ -603,7 +610,7 @@ int launch_resident_rows(hipStream_t st, int dtype, const ResidentArgs &a, const
     if (!ok) return fail(MRS_E_SHAPE, "resident step: shape outside the route (d_model=%d d_inner=%d d_state=%d workgroups=%d rows=%d)", a.dm, a.di, a.ds, a.G, a.rows);
     return rows_shape(a, [&](auto s) {
         constexpr int KI = decltype(s)::dm / 256;
-        return dtype == MRS_BF16 ? launch_rows_k<bf16_t, KI>(st, a, dev) : launch_rows_k<f16_t, KI>(st, a, dev);
+        return dtype == MRS_BF16 ? launch_rows_k<bf16_t, KI>(st, a, dev, rows) : launch_rows_k<f16_t, KI>(st, a, dev, rows);
     }, MRS_E_SHAPE);
 }
 
