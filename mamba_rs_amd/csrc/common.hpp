@@ -312,9 +312,22 @@ struct LmHooks {
 int launch_embed_gather(hipStream_t st, int dtype, float *out, const void *embed, const int *tokens, int64_t rows, int dm, int vocab,
                         const int *finished = nullptr);
 
-// sample_token for every active row (sampling.hip); all pointers device memory
+// A generation's bookkeeping (src/module/gpu_lm.rs:404-513)
+constexpr int kMaxEos = 16;
+struct GenSlots {            // per-slot arrays, [batch] each unless noted
+    int *prompt_off, *prompt_len, *prompt_pos, *finished, *active, *max_tokens, *n_eos, *eos /*[batch, kMaxEos]*/, *out_len, *sampled;
+    unsigned *seen;          // [batch, vocab] occurrences in the slot's seen list
+    int *n_running;          // [1] slots not finished after the latest step
+};
+struct GenDyn {              // buffers that grow between calls; read through device memory so a captured step stays valid
+    const int *prompts;
+    int *out;
+    int out_stride;
+};
+struct GenAdvance { GenSlots g; const GenDyn *dyn; int *last_token; };   // dyn null: no slots to advance
+// sample_token for every active row (sampling.hip), and with `adv` the step of every row's slot behind it; all pointers device memory
 int launch_sample_rows(hipStream_t st, int *tokens, const float *logits, float *work, int64_t ld, int rows, int vocab,
-                       const mrs_sampler *samplers, const unsigned *seen, unsigned long long *rng, const int *active);
+                       const mrs_sampler *samplers, const unsigned *seen, unsigned long long *rng, const int *active, const GenAdvance &adv = {});
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }

@@ -156,18 +156,6 @@ template <int V> __global__ __launch_bounds__(256) void argmax_kernel(int *__res
 }
 
 // ---- generate_batch bookkeeping on the device (src/module/gpu_lm.rs:404-513) ------------------------------
-constexpr int kMaxEos = 16;
-struct GenSlots {            // per-slot arrays, [batch] each unless noted
-    int *prompt_off, *prompt_len, *prompt_pos, *finished, *active, *max_tokens, *n_eos, *eos /*[batch, kMaxEos]*/, *out_len, *sampled;
-    unsigned *seen;          // [batch, vocab] occurrences in the slot's seen list
-    int *n_running;          // [1] slots not finished after the latest step
-};
-struct GenDyn {              // buffers that grow between calls; read through device memory so a captured step stays valid
-    const int *prompts;
-    int *out;
-    int out_stride;
-};
-
 // Seen list of generate_streaming starts as the prompt (gpu_lm.rs:364).
 __global__ __launch_bounds__(256) void gen_seen_prompt_kernel(GenSlots g, const GenDyn *__restrict__ dyn, int batch, int vocab) {
     const int slot = blockIdx.y;
@@ -186,41 +174,6 @@ __global__ __launch_bounds__(256) void gen_prefix_kernel(float *__restrict__ row
     const int tok = min(max(dyn->prompts[g.prompt_off[slot] + t0 + t], 0), vocab - 1);   // (clamped as embed_gather_kernel does)
     float *out = rows + ((int64_t)slot * gridDim.x + t) * dm;
     for (int i = threadIdx.x; i < dm; i += 256) out[i] = Store<T>::ld(embed + (int64_t)tok * dm + i);
-}
-
-// After a step: slots still inside their prompt take the next prompt token; slots past it take the sampled token,
-// unless it is an EOS id or max_tokens are out already -- then the slot is finished (gpu_lm.rs:494-511).  Also
-// marks which slots sample after the next step (prompt consumed, not finished) and counts the running ones.
-__global__ __launch_bounds__(1024) void gen_advance_kernel(GenSlots g, const GenDyn *__restrict__ dyn, int *__restrict__ last_token,
-                                                           int batch, int vocab) {
-    __shared__ int running;
-    if (threadIdx.x == 0) running = 0;
-    __syncthreads();
-    for (int i = threadIdx.x; i < batch; i += blockDim.x) {
-        if (!g.finished[i]) {
-            if (g.prompt_pos[i] < g.prompt_len[i]) {
-                last_token[i] = dyn->prompts[g.prompt_off[i] + g.prompt_pos[i]];
-                g.prompt_pos[i] += 1;
-            } else {
-                const int next = g.sampled[i];
-                bool stop = g.out_len[i] >= g.max_tokens[i];
-                for (int e = 0; e < g.n_eos[i]; e++) stop = stop || g.eos[i * kMaxEos + e] == next;
-                if (stop) {
-                    g.finished[i] = 1;
-                } else {
-                    dyn->out[(int64_t)i * dyn->out_stride + g.out_len[i]] = next;
-                    g.out_len[i] += 1;
-                    last_token[i] = next;
-                    if (next >= 0 && next < vocab) g.seen[(int64_t)i * vocab + next] += 1u;
-                }
-            }
-        }
-        const int fin = g.finished[i];
-        g.active[i] = !fin && g.prompt_pos[i] >= g.prompt_len[i];
-        if (!fin) atomicAdd(&running, 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) *g.n_running = running;
 }
 
 }  // namespace mrs
@@ -1477,10 +1430,8 @@ static int gen_alloc(mrs_lm *lm) {
 // sample the active slots from the current logits, then advance every slot
 static int gen_pick(mrs_lm *lm) {
     hipStream_t st = lm->eng.stream;
-    MRS_TRY(launch_sample_rows(st, lm->gen.sampled, lm->logits, lm->gen_work, lm->vocab_padded, lm->batch, lm->vocab, lm->gen_samplers,
-                               lm->gen.seen, lm->gen_rng, lm->gen.active));
-    hipLaunchKernelGGL(gen_advance_kernel, dim3(1), dim3(1024), 0, st, lm->gen, lm->gen_dyn, lm->tokens, lm->batch, lm->vocab);
-    return check_launch("gen_advance_kernel");
+    return launch_sample_rows(st, lm->gen.sampled, lm->logits, lm->gen_work, lm->vocab_padded, lm->batch, lm->vocab, lm->gen_samplers,
+                              lm->gen.seen, lm->gen_rng, lm->gen.active, {lm->gen, lm->gen_dyn, lm->tokens});
 }
 
 // gather the slots' current tokens (zeros for finished slots), one backbone step, head

@@ -39,11 +39,12 @@ struct SampShared {
     unsigned long long res_ge, res_gt;
     uint32_t res_key;
     alignas(16) uint32_t group_max[kGroups];
-    struct { float x; int i; } cand[kFinish];          // the short route's candidates, in no order
+    alignas(16) unsigned long long cand[kFinish];      // the short route's candidates, in no order: ordered key, and below it the index, the lower the larger
+    alignas(16) uint32_t cand_i[kFinish];              // indices of those that stay, the others all ones
     float kept_x[kShortK];                             // the top-k survivors in index order
     int kept_i[kShortK];
-    uint32_t kept_key[kShortK];                        // bit patterns of their weights
-    unsigned long long kept_mass[kShortK];
+    alignas(16) uint32_t kept_key[kShortK];            // bit patterns of their weights
+    alignas(16) unsigned long long kept_mass[kShortK];
 };
 
 template <typename T> __device__ __forceinline__ T wave_sum(T v) {
@@ -139,6 +140,20 @@ struct Row {
 };
 
 struct SearchOut { uint32_t key; unsigned long long ge, gt, thr; };
+
+// A row held in registers, walked in the same order: kSampThreads * kHeld pieces of four entries.
+constexpr int kHeld = 16;
+struct HeldRow {
+    float4 v[kHeld];
+    int n4;
+    template <typename F> __device__ __forceinline__ void each(F f) {
+#pragma unroll
+        for (int k = 0; k < kHeld; k++) {
+            const int q = threadIdx.x + k * kSampThreads;
+            if (q < n4) { f(4 * q, v[k].x); f(4 * q + 1, v[k].y); f(4 * q + 2, v[k].z); f(4 * q + 3, v[k].w); }
+        }
+    }
+};
 
 // Weight in 2^-32 units (saturating at 1): masses are summed as integers, so the totals do not depend on the order in
 // which the lanes' additions land.
@@ -361,8 +376,10 @@ template <typename W> __device__ int ordered_find(const Row &row, W w, double ta
 // entry that can matter and all that follows walks a list of that length.  It does not fit for rows whose large values crowd
 // into few groups (an ascending vocabulary) or with long runs of equal values.
 // Row passes are what a draw costs (about 7 us each at 50280 entries, one workgroup per row): eight with both filters through the
-// searches, two through here.
-__device__ bool short_top_k(const Row &row, uint32_t group_key, int k, SampShared &sh) {
+// searches, one and a walk over registers through here; then the ranks, whose lists are read sixteen bytes at a time, several at once (read one entry after
+// the other, each behind the last one's way through LDS, and with a second pass over memory the draw took 30.6 us at 13 rows, top-k 50
+// and top-p, as it takes 21; the slots' step behind it was a launch of 4.6).
+template <typename R> __device__ __forceinline__ bool short_top_k(R &row, uint32_t group_key, int k, SampShared &sh) {
     const int tid = threadIdx.x;
     group_key = max(group_key, (uint32_t)__shfl_xor((int)group_key, 1, kWave));
     group_key = max(group_key, (uint32_t)__shfl_xor((int)group_key, 2, kWave));
@@ -383,34 +400,46 @@ __device__ bool short_top_k(const Row &row, uint32_t group_key, int k, SampShare
     __syncthreads();
     const uint32_t floor_key = sh.res_key;
     row.each([&](int i, float x) {
-        if (ordered_key(x) >= floor_key) {
+        const uint32_t key = ordered_key(x);
+        if (key >= floor_key) {
             const int slot = atomicAdd(&sh.n_list, 1);
-            if (slot < kFinish) { sh.cand[slot].x = x; sh.cand[slot].i = i; }
+            if (slot < kFinish) sh.cand[slot] = (unsigned long long)key << 32 | (uint32_t)~i;
         }
     });
     __syncthreads();
-    const int n = sh.n_list;
+    const int n = sh.n_list, n8 = (n + 7) & ~7;
     if (n < k || n > kFinish) return false;   // (uniform)
+    if (tid >= n && tid < n8) sh.cand[tid] = 0;   // below all others
+    __syncthreads();
     bool keep = false;
-    uint32_t key = 0;
-    int idx = 0;
+    unsigned long long mine = 0;
     if (tid < n) {
-        key = ordered_key(sh.cand[tid].x);
-        idx = sh.cand[tid].i;
+        mine = sh.cand[tid];
         int rank = 0;
-        for (int u = 0; u < n; u++) {
-            const uint32_t ku = ordered_key(sh.cand[u].x);
-            rank += ku > key || (ku == key && sh.cand[u].i < idx);
+        for (int u = 0; u < n8; u += 8) {
+            ulonglong2 o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = *reinterpret_cast<const ulonglong2 *>(&sh.cand[u + 2 * j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) rank += (o[j].x > mine) + (o[j].y > mine);
         }
         keep = rank < k;
-        sh.list[tid] = keep ? (uint32_t)idx : 0xffffffffu;
     }
+    const uint32_t idx = ~(uint32_t)mine;
+    if (tid < n8) sh.cand_i[tid] = keep ? idx : 0xffffffffu;
     __syncthreads();
     if (keep) {
         int pos = 0;
-        for (int u = 0; u < n; u++) pos += sh.list[u] < (uint32_t)idx;
-        sh.kept_x[pos] = sh.cand[tid].x;
-        sh.kept_i[pos] = idx;
+        for (int u = 0; u < n8; u += 8) {
+            uint4 o[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) o[j] = *reinterpret_cast<const uint4 *>(&sh.cand_i[u + 4 * j]);
+#pragma unroll
+            for (int j = 0; j < 2; j++) pos += (o[j].x < idx) + (o[j].y < idx) + (o[j].z < idx) + (o[j].w < idx);
+        }
+        const uint32_t key = (uint32_t)(mine >> 32);
+        sh.kept_x[pos] = __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);   // ordered_key, turned back
+        sh.kept_i[pos] = (int)idx;
     }
     __syncthreads();
     return true;
@@ -418,7 +447,7 @@ __device__ bool short_top_k(const Row &row, uint32_t group_key, int k, SampShare
 
 // Softmax, top-p, min-p and the draw over the m <= kShortK survivors that short_top_k left, by the rules of the general route below: the
 // same integer masses, the running sums in f64.
-__device__ int short_draw(int m, int vocab, float xmax, const mrs_sampler &sp, bool topp_on, SampShared &sh) {
+__device__ __forceinline__ int short_draw(int m, int vocab, float xmax, const mrs_sampler &sp, bool topp_on, SampShared &sh) {
     const int tid = threadIdx.x;
     float e = 0.0f;
     uint32_t key = 0;
@@ -427,18 +456,26 @@ __device__ int short_draw(int m, int vocab, float xmax, const mrs_sampler &sp, b
         key = __float_as_uint(e);
         sh.kept_key[tid] = key;
         sh.kept_mass[tid] = fixed_weight(key);
+    } else if (tid < kShortK) {   // (a survivor's weight may be 0 as well, but none of these lies before one)
+        sh.kept_key[tid] = 0;
+        sh.kept_mass[tid] = 0;
     }
     __syncthreads();
     if (tid < m && topp_on) {
         unsigned long long total = 0, above = 0, equal = 0;
         int ties_before = 0;
-        for (int u = 0; u < m; u++) {
-            const uint32_t ku = sh.kept_key[u];
-            const unsigned long long c = sh.kept_mass[u];
-            total += c;
-            above += ku > key ? c : 0ull;
-            equal += ku == key ? c : 0ull;
-            ties_before += ku == key && u < tid;
+        for (int u0 = 0; u0 < m; u0 += 4) {
+            const uint4 k4 = *reinterpret_cast<const uint4 *>(&sh.kept_key[u0]);
+            const ulonglong2 c2[2] = {*reinterpret_cast<const ulonglong2 *>(&sh.kept_mass[u0]), *reinterpret_cast<const ulonglong2 *>(&sh.kept_mass[u0 + 2])};
+            const uint32_t ks[4] = {k4.x, k4.y, k4.z, k4.w};
+            const unsigned long long cs[4] = {c2[0].x, c2[0].y, c2[1].x, c2[1].y};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                total += cs[j];
+                above += ks[j] > key ? cs[j] : 0ull;
+                equal += ks[j] == key ? cs[j] : 0ull;
+                ties_before += ks[j] == key && u0 + j < tid;
+            }
         }
         const unsigned long long thr = (unsigned long long)((double)sp.top_p * (double)total);
         // an entry goes if what lies above it crosses the goal already, or its equals of lower index take the sum across
@@ -476,6 +513,36 @@ __device__ int short_draw(int m, int vocab, float xmax, const mrs_sampler &sp, b
 
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
 
+// After a step: a slot still inside its prompt takes the next prompt token; one past it takes the sampled token, unless it is an EOS id or max_tokens
+// are out already -- then the slot is finished (gpu_lm.rs:494-511).  Also marks whether the slot samples after the next step (prompt consumed, not
+// finished) and keeps the count of those that run.  By one thread of the row's workgroup (a launch of its own: 4.6 us).
+__device__ __forceinline__ void advance_slot(const GenAdvance &adv, int i, int next, int vocab) {
+    const GenSlots &g = adv.g;
+    bool fin = g.finished[i];
+    int pos = g.prompt_pos[i];
+    const int len = g.prompt_len[i];
+    if (!fin) {
+        if (pos < len) {
+            adv.last_token[i] = adv.dyn->prompts[g.prompt_off[i] + pos];
+            g.prompt_pos[i] = ++pos;
+        } else {
+            const int n = g.out_len[i];
+            fin = n >= g.max_tokens[i];
+            for (int e = 0; e < g.n_eos[i]; e++) fin = fin || g.eos[i * kMaxEos + e] == next;
+            if (fin) {
+                g.finished[i] = 1;
+                atomicSub(g.n_running, 1);
+            } else {
+                adv.dyn->out[(int64_t)i * adv.dyn->out_stride + n] = next;
+                g.out_len[i] = n + 1;
+                adv.last_token[i] = next;
+                if (next >= 0 && next < vocab) g.seen[(int64_t)i * vocab + next] += 1u;
+            }
+        }
+    }
+    g.active[i] = !fin && pos >= len;
+}
+
 // logits [rows, ld] f32 are read only; `work` [rows, ld] receives the penalised logits of rows with a penalty.  seen [rows, vocab] counts how often a token sits in the row's seen list (the penalty is applied once per
 // occurrence, sample.rs:100-109).  rng [rows, 4] advances by one draw per sampled row (none on the greedy branch).
 // Rows with active[row] == 0 are left alone.
@@ -484,10 +551,19 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
                                                                    const mrs_sampler *__restrict__ samplers,
                                                                    const unsigned *__restrict__ seen,
                                                                    unsigned long long *__restrict__ rng,
-                                                                   const int *__restrict__ active) {
+                                                                   const int *__restrict__ active, GenAdvance adv) {
     __shared__ SampShared sh;
     const int rowi = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (active && !active[rowi]) return;
+    const auto done = [&](int tok, bool sampled) {
+        if (tid != 0) return;
+        if (sampled) tokens[rowi] = tok;
+        if (adv.dyn) advance_slot(adv, rowi, tok, vocab);
+    };
+    if (active) {
+        const bool on = active[rowi];
+        __syncthreads();   // everybody has looked before the slot moves on
+        if (!on) { done(0, false); return; }
+    }
     const mrs_sampler sp = samplers[rowi];
     const float *lrow = logits + (int64_t)rowi * ld;
     const float pen = sp.repetition_penalty;
@@ -502,7 +578,19 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
     float best = -INFINITY;
     int bi = 0;
     uint32_t top_key = 0;   // the largest ordered key this thread meets
-    if (pen_on) {   // the penalised (and scaled) row goes to `work`; later passes read it from there
+    const bool topk_on = sp.top_k > 0 && sp.top_k < vocab, short_on = topk_on && !greedy && sp.top_k <= kShortK;
+    HeldRow held = {};
+    held.n4 = vocab >> 2;
+    const bool hold = short_on && vec && !pen_on && vocab % 4 == 0 && held.n4 <= kHeld * kSampThreads;   // (the penalty's counts would want registers too)
+    if (hold) {
+        row.scale = inv_t;
+#pragma unroll
+        for (int k = 0; k < kHeld; k++) held.v[k] = row.at4(4 * min(tid + k * kSampThreads, held.n4 - 1));
+        held.each([&](int i, float x) {
+            if (x >= best) { best = x; bi = i; }
+            top_key = max(top_key, ordered_key(x));
+        });
+    } else if (pen_on) {   // the penalised (and scaled) row goes to `work`; later passes read it from there
         float *wrow = work + (int64_t)rowi * ld;
         const unsigned *srow = seen + (int64_t)rowi * vocab;
         row.each([&](int i, float x) {
@@ -536,7 +624,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
         if (ov > best || (ov == best && oi > bi)) { best = ov; bi = oi; }
     }
     if (greedy) {
-        if (tid == 0) tokens[rowi] = bi;
+        done(bi, true);
         return;
     }
     const float xmax = best;
@@ -553,13 +641,11 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
     }
 
     // top-k: key of the k-th largest value, then how many entries equal to it stay (lowest indices first)
-    const bool topk_on = sp.top_k > 0 && sp.top_k < vocab;
     const bool topp_on = isfinite(sp.top_p) && sp.top_p > 0.0f && sp.top_p < 1.0f;
-    if (topk_on && sp.top_k <= kShortK) {
+    if (short_on) {
         __syncthreads();   // sh.draw
-        if (short_top_k(row, top_key, sp.top_k, sh)) {
-            const int tok = short_draw(sp.top_k, vocab, xmax, sp, topp_on, sh);
-            if (tid == 0) tokens[rowi] = tok;
+        if (hold ? short_top_k(held, top_key, sp.top_k, sh) : short_top_k(row, top_key, sp.top_k, sh)) {
+            done(short_draw(sp.top_k, vocab, xmax, sp, topp_on, sh), true);
             return;
         }
         __syncthreads();
@@ -617,15 +703,14 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restri
 
     // first index whose running sum of kept weights exceeds draw x (their total)
     __syncthreads();   // sh.draw
-    const int tok = ordered_find(row, final_weight, (double)sh.draw, true, sh);
-    if (tid == 0) tokens[rowi] = tok;
+    done(ordered_find(row, final_weight, (double)sh.draw, true, sh), true);
 }
 
 int launch_sample_rows(hipStream_t st, int *tokens, const float *logits, float *work, int64_t ld, int rows, int vocab,
-                       const mrs_sampler *samplers, const unsigned *seen, unsigned long long *rng, const int *active) {
+                       const mrs_sampler *samplers, const unsigned *seen, unsigned long long *rng, const int *active, const GenAdvance &adv) {
     if (rows < 1 || vocab < 1 || ld < vocab) return fail(MRS_E_SHAPE, "sample: rows=%d vocab=%d ld=%lld", rows, vocab, (long long)ld);
     hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)rows), dim3(kSampThreads), 0, st, tokens, logits, work, ld, vocab, samplers,
-                       seen, rng, active);
+                       seen, rng, active, adv);
     return check_launch("sample_rows_kernel");
 }
 
