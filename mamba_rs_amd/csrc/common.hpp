@@ -259,6 +259,13 @@ bool resident_m3_plan(ResidentM3Args &a, int dtype);
 size_t resident_m3_layer_bytes(const ResidentM3Args &a);
 int launch_resident_m3_pack(hipStream_t st, const ResidentM3Args &a, void *dst, const ResidentM3Layer &w);
 int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, const ResidentM3Args *dev, const TokenRows &rows);
+// conv1d + SiLU over a sequence and x_proj behind it in one launch (conv_xproj.hip), d_conv 4: u [batch * T][di], xdbl [batch * T][xd] from x (rows x_stride apart) and
+// wp, the tiled copy of x_proj (launch_tile_weight); state as mrs_conv1d_seq_silu
+bool conv_xproj_ok(int dtype, const void *u, const void *xdbl, const float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
+                   int di, int dc, int xd);
+bool conv_xproj_wins(int batch, int T, int xd);
+int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
+                      int di, int xd);
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,
                             int64_t rows, int di, int dr);

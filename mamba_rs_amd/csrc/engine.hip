@@ -525,8 +525,11 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
                                               xb + es * (dr + ds), xd, z, 2 * di, 2, lw.a_neg, lw.D, B, di, ds));
             }
         } else {
-            MRS_TRY(mrs_conv1d_seq_silu(bb->stream, dt, s->u, conv, s->proj, 2 * di, lw.conv_w, lw.conv_b, B, T, di, dc));
-            if (own_xproj(lw, rows, xd)) {
+            const bool one = !prefix && conv_xproj_wins(B, T, xd) && conv_xproj_ok(dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, dc, xd);
+            if (one) MRS_TRY(launch_conv_xproj(bb->stream, dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, xd));
+            else MRS_TRY(mrs_conv1d_seq_silu(bb->stream, dt, s->u, conv, s->proj, 2 * di, lw.conv_w, lw.conv_b, B, T, di, dc));
+            if (one) {
+            } else if (own_xproj(lw, rows, xd)) {
                 SkinnyEpi xp = {};
                 xp.w_tiled = 1; xp.any_rows = 1;
                 MRS_TRY(launch_skinny_gemm(bb->stream, dt, s->xdbl, 0, xd, s->u, di, lw.x_proj_p, (int)rows, xd, di, xp));
