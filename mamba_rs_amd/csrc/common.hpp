@@ -82,7 +82,9 @@ int check_launch(const char *what);
 // StepFold: the step kernel forms the x_proj row itself from per-tile shares [n_tiles][rows][xd] f32 (summed in tile
 // order, rounded to the storage type); dt input at element 0, B at b_off, C at c_off of the row.
 // y_mt != 0: y is written in the tiled order of tiled_a_index (y_mt row tiles) instead of row-major.
-struct StepFold { const float *xpart; int n_tiles, rows, xd, b_off, c_off, y_mt; };
+// next (may be null): a weight that the launch behind streams, next_units pieces of next_bytes bytes, piece i by its workgroup i; the step kernel asks for its
+// lines (wide dt_rank only).
+struct StepFold { const float *xpart; int n_tiles, rows, xd, b_off, c_off, y_mt; const void *next; int next_units, next_bytes; };
 // Element (row, k) of an activation matrix stored as the matrix-core A operand in lane order -- [k-step][row tile][lane][8],
 // lane = row % 16 + 16 * ((k % 32) / 8), mt row tiles of 16 rows -- so that a wave's load of one operand piece is one
 // contiguous kilobyte (gemm_wide.hip reads it; the kernels that produce such a matrix write it this way).
@@ -142,6 +144,7 @@ struct SkinnyEpi {
 // the x_proj shares (SkinnyEpi::xw, ksplit).
 bool tiled_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, const void *Wp);
 size_t tiled_weight_elems(int N, int K);
+int tiled_gemm_unit(int N);   // column tiles of a workgroup
 int launch_tile_weight(hipStream_t st, int dtype, void *Wp, const void *Wt, int N, int K);
 int launch_tiled_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wp, int M,
                       int N, int K, const SkinnyEpi &ep);

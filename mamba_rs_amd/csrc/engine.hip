@@ -427,7 +427,11 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         // x_proj as a launch of its own: K split into slices when the step kernel can sum the shares
         const bool step_sums = xpart && xd <= 256 && lw.dt_t_step && di % (1024 / ds) == 0 && dr % 4 == 0 && (int64_t)nr * dr <= fuse_limit;
         const int ksplit = (!fold_x && step_sums && dt != MRS_F32) ? xproj_slices(nr, xd, di) : 1;
-        const StepFold fold = {xpart, fold_x ? di / 16 : ksplit, nr, xd, dr, dr + ds};
+        StepFold fold = {xpart, fold_x ? di / 16 : ksplit, nr, xd, dr, dr + ds, 0, nullptr, 0, 0};
+        if (a_mt && bb->wide && (int64_t)dm * di < (int64_t)1 << 30) {   // the step kernel asks for out_proj's lines while it waits for its states
+            const int unit = tiled_gemm_unit(dm);
+            fold.next = lw.out_proj_p; fold.next_units = (dm / 16 + unit - 1) / unit; fold.next_bytes = unit * (di / 32) * 1024;
+        }
         if (a_mt) {
             inp.a_tiled = 1; inp.w_tiled = 1;
             if (!fold_x) { inp.u_tiled = s->u_tiled; inp.u_tiled_mt = a_mt; }

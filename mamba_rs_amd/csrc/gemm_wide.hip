@@ -259,23 +259,33 @@ __global__ __launch_bounds__(256) void tile_weight_kernel(uint4 *__restrict__ Wp
     Wp[p] = col < N ? *reinterpret_cast<const uint4 *>(Wt + (int64_t)col * K + 32 * ks + 8 * (lane >> 4)) : make_uint4(0, 0, 0, 0);
 }
 
-template <typename T>
-int launch_tiled_t(hipStream_t st, void *C, int out_f32, int64_t ldc, const T *A, int64_t lda, const T *Wp, int M, int N, int K,
-                   const SkinnyEpi &ep) {
-    const int mt = (M + 15) / 16;
+}  // namespace
+
+// Column tiles per workgroup.  A compute unit keeps about 64 KB of requests in flight whatever runs on it (measured
+// with time stamps per workgroup: two workgroups sharing a unit each take twice as long), so a launch takes as long
+// as the unit with the most tiles: ceil(workgroups / 256) NT of them.  NT is the count of up to three that makes
+// this smallest, the larger on a tie (fewer workgroups read the activation operand).  in_proj of the 2.8b shape,
+// 640 tiles: 214 workgroups of three tiles -- with two tiles 320 workgroups, 64 units run two of them one after the
+// other while the rest of the chip idles (alone, with a plain store, 64 rows: 22.6 us against 15.4 us; 16 rows, one
+// tile: 12.9 against 11.4).
+int tiled_gemm_unit(int N) {
     const int ntiles = (N + 15) / 16;
-    // Column tiles per workgroup.  A compute unit keeps about 64 KB of requests in flight whatever runs on it (measured
-    // with time stamps per workgroup: two workgroups sharing a unit each take twice as long), so a launch takes as long
-    // as the unit with the most tiles: ceil(workgroups / 256) NT of them.  NT is the count of up to three that makes
-    // this smallest, the larger on a tie (fewer workgroups read the activation operand).  in_proj of the 2.8b shape,
-    // 640 tiles: 214 workgroups of three tiles -- with two tiles 320 workgroups, 64 units run two of them one after the
-    // other while the rest of the chip idles (alone, with a plain store, 64 rows: 22.6 us against 15.4 us; 16 rows, one
-    // tile: 12.9 against 11.4).
     int nt = 1, worst = 1 << 30;
     for (int c = 1; c <= 3; c++) {
         const int wgs = (ntiles + c - 1) / c, load = (wgs + 255) / 256 * c;
         if (load <= worst) { worst = load; nt = c; }
     }
+    return nt;
+}
+
+namespace {
+
+template <typename T>
+int launch_tiled_t(hipStream_t st, void *C, int out_f32, int64_t ldc, const T *A, int64_t lda, const T *Wp, int M, int N, int K,
+                   const SkinnyEpi &ep) {
+    const int mt = (M + 15) / 16;
+    const int ntiles = (N + 15) / 16;
+    const int nt = tiled_gemm_unit(N);
     // Streaming waves WS (they split K) and k-steps R each keeps requested ahead: WS R (NT + MT) KB in flight per
     // workgroup, 48 to 64 of them -- more only queues in front of the unit's memory pipeline (alone, with a plain
     // store, in_proj at 16 rows and one tile takes 13.7 us with one streaming wave and 18.3 us with eight).  In the

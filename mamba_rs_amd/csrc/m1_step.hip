@@ -114,6 +114,23 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(
             }
         }
     }
+    // Lines of the weight that the launch behind streams, a dword of each to LDS nobody reads, behind this kernel's own requests.  The units of one die (workgroup
+    // index modulo 8) ask for the pieces that units of the same die will read: their L2 then has them.  16 rows of the 2.8b shape: this kernel 8.4 -> 11.5 us,
+    // out_proj (26 MB) 10.2 -> 5.9; a step of eight layers at 3, 8, 16, 24, 32, 40 rows 280 / 306 / 334 / 391 / 401 / 458 -> 275 / 299 / 325 / 383 / 389 / 438 (small head); half of them here, or some in the x_proj launch in front, or in_proj's in
+    // out_proj's, gave back what they took.
+    if constexpr (FOLD && PRE == 12) {
+        if (fold.next) {
+            __shared__ alignas(16) char spare[256];
+            const int die = blockIdx.x & 7, mine = blockIdx.x >> 3, all = (gridDim.x - die + 7) >> 3;
+            const int units = (fold.next_units - die + 7) >> 3, per_unit = fold.next_bytes >> 7, lines = units * per_unit, each = (lines + all - 1) / all;
+            const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)spare);
+            for (int i = threadIdx.x; i < each; i += 256) {
+                const int line = min(mine * each + i, lines - 1), unit = line / per_unit;
+                const unsigned voff = (unsigned)(die + 8 * unit) * (unsigned)fold.next_bytes + (unsigned)(line - unit * per_unit) * 128u;
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(fold.next) : "m0", "memory");
+            }
+        }
+    }
     if constexpr (FOLD) {
         const int xd = fold.xd;
         if (fold_tg < fold_G) {
@@ -227,6 +244,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(
             Store<T>::st(y + (fold.y_mt ? tiled_a_index(b, d, fold.y_mt) : r), acc);
         }
     }
+    if constexpr (FOLD && PRE == 12) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // what was asked for is in before the workgroup's LDS is another's
 }
 
 // Any d_state (1..=256), one lane per (b,d), states streamed in order.
