@@ -155,6 +155,10 @@ int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc
 // The same for a prefill of thousands of rows (gemm_big.hip), C in the storage type
 bool big_gemm_ok(int dtype, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 bool big_gemm_wins(int64_t M, int N, int K);
+struct BigSplit { float *C2; int64_t ldc2; int n1; };   // columns from n1 on as f32 in C2
+bool big_gemm_split_ok(int dtype, const void *C, int64_t ldc, const BigSplit &split, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
+bool big_gemm_split_wins(int64_t M, int n1, int N, int K);   // against two products
+int launch_big_gemm_split(hipStream_t st, int dtype, void *C, int64_t ldc, const BigSplit &split, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 int launch_big_gemm(hipStream_t st, int dtype, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 int skinny_max_rows();   // rows the 16-bit matrix-core route takes (128; MRS_SKINNY_MAX_ROWS overrides)
 bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, const void *Wt);

@@ -41,9 +41,10 @@ template <typename T> __device__ __forceinline__ unsigned pack2(float a, float b
     return __builtin_bit_cast(unsigned, o);
 }
 
-template <typename T, int NB>
+// SPLIT: columns from n1 on (a multiple of 16) leave as f32 in C2, n1 columns to the left
+template <typename T, int NB, bool SPLIT>
 __global__ __launch_bounds__(kBigThreads, 2) void gemm_big_kernel(T *__restrict__ C, int64_t ldc, const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt,
-                                                                  int M, int N, int K, int mtiles, int ntiles) {
+                                                                  int M, int N, int K, int mtiles, int ntiles, BigSplit split) {
     constexpr int BN = 64 * NB, kA = kTileM * 128, kStage = kA + BN * 128;   // bytes of a k-step: A's rows, then Wt's
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(kBigThreads, 2) void gemm_big_kernel(T *__restrict_
     auto out_pair = [&](const v4f &x, const v4f &y, int row, int col) {
         unsigned x0 = pack2<T>(x[0], x[1]), x1 = pack2<T>(x[2], x[3]), y0 = pack2<T>(y[0], y[1]), y1 = pack2<T>(y[2], y[3]);
         swap16(x0, y0); swap16(x1, y1);
-        if (row < M && col < N) *reinterpret_cast<uint4 *>(C + (int64_t)row * ldc + col) = make_uint4(x0, x1, y0, y1);
+        if (row < M && col < (SPLIT ? split.n1 : N)) *reinterpret_cast<uint4 *>(C + (int64_t)row * ldc + col) = make_uint4(x0, x1, y0, y1);
     };
 #pragma unroll
     for (int a = 0; a < 2; a++)
@@ -157,17 +158,27 @@ __global__ __launch_bounds__(kBigThreads, 2) void gemm_big_kernel(T *__restrict_
             for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int j = 0; j + 1 < NB; j += 2) out_pair(acc[a][i][b][j], acc[a][i][b][j + 1], row + 16 * i, col + 16 * (j + (lg & 1)));
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < NB; j++) {
+                        const int c = n0 + b * 32 * NB + wn * 16 * NB + 16 * j;   // (the same for the wave)
+                        if (c >= split.n1 && row + 16 * i < M && c + 4 * lg < N)
+                            *reinterpret_cast<v4f *>(split.C2 + (int64_t)(row + 16 * i) * split.ldc2 + (c + 4 * lg - split.n1)) = acc[a][i][b][j];
+                    }
+            }
             if constexpr (NB & 1) out_pair(acc[a][0][b][NB - 1], acc[a][1][b][NB - 1], row + 16 * (lg & 1), col + 16 * (NB - 1));
         }
 }
 
-template <typename T, int NB>
-int launch_big(hipStream_t st, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int M, int N, int K) {
+template <typename T, int NB, bool SPLIT = false>
+int launch_big(hipStream_t st, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int M, int N, int K, const BigSplit &split = {}) {
     constexpr size_t lds = 2 * (kTileM + 64 * NB) * 128;
-    static const hipError_t attr = hipFuncSetAttribute((const void *)gemm_big_kernel<T, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)gemm_big_kernel<T, NB, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "big gemm: LDS size: %s", hipGetErrorString(attr));
     const int mt = (M + kTileM - 1) / kTileM, nt = (N + 64 * NB - 1) / (64 * NB);
-    hipLaunchKernelGGL((gemm_big_kernel<T, NB>), dim3((unsigned)(mt * nt)), dim3(kBigThreads), lds, st, (T *)C, ldc, (const T *)A, lda, (const T *)Wt, M, N, K, mt, nt);
+    hipLaunchKernelGGL((gemm_big_kernel<T, NB, SPLIT>), dim3((unsigned)(mt * nt)), dim3(kBigThreads), lds, st, (T *)C, ldc, (const T *)A, lda, (const T *)Wt, M, N, K, mt, nt, split);
     return check_launch("gemm_big_kernel");
 }
 
@@ -211,6 +222,29 @@ int launch_big_gemm(hipStream_t st, int dtype, void *C, int64_t ldc, const void 
         return fail(MRS_E_SHAPE, "big gemm: 16-bit storage, N %% 8 == 0, K %% 64 == 0 from 128 up, 16-byte aligned operands (M=%lld N=%d K=%d)", (long long)M, N, K);
     const int nb = big_plan(M, N, K).nb;
     return dtype == MRS_BF16 ? launch_big_type<bf16_t>(st, nb, C, ldc, A, lda, Wt, (int)M, N, K) : launch_big_type<f16_t>(st, nb, C, ldc, A, lda, Wt, (int)M, N, K);
+}
+
+bool big_gemm_split_ok(int dtype, const void *C, int64_t ldc, const BigSplit &split, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {
+    return big_gemm_ok(dtype, C, ldc, A, lda, Wt, M, split.n1, K) && split.n1 % 16 == 0 && N > split.n1 && N % 4 == 0 && split.ldc2 % 4 == 0 && split.ldc2 >= N - split.n1 &&
+           aligned(split.C2, 16) && (M + kTileM - 1) / kTileM * ((N + 191) / 192) < (int64_t)1 << 28;
+}
+
+static double split_us(int64_t M, int N, int K) { return (double)(((M + kTileM - 1) / kTileM * ((N + 319) / 320) + 255) / 256) * (K / kStepK * 1.75 + 5.5); }
+
+// One launch over all columns, 320 to a tile, against the first n1 on whichever kernel big_gemm_wins() names and the rest on the library's (5 us and what it moves at
+// 3 TB/s: 16384 x 216 x 768 18.4).  The rest often rides in rounds that the first columns leave partly empty.  Four layers of a bf16 Mamba-3 prefill, d_model 768
+// (3072 + 216 columns), two products / one: 2000 rows 487 / 492, 3000 540 / 533, 5000 723 / 678, 6000 792 / 845, 10000 1054 / 1011, 12000
+// 1185 / 1232, 16384 1249 / 1219.
+bool big_gemm_split_wins(int64_t M, int n1, int N, int K) {
+    const int64_t tiles = (M + 255) / 256 * ((n1 + 255) / 256);
+    const double first = big_gemm_wins(M, n1, K) ? big_plan(M, n1, K).us : 1.1 * (double)((tiles + 255) / 256) * (K / kStepK * 1.24 + 4.0);
+    return M >= 2560 && split_us(M, N, K) < first + 5.0 + (double)M * (2.0 * K + 4.0 * (N - n1)) / 3e6;
+}
+
+int launch_big_gemm_split(hipStream_t st, int dtype, void *C, int64_t ldc, const BigSplit &split, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {
+    if (!big_gemm_split_ok(dtype, C, ldc, split, A, lda, Wt, M, N, K))
+        return fail(MRS_E_SHAPE, "big gemm: columns %d of %d in f32 (M=%lld K=%d)", N - split.n1, N, (long long)M, K);
+    return dtype == MRS_BF16 ? launch_big<bf16_t, 5, true>(st, C, ldc, A, lda, Wt, (int)M, N, K, split) : launch_big<f16_t, 5, true>(st, C, ldc, A, lda, Wt, (int)M, N, K, split);
 }
 
 }  // namespace mrs

@@ -71,3 +71,29 @@ def test_long_prefill_on_the_large_tiles_follows_the_cpu_route(dm, B, T, dtype):
         hs, cs = s[0].reshape(di, 16), c[0].reshape(di, 3)
         assert cosine(ssm[b], hs) >= 0.999 and scaled_err(ssm[b], hs) < 5e-2, (b, cosine(ssm[b], hs), scaled_err(ssm[b], hs))
         assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
+
+
+@pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
+@pytest.mark.parametrize("dm,B,T", [
+    (128, 3, 867),    # 512 + 156 columns in three column tiles, the line between storage type and f32 inside the second; two k-steps; 41 rows in the last row tile
+    (256, 2, 1409),   # 1024 + 168, the line inside the fourth; the last row tile holds two rows
+])
+def test_long_mamba3_prefill_with_all_columns_of_in_proj_at_once_follows_the_cpu_route(dm, B, T, dtype):
+    """z and x in the storage type and the shared columns in f32 out of one launch; bounds as above."""
+    from mamba_rs_amd import GpuMamba3Backbone, Mamba3Config
+    from test_m3_engine_gpu import oracle_params as oracle_params3, perturbed
+    cfg = Mamba3Config(d_model=dm, d_state=64, expand=2, headdim=64, ngroups=1, n_layers=1, rope_fraction=0.5)
+    w = perturbed(cfg, dm, 3)
+    P = oracle_params3(w, cfg, dm, round_to=orc.BF16 if dtype == WeightDtype.BF16 else orc.F16)
+    x = (np.random.default_rng(T).standard_normal((B, T, dm)) * 0.5).astype(np.float32)
+    print(f"case m3 in_proj at once d_model={dm} rows={B * T} {dtype.name}", flush=True)
+    eng = GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    last = eng.prefill_sequence(x)
+    ssm = eng.download_state(0)[0]
+    eng.close()
+    for b in (0, B - 1):
+        st = P.zero_state()
+        for t in range(T):
+            want = orc.m3_backbone_step(P, x[b, t], st)
+        assert cosine(last[b], want) >= 0.999 and scaled_err(last[b], want) < 5e-2, (b, cosine(last[b], want), scaled_err(last[b], want))
+        assert cosine(ssm[b], st[0][0].reshape(ssm[b].shape)) >= 0.999, (b, cosine(ssm[b], st[0][0].reshape(ssm[b].shape)))
