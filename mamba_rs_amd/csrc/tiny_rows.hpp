@@ -82,5 +82,86 @@ inline int sweep_rounds(int K, int N) {
     return (kper + 15) / 16;
 }
 
+// ---- the streamed form: a layer's weights are on their way before the layer begins ----
+
+// A [K][N] product whose every thread owns four columns, 4 q .. 4 q + 3, of one of n slices of `rows` rows.
+template <int K, int N> struct Sweep {
+    static constexpr int most = kTinyThreads / (N / 4) < 32 ? kTinyThreads / (N / 4) : 32;
+    static constexpr int rows = ((K + most - 1) / most + 3) / 4 * 4, n = K / rows;
+    static_assert(N % 4 == 0 && K % rows == 0 && n * N <= kTinyPart, "whole slices");
+    int q, j;       // (a thread behind the last slice works on slice 0 and its sum goes nowhere)
+    bool on;
+    unsigned off;   // its first row's bytes
+    __device__ explicit Sweep(int tid) : q(tid % (N / 4)), j(tid / (N / 4)), on(j < n) {
+        if (!on) j = 0;
+        off = 4u * (j * rows * N + 4 * q);
+        asm volatile("" : "+v"(off));   // (kept as 32 bits beside a scalar base)
+    }
+};
+
+template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
+    return v + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_sum(float v) { return dpp_add<0x4e>(dpp_add<0xb1>(v)); }   // quad_perm [1,0,3,2], [2,3,0,1]
+__device__ __forceinline__ float oct_sum(float v) { return dpp_add<0x141>(quad_sum(v)); }          // row_half_mirror
+// sum over the wave, the same in every lane
+__device__ __forceinline__ float wave_sum(float v) {
+    v = dpp_add<0x140>(oct_sum(v));
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x142, 0xa, 0xf, false));   // row_bcast:15 into rows 1 and 3
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x143, 0xc, 0xf, false));   // row_bcast:31 into rows 2 and 3
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
+}
+
+// Memory operations stay on their side of this line.
+__device__ __forceinline__ void pin() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// ... and so do the sums so far: without this the compiler moves them to their one use, behind the requests into the registers they read.
+__device__ __forceinline__ void pin(float4 &v) {
+    asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)::"memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// One workgroup's LDS is handed on; loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+// A table entry by scalar loads, and reads through the pointers it holds: they come out of memory, so the compiler has to be told
+// that they point to global memory (a flat load would count as an LDS operation too, and every LDS wait would wait for it).
+template <typename T> __device__ __forceinline__ T table_entry(const T *p) {
+    constexpr int n = sizeof(T) / 8;
+    union { T t; uint64_t w[n]; } v = {};
+    const auto *q = (const __attribute__((address_space(4))) uint64_t *)(uintptr_t)p;
+#pragma unroll
+    for (int i = 0; i < n; i++) v.w[i] = q[i];
+    return v.t;
+}
+using gbytes = const __attribute__((address_space(1))) char *;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ gbytes global(const void *p) { return (gbytes)(uintptr_t)p; }
+__device__ __forceinline__ float ld1(gbytes p, unsigned off) { return *(const __attribute__((address_space(1))) float *)(p + off); }
+__device__ __forceinline__ float4 ld4(gbytes p, unsigned off) {
+    const f32x4 v = *(const __attribute__((address_space(1))) f32x4 *)(p + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+// A byte offset the compiler keeps as 32 bits beside a scalar base and computes where it is used.
+__device__ __forceinline__ unsigned own(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ void fma4(float4 &acc, float x, float4 w) {
+    acc.x = fmaf(x, w.x, acc.x); acc.y = fmaf(x, w.y, acc.y); acc.z = fmaf(x, w.z, acc.z); acc.w = fmaf(x, w.w, acc.w);
+}
+// column c of a product: the partial sums j0, j0 + STEP, .. of n; `meanwhile` runs while they come
+template <int N, int NS, int STEP, typename F> __device__ __forceinline__ float part_sum(const float *part, int c, int j0, const F &meanwhile) {
+    float v[(NS + STEP - 1) / STEP], s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NS; j += STEP) v[j / STEP] = part[(j0 + j) * N + c];
+    meanwhile();
+#pragma unroll
+    for (int j = 0; j < NS; j += STEP) s += v[j / STEP];
+    return s;
+}
+
 }  // namespace
 }  // namespace mrs

@@ -9,7 +9,9 @@
 // accumulation); only the order of the dot-product sums differs, and it is fixed (same result on every run).
 #include "tiny_rows.hpp"
 #include "host_io.hpp"
+#include "mfma_tiles.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace mrs {
 namespace {
@@ -164,6 +166,297 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     if (a.host.out) host_row_done(a.host, b);
 }
 
+// The same step with the weights streamed, for models of the default expand, d_state, d_conv and dt_rank; of those this route takes
+// d_model 64 and 128 (x_proj's row is a multiple of four floats there), and each is an instance.  In the kernel above every product asks
+// for its weights when its operand is ready: a layer of d_model 128 takes 10.4 us, while its 442 KB come in in 3.3 (one CU takes in at most
+// 58 bytes a clock from L2, measured with 1 to 256 of them reading, however many loads are in flight).  Here the requests never stop:
+// a thread holds its rows of the next layer's in_proj and x_proj in registers and those of out_proj in LDS, and each is asked for again
+// behind its use, in portions that go out while the LDS reads of the chain are under way: all of them at once would hold the waves at
+// their next instruction until the last is taken in (5.65 us against 5.3).  The chain is shorter as well: seven barriers a layer, the sum of squares
+// taken by every wave for itself and applied behind in_proj, partial sums added by the thread that needs the column, the vectors brought
+// by one request a wave.  A layer 5.3 us at d_model 128 and 2.25 at 64 (before: 10.4 and 8); the step of three layers, with the host's rows,
+// 44.1 -> 27.9 us and 37.4 -> 20.1, 256 rows 82.7 -> 72.0, 1024 rows 321 -> 272.
+constexpr int kStreamInput = 512;   // widest input row
+template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_step_kernel(TinyStepArgs a) {
+    extern __shared__ float lds[];
+    constexpr int di = 2 * DM, ds = 16, dr = DM / 16, xd = dr + 2 * ds;
+    constexpr int lg = ds / 4, rows_pp = kTinyThreads / lg, passes = (di + rows_pp - 1) / rows_pp;   // scan step: a float4 of state per lane
+    using In = Sweep<DM, 2 * di>;
+    using Xp = Sweep<di, xd>;
+    using Out = Sweep<di, DM>;
+    static_assert(di % rows_pp == 0 && 4 * DM <= kTinyThreads && 8 * xd <= kTinyThreads && 2 * di <= kTinyThreads, "one thread each");
+    float *part = lds;                  // [kTinyPart]
+    float *res = part + kTinyPart;      // [DM]   residual stream of this row
+    float *gate = res + DM;             // [di]   silu(gate half)
+    float *u = gate + di;               // [di]   conv + SiLU output
+    float *dl = u + di;                 // [di]   delta
+    float *y = dl + di;                 // [di]   gated scan output
+    float *xdbl = y + di;               // [xd]   x_proj output: dt input, B, C
+    float *xin = xdbl + xd;             // [kStreamInput]  input row, then residual stream times norm weight
+    float *vec = xin + kStreamInput;    // [8][256]   the layer's vectors: conv taps (four chunks of di floats), conv bias, dt bias, D, next norm weight
+    float *dtl = vec + 2048;            // [dr][di]   dt_proj
+    float *wo = dtl + (dr * di + 255) / 256 * 256;   // [Out::rows][threads] float4: out_proj's rows, each thread its own (last: the others are reached by constant offsets)
+    const int tid = threadIdx.x, lane = tid & 63, b = blockIdx.x;
+    const In in(tid);
+    const Xp xp(tid);
+    const Out op(tid);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto at = [&](const float *p) { return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const float *)p + (unsigned)wave * 1024u; };
+    const unsigned wo_at = at(wo), vec_at = at(vec), dt_at = at(dtl);
+    const int cx = min(tid >> 3, xd - 1), co = min(tid >> 2, DM - 1);
+
+    float4 wi[In::rows], wx[Xp::rows];
+    auto ask_in = [&](const float *W, int j0, int n) {
+#pragma unroll
+        for (int j = j0; j < j0 + n; j++) wi[j] = ld4(global(W + j * 2 * di), in.off);
+    };
+    auto ask_x = [&](const float *W) {
+#pragma unroll
+        for (int j = 0; j < Xp::rows; j++) wx[j] = ld4(global(W + j * xd), xp.off);
+    };
+    auto ask_out = [&](const float *W, int j0, int n) {
+#pragma unroll
+        for (int j = j0; j < j0 + n; j++) dma_kb(wo_at + (unsigned)j * (16u * kTinyThreads), W + j * DM, op.off);
+    };
+
+    // input row -> residual stream (identity or projection + bias); the first eight rows of a slice of its weights are asked for ahead of the layers'
+    TinyStepLayer lw = table_entry(a.layers), lnext = table_entry(a.layers + min(1, a.n_layers - 1));
+    {
+        constexpr int nq = DM / 4, sn = kTinyThreads / nq < kTinySlices ? kTinyThreads / nq : kTinySlices;
+        const int kper = (a.input_dim + sn - 1) / sn, q = tid % nq, s = tid / nq;
+        const int k0 = min(s * kper, a.input_dim), k1 = min(a.input_dim, k0 + kper);
+        float4 w[8];
+        const float v0 = a.input[(int64_t)b * a.input_dim + min(tid, a.input_dim - 1)];
+        auto ask = [&](int kb) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) w[j] = ld4(global(a.in_w), 4u * (min(kb + j, a.input_dim - 1) * DM + 4 * q));
+        };
+        if (a.in_w) ask(k0);
+        const float nw0 = ld1(global(lw.norm_w), 4u * co), bias = a.in_w ? a.in_b[co] : 0.0f;
+        pin();
+        ask_in(lw.in_proj, 0, In::rows);
+        ask_x(lw.x_proj);
+        pin();
+        for (int i = tid; i < a.input_dim; i += kTinyThreads) {
+            const float v = i == tid ? v0 : a.input[(int64_t)b * a.input_dim + i];
+            xin[i] = v;
+            if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + i] = v;   // (the input came straight from host memory)
+        }
+        lds_barrier();
+        float r;
+        if (a.in_w) {
+            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int kb = k0; kb < k1; kb += 8) {
+                if (kb != k0) ask(kb);
+#pragma unroll
+                for (int j = 0; j < 8; j++) fma4(acc, kb + j < k1 ? xin[kb + j] : 0.0f, w[j]);
+            }
+            if (s < sn) *reinterpret_cast<float4 *>(&part[s * DM + 4 * q]) = acc;
+            lds_barrier();
+            r = bias + part_sum<DM, sn, 1>(part, co, 0, [] {});
+        } else {
+            r = xin[co];
+            lds_barrier();   // xin is read before it is written again
+        }
+        if ((tid & 3) == 0 && tid < 4 * DM) { res[co] = r; xin[co] = r * nw0; }
+        lds_barrier();
+    }
+
+    auto layer = [&](auto last_layer, int l) {
+        constexpr bool kLast = decltype(last_layer)::value;
+        const int tid = (int)own(threadIdx.x), lane = tid & 63, cx = min(tid >> 3, xd - 1), co = min(tid >> 2, DM - 1);   // (not held over the layers)
+        // what the layer needs besides its products, and the norm weight of the next one
+        float *cst = a.conv_state + ((int64_t)l * a.batch + b) * di * 4;
+        float *hst = a.ssm_state + ((int64_t)l * a.batch + b) * di * ds;
+        {   // One request a wave each, into LDS: a load of 4 bytes a lane takes as long as one of 16.
+            const float *v = wave < 4 ? lw.conv_w + wave * di : wave == 4 ? lw.conv_b : wave == 5 ? lw.dt_b : wave == 6 ? lw.D : kLast ? a.norm_f : lnext.norm_w;
+            dma_kb(vec_at, v, (16u * lane) & (wave == 7 ? 4u * DM - 1 : 4u * di - 1));   // (a shorter vector is read around)
+            if (wave < dr * di / 256) dma_kb(dt_at, lw.dt_w + wave * 256, 16u * lane);
+        }
+        const unsigned ch16 = own(16u * min(tid, di - 1)), st4 = own(16u * tid);
+        float4 win = make_float4(0.f, 0.f, 0.f, 0.f), hv[passes], av[passes];
+        if (tid < di) win = ld4(global(cst), ch16);
+#pragma unroll
+        for (int p = 0; p < passes; p++) {
+            hv[p] = ld4(global(hst + p * rows_pp * ds), st4);
+            av[p] = ld4(global(lw.a_neg + p * rows_pp * ds), st4);
+        }
+        // the k-th eighth of the next layer's in_proj, asked for while the LDS reads before it are under way
+        auto feed = [&](int k) {
+            pin();
+            if (!kLast) ask_in(lnext.in_proj, k * In::rows / 8, In::rows / 8);
+            pin();
+        };
+        pin();
+        // out_proj's rows: half of them during in_proj, a quarter each during the conv and x_proj
+        constexpr int out_part = Out::rows * 2 / In::rows;
+        auto feed_out = [&](int quarter) {
+            pin();
+            ask_out(lw.out_proj, quarter * Out::rows / 4, Out::rows / 4);
+            pin();
+        };
+        // RMSNorm and in_proj: 1 / rms is a factor of every column
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < DM; i += 64) ss = fmaf(res[i + lane], res[i + lane], ss);
+#pragma unroll
+        for (int j = 0; j < In::rows; j += 4) {
+            const float4 x = *reinterpret_cast<const float4 *>(&xin[in.j * In::rows + j]);
+            fma4(acc, x.x, wi[j]); fma4(acc, x.y, wi[j + 1]); fma4(acc, x.z, wi[j + 2]); fma4(acc, x.w, wi[j + 3]);
+            pin(acc);
+            ask_out(lw.out_proj, j / 4 * out_part, out_part);   // (the wave has read what these rows replace)
+            pin();
+        }
+        const float inv = rms_inv(wave_sum(ss), DM, a.eps);
+        if (in.on) *reinterpret_cast<float4 *>(&part[in.j * 2 * di + 4 * in.q]) = acc;
+        // The vectors are in LDS: half of out_proj's requests are newer, and loads come back in order (stores that are still open only raise the count).
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Out::rows / 4) : "memory");
+        lds_barrier();
+        // conv1d step + SiLU on the x half (window slot k holds the input d_conv - k steps back; the new input goes last), SiLU of the gate half
+        const float4 tap = *reinterpret_cast<const float4 *>(&vec[min(tid, di - 1) / (di / 4) * 256 + min(tid, di - 1) % (di / 4) * 4]);
+        const float cb = vec[4 * 256 + min(tid, di - 1)];
+        const float p = inv * part_sum<2 * di, In::n, 1>(part, min(tid, 2 * di - 1), 0, [&] { feed_out(2); });
+        if (tid < di) {
+            float s = fmaf(win.y, tap.x, cb);
+            s = fmaf(win.z, tap.y, s);
+            s = fmaf(win.w, tap.z, s);
+            s = fmaf(p, tap.w, s);
+            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(cst) + ch16) = make_float4(win.y, win.z, win.w, p);
+            u[tid] = silu(s);
+        } else if (tid < 2 * di) {
+            gate[tid - di] = silu(p);
+        }
+        lds_barrier();
+        // x_proj
+        acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        {
+            float4 x[Xp::rows / 4];
+#pragma unroll
+            for (int j = 0; j < Xp::rows; j += 4) x[j / 4] = *reinterpret_cast<const float4 *>(&u[xp.j * Xp::rows + j]);
+            feed_out(3);
+#pragma unroll
+            for (int j = 0; j < Xp::rows; j += 4) {
+                fma4(acc, x[j / 4].x, wx[j]); fma4(acc, x[j / 4].y, wx[j + 1]); fma4(acc, x[j / 4].z, wx[j + 2]); fma4(acc, x[j / 4].w, wx[j + 3]);
+            }
+        }
+        pin(acc);
+        if (xp.on) *reinterpret_cast<float4 *>(&part[xp.j * xd + 4 * xp.q]) = acc;
+        lds_barrier();
+        const float xs = oct_sum(part_sum<xd, Xp::n, 8>(part, cx, tid & 7, [&] { feed(0); }));
+        if ((tid & 7) == 0 && tid < 8 * xd) xdbl[cx] = xs;
+        pin();
+        if (!kLast) ask_x(lnext.x_proj);
+        pin();
+        lds_barrier();
+        // dt_proj + bias + softplus
+        {
+            float v[dr], w[dr], s = 0.0f;
+            const int c = min(tid, di - 1);
+#pragma unroll
+            for (int j = 0; j < dr; j++) { v[j] = xdbl[j]; w[j] = dtl[j * di + c]; }
+            const float dtb = vec[5 * 256 + c];
+            feed(1);
+            if (tid < di) {
+#pragma unroll
+                for (int j = 0; j < dr; j++) s = fmaf(v[j], w[j], s);
+                dl[tid] = softplus20(s + dtb);
+            }
+        }
+        lds_barrier();
+        // scan step + D skip + gate (the arithmetic of ssm_step_kernel)
+        if (kLast) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // out_proj's rows (ahead of the stores)
+        const int g = tid % lg;
+        float Bv[4], Cv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) { Bv[k] = xdbl[dr + 4 * g + k]; Cv[k] = xdbl[dr + ds + 4 * g + k]; }
+#pragma unroll
+        for (int p = 0; p < passes; p++) {
+            const int d = tid / lg + p * rows_pp;
+            const float dv = dl[d], uv = u[d], gv = gate[d], Dv = vec[6 * 256 + d];
+            feed(2 + p);
+            const float du = dv * uv, x = dv * kLog2e;
+            float4 h = hv[p];
+            h.x = fmaf(fast_exp2(x * av[p].x), h.x, du * Bv[0]);
+            h.y = fmaf(fast_exp2(x * av[p].y), h.y, du * Bv[1]);
+            h.z = fmaf(fast_exp2(x * av[p].z), h.z, du * Bv[2]);
+            h.w = fmaf(fast_exp2(x * av[p].w), h.w, du * Bv[3]);
+            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(hst + p * rows_pp * ds) + st4) = h;
+            float s = h.x * Cv[0];
+            s = fmaf(h.y, Cv[1], s);
+            s = fmaf(h.z, Cv[2], s);
+            s = fmaf(h.w, Cv[3], s);
+            s = quad_sum(s);
+            if (g == 0) y[d] = fmaf(Dv, uv, s) * gv;
+        }
+        if (passes == 1) feed(3);
+        // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer.
+        if (!kLast) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(In::rows / 4) : "memory");
+        pin();
+        lds_barrier();
+        // out_proj and residual
+        acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        {
+            constexpr int turns = Out::rows / 4;
+            float4 x[2], w[2][4];
+            auto take = [&](int t) {
+                x[t % 2] = *reinterpret_cast<const float4 *>(&y[op.j * Out::rows + 4 * t]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) w[t % 2][k] = reinterpret_cast<const float4 *>(wo)[(4 * t + k) * kTinyThreads + tid];
+            };
+            take(0);
+#pragma unroll
+            for (int t = 0; t < turns; t++) {
+                if (t + 1 < turns) take(t + 1);
+                if (t < 3) feed(4 + t);
+                fma4(acc, x[t % 2].x, w[t % 2][0]); fma4(acc, x[t % 2].y, w[t % 2][1]); fma4(acc, x[t % 2].z, w[t % 2][2]); fma4(acc, x[t % 2].w, w[t % 2][3]);
+            }
+#pragma unroll
+            for (int t = turns; t < 3; t++) feed(4 + t);
+        }
+        pin(acc);
+        if (op.on) *reinterpret_cast<float4 *>(&part[op.j * DM + 4 * op.q]) = acc;
+        lds_barrier();
+        const float os = quad_sum(part_sum<DM, Out::n, 4>(part, co, tid & 3, [&] { feed(7); }));
+        if ((tid & 3) == 0 && tid < 4 * DM) {
+            const float r = res[co] + os;
+            res[co] = r;
+            xin[co] = r * vec[7 * 256 + co];
+        }
+        lds_barrier();
+    };
+    for (int l = 0; l + 1 < a.n_layers; l++) {
+        const TinyStepLayer after = table_entry(a.layers + min(l + 2, a.n_layers - 1));
+        layer(std::false_type(), l);
+        lw = lnext;
+        lnext = after;
+    }
+    layer(std::true_type(), a.n_layers - 1);
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < DM; i += 64) ss = fmaf(res[i + lane], res[i + lane], ss);
+    const float inv = rms_inv(wave_sum(ss), DM, a.eps);
+    if (tid < DM) {
+        const float v = xin[tid] * inv;   // (times norm_f already)
+        a.temporal[(int64_t)b * DM + tid] = v;
+        if (a.host.out) a.host.out[(int64_t)b * DM + tid] = v;
+    }
+    if (a.host.out) host_row_done(a.host, b);
+}
+
+template <int DM> bool tiny_stream_fits(const TinyStepArgs &a) {
+    return a.dm == DM && a.di == 2 * DM && a.ds == 16 && a.dc == 4 && a.dr == DM / 16 && a.input_dim <= kStreamInput;
+}
+template <int DM> int launch_tiny_stream(hipStream_t st, const TinyStepArgs &a) {
+    constexpr int dr = DM / 16, di = 2 * DM, xd = dr + 32;
+    constexpr size_t lds = sizeof(float) * (kTinyPart + DM + 4 * di + xd + kStreamInput + 2048 + (dr * di + 255) / 256 * 256 + (size_t)Sweep<di, DM>::rows * 4 * kTinyThreads);
+    static_assert(lds <= 160 * 1024, "LDS");
+    static const hipError_t attr = hipFuncSetAttribute((const void *)tiny_stream_step_kernel<DM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (attr != hipSuccess) return fail(MRS_E_HIP, "tiny backbone step: LDS size: %s", hipGetErrorString(attr));
+    hipLaunchKernelGGL(tiny_stream_step_kernel<DM>, dim3((unsigned)a.batch), dim3(kTinyThreads), lds, st, a);
+    return check_launch("tiny_stream_step_kernel");
+}
+
 size_t tiny_lds_bytes(const TinyStepArgs &a) {
     const int xin_n = rup4(a.input_dim > a.dm ? a.input_dim : a.dm);
     return sizeof(float) * ((size_t)rup4(a.dm) + xin_n + rup4(2 * a.di) + 3 * (size_t)rup4(a.di) + rup4(a.xd) + kTinyPart + kTinyThreads / 64);
@@ -186,6 +479,8 @@ int launch_tiny_step(hipStream_t st, const TinyStepArgs &a) {
         !a.conv_state || !a.ssm_state || !a.temporal || !a.norm_f)
         return fail(MRS_E_SHAPE, "tiny backbone step: shape outside the single-launch route (d_model=%d d_inner=%d d_state=%d xdbl=%d)", a.dm, a.di,
                     a.ds, a.xd);
+    if (tiny_stream_fits<128>(a)) return launch_tiny_stream<128>(st, a);
+    if (tiny_stream_fits<64>(a)) return launch_tiny_stream<64>(st, a);
     const size_t lds = tiny_lds_bytes(a);
     if (lds > 64 * 1024) return fail(MRS_E_SHAPE, "tiny backbone step: %zu bytes of LDS", lds);
     hipLaunchKernelGGL(tiny_backbone_step_kernel, dim3((unsigned)a.batch), dim3(kTinyThreads), lds, st, a);

@@ -484,6 +484,51 @@ def test_small_f32_models_step_in_one_launch(shape, monkeypatch):
     ref.close()
 
 
+@pytest.mark.parametrize("dm,L,idim,B", [
+    (128, 1, 128, 1),      # one layer: nothing is asked for ahead
+    (128, 2, 1, 3),        # narrowest input row: slices of its projection without rows
+    (128, 3, 512, 2),      # widest input row of the streamed kernel
+    (128, 2, 513, 2),      # one more: the other kernel
+    (128, 5, 0, 300),      # identity input projection, more rows than compute units
+    (64, 1, 64, 1),
+    (64, 4, 0, 5),
+    (64, 2, 131, 7),       # rows of the projection's last slice missing
+])
+def test_small_f32_step_with_streamed_weights_follows_the_cpu_route(dm, L, idim, B):
+    """Single-launch step of f32 models of the default expand, d_state, d_conv and dt_rank: the weights of a layer are requested during the one
+    before.  Outputs and states of every layer against the CPU route over several steps; f32 sums of at most 513 terms in another order,
+    1e-4 of the scale as for the other single-launch steps."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
+    w = MambaWeights.init(cfg, idim or dm, 5)
+    if not idim:
+        w.input_proj_w = np.zeros(0, np.float32); w.input_proj_b = np.zeros(0, np.float32)
+    rng = np.random.default_rng(L + B)
+    for lw in w.layers:   # vectors that are constant in a fresh model
+        for n in ("norm_weight", "conv1d_bias", "d_param"):
+            getattr(lw, n)[:] = 1.0 + 0.2 * rng.standard_normal(getattr(lw, n).shape)
+    w.norm_f_weight[:] = 1.0 + 0.2 * rng.standard_normal(dm)
+    P = oracle_params(w, cfg, idim or dm)
+    if not idim:
+        P.input_proj_w[:] = np.eye(dm, dtype=np.float32).reshape(P.input_proj_w.shape); P.input_proj_b[:] = 0
+    print(f"case streamed step {dm} {L} {idim} {B}", flush=True)
+    eng = GpuMambaBackbone.new(0, w, cfg, idim or dm, B)
+    assert eng.decode_route() == 2
+    rows = sorted({0, B // 2, B - 1})
+    st = {b: orc.m1_zero_state(P) for b in rows}
+    for t in range(4):
+        x = rng.standard_normal((B, idim or dm)).astype(np.float32)
+        if t == 2:
+            eng.capture_graph()
+        got = eng.step(x)
+        for b in rows:
+            assert scaled_err(got[b], orc.m1_backbone_step(P, x[b], *st[b])) < 1e-4, (t, b)
+    for l in range(L):
+        conv, ssm = eng.download_state(l)
+        for b in rows:
+            assert scaled_err(conv[b][:, 1:], st[b][0][l].reshape(2 * dm, 3)) < 1e-4 and scaled_err(ssm[b], st[b][1][l].reshape(2 * dm, 16)) < 1e-4, (l, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,lens,dtype", [
     (128, (9, 5), WeightDtype.F16),              # four tokens; dt_rank 8: a quarter of a k-step of dt_proj
     (256, (6, 40, 18), WeightDtype.BF16),        # five
