@@ -2,6 +2,7 @@
 // walks one batch row through the whole network, its products are matrix-vector sweeps over weights that sit in L2.
 #pragma once
 #include "common.hpp"
+#include "host_io.hpp"
 
 namespace mrs {
 namespace {
@@ -84,17 +85,17 @@ inline int sweep_rounds(int K, int N) {
 
 // ---- the streamed form: a layer's weights are on their way before the layer begins ----
 
-// A [K][N] product whose every thread owns four columns, 4 q .. 4 q + 3, of one of n slices of `rows` rows.
-template <int K, int N> struct Sweep {
+// A [K][N] product (rows LD floats apart) whose every thread owns four columns, 4 q .. 4 q + 3, of one of n slices of `rows` rows.
+template <int K, int N, int LD = N> struct Sweep {
     static constexpr int most = kTinyThreads / (N / 4) < 32 ? kTinyThreads / (N / 4) : 32;
     static constexpr int rows = ((K + most - 1) / most + 3) / 4 * 4, n = K / rows;
-    static_assert(N % 4 == 0 && K % rows == 0 && n * N <= kTinyPart, "whole slices");
+    static_assert(N % 4 == 0 && LD % 4 == 0 && K % rows == 0 && n * N <= kTinyPart, "whole slices");
     int q, j;       // (a thread behind the last slice works on slice 0 and its sum goes nowhere)
     bool on;
     unsigned off;   // its first row's bytes
     __device__ explicit Sweep(int tid) : q(tid % (N / 4)), j(tid / (N / 4)), on(j < n) {
         if (!on) j = 0;
-        off = 4u * (j * rows * N + 4 * q);
+        off = 4u * (j * rows * LD + 4 * q);
         asm volatile("" : "+v"(off));   // (kept as 32 bits beside a scalar base)
     }
 };
@@ -121,10 +122,6 @@ __device__ __forceinline__ void pin() {
 __device__ __forceinline__ void pin(float4 &v) {
     asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)::"memory");
     __builtin_amdgcn_sched_barrier(0);
-}
-// One workgroup's LDS is handed on; loads from memory stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 // A table entry by scalar loads, and reads through the pointers it holds: they come out of memory, so the compiler has to be told
 // that they point to global memory (a flat load would count as an LDS operation too, and every LDS wait would wait for it).
@@ -161,6 +158,94 @@ template <int N, int NS, int STEP, typename F> __device__ __forceinline__ float 
 #pragma unroll
     for (int j = 0; j < NS; j += STEP) s += v[j / STEP];
     return s;
+}
+
+__device__ __forceinline__ unsigned lds_address(const float *p) { return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const float *)p; }
+
+constexpr int kStreamInput = 512;   // widest input row
+
+// Input row -> residual stream `res` (identity or projection + bias) and its product with the first layer's norm weight, `xin`
+// (kStreamInput floats, which first hold the row).  The first eight rows of a slice of the projection are asked for ahead of `ahead`'s requests.
+template <int DM, typename Args, typename F>
+__device__ __forceinline__ void stream_input(const Args &a, const float *norm_w, float *xin, float *res, float *part, const F &ahead) {
+    constexpr int nq = DM / 4, sn = kTinyThreads / nq < kTinySlices ? kTinyThreads / nq : kTinySlices;
+    const int tid = threadIdx.x, b = blockIdx.x, co = min(tid >> 2, DM - 1);
+    const int kper = (a.input_dim + sn - 1) / sn, q = tid % nq, s = tid / nq;
+    const int k0 = min(s * kper, a.input_dim), k1 = min(a.input_dim, k0 + kper);
+    float4 w[8];
+    const float v0 = a.input[(int64_t)b * a.input_dim + min(tid, a.input_dim - 1)];
+    auto ask = [&](int kb) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) w[j] = ld4(global(a.in_w), 4u * (min(kb + j, a.input_dim - 1) * DM + 4 * q));
+    };
+    if (a.in_w) ask(k0);
+    const float nw = ld1(global(norm_w), 4u * co), bias = a.in_w ? a.in_b[co] : 0.0f;
+    pin();
+    ahead();
+    pin();
+    if (tid < a.input_dim) {
+        xin[tid] = v0;
+        if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + tid] = v0;   // (the input came straight from host memory)
+    }
+    lds_barrier();
+    float r;
+    if (a.in_w) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int kb = k0; kb < k1; kb += 8) {
+            if (kb != k0) ask(kb);
+#pragma unroll
+            for (int j = 0; j < 8; j++) fma4(acc, kb + j < k1 ? xin[kb + j] : 0.0f, w[j]);
+        }
+        if (s < sn) *reinterpret_cast<float4 *>(&part[s * DM + 4 * q]) = acc;
+        lds_barrier();
+        r = bias + part_sum<DM, sn, 1>(part, co, 0, [] {});
+    } else {
+        r = xin[co];
+        lds_barrier();   // xin is read before it is written again
+    }
+    if ((tid & 3) == 0 && tid < 4 * DM) { res[co] = r; xin[co] = r * nw; }
+    lds_barrier();
+}
+// this lane's part of the residual stream's sum of squares (every wave takes all of it)
+template <int DM> __device__ __forceinline__ float lane_squares(const float *res) {
+    const int lane = threadIdx.x & 63;
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < DM; i += 64) ss = fmaf(res[i + lane], res[i + lane], ss);
+    return ss;
+}
+// This thread's sum of out_proj's sweep: its rows are at wo[row][thread].  feed(0), feed(1) and feed(2) run while the LDS reads are under way.
+template <typename S, typename F> __device__ __forceinline__ float4 stream_out_sweep(const S &op, const float *y, const float *wo, const F &feed) {
+    constexpr int turns = S::rows / 4;
+    const int tid = threadIdx.x;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f), x[2], w[2][4];
+    auto take = [&](int t) {
+        x[t % 2] = *reinterpret_cast<const float4 *>(&y[op.j * S::rows + 4 * t]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[t % 2][k] = reinterpret_cast<const float4 *>(wo)[(4 * t + k) * kTinyThreads + tid];
+    };
+    take(0);
+#pragma unroll
+    for (int t = 0; t < turns; t++) {
+        if (t + 1 < turns) take(t + 1);
+        if (t < 3) feed(t);
+        fma4(acc, x[t % 2].x, w[t % 2][0]); fma4(acc, x[t % 2].y, w[t % 2][1]); fma4(acc, x[t % 2].z, w[t % 2][2]); fma4(acc, x[t % 2].w, w[t % 2][3]);
+    }
+#pragma unroll
+    for (int t = turns; t < 3; t++) feed(t);
+    pin(acc);
+    return acc;
+}
+// The final norm: xin holds the residual stream times norm_f.
+template <int DM, typename Args> __device__ __forceinline__ void stream_output(const Args &a, const float *xin, const float *res) {
+    const int tid = threadIdx.x, b = blockIdx.x;
+    const float inv = rms_inv(wave_sum(lane_squares<DM>(res)), DM, a.eps);
+    if (tid < DM) {
+        const float v = xin[tid] * inv;
+        a.temporal[(int64_t)b * DM + tid] = v;
+        if (a.host.out) a.host.out[(int64_t)b * DM + tid] = v;
+    }
+    if (a.host.out) host_row_done(a.host, b);
 }
 
 }  // namespace

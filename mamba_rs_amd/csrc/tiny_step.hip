@@ -175,8 +175,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
 // their next instruction until the last is taken in (5.65 us against 5.3).  The chain is shorter as well: seven barriers a layer, the sum of squares
 // taken by every wave for itself and applied behind in_proj, partial sums added by the thread that needs the column, the vectors brought
 // by one request a wave.  A layer 5.3 us at d_model 128 and 2.25 at 64 (before: 10.4 and 8); the step of three layers, with the host's rows,
-// 44.1 -> 27.9 us and 37.4 -> 20.1, 256 rows 82.7 -> 72.0, 1024 rows 321 -> 272.
-constexpr int kStreamInput = 512;   // widest input row
+// 44.1 -> 28.4 us and 37.4 -> 20.5, 256 rows 82.7 -> 72.0, 1024 rows 321 -> 272.
 template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_step_kernel(TinyStepArgs a) {
     extern __shared__ float lds[];
     constexpr int di = 2 * DM, ds = 16, dr = DM / 16, xd = dr + 2 * ds;
@@ -196,75 +195,36 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
     float *vec = xin + kStreamInput;    // [8][256]   the layer's vectors: conv taps (four chunks of di floats), conv bias, dt bias, D, next norm weight
     float *dtl = vec + 2048;            // [dr][di]   dt_proj
     float *wo = dtl + (dr * di + 255) / 256 * 256;   // [Out::rows][threads] float4: out_proj's rows, each thread its own (last: the others are reached by constant offsets)
-    const int tid = threadIdx.x, lane = tid & 63, b = blockIdx.x;
-    const In in(tid);
+    const int tid = threadIdx.x, b = blockIdx.x;
     const Xp xp(tid);
-    const Out op(tid);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    auto at = [&](const float *p) { return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const float *)p + (unsigned)wave * 1024u; };
-    const unsigned wo_at = at(wo), vec_at = at(vec), dt_at = at(dtl);
-    const int cx = min(tid >> 3, xd - 1), co = min(tid >> 2, DM - 1);
+    const unsigned wo_at = lds_address(wo) + 1024u * wave, vec_at = lds_address(vec) + 1024u * wave, dt_at = lds_address(dtl) + 1024u * wave;
 
     float4 wi[In::rows], wx[Xp::rows];
-    auto ask_in = [&](const float *W, int j0, int n) {
+    auto ask_in = [&](const float *W, unsigned off, int j0, int n) {
 #pragma unroll
-        for (int j = j0; j < j0 + n; j++) wi[j] = ld4(global(W + j * 2 * di), in.off);
+        for (int j = j0; j < j0 + n; j++) wi[j] = ld4(global(W + j * 2 * di), off);
     };
-    auto ask_x = [&](const float *W) {
+    auto ask_x = [&](const float *W, unsigned off) {
 #pragma unroll
-        for (int j = 0; j < Xp::rows; j++) wx[j] = ld4(global(W + j * xd), xp.off);
+        for (int j = 0; j < Xp::rows; j++) wx[j] = ld4(global(W + j * xd), off);
     };
-    auto ask_out = [&](const float *W, int j0, int n) {
+    auto ask_out = [&](const float *W, unsigned off, int j0, int n) {
 #pragma unroll
-        for (int j = j0; j < j0 + n; j++) dma_kb(wo_at + (unsigned)j * (16u * kTinyThreads), W + j * DM, op.off);
+        for (int j = j0; j < j0 + n; j++) dma_kb(wo_at + (unsigned)j * (16u * kTinyThreads), W + j * DM, off);
     };
 
-    // input row -> residual stream (identity or projection + bias); the first eight rows of a slice of its weights are asked for ahead of the layers'
     TinyStepLayer lw = table_entry(a.layers), lnext = table_entry(a.layers + min(1, a.n_layers - 1));
-    {
-        constexpr int nq = DM / 4, sn = kTinyThreads / nq < kTinySlices ? kTinyThreads / nq : kTinySlices;
-        const int kper = (a.input_dim + sn - 1) / sn, q = tid % nq, s = tid / nq;
-        const int k0 = min(s * kper, a.input_dim), k1 = min(a.input_dim, k0 + kper);
-        float4 w[8];
-        const float v0 = a.input[(int64_t)b * a.input_dim + min(tid, a.input_dim - 1)];
-        auto ask = [&](int kb) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) w[j] = ld4(global(a.in_w), 4u * (min(kb + j, a.input_dim - 1) * DM + 4 * q));
-        };
-        if (a.in_w) ask(k0);
-        const float nw0 = ld1(global(lw.norm_w), 4u * co), bias = a.in_w ? a.in_b[co] : 0.0f;
-        pin();
-        ask_in(lw.in_proj, 0, In::rows);
-        ask_x(lw.x_proj);
-        pin();
-        for (int i = tid; i < a.input_dim; i += kTinyThreads) {
-            const float v = i == tid ? v0 : a.input[(int64_t)b * a.input_dim + i];
-            xin[i] = v;
-            if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + i] = v;   // (the input came straight from host memory)
-        }
-        lds_barrier();
-        float r;
-        if (a.in_w) {
-            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int kb = k0; kb < k1; kb += 8) {
-                if (kb != k0) ask(kb);
-#pragma unroll
-                for (int j = 0; j < 8; j++) fma4(acc, kb + j < k1 ? xin[kb + j] : 0.0f, w[j]);
-            }
-            if (s < sn) *reinterpret_cast<float4 *>(&part[s * DM + 4 * q]) = acc;
-            lds_barrier();
-            r = bias + part_sum<DM, sn, 1>(part, co, 0, [] {});
-        } else {
-            r = xin[co];
-            lds_barrier();   // xin is read before it is written again
-        }
-        if ((tid & 3) == 0 && tid < 4 * DM) { res[co] = r; xin[co] = r * nw0; }
-        lds_barrier();
-    }
+    stream_input<DM>(a, lw.norm_w, xin, res, part, [&] {
+        ask_in(lw.in_proj, In(tid).off, 0, In::rows);
+        ask_x(lw.x_proj, own(xp.off));
+    });
 
     auto layer = [&](auto last_layer, int l) {
         constexpr bool kLast = decltype(last_layer)::value;
         const int tid = (int)own(threadIdx.x), lane = tid & 63, cx = min(tid >> 3, xd - 1), co = min(tid >> 2, DM - 1);   // (not held over the layers)
+        const In in(tid);
+        const Out op(tid);
         // what the layer needs besides its products, and the norm weight of the next one
         float *cst = a.conv_state + ((int64_t)l * a.batch + b) * di * 4;
         float *hst = a.ssm_state + ((int64_t)l * a.batch + b) * di * ds;
@@ -284,7 +244,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         // the k-th eighth of the next layer's in_proj, asked for while the LDS reads before it are under way
         auto feed = [&](int k) {
             pin();
-            if (!kLast) ask_in(lnext.in_proj, k * In::rows / 8, In::rows / 8);
+            if (!kLast) ask_in(lnext.in_proj, own(in.off), k * In::rows / 8, In::rows / 8);
             pin();
         };
         pin();
@@ -292,20 +252,18 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         constexpr int out_part = Out::rows * 2 / In::rows;
         auto feed_out = [&](int quarter) {
             pin();
-            ask_out(lw.out_proj, quarter * Out::rows / 4, Out::rows / 4);
+            ask_out(lw.out_proj, op.off, quarter * Out::rows / 4, Out::rows / 4);
             pin();
         };
         // RMSNorm and in_proj: 1 / rms is a factor of every column
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        float ss = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DM; i += 64) ss = fmaf(res[i + lane], res[i + lane], ss);
+        const float ss = lane_squares<DM>(res);
 #pragma unroll
         for (int j = 0; j < In::rows; j += 4) {
             const float4 x = *reinterpret_cast<const float4 *>(&xin[in.j * In::rows + j]);
             fma4(acc, x.x, wi[j]); fma4(acc, x.y, wi[j + 1]); fma4(acc, x.z, wi[j + 2]); fma4(acc, x.w, wi[j + 3]);
             pin(acc);
-            ask_out(lw.out_proj, j / 4 * out_part, out_part);   // (the wave has read what these rows replace)
+            ask_out(lw.out_proj, op.off, j / 4 * out_part, out_part);   // (the wave has read what these rows replace)
             pin();
         }
         const float inv = rms_inv(wave_sum(ss), DM, a.eps);
@@ -346,7 +304,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         const float xs = oct_sum(part_sum<xd, Xp::n, 8>(part, cx, tid & 7, [&] { feed(0); }));
         if ((tid & 7) == 0 && tid < 8 * xd) xdbl[cx] = xs;
         pin();
-        if (!kLast) ask_x(lnext.x_proj);
+        if (!kLast) ask_x(lnext.x_proj, own(xp.off));
         pin();
         lds_barrier();
         // dt_proj + bias + softplus
@@ -395,25 +353,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         pin();
         lds_barrier();
         // out_proj and residual
-        acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        {
-            constexpr int turns = Out::rows / 4;
-            float4 x[2], w[2][4];
-            auto take = [&](int t) {
-                x[t % 2] = *reinterpret_cast<const float4 *>(&y[op.j * Out::rows + 4 * t]);
-#pragma unroll
-                for (int k = 0; k < 4; k++) w[t % 2][k] = reinterpret_cast<const float4 *>(wo)[(4 * t + k) * kTinyThreads + tid];
-            };
-            take(0);
-#pragma unroll
-            for (int t = 0; t < turns; t++) {
-                if (t + 1 < turns) take(t + 1);
-                if (t < 3) feed(4 + t);
-                fma4(acc, x[t % 2].x, w[t % 2][0]); fma4(acc, x[t % 2].y, w[t % 2][1]); fma4(acc, x[t % 2].z, w[t % 2][2]); fma4(acc, x[t % 2].w, w[t % 2][3]);
-            }
-#pragma unroll
-            for (int t = turns; t < 3; t++) feed(4 + t);
-        }
+        acc = stream_out_sweep(op, y, wo, [&](int turn) { feed(4 + turn); });
         pin(acc);
         if (op.on) *reinterpret_cast<float4 *>(&part[op.j * DM + 4 * op.q]) = acc;
         lds_barrier();
@@ -432,16 +372,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         lnext = after;
     }
     layer(std::true_type(), a.n_layers - 1);
-    float ss = 0.0f;
-#pragma unroll
-    for (int i = 0; i < DM; i += 64) ss = fmaf(res[i + lane], res[i + lane], ss);
-    const float inv = rms_inv(wave_sum(ss), DM, a.eps);
-    if (tid < DM) {
-        const float v = xin[tid] * inv;   // (times norm_f already)
-        a.temporal[(int64_t)b * DM + tid] = v;
-        if (a.host.out) a.host.out[(int64_t)b * DM + tid] = v;
-    }
-    if (a.host.out) host_row_done(a.host, b);
+    stream_output<DM>(a, xin, res);
 }
 
 template <int DM> bool tiny_stream_fits(const TinyStepArgs &a) {

@@ -331,6 +331,48 @@ def test_small_f32_models_step_in_one_launch(case, monkeypatch):
     ref.close()
 
 
+@pytest.mark.parametrize("dm,L,idim,B", [
+    (128, 1, 128, 1),      # one layer: nothing is asked for ahead
+    (128, 2, 1, 3),        # narrowest input row
+    (128, 3, 512, 2),      # widest input row of the streamed kernel
+    (128, 2, 513, 2),      # one more: the other kernel
+    (128, 5, 0, 300),      # identity input projection, more rows than compute units
+    (64, 1, 64, 1),
+    (64, 4, 0, 5),
+    (64, 2, 131, 7),
+])
+def test_small_f32_step_with_streamed_weights_follows_the_cpu_route(dm, L, idim, B):
+    """Single-launch step of f32 models of the default hyperparameters: the weights of a layer are requested during the one before.  Outputs
+    and states of every layer against the CPU route over several steps; f32 sums of at most 513 terms in another order, 2e-4 of the
+    scale as for the other single-launch steps (angles 1e-3, where the accumulated f32 angle is all that differs)."""
+    cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=L, rope_fraction=0.5, a_floor=1e-4)
+    w = perturbed(cfg, idim or dm, 23)
+    if not idim:
+        w.input_proj_w = np.eye(dm, dtype=np.float32); w.input_proj_b = np.zeros(dm, np.float32)
+    P = oracle_params(w, cfg, idim or dm)
+    if not idim:
+        w.input_proj_w = np.zeros(0, np.float32); w.input_proj_b = np.zeros(0, np.float32)
+    rng = np.random.default_rng(L + B)
+    print(f"case m3 streamed step {dm} {L} {idim} {B}", flush=True)
+    eng = GpuMamba3Backbone.new(0, w, cfg, idim or dm, B)
+    assert eng.decode_route() == 2
+    rows = sorted({0, B // 2, B - 1})
+    st = {b: P.zero_state() for b in rows}
+    for t in range(5):
+        x = rng.standard_normal((B, idim or dm)).astype(np.float32)
+        if t == 2:
+            eng.capture_graph()
+        got = eng.step(x)
+        for b in rows:
+            assert scaled_err(got[b], orc.m3_backbone_step(P, x[b], st[b])) < 2e-4, (t, b)
+    for l in range(L):
+        ssm, k, v, ang = eng.download_state(l)
+        for b in rows:
+            assert scaled_err(ssm[b], st[b][0][l]) < 2e-4 and scaled_err(k[b], st[b][1][l]) < 2e-4 and scaled_err(v[b], st[b][2][l]) < 2e-4, (l, b)
+            assert np.max(np.abs(np.sin(ang[b]) - np.sin(st[b][3][l]))) < 1e-3 and np.max(np.abs(np.cos(ang[b]) - np.cos(st[b][3][l]))) < 1e-3, (l, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("B,T,dtype", [(1, 16, WeightDtype.BF16), (5, 17, WeightDtype.F16), (128, 16, WeightDtype.BF16)])
 def test_prefill_projects_the_last_steps_alone_in_its_last_layer(B, T, dtype):
     """Behind the last layer's scan only the last step of each sequence goes on.  Against the same prompt in two calls, the second of eight
