@@ -273,6 +273,10 @@ bool conv_xproj_ok(int dtype, const void *u, const void *xdbl, const float *stat
 bool conv_xproj_wins(int batch, int T, int xd);
 int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
                       int di, int xd);
+// mrs_ssm_scan_fwd_ex where of y the last step of each sequence is all that is wanted: its other rows are written or not, and the gate is looked at there alone
+// (rows of the last chunk in front hold any values)
+int launch_scan_last(hipStream_t st, int dtype, float *h, void *y, const void *delta, const void *u, const void *B, const void *C, int64_t bc_stride, const float *a_neg, const float *D,
+                     const void *gate, int64_t gate_stride, unsigned flags, void *workspace, size_t workspace_bytes, int batch, int T, int d_inner, int d_state);
 bool dt_proj_softplus_ok(int dtype, int di, int dr, int64_t xs, const void *delta, const void *dt_in, const void *wt);
 int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *dt_in, int64_t xs, const void *wt, const float *bias,
                             int64_t rows, int di, int dr);

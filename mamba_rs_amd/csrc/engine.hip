@@ -428,7 +428,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         const bool step_sums = xpart && xd <= 256 && lw.dt_t_step && di % (1024 / ds) == 0 && dr % 4 == 0 && (int64_t)nr * dr <= fuse_limit;
         const int ksplit = (!fold_x && step_sums && dt != MRS_F32) ? xproj_slices(nr, xd, di) : 1;
         StepFold fold = {xpart, fold_x ? di / 16 : ksplit, nr, xd, dr, dr + ds, 0, nullptr, 0, 0};
-        if (a_mt && bb->wide && (int64_t)dm * di < (int64_t)1 << 30) {   // the step kernel asks for out_proj's lines while it waits for its states
+        if (a_mt && bb->wide && (int64_t)dm * di < (int64_t)1 << 30 && dm / 16 % tiled_gemm_unit(dm) == 0) {   // the step kernel asks for out_proj's lines while it waits for its states
             const int unit = tiled_gemm_unit(dm);
             fold.next = lw.out_proj_p; fold.next_units = (dm / 16 + unit - 1) / unit; fold.next_bytes = unit * (di / 32) * 1024;
         }
@@ -497,7 +497,16 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
         const char *z = (const char *)s->proj + (size_t)di * es;  // gate half of in_proj's output
         const char *xb = (const char *)s->xdbl;
         MRS_TRY(launch_add_rmsnorm(bb, s->residual, l == 0 ? nullptr : s->out, s->normed, false, lw.norm_w, rows, dm));
-        if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, 2 * di, dm));
+        // Behind the last layer only the last step of each sequence goes on (below), so its gate and its scan's outputs are formed there alone.  The gate half of
+        // `proj` and the other rows of y then hold what they held before.  The scan's last chunk alone: 16384 x 5120 298 -> 165 us, x 1536 99 -> 60.  The gate as a product
+        // of its own is a launch of 6 us, so it takes work to be ahead (777 x 2048 x 1024, 1.6e9: even; 16384 x 1536 x 768, 19e9: 75 -> 43 us).
+        const bool last = T > 1 && !prefix && l + 1 == L && last_step_gemm_ok(dt, s->y, lw.out_proj_t, B, T, dm, di);
+        if (last && (double)rows * di * dm >= 4e9 && lw.in_proj_t && skinny_gemm_ok(dt, B, di, dm, (int64_t)T * dm, s->normed, (const char *)lw.in_proj_t + es * di * dm)) {
+            const size_t r = T - 1;
+            MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, di, dm));
+            MRS_TRY(launch_skinny_gemm(bb->stream, dt, (char *)s->proj + es * (r * 2 * di + di), 0, (int64_t)T * 2 * di, (const char *)s->normed + es * r * dm, (int64_t)T * dm,
+                                       (const char *)lw.in_proj_t + es * di * dm, B, di, dm, SkinnyEpi()));
+        } else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, 2 * di, dm));
         else if (lw.in_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj_t, (int)rows, 2 * di, dm));
         else MRS_TRY(gemm_rm(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, (int)rows, 2 * di, dm));
         if (T == 1) {
@@ -542,7 +551,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
             }
             if (prefix) {   // delta stays in f32, as the steps of these tokens would have kept it (prefix_ok has looked at the shapes)
                 MRS_TRY(launch_scan_quad(bb->stream, dt, 2, {ssm, s->y, nullptr, s->u, xb + es * dr, xb + es * (dr + ds), z, xd, 2 * di, lw.a_neg, lw.D, nullptr, nullptr, nullptr,
-                                                             B, T, di, (di + 63) / 64, 1, T, s->xdbl, lw.dt_w_t, lw.dt_b, dr}));
+                                                             B, T, di, (di + 63) / 64, 1, T, 0, s->xdbl, lw.dt_w_t, lw.dt_b, dr}));
             } else {
                 if (lw.dt_w_t && dt_proj_softplus_ok(dt, di, dr, xd, s->delta, s->xdbl, lw.dt_w_t)) {
                     // dt_proj + bias + softplus in one matrix-core kernel (K = dt_rank is tiny: the op is one write of delta)
@@ -564,12 +573,14 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
                 // An explicit mode is honoured; in Auto the op picks the kernel itself (same recurrence, same tolerance).
                 if (bb->cfg.scan_mode == MRS_SCAN_SEQUENTIAL) flags |= MRS_FORCE_SEQUENTIAL;
                 else if (bb->cfg.scan_mode == MRS_SCAN_PARALLEL && ds == 16 && T >= 64) flags |= MRS_FORCE_PARALLEL;
-                MRS_TRY(mrs_ssm_scan_fwd_ex(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg,
-                                            lw.D, z, 2 * di, flags, s->scan_ws, s->scan_ws_bytes, B, T, di, ds));
+                if (last) MRS_TRY(launch_scan_last(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg, lw.D, z, 2 * di, flags, s->scan_ws,
+                                                   s->scan_ws_bytes, B, T, di, ds));
+                else MRS_TRY(mrs_ssm_scan_fwd_ex(bb->stream, dt, ssm, s->y, s->delta, s->u, xb + es * dr, xb + es * (dr + ds), xd, lw.a_neg,
+                                                 lw.D, z, 2 * di, flags, s->scan_ws, s->scan_ws_bytes, B, T, di, ds));
             }
         }
         if (prefix && l + 1 == L) return MRS_OK;
-        if (l + 1 == L && last_step_gemm_ok(dt, s->y, lw.out_proj_t, B, T, dm, di)) MRS_TRY(launch_last_step_gemm(bb->stream, dt, s->out, s->y, lw.out_proj_t, B, T, dm, di));
+        if (last) MRS_TRY(launch_last_step_gemm(bb->stream, dt, s->out, s->y, lw.out_proj_t, B, T, dm, di));
         else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
         else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));

@@ -827,19 +827,20 @@ __device__ __forceinline__ void pass_b_body(
     }
 }
 
+// chunks from `first` on
 template <typename T, bool S4D, int GATE>
 __global__ __launch_bounds__(kWave) void chunk_out_kernel(
     float *__restrict__ h, T *__restrict__ y, const T *__restrict__ delta, const T *__restrict__ u,
     const T *__restrict__ Bm, const T *__restrict__ Cm, int64_t bc_stride,
     const float *__restrict__ a_neg, const float *__restrict__ Dp, const T *__restrict__ gate, int64_t gate_stride,
     const float *__restrict__ h0copy, const float *__restrict__ S, const float *__restrict__ sumd,
-    int Tlen, int di, int tiles, int nchunk, int len) {
+    int Tlen, int di, int tiles, int nchunk, int len, int first) {
     __shared__ alignas(16) StagedRows Bs, Cs;
     const int tile = blockIdx.x % tiles;
-    const int rest = blockIdx.x / tiles;
+    const int rest = blockIdx.x / tiles, out = nchunk - first;
     const float unused[16] = {};
     pass_b_body<T, S4D, GATE, false>(Bs, Cs, h, y, delta, u, Bm, Cm, bc_stride, a_neg, Dp, gate, gate_stride, h0copy, S, sumd, nullptr,
-                                     nullptr, unused, Tlen, di, tiles, nchunk, len, rest / nchunk, rest % nchunk, tile);
+                                     nullptr, unused, Tlen, di, tiles, nchunk, len, rest / out, first + rest % out, tile);
 }
 
 // Both passes in one launch: the wave (chunk c, batch row b, channel tile) summarises its chunk, publishes the summary,
@@ -877,17 +878,18 @@ template <typename T> struct IsF32 { static constexpr bool value = false; };
 template <> struct IsF32<float> { static constexpr bool value = true; };
 
 // one_launch: 0 = two launches (pass A, pass B); 1 = one launch behind a small kernel that clears the flag area;
-// 2 = one launch, the caller vouches that the flag area is all zero (MRS_SCAN_FLAGS_ZERO, or the library's own buffer)
+// 2 = one launch, the caller vouches that the flag area is all zero (MRS_SCAN_FLAGS_ZERO, or the library's own buffer).  first: the first chunk whose outputs
+// are wanted (two launches only).
 template <typename T, bool S4D>
 static int launch_split_s4d(hipStream_t st, int gate_mode, float *h, T *y, const T *delta, const T *u,
                             const T *Bm, const T *Cm, int64_t bc_stride, const float *a_neg,
                             const float *D, const T *gate, int64_t gate_stride, float *ws, SplitPlan plan, int batch,
-                            int Tlen, int di, int one_launch) {
+                            int Tlen, int di, int one_launch, int first) {
     const int tiles = (di + kWave - 1) / kWave;
     const int C = plan.nchunk, L = plan.len;
     const SplitWs w = carve_workspace(ws, batch, Tlen, di, C);
     const dim3 block(kWave);
-    const dim3 gridA((unsigned)(batch * (C - 1) * tiles)), gridB((unsigned)(batch * C * tiles));
+    const dim3 gridA((unsigned)(batch * (C - 1) * tiles)), gridB((unsigned)(batch * (C - first) * tiles));
     if (one_launch) {
         if (one_launch == 1) {
             const int used = batch * tiles * (kMaxChunks + 1);   // the words this shape's waves touch
@@ -910,7 +912,7 @@ static int launch_split_s4d(hipStream_t st, int gate_mode, float *h, T *y, const
     if (rc) return rc;
 #define MRS_LAUNCH(G)                                                                                      \
     hipLaunchKernelGGL((chunk_out_kernel<T, S4D, G>), gridB, block, 0, st, h, y, delta, u, Bm, Cm, bc_stride, \
-                       a_neg, D, gate, gate_stride, w.h0copy, w.S, w.sumd, Tlen, di, tiles, C, L)
+                       a_neg, D, gate, gate_stride, w.h0copy, w.S, w.sumd, Tlen, di, tiles, C, L, first)
     if (gate_mode == 0) MRS_LAUNCH(0);
     else if (gate_mode == 1) MRS_LAUNCH(1);
     else MRS_LAUNCH(2);
@@ -922,10 +924,10 @@ template <typename T>
 static int launch_split(hipStream_t st, bool s4d, int gate_mode, float *h, void *y, const void *delta,
                         const void *u, const void *Bm, const void *Cm, int64_t bc_stride,
                         const float *a_neg, const float *D, const void *gate, int64_t gate_stride, float *ws, SplitPlan plan,
-                        int batch, int Tlen, int di, int one_launch) {
+                        int batch, int Tlen, int di, int one_launch, int first) {
 #define MRS_ARGS                                                                                       \
     st, gate_mode, h, (T *)y, (const T *)delta, (const T *)u, (const T *)Bm, (const T *)Cm, bc_stride, \
-        a_neg, D, (const T *)gate, gate_stride, ws, plan, batch, Tlen, di, one_launch
+        a_neg, D, (const T *)gate, gate_stride, ws, plan, batch, Tlen, di, one_launch, first
     return s4d ? launch_split_s4d<T, true>(MRS_ARGS) : launch_split_s4d<T, false>(MRS_ARGS);
 #undef MRS_ARGS
 }
@@ -977,11 +979,12 @@ static bool quad_wins(bool s4d, int64_t waves, int64_t elements, int len) {
 // As one pass up to this many steps (64 steps 9.2 us, 128 steps 16.0 where two passes take 11).
 constexpr int kQuadSingle = 64;
 
-// Shared body of the scan entry points: argument checks, route choice, launches.  `fn` names the caller in messages.
+// Shared body of the scan entry points: argument checks, route choice, launches.  `fn` names the caller in messages.  last: of y the last step of each
+// sequence is all that is wanted.  The chunks in front of the last one are then summarised only, and always as two launches.
 static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void *y, const void *delta, const void *u,
                          const void *B, const void *C, int64_t bc_stride, const float *a_neg, const float *D,
                          const void *gate, int64_t gate_stride, unsigned flags, void *workspace, size_t workspace_bytes,
-                         int batch, int T, int d_inner, int d_state, bool own_buffer = false) {
+                         int batch, int T, int d_inner, int d_state, bool own_buffer = false, bool last = false) {
     int rc = scan_check(fn, dtype, h, y, delta, u, B, C, a_neg, D, bc_stride, batch, T, d_inner, d_state);
     if (rc) return rc;
     int gate_mode = 0;
@@ -1030,16 +1033,16 @@ static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void
         static const bool env_two = [] { const char *e = getenv("MRS_SCAN_TWO_LAUNCHES"); return e && atoi(e) != 0; }();
         const int64_t waves = (int64_t)batch * ((d_inner + kWave - 1) / kWave) * plan.nchunk;
         const bool wins = (s4d && waves >= 2048) || (flags & MRS_FORCE_PARALLEL);
-        int one_launch = (env_two || (flags & MRS_SCAN_TWO_LAUNCHES) || !wins || !flags_fit(batch, d_inner)) ? 0
+        int one_launch = (last || env_two || (flags & MRS_SCAN_TWO_LAUNCHES) || !wins || !flags_fit(batch, d_inner)) ? 0
                          : ((own_buffer || (flags & MRS_SCAN_FLAGS_ZERO)) ? 2 : 1);
         if (!one_launch && !(flags & MRS_SCAN_TWO_LAUNCHES) && !env_two && quad_wins(s4d, waves, (int64_t)batch * T * d_inner, plan.len)) {
             const SplitWs w = carve_workspace((float *)workspace, batch, T, d_inner, plan.nchunk);
             const bool single = T <= kQuadSingle;
             return launch_scan_quad(st, dtype, gate_mode, {h, y, delta, u, B, C, gate, bc_stride, gate_stride, a_neg, D, w.h0copy, w.S, w.sumd, batch, T, d_inner,
-                                                           (d_inner + kWave - 1) / kWave, single ? 1 : plan.nchunk, single ? T : plan.len});
+                                                           (d_inner + kWave - 1) / kWave, single ? 1 : plan.nchunk, single ? T : plan.len, last && !single ? plan.nchunk - 1 : 0});
         }
         MRS_DISPATCH_DTYPE(dtype, T_, return launch_split<T_>(st, s4d, gate_mode, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride,
-                                                             (float *)workspace, plan, batch, T, d_inner, one_launch));
+                                                             (float *)workspace, plan, batch, T, d_inner, one_launch, last ? plan.nchunk - 1 : 0));
     }
     MRS_DISPATCH_DTYPE(dtype, T_, return launch_seq<T_>(st, s4d, gate_mode, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride, batch, T, d_inner, d_state));
     return MRS_OK;
@@ -1052,6 +1055,12 @@ extern "C" int mrs_ssm_scan_fwd_ex(void *stream, int dtype, float *h, void *y, c
                                    int d_inner, int d_state) {
     return scan_dispatch("mrs_ssm_scan_fwd_ex", stream, dtype, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride, flags,
                          workspace, workspace_bytes, batch, T, d_inner, d_state);
+}
+
+int mrs::launch_scan_last(hipStream_t st, int dtype, float *h, void *y, const void *delta, const void *u, const void *B, const void *C, int64_t bc_stride, const float *a_neg, const float *D,
+                          const void *gate, int64_t gate_stride, unsigned flags, void *workspace, size_t workspace_bytes, int batch, int T, int d_inner, int d_state) {
+    return scan_dispatch("scan of the last steps", st, dtype, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride, flags, workspace, workspace_bytes, batch, T, d_inner, d_state,
+                         false, true);
 }
 
 // ---- the scan without any allocation: chunk summaries in a buffer the library itself holds ---------------------------

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void scan_quad_kernel(ScanQuadArgs a) {
     constexpr int kLen = DT ? kQuadDtLen : kQuadLen;
     __shared__ alignas(16) float Bs[kLen][16], Cs[OUT ? kLen : 1][16];
     __shared__ float Ds[DT ? kLen : 1][80];   // [step][channel of the workgroup]
-    const int tile = blockIdx.x % a.tiles, rest = blockIdx.x / a.tiles, b = rest % a.batch, c = rest / a.batch;
+    const int tile = blockIdx.x % a.tiles, rest = blockIdx.x / a.tiles, b = rest % a.batch, c = (OUT ? a.first : 0) + rest / a.batch;
     const int tid = threadIdx.x, lane = tid & 63, g = lane & 3, di = a.di;
     const int d = tile * 64 + (tid >> 2);
     const bool live = d < di;
@@ -212,7 +212,7 @@ template <typename T> int launch_quad_t(hipStream_t st, int gate_mode, const Sca
         const int rc = check_launch("scan_quad_kernel (states)");
         if (rc) return rc;
     }
-    const dim3 grid(per * (unsigned)a.nchunk);
+    const dim3 grid(per * (unsigned)(a.nchunk - a.first));
     if constexpr (sizeof(T) == 2) {
         if (a.dt_w) {
             if (gate_mode != 2) return fail(MRS_E_SHAPE, "scan with dt_proj: gate mode %d", gate_mode);
@@ -236,7 +236,7 @@ bool scan_quad_dt_ok(int dtype, int T, int dr, int64_t bc_stride, const void *dt
 int launch_scan_quad(hipStream_t st, int dtype, int gate_mode, const ScanQuadArgs &a) {
     if (a.dt_w && (!scan_quad_dt_ok(dtype, a.Tlen, a.dr, a.bc_stride, a.dt_in, a.dt_w) || a.nchunk != 1 || !a.dt_b))
         return fail(MRS_E_SHAPE, "scan with dt_proj: %d steps in %d chunks, dt_rank %d", a.Tlen, a.nchunk, a.dr);
-    if (a.len < 1 || a.len > kQuadLen || a.nchunk < 1 || (int64_t)a.nchunk * a.len < a.Tlen || (int64_t)(a.nchunk - 1) * a.len >= a.Tlen || a.tiles * 64 < a.di)
+    if (a.len < 1 || a.len > kQuadLen || a.nchunk < 1 || (int64_t)a.nchunk * a.len < a.Tlen || (int64_t)(a.nchunk - 1) * a.len >= a.Tlen || a.tiles * 64 < a.di || a.first < 0 || a.first >= a.nchunk)
         return fail(MRS_E_SHAPE, "scan: %d chunks of %d for %d steps", a.nchunk, a.len, a.Tlen);
     MRS_DISPATCH_DTYPE(dtype, T_, return launch_quad_t<T_>(st, gate_mode, a));
     return MRS_OK;

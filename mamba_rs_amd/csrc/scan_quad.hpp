@@ -14,6 +14,7 @@ struct ScanQuadArgs {
     const float *a_neg, *D;
     float *h0copy, *S, *sumd;   // [batch][16][di], [batch][nchunk - 1][16][di], [batch][nchunk - 1][di]; unused with one chunk
     int batch, Tlen, di, tiles, nchunk, len;
+    int first = 0;   // the first chunk whose outputs are wanted
     // with dt_w (then delta is not read, 16-bit storage, one chunk of at most kQuadDtLen steps): the kernel forms delta = softplus(dt_in row . dt_w
     // row of the channel + dt_b) itself, in f32.  dt_in: rows of dr elements bc_stride apart, dt_w [di][dr]; dr a multiple of 8, both 16-byte aligned.
     const void *dt_in = nullptr, *dt_w = nullptr;

@@ -592,3 +592,33 @@ def test_prefill_projects_the_last_steps_alone_in_its_last_layer(dm, B, T, dtype
     e.close()
     for p, q in zip(got, want):
         assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
+
+
+@pytest.mark.parametrize("dm,B,T,trained,dtype", [
+    (256, 1, 72, False, WeightDtype.BF16),     # a first call of 64 steps: the longest single pass
+    (512, 1, 105, True, WeightDtype.F16),      # two chunks and more, four lanes per channel; a last chunk of one step
+    (1024, 1, 777, True, WeightDtype.BF16),
+    (768, 2, 1033, False, WeightDtype.BF16),   # one lane per channel, one launch where all outputs are wanted
+    (768, 8, 1040, True, WeightDtype.F16),     # general A, two launches
+    (768, 4, 2056, False, WeightDtype.BF16),   # in_proj on the large tiles
+])
+def test_prefill_forms_gate_and_outputs_of_the_last_steps_alone_in_its_last_layer(dm, B, T, trained, dtype):
+    """The same over the routes of the scan and of in_proj, where the last layer has half an in_proj and outputs of its last chunk: against two calls, the second of
+    eight steps, which form everything.  Tolerance as above."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+    w = MambaWeights.init(cfg, dm, 5)
+    w.input_proj_w = np.zeros((0, dm), np.float32)
+    rng = np.random.default_rng(B + T)
+    if trained:
+        for lw in w.layers:
+            lw.a_log = lw.a_log + 0.15 * rng.standard_normal(lw.a_log.shape).astype(np.float32)
+    x = rng.standard_normal((B, T, dm)).astype(np.float32)
+    print(f"case last layer {dm} {B}x{T} {trained} {dtype.name}", flush=True)
+    e = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    got = [e.prefill_sequence(x).copy()] + [p for l in range(2) for p in e.download_state(l)]
+    e.reset()
+    e.prefill_sequence(x[:, :T - 8].copy())
+    want = [e.prefill_sequence(x[:, T - 8:].copy()).copy()] + [p for l in range(2) for p in e.download_state(l)]
+    e.close()
+    for p, q in zip(got, want):
+        assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
