@@ -979,6 +979,27 @@ static bool quad_wins(bool s4d, int64_t waves, int64_t elements, int len) {
 // As one pass up to this many steps (64 steps 9.2 us, 128 steps 16.0 where two passes take 11).
 constexpr int kQuadSingle = 64;
 
+// Steps of a chunk there, a multiple of four, and no more chunks than the plan (and so the workspace) has.  A workgroup of a chunk brings a wave to every SIMD of a compute unit, so
+// a launch takes as long as the unit with the most of them: 1 x 777 x 2048 in 25 chunks of 32 steps is 800 workgroups, four on some units and three on most;
+// 15 of 52 steps are 480, two on any.  The best of at most one to four on a unit: a step counts once per wave of a SIMD (a lone wave's one and a half times), a summary to
+// fold a third of a step, a step without outputs 0.6.  Both launches: 1 x 1024 x 1536 26.3 -> 24.5 us, 1 x 1500 x 2048 36.8 -> 33.8, 2 x 700 x 2048 33.6 -> 31.1,
+// 1 x 400 x 5120 26.4 -> 25.4, 1 x 777 x 2048 24.5 -> 24.0, 1 x 2048 x 1536 36.7 -> 36.3, 1 x 4000 x 1536 58.7 -> 58.8.
+static int quad_len(int batch, int T, int tiles, const SplitPlan &plan) {
+    const int64_t per = (int64_t)batch * tiles;
+    int best = plan.len;
+    double best_cost = 1e30;
+    for (int w = 1; w <= 4; w++) {
+        const int most = (int)std::min<int64_t>(256 * w / per, plan.nchunk);
+        if (most < 1) continue;
+        const int len = std::max(32, ((T + most - 1) / most + 3) / 4 * 4), n = (T + len - 1) / len;
+        if (len > kQuadLen) continue;
+        auto waves = [&](int64_t wgs) { return std::max(1.5, (double)((wgs + 255) / 256)); };
+        const double cost = waves(per * n) * (len + 0.33 * n) + 0.6 * waves(per * (n - 1)) * len;
+        if (cost < best_cost) { best = len; best_cost = cost; }
+    }
+    return best;
+}
+
 // Shared body of the scan entry points: argument checks, route choice, launches.  `fn` names the caller in messages.  last: of y the last step of each
 // sequence is all that is wanted.  The chunks in front of the last one are then summarised only, and always as two launches.
 static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void *y, const void *delta, const void *u,
@@ -1038,8 +1059,9 @@ static int scan_dispatch(const char *fn, void *stream, int dtype, float *h, void
         if (!one_launch && !(flags & MRS_SCAN_TWO_LAUNCHES) && !env_two && quad_wins(s4d, waves, (int64_t)batch * T * d_inner, plan.len)) {
             const SplitWs w = carve_workspace((float *)workspace, batch, T, d_inner, plan.nchunk);
             const bool single = T <= kQuadSingle;
+            const int tiles = (d_inner + kWave - 1) / kWave, len = single ? T : quad_len(batch, T, tiles, plan), chunks = (T + len - 1) / len;
             return launch_scan_quad(st, dtype, gate_mode, {h, y, delta, u, B, C, gate, bc_stride, gate_stride, a_neg, D, w.h0copy, w.S, w.sumd, batch, T, d_inner,
-                                                           (d_inner + kWave - 1) / kWave, single ? 1 : plan.nchunk, single ? T : plan.len, last && !single ? plan.nchunk - 1 : 0});
+                                                           tiles, chunks, len, last ? chunks - 1 : 0});
         }
         MRS_DISPATCH_DTYPE(dtype, T_, return launch_split<T_>(st, s4d, gate_mode, h, y, delta, u, B, C, bc_stride, a_neg, D, gate, gate_stride,
                                                              (float *)workspace, plan, batch, T, d_inner, one_launch, last ? plan.nchunk - 1 : 0));

@@ -125,6 +125,27 @@ def test_scan_with_four_lanes_per_channel_matches_oracle(shape, dtype, s4d):
             assert_close(h, h_ref, orc.F32, "h")
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 65, 64),       # two chunks of 36 and 29 steps
+    (1, 777, 2048),    # fifteen of 52, the last of 49
+    (2, 700, 2048),    # eight of 88
+    (3, 131, 1000),    # part of a channel tile
+    (1, 4093, 1536),   # the longest chunks: 128 steps, the last of 125
+])
+@pytest.mark.parametrize("dtype", [orc.BF16, orc.F32])
+def test_scan_with_four_lanes_per_channel_in_chunks_of_no_whole_spans(shape, dtype):
+    """Chunks there are a multiple of four steps, as many as fill whole rounds of the compute units; outputs and states as the oracle has them."""
+    batch, T, di = shape
+    rng = np.random.default_rng(T)
+    inp = quantised(rng, batch, T, di, 16, dtype)
+    h0 = (rng.standard_normal((batch, di, 16)) * 0.1).astype(np.float32)
+    print(f"case chunks of no whole spans shape={shape} dtype={dtype}", flush=True)
+    y_ref, h_ref = orc.m1_scan_f64(h0, inp["delta"], inp["u"], inp["B"], inp["C"], inp["a_neg"], inp["D"], gate=inp["z"], gate_mode=2)
+    y, h = run_scan(inp, h0, dtype, 2, split="auto")
+    assert_close(y, y_ref, dtype, "y")
+    assert_close(h, h_ref, orc.F32, "h")
+
+
 def test_scan_auto_route_threshold_and_workspace_errors():
     """Up to 256 steps (the reference's serial range, src/config.rs:21-37) the single pass is kept when its (batch row,
     channel tile) pairs fill the machine -- bitwise equal to the no-workspace call -- and MRS_FORCE_SEQUENTIAL keeps it
