@@ -15,6 +15,7 @@
 // eight waves that all do everything, and so wait for their own LDS reads in front of each other's arithmetic: 39 at d_inner 1536.
 #include "common.hpp"
 #include "mfma_tiles.hpp"
+#include <algorithm>
 
 namespace mrs {
 namespace {
@@ -29,6 +30,9 @@ struct ConvXprojArgs {
     const float *w, *bias;
     int64_t x_stride;
     int T, di, xd, tiles;   // tiles: of a sequence
+    float *shares;          // with several slices of the channels: the products' shares, [slice][step][xd]
+    int slices, pieces;     // pieces of a slice
+    int64_t share_stride;
 };
 
 template <typename T> __device__ __forceinline__ void unpack2(unsigned v, float &a, float &b) {
@@ -45,10 +49,11 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
     constexpr int kReq = kStage / 1024, R = (kReq + kMoveWaves - 1) / kMoveWaves;   // requests of a piece, and of a wave
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
-    const int b = blockIdx.x / g.tiles, t0 = (blockIdx.x - b * g.tiles) * ROWS, Tlen = g.T, di = g.di, np = di / kPiece;
+    const int slice = blockIdx.x % g.slices, bt = blockIdx.x / g.slices, p0 = slice * g.pieces;
+    const int b = bt / g.tiles, t0 = (bt - b * g.tiles) * ROWS, Tlen = g.T, di = g.di, np = min(g.pieces, di / kPiece - p0);
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
     char *ut = smem + S * kStage;   // u of two pieces, 8 KB each
-    const T *xs = (const T *)g.x + (int64_t)b * Tlen * g.x_stride;
+    const T *xs = (const T *)g.x + (int64_t)b * Tlen * g.x_stride + p0 * kPiece;   // (the slice's first channel)
 
     if (w < kConvWaves) {
         // ---- conv: channels 2 c and + 1, kSteps steps of the tile from kSteps r on
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
 #pragma unroll
             for (int i = 0; i < ROWS / 32; i++) o[i] = *reinterpret_cast<const v4u *>(uin + (srow + 32 * i) * 128 + spl);
 #pragma unroll
-            for (int i = 0; i < ROWS / 32; i++) __builtin_amdgcn_raw_buffer_store_b128(o[i], ures, uoff + 64u * (unsigned)(i * di), p * (kPiece * 2), 0);
+            for (int i = 0; i < ROWS / 32; i++) __builtin_amdgcn_raw_buffer_store_b128(o[i], ures, uoff + 64u * (unsigned)(i * di), (p0 + p) * (kPiece * 2), 0);
             uin = uin == ut ? ut + ROWS * 128 : ut;
         }
     } else {
@@ -125,14 +130,14 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
                 const int t = min(max(t0 - 8 + 8 * q + (l >> 3), 0), Tlen - 1);
                 from[i] = (const char *)xs; step[i] = kPiece * 2; voff[i] = (unsigned)t * (unsigned)g.x_stride * 2u + 16u * (unsigned)(l & 7);
             } else if (q == kTaps / 1024) {
-                from[i] = (const char *)g.w; step[i] = kPiece * 16;
+                from[i] = (const char *)(g.w + p0 * kPiece * 4); step[i] = kPiece * 16;
             } else if (q == kWin / 1024) {   // (read by the first workgroup of a sequence alone)
-                from[i] = (const char *)(t0 == 0 ? g.state + (int64_t)b * di * 4 : g.w); step[i] = kPiece * 16;
+                from[i] = (const char *)((t0 == 0 ? g.state + (int64_t)b * di * 4 : g.w) + p0 * kPiece * 4); step[i] = kPiece * 16;
             } else if (q == kBias / 1024) {
-                from[i] = (const char *)g.bias; step[i] = kPiece * 4; voff[i] = 16u * (unsigned)min(l, 15);
+                from[i] = (const char *)(g.bias + p0 * kPiece); step[i] = kPiece * 4; voff[i] = 16u * (unsigned)min(l, 15);
             } else {
                 const int j = q - kW / 1024;   // column tile j / 2, half j % 2 of the piece
-                from[i] = (const char *)g.wp + ((int64_t)(j >> 1) * (di >> 5) + (j & 1)) * 1024; step[i] = 2048;
+                from[i] = (const char *)g.wp + ((int64_t)(j >> 1) * (di >> 5) + (j & 1) + 2 * p0) * 1024; step[i] = 2048;
             }
         }
         unsigned ring = 0;
@@ -197,6 +202,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
             for (int j = 0; j < kN; j++) {
                 const int col = 16 * (n0 + j) + 4 * lg;
                 if (t < Tlen && n0 + j < NT && col < g.xd) {
+                    if (g.slices > 1) {
+                        *reinterpret_cast<v4f *>(g.shares + slice * g.share_stride + ((int64_t)b * Tlen + t) * g.xd + col) = acc[i][j];
+                        continue;
+                    }
                     struct alignas(8) T4 { T v[4]; } o;
 #pragma unroll
                     for (int e = 0; e < 4; e++) Store<T>::st(&o.v[e], acc[i][j][e]);
@@ -207,8 +216,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
     }
     // The sequence's last four inputs are the window from now on; the workgroup that read the old one writes it.
     if (t0 == 0) {
-        float *sout = g.state + (int64_t)b * di * 4;
-        for (int ch = tid; ch < di; ch += kConvThreads) {
+        float *sout = g.state + ((int64_t)b * di + p0 * kPiece) * 4;
+        for (int ch = tid; ch < np * kPiece; ch += kConvThreads) {
             const T *px = xs + (int64_t)(Tlen - 4) * g.x_stride + ch;
             *reinterpret_cast<float4 *>(sout + 4 * ch) = make_float4(Store<T>::ld(px), Store<T>::ld(px + g.x_stride), Store<T>::ld(px + 2 * g.x_stride), Store<T>::ld(px + 3 * g.x_stride));
         }
@@ -221,7 +230,7 @@ int launch_conv_xproj_t(hipStream_t st, const ConvXprojArgs &g, int batch) {
     static_assert(lds <= 160 * 1024, "");
     static const hipError_t attr = hipFuncSetAttribute((const void *)conv_xproj_kernel<T, ROWS, NT, S>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "conv + x_proj: LDS size: %s", hipGetErrorString(attr));
-    hipLaunchKernelGGL((conv_xproj_kernel<T, ROWS, NT, S>), dim3((unsigned)(batch * g.tiles)), dim3(kConvThreads), lds, st, g);
+    hipLaunchKernelGGL((conv_xproj_kernel<T, ROWS, NT, S>), dim3((unsigned)(batch * g.tiles * g.slices)), dim3(kConvThreads), lds, st, g);
     return check_launch("conv_xproj_kernel");
 }
 template <typename T>
@@ -258,8 +267,50 @@ int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *sta
                       int di, int xd) {
     if (!conv_xproj_ok(dtype, u, xdbl, state, x, x_stride, wp, w, bias, batch, T, di, 4, xd)) return fail(MRS_E_SHAPE, "conv + x_proj: shape outside the route (T=%d d_inner=%d columns=%d)", T, di, xd);
     const int rows = conv_xproj_rows(batch, T);
-    const ConvXprojArgs g = {u, xdbl, state, x, wp, w, bias, x_stride, T, di, xd, (T + rows - 1) / rows};
+    const ConvXprojArgs g = {u, xdbl, state, x, wp, w, bias, x_stride, T, di, xd, (T + rows - 1) / rows, nullptr, 1, di / kPiece, 0};
     return dtype == MRS_BF16 ? launch_conv_xproj_n<bf16_t>(st, g, batch, rows) : launch_conv_xproj_n<f16_t>(st, g, batch, rows);
+}
+
+// Fewer rows: the channels in slices as well, for about one workgroup per compute unit, whose products are summed in f32, in the order of the slices, by a second launch.  The
+// shares fit in as many bytes as u has.  At 777 x 2048, 96 columns: conv 5.4, x_proj 8.0 as two launches, here 6.3 + 3.7 us.  Four layers of a bf16 prefill, two
+// launches / this: d_model 768, 500 rows 272 / 276, 1000 rows 322 / 317, 1500 rows 384 / 376; 1024, 300 rows even, 777 rows 364 / 353; 2560, 300 rows even, 1000 rows 847 / 811, 2000 rows
+// 1150 / 1113, 4 x 700 1560 / 1429.
+constexpr int kMaxSlices = 16;
+int conv_xproj_slices(int batch, int T, int di, int xd) {
+    const int64_t tiles = (int64_t)batch * ((T + 31) / 32);
+    return tiles < 24 ? 1 : (int)std::min<int64_t>(std::min(std::min(di / (2 * xd), di / kPiece / 2), kMaxSlices), 256 / tiles);
+}
+
+template <typename T> static __global__ __launch_bounds__(256) void conv_xproj_sum_kernel(T *__restrict__ out, const float *__restrict__ shares, int slices, int64_t n4) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const v4f *p = reinterpret_cast<const v4f *>(shares) + i;
+    v4f v[kMaxSlices], s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kMaxSlices; k++) v[k] = p[min(k, slices - 1) * n4];   // all asked for at once
+#pragma unroll
+    for (int k = 0; k < kMaxSlices; k++)
+        if (k < slices) s += v[k];
+    struct alignas(4 * sizeof(T)) T4 { T v[4]; } o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) Store<T>::st(&o.v[e], s[e]);
+    reinterpret_cast<T4 *>(out)[i] = o;
+}
+
+int launch_conv_xproj_sliced(hipStream_t st, int dtype, void *u, void *xdbl, float *shares, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias,
+                             int batch, int T, int di, int xd) {
+    const int slices = conv_xproj_slices(batch, T, di, xd);
+    if (!conv_xproj_ok(dtype, u, xdbl, state, x, x_stride, wp, w, bias, batch, T, di, 4, xd) || slices < 2 || !aligned(shares, 16))
+        return fail(MRS_E_SHAPE, "conv + x_proj in slices: shape outside the route (T=%d d_inner=%d columns=%d)", T, di, xd);
+    const int pieces = (di / kPiece + slices - 1) / slices;
+    const int64_t n = (int64_t)batch * T * xd;
+    const ConvXprojArgs g = {u, xdbl, state, x, wp, w, bias, x_stride, T, di, xd, (T + 31) / 32, shares, (di / kPiece + pieces - 1) / pieces, pieces, n};
+    const int rc = dtype == MRS_BF16 ? launch_conv_xproj_n<bf16_t>(st, g, batch, 32) : launch_conv_xproj_n<f16_t>(st, g, batch, 32);
+    if (rc) return rc;
+    const dim3 grid((unsigned)((n / 4 + 255) / 256));
+    if (dtype == MRS_BF16) hipLaunchKernelGGL(conv_xproj_sum_kernel<bf16_t>, grid, dim3(256), 0, st, (bf16_t *)xdbl, shares, g.slices, n / 4);
+    else hipLaunchKernelGGL(conv_xproj_sum_kernel<f16_t>, grid, dim3(256), 0, st, (f16_t *)xdbl, shares, g.slices, n / 4);
+    return check_launch("conv_xproj_sum_kernel");
 }
 
 }  // namespace mrs

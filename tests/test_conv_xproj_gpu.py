@@ -45,7 +45,21 @@ def test_long_prefill_behind_a_short_one_follows_the_cpu_route(dm, B, T, dtype):
         assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
 
 
-@pytest.mark.parametrize("dm,B,T", [(768, 3, 600), (768, 6, 1801), (1024, 4, 421), (2560, 32, 112)])
+@pytest.mark.parametrize("dm,B,T,dtype", [
+    (768, 1, 737, WeightDtype.BF16),     # the fewest rows: eight slices of three pieces; the last tile has one step
+    (768, 12, 61, WeightDtype.F16),      # two tiles a sequence
+    (768, 25, 4, WeightDtype.BF16),      # sequences of a window's length
+    (1024, 1, 777, WeightDtype.BF16),    # eight slices of four pieces
+    (1024, 3, 530, WeightDtype.F16),     # five of seven pieces, the last of four
+    (2560, 1, 768, WeightDtype.BF16),    # twelve column tiles, ten slices of eight
+    (2560, 3, 1130, WeightDtype.F16),    # two of 40
+])
+def test_prefill_in_slices_of_the_channels_follows_the_cpu_route(dm, B, T, dtype):
+    """Fewer rows: the workgroups share out the channels too.  As above."""
+    test_long_prefill_behind_a_short_one_follows_the_cpu_route(dm, B, T, dtype)
+
+
+@pytest.mark.parametrize("dm,B,T", [(768, 3, 600), (768, 6, 1801), (1024, 4, 421), (2560, 32, 112), (768, 25, 4), (1024, 3, 530)])
 def test_rows_do_not_depend_on_the_sequences_beside_them(dm, B, T):
     """The same sequence in every place of the batch, in front of it a window of its own: all of them end with the same bits."""
     cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
