@@ -19,6 +19,7 @@
 #include "mfma_tiles.hpp"
 #include <stdlib.h>
 #include <algorithm>
+#include <type_traits>
 
 namespace mrs {
 
@@ -393,7 +394,6 @@ template <typename T>
 __global__ __launch_bounds__(256) void prenorm_rows_kernel(float *__restrict__ partials, int n_partials, T *__restrict__ prenorm,
                                                            float *__restrict__ x, float *__restrict__ copy_to,
                                                            const float *__restrict__ w, int K, int a_mt, TokenRows rows) {
-    constexpr int kAhead = 16;
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
     const T *e = nullptr;
@@ -409,21 +409,27 @@ __global__ __launch_bounds__(256) void prenorm_rows_kernel(float *__restrict__ p
         if (copy_to) copy_to[row * K + i] = v;   // the residual stream, when x is the step's input buffer
         Store<T>::st(prenorm + (a_mt ? tiled_a_index((int)row, i, a_mt) : row * K + i), v * nw);
     };
-    float v[kAhead], nw[kAhead];
     const int tid = threadIdx.x;
-    if (e) {
+    const auto take = [&](auto count) {
+        constexpr int kAhead = decltype(count)::value;
+        float v[kAhead], nw[kAhead];
+        if (e) {
 #pragma unroll
-        for (int k = 0; k < kAhead; k++) v[k] = tid + 256 * k < K ? Store<T>::ld(e + tid + 256 * k) : 0.0f;
-    } else {
+            for (int k = 0; k < kAhead; k++) v[k] = tid + 256 * k < K ? Store<T>::ld(e + tid + 256 * k) : 0.0f;
+        } else {
 #pragma unroll
-        for (int k = 0; k < kAhead; k++) v[k] = tid + 256 * k < K ? x[row * K + tid + 256 * k] : 0.0f;
-    }
+            for (int k = 0; k < kAhead; k++) v[k] = tid + 256 * k < K ? x[row * K + tid + 256 * k] : 0.0f;
+        }
 #pragma unroll
-    for (int k = 0; k < kAhead; k++) nw[k] = tid + 256 * k < K ? w[tid + 256 * k] : 0.0f;
+        for (int k = 0; k < kAhead; k++) nw[k] = tid + 256 * k < K ? w[tid + 256 * k] : 0.0f;
 #pragma unroll
-    for (int k = 0; k < kAhead; k++)
-        if (tid + 256 * k < K) put(tid + 256 * k, zero ? 0.0f : v[k], nw[k]);
-    for (int i = tid + 256 * kAhead; i < K; i += 256) put(i, e ? (zero ? 0.0f : Store<T>::ld(e + i)) : x[row * K + i], w[i]);
+        for (int k = 0; k < kAhead; k++)
+            if (tid + 256 * k < K) put(tid + 256 * k, zero ? 0.0f : v[k], nw[k]);
+        for (int i = tid + 256 * kAhead; i < K; i += 256) put(i, e ? (zero ? 0.0f : Store<T>::ld(e + i)) : x[row * K + i], w[i]);
+    };
+    if (K <= 256) take(std::integral_constant<int, 1>());   // (narrow models: 1 us less than past the empty places of sixteen)
+    else if (K <= 1024) take(std::integral_constant<int, 4>());
+    else take(std::integral_constant<int, 16>());
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
