@@ -459,7 +459,7 @@ __global__ __launch_bounds__(256) void prenorm_rows_kernel(float *__restrict__ p
 // projection to the storage type and back, bias, softplus, packing).  Measured per layer, 130m prefill shape (50 MB of
 // delta) / 2.8b shape (168 MB): the row-major product with its LDS transpose and a twelve-slot softplus 21.4 / 94 us; this
 // kernel with the same softplus 21.1 / 93; with softplus20_16 as it is now 20.3 / 84.8; with the row tiles dealt evenly
-// among the workgroups (launch_dt_proj_softplus) 18.7 / 77.2.
+// among the workgroups (launch_dt_proj_softplus) 18.7 / 77.2; dt_rank 160 as five k-steps where it had been padded to six, in the prefill 72.5 -> 69.6.
 template <typename T, int KS, int CT, bool WLDS>
 __global__ __launch_bounds__(256) void dt_proj_softplus_kernel(T *__restrict__ delta, const T *__restrict__ dt_in, int64_t xs,
                                                                const T *__restrict__ wt, const float *__restrict__ bias, int64_t rows,
@@ -688,7 +688,8 @@ int launch_dt_proj_softplus(hipStream_t st, int dtype, void *delta, const void *
         case 2: MRS_DTP(T_, 2); break;                      \
         case 3: MRS_DTP(T_, 3); break;                      \
         case 4: MRS_DTP(T_, 4); break;                      \
-        case 5: case 6: MRS_DTP(T_, 6); break;              \
+        case 5: MRS_DTP(T_, 5); break;                      \
+        case 6: MRS_DTP(T_, 6); break;                      \
         default: MRS_DTP(T_, 8); break;                     \
     }
     if (dtype == MRS_BF16) { MRS_DTP_KS(bf16_t) } else { MRS_DTP_KS(f16_t) }
