@@ -1226,6 +1226,11 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         // on purpose: with B and C in it the 768-wide shape's 3200 columns cost the vendor kernel a third more time
         // than 3072 do.)
         const int nb = 2 * di, ns = ip - nb, nbc = 2 * c.ngroups * ds;
+        // Behind the last layer only the last step of each sequence goes on (below), so its gate and the scan's outputs are formed there alone.  The gate columns and the
+        // other rows of y then hold what they held before.  The gate as a product of its own is a launch of 6 us, so it takes work to be ahead (the line: run_layers
+        // of the Mamba-1 engine).
+        const bool last = l + 1 == L && last_step_gemm_ok(dt, bb->pf_gated, lw.out_proj_t, B, T, dm, di);
+        const int skip = last && (double)rows * di * dm >= 4e9 && lw.in_proj_t && skinny_gemm_ok(dt, B, di, dm, (int64_t)T * dm, bb->pf_normed, lw.in_proj_t) ? di : 0;
         const void *bulk; int64_t ldb; const float *scp, *bcp; int64_t lds_;
         {
             const rocblas_datatype t = blas_type3(dt), f32t = rocblas_datatype_f32_r;
@@ -1238,15 +1243,20 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             } else {
                 // the vendor kernels for the transposed operand are faster at these shapes (the copy's first nb rows, then the rest)
                 if (lw.in_proj_t) {
-                    const char *wt = (const char *)lw.in_proj_t, *wt_rest = wt + (size_t)nb * dm * es;
-                    const BigSplit split = {bb->pf_proj, ns, nb};
+                    const char *wt = (const char *)lw.in_proj_t + (size_t)skip * dm * es, *wt_rest = (const char *)lw.in_proj_t + (size_t)nb * dm * es;
+                    char *out = (char *)bb->pf_bulk + (size_t)skip * es;
+                    const int n1 = nb - skip;
+                    const BigSplit split = {bb->pf_proj, ns, n1};
+                    if (skip)
+                        MRS_TRY(launch_skinny_gemm(bb->stream, dt, (char *)bb->pf_bulk + es * (size_t)(T - 1) * nb, 0, (int64_t)T * nb, (const char *)bb->pf_normed + es * (size_t)(T - 1) * dm,
+                                                   (int64_t)T * dm, lw.in_proj_t, B, di, dm, SkinnyEpi()));
                     // all columns as one product where that is ahead
-                    if (!gemm_tuner_enabled(bb->tuner) && big_gemm_split_wins(rows, nb, ip, dm) && big_gemm_split_ok(dt, bb->pf_bulk, nb, split, bb->pf_normed, dm, wt, rows, ip, dm)) {
-                        MRS_TRY(launch_big_gemm_split(bb->stream, dt, bb->pf_bulk, nb, split, bb->pf_normed, dm, wt, rows, ip, dm));
+                    if (!gemm_tuner_enabled(bb->tuner) && big_gemm_split_wins(rows, n1, ip - skip, dm) && big_gemm_split_ok(dt, out, nb, split, bb->pf_normed, dm, wt, rows, ip - skip, dm)) {
+                        MRS_TRY(launch_big_gemm_split(bb->stream, dt, out, nb, split, bb->pf_normed, dm, wt, rows, ip - skip, dm));
                     } else {
-                        if (const OwnProjection own = own_projection(bb, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm))
-                            MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_bulk, nb, bb->pf_normed, wt, rows, nb, dm));
-                        else MRS_TRY(gemm(1, nb, wt, dm, bb->pf_bulk, t, nb));
+                        if (const OwnProjection own = own_projection(bb, 0, out, nb, bb->pf_normed, wt, rows, n1, dm))
+                            MRS_TRY(launch_own_projection(bb, own, 0, out, nb, bb->pf_normed, wt, rows, n1, dm));
+                        else MRS_TRY(gemm(1, n1, wt, dm, out, t, nb));
                         if (const OwnProjection own = own_projection(bb, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm))
                             MRS_TRY(launch_own_projection(bb, own, 1, bb->pf_proj, ns, bb->pf_normed, wt_rest, rows, ns, dm));
                         else MRS_TRY(gemm(1, ns, wt_rest, dm, bb->pf_proj, f32t, ns));
@@ -1291,7 +1301,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             // pass, and y itself is never written
             gate_in_scan = !c.is_outproj_norm && ldb % 8 == 0;
             const SsdGenArgs gen = {bb->pf_bcn, (const char *)bb->pf_bcn + (size_t)ds * es, 2 * (int64_t)ds, bb->pf_angle, lw.b_bias, lw.c_bias, nr, head_major ? 1 : 0,
-                                    gate_in_scan ? bulk : nullptr, ldb};
+                                    gate_in_scan ? bulk : nullptr, ldb, last};
             const char *xb = (const char *)bulk + (size_t)di * es;
             MRS_TRY(m3_ssd_fwd_ex(bb->stream, dt, ssm, kst, vst, gate_in_scan ? bb->pf_gated : bb->pf_y, xb, ldb, nullptr, nullptr, head_major ? bb->pf_dtT : bb->pf_dt,
                                   head_major ? bb->pf_trapT : bb->pf_trap, head_major ? bb->pf_aT : bb->pf_a, lw.D,
@@ -1312,7 +1322,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             MRS_TRY(mrs_m3_seq_fwd(bb->stream, dt, ssm, kst, vst, bb->pf_y, bb->pf_x, bb->pf_K, bb->pf_Q, al, be, ga, lw.D, B, T, nh, hd, ds));
         }
         if (!gate_in_scan) MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_gate_t<T_>(bb, lw, rows, bulk, ldb)));
-        if (l + 1 == L && last_step_gemm_ok(dt, bb->pf_gated, lw.out_proj_t, B, T, dm, di))
+        if (last)
             MRS_TRY(launch_last_step_gemm(bb->stream, dt, bb->pf_out, bb->pf_gated, lw.out_proj_t, B, T, dm, di));
         else if (const OwnProjection own = own_projection(bb, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
             MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di));

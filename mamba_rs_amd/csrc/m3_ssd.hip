@@ -114,6 +114,7 @@ struct SsdSplit {
     // engine-only extra: y leaves multiplied by silu(z), z rows g_zs elements apart in the storage type (GATE)
     const void *g_z;
     int64_t g_zs;
+    int g_first = 0;      // the first super-chunk whose outputs are wanted
 };
 
 // Cross-lane moves on the data-parallel-primitive path of the vector ALU (no LDS round trip, unlike the shuffle
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(HD * 4) __attribute__((amdgpu_waves_per_eu(HD == 64
     constexpr int NV = (NVEC + NTHR - 1) / NTHR;   // vectors per thread per tile
     __shared__ SsdSmem<HD, DS> sm;
 
-    const int nscg = STATE_ONLY ? sp.nsc - 1 : sp.nsc;   // the state-only pass skips the last super-chunk
+    const int nscg = STATE_ONLY ? sp.nsc - 1 : sp.nsc - (GEN ? sp.g_first : 0);   // the state-only pass skips the last super-chunk
     int b, h, sc;
     if constexpr (GEN) {
         // Workgroups go to the 8 L2 domains of the chip round-robin by index.  The heads of one (batch row, super-chunk)
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(HD * 4) __attribute__((amdgpu_waves_per_eu(HD == 64
         // indices of one residue mod 8, so they meet in one L2.  The grid is padded to whole rounds of 8 groups.
         const int slot = blockIdx.x >> 3, g = (slot / nh) * 8 + (blockIdx.x & 7);
         if (g >= sp.g_groups) return;   // padding: the whole workgroup leaves before any barrier
-        h = slot % nh; b = g / nscg; sc = g - b * nscg;
+        h = slot % nh; b = g / nscg; sc = g - b * nscg + (STATE_ONLY ? 0 : sp.g_first);
     } else {
         const int bhi = blockIdx.x / nscg;
         sc = blockIdx.x - bhi * nscg; b = bhi / nh; h = bhi - b * nh;
@@ -637,7 +638,7 @@ static void launch_ssd_shape(hipStream_t st, float *ssm, float *kst, float *vst,
                 hipLaunchKernelGGL((m3_ssd_kernel<T, HD, DS, true, true>), padded(sp.g_groups), dim3(HD * 4), 0, st,
                                    ssm, kst, vst, (T *)y, (const T *)x, (const T *)K, (const T *)Q, dt, trap, a_val, D, sp, Tlen, nh, carry);
             }
-            sp.g_groups = batch * sp.nsc;
+            sp.g_groups = batch * (sp.nsc - sp.g_first);
             if (sp.g_z)
                 hipLaunchKernelGGL((m3_ssd_kernel<T, HD, DS, false, true, true>), padded(sp.g_groups), dim3(HD * 4), 0, st, ssm, kst, vst,
                                    (T *)y, (const T *)x, (const T *)K, (const T *)Q, dt, trap, a_val, D, sp, Tlen, nh, carry);
@@ -762,7 +763,7 @@ int mrs::m3_ssd_fwd_ex(void *stream, int dtype, float *ssm_state, float *k_state
     // Super-chunk split when the caller's workspace holds it; otherwise one workgroup walks the whole sequence.
     SsdSplit sp = {nullptr, nullptr, nullptr, 1, (T + kCS - 1) / kCS, x_stride, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, nullptr, 0};
     auto with_gen = [&](SsdSplit &o) {
-        if (gen) { o.g_bn = gen->bn; o.g_cn = gen->cn; o.g_ang = gen->angle; o.g_bb = gen->b_bias; o.g_cb = gen->c_bias; o.g_bcs = gen->bc_stride; o.g_nr = gen->n_rope; o.g_head_major = gen->head_major; o.g_z = gen->gate; o.g_zs = gen->gate_stride; }
+        if (gen) { o.g_bn = gen->bn; o.g_cn = gen->cn; o.g_ang = gen->angle; o.g_bb = gen->b_bias; o.g_cb = gen->c_bias; o.g_bcs = gen->bc_stride; o.g_nr = gen->n_rope; o.g_head_major = gen->head_major; o.g_z = gen->gate; o.g_zs = gen->gate_stride; o.g_first = gen->last ? o.nsc - 1 : 0; }
     };
     with_gen(sp);
     {

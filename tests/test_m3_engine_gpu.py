@@ -390,3 +390,28 @@ def test_prefill_projects_the_last_steps_alone_in_its_last_layer(B, T, dtype):
     want = e.prefill_sequence(x[:, T - 8:].copy()).copy()
     e.close()
     assert np.linalg.norm(got - want) <= 1e-2 * np.linalg.norm(want), np.linalg.norm(got - want) / np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("dm,B,T,dtype", [
+    (128, 2, 72, WeightDtype.BF16),     # one super-chunk
+    (256, 1, 521, WeightDtype.F16),     # several, the last chunk of nine steps
+    (768, 1, 1033, WeightDtype.BF16),
+    (768, 4, 900, WeightDtype.BF16),    # the gate as a product of its own
+    (768, 2, 4104, WeightDtype.F16),    # ... and all other columns as one product
+])
+def test_prefill_forms_gate_and_outputs_of_the_last_steps_alone_in_its_last_layer(dm, B, T, dtype):
+    """The same where the scan forms K and Q itself, over one and many super-chunks: against two calls, the second of eight steps, which form everything; the
+    states too.  Tolerance as above."""
+    cfg = Mamba3Config(d_model=dm, d_state=64, expand=2, headdim=64, ngroups=1, n_layers=2, rope_fraction=0.5)
+    w = perturbed(cfg, dm, 19)
+    w.input_proj_w = np.zeros(0, np.float32)
+    x = np.random.default_rng(B + T).standard_normal((B, T, dm)).astype(np.float32)
+    print(f"case m3 last layer {dm} {B}x{T} {dtype}", flush=True)
+    e = GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    got = [e.prefill_sequence(x).copy()] + [p for l in range(2) for p in e.download_state(l)[:3]]
+    e.reset()
+    e.prefill_sequence(x[:, :T - 8].copy())
+    want = [e.prefill_sequence(x[:, T - 8:].copy()).copy()] + [p for l in range(2) for p in e.download_state(l)[:3]]
+    e.close()
+    for p, q in zip(got, want):
+        assert np.linalg.norm(p - q) <= 1e-2 * np.linalg.norm(q), np.linalg.norm(p - q) / np.linalg.norm(q)
