@@ -1230,7 +1230,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         // other rows of y then hold what they held before.  The gate as a product of its own is a launch of 6 us, so it takes work to be ahead (the line: run_layers
         // of the Mamba-1 engine).
         const bool last = l + 1 == L && last_step_gemm_ok(dt, bb->pf_gated, lw.out_proj_t, B, T, dm, di);
-        const int skip = last && (double)rows * di * dm >= 4e9 && lw.in_proj_t && skinny_gemm_ok(dt, B, di, dm, (int64_t)T * dm, bb->pf_normed, lw.in_proj_t) ? di : 0;
+        const int skip = last && (double)rows * di * dm >= 4e9 && !gemm_tuner_enabled(bb->tuner) && lw.in_proj_t && skinny_gemm_ok(dt, B, di, dm, (int64_t)T * dm, bb->pf_normed, lw.in_proj_t) ? di : 0;
         const void *bulk; int64_t ldb; const float *scp, *bcp; int64_t lds_;
         {
             const rocblas_datatype t = blas_type3(dt), f32t = rocblas_datatype_f32_r;
