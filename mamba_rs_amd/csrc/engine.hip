@@ -498,8 +498,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
         const char *xb = (const char *)s->xdbl;
         MRS_TRY(launch_add_rmsnorm(bb, s->residual, l == 0 ? nullptr : s->out, s->normed, false, lw.norm_w, rows, dm));
         // Behind the last layer only the last step of each sequence goes on (below), so its gate and its scan's outputs are formed there alone.  The gate half of
-        // `proj` and the other rows of y then hold what they held before.  The scan's last chunk alone: 16384 x 5120 298 -> 165 us, x 1536 99 -> 60.  The gate as a product
-        // of its own is a launch of 6 us, so it takes work to be ahead (777 x 2048 x 1024, 1.6e9: even; 16384 x 1536 x 768, 19e9: 75 -> 47 us), and not while
+        // `proj` and the other rows of y then hold what they held before.  The scan's last chunk alone: 16384 x 5120 298 -> 94 + 81 us, x 1536 100 -> 35 + 34.  The gate as a product
+        // of its own is a launch of 6 us, so it takes work to be ahead (777 x 2048 x 1024, 1.6e9: even; 16384 x 1536 x 768, 19e9: 73 -> 46 + 6 us), and not while
         // the library's kernels are timed, which would time them for one more shape.
         const bool last = T > 1 && !prefix && l + 1 == L && last_step_gemm_ok(dt, s->y, lw.out_proj_t, B, T, dm, di);
         if (last && (double)rows * di * dm >= 4e9 && !gemm_tuner_enabled(bb->tuner) && lw.in_proj_t && skinny_gemm_ok(dt, B, di, dm, (int64_t)T * dm, s->normed, (const char *)lw.in_proj_t + es * di * dm)) {
