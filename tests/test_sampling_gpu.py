@@ -108,6 +108,26 @@ def test_many_draws_stay_inside_the_filtered_support_and_follow_the_distribution
     assert np.abs(freq - probs[support]).max() < 0.05
 
 
+@pytest.mark.parametrize("vocab", [65536, 65540, 65532, 4099, 132])
+def test_top_k_of_rows_held_in_registers_and_beyond(vocab):
+    """Rows of up to 65536 entries, a multiple of four, stay in registers between the two walks of a draw with top-k up to 128; longer ones and odd lengths are read
+    twice.  The largest entries lie at both ends, with equals on the boundary of k; every draw is checked against the oracle by the rule above."""
+    rng = np.random.default_rng(vocab)
+    row = (rng.standard_normal(vocab) * 2).astype(np.float32)
+    row[-3:], row[:2] = 9.0, 9.0
+    logits = np.repeat(row[None], 24, 0)
+    print(f"case held rows {vocab}", flush=True)
+    for k, top_p in ((3, 1.0), (50, 0.95), (128, 1.0)):
+        p = SampleParams(temperature=0.9, top_k=k, top_p=top_p)
+        tok, state = device_sample(logits, [p] * 24, list(range(24)))
+        off = 0
+        for r in range(24):
+            miss, want_state = check_row(int(tok[r]), logits[r], p, r)
+            off += miss
+            assert tuple(int(v) for v in state[r]) == tuple(int(v) for v in want_state)
+        assert off <= 1, off
+
+
 @pytest.mark.parametrize("shape", ["spread", "ascending", "tied", "short", "crowded"])
 def test_top_k_by_group_maxima_keeps_what_the_search_keeps(shape):
     """top-k up to 128 collects its candidates above a floor taken from the maxima of 256 groups of the row; 129 always searches.
