@@ -545,13 +545,13 @@ __device__ __forceinline__ void advance_slot(const GenAdvance &adv, int i, int n
 
 // logits [rows, ld] f32 are read only; `work` [rows, ld] receives the penalised logits of rows with a penalty.  seen [rows, vocab] counts how often a token sits in the row's seen list (the penalty is applied once per
 // occurrence, sample.rs:100-109).  rng [rows, 4] advances by one draw per sampled row (none on the greedy branch).
-// Rows with active[row] == 0 are left alone.
+// Rows with active[row] == 0 are left alone.  active and seen may be the arrays that advance_slot writes (no __restrict__).
 __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(int *__restrict__ tokens, const float *__restrict__ logits,
                                                                    float *__restrict__ work, int64_t ld, int vocab,
                                                                    const mrs_sampler *__restrict__ samplers,
-                                                                   const unsigned *__restrict__ seen,
+                                                                   const unsigned *seen,
                                                                    unsigned long long *__restrict__ rng,
-                                                                   const int *__restrict__ active, GenAdvance adv) {
+                                                                   const int *active, GenAdvance adv) {
     __shared__ SampShared sh;
     const int rowi = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const auto done = [&](int tok, bool sampled) {
