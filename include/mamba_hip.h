@@ -351,7 +351,8 @@ MRS_API int mrs_backbone_download_state(mrs_backbone *bb, int layer, float *conv
 /* ---- greedy LM loop on top of a backbone ------------------------------------------
  * The decode loop of GpuMambaLM::generate_streaming (src/module/gpu_lm.rs:334-377) with tied
  * embedding / lm_head (gpu_lm.rs:560-679), temperature 0: next token = last index of the maximum
- * logit (src/module/sample.rs:250-257).  Unlike the reference the embedding gather and the argmax
+ * logit (src/module/sample.rs:250-257); NaN is passed over, and a row with nothing above -inf gives vocab - 1.
+ * Unlike the reference the embedding gather and the argmax
  * run on the device, so a decode step needs no host round trip.
  *   embed: [vocab, d_model] f32 on the host (rows >= vocab of the 64-padded table are zero). */
 typedef struct mrs_lm mrs_lm;

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(float *__restrict__ o
 // launch that left 32 partial maxima per row and a second one over those, 4.9 + 4.0 us in a graph at one row, this 4.0; 5.4 + 4.1 at 64, this 6.0; 5.0 + 4.0 at 16, this 4.7.)  The
 // meeting is what many rows cost: a line per row, and longer slices (eight rows to a line, slices of 2048: 6.9 us at 16 rows, 8.1 at 64).
 struct alignas(128) ArgRow { unsigned long long key; unsigned arrived; };
-template <int V> __global__ __launch_bounds__(256) void argmax_kernel(int *__restrict__ tokens, ArgRow *__restrict__ rows, const float *__restrict__ logits, int vocab, int64_t stride, int none) {
+template <int V> __global__ __launch_bounds__(256) void argmax_kernel(int *__restrict__ tokens, ArgRow *__restrict__ rows, const float *__restrict__ logits, int vocab, int64_t stride) {
     __shared__ unsigned long long part[4];
     constexpr int slice = 1024 * V;
     const int slices = (vocab + slice - 1) / slice, row = blockIdx.x / slices, tid = threadIdx.x;
@@ -135,7 +135,7 @@ template <int V> __global__ __launch_bounds__(256) void argmax_kernel(int *__res
         const int i = i0 + 1024 * (k >> 2) + (k & 3);
         if (i < vocab && v[k] >= best) { best = v[k]; bi = i; }   // ascending: >= keeps the last maximum
     }
-    if (best == -INFINITY) bi = max(bi, none);   // nothing above it in the row (or NaN throughout)
+    if (best == -INFINITY) bi = vocab - 1;   // the last of its equals where the row has nothing above it (NaN is passed over)
     const unsigned bits = __float_as_uint(best + 0.0f);   // (the two zeros are equal)
     unsigned long long key = (unsigned long long)((bits & 0x80000000u) ? ~bits : (bits | 0x80000000u)) << 32 | (unsigned)bi;
 #pragma unroll
@@ -1318,10 +1318,9 @@ static int lm_logits(mrs_lm *lm) {
 
 static int lm_argmax(mrs_lm *lm) {
     hipStream_t st = lm->eng.stream;
-    const int per = (lm->vocab + 31) / 32;
     const auto pick = [&](auto kernel, int slice) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)((lm->vocab + slice - 1) / slice * lm->batch)), dim3(256), 0, st, lm->tokens, lm->arg_rows, lm->logits, lm->vocab,
-                           (int64_t)lm->vocab_padded, std::min(31 * per, lm->vocab - 1));
+                           (int64_t)lm->vocab_padded);
     };
     if (lm->batch < 8) pick(argmax_kernel<2>, 2048);
     else pick(argmax_kernel<8>, 8192);

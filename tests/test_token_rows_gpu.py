@@ -92,3 +92,44 @@ def test_the_greedy_token_is_the_last_of_the_largest(V, B):
             got, logits = lm.get_tokens(), lm.last_logits()
             assert (got == V - 1 - logits[:, ::-1].argmax(1)).all()
         bb.close()
+
+
+@pytest.mark.parametrize("V,B", [(1, 3), (7, 3), (2049, 3), (5000, 8), (8193, 8), (20001, 8)])
+def test_the_greedy_token_of_rows_with_masks_infinities_and_nan(V, B):
+    """Head columns that make a logit -inf, inf or NaN in every row: the last of the largest numbers, NaN passed over, and the vocabulary's last entry where
+    nothing is above -inf (Iterator::max_by keeps the later of two that do not compare).  Masked columns take a row's positive entry times -inf,
+    all other terms of the sum being zero."""
+    dm = 64
+    cfg, w, backbone, lm_kind = _model("m1", dm, 1)
+    rng = np.random.default_rng(V)
+    embed = rng.standard_normal((V, dm)).astype(np.float32)
+    tokens = np.arange(B, dtype=np.int32) % min(V, 3)
+    plain = backbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.F32)
+    rows = plain.step(embed[tokens])
+    plain.close()
+    k = int(rows.min(0).argmax())
+    assert rows[:, k].min() > 0
+    head = rng.standard_normal((dm, V)).astype(np.float32)
+    low, high, nan = np.zeros(dm, np.float32), np.zeros(dm, np.float32), np.full(dm, np.nan, np.float32)
+    low[k], high[k] = -np.inf, np.inf
+
+    def some(*columns):   # most columns of the first kind, a few numbers or other kinds among them
+        h = np.tile(columns[0][:, None], (1, V))
+        for i, c in enumerate(columns[1:]):
+            at = rng.integers(0, V, 1 + V // 50)
+            h[:, at] = head[:, at] if c is None else c[:, None]
+        return h
+    for what, lm_head in (("-inf", some(low)), ("nan", some(nan)), ("-inf and nan", some(low, nan)), ("nan and -inf", some(nan, low)), ("-inf, numbers", some(low, None)),
+                          ("nan, numbers", some(nan, None)), ("nan, numbers, -inf", some(nan, None, low)), ("-inf, inf, nan", some(low, high, nan))):
+        print(f"case greedy vocab={V} rows={B}: {what}", flush=True)
+        bb = backbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.F32)
+        lm = lm_kind(bb, embed, lm_head)
+        for _ in range(3):
+            bb.reset()
+            lm.set_tokens(tokens)
+            lm.decode_step()
+            got, logits = lm.get_tokens(), lm.last_logits()
+            assert (np.isnan(logits) == np.isnan(lm_head).any(0)).all() and (np.isneginf(logits) == np.isneginf(lm_head).any(0)).all()
+            v = np.where(np.isnan(logits), -np.inf, logits)
+            assert (got == V - 1 - v[:, ::-1].argmax(1)).all(), (what, got)
+        bb.close()
