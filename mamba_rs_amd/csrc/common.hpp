@@ -270,9 +270,7 @@ int launch_resident_m3_step(hipStream_t st, int dtype, const ResidentM3Args &a, 
 // wp, the tiled copy of x_proj (launch_tile_weight); state as mrs_conv1d_seq_silu
 bool conv_xproj_ok(int dtype, const void *u, const void *xdbl, const float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
                    int di, int dc, int xd);
-bool conv_xproj_wins(int batch, int T, int xd);
-// the same for few rows: shares, the room that conv_xproj_slices() (two or more) times the size of xdbl in f32 takes, at most that of u
-int conv_xproj_slices(int batch, int T, int di, int xd);
+// the same where conv_xproj_form() (size_rules.hpp) says two or more slices: shares, room for that many times the size of xdbl in f32, at most that of u
 int launch_conv_xproj_sliced(hipStream_t st, int dtype, void *u, void *xdbl, float *shares, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias,
                              int batch, int T, int di, int xd);
 int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,

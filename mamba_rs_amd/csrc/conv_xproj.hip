@@ -4,24 +4,24 @@
 // kernels/conv1d.cu:209-315).  As two launches the conv moves x in and u out, and the GEMM, whose result is a few dozen columns, waits for u to
 // come back.  Here a workgroup owns 32 or 64 steps of a sequence and all columns of the x_proj rows, and walks the channels 64 at a time.
 //   * x (with the eight rows in front of the first step), x_proj's rows in matrix-operand order, taps, biases and the carried window go from memory straight to
-//     LDS, three or five pieces of 64 channels ahead of their use.
+//     LDS, three to five pieces of 64 channels ahead of their use.
 //   * Sixteen waves: eight form u of a piece from x, two channels and a few steps a lane; four request the pieces to come and multiply the piece before by
 //     x_proj's rows; four store it.  One barrier per piece: behind it u of the piece is there for the products and the stores, the next
 //     piece's operands are in LDS, and the place of the piece before is free for a request.
 //   * u lies in LDS as the matrix instructions take it, a row's 16-byte piece p at place p ^ (row / 2 % 8), so that neither their reads nor the
-//     stores' meet on banks; its sums are the conv kernel's, term by term.
+//     stores' meet on banks; its sums are the conv kernel's, term by term (and u its bits, but for one f16 value in 4000 that the compiler rounds by way of f32 here).
 // Bound by the exponentials and divisions of SiLU (about 12 us of 16384 x 1536) and by x and u, 100 MB there (20 us at the rate of a copy).  16384 rows,
 // two launches / this: d_inner 1536, 80 columns 23.0 + 23.2 / 28.3 us; 5120, 192 columns 72.7 + 69.8 / 114, where every unit takes in all of x_proj (2 MB).  As
 // eight waves that all do everything, and so wait for their own LDS reads in front of each other's arithmetic: 39 at d_inner 1536.
 #include "common.hpp"
 #include "mfma_tiles.hpp"
-#include <algorithm>
+#include "size_rules.hpp"
 
 namespace mrs {
 namespace {
 
 constexpr int kConvWaves = 8, kMoveWaves = 4, kStoreWaves = 4, kConvThreads = 64 * (kConvWaves + kMoveWaves + kStoreWaves);
-constexpr int kPiece = 64;   // channels of a piece
+constexpr int kPiece = kConvPiece;   // channels of a piece
 
 struct ConvXprojArgs {
     void *u, *xdbl;
@@ -224,44 +224,31 @@ __global__ __launch_bounds__(kConvThreads) void conv_xproj_kernel(ConvXprojArgs 
     }
 }
 
-template <typename T, int ROWS, int NT, int S>
+template <typename T, int ROWS, int NT>
 int launch_conv_xproj_t(hipStream_t st, const ConvXprojArgs &g, int batch) {
-    constexpr size_t stage = (ROWS + 8) * 128 + 3 * 1024 + 2 * NT * 1024, lds = S * stage + 2 * ROWS * 128;
-    static_assert(lds <= 160 * 1024, "");
+    constexpr size_t stage = (ROWS + 8) * 128 + 3 * 1024 + 2 * NT * 1024, ut = 2 * ROWS * 128;
+    constexpr int S = std::min<int>((160 * 1024 - ut) / stage, 6);
+    constexpr size_t lds = S * stage + ut;
     static const hipError_t attr = hipFuncSetAttribute((const void *)conv_xproj_kernel<T, ROWS, NT, S>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "conv + x_proj: LDS size: %s", hipGetErrorString(attr));
     hipLaunchKernelGGL((conv_xproj_kernel<T, ROWS, NT, S>), dim3((unsigned)(batch * g.tiles * g.slices)), dim3(kConvThreads), lds, st, g);
     return check_launch("conv_xproj_kernel");
 }
-template <typename T>
+template <typename T, int NT = kConvMinTiles>
 int launch_conv_xproj_n(hipStream_t st, const ConvXprojArgs &g, int batch, int rows) {
-    switch ((g.xd + 15) / 16 * 100 + rows) {
-        case 564: return launch_conv_xproj_t<T, 64, 5, 6>(st, g, batch);
-        case 664: return launch_conv_xproj_t<T, 64, 6, 6>(st, g, batch);
-        case 1264: return launch_conv_xproj_t<T, 64, 12, 4>(st, g, batch);
-        case 532: return launch_conv_xproj_t<T, 32, 5, 6>(st, g, batch);
-        case 632: return launch_conv_xproj_t<T, 32, 6, 6>(st, g, batch);
-        default: return launch_conv_xproj_t<T, 32, 12, 4>(st, g, batch);
-    }
+    if constexpr (NT < kConvMaxTiles)
+        if (conv_xproj_col_tiles(g.xd) > NT) return launch_conv_xproj_n<T, NT + 1>(st, g, batch, rows);
+    return rows == 64 ? launch_conv_xproj_t<T, 64, NT>(st, g, batch) : launch_conv_xproj_t<T, 32, NT>(st, g, batch);
 }
-// Steps of a workgroup: 32 as long as those are about one round over the compute units, else 64, which read x_proj's rows half as often (four layers of a
-// bf16 prefill, in us, two launches / 64 / 32: d_model 768, 4000 rows 646 / 645 / 621, 8 x 1000 823 / 814 / 783, 6 x 2000 1105 / 1052 / 1069, 8 x 2048
-// 1356 / 1276 / 1287; 2560, 8000 rows 3305 / 3266 / 3221, 4 x 4096 6036 / 5887 / 6038).
-int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
 
 }  // namespace
 
 bool conv_xproj_ok(int dtype, const void *u, const void *xdbl, const float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
                    int di, int dc, int xd) {
-    return (dtype == MRS_BF16 || dtype == MRS_F16) && dc == 4 && di % kPiece == 0 && di >= 2 * kPiece && T >= 4 && xd % 4 == 0 && ((xd + 15) / 16 == 5 || (xd + 15) / 16 == 6 || (xd + 15) / 16 == 12) && x_stride % 8 == 0 && wp &&
+    return (dtype == MRS_BF16 || dtype == MRS_F16) && dc == 4 && di % kPiece == 0 && di >= 2 * kPiece && T >= 4 && conv_xproj_columns_ok(xd) && x_stride % 8 == 0 && wp &&
            x_stride >= di && (int64_t)T * x_stride < (int64_t)1 << 30 && (int64_t)batch * ((T + 31) / 32) < (int64_t)1 << 30 && aligned(u, 16) && aligned(xdbl, 8) && aligned(state, 16) &&
            aligned(x, 16) && aligned(wp, 16) && aligned(w, 16) && aligned(bias, 4);
 }
-
-// A workgroup walks all channels however few there are (32 steps of d_inner 1536 in about 15 us), so it takes a share of the chip to be ahead; wide models' rows
-// of x_proj have more to read per step (as above, two launches / this: d_model 768, 1500 rows 427 / 433, 2000 490 / 478, 3000 565 / 548; 1024,
-// 777 rows 400 / 420, 2000 578 / 556; 2560, 2000 rows 1183 / 1262, 4000 1980 / 1934).
-bool conv_xproj_wins(int batch, int T, int xd) { return (int64_t)batch * ((T + 31) / 32) >= (xd <= 96 ? 52 : 110); }
 
 int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias, int batch, int T,
                       int di, int xd) {
@@ -271,25 +258,17 @@ int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *sta
     return dtype == MRS_BF16 ? launch_conv_xproj_n<bf16_t>(st, g, batch, rows) : launch_conv_xproj_n<f16_t>(st, g, batch, rows);
 }
 
-// Fewer rows: the channels in slices as well, for about one workgroup per compute unit, whose products are summed in f32, in the order of the slices, by a second launch.  The
-// shares fit in as many bytes as u has.  At 777 x 2048, 96 columns: conv 5.4, x_proj 8.0 as two launches, here 6.3 + 3.7 us.  Four layers of a bf16 prefill, two
-// launches / this: d_model 768, 500 rows 272 / 276, 1000 rows 322 / 317, 1500 rows 384 / 376; 1024, 300 rows even, 777 rows 364 / 353; 2560, 300 rows even, 1000 rows 847 / 811, 2000 rows
-// 1150 / 1113, 4 x 700 1560 / 1429.
-constexpr int kMaxSlices = 16;
-int conv_xproj_slices(int batch, int T, int di, int xd) {
-    const int64_t tiles = (int64_t)batch * ((T + 31) / 32);
-    return tiles < 24 ? 1 : (int)std::min<int64_t>(std::min(std::min(di / (2 * xd), di / kPiece / 2), kMaxSlices), 256 / tiles);
-}
-
+// Fewer rows: the channels in slices as well, whose products are summed in f32, in the order of the slices, by a second launch.  At 777 x 2048, 96 columns: conv 5.4, x_proj 8.0 us
+// as two launches, here 6.3 + 3.4.
 template <typename T> static __global__ __launch_bounds__(256) void conv_xproj_sum_kernel(T *__restrict__ out, const float *__restrict__ shares, int slices, int64_t n4) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
     const v4f *p = reinterpret_cast<const v4f *>(shares) + i;
-    v4f v[kMaxSlices], s = {0.f, 0.f, 0.f, 0.f};
+    v4f v[kConvMaxSlices], s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < kMaxSlices; k++) v[k] = p[min(k, slices - 1) * n4];   // all asked for at once
+    for (int k = 0; k < kConvMaxSlices; k++) v[k] = p[min(k, slices - 1) * n4];   // all asked for at once
 #pragma unroll
-    for (int k = 0; k < kMaxSlices; k++)
+    for (int k = 0; k < kConvMaxSlices; k++)
         if (k < slices) s += v[k];
     struct alignas(4 * sizeof(T)) T4 { T v[4]; } o;
 #pragma unroll
@@ -299,7 +278,7 @@ template <typename T> static __global__ __launch_bounds__(256) void conv_xproj_s
 
 int launch_conv_xproj_sliced(hipStream_t st, int dtype, void *u, void *xdbl, float *shares, float *state, const void *x, int64_t x_stride, const void *wp, const float *w, const float *bias,
                              int batch, int T, int di, int xd) {
-    const int slices = conv_xproj_slices(batch, T, di, xd);
+    const int slices = conv_xproj_form(batch, T, di, xd);
     if (!conv_xproj_ok(dtype, u, xdbl, state, x, x_stride, wp, w, bias, batch, T, di, 4, xd) || slices < 2 || !aligned(shares, 16))
         return fail(MRS_E_SHAPE, "conv + x_proj in slices: shape outside the route (T=%d d_inner=%d columns=%d)", T, di, xd);
     const int pieces = (di / kPiece + slices - 1) / slices;

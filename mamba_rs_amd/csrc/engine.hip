@@ -22,6 +22,7 @@
 #include "gemm_tune.hpp"
 #include "host_io.hpp"
 #include "scan_quad.hpp"
+#include "size_rules.hpp"
 #include <rocblas/rocblas.h>
 #include <stdlib.h>
 #include <new>
@@ -539,13 +540,12 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
                                               xb + es * (dr + ds), xd, z, 2 * di, 2, lw.a_neg, lw.D, B, di, ds));
             }
         } else {
-            const bool one_ok = !prefix && conv_xproj_ok(dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, dc, xd);
-            const bool one = one_ok && conv_xproj_wins(B, T, xd);
-            const bool sliced = one_ok && !one && conv_xproj_slices(B, T, di, xd) >= 2;   // (the shares where delta comes later)
-            if (sliced) MRS_TRY(launch_conv_xproj_sliced(bb->stream, dt, s->u, s->xdbl, (float *)s->delta, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, xd));
-            else if (one) MRS_TRY(launch_conv_xproj(bb->stream, dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, xd));
+            const int form = !prefix && conv_xproj_ok(dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, dc, xd) ? conv_xproj_form(B, T, di, xd) : 0;
+            if (form >= 2)   // (the shares where delta comes later)
+                MRS_TRY(launch_conv_xproj_sliced(bb->stream, dt, s->u, s->xdbl, (float *)s->delta, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, xd));
+            else if (form) MRS_TRY(launch_conv_xproj(bb->stream, dt, s->u, s->xdbl, conv, s->proj, 2 * di, lw.x_proj_p, lw.conv_w, lw.conv_b, B, T, di, xd));
             else MRS_TRY(mrs_conv1d_seq_silu(bb->stream, dt, s->u, conv, s->proj, 2 * di, lw.conv_w, lw.conv_b, B, T, di, dc));
-            if (one || sliced) {
+            if (form) {
             } else if (own_xproj(lw, rows, xd)) {
                 SkinnyEpi xp = {};
                 xp.w_tiled = 1; xp.any_rows = 1;

@@ -1,0 +1,45 @@
+// Rules on sizes alone that choose a route, in plain C++ (tests compile them without a GPU).
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace mrs {
+
+// conv1d + SiLU and x_proj of a prefill as one launch (conv_xproj.hip).  Columns of x_proj in tiles of 16: from three (33 columns, the fewest of d_state 16) to
+// twelve, which leave room for four pieces of 64 channels in LDS, the fewest that keep requests ahead of their use.
+constexpr int kConvPiece = 64, kConvMinTiles = 3, kConvMaxTiles = 12, kConvMaxSlices = 16;
+inline int conv_xproj_col_tiles(int xd) { return (xd + 15) / 16; }
+inline bool conv_xproj_columns_ok(int xd) { return xd % 4 == 0 && conv_xproj_col_tiles(xd) >= kConvMinTiles && conv_xproj_col_tiles(xd) <= kConvMaxTiles; }
+
+// 0: two launches; 1: a workgroup has all channels of its steps; two or more: the channels in so many slices as well, for about one workgroup per compute unit, whose
+// products a second launch sums.  In tiles of 32 steps.  Up to half a round of tiles the slices are ahead, as a workgroup that walks all channels takes its time however few
+// there are; models of less than 1024 channels have little to share out.  Nine and eleven column tiles cost what ten and twelve do (a wave has half of
+// them) and need most of a round.  Four layers of a bf16 prefill, two launches / slices / all channels, us:
+//   d_model 256   32 tiles 231 / 227 / 224    64 275 / 273 / 261    128 338 / 315 / 307    200 415 / - / 393
+//           448   32 301 / 297 / 300          64 348 / 346 / 342    128 498 / 481 / 474    200 655 / - / 624
+//           512   32 263 / 266 / 274          64 328 / 326 / 331    128 474 / 459 / 456    200 590 / - / 564
+//           640   24 273 / 276 / 289          64 413 / 395 / 401    128 559 / 542 / 541    200 700 / - / 665
+//           768   32 318 / 312 / 332          64 436 / 414 / 430    128 602 / 585 / 581    200 792 / - / 766
+//          1024   24 351 / 337 / 370          64 565 / 522 / 545    128 781 / 741 / 752    144 809 / - / 781
+//          1280   24 396 / 380 / 432          64 658 / 628 / 670    128 900 / 874 / 895    144 1043 / - / 1037
+//          1536   24 453 / 437 / 508          64 759 / 711 / 767    128 1105 / 1068 / 1100 144 1185 / - / 1170
+//          1792   24 513 / 495 / 606          64 826 / 782 / 867    128 1217 / 1182 / 1224 144 1379 / - / 1375  200 1928 / - / 1864
+//          2048   24 559 / 543 / 684          64 923 / 869 / 965    128 1493 / 1359 / 1404 144 1697 / - / 1624
+//          2304   24 678 / 630 / 794          64 1079 / 1028 / 1160 128 1724 / 1684 / 1758 168 2057 / - / 2078  200 2340 / - / 2287
+//          2560   24 725 / 688 / 856          64 1162 / 1119 / 1262 128 1941 / 1823 / 1909 144 2176 / - / 2113
+inline int conv_xproj_form(int batch, int T, int di, int xd) {
+    const int64_t tiles = (int64_t)batch * ((T + 31) / 32);
+    const int columns = conv_xproj_col_tiles(xd);
+    if (tiles > 128) return columns > 8 && columns % 2 && tiles < 192 ? 0 : 1;
+    if (di < 1024) return tiles >= 64 ? 1 : 0;
+    if (tiles < 24 || tiles * di < 40 * 1024) return 0;
+    // (the shares fit in as many bytes as u has, and a slice has two pieces)
+    const int slices = (int)std::min<int64_t>(std::min(std::min(di / (2 * xd), di / kConvPiece / 2), kConvMaxSlices), 256 / tiles);
+    return slices >= 2 ? slices : 0;
+}
+// Steps of a workgroup with all channels: 32 as long as those are about one round over the compute units, else 64, which read x_proj's rows half as
+// often (as above, 64 / 32: d_model 768, 8 x 1000 814 / 783, 6 x 2000 1052 / 1069, 8 x 2048 1276 / 1287; 1536, 8 x 1000 1702 / 1683, 8 x 2048 2953 / 3003; 2560, 8000 rows
+// 3266 / 3221, 4 x 4096 5887 / 6038).
+inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
+
+}  // namespace mrs

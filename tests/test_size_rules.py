@@ -1,0 +1,56 @@
+"""Rules on sizes that choose a route (csrc/size_rules.hpp), compiled by the host compiler.  No GPU."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "mamba_rs_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """rules("expression", args): the expression for every line of arguments a, b, c, d."""
+    folder = tmp_path_factory.mktemp("rules")
+
+    def run(expression, lines):
+        exe, src = str(folder / "main"), str(folder / "main.cpp")
+        with open(src, "w") as f:
+            f.write(f'#include "size_rules.hpp"\n#include <cstdio>\nusing namespace mrs;\n'
+                    f'int main() {{ long a, b, c, d; while (scanf("%ld %ld %ld %ld", &a, &b, &c, &d) == 4) printf("%ld\\n", (long)({expression})); }}\n')
+        subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, "-o", exe, src], check=True)
+        text = "".join(" ".join(map(str, line)) + "\n" for line in lines)
+        return [int(v) for v in subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split()]
+    return run
+
+
+def _columns(dm, ds=16):
+    return (dm + 15) // 16 + 2 * ds
+
+
+def test_conv_and_x_proj_are_one_launch_at_every_width_that_fits(rules):
+    """Default hyperparameters, d_model 256 to 2560 in steps of 64: a prefill of many rows takes the one launch, one of some hundred rows of a model with enough
+    channels has them in slices, and short ones keep two launches."""
+    dims = range(256, 2561, 64)
+    assert rules("conv_xproj_columns_ok(a)", [(_columns(dm), 0, 0, 0) for dm in dims]) == [1] * len(dims)
+    assert rules("conv_xproj_columns_ok(a)", [(xd, 0, 0, 0) for xd in (32, 33, 34, 194, 196, 208)]) == [0] * 6
+    assert rules("conv_xproj_columns_ok(a)", [(xd, 0, 0, 0) for xd in (36, 48, 52, 188, 192)]) == [1] * 5
+    form = "conv_xproj_form(a, b, c, d)"
+    for B, T in ((8, 2048), (4, 4096), (1, 7000), (300, 5)):
+        assert rules(form, [(B, T, 2 * dm, _columns(dm)) for dm in dims]) == [1] * len(dims)
+    assert all((f >= 2) == (dm >= 512) and f for dm, f in zip(dims, rules(form, [(2, 1664, 2 * dm, _columns(dm)) for dm in dims])))
+    assert rules(form, [(1, 300, 2 * dm, _columns(dm)) for dm in dims]) == [0] * len(dims)
+
+
+def test_slices_of_the_channels_fit_their_room_and_the_chip(rules):
+    """The shares of x_proj's products in f32 take at most the bytes of u in 16 bits, a slice has at least two pieces of channels but perhaps the last, and all workgroups
+    run at once."""
+    lines = [(1, 32 * tiles - 7, 2 * dm, _columns(dm, ds)) for ds in (8, 16, 32, 64) for dm in range(128, 2561, 32) for tiles in range(1, 131)
+             if _columns(dm, ds) % 4 == 0 and 33 <= _columns(dm, ds) <= 192]
+    forms = rules("conv_xproj_form(a, b, c, d)", lines)
+    sliced = 0
+    for (_, T, di, xd), f in zip(lines, forms):
+        if f >= 2:
+            sliced += 1
+            assert f <= 16 and f * xd * 4 <= di * 2 and f * ((T + 31) // 32) <= 256 and di // 64 >= 2 * f, (T, di, xd, f)
+    assert sliced > 1000
