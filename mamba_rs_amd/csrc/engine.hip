@@ -429,7 +429,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         const bool step_sums = xpart && xd <= 256 && lw.dt_t_step && di % (1024 / ds) == 0 && dr % 4 == 0 && (int64_t)nr * dr <= fuse_limit;
         const int ksplit = (!fold_x && step_sums && dt != MRS_F32) ? xproj_slices(nr, xd, di) : 1;
         StepFold fold = {xpart, fold_x ? di / 16 : ksplit, nr, xd, dr, dr + ds, 0, nullptr, 0, 0};
-        if (a_mt && bb->wide && (int64_t)dm * di < (int64_t)1 << 30 && dm / 16 % tiled_gemm_unit(dm) == 0) {   // the step kernel asks for out_proj's lines while it waits for its states
+        if (a_mt && bb->wide && asks_out_proj_ahead((int64_t)es * dm * di, nr) && dm / 16 % tiled_gemm_unit(dm) == 0) {   // the step kernel asks for out_proj's lines while it waits for its states
             const int unit = tiled_gemm_unit(dm);
             fold.next = lw.out_proj_p; fold.next_units = (dm / 16 + unit - 1) / unit; fold.next_bytes = unit * (di / 32) * 1024;
         }

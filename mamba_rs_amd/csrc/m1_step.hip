@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(
         }
     }
     // Lines of the weight that the launch behind streams, a dword of each to LDS nobody reads, behind this kernel's own requests.  The units of one die (workgroup
-    // index modulo 8) ask for the pieces that units of the same die will read: their L2 then has them.  16 rows of the 2.8b shape: this kernel 8.4 -> 11.5 us,
+    // index modulo 8) ask for the pieces that units of the same die will read: their L2 then has them (where they fit: asks_out_proj_ahead).  16 rows of the 2.8b shape: this kernel 8.4 -> 11.5 us,
     // out_proj (26 MB) 10.2 -> 5.9; a step of eight layers at 3, 8, 16, 24, 32, 40 rows 280 / 306 / 334 / 391 / 401 / 458 -> 275 / 299 / 325 / 383 / 389 / 438 (small head); half of them here, or some in the x_proj launch in front, or in_proj's in
     // out_proj's, gave back what they took.
     if constexpr (FOLD && PRE == 12) {

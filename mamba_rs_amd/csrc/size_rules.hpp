@@ -42,4 +42,10 @@ inline int conv_xproj_form(int batch, int T, int di, int xd) {
 // 3266 / 3221, 4 x 4096 5887 / 6038).
 inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
 
+// Decode of wide models: whether the step kernel asks for the lines of out_proj (`bytes` of them) on the dies that will read them (m1_step.hip).  They have to stay in the dies' L2, eight
+// of 4 MB, until the launch behind: more than that is read twice, and then many rows' worth of work must cover it.  Eight layers, bf16, us a step, without / with:
+// 25 MB (d_model 2560) 4 rows 284 / 285, 8 304 / 297, 16 330 / 320, 40 454 / 433; 30 MB (2816) 314 / 317, 333 / 328, 367 / 356, 586 / 586; 36 MB (3072) 329 / 338, 351 / 351,
+// 390 / 382, 522 / 521; 42 MB (3328) 379 / 398, 410 / 428, 465 / 468; 49 MB (3584) 405 / 429, 444 / 457, 499 / 504.  (Asking for the part that would fit: behind both everywhere.)
+inline bool asks_out_proj_ahead(int64_t bytes, int rows) { return bytes <= (int64_t)(rows < 8 ? 28 : 40) << 20; }
+
 }  // namespace mrs

@@ -334,3 +334,26 @@ def test_m3_24_heads_4x4096_both_K_Q_routes_agree(m3w, monkeypatch):
     assert np.array_equal(fa[1][3], se[1][3])
     for a, b in zip(fa[2][:3], se[2][:3]):
         assert cosine(a.ravel(), b.ravel()) >= 0.99
+
+
+@pytest.mark.parametrize("B", [7, 8])
+def test_decode_steps_follow_the_cpu_route_where_out_proj_outgrows_the_l2(B):
+    """d_model 3072, out_proj 36 MB of the eight dies' 32 MB of L2: seven rows leave its lines to the launch that multiplies by them, from eight on the step kernel asks for
+    them ahead.  The bounds are those of the 2.8b-shape steps."""
+    dm = 3072
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.random_lm(cfg, seed=31, std=0.02)
+    P = lm_oracle(cfg, w)
+    print(f"case 3072-wide decode batch {B}", flush=True)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.BF16)
+    x = orc.round_to(np.random.default_rng(B).standard_normal((3, B, dm)).astype(np.float32), orc.BF16)
+    st = {b: orc.m1_zero_state(P) for b in (0, B - 1)}
+    for t in range(3):
+        got = eng.step(x[t])
+        for b in st:
+            want = orc.m1_backbone_step(P, x[t, b], *st[b], identity_proj=True)
+            assert cosine(got[b], want) >= COS, (t, b, cosine(got[b], want))
+    for b in st:
+        s, r = ssm_of(eng, 0, b), st[b][1][0].reshape(2 * dm, 16)
+        assert cosine(s, r) >= COS and scaled_err(s, r) < 5e-2, (b, cosine(s, r), scaled_err(s, r))
+    eng.close()

@@ -54,3 +54,11 @@ def test_slices_of_the_channels_fit_their_room_and_the_chip(rules):
             sliced += 1
             assert f <= 16 and f * xd * 4 <= di * 2 and f * ((T + 31) // 32) <= 256 and di // 64 >= 2 * f, (T, di, xd, f)
     assert sliced > 1000
+
+
+def test_out_proj_is_asked_for_ahead_only_where_it_stays_in_the_l2(rules):
+    """Eight dies have 4 MB of L2 each: few rows ask ahead for what fits, many also where it is a little more, and nobody for much more."""
+    ahead = [(2 * dm * 2 * dm, rows) for rows in (3, 4, 8, 16, 64) for dm in (1536, 2048, 2560, 2816, 3072, 3328, 3584)]
+    want = [nbytes <= (28 if rows < 8 else 40) * 2 ** 20 for nbytes, rows in ahead]
+    assert rules("asks_out_proj_ahead(a, (int)b)", [(nbytes, rows, 0, 0) for nbytes, rows in ahead]) == want
+    assert not any(w for w, (nbytes, _) in zip(want, ahead) if nbytes > 40 * 2 ** 20) and all(w for w, (nbytes, _) in zip(want, ahead) if nbytes <= 25 * 2 ** 20)
