@@ -259,7 +259,7 @@ int launch_conv_xproj(hipStream_t st, int dtype, void *u, void *xdbl, float *sta
 }
 
 // Fewer rows: the channels in slices as well, whose products are summed in f32, in the order of the slices, by a second launch.  At 777 x 2048, 96 columns: conv 5.4, x_proj 8.0 us
-// as two launches, here 6.3 + 3.4.
+// as two launches, here 6.2 + 3.3.
 template <typename T> static __global__ __launch_bounds__(256) void conv_xproj_sum_kernel(T *__restrict__ out, const float *__restrict__ shares, int slices, int64_t n4) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;

@@ -10,7 +10,8 @@
 //     (the lanes fetch permuted pieces of the same line: the copy itself writes in lane order);
 //   * a k-step is four quarters of the tile.  The waves are two groups, one barrier apart: while one group's four waves, one per SIMD, multiply a
 //     quarter, the other's read the operands of theirs from LDS and request what the step after next needs in the places both have read.
-// It is bound by power: at these sizes the card runs at 1.7 to 1.9 GHz with the matrix cores busy 70 to 78 % of the time.  Alone, bf16, the
+// Over a long K it is bound by the clock that the card holds under it: 16384 x 2560 x 5120 in a prefill runs at 1.72 to 1.85 GHz, where the kernels beside it have 2.0 to 2.3, with the matrix cores
+// busy 74 % of the cycles at least.  Over a short one the ends of the rounds count: 16384 x 3288 x 768, 2.75 rounds of twelve k-steps, 41 to 46 %.  Alone, bf16, the
 // library's (torch's copy) / this: 16384 x 2560 x 5120 425 / 284 us, 8000 x 2560 x 5120 161 / 142, 4000 x 10240 x 2560 242 / 149, 2000 x 10240 x 2560 102 / 76,
 // 6000 x 3072 x 768 48 / 28, 12000 x 3072 x 768 79 / 54; but 16384 x 10240 x 2560 561 / 598, 16384 x 3072 x 768 67 / 70, 8192 cubed 694 / 738.
 // Also measured, at 16384 x 3072 x 768 and 8192 cubed with tiles of 256 columns (this: 71, 738): two halves per k-step instead of four quarters 71, 755; the halves of A in turn, which evens

@@ -377,8 +377,8 @@ template <typename W> __device__ int ordered_find(const Row &row, W w, double ta
 // into few groups (an ascending vocabulary) or with long runs of equal values.
 // Row passes are what a draw costs (about 7 us each at 50280 entries, one workgroup per row): eight with both filters through the
 // searches, one and a walk over registers through here; then the ranks, whose lists are read sixteen bytes at a time, several at once (read one entry after
-// the other, each behind the last one's way through LDS, and with a second pass over memory the draw took 30.6 us at 13 rows, top-k 50
-// and top-p, as it takes 21; the slots' step behind it was a launch of 4.6).
+// the other, each behind the last one's way through LDS, and with a second pass over memory the draw of 13 rows, top-k 50
+// and top-p, took 30.6 us and the slots' step behind it, a launch of its own, 4.6; with the slots' step inside it is 25.9).
 template <typename R> __device__ __forceinline__ bool short_top_k(R &row, uint32_t group_key, int k, SampShared &sh) {
     const int tid = threadIdx.x;
     group_key = max(group_key, (uint32_t)__shfl_xor((int)group_key, 1, kWave));

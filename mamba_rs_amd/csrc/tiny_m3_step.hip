@@ -161,9 +161,9 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_m3_backbone_step_kernel(Tin
 
 // The same step with the weights streamed (tiny_step.hip: why and how), for models of the default expand, headdim, d_state, groups and rope
 // fraction without the norm in front of out_proj; of those this route takes d_model 64 and 128.  A thread holds its rows of the next layer's
-// in_proj in registers, z and x columns and the narrow rest as two sweeps, and those of out_proj in LDS.  Five barriers a layer: sums of in_proj |
+// in_proj in registers, z and x columns and the narrow rest as two sweeps, and those of out_proj in LDS.  Six barriers a layer: partial sums of in_proj | its columns |
 // rotations and the heads' coefficients, one lane each | state update, which takes its K and Q from in_proj's columns itself | out_proj | its sums.
-// A layer 5.7 us at d_model 128 with 48 rows (before: 13.3; its 460 KB come in in 3.4); the step of four layers, with the host's rows, 63.8 -> 41.3 us, one
+// A layer 5.7 us at d_model 128 with 48 rows (before: 13.3; its 460 KB come in in 3.4); the step of four layers, with the host's rows, in a loop of steps 63.8 -> 41.3 us, one
 // row 57.7 -> 35.0, 1024 rows 383 -> 282, d_model 64 with 16 rows 47.5 -> 26.3.
 template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_m3_stream_step_kernel(TinyM3StepArgs a) {
     extern __shared__ float lds[];
@@ -261,7 +261,8 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_m3_stream
         const float inv = rms_inv(wave_sum(ss), DM, a.eps);
         if (in.on) *reinterpret_cast<float4 *>(&part[in.j * 2 * di + 4 * in.q]) = acc;
         if (rp.on) *reinterpret_cast<float4 *>(&part2[rp.j * rest + 4 * rp.q]) = acr;
-        // The vectors are in LDS: half of out_proj's requests are newer, and loads come back in order (stores that are still open only raise the count).
+        // The vectors are in LDS: half of out_proj's requests are newer, and loads come back in order (stores that are still open only raise the count).  Of that half
+        // a part is waited for as well: as fast as letting all of it be under way (the step of four layers, 48 rows, 41.4 us both ways).
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Out::rows / 4) : "memory");
         lds_barrier();
         {
@@ -341,7 +342,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_m3_stream
         if (tid < di) vst[tid] = xs[tid];
         if (passes == 1) feed(2);
         feed(3);
-        // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer.
+        // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer (and, as above, a part of them is waited for).
         if (!kLast) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(In::rows / 4) : "memory");
         pin();
         lds_barrier();

@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
 // 58 bytes a clock from L2, measured with 1 to 256 of them reading, however many loads are in flight).  Here the requests never stop:
 // a thread holds its rows of the next layer's in_proj and x_proj in registers and those of out_proj in LDS, and each is asked for again
 // behind its use, in portions that go out while the LDS reads of the chain are under way: all of them at once would hold the waves at
-// their next instruction until the last is taken in (5.65 us against 5.3).  The chain is shorter as well: seven barriers a layer, the sum of squares
+// their next instruction until the last is taken in (5.65 us against 5.3).  The chain is shorter as well: eight barriers a layer, the sum of squares
 // taken by every wave for itself and applied behind in_proj, partial sums added by the thread that needs the column, the vectors brought
 // by one request a wave.  A layer 5.3 us at d_model 128 and 2.25 at 64 (before: 10.4 and 8); the step of three layers, with the host's rows,
 // 44.1 -> 28.4 us and 37.4 -> 20.5, 256 rows 82.7 -> 72.0, 1024 rows 321 -> 272.
@@ -268,7 +268,8 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         }
         const float inv = rms_inv(wave_sum(ss), DM, a.eps);
         if (in.on) *reinterpret_cast<float4 *>(&part[in.j * 2 * di + 4 * in.q]) = acc;
-        // The vectors are in LDS: half of out_proj's requests are newer, and loads come back in order (stores that are still open only raise the count).
+        // The vectors are in LDS: half of out_proj's requests are newer, and loads come back in order (stores that are still open only raise the count).  Of that half
+        // a part is waited for as well: as fast as letting all of it be under way (the step of three layers, one row, 28.1 us both ways; five layers, 100 rows, 54.7 to 55.5).
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Out::rows / 4) : "memory");
         lds_barrier();
         // conv1d step + SiLU on the x half (window slot k holds the input d_conv - k steps back; the new input goes last), SiLU of the gate half
@@ -348,7 +349,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
             if (g == 0) y[d] = fmaf(Dv, uv, s) * gv;
         }
         if (passes == 1) feed(3);
-        // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer.
+        // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer (and, as above, a part of them is waited for).
         if (!kLast) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(In::rows / 4) : "memory");
         pin();
         lds_barrier();
