@@ -243,7 +243,7 @@ template <int DM, typename Args> __device__ __forceinline__ void stream_output(c
     if (tid < DM) {
         const float v = xin[tid] * inv;
         a.temporal[(int64_t)b * DM + tid] = v;
-        if (a.host.out) a.host.out[(int64_t)b * DM + tid] = v;
+        if (a.host.out) host_store(a.host.out + (int64_t)b * DM + tid, v);
     }
     if (a.host.out) host_row_done(a.host, b);
 }

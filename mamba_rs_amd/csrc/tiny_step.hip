@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     for (int i = tid; i < dm; i += kTinyThreads) {
         const float v = res[i] * inv * a.norm_f[i];
         a.temporal[(int64_t)b * dm + i] = v;
-        if (a.host.out) a.host.out[(int64_t)b * dm + i] = v;
+        if (a.host.out) host_store(a.host.out + (int64_t)b * dm + i, v);
     }
     if (a.host.out) host_row_done(a.host, b);
 }

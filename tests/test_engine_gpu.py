@@ -529,6 +529,19 @@ def test_small_f32_step_with_streamed_weights_follows_the_cpu_route(dm, L, idim,
     eng.close()
 
 
+@pytest.mark.parametrize("dm,B,dtype", [(64, 1, WeightDtype.F32), (64, 7, WeightDtype.F32), (64, 8, WeightDtype.F32), (64, 9, WeightDtype.F32), (128, 130, WeightDtype.F32),
+                                        (128, 17, WeightDtype.BF16)])
+def test_rows_a_step_hands_to_the_host_are_the_rows_it_leaves_on_the_device(dm, B, dtype):
+    """The host waits for one flag per row, eight at a time (single-launch steps and the kernel behind the others): every row of every step, bit for bit."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    eng = GpuMambaBackbone.new_with_dtype(0, MambaWeights.init(cfg, dm, 5), cfg, dm, B, dtype)
+    rng = np.random.default_rng(B)
+    for _ in range(20):
+        got = eng.step(rng.standard_normal((B, dm)).astype(np.float32))
+        assert np.isfinite(got).all() and np.array_equal(got, eng.download_temporal())
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,lens,dtype", [
     (128, (9, 5), WeightDtype.F16),              # four tokens; dt_rank 8: a quarter of a k-step of dt_proj
     (256, (6, 40, 18), WeightDtype.BF16),        # five
