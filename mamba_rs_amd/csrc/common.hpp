@@ -152,6 +152,12 @@ int launch_tiled_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t l
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 bool mid_gemm_wins(int64_t M, int N, int K);
 int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
+// Logits of up to 64 rows (lm_head.hip) from a tiled table, f32 from 16-bit storage; with `keys` (lm_head_keys of them) each row's greedy pick as a key per workgroup, which
+// launch_pick turns into the token
+bool lm_head_ok(int dtype, int M, int N, int K);
+size_t lm_head_keys(int M, int N, int K);
+int launch_lm_head(hipStream_t st, int dtype, float *C, int64_t ldc, const void *A, const void *Wp, int M, int N, int K, int vocab, unsigned long long *keys, bool stream);   // stream: the table is read past the caches
+int launch_pick(hipStream_t st, int *tokens, const unsigned long long *keys, int M, int N, int K);
 // The same for a prefill of thousands of rows (gemm_big.hip), C in the storage type
 bool big_gemm_ok(int dtype, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 bool big_gemm_wins(int64_t M, int N, int K);
@@ -318,6 +324,7 @@ struct LmHooks {
     int (*step)(void *self, const TokenRows &rows);  // one decode step on those rows (capturable: launches only)
     int (*reset)(void *self);
     size_t (*state_bytes)(void *self);               // recurrent state, for save / restore around a warm-up run
+    size_t weight_bytes;                             // the projections of all layers
     int (*state_copy)(void *self, void *buf, int restore);
     int (*prefill)(void *self, const int *dev_tokens, const void *embed, int vocab, int T);   // tokens [batch, T] on device
     // Prompts of a generation, prefix_steps steps at a time: prefix_rows gives the f32 rows [batch * steps, d_model] to fill (null: no such route),

@@ -1153,6 +1153,9 @@ struct mrs_lm {
     float *logits;      // [batch, vocab_padded] f32
     int *tokens;        // [batch] current token ids on device
     ArgRow *arg_rows;   // [batch], zero between two picks
+    unsigned long long *arg_keys;   // the own head's: its part of the greedy pick, and the head's table in tiles (null: the library's head)
+    void *table_p;
+    bool stream_table;
     std::vector<void *> allocs;
     hipGraph_t graph;
     hipGraphExec_t graph_exec;
@@ -1189,6 +1192,12 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     MRS_LM_HIP(hipMalloc((void **)&lm->tokens, (size_t)lm->batch * sizeof(int))); lm->allocs.push_back(lm->tokens);
     MRS_LM_HIP(hipMalloc((void **)&lm->arg_rows, (size_t)lm->batch * sizeof(ArgRow))); lm->allocs.push_back(lm->arg_rows);
     MRS_LM_HIP(hipMemsetAsync(lm->arg_rows, 0, (size_t)lm->batch * sizeof(ArgRow), eng.stream));
+    lm->arg_keys = nullptr; lm->table_p = nullptr;
+    lm->stream_table = step_outgrows_cache((int64_t)(ne * es + eng.weight_bytes + eng.state_bytes(eng.self)));
+    if (lm_head_ok(lm->dtype, lm->batch, lm->vocab_padded, lm->dm)) {
+        MRS_LM_HIP(hipMalloc((void **)&lm->arg_keys, lm_head_keys(lm->batch, lm->vocab_padded, lm->dm) * 8)); lm->allocs.push_back(lm->arg_keys);
+        MRS_LM_HIP(hipMalloc(&lm->table_p, ne * es)); lm->allocs.push_back(lm->table_p);
+    }
     MRS_LM_HIP(hipMalloc((void **)&stage, ne * 4));
     MRS_LM_HIP(hipMemsetAsync(stage, 0, ne * 4, eng.stream));  // padded rows are zero
     MRS_LM_HIP(hipMemcpyAsync(stage, embed, (size_t)vocab * lm->dm * 4, hipMemcpyHostToDevice, eng.stream));
@@ -1196,6 +1205,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     if (lm->dtype == MRS_F32) MRS_LM_HIP(hipMemcpyAsync(lm->embed, stage, ne * 4, hipMemcpyDeviceToDevice, eng.stream));
     else if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, eng.stream, (bf16_t *)lm->embed, stage, (int64_t)ne);
     else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, eng.stream, (f16_t *)lm->embed, stage, (int64_t)ne);
+    if (lm->table_p) { const int rc = launch_tile_weight(eng.stream, lm->dtype, lm->table_p, lm->embed, lm->vocab_padded, lm->dm); if (rc) { cleanup(); return rc; } }
     MRS_LM_HIP(hipStreamSynchronize(eng.stream));
 #undef MRS_LM_HIP
     hipFree(stage);
@@ -1237,7 +1247,9 @@ static LmHooks m1_hooks(mrs_backbone *bb) {
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
-    h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy; h.prefill = m1_hook_prefill;
+    h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy;
+    h.weight_bytes = (size_t)bb->cfg.n_layers * ((size_t)3 * bb->cfg.d_model * bb->di + (size_t)bb->di * (bb->xd + bb->dr)) * esize(bb->dtype);
+    h.prefill = m1_hook_prefill;
     h.prefix_rows = m1_hook_prefix_rows; h.prefix_run = m1_hook_prefix_run; h.prefix_steps = kPrefixSteps;
     h.seat = &bb->seat; h.check = m1_hook_check; h.go_on_chain = m1_hook_go_on_chain;
     return h;
@@ -1279,7 +1291,7 @@ extern "C" int mrs_lm_set_untied_head(mrs_lm *lm, const float *lm_head) {
     if (stage) hipFree(stage);
     if (e != hipSuccess) { if (!lm->head) hipFree(dst); return fail(MRS_E_HIP, "mrs_lm_set_untied_head: %s", hipGetErrorString(e)); }
     if (!lm->head) { lm->head = dst; lm->allocs.push_back(dst); }
-    return MRS_OK;
+    return lm->table_p ? launch_tile_weight(bb->stream, lm->dtype, lm->table_p, dst, lm->vocab_padded, lm->dm) : MRS_OK;
 }
 
 extern "C" void mrs_lm_destroy(mrs_lm *lm) {
@@ -1297,7 +1309,8 @@ extern "C" void mrs_lm_destroy(mrs_lm *lm) {
 
 // logits = norm_f(hidden) . table^T, table = the embedding (tied head) or the head's own weights
 // (OP_T on the row-major [V, dm] table: src/mamba_ssm/gpu/blas.rs:709-740)
-static int lm_logits(mrs_lm *lm) {
+// pick: the next lm_argmax is the pick of these logits
+static int lm_logits(mrs_lm *lm, bool pick = false) {
     const LmHooks *bb = &lm->eng;
     const int dm = lm->dm, V = lm->vocab_padded, B = lm->batch;
     const float one = 1.0f, zero = 0.0f;
@@ -1305,6 +1318,7 @@ static int lm_logits(mrs_lm *lm) {
     // f32 tables at one to four rows: the table is already [vocab][d_model], the layout the row-wise route of the
     // library's own GEMM walks (the vendor kernel for this shape moves the 154 MB of a 50k x 768 table at 1.6 TB/s)
     const void *table = lm->head ? lm->head : lm->embed;
+    if (lm->arg_keys) return launch_lm_head(bb->stream, lm->dtype, lm->logits, V, hid, lm->table_p, B, V, dm, lm->vocab, pick ? lm->arg_keys : nullptr, lm->stream_table);
     if (lm->dtype == MRS_F32 && skinny_gemm_ok(MRS_F32, B, V, dm, dm, hid, table)) {
         const SkinnyEpi none = {};
         return launch_skinny_gemm(bb->stream, MRS_F32, lm->logits, 1, V, hid, dm, table, B, V, dm, none);
@@ -1318,6 +1332,7 @@ static int lm_logits(mrs_lm *lm) {
 
 static int lm_argmax(mrs_lm *lm) {
     hipStream_t st = lm->eng.stream;
+    if (lm->arg_keys) return launch_pick(st, lm->tokens, lm->arg_keys, lm->batch, lm->vocab_padded, lm->dm);
     const auto pick = [&](auto kernel, int slice) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)((lm->vocab + slice - 1) / slice * lm->batch)), dim3(256), 0, st, lm->tokens, lm->arg_rows, lm->logits, lm->vocab,
                            (int64_t)lm->vocab_padded);
@@ -1330,7 +1345,7 @@ static int lm_argmax(mrs_lm *lm) {
 static int lm_decode_body(mrs_lm *lm) {
     const LmHooks *bb = &lm->eng;
     MRS_TRY(bb->step(bb->self, {lm->embed, lm->tokens, nullptr, lm->vocab}));
-    MRS_TRY(lm_logits(lm));
+    MRS_TRY(lm_logits(lm, true));
     return lm_argmax(lm);
 }
 
@@ -1418,7 +1433,7 @@ extern "C" int mrs_lm_prefill(mrs_lm *lm, mrs_backbone *prefill_bb, const int *t
     hipMemcpyAsync(dtok, tokens, rows * sizeof(int), hipMemcpyHostToDevice, eng->stream);
     int rc = eng->prefill(eng->self, dtok, lm->embed, lm->vocab, T);
     if (!rc && own) {
-        rc = lm_logits(lm);
+        rc = lm_logits(lm, true);
         if (!rc) rc = lm_argmax(lm);
     }
     hipStreamSynchronize(eng->stream);

@@ -1446,7 +1446,9 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     LmHooks h = {};
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = bb->temporal_t;
-    h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes; h.state_copy = m3_hook_state_copy;
+    h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes;
+    h.weight_bytes = (size_t)bb->cfg.n_layers * bb->cfg.d_model * ((size_t)bb->ip + bb->di) * (bb->dtype == MRS_F32 ? 4 : 2);
+    h.state_copy = m3_hook_state_copy;
     h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check; h.go_on_chain = m3_hook_go_on_chain;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");
 }

@@ -48,4 +48,10 @@ inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31)
 // 390 / 382, 522 / 521; 42 MB (3328) 379 / 398, 410 / 428, 465 / 468; 49 MB (3584) 405 / 429, 444 / 457, 499 / 504.  (Asking for the part that would fit: behind both everywhere.)
 inline bool asks_out_proj_ahead(int64_t bytes, int rows) { return bytes <= (int64_t)(rows < 8 ? 28 : 40) << 20; }
 
+// Whether what a decode step touches (`bytes`: weights, states, the head's table) is more than the chip's last cache holds, 256 MB.  What is read once a step and not kept from one
+// step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
+// The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)
+// 168.7 / 174.2, 16 rows (266 MB) 241.7 / 235.2; 16 of them 16 rows (228 MB) 189.2 / 194.5, 64 rows (323 MB) 243.1 / 234.8; 12 of them 64 rows (262 MB) 184.4 / 182.9.
+inline bool step_outgrows_cache(int64_t bytes) { return bytes > (int64_t)240 << 20; }
+
 }  // namespace mrs

@@ -1,0 +1,42 @@
+"""The language model head (csrc/lm_head.hip): logits of every row against the product in 64 bits, and the greedy pick against numpy."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from mamba_rs_amd import GpuMambaBackbone, GpuMambaLM, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
+
+
+@pytest.mark.parametrize("dm,B,vocab,dtype,untied", [
+    (64, 1, 5, WeightDtype.BF16, False),         # fewer columns than one workgroup, fewer k-steps than are asked for ahead
+    (64, 16, 64, WeightDtype.F16, False),
+    (64, 17, 1090, WeightDtype.BF16, True),      # one row more than a row tile; a last workgroup with one tile; a head of its own
+    (288, 33, 2100, WeightDtype.BF16, False),    # k-steps that are no multiple of those ahead
+    (768, 49, 700, WeightDtype.BF16, False),     # workgroups of sixteen waves
+    (1024, 64, 1500, WeightDtype.F16, False),    # the most rows of the widest model they go to
+    (1088, 64, 300, WeightDtype.BF16, False),    # one step wider: the library's
+    (64, 65, 300, WeightDtype.BF16, False),      # one row more: the library's
+    (768, 3, 170000, WeightDtype.BF16, False),   # a table past the cache's size: read past it
+])
+def test_logits_and_pick(dm, B, vocab, dtype, untied):
+    """f32 sums of K products of 16-bit values: 2 K eps of the sum of the products' magnitudes bounds them."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 3)
+    w.input_proj_w = np.zeros(0, np.float32); w.input_proj_b = np.zeros(0, np.float32)
+    g = torch.Generator().manual_seed(B)
+    embed = torch.randn(vocab, dm, generator=g)
+    embed[vocab // 2:vocab // 2 + 2] = embed[:2] if vocab > 4 else embed[vocab // 2:vocab // 2 + 2]   # equal columns: the last of them is the pick
+    head = torch.randn(dm, vocab, generator=g) if untied else embed.T
+    lm = GpuMambaLM(GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype), embed.numpy(), head.contiguous().numpy() if untied else None)
+    tt = dtype.torch_dtype()
+    for step in range(2):
+        lm.set_tokens(((np.arange(B) * 7 + step) % vocab).astype(np.int32))
+        lm.decode_step()
+        got = torch.from_numpy(lm.last_logits()).reshape(B, -1)[:, :vocab]
+        hid = torch.from_numpy(lm.backbone.download_temporal()).to(tt).double()
+        table = head.to(tt).double()
+        bound = 2 * dm * 2.0 ** -24 * (hid.abs() @ table.abs()) + 1e-30
+        assert ((got.double() - hid @ table).abs() <= bound).all(), step
+        last = vocab - 1 - np.argmax(got.numpy()[:, ::-1], axis=1)
+        assert np.array_equal(lm.get_tokens(), last), step
