@@ -133,6 +133,7 @@ struct SkinnyEpi {
     int prenorm_mt;      // mode 2: != 0 writes prenorm in that tiled order (prenorm_mt row tiles) for the next tiled in_proj
     // matrix-core route of gemm_skinny.hip: the weight is the tiled copy (launch_tile_weight) instead of Wt[N][K]
     int w_tiled;
+    int w_stream;            // (gemm_wide.hip) the weight is read past the last cache
     // mode 1, optional: a second copy of u in tiled order (u_tiled_mt row tiles), the operand of a tiled x_proj
     void *u_tiled;
     int u_tiled_mt;
@@ -237,6 +238,7 @@ struct ResidentArgs {
     float eps;
     int n_layers, batch, dm, di, ds, dc, dr, xd, G, nc, oc;
     void *rows_buf;     // resident_rows_bytes() of operand rows
+    int cached;         // layers whose weights come through the last cache (resident.hpp)
     int groups, rows;   // groups of G workgroups, batch rows of the largest group (more than one: resident_rows.hip)
 };
 bool resident_plan(ResidentArgs &a, int dtype);   // false: the shape is outside the route
@@ -267,6 +269,7 @@ struct ResidentM3Args {
     unsigned wait;
     float eps, a_floor;
     int n_layers, batch, dm, di, nh, hd, ds, ng, nr, G, nc, oc, ex, row_order;
+    int cached;         // as in ResidentArgs
 };
 bool resident_m3_plan(ResidentM3Args &a, int dtype);
 size_t resident_m3_layer_bytes(const ResidentM3Args &a);

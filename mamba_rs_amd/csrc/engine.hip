@@ -328,6 +328,11 @@ static int alloc_scratch(mrs_backbone *bb, Scratch *s, int64_t rows, int T) {
     return MRS_OK;
 }
 
+static int64_t layer_weight_bytes(const mrs_backbone *bb) {
+    return ((int64_t)3 * bb->cfg.d_model * bb->di + (int64_t)bb->di * (bb->xd + bb->dr)) * (int64_t)esize(bb->dtype);
+}
+static int64_t state_bytes(const mrs_backbone *bb) { return (int64_t)bb->cfg.n_layers * bb->batch * bb->di * (bb->cfg.d_conv + bb->cfg.d_state) * 4; }
+
 // C[M,N] = A[M,K] (row stride lda) . W[K,N], all row-major; f32 accumulate.
 static int gemm_rm(mrs_backbone *bb, int dtype, void *C, int ldc, const void *A, int lda, const void *W, int M, int N, int K) {
     const rocblas_datatype t = blas_type(dtype);
@@ -408,6 +413,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
     // that cannot split K (nobody would sum the shares): 12.5 us at 32 and 64 rows of the 2.8b shape, against 4.7 us split.
     // Per step at that shape, dt_proj in the step kernel / on its own: 32 rows 3.57 / 3.84 ms, 48 rows 4.32 / 4.34, 64 rows 5.04 / 4.89.
     static const int64_t wide_fuse = [] { const char *e = getenv("MRS_DECODE_FUSE_DT_LIMIT"); return e ? (int64_t)atoll(e) : (int64_t)6400; }();
+    const bool stream_in = bb->wide && streams_in_proj(L * layer_weight_bytes(bb) + state_bytes(bb), nr);
     const int64_t fuse_limit = (a_mt && bb->wide) ? wide_fuse : kFuseDtProjLimit;
     for (int l = 0; l < L; l++) {
         const LayerDev &lw = bb->layers[l];
@@ -434,7 +440,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
             fold.next = lw.out_proj_p; fold.next_units = (dm / 16 + unit - 1) / unit; fold.next_bytes = unit * (di / 32) * 1024;
         }
         if (a_mt) {
-            inp.a_tiled = 1; inp.w_tiled = 1;
+            inp.a_tiled = 1; inp.w_tiled = 1; inp.w_stream = stream_in;
             if (!fold_x) { inp.u_tiled = s->u_tiled; inp.u_tiled_mt = a_mt; }
             if (bb->wide) MRS_TRY(launch_tiled_gemm(st, dt, proj, 0, 2 * di, normed, dm, lw.in_proj_p, nr, 2 * di, dm, inp));
             else MRS_TRY(launch_skinny_gemm(st, dt, proj, 0, 2 * di, normed, dm, lw.in_proj_p, nr, 2 * di, dm, inp));
@@ -644,6 +650,7 @@ static int setup_resident(mrs_backbone *bb) {
     a.roll = a.epoch + (size_t)a.groups * 32;
     if (bb->resident == 2) MRS_TRY(dev_alloc(bb, &a.rows_buf, resident_rows_bytes(a)));
     a.wait = kResidentWait;
+    a.cached = layers_in_cache(bb->cfg.n_layers, layer_weight_bytes(bb), state_bytes(bb));
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident(bb));
@@ -1217,9 +1224,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
 static int m1_hook_step(void *self, const TokenRows &rows) { return step_body((mrs_backbone *)self, nullptr, rows); }
 static int m1_hook_reset(void *self) { return mrs_backbone_reset((mrs_backbone *)self); }
 static size_t m1_hook_state_bytes(void *self) {
-    mrs_backbone *bb = (mrs_backbone *)self;
-    const size_t L = bb->cfg.n_layers, B = bb->batch;
-    return L * B * bb->di * (size_t)(bb->cfg.d_conv + bb->cfg.d_state) * 4;
+    return (size_t)state_bytes((mrs_backbone *)self);
 }
 static int m1_hook_state_copy(void *self, void *buf, int restore) {
     mrs_backbone *bb = (mrs_backbone *)self;
@@ -1248,7 +1253,7 @@ static LmHooks m1_hooks(mrs_backbone *bb) {
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal;
     h.temporal_t = bb->dtype != MRS_F32 ? bb->temporal_t : nullptr;
     h.step = m1_hook_step; h.reset = m1_hook_reset; h.state_bytes = m1_hook_state_bytes; h.state_copy = m1_hook_state_copy;
-    h.weight_bytes = (size_t)bb->cfg.n_layers * ((size_t)3 * bb->cfg.d_model * bb->di + (size_t)bb->di * (bb->xd + bb->dr)) * esize(bb->dtype);
+    h.weight_bytes = (size_t)(bb->cfg.n_layers * layer_weight_bytes(bb));
     h.prefill = m1_hook_prefill;
     h.prefix_rows = m1_hook_prefix_rows; h.prefix_run = m1_hook_prefix_run; h.prefix_steps = kPrefixSteps;
     h.seat = &bb->seat; h.check = m1_hook_check; h.go_on_chain = m1_hook_go_on_chain;

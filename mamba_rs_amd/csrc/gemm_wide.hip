@@ -37,9 +37,10 @@
 namespace mrs {
 namespace {
 
+constexpr int kNontemporal = 2;      // of a buffer load's cache policy bits
 constexpr int kTiledThreads = 512;   // eight waves per workgroup: WS of them stream the operands, all of them run the epilogue
 
-template <typename T, int MT, int NT, int R, int WS = 8>
+template <typename T, int MT, int NT, int R, int WS, int AUX>
 __global__ __launch_bounds__(kTiledThreads) void tiled_gemm_kernel(void *__restrict__ Cv, int out_f32, int64_t ldc, const T *__restrict__ A,
                                                                    int64_t lda, const T *__restrict__ Wp, int M, int N, int K, SkinnyEpi ep) {
     constexpr int kPark = WS;   // partial tiles that meet in LDS, one per streaming wave
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(kTiledThreads) void tiled_gemm_kernel(void *__restr
     const unsigned astep = a_tiled ? (unsigned)MT * 1024u : 64u;
     const unsigned woff = 16u * (unsigned)l;
     auto ldw = [&](int nt, int s_) {
-        return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres[nt], woff, 1024u * (unsigned)(w + WS * s_), 0));
+        return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres[nt], woff, 1024u * (unsigned)(w + WS * s_), AUX));
     };
     auto lda_ = [&](int mt, int s_) {
         const int ks = w + WS * s_;
@@ -292,8 +293,9 @@ int launch_tiled_t(hipStream_t st, void *C, int out_f32, int64_t ldc, const T *A
     // 2.8b-shape decode chain, per step with 1 / 2 / 4 / 8 streaming waves: 16 rows 2.85 / 2.75 / 2.65 / 2.72 ms,
     // 32 rows 3.48 / 3.35 / 3.44 / 3.62, 64 rows 5.29 / 4.77 / 4.81 / 4.92.
     const dim3 grid((unsigned)((ntiles + nt - 1) / nt)), block(kTiledThreads);
-#define MRS_TG(MT_, NT_, R_, W_) \
-    hipLaunchKernelGGL((tiled_gemm_kernel<T, MT_, NT_, R_, W_>), grid, block, 0, st, C, out_f32, ldc, A, lda, Wp, M, N, K, ep)
+#define MRS_TG(MT_, NT_, R_, W_)                                                                                                                              \
+    if (ep.w_stream) hipLaunchKernelGGL((tiled_gemm_kernel<T, MT_, NT_, R_, W_, kNontemporal>), grid, block, 0, st, C, out_f32, ldc, A, lda, Wp, M, N, K, ep); \
+    else hipLaunchKernelGGL((tiled_gemm_kernel<T, MT_, NT_, R_, W_, 0>), grid, block, 0, st, C, out_f32, ldc, A, lda, Wp, M, N, K, ep)
     switch (mt * 10 + nt) {
         case 11: MRS_TG(1, 1, 10, 4); break;
         case 12: MRS_TG(1, 2, 5, 4); break;

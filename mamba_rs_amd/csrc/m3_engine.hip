@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "gemm_tune.hpp"
 #include "host_io.hpp"
+#include "size_rules.hpp"
 #include <stdlib.h>
 #include "glue.hpp"
 #include "m3_math.hpp"
@@ -665,6 +666,9 @@ int project_input3(mrs_m3_backbone *bb) {
 // (24 layers of d_model 768 at two rows: 230 against 317 us a step).
 constexpr int kResidentM3Layers = 4;
 
+int64_t layer_weight_bytes3(const mrs_m3_backbone *bb) { return (int64_t)bb->cfg.d_model * (bb->ip + bb->di) * (int64_t)esize3(bb->dtype); }
+size_t m3_hook_state_bytes(void *self);
+
 // Resident step for the rows whose workgroups fit on the chip together.  One row takes the chain's own order (resident_m3_row.hip) wherever
 // the chain is on its row-wise route, at any depth: the same bits, and the faster of the two (its comment has both).  The kernel chain
 // stays ready beside it, for the steps that do not get a turn.
@@ -705,6 +709,7 @@ int setup_resident3(mrs_m3_backbone *bb) {
     MRS_TRY(dev_alloc3(bb, (void **)&a.epoch, ((size_t)a.batch * 32 + kRollHead + kRollMax) * 4));
     a.roll = a.epoch + (size_t)a.batch * 32;
     a.wait = kResidentWait;
+    a.cached = layers_in_cache(bb->cfg.n_layers, layer_weight_bytes3(bb), (int64_t)m3_hook_state_bytes(bb));
     MRS_HIP(hipHostMalloc((void **)&bb->res_broken, 64, 0));
     a.broken = bb->res_broken;
     MRS_TRY(arm_resident3(bb));
@@ -1447,7 +1452,7 @@ extern "C" int mrs_lm3_create(mrs_lm **out, mrs_m3_backbone *bb, const float *em
     h.self = bb; h.batch = bb->batch; h.d_model = bb->cfg.d_model; h.dtype = bb->dtype; h.identity_proj = bb->identity_proj;
     h.stream = bb->stream; h.blas = bb->blas; h.d_input = bb->d_input; h.temporal = bb->temporal; h.temporal_t = bb->temporal_t;
     h.step = m3_hook_step; h.reset = m3_hook_reset; h.state_bytes = m3_hook_state_bytes;
-    h.weight_bytes = (size_t)bb->cfg.n_layers * bb->cfg.d_model * ((size_t)bb->ip + bb->di) * (bb->dtype == MRS_F32 ? 4 : 2);
+    h.weight_bytes = (size_t)(bb->cfg.n_layers * layer_weight_bytes3(bb));
     h.state_copy = m3_hook_state_copy;
     h.prefill = m3_hook_prefill; h.seat = &bb->seat; h.check = m3_hook_check; h.go_on_chain = m3_hook_go_on_chain;
     return mrs_lm_create_from_hooks(out, h, embed, vocab, "mrs_lm3_create");

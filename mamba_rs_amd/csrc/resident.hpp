@@ -143,10 +143,18 @@ template <typename V> __device__ __forceinline__ V ld_off(const void *base, unsi
 // aligned) without passing through registers.  The compiler's wait counting does not see it: dma_wait() by the same wave and a
 // workgroup barrier come before the data is read.  Requests are spaced (s_sleep: 64 clocks each): a compute unit's requests are
 // served in order, and a burst of them would stand in front of the exchange's stores and polls.
-template <int SLEEP = 1> __device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int first, int pieces, int step) {
+template <int SLEEP = 1> __device__ __forceinline__ void dma_to_lds(unsigned to, const void *from, int first, int pieces, int step, bool stream = false) {
     const u64 at = (u64)(uintptr_t)from;   // the same for the whole wave
     const u64 src = (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)at) | (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32;
     const unsigned lane16 = (unsigned)(threadIdx.x & 63) * 16u, dst0 = __builtin_amdgcn_readfirstlane(to);
+    if (stream) {
+#pragma unroll 1
+        for (int i = first; i < pieces; i += step) {
+            const unsigned voff = (unsigned)i * 1024u + lane16, dst = dst0 + (unsigned)i * 1024u;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_sleep %3" ::"s"(dst), "v"(voff), "s"(src), "n"(SLEEP) : "m0", "memory");
+        }
+        return;
+    }
 #pragma unroll 1
     for (int i = first; i < pieces; i += step) {
         const unsigned voff = (unsigned)i * 1024u + lane16, dst = dst0 + (unsigned)i * 1024u;
@@ -277,19 +285,20 @@ struct WeightFeed {
     size_t next;                  // ... to that of the next layer
     unsigned win, wout, small;    // LDS byte addresses; the small blocks of two layers lie one after the other
     int out, small_at, small_bytes;   // offsets in the block
+    int cached;                   // layers whose weights come through the last cache; the others' are read past it
 };
 __device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int nl, int &state, RollCall call) {
     const char *blk = f.blk;
     const bool first = (threadIdx.x & 63) == 0, out_wave = wave == 10, small_wave = wave == 11;
-    const int iw = wave == 11 ? 2 : wave - 8, in_pieces = f.out >> 10, in_mid = in_pieces / 2, out_pieces = (f.small_at - f.out) >> 10;
-    auto bring_in = [&](const char *p, int from, int to) { dma_to_lds(f.win, p, from + iw, to, 3); };
-    auto bring_out = [&](const char *p) { dma_to_lds(f.wout, p + f.out, 0, out_pieces, 1); };
+    const int iw = wave == 11 ? 2 : wave - 8, cached = f.cached, in_pieces = f.out >> 10, in_mid = in_pieces / 2, out_pieces = (f.small_at - f.out) >> 10;
+    auto bring_in = [&](const char *p, int l, int from, int to) { dma_to_lds(f.win, p, from + iw, to, 3, l >= cached); };
+    auto bring_out = [&](const char *p, int l) { dma_to_lds(f.wout, p + f.out, 0, out_pieces, 1, l >= cached); };
     auto bring_small = [&](const char *p, int l) { dma_to_lds(f.small + (l & 1) * f.small_bytes, p + f.small_at, 0, f.small_bytes >> 10, 1); };
     if (out_wave) {
         const int s = call.answer();
         if (first) state = s;
-        bring_out(blk);
-    } else bring_in(blk, 0, in_pieces);
+        bring_out(blk, 0);
+    } else bring_in(blk, 0, 0, in_pieces);
     if (small_wave) bring_small(blk, 0);
     if (!out_wave) dma_wait();
     lds_barrier();   // layer 0's row is there
@@ -299,7 +308,7 @@ __device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int 
         blk += f.next;   // the next layer's
         lds_barrier();   // 1
         if (small_wave && more) bring_small(blk, l + 1);
-        if (!out_wave && more) bring_in(blk, 0, in_mid);
+        if (!out_wave && more) bring_in(blk, l + 1, 0, in_mid);
         if (out_wave) {
             if (l == 0 && state == kRollCall) {
                 const int s = call.outcome();
@@ -309,12 +318,12 @@ __device__ __forceinline__ void bring_weights(const WeightFeed f, int wave, int 
         }
         lds_barrier();   // 2
         if (state) return;
-        if (!out_wave && more) bring_in(blk, in_mid, in_pieces);
+        if (!out_wave && more) bring_in(blk, l + 1, in_mid, in_pieces);
         lds_barrier();   // 3
         if (state) return;
         if (!out_wave) dma_wait();
         lds_barrier();   // 4
-        if (out_wave && more) bring_out(blk);
+        if (out_wave && more) bring_out(blk, l + 1);
         lds_barrier();   // 5
         if (state) return;
     }

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_row_kernel(const Resi
         const LayerBlock lb = layer_block(dm, di, cols, oc, ds);
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         bring_weights({(const char *)a->weights + (size_t)src * lb.bytes, (size_t)G * lb.bytes, lds0 + S::win(sb.bytes, oc), lds0 + S::wout(sb.bytes),
-                       lds0 + S::small, lb.out, lb.small, sb.bytes}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
+                       lds0 + S::small, lb.out, lb.small, sb.bytes, a->cached}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
         return;
     }
 

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kResThreads) void resident_m3_step_kernel(const Res
         const LayerBlock lb = layer_block(dm, di, cols, oc, ds);
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         bring_weights({(const char *)a->weights + (size_t)src * lb.bytes, (size_t)G * lb.bytes, lds0 + L.win, lds0 + L.wout, lds0 + L.small, lb.out, lb.small,
-                       sb.bytes}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
+                       sb.bytes, a->cached}, wave, nl, state, {a->roll, a->broken, gridDim.x, a->wait, 0});
         return;
     }
 

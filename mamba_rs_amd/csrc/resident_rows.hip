@@ -70,6 +70,7 @@ struct RowsFeed {
     size_t conv_next, ssm_next;   // ... to those of the next layer
     int rows;
     unsigned spare;
+    int cached;                   // layers whose weights come through the last cache; the others' are read past it
     bool hurry;                   // the workgroup forms x_proj rows: it does not wait for them, but for u, a barrier earlier
 };
 // One request: a lane asks for a line, number `first` + lane of `lines` of 128 bytes per row.
@@ -111,10 +112,10 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
         lds_barrier();   // X
         const auto early_part = [&](auto sleep) {
             constexpr int Z = decltype(sleep)::value;
-            dma_to_lds<Z>(f.wout, blk + S::lb.out, w, out_pieces, 4);
+            dma_to_lds<Z>(f.wout, blk + S::lb.out, w, out_pieces, 4, l >= f.cached);
             if (more) {
                 dma_to_lds<Z>(f.small + ((l + 1) & 1) * S::sb.bytes, next + S::lb.small, w, small_pieces, 4);
-                dma_to_lds<Z>(f.win, next, w, early, 4);
+                dma_to_lds<Z>(f.win, next, w, early, 4, l + 1 >= f.cached);
             }
         };
         if (f.hurry) early_part(std::integral_constant<int, 1>());
@@ -126,7 +127,7 @@ template <class S> __device__ __forceinline__ void bring_rows_weights(const Rows
         if (more) {
             if (w < 3) touch_lines<S::nc * kDs * 4 / 128, S::di * kDs * 4>(f.spare, ssm, f.rows, w * 64);
             else touch_lines<S::nc * kDc * 4 / 128, S::di * kDc * 4>(f.spare, conv, f.rows, 0);
-            dma_to_lds<1>(f.win, next, early + w, in_pieces, 4);
+            dma_to_lds<1>(f.win, next, early + w, in_pieces, 4, l + 1 >= f.cached);
         }
         blk = next;
         lds_barrier();   // D
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(kResThreads) void resident_rows_kernel(const Reside
     if (wave >= kComputeWaves) {
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         bring_rows_weights<S>({(const char *)a->weights + (size_t)src * S::lb.bytes, S::layer_bytes, lds0, lds0 + S::wout, lds0 + S::small, (const char *)(a->conv_state + cst_l + (size_t)(r0 * di + c0) * kDc),
-                               (const char *)(a->ssm_state + hst_l + (size_t)(r0 * di + c0) * kDs), cst_l * 4, hst_l * 4, nr, lds0 + S::spare, src < S::xt}, wave, nl, state,
+                               (const char *)(a->ssm_state + hst_l + (size_t)(r0 * di + c0) * kDs), cst_l * 4, hst_l * 4, nr, lds0 + S::spare, a->cached, src < S::xt}, wave, nl, state,
                               {a->roll, a->broken, gridDim.x, a->wait, 0});
         return;
     }

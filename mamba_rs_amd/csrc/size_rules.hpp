@@ -42,16 +42,32 @@ inline int conv_xproj_form(int batch, int T, int di, int xd) {
 // 3266 / 3221, 4 x 4096 5887 / 6038).
 inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
 
-// Decode of wide models: whether the step kernel asks for the lines of out_proj (`bytes` of them) on the dies that will read them (m1_step.hip).  They have to stay in the dies' L2, eight
-// of 4 MB, until the launch behind: more than that is read twice, and then many rows' worth of work must cover it.  Eight layers, bf16, us a step, without / with:
-// 25 MB (d_model 2560) 4 rows 284 / 285, 8 304 / 297, 16 330 / 320, 40 454 / 433; 30 MB (2816) 314 / 317, 333 / 328, 367 / 356, 586 / 586; 36 MB (3072) 329 / 338, 351 / 351,
-// 390 / 382, 522 / 521; 42 MB (3328) 379 / 398, 410 / 428, 465 / 468; 49 MB (3584) 405 / 429, 444 / 457, 499 / 504.  (Asking for the part that would fit: behind both everywhere.)
-inline bool asks_out_proj_ahead(int64_t bytes, int rows) { return bytes <= (int64_t)(rows < 8 ? 28 : 40) << 20; }
-
 // Whether what a decode step touches (`bytes`: weights, states, the head's table) is more than the chip's last cache holds, 256 MB.  What is read once a step and not kept from one
 // step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
 // The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)
 // 168.7 / 174.2, 16 rows (266 MB) 241.7 / 235.2; 16 of them 16 rows (228 MB) 189.2 / 194.5, 64 rows (323 MB) 243.1 / 234.8; 12 of them 64 rows (262 MB) 184.4 / 182.9.
 inline bool step_outgrows_cache(int64_t bytes) { return bytes > (int64_t)240 << 20; }
+
+// Layers whose weights (`layer_bytes` each) come through that cache in a decode step: all of them where the states and they fit, else as many as leave room for the states, and the
+// others are read past it.  Walked from first to last at every step, more than it holds would leave nothing of it.  Us a step, bf16, 24 layers of which so many come through it:
+//   d_model 1024 (13.1 MB a layer)   1 row 24 286, 20 278, 16 267, 12 271, 0 281     4 rows 316, 312, 295, 298, 301    13 rows 337, 332, 327, 320, 328   32 rows 371, 369, 364, 361, 362
+//           768 (7.5)                32 rows 305, 301, 301, 305, 308     64 rows 351, 351, 349, 347, 351 (8 345)     16 rows, which fit 277, 281, 278, 279, 283
+inline int layers_in_cache(int layers, int64_t layer_bytes, int64_t state_bytes) {
+    if (!step_outgrows_cache(layers * layer_bytes + state_bytes)) return layers;
+    return (int)std::min<int64_t>(layers, std::max<int64_t>(0, ((int64_t)220 << 20) - state_bytes) / std::max<int64_t>(layer_bytes, 1));
+}
+
+// Decode of wide models, a launch per product: in_proj's weights, two thirds of a layer's, are read past that cache where a step (`bytes` of weights and states) outgrows it, so that
+// out_proj's and the states may stay and nothing has to be written back for what is read once.  Us a step, bf16, cached / past: d_model 2560, 8 layers 4 rows 322 / 294, 16 358 / 322,
+// 32 438 / 426, 64 577 / 573; 24 layers 4 rows 833 / 808, 16 938 / 877; 2048, 12 layers 4 rows 354 / 331, 16 392 / 370, 48 557 / 563 (there states are most of it).  Some of the
+// layers' through the cache, as layers_in_cache: behind it everywhere (2560, 16 rows, two of eight 341).  out_proj's past it as well: no difference, and where the step kernel asks for
+// its lines ahead that request past it costs 40.
+inline bool streams_in_proj(int64_t bytes, int rows) { return rows <= 32 && step_outgrows_cache(bytes); }
+
+// Decode of wide models: whether the step kernel asks for the lines of out_proj (`bytes` of them) on the dies that will read them (m1_step.hip).  They have to stay in the dies' L2, eight
+// of 4 MB, until the launch behind: more than that is read twice, and then many rows' worth of work must cover it.  Eight layers, bf16, us a step, without / with:
+// 25 MB (d_model 2560) 4 rows 284 / 285, 8 304 / 297, 16 330 / 320, 40 454 / 433; 30 MB (2816) 314 / 317, 333 / 328, 367 / 356, 586 / 586; 36 MB (3072) 329 / 338, 351 / 351,
+// 390 / 382, 522 / 521; 42 MB (3328) 379 / 398, 410 / 428, 465 / 468; 49 MB (3584) 405 / 429, 444 / 457, 499 / 504.  (Asking for the part that would fit: behind both everywhere.)
+inline bool asks_out_proj_ahead(int64_t bytes, int rows) { return bytes <= (int64_t)(rows < 8 ? 28 : 40) << 20; }
 
 }  // namespace mrs

@@ -12,6 +12,27 @@ pytestmark = pytest.mark.gpu
 from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
 
 
+@pytest.mark.parametrize("dm,L,B", [(1024, 20, 1), (1024, 20, 3), (2560, 4, 3)])
+def test_weights_past_the_last_cache(dm, L, B):
+    """Models whose weights are more than the last cache holds, so that some layers' (resident steps of a row and of several) or all layers' in_proj (wide models) are read past it:
+    outputs against the CPU route, as below."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 11)
+    w.input_proj_w = np.zeros((0, dm), np.float32)
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
+    w.layers = w.layers * L
+    P = oracle_params(w, cfg, dm, round_to=orc.BF16)
+    print(f"case past the cache {dm} {L} {B}", flush=True)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.BF16)
+    st = orc.m1_zero_state(P)
+    for t in range(2):
+        x = np.random.default_rng(t).standard_normal((B, dm)).astype(np.float32)
+        got = eng.step(x)
+        want = orc.m1_backbone_step(P, x[B - 1], *st, identity_proj=True)
+        assert cosine(got[B - 1], want) >= 0.999, (t, cosine(got[B - 1], want))
+    eng.close()
+
+
 @pytest.mark.parametrize("shape", [
     (32, 2, 32, 1),       # one k-step, four workgroups; an x_proj row of 34: a last tile of two entries
     (64, 3, 20, 16),      # input projection; dt_rank 4; a group of workgroups per row, sixteen of them

@@ -99,6 +99,7 @@ def test_deep_models_keep_the_kernel_chain(layers, route, monkeypatch):
     (cfg_(512, 32, 8, 1, 5), 512, WeightDtype.F16),                # eight channels and four columns of out_proj per workgroup: idle waves
     (cfg_(768, 64, 64, 1, 3), 768, WeightDtype.F16),
     (cfg_(1024, 64, 64, 1, 2), 1024, WeightDtype.BF16),
+    (cfg_(1024, 64, 64, 1, 20), 1024, WeightDtype.BF16),           # more weights than the last cache holds: some layers' are read past it
 ])
 def test_one_row_keeps_the_chain_s_bits(cfg, idim, dtype, monkeypatch):
     """One row at any depth: one launch, and output and states are the kernel chain's bit for bit -- eager, replayed, in steps that

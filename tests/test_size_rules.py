@@ -62,3 +62,11 @@ def test_out_proj_is_asked_for_ahead_only_where_it_stays_in_the_l2(rules):
     want = [nbytes <= (28 if rows < 8 else 40) * 2 ** 20 for nbytes, rows in ahead]
     assert rules("asks_out_proj_ahead(a, (int)b)", [(nbytes, rows, 0, 0) for nbytes, rows in ahead]) == want
     assert not any(w for w, (nbytes, _) in zip(want, ahead) if nbytes > 40 * 2 ** 20) and all(w for w, (nbytes, _) in zip(want, ahead) if nbytes <= 25 * 2 ** 20)
+
+
+def test_layers_whose_weights_come_through_the_last_cache(rules):
+    """All of them while they fit beside the states (240 MB), else no more than leave the states their room, and never fewer than none."""
+    mb = 2 ** 20
+    cases = [(24, 7 * mb, 3 * mb), (24, 7 * mb, 72 * mb), (24, 7 * mb, 73 * mb), (24, 13 * mb, 3 * mb), (24, 13 * mb, 50 * mb), (24, 7 * mb, 400 * mb), (8, 78 * mb, 40 * mb), (64, 0, 300 * mb)]
+    assert rules("layers_in_cache((int)a, b, c)", [(*c, 0) for c in cases]) == [24, 24, 21, 16, 13, 0, 2, 0]
+    assert rules("streams_in_proj(a, (int)b)", [(240 * mb, 4, 0, 0), (240 * mb + 1, 4, 0, 0), (10 ** 9, 32, 0, 0), (10 ** 9, 33, 0, 0)]) == [0, 1, 1, 0]
