@@ -413,7 +413,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
     // that cannot split K (nobody would sum the shares): 12.5 us at 32 and 64 rows of the 2.8b shape, against 4.7 us split.
     // Per step at that shape, dt_proj in the step kernel / on its own: 32 rows 3.57 / 3.84 ms, 48 rows 4.32 / 4.34, 64 rows 5.04 / 4.89.
     static const int64_t wide_fuse = [] { const char *e = getenv("MRS_DECODE_FUSE_DT_LIMIT"); return e ? (int64_t)atoll(e) : (int64_t)6400; }();
-    const bool stream_in = bb->wide && streams_in_proj(L * layer_weight_bytes(bb) + state_bytes(bb), nr);
+    const bool stream_in = streams_in_proj(L * layer_weight_bytes(bb) + state_bytes(bb), nr);
     const int64_t fuse_limit = (a_mt && bb->wide) ? wide_fuse : kFuseDtProjLimit;
     for (int l = 0; l < L; l++) {
         const LayerDev &lw = bb->layers[l];
@@ -445,6 +445,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
             if (bb->wide) MRS_TRY(launch_tiled_gemm(st, dt, proj, 0, 2 * di, normed, dm, lw.in_proj_p, nr, 2 * di, dm, inp));
             else MRS_TRY(launch_skinny_gemm(st, dt, proj, 0, 2 * di, normed, dm, lw.in_proj_p, nr, 2 * di, dm, inp));
         } else {
+            inp.w_stream = stream_in;
             MRS_TRY(launch_skinny_gemm(st, dt, proj, 0, 2 * di, normed, dm, lw.in_proj_t, nr, 2 * di, dm, inp));
         }
         const SkinnyEpi none = {};
@@ -1325,7 +1326,8 @@ static int lm_logits(mrs_lm *lm, bool pick = false) {
     const void *table = lm->head ? lm->head : lm->embed;
     if (lm->arg_keys) return launch_lm_head(bb->stream, lm->dtype, lm->logits, V, hid, lm->table_p, B, V, dm, lm->vocab, pick ? lm->arg_keys : nullptr, lm->stream_table);
     if (lm->dtype == MRS_F32 && skinny_gemm_ok(MRS_F32, B, V, dm, dm, hid, table)) {
-        const SkinnyEpi none = {};
+        SkinnyEpi none = {};
+        none.w_stream = lm->stream_table;
         return launch_skinny_gemm(bb->stream, MRS_F32, lm->logits, 1, V, hid, dm, table, B, V, dm, none);
     }
     const rocblas_datatype ht = lm->dtype != MRS_F32 ? blas_type(lm->dtype) : rocblas_datatype_f32_r;

@@ -52,7 +52,14 @@ constexpr int kStepsPerBatch = 6;  // k-steps whose loads are issued together (c
 // 16-byte pieces -- whole kilobytes of one row per load instruction instead of 64-byte pieces of 16 rows -- each wave
 // owns two of the workgroup's 16 columns, all of its loads are in flight at once (in groups of JB per column), and
 // the products are v_dot2 with f32 accumulate.  The epilogues are the same code.  MR = rows computed (1, 2 or 4; at 8 rows the route was slower than the matrix-core tiles: 642 vs 435 us per 130m-shape step).
-template <typename T, typename TO, int EPI, int PRO, int LPR = 0, int MR = 1>
+// STREAM: the weight is read past the last cache (row-wise route; ep.w_stream)
+typedef unsigned piece4 __attribute__((ext_vector_type(4)));
+template <bool STREAM, typename T> __device__ __forceinline__ uint4 weight_piece(const T *p) {
+    if constexpr (STREAM) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const piece4 *>(p)));
+    else return *reinterpret_cast<const uint4 *>(p);
+}
+
+template <typename T, typename TO, int EPI, int PRO, int LPR = 0, int MR = 1, bool STREAM = false>
 __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu(6))) void skinny_gemm_kernel(
     TO *__restrict__ C, int64_t ldc, const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt, int M, int N, int K,
     SkinnyEpi ep) {
@@ -203,7 +210,7 @@ __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu
                     if (jb + j < per) {
                         const int off = EPV * LPR * (jb + j);
 #pragma unroll
-                        for (int t = 0; t < NC; t++) wv[t][j] = *reinterpret_cast<const uint4 *>(wp[t] + off);
+                        for (int t = 0; t < NC; t++) wv[t][j] = weight_piece<STREAM>(wp[t] + off);
                         av[j] = *reinterpret_cast<const uint4 *>(A + EPV * ll + off);
                     }
                 }
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu
         for (int j = 0; j < JB; j++)
             if (j < per) {
 #pragma unroll
-                for (int t = 0; t < NC; t++) wv[t][j] = *reinterpret_cast<const uint4 *>(wp[t] + EPV * LPR * j);
+                for (int t = 0; t < NC; t++) wv[t][j] = weight_piece<STREAM>(wp[t] + EPV * LPR * j);
             }
         early_requests();
         lds_barrier();   // the rows are in LDS; the weight loads above stay in flight
@@ -244,7 +251,7 @@ __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu
             for (int j = 0; j < JB; j++)
                 if (jb + JB + j < per) {
 #pragma unroll
-                    for (int t = 0; t < NC; t++) nx[t][j] = *reinterpret_cast<const uint4 *>(wp[t] + EPV * LPR * (jb + JB + j));
+                    for (int t = 0; t < NC; t++) nx[t][j] = weight_piece<STREAM>(wp[t] + EPV * LPR * (jb + JB + j));
                 }
 #pragma unroll
             for (int j = 0; j < JB; j++) {
@@ -571,14 +578,20 @@ static int launch_skinny_t(hipStream_t st, TO *C, int64_t ldc, const T *A, int64
         return fail(MRS_E_SHAPE, "skinny gemm: K split needs the matrix-core route, a plain product, a share buffer and ksplit <= K / 32 (ksplit=%d)", ksplit);
     ep.kslice = ((K >> 5) + ksplit - 1) / ksplit;
     const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 15) / 16), (unsigned)(((K >> 5) + ep.kslice - 1) / ep.kslice));
+#define MRS_SG_ROWS(EPI_, PRO_, LPR_, MR_)                                                                                                                \
+    do {                                                                                                                                                 \
+        const size_t lds = MR_ == 1 ? 0 : (size_t)K * MR_ * sizeof(T);                                                                                   \
+        if (ep.w_stream) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_, true>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep); \
+        else hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep);               \
+    } while (0)
 #define MRS_SG(EPI_, PRO_)                                                                                                               \
     do {                                                                                                                                 \
-        if (lpr == 64 && M == 1) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 64, 1>), grid, block, 0, st, C, ldc, A, lda, Wt, M, N, K, ep); \
-        else if (lpr == 64 && M == 2) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 64, 2>), grid, block, (size_t)K * 2 * sizeof(T), st, C, ldc, A, lda, Wt, M, N, K, ep); \
-        else if (lpr == 32 && M == 2) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 32, 2>), grid, block, (size_t)K * 2 * sizeof(T), st, C, ldc, A, lda, Wt, M, N, K, ep); \
-        else if (lpr == 64) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 64, 4>), grid, block, (size_t)K * 4 * sizeof(T), st, C, ldc, A, lda, Wt, M, N, K, ep);     \
-        else if (lpr == 32 && M == 1) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 32, 1>), grid, block, 0, st, C, ldc, A, lda, Wt, M, N, K, ep); \
-        else if (lpr == 32) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, 32, 4>), grid, block, (size_t)K * 4 * sizeof(T), st, C, ldc, A, lda, Wt, M, N, K, ep);     \
+        if (lpr == 64 && M == 1) MRS_SG_ROWS(EPI_, PRO_, 64, 1);                                                                         \
+        else if (lpr == 64 && M == 2) MRS_SG_ROWS(EPI_, PRO_, 64, 2);                                                                    \
+        else if (lpr == 32 && M == 2) MRS_SG_ROWS(EPI_, PRO_, 32, 2);                                                                    \
+        else if (lpr == 64) MRS_SG_ROWS(EPI_, PRO_, 64, 4);                                                                              \
+        else if (lpr == 32 && M == 1) MRS_SG_ROWS(EPI_, PRO_, 32, 1);                                                                    \
+        else if (lpr == 32) MRS_SG_ROWS(EPI_, PRO_, 32, 4);                                                                              \
         else hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_>), grid, block, 0, st, C, ldc, A, lda, Wt, M, N, K, ep);           \
     } while (0)
     const bool pro = ep.row_scale != 0;
@@ -590,6 +603,7 @@ static int launch_skinny_t(hipStream_t st, TO *C, int64_t ldc, const T *A, int64
     }
     if (pro) MRS_SG(0, 1); else MRS_SG(0, 0);
 #undef MRS_SG
+#undef MRS_SG_ROWS
     return check_launch("skinny_gemm_kernel");
 }
 

@@ -812,6 +812,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenR
                 MRS_TRY(launch_prenorm_rows(bb->stream, dt, bb->partials, P, bb->normed, src ? src : bb->residual, src ? bb->residual : nullptr,
                                             lw.norm_w, B, dm, a_mt, taken ? rows : TokenRows()));
             SkinnyEpi inp = {};
+            inp.w_stream = streams_in_proj(L * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb), B);
             inp.row_scale = 1; inp.partials = bb->partials; inp.n_partials = P; inp.eps = c.rms_norm_eps;
             inp.a_tiled = inp.w_tiled = a_mt ? 1 : 0;
             MRS_TRY(launch_skinny_gemm(bb->stream, dt, bb->proj, 1, ip, bb->normed, dm, a_mt ? lw.in_proj_p : lw.in_proj_t, B, ip, dm, inp));

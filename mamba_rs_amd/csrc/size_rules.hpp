@@ -57,11 +57,11 @@ inline int layers_in_cache(int layers, int64_t layer_bytes, int64_t state_bytes)
     return (int)std::min<int64_t>(layers, std::max<int64_t>(0, ((int64_t)220 << 20) - state_bytes) / std::max<int64_t>(layer_bytes, 1));
 }
 
-// Decode of wide models, a launch per product: in_proj's weights, two thirds of a layer's, are read past that cache where a step (`bytes` of weights and states) outgrows it, so that
+// Decode of a launch per product (wide models, and one to four rows of f32 ones): in_proj's weights, two thirds of a layer's, are read past that cache where a step (`bytes` of weights and states) outgrows it, so that
 // out_proj's and the states may stay and nothing has to be written back for what is read once.  Us a step, bf16, cached / past: d_model 2560, 8 layers 4 rows 322 / 294, 16 358 / 322,
 // 32 438 / 426, 64 577 / 573; 24 layers 4 rows 833 / 808, 16 938 / 877; 2048, 12 layers 4 rows 354 / 331, 16 392 / 370, 48 557 / 563 (there states are most of it).  Some of the
 // layers' through the cache, as layers_in_cache: behind it everywhere (2560, 16 rows, two of eight 341).  out_proj's past it as well: no difference, and where the step kernel asks for
-// its lines ahead that request past it costs 40.
+// its lines ahead that request past it costs 40.  f32, one row, 24 layers, with the head's table past it as well: all cached 383, in_proj's past 341, all past 362 (768); 510, 458, 468 (1024).
 inline bool streams_in_proj(int64_t bytes, int rows) { return rows <= 32 && step_outgrows_cache(bytes); }
 
 // Decode of wide models: whether the step kernel asks for the lines of out_proj (`bytes` of them) on the dies that will read them (m1_step.hip).  They have to stay in the dies' L2, eight
