@@ -757,9 +757,8 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
     {
         static const bool off = [] { const char *e = getenv("MRS_DECODE_LIBRARY_GEMM"); return e && atoi(e) != 0; }();
         // Rows up to which the own chain beats the library chain (in_proj / out_proj from the transposed copies, default
-        // vendor kernels), measured: 128 at the 130m shape (1032 vs 1091 us per step; at 256 rows 1490 vs 1392), 40 at the
-        // 2.8b shape (32 rows 5.13 vs 8.35 ms, 40 rows 5.74 vs 5.92, 48 rows 6.13 vs 5.98, 64 rows 7.58 vs 6.19).  "Narrow"
-        // as for the x_proj shares.
+        // vendor kernels): 128 where own_chain_to_the_last_row says so, 40 at the
+        // 2.8b shape (32 rows 5.13 vs 8.35 ms, 40 rows 5.74 vs 5.92, 48 rows 6.13 vs 5.98, 64 rows 7.58 vs 6.19; 64 with the column-tile kernel).
         // From two (narrow models) or three rows up the projections of the own chain run on the matrix cores and read TILED operands -- weights tiled at load,
         // activation operands written tiled by their producers.  On wide models in_proj / out_proj also run on the
         // column-tile kernel of gemm_wide.hip, which carries the own chain up to 64 rows there.
@@ -773,7 +772,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
         const int tiled_min_rows = forced_min_rows > 0 ? forced_min_rows : (narrow_model(di, xd) ? 2 : 3);
         const bool can_tile = !off && !no_tiled && (dtype == MRS_BF16 || dtype == MRS_F16) && batch >= tiled_min_rows && dm % 32 == 0 && di % 32 == 0 && pow2_state;
         bb->wide = can_tile && batch <= std::min(tiled_max_rows, 64) && (int64_t)dm * 2 * di >= (int64_t)8 << 20 && !narrow_model(di, xd);
-        const int max_rows = std::min(skinny_max_rows(), narrow_model(di, xd) ? 128 : (bb->wide ? 64 : 40));
+        const int max_rows = std::min(skinny_max_rows(), narrow_model(di, xd) || own_chain_to_the_last_row(dm, di) ? 128 : (bb->wide ? 64 : 40));
         bb->skinny = !off && (dtype == MRS_BF16 || dtype == MRS_F16) && batch <= max_rows && dm % 32 == 0 && di % 32 == 0;
         bb->tiled = can_tile && bb->skinny;
         if (!bb->skinny) bb->wide = 0;

@@ -909,8 +909,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
         rocblas_set_pointer_mode(bb->blas, rocblas_pointer_mode_host);
     }
     const int dm = cfg->d_model, di = bb->di, ip = bb->ip, L = cfg->n_layers;
-    // (above 64 rows the library chain is the faster one for this layer: 1261 vs 1318 us per step at 128 rows, 768-wide shape)
-    bb->skinny = (dtype == MRS_BF16 || dtype == MRS_F16) && batch <= std::min(64, skinny_max_rows()) && dm % 32 == 0 && di % 32 == 0;
+    bb->skinny = (dtype == MRS_BF16 || dtype == MRS_F16) && batch <= std::min(own_chain_to_the_last_row(dm, di) ? 128 : 64, skinny_max_rows()) && dm % 32 == 0 && di % 32 == 0;
     // from two rows up the two projections run on the matrix cores and read tiled weights and tiled activation operands
     // (768-wide shape, per step, row-wise / tiled route: 282 / 302 us at 1 row, 326 / 308 at 2, 364 / 308 at 3, 368 / 314 at 4)
     { const char *e = getenv("MRS_DECODE_NO_TILED"), *m = getenv("MRS_DECODE_TILED_MIN_ROWS");

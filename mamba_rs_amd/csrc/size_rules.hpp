@@ -42,6 +42,13 @@ inline int conv_xproj_form(int batch, int T, int di, int xd) {
 // 3266 / 3221, 4 x 4096 5887 / 6038).
 inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
 
+// Rows up to which a decode step's projections are the own kernels'.  Weights of up to ten million elements of in_proj (d_model 1536): as many as those kernels take; past that its
+// tiles of 16 x 16 read too much over again.  Us a step, bf16, library / own:
+//   12 layers of d_model 1024   48 rows 512 / 289, 64 540 / 329, 96 649 / 445, 128 682 / 511         1280   48 593 / 389, 64 675 / 485, 96 681 / 587, 128 821 / 697
+//                   1536        65 rows 668 / 551, 96 735 / 628, 128 840 / 716    six of 1792        65 rows 411 / 399, 96 447 / 464, 128 485 / 554    2560   65 551 / 595, 128 716 / 821
+//   Mamba-3, eight of 512       65 rows 288 / 212, 128 463 / 316    768   65 388 / 293, 128 496 / 420    1024   65 467 / 370, 128 623 / 540    1536   65 589 / 530, 128 841 / 811
+inline bool own_chain_to_the_last_row(int64_t d_model, int64_t d_inner) { return d_model * 2 * d_inner <= 10 * 1000 * 1000; }
+
 // Whether what a decode step touches (`bytes`: weights, states, the head's table) is more than the chip's last cache holds, 256 MB.  What is read once a step and not kept from one
 // step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
 // The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)

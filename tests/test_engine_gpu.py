@@ -282,6 +282,26 @@ def test_narrow_model_keeps_the_own_chain_up_to_128_rows(B):
     eng.close()
 
 
+@pytest.mark.parametrize("dm,B", [(1024, 41), (1024, 65), (1280, 128), (1536, 97)])
+def test_models_of_middle_width_keep_the_own_chain_up_to_128_rows(dm, B):
+    """Widths between those of the narrow models and of the column-tile kernel's, at rows that were the library's: as above."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+    w = MambaWeights.random_lm(cfg, seed=B, std=0.05)
+    P = oracle_params(w, cfg, dm, round_to=orc.BF16)
+    P.input_proj_w[:] = np.eye(dm, dtype=np.float32); P.input_proj_b[:] = 0
+    rng = np.random.default_rng(B)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.BF16)
+    x = rng.standard_normal((3, B, dm)).astype(np.float32)
+    rows = (0, B // 2, B - 1)
+    st = {b: orc.m1_zero_state(P) for b in rows}
+    for t in range(3):
+        got = eng.step(x[t])
+        for b in rows:
+            want = orc.m1_backbone_step(P, x[t, b], *st[b])
+            assert cosine(got[b], want) >= 0.999, (B, t, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("B", [1, 3, 20])
 def test_wide_model_runs_x_proj_as_a_split_k_launch(B):
     """d_inner 2048 x xdbl 96: a row's per-tile shares would be 48 KB, so x_proj does not ride in the in_proj launch; it

@@ -120,7 +120,8 @@ def test_batch_rows_are_independent_and_graph_equals_eager():
 
 
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
-@pytest.mark.parametrize("ci,B", [(0, 2), (1, 2), (0, 7), (1, 21), (2, 16)])
+@pytest.mark.parametrize("ci,B", [(0, 2), (1, 2), (0, 7), (1, 21), (2, 16),
+                                  (0, 65), (2, 113), (1, 128), (0, 129)])   # the last row tiles of the own chain, and past it
 def test_16bit_engine_tracks_cpu_path_on_rounded_weights(dtype, ci, B):
     """bf16/f16 storage (own-GEMM decode chain: folded RMSNorm, residual epilogue) vs the CPU route on weights
     rounded to the storage type: cosine >= 0.999 per step, the reference's mixed-precision bar.  From two rows up the
