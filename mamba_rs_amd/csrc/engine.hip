@@ -369,6 +369,7 @@ static int project_input(mrs_backbone *bb, float *residual, const float *input_d
         MRS_HIP(hipMemcpyAsync(residual, input_dev, rows * dm * sizeof(float), hipMemcpyDeviceToDevice, bb->stream));
         return MRS_OK;
     }
+    if (project_rows_ok(rows, bb->input_dim, dm)) return launch_project_rows(bb->stream, residual, nullptr, input_dev, bb->input_proj_w, bb->input_proj_b, (int)rows, bb->input_dim, dm);
     // bias rows first, then accumulate the GEMM on top (beta = 1)
     {
         const int64_t n = rows * dm;
@@ -906,11 +907,12 @@ extern "C" int mrs_backbone_reset(mrs_backbone *bb) {
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
-static int step_body(mrs_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}) {
+// projected: the projection of its rows is done
+static int step_body(mrs_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}, bool projected = false) {
     if (bb->resident) {
         const ResidentTurn turn(&bb->seat);
         if (turn.go()) {
-            if (!bb->identity_proj) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
+            if (!bb->identity_proj && !projected) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
             return (bb->resident == 1 ? launch_resident_step : launch_resident_rows)(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev, rows);
         }
     }
@@ -930,18 +932,27 @@ static int step_body(mrs_backbone *bb, const HostRows *host = nullptr, const Tok
     // residual stream itself, so no copy is needed
     bb->step_src = taken ? bb->d_input : nullptr;
     bb->step_rows = taken ? rows : TokenRows();
-    if (!bb->step_src) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
+    if (!bb->step_src && !projected) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
     return run_layers(bb, &bb->step_s, 1);
+}
+
+// (the recorded step starts behind an input projection)
+static int step_or_replay(mrs_backbone *bb, bool projected) {
+    const bool one_launch = bb->tiny_layers || bb->resident;   // launched quicker than a graph of one node
+    if (bb->graph_ready && !one_launch) {
+        const ResidentTurn turn(&bb->seat);
+        if (turn.go()) {
+            if (!bb->identity_proj && !projected) MRS_TRY(project_input(bb, bb->step_s.residual, bb->d_input, bb->batch));
+            MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream));
+            return MRS_OK;
+        }
+    }
+    return step_body(bb, nullptr, {}, projected);
 }
 
 extern "C" int mrs_backbone_step_gpu_only(mrs_backbone *bb) {
     if (!bb) return fail(MRS_E_NULL, "mrs_backbone_step_gpu_only: null engine");
-    const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
-    if (bb->graph_ready && !one_launch) {
-        const ResidentTurn turn(&bb->seat);
-        if (turn.go()) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
-    }
-    return step_body(bb);
+    return step_or_replay(bb, false);
 }
 
 extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *output) {
@@ -954,8 +965,10 @@ extern "C" int mrs_backbone_step(mrs_backbone *bb, const float *input, float *ou
     if (bb->tiny_layers) {
         MRS_TRY(step_body(bb, &host));
     } else {
-        hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
-        MRS_TRY(mrs_backbone_step_gpu_only(bb));
+        const bool projected = !bb->identity_proj && project_rows_ok(B, bb->input_dim, dm);
+        if (projected) MRS_TRY(launch_project_rows(bb->stream, bb->step_s.residual, bb->d_input, io.in, bb->input_proj_w, bb->input_proj_b, B, bb->input_dim, dm));
+        else hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
+        MRS_TRY(step_or_replay(bb, projected));
         hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
         MRS_TRY(check_launch("host row kernels"));
     }
@@ -994,7 +1007,7 @@ extern "C" int mrs_backbone_capture_graph(mrs_backbone *bb) {
     MRS_TRY(check_resident(bb));
     const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
-    rc = step_body(bb);
+    rc = step_body(bb, nullptr, {}, !bb->identity_proj);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(bb->stream, &g);
     if (rc) { if (g) hipGraphDestroy(g); return rc; }

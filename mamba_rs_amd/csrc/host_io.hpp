@@ -76,6 +76,62 @@ static __global__ __launch_bounds__(256) void host_in_kernel(float *__restrict__
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) dst[i] = src[i];
 }
+// A step's input projection: out[row][n] = bias[n] + sum_k in[row][k] W[k][n], W [K][N] row-major, N a multiple of 4, and the row once more into `copy` (or null): it may come
+// straight from host memory.  A workgroup has a row: a thread four consecutive columns over one slice of K, its first eight weight rows on their way while the row is, and the
+// slices' sums meet in LDS.  Bound by its trips to memory.  As a kernel for the bias, the library's product (about 5 us for one row) and, from host memory, a copy in front, they
+// were three launches: a step of four bf16 layers of d_model 128, 1 row 51 us, this 41 (48 rows 85 / 78); Mamba-3 53 / 41 and 73 / 68; four f32 layers of 192, 48 rows, 120 / 111.
+constexpr int kProjThreads = 512, kProjMaxK = 4096;
+inline bool project_rows_ok(int64_t rows, int K, int N) { return rows >= 1 && rows <= 128 && K >= 1 && K <= kProjMaxK && N >= 4 && N % 4 == 0 && N <= 4 * kProjThreads; }
+static __global__ __launch_bounds__(kProjThreads) void project_rows_kernel(float *__restrict__ out, float *__restrict__ copy, const float *__restrict__ in, const float *__restrict__ W,
+                                                                            const float *__restrict__ bias, int K, int N) {
+    extern __shared__ float proj_x[];   // [slices][rows of a slice, in whole rounds], zeros behind K
+    __shared__ float4 part[kProjThreads];
+    constexpr int kRound = 8;
+    const int tid = threadIdx.x, nq = N >> 2, slices = kProjThreads / nq, per = (K + slices - 1) / slices, padded = (per + kRound - 1) / kRound * kRound;
+    const int q = tid % nq, s = min(tid / nq, slices - 1), k0 = s * per;   // (threads behind the last slice repeat it)
+    const int64_t row = blockIdx.x;
+    float4 w[kRound];
+    auto ask = [&](int j0) {
+#pragma unroll
+        for (int j = 0; j < kRound; j++) w[j] = *reinterpret_cast<const float4 *>(W + (int64_t)min(k0 + j0 + j, K - 1) * N + 4 * q);
+    };
+    ask(0);
+    for (int i = tid; i < slices * padded; i += kProjThreads) {
+        const int sl = i / padded, j = i - sl * padded, k = sl * per + j;
+        float v = 0.0f;
+        if (j < per && k < K) {
+            v = in[row * K + k];
+            if (copy) copy[row * K + k] = v;
+        }
+        proj_x[i] = v;
+    }
+    __syncthreads();
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j0 = 0; j0 < per; j0 += kRound) {
+        if (j0) ask(j0);
+#pragma unroll
+        for (int j = 0; j < kRound; j++) {
+            const float x = proj_x[s * padded + j0 + j];
+            acc.x = fmaf(x, w[j].x, acc.x); acc.y = fmaf(x, w[j].y, acc.y); acc.z = fmaf(x, w[j].z, acc.z); acc.w = fmaf(x, w[j].w, acc.w);
+        }
+    }
+    part[tid] = acc;
+    __syncthreads();
+    if (tid < nq) {
+        float4 o = *reinterpret_cast<const float4 *>(bias + 4 * tid);
+        for (int t = 0; t < slices; t++) {
+            const float4 p = part[t * nq + tid];
+            o.x += p.x; o.y += p.y; o.z += p.z; o.w += p.w;
+        }
+        *reinterpret_cast<float4 *>(out + row * N + 4 * tid) = o;
+    }
+}
+inline int launch_project_rows(hipStream_t st, float *out, float *copy, const float *in, const float *W, const float *bias, int rows, int K, int N) {
+    const int slices = kProjThreads / (N / 4), per = (K + slices - 1) / slices;
+    hipLaunchKernelGGL(project_rows_kernel, dim3((unsigned)rows), dim3(kProjThreads), (size_t)slices * ((per + 7) / 8 * 8) * 4, st, out, copy, in, W, bias, K, N);
+    return check_launch("project_rows_kernel");
+}
+
 static __global__ __launch_bounds__(256) void host_out_kernel(HostRows h, const float *__restrict__ rows, int dm) {
     const int r = blockIdx.x;
     for (int i = threadIdx.x; i < dm; i += 256) host_store(h.out + (size_t)r * dm + i, rows[(size_t)r * dm + i]);

@@ -644,6 +644,7 @@ int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
 int project_input3(mrs_m3_backbone *bb) {
     const int B = bb->batch, dm = bb->cfg.d_model;
     const int64_t n = (int64_t)B * dm;
+    if (project_rows_ok(B, bb->input_dim, dm)) return launch_project_rows(bb->stream, bb->residual, nullptr, bb->d_input, bb->input_proj_w, bb->input_proj_b, B, bb->input_dim, dm);
     hipLaunchKernelGGL(bias_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->residual, bb->input_proj_b, n, dm);
     const float one = 1.0f;
     MRS_BLAS(rocblas_gemm_ex(bb->blas, rocblas_operation_none, rocblas_operation_none, dm, B, bb->input_dim, &one, bb->input_proj_w,
@@ -772,12 +773,13 @@ bool go_on_chain3(mrs_m3_backbone *bb) {
 }
 
 // host: where the rows of a step that starts from bb->io.in go (tiny models do both themselves), or null
-int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}) {
+// projected: the projection of its rows is done
+int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenRows &rows = {}, bool projected = false) {
     const mrs_m3_config &c = bb->cfg;
     if (bb->resident) {
         const ResidentTurn turn(&bb->seat);
         if (turn.go()) {
-            if (!bb->identity_proj) MRS_TRY(project_input3(bb));
+            if (!bb->identity_proj && !projected) MRS_TRY(project_input3(bb));
             return launch_resident_m3_step(bb->stream, bb->dtype, bb->res_args, bb->res_args_dev, rows);
         }
     }
@@ -802,7 +804,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenR
     if (bb->identity_proj) {
         if (taken) src = bb->d_input;   // the first prenorm kernel reads the input and writes the residual stream
         else MRS_HIP(hipMemcpyAsync(bb->residual, bb->d_input, (size_t)B * dm * 4, hipMemcpyDeviceToDevice, bb->stream));
-    } else {
+    } else if (!projected) {
         MRS_TRY(project_input3(bb));
     }
     for (int l = 0; l < L; l++) {
@@ -1006,14 +1008,23 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     return MRS_OK;
 }
 
-extern "C" int mrs_m3_backbone_step_gpu_only(mrs_m3_backbone *bb) {
-    if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_step_gpu_only: null engine");
-    const bool one_launch = bb->tiny_layers || (bb->resident && bb->identity_proj);   // launched quicker than a graph of one node
+// (the recorded step starts behind an input projection)
+static int step_or_replay3(mrs_m3_backbone *bb, bool projected) {
+    const bool one_launch = bb->tiny_layers || bb->resident;   // launched quicker than a graph of one node
     if (bb->graph_ready && !one_launch) {
         const ResidentTurn turn(&bb->seat);
-        if (turn.go()) { MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream)); return MRS_OK; }
+        if (turn.go()) {
+            if (!bb->identity_proj && !projected) MRS_TRY(project_input3(bb));
+            MRS_HIP(hipGraphLaunch(bb->graph_exec, bb->stream));
+            return MRS_OK;
+        }
     }
-    return step_body3(bb);
+    return step_body3(bb, nullptr, {}, projected);
+}
+
+extern "C" int mrs_m3_backbone_step_gpu_only(mrs_m3_backbone *bb) {
+    if (!bb) return fail(MRS_E_NULL, "mrs_m3_backbone_step_gpu_only: null engine");
+    return step_or_replay3(bb, false);
 }
 
 extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, float *output) {
@@ -1026,8 +1037,10 @@ extern "C" int mrs_m3_backbone_step(mrs_m3_backbone *bb, const float *input, flo
     if (bb->tiny_layers) {
         MRS_TRY(step_body3(bb, &host));
     } else {
-        hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
-        MRS_TRY(mrs_m3_backbone_step_gpu_only(bb));
+        const bool projected = !bb->identity_proj && project_rows_ok(B, bb->input_dim, dm);
+        if (projected) MRS_TRY(launch_project_rows(bb->stream, bb->residual, bb->d_input, io.in, bb->input_proj_w, bb->input_proj_b, B, bb->input_dim, dm));
+        else hipLaunchKernelGGL(host_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bb->stream, bb->d_input, io.in, n);
+        MRS_TRY(step_or_replay3(bb, projected));
         hipLaunchKernelGGL(host_out_kernel, dim3((unsigned)B), dim3(256), 0, bb->stream, host, bb->temporal, dm);
         MRS_TRY(check_launch("host row kernels"));
     }
@@ -1070,7 +1083,7 @@ extern "C" int mrs_m3_backbone_capture_graph(mrs_m3_backbone *bb) {
     MRS_TRY(check_resident3(bb));
     const ResidentRecording rec(&bb->seat);
     MRS_HIP(hipStreamBeginCapture(bb->stream, hipStreamCaptureModeThreadLocal));
-    rc = step_body3(bb);
+    rc = step_body3(bb, nullptr, {}, !bb->identity_proj);
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(bb->stream, &g);
     if (rc) { if (g) hipGraphDestroy(g); return rc; }

@@ -562,6 +562,34 @@ def test_rows_a_step_hands_to_the_host_are_the_rows_it_leaves_on_the_device(dm, 
     eng.close()
 
 
+@pytest.mark.parametrize("dm,idim,B", [(192, 1, 1), (192, 9, 3), (160, 513, 2), (320, 88, 128), (320, 88, 129), (36, 4096, 2), (36, 4097, 2)])
+def test_input_rows_through_the_projection_kernel(dm, idim, B):
+    """One row's product per workgroup, from host memory (step) and from the device (step_gpu_only), eager and in front of a recorded step; past 128 rows or 4096 inputs the library's.
+    f32: sums of at most 4097 terms in another order, 1e-4 of the scale as above."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, idim, 5)
+    rng = np.random.default_rng(idim)
+    w.input_proj_b[:] = rng.standard_normal(dm)
+    P = oracle_params(w, cfg, idim)
+    print(f"case projected rows {dm} {idim} {B}", flush=True)
+    eng = GpuMambaBackbone.new(0, w, cfg, idim, B)
+    rows = sorted({0, B // 2, B - 1})
+    st = {b: orc.m1_zero_state(P) for b in rows}
+    for t in range(6):
+        x = rng.standard_normal((B, idim)).astype(np.float32)
+        if t == 2:
+            eng.capture_graph()
+        got = eng.step(x)
+        for b in rows:
+            assert scaled_err(got[b], orc.m1_backbone_step(P, x[b], *st[b])) < 1e-4, (t, b)
+        if t % 2:   # the same rows once more: they are on the device
+            eng.step_gpu_only()
+            got = eng.download_temporal()
+            for b in rows:
+                assert scaled_err(got[b], orc.m1_backbone_step(P, x[b], *st[b])) < 1e-4, (t, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,lens,dtype", [
     (128, (9, 5), WeightDtype.F16),              # four tokens; dt_rank 8: a quarter of a k-step of dt_proj
     (256, (6, 40, 18), WeightDtype.BF16),        # five
