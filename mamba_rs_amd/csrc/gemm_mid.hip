@@ -9,13 +9,15 @@
 //     rows a matrix operand takes the same piece of spread over the banks (the lanes fetch permuted pieces of the same line:
 //     the copy itself writes in lane order);
 //   * workgroups are numbered so that the units of one die (block index modulo 8) share column tiles: each die's L2 then takes in an
-//     eighth of the weight instead of all of it.
+//     eighth of the weight instead of all of it;
+//   * K may be cut into slices over the second grid dimension, which leave f32 products side by side.
 // It is bound by what a compute unit takes in (about 34 bytes a clock).  In a bf16 prefill, vendor / this: 64 x 3072 x 768 7.6 / 6.1 us, 64 x 768 x 1536
 // 7.8 / 8.5, 777 x 4096 x 1024 14.5 / 16.2, 777 x 1024 x 2048 12.9 / 11.1, 1500 x 768 x 1536 13.8 / 11.0, 300 x 2560 x 5120 27.2 / 26.0.  Also measured: more
 // buffers (6, 8: fewer workgroups per unit, 24 us at 777 x 4096 x 1024), tiles of 128 x 128 (15.8 there, 23 at 777 x 1024 x 2048) and
 // 64 x 128 (18.3 / 14.7), and the operands of the next k-step read from LDS under the products (no change).
 #include "common.hpp"
 #include "mfma_tiles.hpp"
+#include <algorithm>
 
 namespace mrs {
 namespace {
@@ -24,7 +26,7 @@ constexpr int kMidThreads = 256, kTile = 64, kStepK = 64, kStages = 4;
 
 template <typename T, typename TO>
 __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ C, int64_t ldc, const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt,
-                                                               int M, int N, int K, int mtiles) {
+                                                               int M, int N, int K, int mtiles, int per) {
     constexpr int MT = kTile / 32, NT = kTile / 32;             // 16 x 16 tiles of a wave
     constexpr int kRows = 2 * kTile, kStage = kRows * 2 * kStepK;  // bytes of a k-step: A's rows, then Wt's
     constexpr int kLoads = kRows / 8 / 4;                      // 1 KB requests of a wave per k-step
@@ -32,7 +34,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ 
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
     const int total = gridDim.x, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
     const int p = xcd * each + min(xcd, rest) + (blockIdx.x >> 3);
-    const int m0 = p % mtiles * kTile, n0 = p / mtiles * kTile, nk = K / kStepK;
+    const int m0 = p % mtiles * kTile, n0 = p / mtiles * kTile, ks0 = blockIdx.y * per, nk = min(K / kStepK - ks0, per);   // this slice's k-steps
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
     // request q of a wave: rows 8 (w + 4 q) .. + 7 of the stage, lane l row l / 8 and place l % 8; rows past the end repeat the last
@@ -42,7 +44,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ 
         const int r = 8 * (w + 4 * q) + (l >> 3), piece = (l & 7) ^ (l >> 3);
         const bool is_a = 8 * (w + 4 * q) < kTile;   // (the same for the wave)
         const unsigned row = is_a ? (unsigned)min(m0 + r, M - 1) * (unsigned)lda : (unsigned)min(n0 + r - kTile, N - 1) * (unsigned)K;
-        voff[q] = (row + 8u * (unsigned)piece) * 2u;
+        voff[q] = (row + 8u * (unsigned)piece) * 2u + (unsigned)ks0 * (2u * kStepK);
     }
     auto request = [&](int kt) {
         const unsigned buf = lds0 + (unsigned)(kt % kStages) * kStage;
@@ -84,6 +86,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ 
                 for (int j = 0; j < NT; j++) acc[i][j] = Mma32<T>::mma(wf[j], af[i], acc[i][j]);   // (transposed: a lane holds four columns of a row)
         }
     }
+    C += (int64_t)blockIdx.y * M * ldc;
 #pragma unroll
     for (int i = 0; i < MT; i++) {
         const int row = m0 + wm + 16 * i + lr;
@@ -101,12 +104,14 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ 
 }
 
 template <typename T, typename TO>
-int launch_mid(hipStream_t st, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int M, int N, int K) {
+int launch_mid(hipStream_t st, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int M, int N, int K, int slices = 1) {
     constexpr size_t lds = (size_t)kStages * 2 * kTile * 2 * kStepK;
     static const hipError_t attr = hipFuncSetAttribute((const void *)gemm_mid_kernel<T, TO>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "mid gemm: LDS size: %s", hipGetErrorString(attr));
     const int mt = (M + kTile - 1) / kTile, nt = (N + kTile - 1) / kTile;
-    hipLaunchKernelGGL((gemm_mid_kernel<T, TO>), dim3((unsigned)(mt * nt)), dim3(kMidThreads), lds, st, (TO *)C, ldc, (const T *)A, lda, (const T *)Wt, M, N, K, mt);
+    const int steps = K / kStepK, per = (steps + slices - 1) / slices;
+    hipLaunchKernelGGL((gemm_mid_kernel<T, TO>), dim3((unsigned)(mt * nt), (unsigned)((steps + per - 1) / per)), dim3(kMidThreads), lds, st, (TO *)C, ldc, (const T *)A, lda,
+                       (const T *)Wt, M, N, K, mt, per);
     return check_launch("gemm_mid_kernel");
 }
 
@@ -121,6 +126,21 @@ bool mid_gemm_wins(int64_t M, int N, int K) {
     return steps <= 40 && (tiles <= 256 || tiles * steps <= 10000);
 }
 
+// Slices of K for out_proj, whose products the next kernel sums (it reads the result anyway).  A compute unit takes in some 60 bytes a nanosecond whatever it has asked for, so 24
+// tiles of 64 x 64 over K 1536 take 10 us with nine tenths of the chip idle.  As many slices as make a workgroup for every unit, or two where their walk stays
+// long, four at most.  Us a layer of a bf16 prefill, one / two / three / four slices (six and eight: four's or behind):
+//   d_model 768   64 rows 54.1 / 51.5 / 50.5 / 50.1    256 63.8 / 60.8 / 60.0 / 59.3    512 71.8 / 68.7 / 69.8 / 69.2    1024 83.9 / 85.6 / 87.2 / 87.4
+//           1024  64 rows 65.5 / 61.9 / 60.7 / 60.0    256 71.2 / 66.9 / 65.5 / 65.4    512 79.6 / 75.9 / 77.1 / 77.1    777 92.0 / 91.5 / 93.0 / 94.3
+//           2560  64 rows 129 / 128 / 125 / 124        128 154 / 141 / 139 / 141        256 172 / 170 / 164 / 167 (one: the vendor kernel)
+//   Mamba-3 768   256 rows 80.5 / 77.8 / 77.0 / 76.7   512 84.9 / 82.0 / 82.8 / 82.5
+int mid_gemm_slices(int64_t M, int N, int K) {
+    const int64_t tiles = (M + kTile - 1) / kTile * ((N + kTile - 1) / kTile), steps = K / kStepK;
+    const int64_t want = std::min<int64_t>(std::min(std::max(256 / tiles, std::min(512 / tiles, steps / 24)), steps / 3), kMaxMidSlices);
+    if (want < 2 || K % kStepK != 0) return 1;
+    const int64_t per = (steps + want - 1) / want;
+    return (int)((steps + per - 1) / per);
+}
+
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {
     return (dtype == MRS_BF16 || dtype == MRS_F16) && M >= 1 && N >= 4 && N % 4 == 0 && K >= kStepK && K % kStepK == 0 && lda % 8 == 0 && lda >= K && ldc % 4 == 0 &&
            ldc >= N && aligned(C, out_f32 ? 16 : 8) && aligned(A, 16) && aligned(Wt, 16) && M * lda < (int64_t)1 << 30 && (int64_t)N * K < (int64_t)1 << 30;
@@ -132,6 +152,11 @@ int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc
     if (dtype == MRS_BF16)
         return out_f32 ? launch_mid<bf16_t, float>(st, C, ldc, A, lda, Wt, (int)M, N, K) : launch_mid<bf16_t, bf16_t>(st, C, ldc, A, lda, Wt, (int)M, N, K);
     return out_f32 ? launch_mid<f16_t, float>(st, C, ldc, A, lda, Wt, (int)M, N, K) : launch_mid<f16_t, f16_t>(st, C, ldc, A, lda, Wt, (int)M, N, K);
+}
+
+int launch_mid_gemm_parts(hipStream_t st, int dtype, float *parts, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K, int slices) {
+    if (!mid_gemm_ok(dtype, 1, parts, N, A, lda, Wt, M, N, K) || slices < 1 || slices > K / kStepK) return fail(MRS_E_SHAPE, "mid gemm: %d slices of M=%lld N=%d K=%d", slices, (long long)M, N, K);
+    return dtype == MRS_BF16 ? launch_mid<bf16_t, float>(st, parts, N, A, lda, Wt, (int)M, N, K, slices) : launch_mid<f16_t, float>(st, parts, N, A, lda, Wt, (int)M, N, K, slices);
 }
 
 }  // namespace mrs

@@ -179,6 +179,81 @@ __global__ __launch_bounds__(256) void add_rmsnorm_block_kernel(float *__restric
     }
 }
 
+// The same where the product to add lies in slices of K, parts [n][rows][dm] f32 (launch_mid_gemm_parts): their sum, in slice order, is rounded to the storage type as the whole
+// product would have been.  All slices' pieces are on their way together.
+template <typename T, int TRIPS>
+__global__ __launch_bounds__(256) void add_rmsnorm_parts_kernel(float *__restrict__ residual, const float *__restrict__ parts, int n, int64_t stride, T *__restrict__ out,
+                                                                const float *__restrict__ w, float eps, int dm) {
+    __shared__ float part[4];
+    const int64_t row = blockIdx.x;
+    const int nv = dm >> 2;
+    float4 *r4 = reinterpret_cast<float4 *>(residual + row * dm);
+    struct alignas(4 * sizeof(T)) V4 { T v[4]; };
+    const float4 *w4 = reinterpret_cast<const float4 *>(w);
+    float4 v[TRIPS], ww[TRIPS], s[TRIPS];
+#pragma unroll
+    for (int k = 0; k < TRIPS; k++) {
+        const int c = min((int)threadIdx.x + 256 * k, nv - 1);
+        v[k] = r4[c];
+        ww[k] = w4[c];
+        s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float4 a[kMaxMidSlices][TRIPS];
+#pragma unroll
+    for (int q = 0; q < kMaxMidSlices; q++)
+#pragma unroll
+        for (int k = 0; k < TRIPS; k++)
+            a[q][k] = reinterpret_cast<const float4 *>(parts + min(q, n - 1) * stride + row * dm)[min((int)threadIdx.x + 256 * k, nv - 1)];
+#pragma unroll
+    for (int q = 0; q < kMaxMidSlices; q++)
+        if (q < n) {
+#pragma unroll
+            for (int k = 0; k < TRIPS; k++) { s[k].x += a[q][k].x; s[k].y += a[q][k].y; s[k].z += a[q][k].z; s[k].w += a[q][k].w; }
+        }
+    float ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < TRIPS; k++) {
+        const int c = threadIdx.x + 256 * k;
+        V4 a;
+        Store<T>::st(&a.v[0], s[k].x); Store<T>::st(&a.v[1], s[k].y); Store<T>::st(&a.v[2], s[k].z); Store<T>::st(&a.v[3], s[k].w);
+        if (c < nv) {
+            v[k].x += Store<T>::ld(&a.v[0]); v[k].y += Store<T>::ld(&a.v[1]); v[k].z += Store<T>::ld(&a.v[2]); v[k].w += Store<T>::ld(&a.v[3]);
+            r4[c] = v[k];
+            ss = fmaf(v[k].x, v[k].x, ss); ss = fmaf(v[k].y, v[k].y, ss); ss = fmaf(v[k].z, v[k].z, ss); ss = fmaf(v[k].w, v[k].w, ss);
+        }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = part[0] + part[1] + part[2] + part[3];
+    float rms = sqrtf(ss / (float)dm + eps);
+    if (!isfinite(rms) || rms < 1e-20f) rms = 1.0f;
+    const float inv = 1.0f / rms;
+    V4 *o4 = reinterpret_cast<V4 *>(out + row * dm);
+#pragma unroll
+    for (int k = 0; k < TRIPS; k++) {
+        const int c = threadIdx.x + 256 * k;
+        if (c < nv) {
+            V4 o;
+            Store<T>::st(&o.v[0], v[k].x * inv * ww[k].x); Store<T>::st(&o.v[1], v[k].y * inv * ww[k].y);
+            Store<T>::st(&o.v[2], v[k].z * inv * ww[k].z); Store<T>::st(&o.v[3], v[k].w * inv * ww[k].w);
+            o4[c] = o;
+        }
+    }
+}
+inline bool add_rmsnorm_parts_ok(int dm) { return dm % 4 == 0 && dm <= 4096; }
+inline int launch_add_rmsnorm_parts(hipStream_t st, int dtype, float *residual, const float *parts, int n, void *out, const float *w, float eps, int64_t rows, int dm) {
+    const dim3 grid((unsigned)rows), block(256);
+#define MRS_PARTS(TR) MRS_DISPATCH_DTYPE(dtype, T_, hipLaunchKernelGGL((add_rmsnorm_parts_kernel<T_, TR>), grid, block, 0, st, residual, parts, n, rows * dm, (T_ *)out, w, eps, dm))
+    const int trips = (dm / 4 + 255) / 256;
+    if (trips <= 1) { MRS_PARTS(1); }
+    else if (trips <= 2) { MRS_PARTS(2); }
+    else { MRS_PARTS(4); }
+#undef MRS_PARTS
+    return check_launch("add_rmsnorm_parts_kernel");
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void cast_from_f32_kernel(T *__restrict__ out, const float *__restrict__ in, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

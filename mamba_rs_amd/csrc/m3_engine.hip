@@ -587,6 +587,8 @@ struct mrs_m3_backbone {
     float *pf_dtT, *pf_aT, *pf_trapT;   // [batch, nh, T] copies of dt, a, trap for the scan that forms K and Q itself
     double *pf_angle_sums;   // [batch][kAngleSegs][nh * n_rope] per-segment angle increments of the prefill
     void *pf_bcn;            // [rows][2 * d_state] normalised and weighted B | C rows (activation type) for the scan that forms K and Q itself
+    float *pf_parts;        // out_proj as pf_n_parts products over slices of K, [pf_n_parts][rows][d_model] (few rows)
+    int pf_n_parts;
     void *pf_normed, *pf_bulk, *pf_x, *pf_K, *pf_Q, *pf_y, *pf_gated, *pf_out, *pf_ws;
     size_t pf_ws_bytes;
 };
@@ -1152,6 +1154,8 @@ static int alloc_prefill_scratch3(mrs_m3_backbone *bb, int T) {
     MRS_TRY(dev_alloc3(bb, &bb->pf_y, rows * di * es));
     MRS_TRY(dev_alloc3(bb, &bb->pf_gated, rows * di * es));
     MRS_TRY(dev_alloc3(bb, &bb->pf_out, rows * dm * es));
+    bb->pf_n_parts = bb->dtype != MRS_F32 && add_rmsnorm_parts_ok((int)dm) ? mid_gemm_slices(rows, (int)dm, (int)di) : 1;
+    if (bb->pf_n_parts > 1) MRS_TRY(dev_alloc3(bb, (void **)&bb->pf_parts, (size_t)bb->pf_n_parts * rows * dm * sizeof(float)));
     size_t wsb = mrs_m3_ssd_workspace_bytes(bb->batch, T, (int)nh, c.headdim, c.d_state, 64);
     const size_t abg = 3 * rows * nh * 4;   // alpha, beta, gamma for shapes the chunked kernel does not take
     if (abg > wsb) wsb = abg;
@@ -1237,7 +1241,9 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         const Layer3 &lw = bb->layers[l];
         float *ssm = bb->ssm + (size_t)l * B * nh * hd * ds, *kst = bb->kst + (size_t)l * B * nh * ds;
         float *vst = bb->vst + (size_t)l * B * nh * hd, *ang = bb->angle + (size_t)l * B * nh * (nr > 0 ? nr : 1);
-        MRS_TRY(launch_add_rmsnorm3(bb, bb->pf_residual, l == 0 ? nullptr : bb->pf_out, bb->pf_normed, false, lw.norm_w, rows));
+        const bool in_parts = bb->pf_n_parts > 1 && mid_gemm_ok(dt, 1, bb->pf_parts, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di);   // (the same for every layer)
+        if (in_parts && l > 0) MRS_TRY(launch_add_rmsnorm_parts(bb->stream, dt, bb->pf_residual, bb->pf_parts, bb->pf_n_parts, bb->pf_normed, lw.norm_w, c.rms_norm_eps, rows, dm));
+        else MRS_TRY(launch_add_rmsnorm3(bb, bb->pf_residual, l == 0 ? nullptr : bb->pf_out, bb->pf_normed, false, lw.norm_w, rows));
         // in_proj.  The bulk columns (z, x) come out in the storage type; B, C, the head scalars and the angle inputs
         // (the last 2 ng ds + 3 nh + nr columns) in f32 whatever the storage type, as the decode step sees them -- two
         // GEMMs over column slices of the same weight for 16-bit storage (or the own kernel over all of them), one for f32.  (The bulk slice is 2 d_inner wide
@@ -1342,6 +1348,8 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         if (!gate_in_scan) MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_gate_t<T_>(bb, lw, rows, bulk, ldb)));
         if (last)
             MRS_TRY(launch_last_step_gemm(bb->stream, dt, bb->pf_out, bb->pf_gated, lw.out_proj_t, B, T, dm, di));
+        else if (in_parts && l + 1 < L)
+            MRS_TRY(launch_mid_gemm_parts(bb->stream, dt, bb->pf_parts, bb->pf_gated, di, lw.out_proj_t, rows, dm, di, bb->pf_n_parts));
         else if (const OwnProjection own = own_projection(bb, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
             MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di));
         else if (lw.out_proj_t) {   // (the vendor kernels for the transposed operand: 16384 x 768 x 1536 44.4 -> 41.0 us)

@@ -44,6 +44,34 @@ def test_prefill_of_few_rows_follows_the_cpu_route(dm, B, T, dtype):
         assert cosine(conv[b][:, 1:], cs) >= 0.999 and scaled_err(conv[b][:, 1:], cs) < 5e-2, (b, cosine(conv[b][:, 1:], cs))
 
 
+@pytest.mark.parametrize("dm,B,T,dtype", [
+    (192, 3, 43, WeightDtype.BF16),     # six k-steps in two slices; 129 rows
+    (320, 1, 63, WeightDtype.F16),      # ten in three, the last of two; a row tile short of its last row
+    (448, 1, 130, WeightDtype.BF16),    # fourteen in four, the last of two
+    (384, 2, 8, WeightDtype.F16),       # sixteen rows, four slices of three
+    (1088, 1, 40, WeightDtype.BF16),    # rows of more than one piece a lane
+    (768, 1, 700, WeightDtype.BF16),    # one slice: tiles for half of the units
+])
+def test_out_proj_in_slices_of_k(dm, B, T, dtype):
+    """Two layers: the first one's out_proj leaves products over slices of K, which the second one's norm sums.  Bounds as above."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+    w = MambaWeights.init(cfg, dm, 7)
+    P = oracle_params(w, cfg, dm, round_to=orc.BF16 if dtype == WeightDtype.BF16 else orc.F16)
+    x = (np.random.default_rng(dm + T).standard_normal((B, T, dm)) * 0.5).astype(np.float32)
+    print(f"case out_proj in slices d_model={dm} rows={B * T} {dtype.name}", flush=True)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    last = eng.prefill_sequence(x)
+    state = [eng.download_state(l) for l in range(2)]
+    eng.close()
+    for b in range(B):
+        c, s = orc.m1_zero_state(P)
+        want = orc.m1_backbone_prefill(P, x[b], c, s)[-1]
+        assert cosine(last[b], want) >= 0.999 and scaled_err(last[b], want) < 5e-2, (b, cosine(last[b], want), scaled_err(last[b], want))
+        for l in range(2):
+            hs = s[l].reshape(2 * dm, 16)
+            assert cosine(state[l][1][b], hs) >= 0.999 and scaled_err(state[l][1][b], hs) < 5e-2, (b, l, cosine(state[l][1][b], hs), scaled_err(state[l][1][b], hs))
+
+
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
 @pytest.mark.parametrize("dm,B,T", [
     (128, 33, 1000),   # tiles of 192 columns, the last a third empty; two k-steps, one pair of buffers
