@@ -133,6 +133,7 @@ struct SkinnyEpi {
     int prenorm_mt;      // mode 2: != 0 writes prenorm in that tiled order (prenorm_mt row tiles) for the next tiled in_proj
     // matrix-core route of gemm_skinny.hip: the weight is the tiled copy (launch_tile_weight) instead of Wt[N][K]
     int w_tiled;
+    int f32_rows;            // f32 storage past four rows or K % 128: on the matrix cores' f32 instructions
     int w_stream;            // (gemm_wide.hip) the weight is read past the last cache
     // mode 1, optional: a second copy of u in tiled order (u_tiled_mt row tiles), the operand of a tiled x_proj
     void *u_tiled;

@@ -435,7 +435,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         }
         SkinnyEpi inp = {};
         inp.mode = 1; inp.conv_state = conv; inp.conv_w = lw.conv_w; inp.conv_b = lw.conv_b; inp.u = u; inp.di = di; inp.dc = dc;
-        inp.row_scale = 1; inp.partials = partials; inp.n_partials = P; inp.eps = bb->cfg.rms_norm_eps;
+        inp.row_scale = 1; inp.partials = partials; inp.n_partials = P; inp.eps = bb->cfg.rms_norm_eps; inp.f32_rows = 1;
         const bool fold_x = xpart && nr <= fold_rows_for(di, xd) && xd <= 256 && (int64_t)(di / 16) * nr * xd <= s->xpart_floats && lw.dt_t_step &&
                             di % (1024 / ds) == 0 && dr % 4 == 0 && (int64_t)nr * dr <= fuse_limit;
         if (fold_x) { inp.xw = lw.x_proj; inp.xd = xd; inp.xpart = xpart; }
@@ -459,6 +459,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
         const SkinnyEpi none = {};
         if (!fold_x) {
             SkinnyEpi xp = {};
+            xp.f32_rows = 1;
             if (ksplit > 1) { xp.ksplit = ksplit; xp.xpart = xpart; }
             if (a_mt) {
                 xp.a_tiled = 1; xp.w_tiled = 1;
@@ -478,6 +479,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
                                           (fold_x || ksplit > 1) ? &fold : nullptr, a_mt));
         }
         SkinnyEpi outp = {};
+        outp.f32_rows = 1;
         outp.mode = 2; outp.residual = residual; outp.partials = partials; outp.n_partials = P;
         outp.next_norm_w = l + 1 < L ? bb->layers[l + 1].norm_w : nullptr; outp.prenorm = normed;
         if (a_mt) {
@@ -765,6 +767,10 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
         else { MRS_CREATE_TRY(dev_alloc(bb, (void **)&bb->input_proj_b, dm * 4)); hipMemsetAsync(bb->input_proj_b, 0, dm * 4, bb->stream); }
     }
     bb->layers.resize(L);
+    const bool tiny = [&] {   // small f32 models: a step is one launch (MRS_DECODE_NO_TINY=1 keeps the kernel chains)
+        const char *e = getenv("MRS_DECODE_NO_TINY");
+        return !(e && atoi(e) != 0) && tiny_step_ok(dtype, input_dim, dm, di, ds, dc, dr, xd) && (!identity || input_dim == dm);
+    }();
     {
         static const bool off = [] { const char *e = getenv("MRS_DECODE_LIBRARY_GEMM"); return e && atoi(e) != 0; }();
         // Rows up to which the own chain beats the library chain (in_proj / out_proj from the transposed copies, default
@@ -789,10 +795,11 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
         if (!bb->skinny) bb->wide = 0;
         bb->split_xproj = !off && !bb->skinny && (dtype == MRS_BF16 || dtype == MRS_F16) && batch <= 128 && di % 256 == 0 && xd % 8 == 0 &&
                           !narrow_model(di, xd);
-        // f32 storage: the same chain on the row-wise route of the GEMM (one to four rows, rows of the operand in LDS)
+        // f32 storage: the same chain, on the row-wise route of the GEMM (one to four rows, rows of the operand in LDS) and on the matrix cores (own_f32_chain_rows)
         if (!off && dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 &&
             getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
             bb->skinny = 1;
+        if (!off && dtype == MRS_F32 && batch <= std::min(skinny_max_rows(), own_f32_chain_rows(dm, di, false)) && dm % 32 == 0 && di % 32 == 0 && !tiny) bb->skinny = 1;
     }
     choose_resident(bb);
     int *flag = nullptr;
@@ -859,9 +866,7 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
     }
     MRS_CREATE_TRY(upload_f32(bb, &bb->norm_f, w->norm_f_weight, dm));
     {
-        // small f32 models: a step is one launch (MRS_DECODE_NO_TINY=1 keeps the kernel chains)
-        const char *e = getenv("MRS_DECODE_NO_TINY");
-        if (!(e && atoi(e) != 0) && tiny_step_ok(dtype, input_dim, dm, di, ds, dc, dr, xd) && (!identity || input_dim == dm)) {
+        if (tiny) {
             std::vector<TinyStepLayer> tl((size_t)L);
             for (int l = 0; l < L; l++) {
                 const LayerDev &d = bb->layers[l];

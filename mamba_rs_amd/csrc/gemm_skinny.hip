@@ -281,6 +281,37 @@ __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu
                 if (ll == 0) gv[m][2 * w + (LPR == 64 ? t : half)] = v;
             }
         lds_barrier();
+    } else if constexpr (sizeof(T) == 4) {
+    // f32 rows: a lane brings the same eight k of a step, and each of eight matrix instructions takes one of them from every lane (any order of k will do that both operands share).
+    uint4 bf[2][2], af[2][2];
+    auto request = [&](int h, int ks) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            bf[h][q] = ks < nk ? *reinterpret_cast<const uint4 *>(wrow + wks * ks + 4 * q) : make_uint4(0, 0, 0, 0);
+            af[h][q] = ks < nk ? *reinterpret_cast<const uint4 *>(arow + aks * ks + 4 * q) : make_uint4(0, 0, 0, 0);
+        }
+    };
+    auto multiply = [&](int h) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[h][q].x), __uint_as_float(bf[h][q].x), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[h][q].y), __uint_as_float(bf[h][q].y), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[h][q].z), __uint_as_float(bf[h][q].z), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[h][q].w), __uint_as_float(bf[h][q].w), acc, 0, 0, 0);
+        }
+    };
+    request(0, w);
+    request(1, w + kGemmWaves);
+    early_requests();
+    for (int ks = w; ks < nk; ks += 2 * kGemmWaves) {
+        multiply(0);
+        request(0, ks + 2 * kGemmWaves);
+        multiply(1);   // (past K: zeros)
+        request(1, ks + 3 * kGemmWaves);
+    }
+    row_scale();
+    red[w][l] = acc;
+    lds_barrier();
     } else if constexpr (sizeof(T) == 2) {
     // Two half-batches of fragments: the next one is requested as soon as the current one has been multiplied, so a
     // long K (wide models: 20 k-steps per wave at K = 5120) streams instead of draining after every round of loads.
@@ -573,7 +604,7 @@ static int launch_skinny_t(hipStream_t st, TO *C, int64_t ldc, const T *A, int64
     const int ksplit = (ep.mode == 0 && ep.ksplit > 1) ? ep.ksplit : 1;
     if (ksplit > 1) lpr = 0;   // a split K runs on the matrix-core route at any row count
     if (ep.w_tiled || ep.a_tiled) lpr = 0;   // tiled operands are matrix-core operands
-    if (sizeof(T) == 4 && lpr == 0) return fail(MRS_E_SHAPE, "skinny gemm: f32 storage runs on the row-wise route only (M <= 4, K %% 128 == 0, no K split)");
+    if (sizeof(T) == 4 && lpr == 0 && (!ep.f32_rows || ksplit > 1 || ep.w_tiled || ep.a_tiled)) return fail(MRS_E_SHAPE, "skinny gemm: f32 storage runs on the row-wise route only (M <= 4, K %% 128 == 0, no K split)");
     if (ksplit > 1 && (ep.row_scale || !ep.xpart || ksplit > (K >> 5)))
         return fail(MRS_E_SHAPE, "skinny gemm: K split needs the matrix-core route, a plain product, a share buffer and ksplit <= K / 32 (ksplit=%d)", ksplit);
     ep.kslice = ((K >> 5) + ksplit - 1) / ksplit;
@@ -623,7 +654,8 @@ bool skinny_gemm_ok(int dtype, int M, int N, int K, int64_t lda, const void *A, 
 int launch_skinny_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t ldc, const void *A, int64_t lda, const void *Wt,
                        int M, int N, int K, const SkinnyEpi &ep) {
     const int row_check = ep.any_rows && ep.mode == 0 && dtype != MRS_F32 ? std::min(M, 1) : M;
-    if (!skinny_gemm_ok(dtype, row_check, N, K, lda, A, Wt))
+    const bool f32_rows = dtype == MRS_F32 && ep.f32_rows && M >= 1 && M <= skinny_max_rows() && N >= 1 && K >= 32 && K % 32 == 0 && lda % 4 == 0 && aligned(A, 16) && aligned(Wt, 16);
+    if (!f32_rows && !skinny_gemm_ok(dtype, row_check, N, K, lda, A, Wt))
         return fail(MRS_E_SHAPE, "skinny gemm: needs 16-bit storage with 1 <= M <= 128, K %% 32 == 0, lda %% 8 == 0, or f32 storage with M <= 4, "
                                  "K %% 128 == 0, lda %% 4 == 0; 16-byte aligned A and Wt (got dtype=%d M=%d N=%d K=%d lda=%lld)", dtype, M, N, K,
                     (long long)lda);

@@ -817,6 +817,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenR
                                             lw.norm_w, B, dm, a_mt, taken ? rows : TokenRows()));
             SkinnyEpi inp = {};
             inp.w_stream = streams_in_proj(L * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb), B);
+            inp.f32_rows = 1;
             inp.row_scale = 1; inp.partials = bb->partials; inp.n_partials = P; inp.eps = c.rms_norm_eps;
             inp.a_tiled = inp.w_tiled = a_mt ? 1 : 0;
             MRS_TRY(launch_skinny_gemm(bb->stream, dt, bb->proj, 1, ip, bb->normed, dm, a_mt ? lw.in_proj_p : lw.in_proj_t, B, ip, dm, inp));
@@ -828,6 +829,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenR
         MRS_DISPATCH_DTYPE(dt, T_, MRS_TRY(launch_layer_step_t<T_>(bb, l)));
         if (bb->skinny) {
             SkinnyEpi outp = {};
+            outp.f32_rows = 1;
             outp.mode = 2; outp.residual = bb->residual; outp.partials = bb->partials; outp.n_partials = P;
             outp.next_norm_w = l + 1 < L ? bb->layers[l + 1].norm_w : nullptr; outp.prenorm = bb->normed;
             outp.a_tiled = outp.w_tiled = a_mt ? 1 : 0; outp.prenorm_mt = a_mt;
@@ -921,6 +923,12 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     // f32 storage: the row-wise route of the same GEMM, one to four rows
     if (dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 && getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
         bb->skinny = 1;
+    const bool tiny = [&] {   // small f32 models: a step is one launch (MRS_DECODE_NO_TINY=1 keeps the kernel chains)
+        const char *e = getenv("MRS_DECODE_NO_TINY");
+        return !(e && atoi(e) != 0) && tiny_m3_step_ok(dtype, input_dim, dm, di, nh, cfg->headdim, ds, cfg->ngroups, bb->nr, ip);
+    }();
+    // ... and the matrix cores past them
+    if (dtype == MRS_F32 && batch <= std::min(skinny_max_rows(), own_f32_chain_rows(dm, di, true)) && dm % 32 == 0 && di % 32 == 0 && !tiny) bb->skinny = 1;
     choose_resident3(bb);
     float *stage = nullptr;
     {
@@ -970,9 +978,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     }
     MRS_CREATE_TRY(upload_f32_3(bb, &bb->norm_f, w->norm_f_weight, dm));
     {
-        // small f32 models: a step is one launch (MRS_DECODE_NO_TINY=1 keeps the kernel chains)
-        const char *e = getenv("MRS_DECODE_NO_TINY");
-        if (!(e && atoi(e) != 0) && tiny_m3_step_ok(dtype, input_dim, dm, di, nh, cfg->headdim, ds, cfg->ngroups, bb->nr, ip)) {
+        if (tiny) {
             std::vector<TinyM3StepLayer> tl((size_t)L);
             for (int l = 0; l < L; l++) {
                 const Layer3 &d = bb->layers[l];

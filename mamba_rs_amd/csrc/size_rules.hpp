@@ -49,6 +49,18 @@ inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31)
 //   Mamba-3, eight of 512       65 rows 288 / 212, 128 463 / 316    768   65 388 / 293, 128 496 / 420    1024   65 467 / 370, 128 623 / 540    1536   65 589 / 530, 128 841 / 811
 inline bool own_chain_to_the_last_row(int64_t d_model, int64_t d_inner) { return d_model * 2 * d_inner <= 10 * 1000 * 1000; }
 
+// The same for f32 models (16 x 16 tiles on the matrix cores' f32 instructions; one to four rows row by row where the width allows).  Wide rows of many are the library's again, those of
+// Mamba-3 sooner: its launches per layer are fewer.  Us a step of four layers, library / own:
+//   Mamba-1 d_model 192   1 row 101 / 65, 8 rows 106 / 81, 128 rows 112 / 101    256   8 rows 107 / 74, 128 rows 125 / 109    768   5 rows 202 / 97, 64 rows 211 / 175, 128 rows 260 / 250
+//           1024   8 rows 247 / 144, 64 rows 269 / 229, 96 rows 285 / 309        1536  8 rows 361 / 200, 48 rows 425 / 373     2560  8 rows 1600 / 383, 48 rows 1639 / 835
+//   Mamba-3 192   1 row 75 / 59, 128 rows 91 / 94    256   8 rows 87 / 72, 128 rows 103 / 103    512   8 rows 106 / 88, 48 rows 134 / 126, 64 rows 139 / 142
+//           768   8 rows 164 / 102, 48 rows 196 / 168, 96 rows 245 / 249    1024   48 rows 242 / 219, 64 rows 248 / 252    2560   8 rows 1457 / 312, 48 rows 1572 / 757
+inline int own_f32_chain_rows(int64_t d_model, int64_t d_inner, bool mamba3) {
+    const int64_t n = d_model * 2 * d_inner;
+    if (mamba3) return n <= 300 * 1000 ? 96 : 48;
+    return n <= 2400 * 1000 ? 128 : n <= 4200 * 1000 ? 64 : 48;
+}
+
 // Whether what a decode step touches (`bytes`: weights, states, the head's table) is more than the chip's last cache holds, 256 MB.  What is read once a step and not kept from one
 // step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
 // The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)

@@ -562,6 +562,33 @@ def test_rows_a_step_hands_to_the_host_are_the_rows_it_leaves_on_the_device(dm, 
     eng.close()
 
 
+@pytest.mark.parametrize("dm,L,B", [(96, 2, 1), (160, 2, 17), (192, 2, 4), (192, 1, 128), (256, 2, 5), (256, 2, 16), (768, 1, 33), (1088, 1, 7), (800, 1, 64), (192, 1, 129)])
+def test_f32_rows_on_the_own_chain_follow_the_cpu_route(dm, L, B):
+    """f32 models past the single-launch step: the own chain with its products on the matrix cores' f32 instructions (k-steps fewer than the waves, row tiles partly filled, more rows
+    than x_proj rides in in_proj for), and the library's past 128 rows.  f32 sums of at most 2176 terms in another order, 1e-4 of the scale as for the other f32 steps."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
+    w = MambaWeights.init(cfg, 40, 5)
+    P = oracle_params(w, cfg, 40)
+    rng = np.random.default_rng(dm + B)
+    print(f"case f32 rows {dm} {L} {B}", flush=True)
+    eng = GpuMambaBackbone.new(0, w, cfg, 40, B)
+    assert eng.decode_route() == (1 if B <= 128 else 0)
+    rows = sorted({0, B // 2, B - 1})
+    st = {b: orc.m1_zero_state(P) for b in rows}
+    for t in range(4):
+        x = rng.standard_normal((B, 40)).astype(np.float32)
+        if t == 2:
+            eng.capture_graph()
+        got = eng.step(x)
+        for b in rows:
+            assert scaled_err(got[b], orc.m1_backbone_step(P, x[b], *st[b])) < 1e-4, (t, b)
+    for l in range(L):
+        conv, ssm = eng.download_state(l)
+        for b in rows:
+            assert scaled_err(conv[b][:, 1:], st[b][0][l].reshape(2 * dm, 3)) < 1e-4 and scaled_err(ssm[b], st[b][1][l].reshape(2 * dm, 16)) < 1e-4, (l, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,idim,B", [(192, 1, 1), (192, 9, 3), (160, 513, 2), (320, 88, 128), (320, 88, 129), (36, 4096, 2), (36, 4097, 2)])
 def test_input_rows_through_the_projection_kernel(dm, idim, B):
     """One row's product per workgroup, from host memory (step) and from the device (step_gpu_only), eager and in front of a recorded step; past 128 rows or 4096 inputs the library's.

@@ -119,6 +119,29 @@ def test_batch_rows_are_independent_and_graph_equals_eager():
         eng.close()
 
 
+@pytest.mark.parametrize("dm,B", [(160, 3), (192, 17), (256, 5), (768, 33)])
+def test_f32_rows_on_the_own_chain_match_cpu_reference_path(dm, B):
+    """f32 past the single-launch step and the row-wise route: both products on the matrix cores' f32 instructions.  Bound of the f32 steps above."""
+    cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+    w = perturbed(cfg, 24, 5)
+    P = oracle_params(w, cfg, 24)
+    print(f"case m3 f32 rows {dm} {B}", flush=True)
+    eng = GpuMamba3Backbone.new(0, w, cfg, 24, B)
+    assert eng.decode_route() == 1
+    rows = sorted({0, B // 2, B - 1})
+    st = {b: P.zero_state() for b in rows}
+    rng = np.random.default_rng(B)
+    for t in range(6):
+        x = rng.standard_normal((B, 24)).astype(np.float32)
+        if t == 3:
+            eng.capture_graph()
+        got = eng.step(x)
+        for b in rows:
+            want = orc.m3_backbone_step(P, x[b], st[b])
+            assert np.max(np.abs(got[b] - want)) < 1e-4 * max(1.0, np.max(np.abs(want))), (t, b)
+    eng.close()
+
+
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
 @pytest.mark.parametrize("ci,B", [(0, 2), (1, 2), (0, 7), (1, 21), (2, 16),
                                   (0, 65), (2, 113), (1, 128), (0, 129)])   # the last row tiles of the own chain, and past it

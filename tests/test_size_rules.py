@@ -74,3 +74,9 @@ def test_layers_whose_weights_come_through_the_last_cache(rules):
 
 def test_the_own_chain_takes_every_row_count_up_to_d_model_1536(rules):
     assert rules("own_chain_to_the_last_row(a, b)", [(dm, 2 * dm, 0, 0) for dm in (64, 768, 1024, 1536, 1792, 2560)] + [(2048, 2048, 0, 0)]) == [1, 1, 1, 1, 0, 0, 1]
+
+
+def test_rows_of_the_f32_chain(rules):
+    dims = (192, 256, 768, 1024, 1536, 2560)
+    assert rules("own_f32_chain_rows(a, b, false)", [(dm, 2 * dm, 0, 0) for dm in dims]) == [128, 128, 128, 64, 48, 48]
+    assert rules("own_f32_chain_rows(a, b, true)", [(dm, 2 * dm, 0, 0) for dm in dims]) == [96, 96, 48, 48, 48, 48]
