@@ -1231,7 +1231,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     lm->stream_table = step_outgrows_cache((int64_t)(ne * es + eng.weight_bytes + eng.state_bytes(eng.self)));
     if (lm_head_ok(lm->dtype, lm->batch, lm->vocab_padded, lm->dm)) {
         MRS_LM_HIP(hipMalloc((void **)&lm->arg_keys, lm_head_keys(lm->batch, lm->vocab_padded, lm->dm) * 8)); lm->allocs.push_back(lm->arg_keys);
-        MRS_LM_HIP(hipMalloc(&lm->table_p, ne * es)); lm->allocs.push_back(lm->table_p);
+        lm->table_p = lm->embed;   // (a place of its own below)
     }
     MRS_LM_HIP(hipMalloc((void **)&stage, ne * 4));
     MRS_LM_HIP(hipMemsetAsync(stage, 0, ne * 4, eng.stream));  // padded rows are zero
@@ -1240,10 +1240,14 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     if (lm->dtype == MRS_F32) MRS_LM_HIP(hipMemcpyAsync(lm->embed, stage, ne * 4, hipMemcpyDeviceToDevice, eng.stream));
     else if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, eng.stream, (bf16_t *)lm->embed, stage, (int64_t)ne);
     else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, eng.stream, (f16_t *)lm->embed, stage, (int64_t)ne);
-    if (lm->table_p) { const int rc = launch_tile_weight(eng.stream, lm->dtype, lm->table_p, lm->embed, lm->vocab_padded, lm->dm); if (rc) { cleanup(); return rc; } }
+    if (lm->table_p) {   // the head's tiles stay where the f32 rows came in: an allocation of a table's size and a free take 15 ms
+        lm->table_p = stage; lm->allocs.push_back(stage); stage = nullptr;
+        const int rc = launch_tile_weight(eng.stream, lm->dtype, lm->table_p, lm->embed, lm->vocab_padded, lm->dm);
+        if (rc) { cleanup(); return rc; }
+    }
     MRS_LM_HIP(hipStreamSynchronize(eng.stream));
 #undef MRS_LM_HIP
-    hipFree(stage);
+    if (stage) hipFree(stage);
     *out = lm;
     return MRS_OK;
 }
