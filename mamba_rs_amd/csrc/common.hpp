@@ -91,10 +91,22 @@ struct StepFold { const float *xpart; int n_tiles, rows, xd, b_off, c_off, y_mt;
 __host__ __device__ inline int64_t tiled_a_index(int row, int k, int mt) {
     return ((((int64_t)(k >> 5) * mt + (row >> 4)) * 64 + (row & 15) + 16 * ((k >> 3) & 3)) << 3) + (k & 7);
 }
+// Four states, past the last cache where STREAM.
+template <bool STREAM> __device__ __forceinline__ float4 state_ld(const float *p) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    if constexpr (STREAM) return __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f4 *>(p)));
+    else return *reinterpret_cast<const float4 *>(p);
+}
+template <bool STREAM> __device__ __forceinline__ void state_st(float *p, float4 v) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    if constexpr (STREAM) __builtin_nontemporal_store(__builtin_bit_cast(f4, v), reinterpret_cast<f4 *>(p));
+    else *reinterpret_cast<float4 *>(p) = v;
+}
 int launch_ssm_step_fused(hipStream_t st, int dtype, float *h, void *y, const void *delta, const float *dt_bias,
                           const void *dt_in, const void *dt_w, int dr, int dt_transposed, const void *u, const void *Bb, const void *Cb, int64_t bc_stride, const void *gate,
                           int64_t gate_stride, int gate_mode, const float *a_neg, const float *D, int batch,
-                          int di, int ds, const StepFold *fold = nullptr, int y_mt = 0);
+                          int di, int ds, const StepFold *fold = nullptr, int y_mt = 0,
+                          bool stream = false);   // stream: the states are read and written past the last cache (d_state 16)
 int launch_conv1d_step(hipStream_t st, int dtype, void *out, float *state, const void *new_x, int64_t x_stride,
                        const float *weight, const float *bias, int batch, int d_inner, int d_conv, int apply_silu);
 

@@ -422,6 +422,7 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
     // Per step at that shape, dt_proj in the step kernel / on its own: 32 rows 3.57 / 3.84 ms, 48 rows 4.32 / 4.34, 64 rows 5.04 / 4.89.
     static const int64_t wide_fuse = [] { const char *e = getenv("MRS_DECODE_FUSE_DT_LIMIT"); return e ? (int64_t)atoll(e) : (int64_t)6400; }();
     const bool stream_in = streams_in_proj(L * layer_weight_bytes(bb) + state_bytes(bb), nr);
+    const bool stream_states = step_outgrows_cache(L * layer_weight_bytes(bb) + state_bytes(bb));
     const int64_t fuse_limit = (a_mt && bb->wide) ? wide_fuse : kFuseDtProjLimit;
     for (int l = 0; l < L; l++) {
         const LayerDev &lw = bb->layers[l];
@@ -472,11 +473,11 @@ static int decode_chain(mrs_backbone *bb, Scratch *s, int r0, int nr, hipStream_
             // wide dt_rank at a large batch: dt_proj as a GEMM of its own, bias + softplus in the step kernel
             MRS_TRY(launch_skinny_gemm(st, dt, delta, 0, di, xdbl, xd, lw.dt_w_t, nr, di, dr, none));
             MRS_TRY(launch_ssm_step_fused(st, dt, ssm, y, delta, lw.dt_b, nullptr, nullptr, 0, 0, u, xdbl + es * dr, xdbl + es * (dr + ds), xd, z,
-                                          2 * di, 2, lw.a_neg, lw.D, nr, di, ds, nullptr, a_mt));
+                                          2 * di, 2, lw.a_neg, lw.D, nr, di, ds, nullptr, a_mt, stream_states));
         } else {
             MRS_TRY(launch_ssm_step_fused(st, dt, ssm, y, delta, lw.dt_b, xdbl, lw.dt_t_step ? lw.dt_w_t : lw.dt_w, dr, lw.dt_t_step, u,
                                           xdbl + es * dr, xdbl + es * (dr + ds), xd, z, 2 * di, 2, lw.a_neg, lw.D, nr, di, ds,
-                                          (fold_x || ksplit > 1) ? &fold : nullptr, a_mt));
+                                          (fold_x || ksplit > 1) ? &fold : nullptr, a_mt, stream_states));
         }
         SkinnyEpi outp = {};
         outp.f32_rows = 1;

@@ -52,7 +52,7 @@ constexpr int kStepsPerBatch = 6;  // k-steps whose loads are issued together (c
 // 16-byte pieces -- whole kilobytes of one row per load instruction instead of 64-byte pieces of 16 rows -- each wave
 // owns two of the workgroup's 16 columns, all of its loads are in flight at once (in groups of JB per column), and
 // the products are v_dot2 with f32 accumulate.  The epilogues are the same code.  MR = rows computed (1, 2 or 4; at 8 rows the route was slower than the matrix-core tiles: 642 vs 435 us per 130m-shape step).
-// STREAM: the weight is read past the last cache (row-wise route; ep.w_stream)
+// STREAM: the weight is read past the last cache (ep.w_stream; not by f32 rows on the matrix cores)
 typedef unsigned piece4 __attribute__((ext_vector_type(4)));
 template <bool STREAM, typename T> __device__ __forceinline__ uint4 weight_piece(const T *p) {
     if constexpr (STREAM) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const piece4 *>(p)));
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kGemmWaves * 64) __attribute__((amdgpu_waves_per_eu
         for (int s = 0; s < kHalf; s++) {
             const int ks = base + s * kGemmWaves;
             // steps past K multiply zeros (every fragment is defined on every path)
-            bf[h][s] = ks < nk ? *reinterpret_cast<const uint4 *>(wrow + wks * ks) : make_uint4(0, 0, 0, 0);
+            bf[h][s] = ks < nk ? weight_piece<STREAM>(wrow + wks * ks) : make_uint4(0, 0, 0, 0);
             af[h][s] = ks < nk ? *reinterpret_cast<const uint4 *>(arow + aks * ks) : make_uint4(0, 0, 0, 0);
         }
     };
@@ -623,7 +623,7 @@ static int launch_skinny_t(hipStream_t st, TO *C, int64_t ldc, const T *A, int64
         else if (lpr == 64) MRS_SG_ROWS(EPI_, PRO_, 64, 4);                                                                              \
         else if (lpr == 32 && M == 1) MRS_SG_ROWS(EPI_, PRO_, 32, 1);                                                                    \
         else if (lpr == 32) MRS_SG_ROWS(EPI_, PRO_, 32, 4);                                                                              \
-        else hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_>), grid, block, 0, st, C, ldc, A, lda, Wt, M, N, K, ep);           \
+        else MRS_SG_ROWS(EPI_, PRO_, 0, 1);                                                                                              \
     } while (0)
     const bool pro = ep.row_scale != 0;
     if (ep.mode != 0 && sizeof(TO) != sizeof(T)) return fail(MRS_E_DTYPE, "skinny gemm: fused epilogues store the activation type");

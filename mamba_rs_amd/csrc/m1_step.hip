@@ -44,7 +44,8 @@ constexpr int kFoldMaxXd = 256;
 // shares in fold.xpart [tile][row][xd] -- so each workgroup first sums the shares of its batch row, in tile order,
 // rounds them to the storage type as the stored projection would be, and keeps the row in LDS.  A workgroup's 256 / LG
 // channels lie in one batch row (d_inner is a multiple of that).
-template <typename T, int LG, int DT, bool VECBC, bool FOLD = false, int PRE = 4>
+// STREAM: the states are read and written past the last cache.
+template <typename T, int LG, int DT, bool VECBC, bool FOLD = false, int PRE = 4, bool STREAM = false>
 __global__ __launch_bounds__(256) void ssm_step_kernel(
     float *__restrict__ h, T *__restrict__ y, const T *__restrict__ delta, const T *__restrict__ u,
     const T *__restrict__ Bbase, const T *__restrict__ Cbase, int64_t bc_stride,
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(
             share[i] = (fold_tg < fold_G && t < fold.n_tiles) ? *reinterpret_cast<const float4 *>(src + t * tstride) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
-    float4 hv = *reinterpret_cast<const float4 *>(h + r * ds + 4 * g);
+    float4 hv = state_ld<STREAM>(h + r * ds + 4 * g);
     const float4 av = *reinterpret_cast<const float4 *>(a_neg + (int64_t)d * ds + 4 * g);
     const float uu = Store<T>::ld(u + r);
     const float Dd = Dp[d];
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(
 #pragma unroll
     for (int m = 1; m < LG; m <<= 1) acc += __shfl_xor(acc, m, kWave);
     if (live) {
-        *reinterpret_cast<float4 *>(h + r * ds + 4 * g) = hv;
+        state_st<STREAM>(h + r * ds + 4 * g, hv);
         if (g == 0) {
             acc = fmaf(Dd, uu, acc);
             if (gate_mode == 1) acc *= gz;
@@ -290,7 +291,7 @@ static int launch_step(hipStream_t st, float *h, void *y, const void *delta, con
                        const void *Bb, const void *Cb, int64_t bc_stride, const void *gate,
                        int64_t gate_stride, int gate_mode, const float *dt_bias, const void *dt_in,
                        const void *dt_w, int dr, int dt_transposed, const float *a_neg, const float *D, int batch, int di, int ds,
-                       const StepFold *fold = nullptr, int y_mt = 0) {
+                       const StepFold *fold = nullptr, int y_mt = 0, bool stream = false) {
     const int64_t total = (int64_t)batch * di;
     if (!gate) gate_mode = 0;
 #define MRS_ARGS h, (T *)y, (const T *)delta, (const T *)u, (const T *)Bb, (const T *)Cb, bc_stride, \
@@ -323,9 +324,14 @@ static int launch_step(hipStream_t st, float *h, void *y, const void *delta, con
 #define MRS_LGF(L) case L: hipLaunchKernelGGL((ssm_step_kernel<T, L, 2, true, true>), grid, block, 0, st, MRS_ARGS, folded); break
             if constexpr (sizeof(T) == 2) {
                 if (lg == 4 && dr / lg > 16) {   // a wide dt_rank: the whole weight share requested up front
-                    hipLaunchKernelGGL((ssm_step_kernel<T, 4, 2, true, true, 12>), grid, block, 0, st, MRS_ARGS, folded);
+                    if (stream) hipLaunchKernelGGL((ssm_step_kernel<T, 4, 2, true, true, 12, true>), grid, block, 0, st, MRS_ARGS, folded);
+                    else hipLaunchKernelGGL((ssm_step_kernel<T, 4, 2, true, true, 12>), grid, block, 0, st, MRS_ARGS, folded);
                     return check_launch("ssm_step_kernel");
                 }
+            }
+            if (stream && lg == 4) {
+                hipLaunchKernelGGL((ssm_step_kernel<T, 4, 2, true, true, 4, true>), grid, block, 0, st, MRS_ARGS, folded);
+                return check_launch("ssm_step_kernel");
             }
             switch (lg) { MRS_LGF(1); MRS_LGF(2); MRS_LGF(4); MRS_LGF(8); MRS_LGF(16); MRS_LGF(32); MRS_LGF(64); }
 #undef MRS_LGF
@@ -335,6 +341,11 @@ static int launch_step(hipStream_t st, float *h, void *y, const void *delta, con
         nofold.y_mt = y_mt;
         // (delta source, vector B/C): the transposed dt_w route implies vector rows (checked above)
         const int variant = dt_mode == 2 ? 4 : dt_mode * 2 + (vec_bc ? 1 : 0);
+        if (stream && lg == 4 && (variant == 4 || variant == 1)) {
+            if (variant == 4) hipLaunchKernelGGL((ssm_step_kernel<T, 4, 2, true, false, 4, true>), grid, block, 0, st, MRS_ARGS, nofold);
+            else hipLaunchKernelGGL((ssm_step_kernel<T, 4, 0, true, false, 4, true>), grid, block, 0, st, MRS_ARGS, nofold);
+            return check_launch("ssm_step_kernel");
+        }
 #define MRS_LGV(L, DT_, V_) hipLaunchKernelGGL((ssm_step_kernel<T, L, DT_, V_>), grid, block, 0, st, MRS_ARGS, nofold)
 #define MRS_LG(L)                                   \
     case L:                                         \
@@ -363,9 +374,9 @@ int launch_ssm_step_fused(hipStream_t st, int dtype, float *h, void *y, const vo
                           const void *dt_in, const void *dt_w, int dr, int dt_transposed,
                           const void *u, const void *Bb, const void *Cb, int64_t bc_stride, const void *gate,
                           int64_t gate_stride, int gate_mode, const float *a_neg, const float *D, int batch,
-                          int di, int ds, const StepFold *fold, int y_mt) {
+                          int di, int ds, const StepFold *fold, int y_mt, bool stream) {
     MRS_DISPATCH_DTYPE(dtype, T_, return launch_step<T_>(st, h, y, delta, u, Bb, Cb, bc_stride, gate, gate_stride, gate_mode,
-                                                         dt_bias, dt_in, dt_w, dr, dt_transposed, a_neg, D, batch, di, ds, fold, y_mt));
+                                                         dt_bias, dt_in, dt_w, dr, dt_transposed, a_neg, D, batch, di, ds, fold, y_mt, stream));
     return MRS_OK;
 }
 

@@ -22,16 +22,20 @@
 #include "glue.hpp"
 #include "m3_math.hpp"
 #include <rocblas/rocblas.h>
+#include <algorithm>
 #include <new>
 #include <vector>
 
 namespace mrs {
 
-// One workgroup per (batch row, head); blockDim.x = hd * LG, LG = ds / 4 lanes per state row.
+// One workgroup per (batch row, head); blockDim.x = hd * LG / RP, LG = ds / 4 lanes per state row, RP rows to a thread.
+// Bound by the states' bytes at many rows, and there a compute unit has to have many of them under way: all of a workgroup's states are asked for at its beginning, behind which it
+// goes through a chain of short phases, so four rows to a thread, which let eight workgroups of a 64 x 64 head share a unit instead of two, are what fills the time
+// of the others' chains (a step of 24 layers of d_model 768, one row / four: 24 rows 500 / 468 us, 64 737 / 706, 128 1147 / 1026; up to four rows one is as good).  STREAM: the states are read and written past the last cache (step_outgrows_cache), which then keeps the weights.
 // proj: [batch, ip] f32 = [z:di | x:di | B:ng*ds | C:ng*ds | dd_dt:nh | dd_A:nh | trap:nh | angles:nr]
 // gated: [batch, di] activation type (out_proj's operand).
-template <typename T, int LG>
-__global__ __launch_bounds__(1024) void m3_layer_step_kernel(
+template <typename T, int LG, int RP = 1, bool STREAM = false>
+__global__ __launch_bounds__(1024 / RP) void m3_layer_step_kernel(
     float *__restrict__ ssm, float *__restrict__ kst, float *__restrict__ vst, float *__restrict__ angle,
     T *__restrict__ gated, const float *__restrict__ proj, int64_t ip, const float *__restrict__ dt_bias,
     const float *__restrict__ bnw, const float *__restrict__ cnw, const float *__restrict__ b_bias,
@@ -41,7 +45,7 @@ __global__ __launch_bounds__(1024) void m3_layer_step_kernel(
     __shared__ float kl[ds], ql[ds], red[16];
     const int b = blockIdx.x / nh, h = blockIdx.x - b * nh;
     const int tid = threadIdx.x, nthr = blockDim.x;
-    const int p = tid / LG, g = tid % LG;
+    const int p = tid / LG, g = tid % LG, rows = nthr / LG;   // this thread's rows of the head: p, p + rows, ...
     const int di = nh * hd;
     const int grp = h / (nh / ng);
     const int64_t bh = (int64_t)b * nh + h;
@@ -51,12 +55,19 @@ __global__ __launch_bounds__(1024) void m3_layer_step_kernel(
     // Every global load of the kernel up front -- none depends on another -- so that the body below costs one memory
     // round trip, not one per phase; the barriers between the phases publish LDS only (lds_barrier) and leave loads in flight.
     float *Hrow = ssm + (bh * hd + p) * ds + 4 * g;
-    float4 H = *reinterpret_cast<const float4 *>(Hrow);
+    float4 H[RP];
+    float vp[RP], xv[RP], zi[RP], ngv[RP];
+#pragma unroll
+    for (int k = 0; k < RP; k++) H[k] = state_ld<STREAM>(Hrow + (int64_t)k * rows * ds);
     const float4 kp = *reinterpret_cast<const float4 *>(kst + bh * ds + 4 * g);
-    const float vp = vst[bh * hd + p];
-    const float xv = xr[h * hd + p];
-    const float zi = zr[h * hd + p];
-    const float ngv = outproj_norm ? ngw[h * hd + p] : 1.0f;
+#pragma unroll
+    for (int k = 0; k < RP; k++) {
+        const int c = p + k * rows;
+        vp[k] = vst[bh * hd + c];
+        xv[k] = xr[h * hd + c];
+        zi[k] = zr[h * hd + c];
+        ngv[k] = outproj_norm ? ngw[h * hd + c] : 1.0f;
+    }
     const float Dh = Dp[h];
     const float s_dt = sc[h], s_dtb = dt_bias[h], s_A = sc[nh + h], s_tr = sc[2 * nh + h];
     const bool own_n = tid < ds, own_a = tid < nr;   // blockDim.x >= d_state (headdim >= 4)
@@ -106,23 +117,29 @@ __global__ __launch_bounds__(1024) void m3_layer_step_kernel(
     // ---- trapezoidal update of this lane's four states, y = H q + D x ----
     const float4 kc = *reinterpret_cast<const float4 *>(&kl[4 * g]);
     const float4 qc = *reinterpret_cast<const float4 *>(&ql[4 * g]);
-    const float bv = be * vp, gx = ga * xv;
-    H.x = fmaf(al, H.x, fmaf(bv, kp.x, gx * kc.x));
-    H.y = fmaf(al, H.y, fmaf(bv, kp.y, gx * kc.y));
-    H.z = fmaf(al, H.z, fmaf(bv, kp.z, gx * kc.z));
-    H.w = fmaf(al, H.w, fmaf(bv, kp.w, gx * kc.w));
-    float acc = H.x * qc.x;
-    acc = fmaf(H.y, qc.y, acc);
-    acc = fmaf(H.z, qc.z, acc);
-    acc = fmaf(H.w, qc.w, acc);
+    float yv[RP];
 #pragma unroll
-    for (int m = 1; m < LG; m <<= 1) acc += __shfl_xor(acc, m, kWave);
-    const float yv = fmaf(Dh, xv, acc);
-    *reinterpret_cast<float4 *>(Hrow) = H;
+    for (int k = 0; k < RP; k++) {
+        const float bv = be * vp[k], gx = ga * xv[k];
+        H[k].x = fmaf(al, H[k].x, fmaf(bv, kp.x, gx * kc.x));
+        H[k].y = fmaf(al, H[k].y, fmaf(bv, kp.y, gx * kc.y));
+        H[k].z = fmaf(al, H[k].z, fmaf(bv, kp.z, gx * kc.z));
+        H[k].w = fmaf(al, H[k].w, fmaf(bv, kp.w, gx * kc.w));
+        float acc = H[k].x * qc.x;
+        acc = fmaf(H[k].y, qc.y, acc);
+        acc = fmaf(H[k].z, qc.z, acc);
+        acc = fmaf(H[k].w, qc.w, acc);
+#pragma unroll
+        for (int m = 1; m < LG; m <<= 1) acc += __shfl_xor(acc, m, kWave);
+        yv[k] = fmaf(Dh, xv[k], acc);
+        state_st<STREAM>(Hrow + (int64_t)k * rows * ds, H[k]);
+    }
     // ---- gate: y * silu(z), or RMSNormGated over the head first (rmsnorm_gated_forward, ops/norms.rs:84-114) ----
     float inv_y = 1.0f;
     if (outproj_norm) {
-        float sq = (g == 0) ? yv * yv : 0.0f;
+        float sq = 0.0f;
+#pragma unroll
+        for (int k = 0; k < RP; k++) sq += (g == 0) ? yv[k] * yv[k] : 0.0f;
 #pragma unroll
         for (int m = 32; m >= 1; m >>= 1) sq += __shfl_xor(sq, m, kWave);
         if ((tid & 63) == 0) red[wv & 15] = sq;   // (every lane read red before the full barrier above)
@@ -132,10 +149,14 @@ __global__ __launch_bounds__(1024) void m3_layer_step_kernel(
         inv_y = 1.0f / sqrtf(tot / (float)hd + eps);
     }
     if (g == 0) {
-        const float o = outproj_norm ? yv * inv_y * ngv * silu(zi) : yv * silu(zi);
-        // gated_mt != 0: out_proj reads its operand in tile order (tiled_a_index, gated_mt row tiles)
-        Store<T>::st(gated + (gated_mt ? tiled_a_index(b, h * hd + p, gated_mt) : (int64_t)b * di + h * hd + p), o);
-        vst[bh * hd + p] = xv;
+#pragma unroll
+        for (int k = 0; k < RP; k++) {
+            const int c = p + k * rows;
+            const float o = outproj_norm ? yv[k] * inv_y * ngv[k] * silu(zi[k]) : yv[k] * silu(zi[k]);
+            // gated_mt != 0: out_proj reads its operand in tile order (tiled_a_index, gated_mt row tiles)
+            Store<T>::st(gated + (gated_mt ? tiled_a_index(b, h * hd + c, gated_mt) : (int64_t)b * di + h * hd + c), o);
+            vst[bh * hd + c] = xv[k];
+        }
     }
     // every lane has read the previous k_state (kp) at the top; the full barrier after the rotation orders those reads before this write
     if (p == 0) *reinterpret_cast<float4 *>(kst + bh * ds + 4 * g) = kc;
@@ -623,6 +644,9 @@ int gemm3(mrs_m3_backbone *bb, void *C, bool c_f32, const void *A, const void *W
     return gemm_ex_tuned(bb->tuner, bb->blas, bb->stream, 0, N, M, K, W, t, N, A, t, K, C, ct, N);
 }
 
+int64_t layer_weight_bytes3(const mrs_m3_backbone *bb) { return (int64_t)bb->cfg.d_model * (bb->ip + bb->di) * (int64_t)esize3(bb->dtype); }
+size_t m3_hook_state_bytes(void *self);
+
 template <typename T>
 int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
     const mrs_m3_config &c = bb->cfg;
@@ -630,7 +654,19 @@ int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
     const int B = bb->batch, nh = bb->nh, hd = c.headdim, ds = c.d_state, lg = ds / 4;
     float *ssm = bb->ssm + (size_t)l * B * nh * hd * ds, *kst = bb->kst + (size_t)l * B * nh * ds;
     float *vst = bb->vst + (size_t)l * B * nh * hd, *ang = bb->angle + (size_t)l * B * nh * (bb->nr > 0 ? bb->nr : 1);
-    const dim3 grid((unsigned)(B * nh)), block((unsigned)(hd * lg));
+    const dim3 grid((unsigned)(B * nh));
+    // four rows to a thread where that leaves a thread for every state and every pair to rotate
+    const int per = B * nh >= 192 && lg == 16 && hd % 4 == 0 && hd * lg / 4 >= std::max(ds, bb->nr) ? 4 : 1;
+    const bool stream = per == 4 && step_outgrows_cache(c.n_layers * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb));
+    const dim3 block((unsigned)(hd * lg / per));
+    if (per == 4) {
+#define MRS_L4(S) hipLaunchKernelGGL((m3_layer_step_kernel<T, 16, 4, S>), grid, block, 0, bb->stream, ssm, kst, vst, ang, (T *)bb->gated, bb->proj, (int64_t)bb->ip, lw.dt_bias, lw.bnw, lw.cnw, \
+                                       lw.b_bias, lw.c_bias, lw.D, lw.ngw, nh, hd, c.ngroups, bb->nr, c.a_floor, c.rms_norm_eps, c.is_outproj_norm, bb->tiled ? (B + 15) / 16 : 0)
+        if (stream) MRS_L4(true);
+        else MRS_L4(false);
+#undef MRS_L4
+        return check_launch("m3_layer_step_kernel");
+    }
 #define MRS_LG(L)                                                                                                                 \
     case L:                                                                                                                       \
         hipLaunchKernelGGL((m3_layer_step_kernel<T, L>), grid, block, 0, bb->stream, ssm, kst, vst, ang, (T *)bb->gated, bb->proj,  \
@@ -668,9 +704,6 @@ int project_input3(mrs_m3_backbone *bb) {
 // models keep the chain's tokens: at one row through the step that has the chain's bits (resident_m3_row.hip), else on the chain
 // (24 layers of d_model 768 at two rows: 230 against 317 us a step).
 constexpr int kResidentM3Layers = 4;
-
-int64_t layer_weight_bytes3(const mrs_m3_backbone *bb) { return (int64_t)bb->cfg.d_model * (bb->ip + bb->di) * (int64_t)esize3(bb->dtype); }
-size_t m3_hook_state_bytes(void *self);
 
 // Resident step for the rows whose workgroups fit on the chip together.  One row takes the chain's own order (resident_m3_row.hip) wherever
 // the chain is on its row-wise route, at any depth: the same bits, and the faster of the two (its comment has both).  The kernel chain
@@ -816,7 +849,7 @@ int step_body3(mrs_m3_backbone *bb, const HostRows *host = nullptr, const TokenR
                 MRS_TRY(launch_prenorm_rows(bb->stream, dt, bb->partials, P, bb->normed, src ? src : bb->residual, src ? bb->residual : nullptr,
                                             lw.norm_w, B, dm, a_mt, taken ? rows : TokenRows()));
             SkinnyEpi inp = {};
-            inp.w_stream = streams_in_proj(L * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb), B);
+            inp.w_stream = !a_mt && streams_in_proj(L * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb), B);   // (row by row)
             inp.f32_rows = 1;
             inp.row_scale = 1; inp.partials = bb->partials; inp.n_partials = P; inp.eps = c.rms_norm_eps;
             inp.a_tiled = inp.w_tiled = a_mt ? 1 : 0;

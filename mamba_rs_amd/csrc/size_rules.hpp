@@ -65,6 +65,9 @@ inline int own_f32_chain_rows(int64_t d_model, int64_t d_inner, bool mamba3) {
 // step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
 // The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)
 // 168.7 / 174.2, 16 rows (266 MB) 241.7 / 235.2; 16 of them 16 rows (228 MB) 189.2 / 194.5, 64 rows (323 MB) 243.1 / 234.8; 12 of them 64 rows (262 MB) 184.4 / 182.9.
+// The states, which are read and written once a step, cached / past (a launch per product; the weights then stay where they fit): 130m shape 72 rows 609 / 565, 128 rows 788 / 758; 24 layers
+// of 1024 48 rows 591 / 568, 64 rows 659 / 623; 2.8b shape, 8 layers, 16 rows 323 / 316, 64 rows 578 / 565; Mamba-3, 24 layers of 768, 12 rows 390 / 361, 32 rows 494 / 427, 128 rows 1019
+// / 930.  (In the resident step of several rows, which asks for them a phase ahead: 64 rows 344 / 357.)
 inline bool step_outgrows_cache(int64_t bytes) { return bytes > (int64_t)240 << 20; }
 
 // Layers whose weights (`layer_bytes` each) come through that cache in a decode step: all of them where the states and they fit, else as many as leave room for the states, and the
@@ -78,10 +81,10 @@ inline int layers_in_cache(int layers, int64_t layer_bytes, int64_t state_bytes)
 
 // Decode of a launch per product (wide models, and one to four rows of f32 ones): in_proj's weights, two thirds of a layer's, are read past that cache where a step (`bytes` of weights and states) outgrows it, so that
 // out_proj's and the states may stay and nothing has to be written back for what is read once.  Us a step, bf16, cached / past: d_model 2560, 8 layers 4 rows 322 / 294, 16 358 / 322,
-// 32 438 / 426, 64 577 / 573; 24 layers 4 rows 833 / 808, 16 938 / 877; 2048, 12 layers 4 rows 354 / 331, 16 392 / 370, 48 557 / 563 (there states are most of it).  Some of the
+// 32 438 / 426, 64 577 / 573; 24 layers 4 rows 833 / 808, 16 938 / 877; 2048, 12 layers 4 rows 354 / 331, 16 392 / 370, 48 557 / 563 (there states are most of it); 24 of 1024, the states past it, 48 rows 568 / 543, 64 rows 623 / 634.  Some of the
 // layers' through the cache, as layers_in_cache: behind it everywhere (2560, 16 rows, two of eight 341).  out_proj's past it as well: no difference, and where the step kernel asks for
 // its lines ahead that request past it costs 40.  f32, one row, 24 layers, with the head's table past it as well: all cached 383, in_proj's past 341, all past 362 (768); 510, 458, 468 (1024).
-inline bool streams_in_proj(int64_t bytes, int rows) { return rows <= 32 && step_outgrows_cache(bytes); }
+inline bool streams_in_proj(int64_t bytes, int rows) { return rows <= 48 && step_outgrows_cache(bytes); }
 
 // Decode of wide models: whether the step kernel asks for the lines of out_proj (`bytes` of them) on the dies that will read them (m1_step.hip).  They have to stay in the dies' L2, eight
 // of 4 MB, until the launch behind: more than that is read twice, and then many rows' worth of work must cover it.  Eight layers, bf16, us a step, without / with:

@@ -12,10 +12,10 @@ pytestmark = pytest.mark.gpu
 from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
 
 
-@pytest.mark.parametrize("dm,L,B", [(1024, 20, 1), (1024, 20, 3), (2560, 4, 3)])
+@pytest.mark.parametrize("dm,L,B", [(1024, 20, 1), (1024, 20, 3), (2560, 4, 3), (1024, 20, 40), (1024, 20, 65)])
 def test_weights_past_the_last_cache(dm, L, B):
-    """Models whose weights are more than the last cache holds, so that some layers' (resident steps of a row and of several) or all layers' in_proj (wide models) are read past it:
-    outputs against the CPU route, as below."""
+    """Models whose weights are more than the last cache holds, so that some layers' (resident steps of a row and of several) or all layers' in_proj (a launch per product) are read past it,
+    and there the states as well (three forms of the step kernel): outputs against the CPU route, as below."""
     cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
     w = MambaWeights.init(cfg, dm, 11)
     w.input_proj_w = np.zeros((0, dm), np.float32)

@@ -69,7 +69,7 @@ def test_layers_whose_weights_come_through_the_last_cache(rules):
     mb = 2 ** 20
     cases = [(24, 7 * mb, 3 * mb), (24, 7 * mb, 72 * mb), (24, 7 * mb, 73 * mb), (24, 13 * mb, 3 * mb), (24, 13 * mb, 50 * mb), (24, 7 * mb, 400 * mb), (8, 78 * mb, 40 * mb), (64, 0, 300 * mb)]
     assert rules("layers_in_cache((int)a, b, c)", [(*c, 0) for c in cases]) == [24, 24, 21, 16, 13, 0, 2, 0]
-    assert rules("streams_in_proj(a, (int)b)", [(240 * mb, 4, 0, 0), (240 * mb + 1, 4, 0, 0), (10 ** 9, 32, 0, 0), (10 ** 9, 33, 0, 0)]) == [0, 1, 1, 0]
+    assert rules("streams_in_proj(a, (int)b)", [(240 * mb, 4, 0, 0), (240 * mb + 1, 4, 0, 0), (10 ** 9, 48, 0, 0), (10 ** 9, 49, 0, 0)]) == [0, 1, 1, 0]
 
 
 def test_the_own_chain_takes_every_row_count_up_to_d_model_1536(rules):
