@@ -351,3 +351,24 @@ def test_scan_rejects_bad_arguments():
     expect(-2, _10=0)            # batch = 0
     _lib.call("mrs_ssm_scan_fwd", *args)   # and the unmodified call succeeds
     torch.cuda.synchronize()
+
+
+def test_scan_refuses_what_it_cannot_read():
+    """Each operand wrong in turn: another dtype, another shape, strides that are not row-dense, the host's memory."""
+    B, T, di, ds = 2, 24, 64, 16
+    cuda = lambda *s, t=torch.bfloat16: torch.zeros(*s, device="cuda:0", dtype=t)  # noqa: E731
+    good = lambda: {"h": cuda(B, di, ds, t=torch.float32), "y": cuda(B, T, di), "delta": cuda(B, T, di), "u": cuda(B, T, di), "B": cuda(B, T, ds), "C": cuda(B, T, ds),  # noqa: E731
+                    "a_neg": cuda(di, ds, t=torch.float32), "D": cuda(di, t=torch.float32), "gate": cuda(B, T, di)}
+    call = lambda a: ops.ssm_scan_fwd(a["h"], a["y"], a["delta"], a["u"], a["B"], a["C"], a["a_neg"], a["D"], gate=a["gate"], flags=ops.GATE_SILU)  # noqa: E731
+    call(good())
+    xd = cuda(B, T, 80)
+    call({**good(), "B": xd[:, :, 48:64], "C": xd[:, :, 64:]})
+    bad = [(n, t.to(torch.float16)) for n, t in good().items()]
+    bad += [(n, t.cpu()) for n, t in good().items() if n != "gate"]
+    bad += [(n, t[..., :-1]) for n, t in good().items()]
+    bad += [(n, t[:1].contiguous()) for n, t in good().items()]
+    bad += [("B", xd[:, :, 48:64]), ("B", cuda(B, ds, T).transpose(1, 2)), ("C", cuda(T, B, ds).transpose(0, 1)), ("gate", cuda(B, di, T).transpose(1, 2)),
+            ("u", cuda(B, T, 2 * di)[:, :, :di]), ("delta", cuda(B, T, di).to(torch.float64)), ("h", cuda(B, ds, di, t=torch.float32).transpose(1, 2))]
+    for n, t in bad:
+        with pytest.raises(ValueError):
+            call({**good(), n: t})
