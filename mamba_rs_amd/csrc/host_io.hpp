@@ -63,8 +63,9 @@ inline int host_io_wait(HostIo *io, hipStream_t st) {
 }
 
 // A float of the result, written past the caches, and one row's flag behind all of them: every thread of the workgroup that wrote the row calls host_row_done.
-// Nothing but these floats has to be with the host before the flag is, so each wave waits for its own stores and that is all.  (A fence for the whole system writes
-// back every changed line of the die's L2 first, once for each row.)
+// Nothing but these floats has to be out before the flag is, so each wave waits for its own stores and that is all.  (A fence for the whole system writes
+// back every changed line of the die's L2 first, once for each row.)  A single-launch step writes its final rows on the device in the same way: the flags let the caller
+// go on before the launch has ended, and another stream of the caller's may read them through temporal_ptr().
 __device__ __forceinline__ void host_store(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 __device__ __forceinline__ void host_row_done(const HostRows &h, int row) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -242,7 +242,7 @@ template <int DM, typename Args> __device__ __forceinline__ void stream_output(c
     const float inv = rms_inv(wave_sum(lane_squares<DM>(res)), DM, a.eps);
     if (tid < DM) {
         const float v = xin[tid] * inv;
-        a.temporal[(int64_t)b * DM + tid] = v;
+        host_store(a.temporal + (int64_t)b * DM + tid, v);
         if (a.host.out) host_store(a.host.out + (int64_t)b * DM + tid, v);
     }
     if (a.host.out) host_row_done(a.host, b);

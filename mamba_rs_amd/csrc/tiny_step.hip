@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     const float inv = rms_inv(block_sum(ss, red), dm, a.eps);
     for (int i = tid; i < dm; i += kTinyThreads) {
         const float v = res[i] * inv * a.norm_f[i];
-        a.temporal[(int64_t)b * dm + i] = v;
+        host_store(a.temporal + (int64_t)b * dm + i, v);
         if (a.host.out) host_store(a.host.out + (int64_t)b * dm + i, v);
     }
     if (a.host.out) host_row_done(a.host, b);

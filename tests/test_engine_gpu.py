@@ -562,6 +562,32 @@ def test_rows_a_step_hands_to_the_host_are_the_rows_it_leaves_on_the_device(dm, 
     eng.close()
 
 
+@pytest.mark.parametrize("family,dm,B", [("m1", 64, 1), ("m1", 128, 128), ("m1", 96, 3), ("m3", 64, 5), ("m3", 128, 48)])
+def test_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, B):
+    """step() returns on the rows' flags, before its launch has ended: the final rows behind temporal_ptr(), read by another stream with no wait in between, are those of the host, bit
+    for bit (row-streaming and general forms of the single-launch steps)."""
+    import torch
+    from mamba_rs_amd import GpuMamba3Backbone, Mamba3Config, Mamba3Weights
+    if family == "m1":
+        cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+        eng = GpuMambaBackbone.new(0, MambaWeights.init(cfg, 24, 5), cfg, 24, B)
+    else:
+        cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+        eng = GpuMamba3Backbone.new(0, Mamba3Weights.init(cfg, 24, 5), cfg, 24, B)
+
+    class Rows:
+        __cuda_array_interface__ = {"shape": (B, dm), "typestr": "<f4", "version": 3, "data": (eng.temporal_ptr(), False), "strides": None}
+    rows, side = torch.as_tensor(Rows(), device="cuda:0"), torch.cuda.Stream()
+    kept = torch.empty_like(rows)
+    rng = np.random.default_rng(B)
+    with torch.cuda.stream(side):
+        for t in range(20):
+            got = eng.step(rng.standard_normal((B, 24)).astype(np.float32))
+            kept.copy_(rows)
+            assert np.isfinite(got).all() and np.array_equal(got, kept.cpu().numpy()), t
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,L,B", [(96, 2, 1), (160, 2, 17), (192, 2, 4), (192, 1, 128), (256, 2, 5), (256, 2, 16), (768, 1, 33), (1088, 1, 7), (800, 1, 64), (192, 1, 129)])
 def test_f32_rows_on_the_own_chain_follow_the_cpu_route(dm, L, B):
     """f32 models past the single-launch step: the own chain with its products on the matrix cores' f32 instructions (k-steps fewer than the waves, row tiles partly filled, more rows
