@@ -12,8 +12,8 @@
 namespace mrs {
 
 // A flag has a line of host memory to itself: the host reads it over and over while the GPU's writes come in, and with sixteen rows' flags in a line every one
-// of those writes takes the line away from it.  Flags apart and rows written past the caches (host_store below), a step of four f32 layers, before / now, us:
-// d_model 128 1 row 32.7 / 31.3, 48 rows 40.3 / 33.1, 128 rows 52.8 / 34.1; Mamba-3 34.5 / 32.4, 41.4 / 34.6, 53.9 / 35.6.
+// of those writes takes the line away from it.  Flags apart, rows and states written past the caches (host_store below), a step of three f32 layers, before / now, us:
+// d_model 64 1 row 20.1 / 19.1, 48 rows 27.2 / 20.9, 128 rows 38.6 / 21.5; 128 28.1 / 28.4, 35.7 / 30.4, 48.0 / 32.1; Mamba-3, four layers of 128, 34.5 / 32.4, 41.4 / 34.6, 53.9 / 35.6.
 constexpr int kHostFlag = 16;
 
 struct HostIo {
@@ -64,9 +64,15 @@ inline int host_io_wait(HostIo *io, hipStream_t st) {
 
 // A float of the result, written past the caches, and one row's flag behind all of them: every thread of the workgroup that wrote the row calls host_row_done.
 // Nothing but these floats has to be out before the flag is, so each wave waits for its own stores and that is all.  (A fence for the whole system writes
-// back every changed line of the die's L2 first, once for each row.)  A single-launch step writes its final rows on the device in the same way: the flags let the caller
-// go on before the launch has ended, and another stream of the caller's may read them through temporal_ptr().
+// back every changed line of the die's L2 first, once for each row.)  A single-launch step writes its final rows on the device in the same way, and the Mamba-1 ones
+// their states: the flags let the caller go on before the launch has ended, and another stream of the caller's may use what temporal_ptr() and state_ptrs() give.
 __device__ __forceinline__ void host_store(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+// Four of them, `off` bytes (a multiple of 16) into a block of `bytes` that all lanes share.
+__device__ __forceinline__ void host_store4(float *block, int bytes, unsigned off, float4 v) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kSystem = 1 | 16;   // sc0, sc1: what the stores above have
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), __builtin_amdgcn_make_buffer_rsrc(block, 0, bytes, 0x00020000), off, 0, kSystem);
+}
 __device__ __forceinline__ void host_row_done(const HostRows &h, int row) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

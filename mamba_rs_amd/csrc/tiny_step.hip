@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
                 if (k < dc) {
                     const float v = k + 1 < dc ? cwin[k + 1 < 8 ? k + 1 : 7] : proj[tid];
                     s = fmaf(v, ctap[k], s);
-                    cst[(int64_t)tid * dc + k] = v;
+                    host_store(cst + (int64_t)tid * dc + k, v);
                 }
             }
             u[tid] = silu(s);
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
             hv.y = fmaf(fast_exp2(x * av.y), hv.y, du * Bv[1]);
             hv.z = fmaf(fast_exp2(x * av.z), hv.z, du * Bv[2]);
             hv.w = fmaf(fast_exp2(x * av.w), hv.w, du * Bv[3]);
-            *reinterpret_cast<float4 *>(hst + (int64_t)d * ds + 4 * g) = hv;
+            host_store4(hst, 4 * di * ds, 4u * (unsigned)(d * ds + 4 * g), hv);
             float acc = hv.x * Cv[0];
             acc = fmaf(hv.y, Cv[1], acc);
             acc = fmaf(hv.z, Cv[2], acc);
@@ -281,7 +281,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
             s = fmaf(win.z, tap.y, s);
             s = fmaf(win.w, tap.z, s);
             s = fmaf(p, tap.w, s);
-            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(cst) + ch16) = make_float4(win.y, win.z, win.w, p);
+            host_store4(cst, 16 * di, ch16, make_float4(win.y, win.z, win.w, p));
             u[tid] = silu(s);
         } else if (tid < 2 * di) {
             gate[tid - di] = silu(p);
@@ -335,12 +335,11 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
             const float dv = dl[d], uv = u[d], gv = gate[d], Dv = vec[6 * 256 + d];
             feed(2 + p);
             const float du = dv * uv, x = dv * kLog2e;
-            float4 h = hv[p];
+            float4 &h = hv[p];
             h.x = fmaf(fast_exp2(x * av[p].x), h.x, du * Bv[0]);
             h.y = fmaf(fast_exp2(x * av[p].y), h.y, du * Bv[1]);
             h.z = fmaf(fast_exp2(x * av[p].z), h.z, du * Bv[2]);
             h.w = fmaf(fast_exp2(x * av[p].w), h.w, du * Bv[3]);
-            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(hst + p * rows_pp * ds) + st4) = h;
             float s = h.x * Cv[0];
             s = fmaf(h.y, Cv[1], s);
             s = fmaf(h.z, Cv[2], s);
@@ -351,6 +350,10 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         if (passes == 1) feed(3);
         // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer (and, as above, a part of them is waited for).
         if (!kLast) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(In::rows / 4) : "memory");
+        pin();
+        // The states go all the way to memory, which takes about a microsecond: behind the wait above, with out_proj in front of the next one (three layers of 128, one row: 28.7 us, 29.1 in front of it and in halves).
+#pragma unroll
+        for (int p = 0; p < passes; p++) host_store4(hst, 4 * di * ds, st4 + 4u * (unsigned)(p * rows_pp * ds), hv[p]);
         pin();
         lds_barrier();
         // out_proj and residual

@@ -588,6 +588,40 @@ def test_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, B):
     eng.close()
 
 
+@pytest.mark.parametrize("dm,dc,B", [(64, 4, 1), (128, 4, 64), (96, 3, 3)])
+def test_states_of_a_step_are_on_the_device_when_it_returns(dm, dc, B):
+    """The same of the states behind state_ptrs(): another stream reads those that a later download gives, and a step goes on from what another stream put there."""
+    import ctypes
+    import torch
+    from mamba_rs_amd import backbone
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=dc, expand=2, n_layers=2)
+    eng = GpuMambaBackbone.new(0, MambaWeights.init(cfg, 24, 5), cfg, 24, B)
+    bind, di, last = backbone._bind(), 2 * dm, cfg.n_layers - 1
+    conv, ssm = ctypes.c_void_p(), ctypes.c_void_p()
+    assert bind.mrs_backbone_state_ptrs(eng._h, last, ctypes.byref(conv), ctypes.byref(ssm)) == 0
+
+    def view(ptr, *shape):
+        return torch.as_tensor(type("View", (), {"__cuda_array_interface__": {"shape": shape, "typestr": "<f4", "version": 3, "data": (ptr.value, False), "strides": None}})(), device="cuda:0")
+    views, side = [view(conv, B, di, dc), view(ssm, B, di, 16)], torch.cuda.Stream()
+    kept = [torch.empty_like(v) for v in views]
+    rng = np.random.default_rng(B)
+    with torch.cuda.stream(side):
+        for t in range(20):
+            eng.step(rng.standard_normal((B, 24)).astype(np.float32))
+            for k, v in zip(kept, views):
+                k.copy_(v)
+            side.synchronize()
+            for k, d in zip(kept, eng.download_state(last)):
+                assert np.array_equal(k.cpu().numpy().ravel(), np.asarray(d).ravel()), t
+            if t == 10:   # both states back to nothing, behind the step that has just returned
+                eng.step(rng.standard_normal((B, 24)).astype(np.float32))
+                for v in views:
+                    v.zero_()
+                side.synchronize()
+                assert not any(np.asarray(d).any() for d in eng.download_state(last))
+    eng.close()
+
+
 @pytest.mark.parametrize("dm,L,B", [(96, 2, 1), (160, 2, 17), (192, 2, 4), (192, 1, 128), (256, 2, 5), (256, 2, 16), (768, 1, 33), (1088, 1, 7), (800, 1, 64), (192, 1, 129)])
 def test_f32_rows_on_the_own_chain_follow_the_cpu_route(dm, L, B):
     """f32 models past the single-launch step: the own chain with its products on the matrix cores' f32 instructions (k-steps fewer than the waves, row tiles partly filled, more rows
