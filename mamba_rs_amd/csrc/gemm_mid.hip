@@ -17,6 +17,7 @@
 // 64 x 128 (18.3 / 14.7), and the operands of the next k-step read from LDS under the products (no change).
 #include "common.hpp"
 #include "mfma_tiles.hpp"
+#include "size_rules.hpp"
 #include <algorithm>
 
 namespace mrs {
@@ -143,7 +144,7 @@ int mid_gemm_slices(int64_t M, int N, int K) {
 
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {
     return (dtype == MRS_BF16 || dtype == MRS_F16) && M >= 1 && N >= 4 && N % 4 == 0 && K >= kStepK && K % kStepK == 0 && lda % 8 == 0 && lda >= K && ldc % 4 == 0 &&
-           ldc >= N && aligned(C, out_f32 ? 16 : 8) && aligned(A, 16) && aligned(Wt, 16) && M * lda < (int64_t)1 << 30 && (int64_t)N * K < (int64_t)1 << 30;
+           ldc >= N && C && aligned(C, out_f32 ? 16 : 8) && in_pieces(A) && in_pieces(Wt) && M * lda < (int64_t)1 << 30 && (int64_t)N * K < (int64_t)1 << 30;
 }
 
 int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {

@@ -1193,7 +1193,8 @@ static int alloc_prefill_scratch3(mrs_m3_backbone *bb, int T) {
     MRS_TRY(dev_alloc3(bb, &bb->pf_y, rows * di * es));
     MRS_TRY(dev_alloc3(bb, &bb->pf_gated, rows * di * es));
     MRS_TRY(dev_alloc3(bb, &bb->pf_out, rows * dm * es));
-    bb->pf_n_parts = bb->dtype != MRS_F32 && add_rmsnorm_parts_ok((int)dm) ? mid_gemm_slices(rows, (int)dm, (int)di) : 1;
+    // (the slices' kernel reads the transposed copy of out_proj, which is there where the decode runs on the own chain)
+    bb->pf_n_parts = bb->skinny && bb->dtype != MRS_F32 && add_rmsnorm_parts_ok((int)dm) ? mid_gemm_slices(rows, (int)dm, (int)di) : 1;
     if (bb->pf_n_parts > 1) MRS_TRY(dev_alloc3(bb, (void **)&bb->pf_parts, (size_t)bb->pf_n_parts * rows * dm * sizeof(float)));
     size_t wsb = mrs_m3_ssd_workspace_bytes(bb->batch, T, (int)nh, c.headdim, c.d_state, 64);
     const size_t abg = 3 * rows * nh * 4;   // alpha, beta, gamma for shapes the chunked kernel does not take
@@ -1280,7 +1281,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
         const Layer3 &lw = bb->layers[l];
         float *ssm = bb->ssm + (size_t)l * B * nh * hd * ds, *kst = bb->kst + (size_t)l * B * nh * ds;
         float *vst = bb->vst + (size_t)l * B * nh * hd, *ang = bb->angle + (size_t)l * B * nh * (nr > 0 ? nr : 1);
-        const bool in_parts = bb->pf_n_parts > 1 && mid_gemm_ok(dt, 1, bb->pf_parts, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di);   // (the same for every layer)
+        const bool in_parts = bb->pf_n_parts > 1 && lw.out_proj_t && mid_gemm_ok(dt, 1, bb->pf_parts, dm, bb->pf_gated, di, lw.out_proj_t, rows, dm, di);   // (the same for every layer)
         if (in_parts && l > 0) MRS_TRY(launch_add_rmsnorm_parts(bb->stream, dt, bb->pf_residual, bb->pf_parts, bb->pf_n_parts, bb->pf_normed, lw.norm_w, c.rms_norm_eps, rows, dm));
         else MRS_TRY(launch_add_rmsnorm3(bb, bb->pf_residual, l == 0 ? nullptr : bb->pf_out, bb->pf_normed, false, lw.norm_w, rows));
         // in_proj.  The bulk columns (z, x) come out in the storage type; B, C, the head scalars and the angle inputs

@@ -5,6 +5,9 @@
 
 namespace mrs {
 
+// An operand that a kernel reads in pieces of sixteen bytes: it is there (a null pointer lies on such a piece as well) and begins on one.
+inline bool in_pieces(const void *p) { return p && reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 // conv1d + SiLU and x_proj of a prefill as one launch (conv_xproj.hip).  Columns of x_proj in tiles of 16: from three (33 columns, the fewest of d_state 16) to
 // twelve, which leave room for four pieces of 64 channels in LDS, the fewest that keep requests ahead of their use.
 constexpr int kConvPiece = 64, kConvMinTiles = 3, kConvMaxTiles = 12, kConvMaxSlices = 16;

@@ -261,6 +261,34 @@ def test_prefill_equals_T_steps_of_the_cpu_path_and_hands_off_to_step(ci, T, dty
     eng.close()
 
 
+@pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
+@pytest.mark.parametrize("dm,expand,B,T", [
+    (768, 2, 129, 2),   # more rows than the decode's own chain takes
+    (112, 4, 1, 40),    # a width that it does not take
+    (768, 2, 128, 2),   # its most rows: out_proj in slices of K
+])
+def test_short_prefill_with_and_without_transposed_copies(dm, expand, B, T, dtype):
+    """A 16-bit engine has the transposed copies of its weights where its decode runs on the own chain, and a prefill of few rows cuts out_proj's K into slices only there.  Two layers, as
+    the last one's product is never in slices; tolerances as above."""
+    cfg = Mamba3Config(d_model=dm, d_state=64, expand=expand, headdim=64, ngroups=1, n_layers=2, rope_fraction=0.5)
+    w = perturbed(cfg, dm, 3)
+    w.input_proj_w = np.zeros(0, np.float32)
+    wi = Mamba3Weights(np.eye(dm, dtype=np.float32), np.zeros(dm, np.float32), w.layers, w.norm_f_weight)
+    P = oracle_params(wi, cfg, dm, round_to=orc.BF16 if dtype == WeightDtype.BF16 else orc.F16)
+    xs = np.random.default_rng(B).standard_normal((B, T, dm)).astype(np.float32)
+    print(f"case m3 short prefill {dm} {B}x{T} {dtype.name}", flush=True)
+    eng = GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, B, dtype)
+    assert eng.decode_route() == (1 if B == 128 else 0)
+    last = eng.prefill_sequence(xs)
+    ssm = eng.download_state(1)[0]
+    for b in sorted({0, B // 2, B - 1}):
+        st = P.zero_state()
+        for t in range(T):
+            want = orc.m3_backbone_step(P, xs[b, t], st)
+        assert cosine(last[b], want) >= 0.999 and cosine(ssm[b], st[0][1]) >= 0.995, (b, cosine(last[b], want), cosine(ssm[b], st[0][1]))
+    eng.close()
+
+
 def test_prefill_twice_continues_the_state_and_unsupported_chunk_shape_takes_the_sequential_route():
     """Two prefills of T steps == the CPU path over 2T steps (carried ssm/k/v/angle state); d_state 128 is outside the
     chunked kernel's shapes, so the engine forms alpha/beta/gamma and runs the recurrence kernel."""

@@ -24,6 +24,10 @@ def rules(tmp_path_factory):
     return run
 
 
+def test_an_operand_that_is_not_there_lies_on_no_piece(rules):
+    assert rules("in_pieces((const void *)a)", [(p, 0, 0, 0) for p in (0, 16, 4096, 8, 4098)]) == [0, 1, 1, 0, 0]
+
+
 def _columns(dm, ds=16):
     return (dm + 15) // 16 + 2 * ds
 
