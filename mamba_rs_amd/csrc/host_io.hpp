@@ -64,8 +64,8 @@ inline int host_io_wait(HostIo *io, hipStream_t st) {
 
 // A float of the result, written past the caches, and one row's flag behind all of them: every thread of the workgroup that wrote the row calls host_row_done.
 // Nothing but these floats has to be out before the flag is, so each wave waits for its own stores and that is all.  (A fence for the whole system writes
-// back every changed line of the die's L2 first, once for each row.)  A single-launch step writes its final rows on the device in the same way, and the Mamba-1 ones
-// their states: the flags let the caller go on before the launch has ended, and another stream of the caller's may use what temporal_ptr() and state_ptrs() give.
+// back every changed line of the die's L2 first, once for each row.)  A single-launch step writes its final rows and the copy of its input rows on the device in the same way, and the
+// Mamba-1 ones their states: the flags let the caller go on before the launch has ended, and another stream of the caller's may use what temporal_ptr(), input_ptr() and state_ptrs() give.
 __device__ __forceinline__ void host_store(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 // Four of them, `off` bytes (a multiple of 16) into a block of `bytes` that all lanes share.
 __device__ __forceinline__ void host_store4(float *block, int bytes, unsigned off, float4 v) {

@@ -185,7 +185,7 @@ __device__ __forceinline__ void stream_input(const Args &a, const float *norm_w,
     pin();
     if (tid < a.input_dim) {
         xin[tid] = v0;
-        if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + tid] = v0;   // (the input came straight from host memory)
+        if (a.input_copy) host_store(a.input_copy + (int64_t)b * a.input_dim + tid, v0);   // (the input came straight from host memory)
     }
     lds_barrier();
     float r;

@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     for (int i = tid; i < a.input_dim; i += kTinyThreads) {
         const float v = a.input[(int64_t)b * a.input_dim + i];
         xin[i] = v;
-        if (a.input_copy) a.input_copy[(int64_t)b * a.input_dim + i] = v;   // (the input came straight from host memory)
+        if (a.input_copy) host_store(a.input_copy + (int64_t)b * a.input_dim + i, v);   // (the input came straight from host memory)
     }
     __syncthreads();
     if (a.in_w) {

@@ -588,6 +588,45 @@ def test_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, B):
     eng.close()
 
 
+@pytest.mark.parametrize("family,dm,ds,B", [("m1", 64, 16, 1), ("m1", 128, 16, 128), ("m1", 64, 8, 3), ("m3", 64, 16, 5), ("m3", 128, 16, 48), ("m3", 96, 16, 3)])
+def test_input_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, ds, B):
+    """The same of the input rows behind input_ptr(): another stream reads those of the step that has just returned, and what it puts there is what a step on the device starts from."""
+    import torch
+    from mamba_rs_amd import GpuMamba3Backbone, Mamba3Config, Mamba3Weights
+    if family == "m1":
+        cfg = MambaConfig(d_model=dm, d_state=ds, d_conv=4, expand=2, n_layers=2)
+        w = MambaWeights.init(cfg, 24, 5)
+        make = lambda: GpuMambaBackbone.new(0, w, cfg, 24, B)  # noqa: E731
+    else:
+        cfg = Mamba3Config(d_model=dm, d_state=ds, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+        w = Mamba3Weights.init(cfg, 24, 5)
+        make = lambda: GpuMamba3Backbone.new(0, w, cfg, 24, B)  # noqa: E731
+    eng, plain = make(), make()
+    assert eng.decode_route() == 2
+
+    def view(ptr, width):
+        return torch.as_tensor(type("View", (), {"__cuda_array_interface__": {"shape": (B, width), "typestr": "<f4", "version": 3, "data": (ptr, False), "strides": None}})(), device="cuda:0")
+    rows, final, side = view(eng.input_ptr(), 24), view(eng.temporal_ptr(), dm), torch.cuda.Stream()
+    kept = torch.empty_like(rows)
+    rng = np.random.default_rng(B)
+    with torch.cuda.stream(side):
+        for t in range(20):
+            x, follow = (rng.standard_normal((B, 24)).astype(np.float32) for _ in range(2))
+            put = torch.from_numpy(follow).cuda()
+            side.synchronize()
+            eng.step(x)
+            kept.copy_(rows)
+            rows.copy_(put)
+            side.synchronize()
+            assert np.array_equal(kept.cpu().numpy(), x), t
+            eng.step_gpu_only()
+            eng.sync()
+            plain.step(x)
+            assert np.array_equal(final.cpu().numpy(), plain.step(follow)), t
+    eng.close()
+    plain.close()
+
+
 @pytest.mark.parametrize("dm,dc,B", [(64, 4, 1), (128, 4, 64), (96, 3, 3)])
 def test_states_of_a_step_are_on_the_device_when_it_returns(dm, dc, B):
     """The same of the states behind state_ptrs(): another stream reads those that a later download gives, and a step goes on from what another stream put there."""
