@@ -118,8 +118,8 @@ def ssm_scan_fwd(h, y, delta, u, B, C, a_neg, D, *, gate=None, flags: int = 0, w
     gate_stride = 0
     if gate is not None:
         g_strides = gate.stride()
-        if gate.shape != shape or g_strides[2] != 1 or g_strides[0] != T * g_strides[1]:
-            raise ValueError("gate must be [batch,T,d_inner], row-dense over [batch*T], unit inner stride")
+        if not gate.is_cuda or gate.shape != shape or g_strides[2] != 1 or g_strides[0] != T * g_strides[1]:
+            raise ValueError("gate must be a device tensor [batch,T,d_inner], row-dense over [batch*T], unit inner stride")
         gate_stride = g_strides[1]
     if static_scratch:
         if workspace is not None:

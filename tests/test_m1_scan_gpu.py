@@ -364,7 +364,7 @@ def test_scan_refuses_what_it_cannot_read():
     xd = cuda(B, T, 80)
     call({**good(), "B": xd[:, :, 48:64], "C": xd[:, :, 64:]})
     bad = [(n, t.to(torch.float16)) for n, t in good().items()]
-    bad += [(n, t.cpu()) for n, t in good().items() if n != "gate"]
+    bad += [(n, t.cpu()) for n, t in good().items()]
     bad += [(n, t[..., :-1]) for n, t in good().items()]
     bad += [(n, t[:1].contiguous()) for n, t in good().items()]
     bad += [("B", xd[:, :, 48:64]), ("B", cuda(B, ds, T).transpose(1, 2)), ("C", cuda(T, B, ds).transpose(0, 1)), ("gate", cuda(B, di, T).transpose(1, 2)),
