@@ -655,8 +655,7 @@ int launch_layer_step_t(mrs_m3_backbone *bb, int l) {
     float *ssm = bb->ssm + (size_t)l * B * nh * hd * ds, *kst = bb->kst + (size_t)l * B * nh * ds;
     float *vst = bb->vst + (size_t)l * B * nh * hd, *ang = bb->angle + (size_t)l * B * nh * (bb->nr > 0 ? bb->nr : 1);
     const dim3 grid((unsigned)(B * nh));
-    // four rows to a thread where that leaves a thread for every state and every pair to rotate
-    const int per = B * nh >= 192 && lg == 16 && hd % 4 == 0 && hd * lg / 4 >= std::max(ds, bb->nr) ? 4 : 1;
+    const int per = m3_step_rows(B, nh, hd, ds, bb->nr);
     const bool stream = per == 4 && step_outgrows_cache(c.n_layers * layer_weight_bytes3(bb) + (int64_t)m3_hook_state_bytes(bb));
     const dim3 block((unsigned)(hd * lg / per));
     if (per == 4) {

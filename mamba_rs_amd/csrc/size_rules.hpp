@@ -82,6 +82,13 @@ inline int layers_in_cache(int layers, int64_t layer_bytes, int64_t state_bytes)
     return (int)std::min<int64_t>(layers, std::max<int64_t>(0, ((int64_t)220 << 20) - state_bytes) / std::max<int64_t>(layer_bytes, 1));
 }
 
+// Rows of a Mamba-3 head's state that a thread of the step kernel has (m3_engine.hip, the times there): four from 192 heads on, at d_state 64, where the workgroup is then still whole waves
+// (its sums go over 64 lanes; headdim a multiple of 16) with a thread for every state and every pair to rotate.
+inline int m3_step_rows(int64_t batch, int nheads, int headdim, int d_state, int n_rope) {
+    const int threads = headdim * (d_state / 4) / 4;
+    return batch * nheads >= 192 && d_state == 64 && threads % 64 == 0 && threads >= std::max(d_state, n_rope) ? 4 : 1;
+}
+
 // Decode of a launch per product (wide models, and one to four rows of f32 ones): in_proj's weights, two thirds of a layer's, are read past that cache where a step (`bytes` of weights and states) outgrows it, so that
 // out_proj's and the states may stay and nothing has to be written back for what is read once.  Us a step, bf16, cached / past: d_model 2560, 8 layers 4 rows 322 / 294, 16 358 / 322,
 // 32 438 / 426, 64 577 / 573; 24 layers 4 rows 833 / 808, 16 938 / 877; 2048, 12 layers 4 rows 354 / 331, 16 392 / 370, 48 557 / 563 (there states are most of it); 24 of 1024, the states past it, 48 rows 568 / 543, 64 rows 623 / 634.  Some of the

@@ -142,16 +142,18 @@ def test_f32_rows_on_the_own_chain_match_cpu_reference_path(dm, B):
     eng.close()
 
 
-@pytest.mark.parametrize("dm,L,B,norm", [(768, 24, 9, False), (128, 2, 49, True), (128, 2, 49, False), (128, 2, 47, True)])
-def test_heads_of_64_by_64_at_many_rows_track_the_cpu_path(dm, L, B, norm):
-    """Four rows of a head's state to a thread from 192 heads up (49 rows of four heads), with and without the norm over the head; 24 layers of 768 at nine rows are more than the last
+@pytest.mark.parametrize("dm,L,B,norm,hd", [(768, 24, 9, False, 64), (128, 2, 49, True, 64), (128, 2, 49, False, 64), (128, 2, 47, True, 64),
+                                            (96, 2, 25, True, 24), (96, 2, 48, True, 48), (64, 2, 24, True, 16)])
+def test_heads_of_64_by_64_at_many_rows_track_the_cpu_path(dm, L, B, norm, hd):
+    """Four rows of a head's state to a thread from 192 heads up (49 rows of four heads; 48 and 24 of heads of 48 and 16: three waves and one; heads of 24 would be a wave and a half and
+    keep one row to a thread), with and without the norm over the head; 24 layers of 768 at nine rows are more than the last
     cache holds, so the states are read and written past it.  cosine >= 0.999 per step as for the 16-bit engines."""
-    cfg = Mamba3Config(d_model=dm, d_state=64, expand=2, headdim=64, ngroups=1, n_layers=L, rope_fraction=0.5, is_outproj_norm=norm)
+    cfg = Mamba3Config(d_model=dm, d_state=64, expand=2, headdim=hd, ngroups=1, n_layers=L, rope_fraction=0.5, is_outproj_norm=norm)
     w = perturbed(cfg, dm, 23)
     w.input_proj_w = np.zeros(0, np.float32)
     wi = Mamba3Weights(np.eye(dm, dtype=np.float32), np.zeros(dm, np.float32), w.layers, w.norm_f_weight)
     P = oracle_params(wi, cfg, dm, round_to=orc.BF16)
-    print(f"case m3 heads of 64 {dm} {L} {B} {norm}", flush=True)
+    print(f"case m3 heads of 64 {dm} {L} {B} {norm} {hd}", flush=True)
     eng = GpuMamba3Backbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.BF16)
     rows = (0, B - 1)
     st = {b: P.zero_state() for b in rows}

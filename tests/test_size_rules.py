@@ -80,6 +80,15 @@ def test_the_own_chain_takes_every_row_count_up_to_d_model_1536(rules):
     assert rules("own_chain_to_the_last_row(a, b)", [(dm, 2 * dm, 0, 0) for dm in (64, 768, 1024, 1536, 1792, 2560)] + [(2048, 2048, 0, 0)]) == [1, 1, 1, 1, 0, 0, 1]
 
 
+def test_the_mamba3_step_has_whole_waves(rules):
+    """Every head that an engine takes: headdim x d_state / 4 threads, a multiple of 64 of at most 1024."""
+    heads = [(hd, ds) for ds in (4, 8, 16, 32, 64, 128, 256) for hd in range(4, 257) if hd * (ds // 4) % 64 == 0 and hd * (ds // 4) <= 1024]
+    for batch, nh in ((1, 24), (8, 24), (191, 1), (3, 64)):
+        rows = rules("m3_step_rows(a / 1000, a % 1000, b, c, d)", [(1000 * batch + nh, hd, ds, ds // 2) for hd, ds in heads])
+        for (hd, ds), r in zip(heads, rows):
+            assert r == (4 if batch * nh >= 192 and ds == 64 and hd % 16 == 0 else 1) and hd * (ds // 4) // r % 64 == 0 and hd * (ds // 4) // r >= min(ds, 64), (batch, nh, hd, ds, r)
+
+
 def test_rows_of_the_f32_chain(rules):
     dims = (192, 256, 768, 1024, 1536, 2560)
     assert rules("own_f32_chain_rows(a, b, false)", [(dm, 2 * dm, 0, 0) for dm in dims]) == [128, 128, 128, 64, 48, 48]
