@@ -971,6 +971,7 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     if (!identity) {
         MRS_CREATE_TRY(upload_f32_3(bb, &bb->input_proj_w, w->input_proj_w, (size_t)input_dim * dm));
         if (w->input_proj_b) MRS_CREATE_TRY(upload_f32_3(bb, &bb->input_proj_b, w->input_proj_b, dm));
+        else { MRS_CREATE_TRY(dev_alloc3(bb, (void **)&bb->input_proj_b, (size_t)dm * 4)); hipMemsetAsync(bb->input_proj_b, 0, (size_t)dm * 4, bb->stream); }
     }
     bb->layers.resize(L);
     for (int l = 0; l < L; l++) {

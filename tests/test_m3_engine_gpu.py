@@ -263,6 +263,32 @@ def test_prefill_equals_T_steps_of_the_cpu_path_and_hands_off_to_step(ci, T, dty
     eng.close()
 
 
+@pytest.mark.parametrize("dm,B,dtype", [(64, 2, WeightDtype.F32), (128, 3, WeightDtype.BF16), (192, 5, WeightDtype.F32), (64, 129, WeightDtype.BF16)])
+def test_an_input_projection_without_a_bias(dm, B, dtype, monkeypatch):
+    """No bias at the C entry is a bias of zeros: in the single launch, in the projection's kernel, in front of the library's product (129 rows), and in a prefill, bit for bit."""
+    from mamba_rs_amd import mamba3
+    cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+    w = perturbed(cfg, 24, 4)
+    w.input_proj_b[:] = 0
+    print(f"case m3 no bias {dm} {B} {dtype.name}", flush=True)
+    zeros = GpuMamba3Backbone.new_with_dtype(0, w, cfg, 24, B, dtype)
+
+    def create(name, *args, call=mamba3._call):
+        if name == "mrs_m3_backbone_create":
+            args[2]._obj.input_proj_b = None
+        call(name, *args)
+    monkeypatch.setattr(mamba3, "_call", create)
+    none = GpuMamba3Backbone.new_with_dtype(0, w, cfg, 24, B, dtype)
+    rng = np.random.default_rng(B)
+    for _ in range(2):
+        x = rng.standard_normal((B, 24)).astype(np.float32)
+        assert np.array_equal(none.step(x), zeros.step(x))
+    x = rng.standard_normal((B, 5, 24)).astype(np.float32)
+    assert np.array_equal(none.prefill_sequence(x), zeros.prefill_sequence(x))
+    none.close()
+    zeros.close()
+
+
 @pytest.mark.parametrize("dtype", [WeightDtype.BF16, WeightDtype.F16])
 @pytest.mark.parametrize("dm,expand,B,T", [
     (768, 2, 129, 2),   # more rows than the decode's own chain takes
