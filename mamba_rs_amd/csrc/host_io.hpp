@@ -73,6 +73,15 @@ __device__ __forceinline__ void host_store4(float *block, int bytes, unsigned of
     constexpr int kSystem = 1 | 16;   // sc0, sc1: what the stores above have
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), __builtin_amdgcn_make_buffer_rsrc(block, 0, bytes, 0x00020000), off, 0, kSystem);
 }
+// What a single-launch step leaves on the device.  now: flags will say so (above).  Without them the launch's end brings it out, and the next step finds it in the L2.
+__device__ __forceinline__ void leave(bool now, float *p, float v) {
+    if (now) host_store(p, v);
+    else *p = v;
+}
+__device__ __forceinline__ void leave4(bool now, float *block, int bytes, unsigned off, float4 v) {
+    if (now) host_store4(block, bytes, off, v);
+    else *reinterpret_cast<float4 *>(reinterpret_cast<char *>(block) + off) = v;
+}
 __device__ __forceinline__ void host_row_done(const HostRows &h, int row) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

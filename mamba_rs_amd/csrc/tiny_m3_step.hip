@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_m3_backbone_step_kernel(Tin
     const float inv = rms_inv(block_sum(ss, red), dm, a.eps);
     for (int i = tid; i < dm; i += kTinyThreads) {
         const float v = res[i] * inv * a.norm_f[i];
-        host_store(a.temporal + (int64_t)b * dm + i, v);
+        leave(a.host.out != nullptr, a.temporal + (int64_t)b * dm + i, v);
         if (a.host.out) host_store(a.host.out + (int64_t)b * dm + i, v);
     }
     if (a.host.out) host_row_done(a.host, b);
@@ -365,7 +365,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_m3_stream
         lnext = after;
     }
     layer(std::true_type(), a.n_layers - 1);
-    stream_output<DM>(a, xin, res);
+    stream_output<DM>(a, a.host.out != nullptr, xin, res);
 }
 
 template <int DM> bool tiny_m3_stream_fits(const TinyM3StepArgs &a) {

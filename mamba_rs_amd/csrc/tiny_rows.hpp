@@ -237,15 +237,15 @@ template <typename S, typename F> __device__ __forceinline__ float4 stream_out_s
     return acc;
 }
 // The final norm: xin holds the residual stream times norm_f.
-template <int DM, typename Args> __device__ __forceinline__ void stream_output(const Args &a, const float *xin, const float *res) {
+template <int DM, typename Args> __device__ __forceinline__ void stream_output(const Args &a, bool now, const float *xin, const float *res) {
     const int tid = threadIdx.x, b = blockIdx.x;
     const float inv = rms_inv(wave_sum(lane_squares<DM>(res)), DM, a.eps);
     if (tid < DM) {
         const float v = xin[tid] * inv;
-        host_store(a.temporal + (int64_t)b * DM + tid, v);
-        if (a.host.out) host_store(a.host.out + (int64_t)b * DM + tid, v);
+        leave(now, a.temporal + (int64_t)b * DM + tid, v);
+        if (now) host_store(a.host.out + (int64_t)b * DM + tid, v);
     }
-    if (a.host.out) host_row_done(a.host, b);
+    if (now) host_row_done(a.host, b);
 }
 
 }  // namespace

@@ -32,6 +32,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     const int tid = threadIdx.x, b = blockIdx.x;
     const int lg = ds >> 2, rows_pp = kTinyThreads / lg;   // scan step: ds / 4 lanes per channel, one float4 of state each
     const int g = tid % lg, d0 = tid / lg;
+    const bool now = a.host.out != nullptr;
 
     TinyStepLayer lnext = a.layers[0];
     // input row -> residual stream (identity or projection + bias)
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
                 if (k < dc) {
                     const float v = k + 1 < dc ? cwin[k + 1 < 8 ? k + 1 : 7] : proj[tid];
                     s = fmaf(v, ctap[k], s);
-                    host_store(cst + (int64_t)tid * dc + k, v);
+                    leave(now, cst + (int64_t)tid * dc + k, v);
                 }
             }
             u[tid] = silu(s);
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
             hv.y = fmaf(fast_exp2(x * av.y), hv.y, du * Bv[1]);
             hv.z = fmaf(fast_exp2(x * av.z), hv.z, du * Bv[2]);
             hv.w = fmaf(fast_exp2(x * av.w), hv.w, du * Bv[3]);
-            host_store4(hst, 4 * di * ds, 4u * (unsigned)(d * ds + 4 * g), hv);
+            leave4(now, hst, 4 * di * ds, 4u * (unsigned)(d * ds + 4 * g), hv);
             float acc = hv.x * Cv[0];
             acc = fmaf(hv.y, Cv[1], acc);
             acc = fmaf(hv.z, Cv[2], acc);
@@ -160,10 +161,10 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
     const float inv = rms_inv(block_sum(ss, red), dm, a.eps);
     for (int i = tid; i < dm; i += kTinyThreads) {
         const float v = res[i] * inv * a.norm_f[i];
-        host_store(a.temporal + (int64_t)b * dm + i, v);
-        if (a.host.out) host_store(a.host.out + (int64_t)b * dm + i, v);
+        leave(now, a.temporal + (int64_t)b * dm + i, v);
+        if (now) host_store(a.host.out + (int64_t)b * dm + i, v);
     }
-    if (a.host.out) host_row_done(a.host, b);
+    if (now) host_row_done(a.host, b);
 }
 
 // The same step with the weights streamed, for models of the default expand, d_state, d_conv and dt_rank; of those this route takes
@@ -176,7 +177,9 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_backbone_step_kernel(TinySt
 // taken by every wave for itself and applied behind in_proj, partial sums added by the thread that needs the column, the vectors brought
 // by one request a wave.  A layer 5.3 us at d_model 128 and 2.25 at 64 (before: 10.4 and 8); the step of three layers, with the host's rows,
 // 44.1 -> 28.4 us and 37.4 -> 20.5, 256 rows 82.7 -> 72.0, 1024 rows 321 -> 272.
-template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_step_kernel(TinyStepArgs a) {
+// NOW: the host waits for flags (host_io.hpp), for which rows, windows and states are written all the way to memory; without them that costs a step 0.7 us and has the next one fetch its
+// states from there (three layers of 128 queued one behind the other, every step written through / as here: 1 row 19.0 / 18.0 us, 128 rows 20.3 / 19.3; of 64 10.7 / 10.1, 11.2 / 10.9).
+template <int DM, bool NOW> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_step_kernel(TinyStepArgs a) {
     extern __shared__ float lds[];
     constexpr int di = 2 * DM, ds = 16, dr = DM / 16, xd = dr + 2 * ds;
     constexpr int lg = ds / 4, rows_pp = kTinyThreads / lg, passes = (di + rows_pp - 1) / rows_pp;   // scan step: a float4 of state per lane
@@ -197,6 +200,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
     float *wo = dtl + (dr * di + 255) / 256 * 256;   // [Out::rows][threads] float4: out_proj's rows, each thread its own (last: the others are reached by constant offsets)
     const int tid = threadIdx.x, b = blockIdx.x;
     const Xp xp(tid);
+    const bool now = NOW && a.host.out;   // (the stores as blocks of their own behind this branch: with the host 27.8 us, without it 28.2)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned wo_at = lds_address(wo) + 1024u * wave, vec_at = lds_address(vec) + 1024u * wave, dt_at = lds_address(dtl) + 1024u * wave;
 
@@ -281,7 +285,8 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
             s = fmaf(win.z, tap.y, s);
             s = fmaf(win.w, tap.z, s);
             s = fmaf(p, tap.w, s);
-            host_store4(cst, 16 * di, ch16, make_float4(win.y, win.z, win.w, p));
+            win = make_float4(win.y, win.z, win.w, p);
+            if (!kLast || !now) leave4(now, cst, 16 * di, ch16, win);
             u[tid] = silu(s);
         } else if (tid < 2 * di) {
             gate[tid - di] = silu(p);
@@ -324,7 +329,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         }
         lds_barrier();
         // scan step + D skip + gate (the arithmetic of ssm_step_kernel)
-        if (kLast) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // out_proj's rows (ahead of the stores)
+        if (kLast) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // out_proj's rows (ahead of the layer's stores)
         const int g = tid % lg;
         float Bv[4], Cv[4];
 #pragma unroll
@@ -340,6 +345,7 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
             h.y = fmaf(fast_exp2(x * av[p].y), h.y, du * Bv[1]);
             h.z = fmaf(fast_exp2(x * av[p].z), h.z, du * Bv[2]);
             h.w = fmaf(fast_exp2(x * av[p].w), h.w, du * Bv[3]);
+            if (!now) leave4(false, hst + p * rows_pp * ds, 0, st4, h);
             float s = h.x * Cv[0];
             s = fmaf(h.y, Cv[1], s);
             s = fmaf(h.z, Cv[2], s);
@@ -351,9 +357,13 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         // The wave's rows of out_proj are in LDS: half of in_proj's requests are newer (and, as above, a part of them is waited for).
         if (!kLast) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(In::rows / 4) : "memory");
         pin();
-        // The states go all the way to memory, which takes about a microsecond: behind the wait above, with out_proj in front of the next one (three layers of 128, one row: 28.7 us, 29.1 in front of it and in halves).
+        // They take about a microsecond: behind the wait above, with out_proj in front of the next one, and in the last layer, whose wait is for everything, the window as well (three
+        // layers of 128, one row, with the host: 27.8 us; the window where it is formed 28.2, the states in front of the wait and in halves 29.1).
+        if (now) {
 #pragma unroll
-        for (int p = 0; p < passes; p++) host_store4(hst, 4 * di * ds, st4 + 4u * (unsigned)(p * rows_pp * ds), hv[p]);
+            for (int p = 0; p < passes; p++) host_store4(hst, 4 * di * ds, st4 + 4u * (unsigned)(p * rows_pp * ds), hv[p]);
+            if (kLast && tid < di) host_store4(cst, 16 * di, ch16, win);
+        }
         pin();
         lds_barrier();
         // out_proj and residual
@@ -376,19 +386,19 @@ template <int DM> __global__ __launch_bounds__(kTinyThreads) void tiny_stream_st
         lnext = after;
     }
     layer(std::true_type(), a.n_layers - 1);
-    stream_output<DM>(a, xin, res);
+    stream_output<DM>(a, now, xin, res);
 }
 
 template <int DM> bool tiny_stream_fits(const TinyStepArgs &a) {
     return a.dm == DM && a.di == 2 * DM && a.ds == 16 && a.dc == 4 && a.dr == DM / 16 && a.input_dim <= kStreamInput;
 }
-template <int DM> int launch_tiny_stream(hipStream_t st, const TinyStepArgs &a) {
+template <int DM, bool NOW> int launch_tiny_stream(hipStream_t st, const TinyStepArgs &a) {
     constexpr int dr = DM / 16, di = 2 * DM, xd = dr + 32;
     constexpr size_t lds = sizeof(float) * (kTinyPart + DM + 4 * di + xd + kStreamInput + 2048 + (dr * di + 255) / 256 * 256 + (size_t)Sweep<di, DM>::rows * 4 * kTinyThreads);
     static_assert(lds <= 160 * 1024, "LDS");
-    static const hipError_t attr = hipFuncSetAttribute((const void *)tiny_stream_step_kernel<DM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)tiny_stream_step_kernel<DM, NOW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(MRS_E_HIP, "tiny backbone step: LDS size: %s", hipGetErrorString(attr));
-    hipLaunchKernelGGL(tiny_stream_step_kernel<DM>, dim3((unsigned)a.batch), dim3(kTinyThreads), lds, st, a);
+    hipLaunchKernelGGL((tiny_stream_step_kernel<DM, NOW>), dim3((unsigned)a.batch), dim3(kTinyThreads), lds, st, a);
     return check_launch("tiny_stream_step_kernel");
 }
 
@@ -414,8 +424,8 @@ int launch_tiny_step(hipStream_t st, const TinyStepArgs &a) {
         !a.conv_state || !a.ssm_state || !a.temporal || !a.norm_f)
         return fail(MRS_E_SHAPE, "tiny backbone step: shape outside the single-launch route (d_model=%d d_inner=%d d_state=%d xdbl=%d)", a.dm, a.di,
                     a.ds, a.xd);
-    if (tiny_stream_fits<128>(a)) return launch_tiny_stream<128>(st, a);
-    if (tiny_stream_fits<64>(a)) return launch_tiny_stream<64>(st, a);
+    if (tiny_stream_fits<128>(a)) return a.host.out ? launch_tiny_stream<128, true>(st, a) : launch_tiny_stream<128, false>(st, a);
+    if (tiny_stream_fits<64>(a)) return a.host.out ? launch_tiny_stream<64, true>(st, a) : launch_tiny_stream<64, false>(st, a);
     const size_t lds = tiny_lds_bytes(a);
     if (lds > 64 * 1024) return fail(MRS_E_SHAPE, "tiny backbone step: %zu bytes of LDS", lds);
     hipLaunchKernelGGL(tiny_backbone_step_kernel, dim3((unsigned)a.batch), dim3(kTinyThreads), lds, st, a);
