@@ -166,9 +166,7 @@ int launch_tiled_gemm(hipStream_t st, int dtype, void *C, int out_f32, int64_t l
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
 bool mid_gemm_wins(int64_t M, int N, int K);
 int launch_mid_gemm(hipStream_t st, int dtype, int out_f32, void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K);
-// The same with K in slices, whose products are left side by side: parts [slices][M][N] f32, for add_rmsnorm_parts (glue.hpp).  mid_gemm_slices: how many are worth it (1: none)
-constexpr int kMaxMidSlices = 4;
-int mid_gemm_slices(int64_t M, int N, int K);
+// The same with K in slices, whose products are left side by side: parts [slices][M][N] f32, for add_rmsnorm_parts (glue.hpp).  mid_gemm_slices (size_rules.hpp): how many are worth it
 int launch_mid_gemm_parts(hipStream_t st, int dtype, float *parts, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K, int slices);
 // Logits of up to 64 rows (lm_head.hip) from a tiled table, f32 from 16-bit storage; with `keys` (lm_head_keys of them) each row's greedy pick as a key per workgroup, which
 // launch_pick turns into the token

@@ -233,8 +233,7 @@ struct Scratch {  // activations for M rows
     int64_t xpart_floats = 0;
     void *scan_ws = nullptr;
     size_t scan_ws_bytes = 0;
-    float *out_parts = nullptr; // prefill of few rows: out_proj as `n_parts` products over slices of K, [n_parts][rows][d_model]
-    int n_parts = 1;
+    float *out_parts = nullptr; // prefill of few rows: out_proj as products over slices of K, [slices][rows][d_model], the slices those of the call's rows
     int T = 0;
 };
 
@@ -294,7 +293,8 @@ static int upload_bulk(mrs_backbone *bb, void **dst, const float *src, size_t n,
     return check_launch("weight cast");
 }
 
-static int alloc_scratch(mrs_backbone *bb, Scratch *s, int64_t rows, int T) {
+// fewer_rows: calls of fewer steps use it as well
+static int alloc_scratch(mrs_backbone *bb, Scratch *s, int64_t rows, int T, bool fewer_rows = false) {
     const size_t es = esize(bb->dtype);
     const int dm = bb->cfg.d_model, di = bb->di, xd = bb->xd;
     s->rows = rows; s->T = T;
@@ -321,10 +321,10 @@ static int alloc_scratch(mrs_backbone *bb, Scratch *s, int64_t rows, int T) {
         s->xpart_floats = need;
         MRS_TRY(dev_alloc(bb, (void **)&s->xpart, (size_t)need * sizeof(float)));
     }
-    s->n_parts = 1;
     if (T > 1 && bb->dtype != MRS_F32 && add_rmsnorm_parts_ok(dm)) {
-        s->n_parts = mid_gemm_slices(rows, dm, di);
-        if (s->n_parts > 1) MRS_TRY(dev_alloc(bb, (void **)&s->out_parts, (size_t)s->n_parts * rows * dm * sizeof(float)));
+        const int slices = mid_gemm_slices(rows, dm, di);
+        const int64_t floats = fewer_rows ? mid_gemm_parts_floats(rows, dm, di) : slices > 1 ? slices * rows * dm : 0;
+        if (floats) MRS_TRY(dev_alloc(bb, (void **)&s->out_parts, (size_t)floats * sizeof(float)));
     }
     if (T > 1) {
         s->scan_ws_bytes = mrs_ssm_scan_workspace_bytes(bb->batch, T, di, bb->cfg.d_state);
@@ -508,6 +508,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
     const int64_t rows = (int64_t)B * T;
     const size_t es = esize(dt);
     const int L = bb->cfg.n_layers;
+    const int slices = T > 1 && s->out_parts ? mid_gemm_slices(rows, dm, di) : 1;
     if (T == 1 && bb->skinny) MRS_TRY(decode_chain(bb, s, 0, B, bb->stream));
     for (int l = 0; l < L && !(T == 1 && bb->skinny); l++) {
         const LayerDev &lw = bb->layers[l];
@@ -515,8 +516,8 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
         float *ssm = bb->ssm_state + (size_t)l * B * di * ds;
         const char *z = (const char *)s->proj + (size_t)di * es;  // gate half of in_proj's output
         const char *xb = (const char *)s->xdbl;
-        const bool in_parts = T > 1 && s->n_parts > 1 && mid_gemm_ok(dt, 1, s->out_parts, dm, s->y, di, lw.out_proj_t, rows, dm, di);   // (the same for every layer)
-        if (in_parts && l > 0) MRS_TRY(launch_add_rmsnorm_parts(bb->stream, dt, s->residual, s->out_parts, s->n_parts, s->normed, lw.norm_w, bb->cfg.rms_norm_eps, rows, dm));
+        const bool in_parts = slices > 1 && mid_gemm_ok(dt, 1, s->out_parts, dm, s->y, di, lw.out_proj_t, rows, dm, di);   // (the same for every layer)
+        if (in_parts && l > 0) MRS_TRY(launch_add_rmsnorm_parts(bb->stream, dt, s->residual, s->out_parts, slices, s->normed, lw.norm_w, bb->cfg.rms_norm_eps, rows, dm));
         else MRS_TRY(launch_add_rmsnorm(bb, s->residual, l == 0 ? nullptr : s->out, s->normed, false, lw.norm_w, rows, dm));
         // Behind the last layer only the last step of each sequence goes on (below), so its gate and its scan's outputs are formed there alone.  The gate half of
         // `proj` and the other rows of y then hold what they held before.  The scan's last chunk alone: 16384 x 5120 298 -> 94 + 81 us, x 1536 100 -> 35 + 34.  The gate as a product
@@ -605,7 +606,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
         }
         if (prefix && l + 1 == L) return MRS_OK;
         if (last) MRS_TRY(launch_last_step_gemm(bb->stream, dt, s->out, s->y, lw.out_proj_t, B, T, dm, di));
-        else if (in_parts && l + 1 < L) MRS_TRY(launch_mid_gemm_parts(bb->stream, dt, s->out_parts, s->y, di, lw.out_proj_t, rows, dm, di, s->n_parts));
+        else if (in_parts && l + 1 < L) MRS_TRY(launch_mid_gemm_parts(bb->stream, dt, s->out_parts, s->y, di, lw.out_proj_t, rows, dm, di, slices));
         else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
         else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));
@@ -1076,7 +1077,7 @@ static float *m1_hook_prefix_rows(void *self) {
     if (!prefix_ok(bb)) return nullptr;
     if (!bb->prefix_s.rows) {
         const size_t mark = bb->allocs.size();
-        if (alloc_scratch(bb, &bb->prefix_s, (int64_t)bb->batch * kPrefixSteps, kPrefixSteps)) {   // no room: step by step
+        if (alloc_scratch(bb, &bb->prefix_s, (int64_t)bb->batch * kPrefixSteps, kPrefixSteps, true)) {   // no room: step by step
             (void)hipGetLastError();
             for (size_t i = mark; i < bb->allocs.size(); i++) hipFree(bb->allocs[i]);
             bb->allocs.resize(mark);

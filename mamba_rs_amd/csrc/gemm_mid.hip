@@ -23,7 +23,7 @@
 namespace mrs {
 namespace {
 
-constexpr int kMidThreads = 256, kTile = 64, kStepK = 64, kStages = 4;
+constexpr int kMidThreads = 256, kTile = kMidTile, kStepK = kMidStepK, kStages = 4;
 
 template <typename T, typename TO>
 __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(TO *__restrict__ C, int64_t ldc, const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt,
@@ -125,21 +125,6 @@ int launch_mid(hipStream_t st, void *C, int64_t ldc, const void *A, int64_t lda,
 bool mid_gemm_wins(int64_t M, int N, int K) {
     const int64_t tiles = (M + kTile - 1) / kTile * ((N + kTile - 1) / kTile), steps = K / kStepK;
     return steps <= 40 && (tiles <= 256 || tiles * steps <= 10000);
-}
-
-// Slices of K for out_proj, whose products the next kernel sums (it reads the result anyway).  A compute unit takes in some 60 bytes a nanosecond whatever it has asked for, so 24
-// tiles of 64 x 64 over K 1536 take 10 us with nine tenths of the chip idle.  As many slices as make a workgroup for every unit, or two where their walk stays
-// long, four at most.  Us a layer of a bf16 prefill, one / two / three / four slices (six and eight: four's or behind):
-//   d_model 768   64 rows 54.1 / 51.5 / 50.5 / 50.1    256 63.8 / 60.8 / 60.0 / 59.3    512 71.8 / 68.7 / 69.8 / 69.2    1024 83.9 / 85.6 / 87.2 / 87.4
-//           1024  64 rows 65.5 / 61.9 / 60.7 / 60.0    256 71.2 / 66.9 / 65.5 / 65.4    512 79.6 / 75.9 / 77.1 / 77.1    777 92.0 / 91.5 / 93.0 / 94.3
-//           2560  64 rows 129 / 128 / 125 / 124        128 154 / 141 / 139 / 141        256 172 / 170 / 164 / 167 (one: the vendor kernel)
-//   Mamba-3 768   256 rows 80.5 / 77.8 / 77.0 / 76.7   512 84.9 / 82.0 / 82.8 / 82.5
-int mid_gemm_slices(int64_t M, int N, int K) {
-    const int64_t tiles = (M + kTile - 1) / kTile * ((N + kTile - 1) / kTile), steps = K / kStepK;
-    const int64_t want = std::min<int64_t>(std::min(std::max(256 / tiles, std::min(512 / tiles, steps / 24)), steps / 3), kMaxMidSlices);
-    if (want < 2 || K % kStepK != 0) return 1;
-    const int64_t per = (steps + want - 1) / want;
-    return (int)((steps + per - 1) / per);
 }
 
 bool mid_gemm_ok(int dtype, int out_f32, const void *C, int64_t ldc, const void *A, int64_t lda, const void *Wt, int64_t M, int N, int K) {

@@ -1,6 +1,7 @@
 // Glue kernels shared by the backbone engines: residual add + RMSNorm, casts, bias rows.
 #pragma once
 #include "common.hpp"
+#include "size_rules.hpp"
 
 namespace mrs {
 

@@ -45,6 +45,32 @@ inline int conv_xproj_form(int batch, int T, int di, int xd) {
 // 3266 / 3221, 4 x 4096 5887 / 6038).
 inline int conv_xproj_rows(int batch, int T) { return (int64_t)batch * ((T + 31) / 32) <= 320 ? 32 : 64; }
 
+// Slices of K for the out_proj of a prefill of few rows (gemm_mid.hip), whose products the next kernel sums (it reads the result anyway).  A compute unit takes in some 60 bytes a
+// nanosecond whatever it has asked for, so 24 tiles of 64 x 64 over K 1536 take 10 us with nine tenths of the chip idle.  As many slices as make a workgroup for every unit, or two where
+// their walk stays long, four at most.  Us a layer of a bf16 prefill, one / two / three / four slices (six and eight: four's or behind):
+//   d_model 768   64 rows 54.1 / 51.5 / 50.5 / 50.1    256 63.8 / 60.8 / 60.0 / 59.3    512 71.8 / 68.7 / 69.8 / 69.2    1024 83.9 / 85.6 / 87.2 / 87.4
+//           1024  64 rows 65.5 / 61.9 / 60.7 / 60.0    256 71.2 / 66.9 / 65.5 / 65.4    512 79.6 / 75.9 / 77.1 / 77.1    777 92.0 / 91.5 / 93.0 / 94.3
+//           2560  64 rows 129 / 128 / 125 / 124        128 154 / 141 / 139 / 141        256 172 / 170 / 164 / 167 (one: the vendor kernel)
+//   Mamba-3 768   256 rows 80.5 / 77.8 / 77.0 / 76.7   512 84.9 / 82.0 / 82.8 / 82.5
+constexpr int kMidTile = 64, kMidStepK = 64, kMaxMidSlices = 4;
+inline int mid_gemm_slices(int64_t M, int N, int K) {
+    const int64_t tiles = (M + kMidTile - 1) / kMidTile * ((N + kMidTile - 1) / kMidTile), steps = K / kMidStepK;
+    const int64_t want = std::min<int64_t>(std::min(std::max(256 / tiles, std::min(512 / tiles, steps / 24)), steps / 3), kMaxMidSlices);
+    if (want < 2 || K % kMidStepK != 0) return 1;
+    const int64_t per = (steps + want - 1) / want;
+    return (int)((steps + per - 1) / per);
+}
+// Floats that they take at most in a product of up to `rows` rows, which has slices by its own rows (0: none ever)
+inline int64_t mid_gemm_parts_floats(int64_t rows, int N, int K) {
+    const int64_t across = (N + kMidTile - 1) / kMidTile;
+    int64_t most = 0;
+    for (int64_t down = 1; down * across <= 256 && (down - 1) * kMidTile < rows; down++) {   // (a slice for every two units or fewer: past 256 tiles there are none)
+        const int64_t M = std::min(down * kMidTile, rows);
+        if (const int n = mid_gemm_slices(M, N, K); n > 1) most = std::max(most, n * M * N);
+    }
+    return most;
+}
+
 // Rows up to which a decode step's projections are the own kernels'.  Weights of up to ten million elements of in_proj (d_model 1536): as many as those kernels take; past that its
 // tiles of 16 x 16 read too much over again.  Us a step, bf16, library / own:
 //   12 layers of d_model 1024   48 rows 512 / 289, 64 540 / 329, 96 649 / 445, 128 682 / 511         1280   48 593 / 389, 64 675 / 485, 96 681 / 587, 128 821 / 697

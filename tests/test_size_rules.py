@@ -28,6 +28,16 @@ def test_an_operand_that_is_not_there_lies_on_no_piece(rules):
     assert rules("in_pieces((const void *)a)", [(p, 0, 0, 0) for p in (0, 16, 4096, 8, 4098)]) == [0, 1, 1, 0, 0]
 
 
+def test_slices_of_out_proj_are_those_of_the_rows_at_hand(rules):
+    """A generation's buffers are made for 32 steps of all slots and used by shorter pieces: 13 slots of d_model 1024 and 11 or 12 steps are 48 tiles in four slices (in 32 steps, 112 in two), 64 of
+    768 and four steps as well.  What a piece of any length takes is in the buffers, and slices never outgrow the chip or the sum behind them."""
+    assert rules("mid_gemm_slices(a, (int)b, (int)c)", [(13 * 11, 1024, 2048, 0), (13 * 12, 1024, 2048, 0), (13 * 32, 1024, 2048, 0), (64 * 4, 768, 1536, 0), (64 * 32, 768, 1536, 0)]) == [4, 4, 2, 4, 1]
+    lines = [(batch * T, dm, 2 * dm, batch * 32) for batch in (1, 3, 13, 64, 128) for dm in (64, 128, 320, 768, 1024, 1536, 2560, 4096) for T in range(2, 33)]
+    slices, room = rules("mid_gemm_slices(a, (int)b, (int)c)", lines), rules("mid_gemm_parts_floats(d, (int)b, (int)c)", lines)
+    for (rows, dm, _, _), n, r in zip(lines, slices, room):
+        assert 1 <= n <= 4 and (n == 1 or n * rows * dm <= r) and r <= 512 * 64 * 64, (rows, dm, n, r)
+
+
 def _columns(dm, ds=16):
     return (dm + 15) // 16 + 2 * ds
 
