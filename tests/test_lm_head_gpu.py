@@ -40,3 +40,21 @@ def test_logits_and_pick(dm, B, vocab, dtype, untied):
         assert ((got.double() - hid @ table).abs() <= bound).all(), step
         last = vocab - 1 - np.argmax(got.numpy()[:, ::-1], axis=1)
         assert np.array_equal(lm.get_tokens(), last), step
+
+
+@pytest.mark.parametrize("dm,B,dtype", [(768, 1, WeightDtype.BF16), (768, 64, WeightDtype.F16), (1024, 33, WeightDtype.BF16), (2560, 16, WeightDtype.BF16), (2560, 3, WeightDtype.F16)])
+def test_logits_are_sums_of_short_sums(dm, B, dtype):
+    """A rounding is 2^-24 / sqrt(3) of what is summed so far, so sums of four k-steps, added up over K / 128 of them, are off by that times sqrt(2 + K / 256) of their norm and one chain by
+    sqrt(K / 64): 0.8 and 1.2e-7 at 768, 1.2 and 2.2e-7 at 2560.  The matrix cores' sums within a k-step make it up to 1.1 and 1.4 times as much (measured); 1.25 times lies between."""
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 3)
+    w.input_proj_w = np.zeros(0, np.float32); w.input_proj_b = np.zeros(0, np.float32)
+    embed = torch.randn(2000, dm, generator=torch.Generator().manual_seed(B))
+    lm = GpuMambaLM(GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, dtype), embed.numpy(), None)
+    lm.set_tokens((np.arange(B) * 7).astype(np.int32))
+    lm.decode_step()
+    got = torch.from_numpy(lm.last_logits()).reshape(B, -1)[:, :2000].double()
+    want = torch.from_numpy(lm.backbone.download_temporal()).to(dtype.torch_dtype()).double() @ embed.to(dtype.torch_dtype()).double().T
+    off, unit = float((got - want).norm() / want.norm()), 2.0 ** -24 / 3 ** 0.5
+    print(f"logits {dm} {B} {dtype.name} {off:.3e} of {unit * (2 + dm / 256) ** 0.5:.3e}", flush=True)
+    assert off <= 1.25 * unit * (2 + dm / 256) ** 0.5
