@@ -716,6 +716,36 @@ def test_input_rows_through_the_projection_kernel(dm, idim, B):
     eng.close()
 
 
+@pytest.mark.parametrize("family,dm,idim,B,in_front", [("m1", 320, 88, 128, True), ("m1", 320, 88, 129, False), ("m3", 192, 40, 129, False), ("m1", 36, 4097, 2, False), ("m3", 192, 40, 3, True)])
+def test_what_stands_in_front_of_a_recorded_step(family, dm, idim, B, in_front):
+    """The library's products of a projection are part of the recorded step (more than 128 rows, more than 4096 inputs), the projection's kernel stands in front of it, as step() has it take
+    the rows from host memory: the calls of a step on the device, and the rows of steps with the host, bit for bit those of an engine that replays nothing."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    from mamba_rs_amd import GpuMamba3Backbone, Mamba3Config, Mamba3Weights
+    if family == "m1":
+        cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+        w = MambaWeights.init(cfg, idim, 5)
+        make = lambda: GpuMambaBackbone.new(0, w, cfg, idim, B)  # noqa: E731
+    else:
+        cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+        w = Mamba3Weights.init(cfg, idim, 5)
+        make = lambda: GpuMamba3Backbone.new_with_dtype(0, w, cfg, idim, B, WeightDtype.F32)  # noqa: E731
+    eager, recorded = make(), make()
+    rng = np.random.default_rng(B)
+    recorded.capture_graph()
+    for _ in range(3):
+        x = rng.standard_normal((B, idim)).astype(np.float32)
+        assert np.array_equal(eager.step(x), recorded.step(x))
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        recorded.step_gpu_only()
+        recorded.sync()
+    calls = [e.name for e in prof.events() if "Launch" in e.name]
+    assert calls == ["hipLaunchKernel"] * in_front + ["hipGraphLaunch"]
+    eager.close()
+    recorded.close()
+
+
 @pytest.mark.parametrize("dm,lens,dtype", [
     (128, (9, 5), WeightDtype.F16),              # four tokens; dt_rank 8: a quarter of a k-step of dt_proj
     (256, (6, 40, 18), WeightDtype.BF16),        # five
