@@ -1209,6 +1209,32 @@ int mrs::launch_embed_gather(hipStream_t st, int dtype, float *out, const void *
     return check_launch("embed_gather_kernel");
 }
 
+// `rows` rows of a table, f32 on the host, into `table` [vocab_padded, dm] in the storage type, with zeros behind them; 32 MB at a time, which is what the way there takes on the device.
+static hipError_t upload_table(mrs_lm *lm, void *table, const float *host, int64_t rows) {
+    const size_t es = esize(lm->dtype), dm = lm->dm;
+    const hipStream_t st = lm->eng.stream;
+    hipError_t e = rows < lm->vocab_padded ? hipMemsetAsync((char *)table + rows * dm * es, 0, (lm->vocab_padded - rows) * dm * es, st) : hipSuccess;
+    if (lm->dtype == MRS_F32) {
+        if (e == hipSuccess) e = hipMemcpyAsync(table, host, rows * dm * 4, hipMemcpyHostToDevice, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    }
+    const int64_t at_once = std::min<int64_t>(rows, std::max<int64_t>(1, ((int64_t)8 << 20) / (int64_t)dm));
+    float *stage = nullptr;
+    if (e == hipSuccess) e = hipMalloc((void **)&stage, at_once * dm * 4);
+    for (int64_t r = 0; r < rows && e == hipSuccess; r += at_once) {
+        const int64_t n = std::min(at_once, rows - r) * (int64_t)dm;
+        e = hipMemcpyAsync(stage, host + r * dm, n * 4, hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) break;
+        const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+        if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, st, (bf16_t *)table + r * dm, stage, n);
+        else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, st, (f16_t *)table + r * dm, stage, n);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(st);   // the next rows go to the same place
+    }
+    if (stage) hipFree(stage);
+    return e;
+}
+
 int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embed, int vocab, const char *fn) {
     if (!out || !eng.self || !embed) return fail(MRS_E_NULL, "%s: null pointer", fn);
     if (!eng.identity_proj) return fail(MRS_E_SHAPE, "%s: the LM feeds embeddings straight into the backbone (identity input_proj)", fn);
@@ -1223,8 +1249,7 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     lm->gen_prompt_cap = 0; lm->gen_out_cap = 0; lm->gen_dyn = nullptr; lm->gen_dyn_host = GenDyn{nullptr, nullptr, 0};
     *out = nullptr;
     const size_t es = esize(lm->dtype), ne = (size_t)lm->vocab_padded * lm->dm;
-    float *stage = nullptr;
-    auto cleanup = [&]() { for (void *p : lm->allocs) hipFree(p); if (stage) hipFree(stage); delete lm; };
+    auto cleanup = [&]() { for (void *p : lm->allocs) hipFree(p); delete lm; };
 #define MRS_LM_HIP(expr) do { hipError_t e_ = (expr); if (e_ != hipSuccess) { cleanup(); return fail(MRS_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); } } while (0)
     MRS_LM_HIP(hipMalloc(&lm->embed, ne * es)); lm->allocs.push_back(lm->embed);
     MRS_LM_HIP(hipMalloc((void **)&lm->logits, (size_t)lm->batch * lm->vocab_padded * 4)); lm->allocs.push_back(lm->logits);
@@ -1235,23 +1260,15 @@ int mrs_lm_create_from_hooks(mrs_lm **out, const LmHooks &eng, const float *embe
     lm->stream_table = step_outgrows_cache((int64_t)(ne * es + eng.weight_bytes + eng.state_bytes(eng.self)));
     if (lm_head_ok(lm->dtype, lm->batch, lm->vocab_padded, lm->dm)) {
         MRS_LM_HIP(hipMalloc((void **)&lm->arg_keys, lm_head_keys(lm->batch, lm->vocab_padded, lm->dm) * 8)); lm->allocs.push_back(lm->arg_keys);
-        lm->table_p = lm->embed;   // (a place of its own below)
+        MRS_LM_HIP(hipMalloc(&lm->table_p, tiled_weight_elems(lm->vocab_padded, lm->dm) * es)); lm->allocs.push_back(lm->table_p);
     }
-    MRS_LM_HIP(hipMalloc((void **)&stage, ne * 4));
-    MRS_LM_HIP(hipMemsetAsync(stage, 0, ne * 4, eng.stream));  // padded rows are zero
-    MRS_LM_HIP(hipMemcpyAsync(stage, embed, (size_t)vocab * lm->dm * 4, hipMemcpyHostToDevice, eng.stream));
-    const dim3 grid((unsigned)((ne + 255) / 256)), block(256);
-    if (lm->dtype == MRS_F32) MRS_LM_HIP(hipMemcpyAsync(lm->embed, stage, ne * 4, hipMemcpyDeviceToDevice, eng.stream));
-    else if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, eng.stream, (bf16_t *)lm->embed, stage, (int64_t)ne);
-    else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, eng.stream, (f16_t *)lm->embed, stage, (int64_t)ne);
-    if (lm->table_p) {   // the head's tiles stay where the f32 rows came in: an allocation of a table's size and a free take 15 ms
-        lm->table_p = stage; lm->allocs.push_back(stage); stage = nullptr;
+    MRS_LM_HIP(upload_table(lm, lm->embed, embed, vocab));
+    if (lm->table_p) {
         const int rc = launch_tile_weight(eng.stream, lm->dtype, lm->table_p, lm->embed, lm->vocab_padded, lm->dm);
         if (rc) { cleanup(); return rc; }
     }
     MRS_LM_HIP(hipStreamSynchronize(eng.stream));
 #undef MRS_LM_HIP
-    if (stage) hipFree(stage);
     *out = lm;
     return MRS_OK;
 }
@@ -1317,22 +1334,18 @@ extern "C" int mrs_lm_set_untied_head(mrs_lm *lm, const float *lm_head) {
     try { host.assign(ne, 0.0f); } catch (...) { return fail(MRS_E_HIP, "mrs_lm_set_untied_head: out of host memory"); }
     for (int d = 0; d < lm->dm; ++d)
         for (int v = 0; v < lm->vocab; ++v) host[(size_t)v * lm->dm + d] = lm_head[(size_t)d * lm->vocab + v];
-    float *stage = nullptr;
     void *dst = lm->head;
     if (!dst) { MRS_HIP(hipMalloc(&dst, ne * es)); }
-    hipError_t e = hipMalloc((void **)&stage, ne * 4);
-    if (e == hipSuccess) e = hipMemcpyAsync(stage, host.data(), ne * 4, hipMemcpyHostToDevice, bb->stream);
-    if (e == hipSuccess) {
-        const dim3 grid((unsigned)((ne + 255) / 256)), block(256);
-        if (lm->dtype == MRS_F32) e = hipMemcpyAsync(dst, stage, ne * 4, hipMemcpyDeviceToDevice, bb->stream);
-        else if (lm->dtype == MRS_BF16) hipLaunchKernelGGL((cast_from_f32_kernel<bf16_t>), grid, block, 0, bb->stream, (bf16_t *)dst, stage, (int64_t)ne);
-        else hipLaunchKernelGGL((cast_from_f32_kernel<f16_t>), grid, block, 0, bb->stream, (f16_t *)dst, stage, (int64_t)ne);
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(bb->stream);
-    if (stage) hipFree(stage);
-    if (e != hipSuccess) { if (!lm->head) hipFree(dst); return fail(MRS_E_HIP, "mrs_lm_set_untied_head: %s", hipGetErrorString(e)); }
-    if (!lm->head) { lm->head = dst; lm->allocs.push_back(dst); }
-    return lm->table_p ? launch_tile_weight(bb->stream, lm->dtype, lm->table_p, dst, lm->vocab_padded, lm->dm) : MRS_OK;
+    hipError_t e = upload_table(lm, dst, host.data(), lm->vocab_padded);
+    if (lm->table_p) {   // the head's tiles are all that is read of it
+        int rc = e == hipSuccess ? launch_tile_weight(bb->stream, lm->dtype, lm->table_p, dst, lm->vocab_padded, lm->dm) : MRS_OK;
+        if (e == hipSuccess && !rc) e = hipStreamSynchronize(bb->stream);
+        hipFree(dst);
+        if (rc) return rc;
+    } else if (e != hipSuccess) {
+        if (!lm->head) hipFree(dst);
+    } else if (!lm->head) { lm->head = dst; lm->allocs.push_back(dst); }
+    return e == hipSuccess ? MRS_OK : fail(MRS_E_HIP, "mrs_lm_set_untied_head: %s", hipGetErrorString(e));
 }
 
 extern "C" void mrs_lm_destroy(mrs_lm *lm) {

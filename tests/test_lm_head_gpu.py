@@ -5,7 +5,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from mamba_rs_amd import GpuMambaBackbone, GpuMambaLM, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
+from mamba_rs_amd import backbone, GpuMambaBackbone, GpuMambaLM, MambaConfig, MambaWeights, WeightDtype  # noqa: E402
 
 
 @pytest.mark.parametrize("dm,B,vocab,dtype,untied", [
@@ -40,6 +40,34 @@ def test_logits_and_pick(dm, B, vocab, dtype, untied):
         assert ((got.double() - hid @ table).abs() <= bound).all(), step
         last = vocab - 1 - np.argmax(got.numpy()[:, ::-1], axis=1)
         assert np.array_equal(lm.get_tokens(), last), step
+
+
+@pytest.mark.parametrize("untied", [False, True])
+def test_what_a_table_takes(untied):
+    """The rows that tokens are looked up in and the head's tiles, 82 MB each; the f32 rows go through a part of them.  Two uploads of a head of its own take no more, and the second is the
+    one that the logits come from."""
+    dm, vocab = 1024, 40000
+    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
+    w = MambaWeights.init(cfg, dm, 3)
+    w.input_proj_w = np.zeros(0, np.float32); w.input_proj_b = np.zeros(0, np.float32)
+    rng = np.random.default_rng(1)
+    embed = rng.standard_normal((vocab, dm), np.float32)
+    eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, 1, WeightDtype.F16)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    lm = GpuMambaLM(eng, embed, rng.standard_normal((dm, vocab), np.float32) if untied else None)
+    head = embed.T
+    if untied:
+        head = rng.standard_normal((dm, vocab), np.float32)
+        backbone._call("mrs_lm_set_untied_head", lm._h, backbone._fp(head))
+    assert free - torch.cuda.mem_get_info()[0] <= 2 * vocab * dm * 2 + (16 << 20)
+    lm.set_tokens(np.zeros(1, np.int32))
+    lm.decode_step()
+    got, hid = lm.last_logits().reshape(-1)[:vocab], eng.download_temporal().astype(np.float16).astype(np.float64)
+    want = (hid @ head.astype(np.float16).astype(np.float64)).reshape(-1)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+    lm.close()
+    eng.close()
 
 
 @pytest.mark.parametrize("dm,B,dtype", [(768, 1, WeightDtype.BF16), (768, 64, WeightDtype.F16), (1024, 33, WeightDtype.BF16), (2560, 16, WeightDtype.BF16), (2560, 3, WeightDtype.F16)])
