@@ -245,6 +245,7 @@ struct mrs_backbone {
     int split_xproj;  // library chain at up to 128 rows of a wide 16-bit model: x_proj as a K-split launch of the own GEMM
     int tiled;   // own chain from two (narrow models) or three rows up: the projections read tiled weights and tiled activation operands
     int wide;    // ... and in_proj / out_proj run on the column-tile kernel of gemm_wide.hip (wide models, up to 64 rows)
+    int prefill_t;   // a prefill's in_proj and out_proj from the transposed copies (where they are there)
     int skinny;  // decode projections on the library's own GEMM (16-bit storage: batch <= 128 or 64, K % 32 == 0; f32: batch <= 4, K % 128 == 0)
     hipStream_t stream;
     rocblas_handle blas;
@@ -508,6 +509,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
     const int64_t rows = (int64_t)B * T;
     const size_t es = esize(dt);
     const int L = bb->cfg.n_layers;
+    const bool turned = bb->prefill_t;
     const int slices = T > 1 && s->out_parts ? mid_gemm_slices(rows, dm, di) : 1;
     if (T == 1 && bb->skinny) MRS_TRY(decode_chain(bb, s, 0, B, bb->stream));
     for (int l = 0; l < L && !(T == 1 && bb->skinny); l++) {
@@ -529,7 +531,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
             MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, di, dm));
             MRS_TRY(launch_skinny_gemm(bb->stream, dt, (char *)s->proj + es * (r * 2 * di + di), 0, (int64_t)T * 2 * di, (const char *)s->normed + es * r * dm, (int64_t)T * dm,
                                        (const char *)lw.in_proj_t + es * di * dm, B, di, dm, SkinnyEpi()));
-        } else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, lw.in_proj_t, (int)rows, 2 * di, dm));
+        } else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, turned ? lw.in_proj_t : nullptr, (int)rows, 2 * di, dm));
         else if (lw.in_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj_t, (int)rows, 2 * di, dm));
         else MRS_TRY(gemm_rm(bb, dt, s->proj, 2 * di, s->normed, dm, lw.in_proj, (int)rows, 2 * di, dm));
         if (T == 1) {
@@ -607,7 +609,7 @@ static int run_layers(mrs_backbone *bb, Scratch *s, int T, bool prefix = false) 
         if (prefix && l + 1 == L) return MRS_OK;
         if (last) MRS_TRY(launch_last_step_gemm(bb->stream, dt, s->out, s->y, lw.out_proj_t, B, T, dm, di));
         else if (in_parts && l + 1 < L) MRS_TRY(launch_mid_gemm_parts(bb->stream, dt, s->out_parts, s->y, di, lw.out_proj_t, rows, dm, di, slices));
-        else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, lw.out_proj_t, (int)rows, dm, di));
+        else if (T > 1) MRS_TRY(prefill_projection(bb, dt, s->out, dm, s->y, di, lw.out_proj, turned ? lw.out_proj_t : nullptr, (int)rows, dm, di));
         else if (lw.out_proj_t) MRS_TRY(gemm_rm_t(bb, dt, s->out, dm, s->y, di, lw.out_proj_t, (int)rows, dm, di));
         else MRS_TRY(gemm_rm(bb, dt, s->out, dm, s->y, di, lw.out_proj, (int)rows, dm, di));
     }
@@ -798,9 +800,9 @@ extern "C" int mrs_backbone_create(mrs_backbone **out, int gpu_ordinal, const mr
         bb->split_xproj = !off && !bb->skinny && (dtype == MRS_BF16 || dtype == MRS_F16) && batch <= 128 && di % 256 == 0 && xd % 8 == 0 &&
                           !narrow_model(di, xd);
         // f32 storage: the same chain, on the row-wise route of the GEMM (one to four rows, rows of the operand in LDS) and on the matrix cores (own_f32_chain_rows)
-        if (!off && dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 &&
-            getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
-            bb->skinny = 1;
+        const bool row_by_row = !off && dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 && getenv("MRS_DECODE_NO_ROWWISE") == nullptr;
+        if (row_by_row) bb->skinny = 1;
+        bb->prefill_t = dtype != MRS_F32 || f32_prefill_transposed(dm, di, row_by_row);
         if (!off && dtype == MRS_F32 && batch <= std::min(skinny_max_rows(), own_f32_chain_rows(dm, di, false)) && dm % 32 == 0 && di % 32 == 0 && !tiny) bb->skinny = 1;
     }
     choose_resident(bb);

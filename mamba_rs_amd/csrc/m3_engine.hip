@@ -610,6 +610,7 @@ struct mrs_m3_backbone {
     void *pf_bcn;            // [rows][2 * d_state] normalised and weighted B | C rows (activation type) for the scan that forms K and Q itself
     float *pf_parts;        // out_proj as pf_n_parts products over slices of K, [pf_n_parts][rows][d_model] (few rows)
     int pf_n_parts;
+    int prefill_t;          // a prefill's out_proj from the transposed copy (where it is there)
     void *pf_normed, *pf_bulk, *pf_x, *pf_K, *pf_Q, *pf_y, *pf_gated, *pf_out, *pf_ws;
     size_t pf_ws_bytes;
 };
@@ -953,8 +954,9 @@ extern "C" int mrs_m3_backbone_create(mrs_m3_backbone **out, int gpu_ordinal, co
     { const char *e = getenv("MRS_DECODE_NO_TILED"), *m = getenv("MRS_DECODE_TILED_MIN_ROWS");
       bb->tiled = bb->skinny && (dtype == MRS_BF16 || dtype == MRS_F16) && batch >= (m ? atoi(m) : 2) && !(e && atoi(e) != 0); }
     // f32 storage: the row-wise route of the same GEMM, one to four rows
-    if (dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 && getenv("MRS_DECODE_NO_ROWWISE") == nullptr)
-        bb->skinny = 1;
+    const bool row_by_row = dtype == MRS_F32 && batch <= 4 && dm % 128 == 0 && di % 128 == 0 && (int64_t)di * 16 <= 48 * 1024 && getenv("MRS_DECODE_NO_ROWWISE") == nullptr;
+    if (row_by_row) bb->skinny = 1;
+    bb->prefill_t = dtype != MRS_F32 || f32_prefill_transposed(dm, di, row_by_row);
     const bool tiny = [&] {   // small f32 models: a step is one launch (MRS_DECODE_NO_TINY=1 keeps the kernel chains)
         const char *e = getenv("MRS_DECODE_NO_TINY");
         return !(e && atoi(e) != 0) && tiny_m3_step_ok(dtype, input_dim, dm, di, nh, cfg->headdim, ds, cfg->ngroups, bb->nr, ip);
@@ -1394,7 +1396,7 @@ int prefill_body3(mrs_m3_backbone *bb, int T) {
             MRS_TRY(launch_mid_gemm_parts(bb->stream, dt, bb->pf_parts, bb->pf_gated, di, lw.out_proj_t, rows, dm, di, bb->pf_n_parts));
         else if (const OwnProjection own = own_projection(bb, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di))
             MRS_TRY(launch_own_projection(bb, own, 0, bb->pf_out, dm, bb->pf_gated, lw.out_proj_t, rows, dm, di));
-        else if (lw.out_proj_t) {   // (the vendor kernels for the transposed operand: 16384 x 768 x 1536 44.4 -> 41.0 us)
+        else if (lw.out_proj_t && bb->prefill_t) {   // (the vendor kernels for the transposed operand: 16384 x 768 x 1536 44.4 -> 41.0 us)
             const rocblas_datatype t = blas_type3(dt);
             MRS_TRY(gemm_ex_tuned(bb->tuner, bb->blas, bb->stream, 1, dm, (int)rows, di, lw.out_proj_t, t, di, bb->pf_gated, t, di, bb->pf_out, t, dm));
         } else MRS_TRY(gemm3(bb, bb->pf_out, false, bb->pf_gated, lw.out_proj, (int)rows, dm, di));

@@ -90,6 +90,12 @@ inline int own_f32_chain_rows(int64_t d_model, int64_t d_inner, bool mamba3) {
     return n <= 2400 * 1000 ? 128 : n <= 4200 * 1000 ? 64 : 48;
 }
 
+// f32 models in a prefill, whose products are the library's: whether it is handed the transposed weights, which are there for the decode's own chain.  Its kernels for either order are ahead
+// or behind by size, without a line to be drawn: from the transposed ones the prefill takes, of what it takes from the others, at d_model 1024 118 % with 256 rows, 110 % with 512, 91 % with
+// 768 and 82 % with 2048, at 512 109 % with 128 rows, at 1280 119 % with 2048, at 2048 107 % with 32 rows and 77 % with 768; at 2560 60 to 66 % with up to 384 rows, 81 to 104 % past them.
+// So models of that width alone, and as before those of one to four rows whose steps go row by row.
+inline bool f32_prefill_transposed(int64_t d_model, int64_t d_inner, bool row_by_row) { return row_by_row || d_model * 2 * d_inner > 20 * 1000 * 1000; }
+
 // Whether what a decode step touches (`bytes`: weights, states, the head's table) is more than the chip's last cache holds, 256 MB.  What is read once a step and not kept from one
 // step to the next is then better read past it: cached, it drives out what could have stayed, and changed states have to be written back to make room.
 // The head's table, cached / past, us a step, vocabulary 50280: 130m shape 1 row (259 MB) 205.1 / 202.1, 16 rows 292.7 / 277.7, 64 rows 357 / 351; 20 of its layers 1 row (229 MB)

@@ -99,6 +99,11 @@ def test_the_mamba3_step_has_whole_waves(rules):
             assert r == (4 if batch * nh >= 192 and ds == 64 and hd % 16 == 0 else 1) and hd * (ds // 4) // r % 64 == 0 and hd * (ds // 4) // r >= min(ds, 64), (batch, nh, hd, ds, r)
 
 
+def test_f32_prefills_of_many_rows_read_their_weights_as_they_came(rules):
+    """Engines of five rows and more have transposed copies for their decode; the library is handed them in a prefill only where that is ahead at nearly every size."""
+    assert rules("f32_prefill_transposed(a, 2 * a, b)", [(dm, rbr, 0, 0) for rbr in (0, 1) for dm in (192, 768, 1024, 2048, 2560)]) == [0, 0, 0, 0, 1, 1, 1, 1, 1, 1]
+
+
 def test_rows_of_the_f32_chain(rules):
     dims = (192, 256, 768, 1024, 1536, 2560)
     assert rules("own_f32_chain_rows(a, b, false)", [(dm, 2 * dm, 0, 0) for dm in dims]) == [128, 128, 128, 64, 48, 48]
