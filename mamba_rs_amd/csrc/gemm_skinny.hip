@@ -609,11 +609,17 @@ static int launch_skinny_t(hipStream_t st, TO *C, int64_t ldc, const T *A, int64
         return fail(MRS_E_SHAPE, "skinny gemm: K split needs the matrix-core route, a plain product, a share buffer and ksplit <= K / 32 (ksplit=%d)", ksplit);
     ep.kslice = ((K >> 5) + ksplit - 1) / ksplit;
     const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 15) / 16), (unsigned)(((K >> 5) + ep.kslice - 1) / ep.kslice));
+    // (streamed are in_proj, Mamba-1's with the conv step and Mamba-3's plain one, and an f32 head: rows scaled or f32, but not f32 rows on the matrix cores)
 #define MRS_SG_ROWS(EPI_, PRO_, LPR_, MR_)                                                                                                                \
     do {                                                                                                                                                 \
         const size_t lds = MR_ == 1 ? 0 : (size_t)K * MR_ * sizeof(T);                                                                                   \
-        if (ep.w_stream) hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_, true>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep); \
-        else hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep);               \
+        if constexpr (EPI_ != 2 && (PRO_ == 1 || (EPI_ == 0 && sizeof(T) == 4)) && !(sizeof(T) == 4 && LPR_ == 0)) {                                     \
+            if (ep.w_stream) {                                                                                                                           \
+                hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_, true>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep);     \
+                break;                                                                                                                                   \
+            }                                                                                                                                            \
+        }                                                                                                                                                \
+        hipLaunchKernelGGL((skinny_gemm_kernel<T, TO, EPI_, PRO_, LPR_, MR_>), grid, block, lds, st, C, ldc, A, lda, Wt, M, N, K, ep);                   \
     } while (0)
 #define MRS_SG(EPI_, PRO_)                                                                                                               \
     do {                                                                                                                                 \
