@@ -53,28 +53,32 @@ __global__ __launch_bounds__(64 * WAVES) void lm_head_kernel(float *__restrict__
     }
     lds_barrier();
     // Sums of four k-steps, which are added up: one chain over K of 768 to 2560 is 1.5 to 3.1e-7 off the sum in 64 bits (of their norm), the vendor kernels' 0.8 to 1.4e-7 (to 2.0e-7 at 64 rows), these 0.7 to 1.2e-7.
-    v4f acc[MT], sum[MT];
+    // (A sum joins the others behind the next one's second step, when the matrix cores are done with it.)
+    v4f acc[2][MT], sum[MT];
 #pragma unroll
-    for (int i = 0; i < MT; i++) sum[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MT; i++) sum[i] = acc[1][i] = (v4f){0.f, 0.f, 0.f, 0.f};
     for (int kb = 0; kb < nks; kb += R) {
 #pragma unroll
         for (int r = 0; r < R; r++) {
+            const int h = r / 4 % 2;
             if (r % 4 == 0) {
 #pragma unroll
-                for (int i = 0; i < MT; i++) acc[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < MT; i++) acc[h][i] = (v4f){0.f, 0.f, 0.f, 0.f};
             }
             if (kb + r < nks) {
 #pragma unroll
-                for (int i = 0; i < MT; i++) acc[i] = Mma32<T>::mma(wr[r], hid[((kb + r) * MT + i) * 64 + l], acc[i]);   // (a lane holds four columns of a row)
+                for (int i = 0; i < MT; i++) acc[h][i] = Mma32<T>::mma(wr[r], hid[((kb + r) * MT + i) * 64 + l], acc[h][i]);   // (a lane holds four columns of a row)
             }
             wr[r] = load_table<STREAM>(wp + min(kb + r + R, nks - 1) * 64);
             __builtin_amdgcn_sched_barrier(0);   // each refill right behind its use
-            if (r % 4 == 3) {
+            if (r % 4 == 1) {
 #pragma unroll
-                for (int i = 0; i < MT; i++) sum[i] += acc[i];
+                for (int i = 0; i < MT; i++) sum[i] += acc[1 - h][i];
             }
         }
     }
+#pragma unroll
+    for (int i = 0; i < MT; i++) sum[i] += acc[1][i];
     const int col = 16 * tile + 4 * lg;
 #pragma unroll
     for (int i = 0; i < MT; i++) {
