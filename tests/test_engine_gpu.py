@@ -562,18 +562,20 @@ def test_rows_a_step_hands_to_the_host_are_the_rows_it_leaves_on_the_device(dm, 
     eng.close()
 
 
-@pytest.mark.parametrize("family,dm,B", [("m1", 64, 1), ("m1", 128, 128), ("m1", 96, 3), ("m3", 64, 5), ("m3", 128, 48)])
-def test_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, B):
+@pytest.mark.parametrize("family,dm,ds,B", [("m1", 64, 16, 1), ("m1", 128, 16, 128), ("m1", 64, 8, 3), ("m3", 64, 16, 5), ("m3", 128, 16, 48), ("m3", 96, 16, 3), ("m1", 96, 16, 3)])
+def test_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, ds, B):
     """step() returns on the rows' flags, before its launch has ended: the final rows behind temporal_ptr(), read by another stream with no wait in between, are those of the host, bit
-    for bit (row-streaming and general forms of the single-launch steps)."""
+    for bit (row-streaming and general forms of the single-launch steps, and a step of several launches)."""
     import torch
     from mamba_rs_amd import GpuMamba3Backbone, Mamba3Config, Mamba3Weights
     if family == "m1":
-        cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=2)
+        cfg = MambaConfig(d_model=dm, d_state=ds, d_conv=4, expand=2, n_layers=2)
         eng = GpuMambaBackbone.new(0, MambaWeights.init(cfg, 24, 5), cfg, 24, B)
     else:
-        cfg = Mamba3Config(d_model=dm, d_state=16, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
+        cfg = Mamba3Config(d_model=dm, d_state=ds, expand=2, headdim=16, ngroups=1, n_layers=2, rope_fraction=0.5)
         eng = GpuMamba3Backbone.new(0, Mamba3Weights.init(cfg, 24, 5), cfg, 24, B)
+
+    assert eng.decode_route() == (1 if (family, dm) == ("m1", 96) else 2)
 
     class Rows:
         __cuda_array_interface__ = {"shape": (B, dm), "typestr": "<f4", "version": 3, "data": (eng.temporal_ptr(), False), "strides": None}
@@ -627,21 +629,22 @@ def test_input_rows_of_a_step_are_on_the_device_when_it_returns(family, dm, ds, 
     plain.close()
 
 
-@pytest.mark.parametrize("dm,dc,B", [(64, 4, 1), (128, 4, 64), (96, 3, 3)])
-def test_states_of_a_step_are_on_the_device_when_it_returns(dm, dc, B):
+@pytest.mark.parametrize("dm,dc,ds,B", [(64, 4, 16, 1), (128, 4, 16, 64), (96, 3, 16, 3), (64, 3, 8, 3), (128, 2, 16, 5)])
+def test_states_of_a_step_are_on_the_device_when_it_returns(dm, dc, ds, B):
     """The same of the states behind state_ptrs(): another stream reads those that a later download gives, and a step goes on from what another stream put there."""
     import ctypes
     import torch
     from mamba_rs_amd import backbone
-    cfg = MambaConfig(d_model=dm, d_state=16, d_conv=dc, expand=2, n_layers=2)
+    cfg = MambaConfig(d_model=dm, d_state=ds, d_conv=dc, expand=2, n_layers=2)
     eng = GpuMambaBackbone.new(0, MambaWeights.init(cfg, 24, 5), cfg, 24, B)
+    assert eng.decode_route() == (1 if dm == 96 else 2)
     bind, di, last = backbone._bind(), 2 * dm, cfg.n_layers - 1
     conv, ssm = ctypes.c_void_p(), ctypes.c_void_p()
     assert bind.mrs_backbone_state_ptrs(eng._h, last, ctypes.byref(conv), ctypes.byref(ssm)) == 0
 
     def view(ptr, *shape):
         return torch.as_tensor(type("View", (), {"__cuda_array_interface__": {"shape": shape, "typestr": "<f4", "version": 3, "data": (ptr.value, False), "strides": None}})(), device="cuda:0")
-    views, side = [view(conv, B, di, dc), view(ssm, B, di, 16)], torch.cuda.Stream()
+    views, side = [view(conv, B, di, dc), view(ssm, B, di, ds)], torch.cuda.Stream()
     kept = [torch.empty_like(v) for v in views]
     rng = np.random.default_rng(B)
     with torch.cuda.stream(side):

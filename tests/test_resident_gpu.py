@@ -15,21 +15,27 @@ from mamba_rs_amd import GpuMambaBackbone, MambaConfig, MambaWeights, WeightDtyp
 @pytest.mark.parametrize("dm,L,B", [(1024, 20, 1), (1024, 20, 3), (2560, 4, 3), (1024, 20, 40), (1024, 20, 65)])
 def test_weights_past_the_last_cache(dm, L, B):
     """Models whose weights are more than the last cache holds, so that some layers' (resident steps of a row and of several) or all layers' in_proj (a launch per product) are read past it,
-    and there the states as well (three forms of the step kernel): outputs against the CPU route, as below."""
+    and there the states as well (three forms of the step kernel): outputs against the CPU route, as below.  Every layer has weights of its own (one layer's with their columns moved
+    along), so that a block of another layer's shows."""
+    import copy
     cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=1)
     w = MambaWeights.init(cfg, dm, 11)
     w.input_proj_w = np.zeros((0, dm), np.float32)
     cfg = MambaConfig(d_model=dm, d_state=16, d_conv=4, expand=2, n_layers=L)
-    w.layers = w.layers * L
+    w.layers = [copy.copy(w.layers[0]) for _ in range(L)]
+    for l, lw in enumerate(w.layers):
+        for n in ("in_proj_w", "x_proj_w", "dt_proj_w", "out_proj_w"):
+            setattr(lw, n, np.roll(getattr(lw, n), 37 * l, axis=1))
     P = oracle_params(w, cfg, dm, round_to=orc.BF16)
     print(f"case past the cache {dm} {L} {B}", flush=True)
     eng = GpuMambaBackbone.new_with_dtype(0, w, cfg, dm, B, WeightDtype.BF16)
-    st = orc.m1_zero_state(P)
+    st = {b: orc.m1_zero_state(P) for b in {0, B - 1}}
     for t in range(2):
         x = np.random.default_rng(t).standard_normal((B, dm)).astype(np.float32)
         got = eng.step(x)
-        want = orc.m1_backbone_step(P, x[B - 1], *st, identity_proj=True)
-        assert cosine(got[B - 1], want) >= 0.999, (t, cosine(got[B - 1], want))
+        for b in st:
+            want = orc.m1_backbone_step(P, x[b], *st[b], identity_proj=True)
+            assert cosine(got[b], want) >= 0.999, (t, b, cosine(got[b], want))
     eng.close()
 
 
