@@ -23,9 +23,14 @@ SCAN_FLAGS_ZERO = 1 << 5
 SCAN_TWO_LAUNCHES = 1 << 6
 
 
+_raw_stream, _device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))   # (private to torch)
+
+
 def _stream() -> int:
-    """torch's current stream (of the current device), without the Stream object around it: 0.3 us against 1.6."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    """torch's current stream (of the current device), where it can be had without the Stream object around it: 0.3 us against 1.6."""
+    if _raw_stream is None or _device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 def _p(t: torch.Tensor | None) -> int | None:

@@ -353,6 +353,17 @@ def test_scan_rejects_bad_arguments():
     torch.cuda.synchronize()
 
 
+def test_calls_go_to_torch_s_current_stream(monkeypatch):
+    """With torch's private functions and without them."""
+    side = torch.cuda.Stream()
+    for gone in (False, True):
+        if gone:
+            monkeypatch.setattr(ops, "_raw_stream", None)
+        assert ops._stream() == torch.cuda.current_stream().cuda_stream != side.cuda_stream
+        with torch.cuda.stream(side):
+            assert ops._stream() == side.cuda_stream
+
+
 def test_scan_refuses_what_it_cannot_read():
     """Each operand wrong in turn: another dtype, another shape, strides that are not row-dense, the host's memory."""
     B, T, di, ds = 2, 24, 64, 16
