@@ -246,7 +246,7 @@ struct mrs_backbone {
     int tiled;   // own chain from two (narrow models) or three rows up: the projections read tiled weights and tiled activation operands
     int wide;    // ... and in_proj / out_proj run on the column-tile kernel of gemm_wide.hip (wide models, up to 64 rows)
     int prefill_t;   // a prefill's in_proj and out_proj from the transposed copies (where they are there)
-    int skinny;  // decode projections on the library's own GEMM (16-bit storage: batch <= 128 or 64, K % 32 == 0; f32: batch <= 4, K % 128 == 0)
+    int skinny;  // decode projections on the library's own GEMM (batch <= 128 or less by width and storage, K % 32 == 0)
     hipStream_t stream;
     rocblas_handle blas;
     GemmTuner *tuner;       // vendor-kernel choice for the prefill projections (off unless asked for)

@@ -13,7 +13,7 @@
 //      mamba3_layer_step (src/mamba3_siso/cpu/inference.rs:68-258) and kernels/mamba3_ops.cu;
 //   3. out_proj with the residual add, the next layer's pre-scaled operand and row sums of squares as epilogue.
 // At one row of a 16-bit model, and at a few of a shallow one, the whole step is one resident launch (resident_m3_row.hip, resident_m3_step.hip).
-// Shapes the skinny GEMM does not take (f32 storage above four rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
+// Shapes the skinny GEMM does not take (f32 storage past own_f32_chain_rows among them) run RMSNorm + rocBLAS GEMMs around the same step kernel.
 #include "common.hpp"
 #include "gemm_tune.hpp"
 #include "host_io.hpp"
