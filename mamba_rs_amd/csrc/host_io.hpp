@@ -13,7 +13,7 @@ namespace mrs {
 
 // A flag has a line of host memory to itself: the host reads it over and over while the GPU's writes come in, and with sixteen rows' flags in a line every one
 // of those writes takes the line away from it.  Flags apart, rows and states written past the caches (host_store below), a step of three f32 layers, before / now, us:
-// d_model 64 1 row 20.1 / 19.1, 48 rows 27.2 / 20.9, 128 rows 38.6 / 21.5; 128 28.1 / 28.4, 35.7 / 30.4, 48.0 / 32.1; Mamba-3, four layers of 128, 34.5 / 32.4, 41.4 / 34.6, 53.9 / 35.6.
+// d_model 64 1 row 20.2 / 19.2, 48 rows 27.2 / 21.3, 128 rows 38.9 / 21.9; 128 28.3 / 27.4, 36.4 / 29.7, 48.6 / 31.5; Mamba-3, four layers of 128, 35.3 / 33.3, 42.0 / 34.6, 54.4 / 36.3.
 constexpr int kHostFlag = 16;
 
 struct HostIo {
